@@ -146,7 +146,8 @@ DeltaArgs = _struct(
     "DeltaArgs", "msa_delta_args", (c_int, "dtype heads kv_heads dim dp vdim vp gate_act"),
     (c_void_p, "qkv"), (c_int64, "ld"), (c_void_p, "ba"), (c_int, "ldba"),
     (c_void_p, "decay_rate dt_bias decay state o gate"), (c_int64, "ld_gate"), (c_void_p, "w"),
-    (c_float, "eps"), (c_void_p, "out"), (c_int64, "ld_out"), (c_int, "out_mb"))
+    (c_float, "eps"), (c_void_p, "out"), (c_int64, "ld_out"), (c_int, "out_mb"),
+    (c_void_p, "scratch"), (c_int64, "scratch_floats"))
 GroupedArgs = _struct(
     "GroupedArgs", "msa_grouped_args", (c_int, "dtype heads kv_heads hd vd chunk rot_dims rows"),
     (c_float, "scale"), (c_void_p, "inv_freq q k v"), (c_int64, "ld"),
@@ -219,7 +220,8 @@ HYBRID_SIGNATURES = {
                           ctypes.POINTER(c_void_p)],
     "msa_hybrid_step": [_P, ctypes.POINTER(HybridStepArgs), _P],
 }
-HYBRID_OTHER_SYMBOLS = ["msa_hybrid_destroy", "msa_hybrid_workspace_bytes"]
+HYBRID_OTHER_SYMBOLS = ["msa_hybrid_destroy", "msa_hybrid_workspace_bytes",
+                        "msa_delta_scratch_floats"]
 
 _lib = None
 _hybrid_lib = None
@@ -251,6 +253,8 @@ def load_hybrid():
         lib.msa_hybrid_destroy.restype = None
         lib.msa_hybrid_workspace_bytes.argtypes = [_P, ctypes.POINTER(HybridStepArgs)]
         lib.msa_hybrid_workspace_bytes.restype = c_int64
+        lib.msa_delta_scratch_floats.argtypes = [ctypes.POINTER(DeltaArgs), _BP]
+        lib.msa_delta_scratch_floats.restype = c_int64
         _hybrid_lib = lib
     return _hybrid_lib
 

@@ -1,0 +1,728 @@
+// The gated delta rule over segments of many tokens, sixteen tokens at a time on the fp32 matrix cores.
+//
+// With S0 the state in front of a chunk, p_i the decays of tokens 1 .. i multiplied (per key channel), and
+// k'_i = p_i k_i, q'_i = p_i q_i, the recurrence S_i = g_i S_{i-1} + k_i u_i^T,
+// u_i = beta_i (v_i - (g_i S_{i-1})^T k_i), o_i = S_i^T q_i of recurrent.hip's scan is
+//   U = T (V - K' S0),     T = (I + L)^{-1} diag(beta),  L_ij = beta_i k_i . (p_i / p_j) k_j   (j < i),
+//   O = Q' S0 + A U,       A_ij = q_i . (p_i / p_j) k_j                                          (j <= i),
+//   S = p_C S0 + K^^T U,   k^_j = (p_C / p_j) k_j.
+// No quotient of decays is ever formed: p_i / p_j is the product of the decays between the two tokens,
+// multiplied up token by token, so a channel that forgets at once is as exact as in the scan.  All of
+// it is fp32, the products on v_mfma_f32_16x16x4_f32.
+//
+// Two kernels.  What does not depend on S0 (T, A, the norms of k and q) is computed for all chunks of all
+// heads at once, a wave each, and left in a scratch record (20 us for 1500 tokens x 32 heads); then the
+// chunks of a (segment, head, some columns) are walked one after the other.  A scan step's chain of LDS reads, two
+// dots, a sum over lanes and the update takes 500 cycles per token whatever the machine has idle; a
+// chunk's chain takes 2800 (3800 with decays per channel, which are multiplied up while staging) per sixteen.
+// Measured, both kernels against the scan, 32 heads of 128 x 128: one segment of 1500 tokens 132 us against 368
+// (decays per channel 184 against 370), 8 x 1024 tokens 300 against 839 (332 against 1018).
+#include <math.h>
+
+#include <type_traits>
+#include <utility>
+
+#include "attention_tiles.h"
+#include "common.h"
+
+namespace {
+
+constexpr int DC_TOK = 16;
+constexpr int DC_WIDE = 128;  // workgroups of several column tiles from which on they take over
+// A record: T and A (16 x 16, row-major), then per token the factors that are one number for all channels,
+// which the loops below apply to 16 x 16 results and not to the operands: of K' S0 (1 / |k|), Q' S0
+// (scale / |q|) and U (1 / |k|), each times the token's product of decays where a head has one decay, and that
+// product over the chunk.  Past the segment's end the factors are 0.
+constexpr int DC_T = 0, DC_A = 256, DC_FK = 512, DC_FQ = 528, DC_FU = 544, DC_GC = 560, DC_REC = 576;
+// (DC_GC holds sixteen copies: one address for all lanes would be a scalar load, whose latency every LDS
+// barrier waits for)
+
+// records of a segment start here: chunks are counted from each segment's own start, and
+// ceil(n / 16) <= floor((first + n) / 16) - floor(first / 16) + 1
+__device__ __forceinline__ int64_t record_of(int first, int seg, int chunk, int heads, int h) {
+  return ((int64_t)(first / DC_TOK + seg + chunk) * heads + h) * DC_REC;
+}
+
+template <int N, int... I, class F>
+__device__ __forceinline__ void each(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void each(F&& f) {  // f(0) .. f(N - 1), the number a constant
+  each<N>(f, std::make_integer_sequence<int, N>{});
+}
+
+// Sums of 64 values over the 64 lanes, two lanes' worth at a time: the lane keeps one half of the values and
+// gives the other half away, so that 64 sums take 63 additions and not 64 x 6.  Lane l ends with the
+// sum of value l.
+__device__ __forceinline__ float transposed_sums(float (&v)[64], int lane) {
+#pragma unroll
+  for (int t = 0; t < 32; ++t) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, v[t]),
+                                                    __builtin_bit_cast(unsigned, v[t + 32]), false, false);
+    v[t] = __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
+  }
+#pragma unroll
+  for (int t = 0; t < 16; ++t) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, v[t]),
+                                                    __builtin_bit_cast(unsigned, v[t + 16]), false, false);
+    v[t] = __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
+  }
+#define DC_HALVE(W, CTRL)                                    \
+  _Pragma("unroll") for (int t = 0; t < W; ++t) {            \
+    const bool up = lane & W;                                \
+    const float keep = up ? v[t + W] : v[t], give = up ? v[t] : v[t + W]; \
+    v[t] = keep + dpp_move<CTRL, 0xf>(0.f, give);            \
+  }
+  DC_HALVE(8, 0x128)  // row_ror:8
+  DC_HALVE(4, 0x141)  // row_half_mirror: the lane with the other bits 0 .. 2
+  DC_HALVE(2, 0x4E)   // quad_perm [2,3,0,1]
+  DC_HALVE(1, 0xB1)   // quad_perm [1,0,3,2]
+#undef DC_HALVE
+  return v[0];
+}
+
+// Place of a sum in the order the loops below form them: per token j first |k_j|^2, q_j . k_j and |q_j|^2, then
+// for every later token i the sums of L_ij and A_ij.
+constexpr int sum_at(int j) { return 34 * j - j * j; }
+constexpr int DC_SUMS = sum_at(DC_TOK);  // 288
+
+// One wave per (chunk, head).  Bound: the vector ALU (for 128 channels some 800 multiply-adds and
+// 700 steps of the sums per chunk and lane).  The decays between two tokens are multiplied up as j's row moves from token to token.
+template <typename T, int DP, bool CH>
+__global__ __launch_bounds__(256) void delta_prepare_kernel(
+    const T* __restrict__ qkv, int64_t ld, const float* __restrict__ ba, int ldba,
+    const float* __restrict__ decay_rate, const float* __restrict__ dt_bias,
+    const float* __restrict__ decay, int heads, int kv_heads, float q_scale, float* __restrict__ records,
+    const int32_t* __restrict__ seg_start, const int32_t* __restrict__ seg_pos) {
+  constexpr int CE = (DP + 63) / 64;  // channels per lane
+  __shared__ float sums[4][(DC_SUMS + 63) / 64 * 64], tok[4][4][DC_TOK];
+  const int s = blockIdx.z, t0 = blockIdx.x * DC_TOK;
+  const int first = seg_start[s], n = seg_start[s + 1] - first;
+  if (t0 >= n || seg_pos[s] < 0) return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int h_own = blockIdx.y * 4 + wave, h = min(h_own, heads - 1);
+  const int hk = h / (heads / kv_heads), c0 = lane * CE;
+  const bool live = c0 < DP;
+  const T* base = qkv + (int64_t)first * ld + hk * DP + (live ? c0 : 0);
+  float k[DC_TOK][CE], q[DC_TOK][CE], g[CH ? DC_TOK : 1][CE];
+#pragma unroll
+  for (int t = 0; t < DC_TOK; ++t) {
+    const int tt = min(t0 + t, n - 1);
+    const bool use = live && t0 + t < n;
+    const T* p = base + (int64_t)tt * ld;
+#pragma unroll
+    for (int e = 0; e < CE; ++e) {
+      const float qv = (float)p[e], kv = (float)p[kv_heads * DP + e];
+      q[t][e] = use ? qv : 0.f;
+      k[t][e] = use ? kv : 0.f;
+      if constexpr (CH) {
+        const float d = decay[((int64_t)(first + tt) * heads + h) * DP + (live ? c0 : 0) + e];
+        g[t][e] = use ? d : 1.f;
+      }
+    }
+  }
+  if (lane < DC_TOK) {
+    const bool in = t0 + lane < n;
+    const float* z = ba + (int64_t)(first + min(t0 + lane, n - 1)) * ldba;
+    tok[wave][0][lane] = in ? sigmoidf(z[h]) : 0.f;
+    if (!CH) tok[wave][3][lane] = in ? decay_of(z[heads + h] + dt_bias[h], decay_rate[h]) : 1.f;
+  }
+  __syncthreads();
+  float gs[CH ? 1 : DC_TOK];
+  if constexpr (!CH) {
+#pragma unroll
+    for (int t = 0; t < DC_TOK; ++t) gs[t] = tok[wave][3][t];
+  }
+  float v[64];
+  auto emit = [&](auto at, float x) {
+    constexpr int A = decltype(at)::value;
+    v[A & 63] = x;
+    if constexpr ((A & 63) == 63) sums[wave][A - 63 + lane] = transposed_sums(v, lane);
+  };
+  auto dot = [&](const float (&a)[CE], const float (&b)[CE]) {
+    float d = a[0] * b[0];
+#pragma unroll
+    for (int e = 1; e < CE; ++e) d = fmaf(a[e], b[e], d);
+    return d;
+  };
+  each<DC_TOK>([&](auto jc) {
+    constexpr int j = decltype(jc)::value, at = sum_at(j);
+    emit(std::integral_constant<int, at>{}, dot(k[j], k[j]));
+    emit(std::integral_constant<int, at + 1>{}, dot(q[j], k[j]));
+    emit(std::integral_constant<int, at + 2>{}, dot(q[j], q[j]));
+    float w[CE];
+#pragma unroll
+    for (int e = 0; e < CE; ++e) w[e] = k[j][e];
+    each<DC_TOK - 1 - j>([&](auto ic) {
+      constexpr int i = j + 1 + decltype(ic)::value;
+#pragma unroll
+      for (int e = 0; e < CE; ++e) w[e] *= CH ? g[CH ? i : 0][e] : gs[CH ? 0 : i];
+      emit(std::integral_constant<int, at + 1 + 2 * (i - j)>{}, dot(k[i], w));
+      emit(std::integral_constant<int, at + 2 + 2 * (i - j)>{}, dot(q[i], w));
+    });
+  });
+  constexpr int rest = (DC_SUMS + 63) / 64 * 64 - DC_SUMS;
+  each<rest>([&](auto c) { emit(std::integral_constant<int, DC_SUMS + decltype(c)::value>{}, 0.f); });
+  __syncthreads();
+  const float* sm = sums[wave];
+  if (lane < DC_TOK) {
+    const bool in = t0 + lane < n;
+    const int a = 34 * lane - lane * lane;
+    tok[wave][1][lane] = in ? 1.f / sqrtf(sm[a] + 1e-6f) : 0.f;
+    tok[wave][2][lane] = in ? q_scale / sqrtf(sm[a + 2] + 1e-6f) : 0.f;
+  }
+  __syncthreads();
+  if (h_own >= heads) return;
+  float* rec = records + record_of(first, s, blockIdx.x, heads, h);
+  const float *beta = tok[wave][0], *fk = tok[wave][1], *fq = tok[wave][2];
+  if (lane < DC_TOK) {  // column `lane` of T, by substitution
+    float x[DC_TOK];
+    each<DC_TOK>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      float d = 0.f;
+#pragma unroll
+      for (int j = 0; j < i; ++j) d = fmaf(sm[34 * j - j * j + 1 + 2 * (i - j)] * fk[j], x[j], d);
+      x[i] = i < lane ? 0.f : beta[i] * ((i == lane ? 1.f : 0.f) - fk[i] * d);
+      rec[DC_T + i * DC_TOK + lane] = x[i];
+    });
+    float before = 1.f, after = 1.f;
+    if constexpr (!CH) {
+#pragma unroll
+      for (int i = 0; i < DC_TOK; ++i) (i <= lane ? before : after) *= gs[i];
+      rec[DC_GC + lane] = before * after;
+    }
+    rec[DC_FK + lane] = fk[lane] * before;
+    rec[DC_FQ + lane] = fq[lane] * before;
+    rec[DC_FU + lane] = fk[lane] * after;
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int i = (lane >> 4) * 4 + e, j = lane & 15;
+    const int a = 34 * j - j * j;
+    const float raw = sm[i == j ? a + 1 : i > j ? a + 2 + 2 * (i - j) : 0];
+    rec[DC_A + i * DC_TOK + j] = i >= j ? fq[i] * fk[j] * raw : 0.f;
+  }
+}
+
+// What the chunk loops read of a chunk, twice: one is staged while the other is in use.  With one decay
+// per head K' and K^ are both k, the decays being factors of the results.
+template <int DP, bool CH>
+struct Operands {
+  static constexpr int KS = DP + 4;   // a row stride that keeps 16-byte reads free of conflicts
+  float k[2][DC_TOK][KS], q[2][DC_TOK][KS];  // K', Q'
+  float kh[CH ? 2 : 1][CH ? DC_TOK : 1][CH ? KS : 4];  // K^
+  float gc[CH ? 2 : 1][CH ? DP : 4];         // p_C
+  // element (token 4 lg + r, row) of K^ for r = 0 .. 3: the A operand of the state's update
+  __device__ __forceinline__ float4_t key_column(int b, int lg, int row) const {
+    float4_t v;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = CH ? kh[CH ? b : 0][CH ? lg * 4 + r : 0][CH ? row : 0] : k[b][lg * 4 + r][row];
+    return v;
+  }
+};
+
+// The four staging waves of a workgroup (thread t of 256).  One decay per head: a thread moves 8 channels of a
+// token.  Decays per channel: a thread owns two channels of k (the first two waves) or q over half of
+// the chunk's tokens and multiplies the decays up; the lane 32 away has the other half.
+// Chunks are requested two ahead.  The loops of these kernels take chunks in pairs and without conditions
+// around their loads, so that each wait is for the oldest chunk alone; an odd number of chunks is made even
+// by one past the end, whose factors are set to 0 and its decays to 1, which changes nothing.
+template <typename T, int DP, bool CH>
+struct Stager {
+  typedef T t4 __attribute__((ext_vector_type(4), aligned(8)));
+  typedef T t2 __attribute__((ext_vector_type(2), aligned(2 * sizeof(T))));
+  typedef float f2 __attribute__((ext_vector_type(2), aligned(8)));
+  struct Raw {
+    t4 x[CH ? 1 : 4];       // one decay per head: 8 of k, 8 of q
+    t2 y[CH ? 8 : 1];
+    f2 g[CH ? 8 : 1];
+  };
+  const T *ksrc, *qsrc;      // uniform: the head's first channel of the segment's first token
+  const float* dsrc;
+  int64_t ld, ldd;
+  int n, t, half;
+  unsigned at;               // first channel of the thread
+  bool is_k, live;
+
+  __device__ Stager(int t_, const T* rows, int64_t ld_, const float* decay, int first, int heads, int kv_heads,
+                    int h, int n_) {
+    t = t_;
+    n = n_;
+    ld = ld_;
+    const int hk = h / (heads / kv_heads);
+    qsrc = rows + hk * DP;
+    ksrc = qsrc + kv_heads * DP;
+    ldd = (int64_t)heads * DP;
+    dsrc = CH ? decay + ((int64_t)first * heads + h) * DP : nullptr;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    is_k = wave < 2;
+    half = (t >> 5) & 1;
+    const int pair = (wave & 1) * 32 + (t & 31);
+    live = CH ? pair < DP / 2 : t < 2 * DP;
+    at = CH ? min(pair, DP / 2 - 1) * 2 : min(t, 2 * DP - 1) % (DP / 8) * 8;
+  }
+  __device__ __forceinline__ void fetch(Raw& a, int c) const {
+    if constexpr (CH) {
+      const T* src = is_k ? ksrc : qsrc;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int tt = min(c * DC_TOK + half * 8 + i, n - 1);
+        a.y[i] = *reinterpret_cast<const t2*>(src + tt * ld + at);
+        a.g[i] = *reinterpret_cast<const f2*>(dsrc + tt * ldd + at);
+      }
+    } else {
+      const int64_t row = min(c * DC_TOK + min(t, 2 * DP - 1) / (DP / 8), n - 1) * ld + at;
+      a.x[0] = *reinterpret_cast<const t4*>(ksrc + row);
+      a.x[1] = *reinterpret_cast<const t4*>(ksrc + row + 4);
+      a.x[2] = *reinterpret_cast<const t4*>(qsrc + row);
+      a.x[3] = *reinterpret_cast<const t4*>(qsrc + row + 4);
+    }
+  }
+  __device__ __forceinline__ void stage(Operands<DP, CH>& L, const Raw& a, int c) const {
+    const int b = c & 1;
+    if constexpr (!CH) {
+      if (!live) return;
+      const int tok = t / (DP / 8);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<float4_t*>(&(i < 2 ? L.k : L.q)[b][tok][at + (i & 1) * 4]) =
+            float4_t{(float)a.x[i][0], (float)a.x[i][1], (float)a.x[i][2], (float)a.x[i][3]};
+      return;
+    }
+    f2 g[8], p = {1.f, 1.f};
+    const int left = n - c * DC_TOK - half * 8;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      g[i] = a.g[CH ? i : 0];
+      if (i >= left) g[i] = f2{1.f, 1.f};
+      p[0] *= g[i][0], p[1] *= g[i][1];
+    }
+    const f2 other = {__shfl_xor(p[0], 32, MSA_WAVE), __shfl_xor(p[1], 32, MSA_WAVE)};
+    if (!live) return;
+    const int tok = half * 8;
+    f2 m = {half ? other[0] : 1.f, half ? other[1] : 1.f};
+    f2 x[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      x[i] = f2{(float)a.y[CH ? i : 0][0], (float)a.y[CH ? i : 0][1]};
+      m[0] *= g[i][0], m[1] *= g[i][1];
+      *reinterpret_cast<f2*>(&(is_k ? L.k : L.q)[b][tok + i][at]) = f2{x[i][0] * m[0], x[i][1] * m[1]};
+    }
+    if (is_k) {
+      m = f2{half ? 1.f : other[0], half ? 1.f : other[1]};
+#pragma unroll
+      for (int i = 7; i >= 0; --i) {
+        *reinterpret_cast<f2*>(&L.kh[CH ? b : 0][CH ? tok + i : 0][CH ? at : 0]) = f2{x[i][0] * m[0], x[i][1] * m[1]};
+        m[0] *= g[i][0], m[1] *= g[i][1];
+      }
+    } else if (half) {
+      *reinterpret_cast<f2*>(&L.gc[CH ? b : 0][CH ? at : 0]) = m;
+    }
+  }
+};
+
+__device__ __forceinline__ float4_t mfma4(float4_t a, float4_t b, float4_t c) {  // c + a (16 x 16) b (16 x 16)
+#pragma unroll
+  for (int r = 0; r < 4; ++r) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[r], b[r], c, 0, 0, 0);
+  return c;
+}
+// c[t] += a[t] b[t] for N independent accumulators, in turn
+template <int N>
+__device__ __forceinline__ void mfma4(const float4_t (&a)[N], const float4_t (&b)[N], float4_t (&c)[N]) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int t = 0; t < N; ++t) c[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[t][r], b[t][r], c[t], 0, 0, 0);
+}
+__device__ __forceinline__ bool finite(float v) { return fabsf(v) <= 3.4028234663852886e38f; }
+
+// A lane's part of a record: tokens 4 lg .., and row lm of T
+struct Factors {
+  float4_t t, k, q, u;
+  float gc;
+  __device__ __forceinline__ void fetch(const float* rec0, int64_t rec_step, int c, int nch, int lm, int lg, bool ch) {
+    const float* rec = rec0 + min(c, nch - 1) * rec_step;
+    t = *reinterpret_cast<const float4_t*>(rec + DC_T + lm * DC_TOK + lg * 4);
+    k = *reinterpret_cast<const float4_t*>(rec + DC_FK + lg * 4);
+    q = *reinterpret_cast<const float4_t*>(rec + DC_FQ + lg * 4);
+    u = *reinterpret_cast<const float4_t*>(rec + DC_FU + lg * 4);
+    gc = ch ? 1.f : rec[DC_GC + lm];
+  }
+  __device__ __forceinline__ void end(int c, int nch) {  // a chunk past the end changes nothing
+    if (c >= nch) u = float4_t{0.f, 0.f, 0.f, 0.f}, gc = 1.f;
+  }
+};
+
+// V - K' S0 of a lane's four tokens 4 lg .. of one column.  A value that is not finite would reach the
+// earlier tokens of its chunk as 0 x NaN: such a column goes through U with zeros from that token on
+// (returned; 16: all are finite) and gets NaN there afterwards.
+template <typename T>
+__device__ __forceinline__ int right_hand_side(const T (&v)[4], float4_t ks, float4_t f, int lg, float4_t& out) {
+  bool fine = true;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    out[r] = fmaf(-f[r], ks[r], (float)v[r]);
+    fine &= finite(out[r]);
+  }
+  int bad = DC_TOK;
+  if (!__all(fine)) {  // uniform
+#pragma unroll
+    for (int r = 3; r >= 0; --r)
+      if (!finite(out[r])) bad = lg * 4 + r;
+    bad = min(bad, __shfl_xor(bad, 16, MSA_WAVE));
+    bad = min(bad, __shfl_xor(bad, 32, MSA_WAVE));
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (lg * 4 + r >= bad) out[r] = 0.f;
+  }
+  return bad;
+}
+
+template <int DP, bool CH>
+struct FewLds {
+  Operands<DP, CH> op;
+  float a[4][DC_TOK][DC_TOK + 4];            // A of the chunk being staged, used and finished
+  float4_t ks[4][64], qs[2][4][64], u[2][64];
+  int bad[2][16];
+};
+
+// Few segments: a workgroup owns one segment, one head and 16 of its columns for all of the segment's chunks.
+// Waves 0 .. 3 hold the state, a quarter of its rows each, as MFMA accumulators (a lane: four rows of one
+// column), which are the B operands of the next chunk's products as they lie; they sum K' S0 through
+// LDS, form U redundantly and update their rows.  Waves 4 .. 7 run beside them: they stage the next chunk and
+// finish the previous chunk's outputs.  Two barriers per chunk.
+template <typename T, int DP, bool CH>
+__global__ __launch_bounds__(512) void delta_chunk_kernel(
+    const T* __restrict__ qkv, int64_t ld, const float* __restrict__ decay, int heads, int kv_heads, int vp,
+    float* __restrict__ state, const float* __restrict__ records, float* __restrict__ o,
+    const int32_t* __restrict__ seg_start, const int32_t* __restrict__ seg_slot,
+    const int32_t* __restrict__ seg_pos) {
+  constexpr int TILES = DP / 16, TPW = (TILES + 3) / 4;  // 16-row tiles of the state, per wave
+  extern __shared__ __attribute__((aligned(16))) char dc_lds[];
+  FewLds<DP, CH>& L = *reinterpret_cast<FewLds<DP, CH>*>(dc_lds);
+  const int s = blockIdx.z, h = blockIdx.y, col0 = blockIdx.x * 16;
+  const int first = seg_start[s], n = seg_start[s + 1] - first, pos = seg_pos[s];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lm = lane & 15, lg = lane >> 4;
+  float* out = o + (int64_t)first * heads * vp + h * vp + col0;
+  if (pos < 0) {
+    for (int i = tid; i < n * 16; i += 512) out[(int64_t)(i >> 4) * heads * vp + (i & 15)] = 0.f;
+    return;
+  }
+  const int nch = (n + DC_TOK - 1) / DC_TOK;
+  const T* rows = qkv + (int64_t)first * ld;
+  const float* rec0 = records + record_of(first, s, 0, heads, h);
+  const int64_t rec_step = (int64_t)heads * DC_REC;
+
+  if (wave < 4) {
+    const int v_at = 2 * kv_heads * DP + h * vp + col0 + lm;
+    float* st = state + (((int64_t)seg_slot[s] * heads + h) * vp + col0 + lm) * DP + lg * 4;
+    float4_t S[TPW];
+#pragma unroll
+    for (int t = 0; t < TPW; ++t) {
+      S[t] = float4_t{0.f, 0.f, 0.f, 0.f};
+      if (pos > 0 && wave * TPW + t < TILES)
+        S[t] = *reinterpret_cast<const float4_t*>(st + (wave * TPW + t) * 16);
+    }
+    struct Ahead {
+      T v[4];
+      Factors f;
+    } ahead[2];
+    auto fetch = [&](Ahead& a, int c) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) a.v[r] = rows[(int64_t)min(c * DC_TOK + lg * 4 + r, n - 1) * ld + v_at];
+      a.f.fetch(rec0, rec_step, c, nch, lm, lg, CH);
+    };
+    auto chunk = [&](Ahead& a, int c) {
+      const int b = c & 1;
+      auto times_state = [&](const float* x) {
+        // (tiles past the end: a state of zeros times some row in bounds)
+        float4_t sum[TPW], a[TPW];
+#pragma unroll
+        for (int t = 0; t < TPW; ++t) {
+          sum[t] = float4_t{0.f, 0.f, 0.f, 0.f};
+          a[t] = *reinterpret_cast<const float4_t*>(x + min(wave * TPW + t, TILES - 1) * 16);
+        }
+        mfma4(a, S, sum);
+#pragma unroll
+        for (int t = 1; t < TPW; ++t) sum[0] += sum[t];
+        return sum[0];
+      };
+      L.ks[wave][lane] = times_state(&L.op.k[b][lm][lg * 4]);
+      lds_barrier();  // A
+      float4_t ks = L.ks[0][lane];
+#pragma unroll
+      for (int w = 1; w < 4; ++w) ks += L.ks[w][lane];
+      L.qs[b][wave][lane] = times_state(&L.op.q[b][lm][lg * 4]) * a.f.q;
+      float4_t rhs;
+      const int bad = right_hand_side(a.v, ks, a.f.k, lg, rhs);
+      float4_t u = mfma4(a.f.t, rhs, float4_t{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (lg * 4 + r >= bad) u[r] = 0.f;
+      if (wave == 0) {
+        L.u[b][lane] = u;
+        if (lane < 16) L.bad[b][lane] = bad;
+      }
+      a.f.end(c, nch);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) u[r] = lg * 4 + r >= bad ? __builtin_nanf("") : u[r] * a.f.u[r];
+      const float gc = a.f.gc;
+      fetch(a, c + 2);
+      float4_t kh[TPW], us[TPW];
+#pragma unroll
+      for (int t = 0; t < TPW; ++t) {
+        const int row = min(wave * TPW + t, TILES - 1) * 16;
+        if constexpr (CH) S[t] *= *reinterpret_cast<const float4_t*>(&L.op.gc[CH ? b : 0][CH ? row + lg * 4 : 0]);
+        else S[t] *= gc;
+        kh[t] = L.op.key_column(b, lg, row + lm);
+        us[t] = u;
+        if (wave * TPW + t >= TILES) kh[t] = us[t] = float4_t{0.f, 0.f, 0.f, 0.f};
+      }
+      mfma4(kh, us, S);
+      lds_barrier();  // B
+    };
+    fetch(ahead[0], 0);
+    fetch(ahead[1], 1);
+    lds_barrier();  // chunk 0 is staged
+    for (int c = 0; c < nch; c += 2) {
+      chunk(ahead[0], c);
+      chunk(ahead[1], c + 1);
+    }
+#pragma unroll
+    for (int t = 0; t < TPW; ++t)
+      if (wave * TPW + t < TILES) *reinterpret_cast<float4_t*>(st + (wave * TPW + t) * 16) = S[t];
+    return;
+  }
+
+  typedef Stager<T, DP, CH> St;
+  const int ht = tid - 256;
+  const St stager(ht, rows, ld, decay, first, heads, kv_heads, h, n);
+  struct Raw {
+    typename St::Raw r;
+    float a;  // element ht of A
+  } raw[2];
+  auto fetch = [&](Raw& x, int c) {
+    stager.fetch(x.r, c);
+    x.a = rec0[min(c, nch - 1) * rec_step + DC_A + ht];
+  };
+  auto stage = [&](const Raw& x, int c) {
+    L.a[c & 3][ht >> 4][ht & 15] = x.a;
+    stager.stage(L.op, x.r, c);
+  };
+  // outputs of chunk c, by one of the four waves in turn (with decays per channel, of the two that stage q)
+  auto finish = [&](int c) {
+    if (c < 0 || (CH ? (c & 1) != wave - 6 : (c & 3) != wave - 4)) return;
+    const int b = c & 1;
+    float4_t y = L.qs[b][0][lane];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) y += L.qs[b][w][lane];
+    y = mfma4(*reinterpret_cast<const float4_t*>(&L.a[c & 3][lm][lg * 4]), L.u[b][lane], y);
+    const int bad = L.bad[b][lm];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int t = c * DC_TOK + lg * 4 + r;
+      if (t < n) out[(int64_t)t * heads * vp + lm] = lg * 4 + r >= bad ? __builtin_nanf("") : y[r];
+    }
+  };
+  fetch(raw[0], 0);
+  fetch(raw[1], 1);
+  stage(raw[0], 0);
+  fetch(raw[0], 2);
+  lds_barrier();
+  auto beside = [&](Raw& x, int c) {  // x holds chunk c + 1
+    stage(x, c + 1);
+    lds_barrier();  // A
+    fetch(x, c + 3);
+    finish(c - 1);
+    lds_barrier();  // B
+  };
+  for (int c = 0; c < nch; c += 2) {
+    beside(raw[1], c);
+    beside(raw[0], c + 1);
+  }
+  finish((nch + 1) / 2 * 2 - 1);  // (the loop finished all chunks before that one)
+}
+
+// Many segments: a workgroup owns CT x 16 columns of a head, one wave 16 of them with all rows of the state, so
+// that nothing is summed between waves and k, q and decays are staged for CT column tiles at once; four
+// more waves stage.  One barrier per chunk.
+template <typename T, int DP, bool CH, int CT>
+__global__ __launch_bounds__((CT + 4) * 64) void delta_chunk_wide_kernel(
+    const T* __restrict__ qkv, int64_t ld, const float* __restrict__ decay, int heads, int kv_heads, int vp,
+    float* __restrict__ state, const float* __restrict__ records, float* __restrict__ o,
+    const int32_t* __restrict__ seg_start, const int32_t* __restrict__ seg_slot,
+    const int32_t* __restrict__ seg_pos) {
+  constexpr int TILES = DP / 16;
+  extern __shared__ __attribute__((aligned(16))) char dc_lds[];
+  Operands<DP, CH>& L = *reinterpret_cast<Operands<DP, CH>*>(dc_lds);
+  const int s = blockIdx.z, h = blockIdx.y, col0 = blockIdx.x * (CT * 16);
+  const int first = seg_start[s], n = seg_start[s + 1] - first, pos = seg_pos[s];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lm = lane & 15, lg = lane >> 4;
+  if (pos < 0) {
+    for (int i = tid; i < n * CT * 16; i += (CT + 4) * 64)
+      o[(int64_t)(first + i / (CT * 16)) * heads * vp + h * vp + col0 + i % (CT * 16)] = 0.f;
+    return;
+  }
+  const int nch = (n + DC_TOK - 1) / DC_TOK;
+  const T* rows = qkv + (int64_t)first * ld;
+  const float* rec0 = records + record_of(first, s, 0, heads, h);
+  const int64_t rec_step = (int64_t)heads * DC_REC;
+  if (wave >= CT) {
+    typedef Stager<T, DP, CH> St;
+    const St stager(tid - CT * 64, rows, ld, decay, first, heads, kv_heads, h, n);
+    typename St::Raw raw[2];
+    stager.fetch(raw[0], 0);
+    stager.fetch(raw[1], 1);
+    stager.stage(L, raw[0], 0);
+    stager.fetch(raw[0], 2);
+    lds_barrier();
+    auto beside = [&](typename St::Raw& x, int c) {
+      stager.stage(L, x, c + 1);  // (past the last chunk: zeros that nothing, or a surplus chunk, reads)
+      stager.fetch(x, c + 3);
+      lds_barrier();
+    };
+    for (int c = 0; c < nch; c += 2) {
+      beside(raw[1], c);
+      beside(raw[0], c + 1);
+    }
+    return;
+  }
+  const int col = col0 + wave * 16 + lm;
+  const T* vsrc = rows + 2 * kv_heads * DP + h * vp + col;
+  float* out = o + (int64_t)first * heads * vp + h * vp + col;
+  float* st = state + (((int64_t)seg_slot[s] * heads + h) * vp + col) * DP + lg * 4;
+  float4_t S[TILES];
+#pragma unroll
+  for (int t = 0; t < TILES; ++t) {
+    S[t] = float4_t{0.f, 0.f, 0.f, 0.f};
+    if (pos > 0) S[t] = *reinterpret_cast<const float4_t*>(st + t * 16);
+  }
+  struct Ahead {
+    T v[4];
+    float4_t a;
+    Factors f;
+  } ahead[2];
+  auto fetch = [&](Ahead& x, int c) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) x.v[r] = vsrc[(int64_t)min(c * DC_TOK + lg * 4 + r, n - 1) * ld];
+    x.f.fetch(rec0, rec_step, c, nch, lm, lg, CH);
+    x.a = *reinterpret_cast<const float4_t*>(rec0 + min(c, nch - 1) * rec_step + DC_A + lm * DC_TOK + lg * 4);
+  };
+  auto chunk = [&](Ahead& x, int c) {
+    const int b = c & 1;
+    auto times_state = [&](const float* p) {  // two chains
+      float4_t sum[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+      for (int t = 0; t < TILES; t += 2) {
+        const float4_t a[2] = {*reinterpret_cast<const float4_t*>(p + t * 16),
+                               *reinterpret_cast<const float4_t*>(p + t * 16 + 16)};
+        const float4_t x2[2] = {S[t], S[t + 1]};
+        mfma4(a, x2, sum);
+      }
+      return sum[0] + sum[1];
+    };
+    const float4_t ks = times_state(&L.k[b][lm][lg * 4]);
+    float4_t y = times_state(&L.q[b][lm][lg * 4]) * x.f.q;
+    float4_t rhs;
+    const int bad = right_hand_side(x.v, ks, x.f.k, lg, rhs);
+    float4_t u = mfma4(x.f.t, rhs, float4_t{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (lg * 4 + r >= bad) u[r] = 0.f;
+    y = mfma4(x.a, u, y);
+    x.f.end(c, nch);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      u[r] = lg * 4 + r >= bad ? __builtin_nanf("") : u[r] * x.f.u[r];
+      if (lg * 4 + r >= bad) y[r] = __builtin_nanf("");
+    }
+    const float gc = x.f.gc;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int t = c * DC_TOK + lg * 4 + r;
+      if (t < n) out[(int64_t)t * heads * vp] = y[r];
+    }
+    fetch(x, c + 2);
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) {
+      if constexpr (CH) S[t] *= *reinterpret_cast<const float4_t*>(&L.gc[CH ? b : 0][CH ? t * 16 + lg * 4 : 0]);
+      else S[t] *= gc;
+      S[t] = mfma4(L.key_column(b, lg, t * 16 + lm), u, S[t]);
+    }
+    lds_barrier();
+  };
+  fetch(ahead[0], 0);
+  fetch(ahead[1], 1);
+  lds_barrier();
+  for (int c = 0; c < nch; c += 2) {
+    chunk(ahead[0], c);
+    chunk(ahead[1], c + 1);
+  }
+#pragma unroll
+  for (int t = 0; t < TILES; ++t) *reinterpret_cast<float4_t*>(st + t * 16) = S[t];
+}
+
+template <typename T, int DP, bool CH>
+int run_chunks(const msa_delta_args& a, const msa_batch* b, hipStream_t s) {
+  const unsigned chunks = (unsigned)((b->max_count + DC_TOK - 1) / DC_TOK);
+  hipLaunchKernelGGL((delta_prepare_kernel<T, DP, CH>), dim3(chunks, (a.heads + 3) / 4, b->nseg), dim3(256), 0,
+                     s, (const T*)a.qkv, a.ld, a.ba, a.ldba, a.decay_rate, a.dt_bias, a.decay, a.heads,
+                     a.kv_heads, (float)pow((double)a.dim, -0.5), a.scratch, b->seg_start, b->seg_pos);
+#define DC_RUN(KERNEL, COLS, THREADS, BYTES)                                                           \
+  do {                                                                                                 \
+    static std::atomic<uint64_t> raised{0};                                                            \
+    if (!raise_lds((const void*)KERNEL, BYTES, raised)) {                                              \
+      msa_set_error("msa_delta_scan: %d bytes of LDS refused", BYTES);                                 \
+      return MSA_ERR_HIP;                                                                              \
+    }                                                                                                  \
+    hipLaunchKernelGGL(KERNEL, dim3(a.vp / (COLS), a.heads, b->nseg), dim3(THREADS), BYTES, s,         \
+                       (const T*)a.qkv, a.ld, a.decay, a.heads, a.kv_heads, a.vp, a.state, a.scratch,  \
+                       a.o, b->seg_start, b->seg_slot, b->seg_pos);                                    \
+  } while (0)
+  const int64_t units = (int64_t)b->nseg * a.heads;
+  if (a.vp % 128 == 0 && units >= DC_WIDE) {
+    DC_RUN((delta_chunk_wide_kernel<T, DP, CH, 8>), 128, 768, (int)sizeof(Operands<DP, CH>));
+  } else if (a.vp % 64 == 0 && units * (a.vp / 64) >= DC_WIDE) {
+    DC_RUN((delta_chunk_wide_kernel<T, DP, CH, 4>), 64, 512, (int)sizeof(Operands<DP, CH>));
+  } else {
+    DC_RUN((delta_chunk_kernel<T, DP, CH>), 16, 512, (int)sizeof(FewLds<DP, CH>));
+  }
+#undef DC_RUN
+  return MSA_OK;
+}
+
+template <typename T>
+int pick_chunks(const msa_delta_args& a, const msa_batch* b, hipStream_t s) {
+#define DC_CASE(DP) \
+  case DP:          \
+    return a.decay ? run_chunks<T, DP, true>(a, b, s) : run_chunks<T, DP, false>(a, b, s);
+  switch (a.dp) {
+    DC_CASE(32)
+    DC_CASE(64)
+    DC_CASE(96)
+    DC_CASE(128)
+  }
+#undef DC_CASE
+  return MSA_ERR_INVALID_ARG;  // not reached: msa_delta_scratch_floats is 0 for other sizes
+}
+
+}  // namespace
+
+// The scan stays faster for few short segments (both kernels cost some 15 us before the first token; one segment of
+// 64 / 96 / 128 tokens: 21.0 / 23.4 / 25.6 us against 20.1 / 27.8 / 35.3, with decays per channel 24.3 /
+// 28.1 / 32.1 against 20.1 / 28.0 / 36.8); where the segments fill the chip the chunks win from the first length
+// tried (8 x 64 tokens 37 us against 62, seven segments of 20 and one of 64 35 against 40).
+constexpr int DC_FROM = 96, DC_FROM_WIDE = 48;
+
+extern "C" int64_t msa_delta_scratch_floats(const msa_delta_args* a, const msa_batch* b) {
+  if (!a || !b || a->heads <= 0 || a->dp > 128) return 0;
+  if (b->max_count < ((int64_t)b->nseg * a->heads >= DC_WIDE ? DC_FROM_WIDE : DC_FROM)) return 0;
+  return ((int64_t)b->M / DC_TOK + b->nseg) * a->heads * DC_REC;
+}
+
+int msa_launch_delta_chunks(const msa_delta_args& a, const msa_batch* b, hipStream_t s) {
+  return a.dtype == MSA_BF16 ? pick_chunks<bf16_t>(a, b, s) : pick_chunks<float>(a, b, s);
+}

@@ -286,15 +286,17 @@ int Run::delta_core(const msa_hybrid_layer& l, const msa_hybrid_state& st, char*
   void* qkv = alloc((int64_t)M * C * es);
   const bool step = b.max_count == 1;
   t.o = step ? nullptr : (float*)alloc((int64_t)M * l.heads * l.vp * 4);
+  t.heads = l.heads;
+  t.dp = l.dp;
+  t.scratch_floats = step ? 0 : msa_delta_scratch_floats(&t, &b);
+  if (t.scratch_floats > 0) t.scratch = (float*)alloc(t.scratch_floats * 4);
   if (!dry) {
     HY(msa_short_conv(d->cfg.dtype, in, ld, C, l.taps, nullptr, l.conv_w, nullptr, 1, qkv, C, st.conv, &b,
                       stream));
     HY(msa_conv_state(d->cfg.dtype, in, ld, C, l.taps, st.conv, &b, stream));
     t.dtype = d->cfg.dtype;
-    t.heads = l.heads;
     t.kv_heads = l.kv_heads;
     t.dim = l.dim;
-    t.dp = l.dp;
     t.vdim = l.vdim;
     t.vp = l.vp;
     t.qkv = qkv;

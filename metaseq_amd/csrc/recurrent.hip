@@ -701,7 +701,14 @@ extern "C" int msa_delta_scan(const msa_delta_args* a, const msa_batch* b, void*
   int rc = check_delta(name, a, b);
   if (rc) return rc;
   MSA_REQUIRE(a->o, MSA_ERR_INVALID_ARG, "%s: null pointer", name);
-  if (a->dtype == MSA_BF16)
+  const int64_t scratch = a->scratch ? msa_delta_scratch_floats(a, b) : 0;
+  MSA_REQUIRE(scratch == 0 || a->scratch_floats >= scratch, MSA_ERR_CAPACITY,
+              "%s: scratch of %lld floats, %lld needed", name, (long long)a->scratch_floats,
+              (long long)scratch);
+  if (scratch > 0) {
+    rc = msa_launch_delta_chunks(*a, b, (hipStream_t)stream);
+    if (rc) return rc;
+  } else if (a->dtype == MSA_BF16)
     dispatch_delta<bf16_t>(*a, b, false, (hipStream_t)stream);
   else
     dispatch_delta<float>(*a, b, false, (hipStream_t)stream);
