@@ -1065,7 +1065,7 @@ __global__ __launch_bounds__(TB_THREADS) void linear_tiled_big_kernel(
 // 256-byte row pieces per 16 lanes.
 // Workgroup -> tile: consecutive workgroups land on consecutive XCDs; where the default order would
 // give an XCD a long thin strip of a round's tiles, the 256 tiles of a round are regrouped so that
-// every XCD's L2 serves a compact a x b block (rm_a, rm_b, rm_r from the host).
+// every XCD's L2 serves a compact a x b block (rm_a, rm_b, rm_r from the host; rm_a < 0: by panels).
 // Three widths of the workgroup's tile, by the number WF of 16-feature weight fragments per wave:
 // 8 -> 256 x 256 (as described), 4 -> 256 x 128, 2 -> 256 x 64 (fewer accumulators, weight loads and
 // MFMAs per step; the same activation stages).  The two wider forms need M >= 256: a ragged last
@@ -1073,6 +1073,7 @@ __global__ __launch_bounds__(TB_THREADS) void linear_tiled_big_kernel(
 // form repeats the last row in its loads instead and drops the rows past it, so it also serves
 // fewer than 256 rows.  All need K % 64 == 0, K >= 128.
 constexpr int TQ_BM = 256, TQ_THREADS = 256;
+constexpr int TQ_PANEL = 16;  // columns of tiles taken together where many lie across
 constexpr int TQ_RX = 3, TQ_RW = 4;
 constexpr int TQ_XBYTES = TQ_BM * 64 * 2;       // one 64-wide stage of activations
 constexpr int TQ_WOFF = TQ_RX * TQ_XBYTES;
@@ -1186,6 +1187,20 @@ __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
     g_first = gt.tile_row[by];
     M = min((int64_t)gt.group_end[g], g_first + TQ_BM);
     Wp = (const char*)Wp + (int64_t)g * N * K * 2;
+  } else if (rm_a < 0) {
+    // panels of 16 columns, one after the other over all rows: 16 x 16 tiles of a panel at a time as eight
+    // 4 x 8 blocks, one per XCD, the panel's last rows and a narrower last panel row by row
+    const int ncol = gridDim.x, nrow = gridDim.y, L = by * ncol + bx;
+    const int p = L / (TQ_PANEL * nrow), w = min(TQ_PANEL, ncol - p * TQ_PANEL), idx = L - p * TQ_PANEL * nrow;
+    const int i = idx & 255, round = idx >> 8;
+    if (w == TQ_PANEL && (round + 1) * 16 <= nrow) {
+      const int xcd = i & 7, k = i >> 3;
+      bx = p * TQ_PANEL + (xcd & 3) * 4 + (k & 3);
+      by = round * 16 + (xcd >> 2) * 8 + (k >> 2);
+    } else {
+      bx = p * TQ_PANEL + idx % w;
+      by = idx / w;
+    }
   } else if (rm_a > 0) {
     const int ncol = gridDim.x, L = by * ncol + bx, round = L >> 8, i = L & 255;
     if ((round + 1) * rm_r <= (int)gridDim.y) {  // a full round of 256 tiles
@@ -1733,6 +1748,13 @@ void launch_stream(const void* xp, const void* W, const void* scales, float* par
   }
 }
 
+// Row by row, a round of 256 tiles over more than 64 columns leaves each XCD a strip of at least eight columns
+// and a row or two, whose weights come from beyond its L2 (197 columns, the vocabulary: 25 strips of
+// weights and 2 of activations per XCD and round, 4.3 TB/s; in panels 4 and 8).  Measured, 32800 x
+// 50272 x 4096 12.3 -> 10.7 ms, 6038 rows with fp32 results 2372 -> 1963 us, 2005 rows 807 -> 685, 1500
+// rows 600 -> 502; 6038 x 21888 x 4096 (86 columns) 960 -> 918; 48 and 64 columns are the same either way.
+bool wide_panels(int ncol) { return ncol > 64; }
+
 // One launch of the four-wave kernel (WF = 8: 256 x 256 tiles, WF = 4: 256 x 128) on rows
 // 0 .. M_main - 1 (a ragged last row tile is moved up) plus the streaming kernel on the rows from
 // M_main on (at most 128).
@@ -1755,6 +1777,7 @@ void launch_quad(const void* x, const void* W, const void* scales, int64_t M, in
       if (a + b < best) best = a + b, rm_a = a, rm_b = b, rm_r = r;
     }
   }
+  if (wide_panels(ncol)) rm_a = -TQ_PANEL;
   hipLaunchKernelGGL((linear_quad_kernel<MODE, WF>), dim3(ncol, nrow), dim3(TQ_THREADS),
                      tq_lds_bytes(WF), s, (const half_t*)x, W, M_main, N, K, rm_a, rm_b, rm_r, epi,
                      (float*)nullptr, 0);
@@ -1775,8 +1798,9 @@ void launch_quad_partial_w(const void* x, const void* W, float* part, int64_t M,
   const int ncol = (N + tq_bn(WF) - 1) / tq_bn(WF);
   const int nrow = (int)((M + TQ_BM - 1) / TQ_BM);
   Epilogue e{};
+  const int rm_a = wide_panels(ncol) ? -TQ_PANEL : 0;
   hipLaunchKernelGGL(kernel, dim3(ncol, nrow, S), dim3(TQ_THREADS), tq_lds_bytes(WF), s,
-                     (const half_t*)x, W, M, N, K, 0, 0, 0, e, part, K / 64 / S, GroupTiles{});
+                     (const half_t*)x, W, M, N, K, rm_a, 0, 0, e, part, K / 64 / S, GroupTiles{});
 }
 
 // 256 x 64 tiles while their S slices fit the chip in one round; an S beyond that means 256 x 128

@@ -93,6 +93,20 @@ def test_linear_bf16(M, N, K):
         close(part.sum(0), ref, 1e-5, "partial sums, S=%d" % S)
 
 
+@pytest.mark.parametrize("M,N", [(4352, 16656), (600, 24576)])
+def test_linear_partial_bf16_wide_panels(M, N):
+    """More than 64 columns of tiles, taken in panels of 16; sums of one and two slices."""
+    lib, K = _capi.load_hybrid(), 256
+    g = torch.Generator("cuda").manual_seed(M)
+    x = torch.randn(M, K, generator=g, device="cuda").to(BF16)
+    w = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).to(BF16)
+    wp, ref = pack_tiles(w), x.float() @ w.float().t()
+    for S in (1, 2):
+        part = torch.full((S, M, N), float("nan"), device="cuda")
+        check(lib.msa_linear_partial_bf16(ptr(x), ptr(wp), ptr(part), M, N, K, S, 0, _capi.stream_ptr()), lib)
+        close(part.sum(0).cpu(), ref.cpu(), 1e-5, "partial sums, S=%d" % S)
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 16, 32), (70, 80, 96), (200, 144, 128)])
 def test_linear_f32(M, N, K):
     lib = _capi.load_hybrid()

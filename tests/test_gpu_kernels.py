@@ -442,6 +442,22 @@ def test_linear_f16(lib, M, N, K, epi):
             assert torch.equal(unpack_act(y3.cpu(), M, N), y2.cpu())
 
 
+# more than 64 columns of tiles, which are taken in panels of 16: full and partial 16 x 16 blocks, a last
+# panel of one column and of several, a ragged bottom and right edge
+@pytest.mark.parametrize("M,N", [(4096, 16640), (8400, 16400), (700, 20500 // 16 * 16), (4500, 20480), (256, 24592)])
+def test_linear_f16_wide_panels(lib, M, N):
+    K = 128
+    print("panels", M, N, flush=True)
+    x, W = G(rnd(M, K, seed=M)), G(rnd(N, K, seed=N, std=0.05))
+    y = torch.full((M, N), float("nan"), dtype=torch.float16, device=DEV)
+    ok(lib.msa_linear_f16(P(x), P(pack_w(lib, W)), None, None, P(y), M, N, K, 0, None), lib)
+    torch.cuda.synchronize()
+    want = x.float() @ W.float().t()
+    # one rounding to fp16 of a K-term fp32 sum
+    bound = want.abs() * 2.0 ** -11 + 8 * 2.0 ** -24 * K ** 0.5 * float(want.square().mean().sqrt())
+    assert bool(((y.float() - want).abs() <= bound).all())
+
+
 def test_linear_in_place_residual(lib):
     for M, flags in ((32, IN_PACKED), (200, 0)):
         N, K = 768, 3072
