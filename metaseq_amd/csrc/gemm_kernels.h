@@ -1071,16 +1071,18 @@ __global__ __launch_bounds__(TB_THREADS) void linear_tiled_big_kernel(
 // MFMAs per step; the same activation stages).  The two wider forms need M >= 256: a ragged last
 // row tile is moved up to end at M and stores only the rows no other tile owns.  The narrowest
 // form repeats the last row in its loads instead and drops the rows past it, so it also serves
-// fewer than 256 rows.  All need K % 64 == 0, K >= 128.
-constexpr int TQ_BM = 256, TQ_THREADS = 256;
+// fewer than 256 rows, as does any form with FEW.  RF = 4 (16-row activation fragments per wave; else 8): tiles
+// of 128 rows, whose rings are five stages and eight steps deep.  All need K % 64 == 0, K >= 128.
+constexpr int TQ_BM = 256, TQ_THREADS = 256;  // (rows of a tile unless RF is given)
 constexpr int TQ_PANEL = 16;  // columns of tiles taken together where many lie across
-constexpr int TQ_RX = 3, TQ_RW = 4;
-constexpr int TQ_XBYTES = TQ_BM * 64 * 2;       // one 64-wide stage of activations
-constexpr int TQ_WOFF = TQ_RX * TQ_XBYTES;
+constexpr int tq_bm(int RF) { return 32 * RF; }
+constexpr int tq_rx(int RF) { return RF == 8 ? 3 : 5; }    // stages of activations in the ring
+constexpr int tq_rw(int RF) { return RF == 8 ? 4 : 8; }    // steps of weights
+constexpr int tq_xbytes(int RF) { return tq_bm(RF) * 64 * 2; }  // one 64-wide stage of activations
 constexpr int tq_bn(int WF) { return 32 * WF; }
 constexpr int tq_wbytes(int WF) { return 2 * WF * 1024; }  // one 32-wide step of weights
-constexpr int tq_lds_bytes(int WF) {  // 160 / 128 / 112 KB
-  return TQ_RX * TQ_XBYTES + TQ_RW * tq_wbytes(WF);
+constexpr int tq_lds_bytes(int WF, int RF = 8) {  // 160 / 128 / 112 KB; 144 KB with RF = 4
+  return tq_rx(RF) * tq_xbytes(RF) + tq_rw(RF) * tq_wbytes(WF);
 }
 typedef __attribute__((address_space(3))) void tq_lds_void;
 
@@ -1164,7 +1166,7 @@ struct GroupTiles {
 // PART: split-K.  Workgroup (bx, by, z) sums over the K range of ``part_stages`` 64-wide stages
 // that starts at stage z * part_stages and stores its fp32 sums, with no epilogue, as slice z of
 // ``part`` ([gridDim.z][M][N]); a later launch adds the slices in slice order.
-template <int MODE, int WF, bool PART = false, bool GROUPED = false>
+template <int MODE, int WF, bool PART = false, bool GROUPED = false, int RF = 8, bool FEW = false>
 __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
     const half_t* __restrict__ x, const void* __restrict__ Wp, int64_t M, int N, int K,
     int rm_a, int rm_b, int rm_r, Epilogue epi, float* __restrict__ part, int part_stages,
@@ -1173,8 +1175,10 @@ __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 15, lg = lane >> 4;
   const int wm = wave >> 1, wn = wave & 1;
-  constexpr int TQ_BN = tq_bn(WF), TQ_WBYTES = tq_wbytes(WF);
+  constexpr int TQ_BN = tq_bn(WF), TQ_WBYTES = tq_wbytes(WF), TQ_BM = tq_bm(RF), TQ_XBYTES = tq_xbytes(RF);
+  constexpr int TQ_RX = tq_rx(RF), TQ_RW = tq_rw(RF), TQ_WOFF = TQ_RX * TQ_XBYTES;
   constexpr int WL = WF / 2;  // weight load instructions per wave and step
+  constexpr int XL = RF;      // activation load instructions per wave and stage
   int bx = blockIdx.x, by = blockIdx.y;
   int64_t g_first = 0;
   if constexpr (GROUPED) {
@@ -1212,7 +1216,7 @@ __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
   // The narrowest form (WF = 2) also serves fewer than 256 rows: it does not move a ragged tile up
   // but repeats the last row in its loads and drops the rows past it in the epilogue.  So does
   // the split-K form of WF = 4 (decode batches of 129 .. 255 rows cut K eight ways over it).
-  constexpr bool CLAMP = WF == 2 || (WF == 4 && PART) || GROUPED;
+  constexpr bool CLAMP = WF == 2 || (WF == 4 && PART) || GROUPED || RF == 4 || FEW;
   const int64_t m_own = GROUPED ? g_first : (int64_t)by * TQ_BM;  // first row this tile owns
   const int64_t m0 = !CLAMP && m_own + TQ_BM > M ? M - TQ_BM : m_own;
   const int n0 = bx * TQ_BN;
@@ -1227,13 +1231,13 @@ __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
   // (l % 8) ^ ((row / 2) % 8) = (l % 8) ^ (4 * (i % 2) + l / 16)), with M0 at the wave's piece
   // + 4 KB and instruction offset 1024 * (i - 4).  Weights, per step: the wave copies the blocks
   // of tiles 4 * wave .. 4 * wave + 3, instruction offset 1024 * j.
-  const char* xb[8];
+  const char* xb[XL];
   const char* wb[WL];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int64_t r = m0 + wave * 64 + i * 8;
+  for (int i = 0; i < XL; ++i) {
+    const int64_t r = m0 + wave * (TQ_BM / 4) + i * 8;
     const int64_t base_row = GROUPED ? 0 : CLAMP ? min(r, M - 1) : r;
-    xb[i] = (const char*)(x + base_row * K + (int64_t)st_first * 64) - (i - 4) * 1024;
+    xb[i] = (const char*)(x + base_row * K + (int64_t)st_first * 64) - (i - XL / 2) * 1024;
   }
 #pragma unroll
   for (int j = 0; j < WL; ++j) {
@@ -1245,11 +1249,11 @@ __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
   const uint32_t xlane1 = xrow + (((lane & 7) ^ (4 + (lane >> 4))) * 16);
   const uint32_t wlane = lane * 16;
   // CLAMP: per instruction, the lane's row offset from the (clamped) scalar base row
-  uint32_t xl[CLAMP ? 8 : 1];
+  uint32_t xl[CLAMP ? XL : 1];
   if (CLAMP) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int64_t r = m0 + wave * 64 + i * 8;
+    for (int i = 0; i < XL; ++i) {
+      const int64_t r = m0 + wave * (TQ_BM / 4) + i * 8;
       int64_t d = min(r + (lane >> 3), M - 1);
       if (GROUPED) {
         if (gt.perm) d = gt.perm[d] / gt.rows_per_x;
@@ -1270,7 +1274,7 @@ __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
     xst = st * 128;
     xv0 = xlane0 + st * 128;
     xv1 = xlane1 + st * 128;
-    xm0 = lds0 + slot * TQ_XBYTES + wave * (64 * 128) + 4096;
+    xm0 = lds0 + slot * TQ_XBYTES + wave * (TQ_BM / 4 * 128) + XL / 2 * 1024;
   };
   auto set_w = [&](int slot, int ks) {
     ks = min(ks, nks - 1);
@@ -1283,7 +1287,7 @@ __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
     const char* sb = xb[i];
     const uint32_t base = xm0;
     asm volatile("global_load_lds_dwordx4 %0, %1 offset:%2" ::"v"(vo), "s"(sb),
-                 "n"((i - 4) * 1024), "{m0}"(base)
+                 "n"((i - XL / 2) * 1024), "{m0}"(base)
                  : "memory");
   };
   auto issue_w = [&](auto jc) {
@@ -1297,7 +1301,7 @@ __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
   };
   auto group_x = [&](int slot, int st) {
     set_x(slot, st);
-    tq_static_for<8>([&](auto ic) { issue_x(ic); });
+    tq_static_for<XL>([&](auto ic) { issue_x(ic); });
   };
   auto group_w = [&](int slot, int ks) {
     set_w(slot, ks);
@@ -1307,8 +1311,8 @@ __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
   // fragment reads.  Activation fragment i of half h of a stage: row 128 * wm + 16 * i + lr, chunk
   // 4 * h + lg at position (4 * h + lg) ^ ((lr / 2) % 8); weight fragment j: tile 8 * wn + j.
   const int sw = (lr >> 1) & 7;
-  const uint32_t xoff0 = (uint32_t)(wm * 128 + lr) * 128 + ((lg ^ sw) * 16);
-  const uint32_t xoff1 = (uint32_t)(wm * 128 + lr) * 128 + ((lg ^ sw ^ 4) * 16);
+  const uint32_t xoff0 = (uint32_t)(wm * (TQ_BM / 2) + lr) * 128 + ((lg ^ sw) * 16);
+  const uint32_t xoff1 = (uint32_t)(wm * (TQ_BM / 2) + lr) * 128 + ((lg ^ sw ^ 4) * 16);
   const uint32_t woff = TQ_WOFF + (uint32_t)(wn * WF) * 1024 + lane * 16;
   auto xfrag = [&](int slot, int h, int i) {
     return *reinterpret_cast<const half8_t*>(tq_lds + slot * TQ_XBYTES + (h ? xoff1 : xoff0) +
@@ -1318,9 +1322,9 @@ __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
     return *reinterpret_cast<const half8_t*>(tq_lds + slot * TQ_WBYTES + woff + j * 1024);
   };
 
-  float4_t acc[8][WF];
+  float4_t acc[RF][WF];
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < RF; ++i)
 #pragma unroll
     for (int j = 0; j < WF; ++j) {
       acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
@@ -1329,17 +1333,26 @@ __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
 
   // prologue: activation stages 0 and 1, weight steps 0..3 requested; stages 0, 1 and steps 0, 1
   // landed
-  half8_t xf[2][8], wf[2][WF];
-  group_x(0, 0);
-  group_w(0, 0);
-  group_x(1, 1);
-  group_w(1, 1);
-  group_w(2, 2);
-  group_w(3, 3);
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * WL) : "memory");
+  half8_t xf[2][RF], wf[2][WF];
+  if constexpr (RF == 8) {
+    group_x(0, 0);
+    group_w(0, 0);
+    group_x(1, 1);
+    group_w(1, 1);
+    group_w(2, 2);
+    group_w(3, 3);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * WL) : "memory");
+  } else {  // as the steps -TQ_RW .. -1 would have requested them; stage 0 and step 0 landed
+#pragma unroll
+    for (int v = 0; v < TQ_RW; ++v) {
+      if (v % 2 == 0) group_x(v / 2, v / 2);
+      group_w(v, v);
+    }
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(TQ_RW / 2 * XL + TQ_RW * WL - XL - WL) : "memory");
+  }
   __syncthreads();
 #pragma unroll
-  for (int i = 0; i < 8; ++i) xf[0][i] = xfrag(0, 0, i);
+  for (int i = 0; i < RF; ++i) xf[0][i] = xfrag(0, 0, i);
 #pragma unroll
   for (int j = 0; j < WF; ++j) wf[0][j] = wfrag(0, j);
 
@@ -1352,47 +1365,58 @@ __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
   // loads (even steps: activations under rows 0..3, weights under rows 4..7).
   auto step = [&](int t, int xs, int ws, auto hc) {
     constexpr int H = decltype(hc)::value;
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(8 + 2 * WL) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((TQ_RW - 2) / 2 * XL + (TQ_RW - 2) * WL) : "memory");
     __syncthreads();
     const int S = t >> 1;
-    const int xfree = xs == 0 ? TQ_RX - 1 : xs - 1;  // slot of stage S - 1 = slot of stage S + 2
+    const int xfree = xs == 0 ? TQ_RX - 1 : xs - 1;  // slot of stage S - 1 = slot of stage S + TQ_RX - 1
     const int xnext = xs == TQ_RX - 1 ? 0 : xs + 1;  // slot of stage S + 1
     const int wnext = ws == TQ_RW - 1 ? 0 : ws + 1;  // slot of step t + 1
-    tq_static_for<8>([&](auto ic) {
+    tq_static_for<RF>([&](auto ic) {
       constexpr int i = decltype(ic)::value;
       tq_static_for<WF>([&](auto jc) {
         constexpr int j = decltype(jc)::value;
         tq_mfma<MODE>(acc[i][j], wf[H][j], xf[H][i]);
-        if (j == 1) xf[H ^ 1][i] = H == 0 ? xfrag(xs, 1, i) : xfrag(xnext, 0, i);
-        if constexpr (WF == 8) {
-          if (j == 5) wf[H ^ 1][i % WF] = wfrag(wnext, i % WF);
-        } else if constexpr (WF == 4) {
-          if constexpr (j == 3 && (i & 1)) wf[H ^ 1][(i >> 1) % WF] = wfrag(wnext, (i >> 1) % WF);
-        } else {
-          if constexpr (j == 0 && (i == 1 || i == 5)) wf[H ^ 1][(i >> 2) % WF] = wfrag(wnext, (i >> 2) % WF);
-        }
-        if constexpr (H == 0) {
-          if (i == 0 && j == 0) set_x(xfree, S + 2);
-          if constexpr (i < 4 && j == WF / 2 - 1) issue_x(std::integral_constant<int, (i & 3) * 2>{});
-          if constexpr (i < 4 && j == WF - 1) issue_x(std::integral_constant<int, (i & 3) * 2 + 1>{});
-          if (i == 4 && j == 0) set_w(ws, t + TQ_RW);
-          if constexpr (WF == 8) {
-            if constexpr (i >= 4 && j == 3) issue_w(std::integral_constant<int, (i & 3) % WL>{});
-          } else if constexpr (WF == 4) {
-            if constexpr ((i == 4 || i == 6) && j == 2)
-              issue_w(std::integral_constant<int, ((i >> 1) & 1) % WL>{});
-          } else {
-            if constexpr (i == 4 && j == 1) issue_w(std::integral_constant<int, 0>{});
+        if constexpr (RF == 4) {
+          if (j == 1) xf[H ^ 1][i] = H == 0 ? xfrag(xs, 1, i) : xfrag(xnext, 0, i);
+          if (j == 3) wf[H ^ 1][i] = wfrag(wnext, i);
+          if constexpr (H == 0) {
+            if (i == 0 && j == 0) set_x(xfree, S + TQ_RX - 1);
+            if (j == 0) issue_x(ic);
           }
+          if (i == 0 && j == 1) set_w(ws, t + TQ_RW);
+          if constexpr (j == 2 && (i & 1)) issue_w(std::integral_constant<int, (i >> 1)>{});
         } else {
-          if (i == 0 && j == 0) set_w(ws, t + TQ_RW);
+          if (j == 1) xf[H ^ 1][i] = H == 0 ? xfrag(xs, 1, i) : xfrag(xnext, 0, i);
           if constexpr (WF == 8) {
-            if constexpr (j == 3 && (i & 1)) issue_w(std::integral_constant<int, (i >> 1) % WL>{});
+            if (j == 5) wf[H ^ 1][i % WF] = wfrag(wnext, i % WF);
           } else if constexpr (WF == 4) {
-            if constexpr ((i == 2 || i == 6) && j == 2)
-              issue_w(std::integral_constant<int, ((i >> 2) & 1) % WL>{});
+            if constexpr (j == 3 && (i & 1)) wf[H ^ 1][(i >> 1) % WF] = wfrag(wnext, (i >> 1) % WF);
           } else {
-            if constexpr (i == 2 && j == 1) issue_w(std::integral_constant<int, 0>{});
+            if constexpr (j == 0 && (i == 1 || i == 5)) wf[H ^ 1][(i >> 2) % WF] = wfrag(wnext, (i >> 2) % WF);
+          }
+          if constexpr (H == 0) {
+            if (i == 0 && j == 0) set_x(xfree, S + 2);
+            if constexpr (i < 4 && j == WF / 2 - 1) issue_x(std::integral_constant<int, (i & 3) * 2>{});
+            if constexpr (i < 4 && j == WF - 1) issue_x(std::integral_constant<int, (i & 3) * 2 + 1>{});
+            if (i == 4 && j == 0) set_w(ws, t + TQ_RW);
+            if constexpr (WF == 8) {
+              if constexpr (i >= 4 && j == 3) issue_w(std::integral_constant<int, (i & 3) % WL>{});
+            } else if constexpr (WF == 4) {
+              if constexpr ((i == 4 || i == 6) && j == 2)
+                issue_w(std::integral_constant<int, ((i >> 1) & 1) % WL>{});
+            } else {
+              if constexpr (i == 4 && j == 1) issue_w(std::integral_constant<int, 0>{});
+            }
+          } else {
+            if (i == 0 && j == 0) set_w(ws, t + TQ_RW);
+            if constexpr (WF == 8) {
+              if constexpr (j == 3 && (i & 1)) issue_w(std::integral_constant<int, (i >> 1) % WL>{});
+            } else if constexpr (WF == 4) {
+              if constexpr ((i == 2 || i == 6) && j == 2)
+                issue_w(std::integral_constant<int, ((i >> 2) & 1) % WL>{});
+            } else {
+              if constexpr (i == 2 && j == 1) issue_w(std::integral_constant<int, 0>{});
+            }
           }
         }
       });
@@ -1412,7 +1436,7 @@ __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
   asm volatile("s_waitcnt vmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");
   // ties every accumulator to this point: none of their reads may be scheduled above the wait
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < RF; ++i)
 #pragma unroll
     for (int j = 0; j < WF; ++j) asm volatile("" : "+a"(acc[i][j]));
   __syncthreads();  // every wave is done with the operand rings
@@ -1422,8 +1446,8 @@ __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
     // 128, features 16 * j + 4 * lg .. + 3 of the wave's 16 WF (16 bytes per lane, 64 per row)
     float* slice = part + (int64_t)blockIdx.z * M * N;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int64_t m = m0 + wm * 128 + i * 16 + lr;
+    for (int i = 0; i < RF; ++i) {
+      const int64_t m = m0 + wm * (TQ_BM / 2) + i * 16 + lr;
 #pragma unroll
       for (int j = 0; j < WF; ++j) {
         const int n = n0 + wn * (16 * WF) + 16 * j + 4 * lg;
@@ -1454,9 +1478,9 @@ __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
       for (int j = 0; j < WF; ++j) post[j] = post_vectors(epi, min(nw + 16 * j, N - 16) + 4 * lg);
     }
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < RF; ++i) {
       char* buf = stage + (i & 1) * 4096;
-      const int64_t mf = m0 + wm * 128 + i * 16 + lr;
+      const int64_t mf = m0 + wm * (TQ_BM / 2) + i * 16 + lr;
 #pragma unroll
       for (int j = 0; j < WF; ++j) {
         const int n = nw + 16 * j + 4 * lg;
@@ -1481,7 +1505,7 @@ __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
         if (row >= 16) continue;
         const half8_t v = *reinterpret_cast<const half8_t*>(buf + row * BRB +
                                                             ((bc ^ (row & (BCH - 1))) * 16));
-        const int64_t m = m0 + wm * 128 + i * 16 + row;
+        const int64_t m = m0 + wm * (TQ_BM / 2) + i * 16 + row;
         bf16_t* y = epi.yb + m * epi.ldy + bn;
         if constexpr (MODE == MODE_BF_POST)
           if (bn >= epi.n2) y = epi.y2 + m * epi.ld2 + (bn - epi.n2);
@@ -1514,7 +1538,7 @@ __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
     if (MODE != MODE_PLAIN || !epi.residual) return;
 #pragma unroll
     for (int r = 0; r < ENR; ++r) {
-      const int64_t m = m0 + wm * 128 + i * 16 + ERPI * r + erow;
+      const int64_t m = m0 + wm * (TQ_BM / 2) + i * 16 + ERPI * r + erow;
       if (col_ok && m >= m_own && m < M)
         dst[r] = *reinterpret_cast<const half8_t*>(epi.residual + m * epi.N + en);
     }
@@ -1525,12 +1549,12 @@ __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
   // previous row's without a division
   int qb = 0, qt = 0;
   if (MODE == MODE_QKV) {
-    const int mf = (int)(m0 + wm * 128 + erow);
+    const int mf = (int)(m0 + wm * (TQ_BM / 2) + erow);
     qb = epi.T == 1 ? mf : mf / epi.T;
     qt = mf - qb * epi.T;
   }
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
+  for (int i = 0; i < RF; ++i) {
     char* buf = mine + (i & 1) * 4096;
 #pragma unroll
     for (int j = 0; j < WF; ++j) {
@@ -1545,7 +1569,7 @@ __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
       const int row = ERPI * r + erow;
       const half8_t v = *reinterpret_cast<const half8_t*>(buf + row * ERB +
                                                           ((ec ^ (row & (ECH - 1))) * 16));
-      const int64_t m = m0 + wm * 128 + i * 16 + row;
+      const int64_t m = m0 + wm * (TQ_BM / 2) + i * 16 + row;
       if (col_ok && m >= m_own && m < M)
         epilogue8<MODE>(epi, m, en, v, bias8, res8[i % TQ_RES_AHEAD][r], qb, qt);
       if (MODE == MODE_QKV) {
@@ -1553,7 +1577,7 @@ __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
         while (qt >= epi.T) qt -= epi.T, ++qb;
       }
     }
-    if (i + TQ_RES_AHEAD < 8) load_res(i + TQ_RES_AHEAD, res8[i % TQ_RES_AHEAD]);
+    if (i + TQ_RES_AHEAD < RF) load_res(i + TQ_RES_AHEAD, res8[i % TQ_RES_AHEAD]);
   }
 }
 
@@ -1786,6 +1810,23 @@ void launch_quad(const void* x, const void* W, const void* scales, int64_t M, in
                                      K, epi, s, m0);
 }
 
+// One round of tiles over fewer rows than a 256-row tile holds, or a little more than one of 128.
+//   RF = 4: 128 x 128 tiles, two rows of them side by side on one XCD.  Of 129 .. 256 rows a CU then reads half as
+//   many activations as with the 256 x 64 form, its weights once more from L2: 200 x 12288 x 4096 44.3 ->
+//   39.5 us, 200 x 16384 x 4096 48.4 -> 46.8, 129 x 8192 x 2048 22.5 -> 19.3.  (As split-K sums they
+//   gained nothing: 200 x 4096 x 16384 49.8 -> 53.5.)
+//   RF = 8: 256 x 256 tiles that repeat the last row, for outputs wide enough that one row of them fills
+//   the chip (the vocabulary): 200 x 50272 x 4096 171 -> 115 us.
+template <int MODE, int WF, int RF>
+void launch_few_rows(const void* x, const void* W, int64_t M, int N, int K, const Epilogue& epi, hipStream_t s) {
+  static std::atomic<uint64_t> lds_allowed_s{0};
+  auto kernel = linear_quad_kernel<MODE, WF, false, false, RF, true>;
+  if (!allow_lds((const void*)kernel, tq_lds_bytes(WF, RF), lds_allowed_s)) return;
+  const int ncol = (N + tq_bn(WF) - 1) / tq_bn(WF), nrow = (int)((M + tq_bm(RF) - 1) / tq_bm(RF));
+  hipLaunchKernelGGL(kernel, dim3(ncol, nrow), dim3(TQ_THREADS), tq_lds_bytes(WF, RF), s, (const half_t*)x, W, M,
+                     N, K, -TQ_PANEL, 0, 0, epi, (float*)nullptr, 0, GroupTiles{});
+}
+
 // Split-K launch of a narrow four-wave form (WF = 2: 256 x 64 tiles, WF = 4: 256 x 128) on
 // row-major activations: S slices of K, each a whole number of 64-wide stages (at least two),
 // fp32 sums into part[S][M][N].
@@ -1858,7 +1899,9 @@ void launch_tiled(const void* x, const void* W, const void* scales, int64_t M, i
   // the 256 x 256 kernel once it fills the chip; the 128 x 128 one for the shapes in between
   const int64_t big_tiles = ((M + TB_BM - 1) / TB_BM) * ((N + TB_BN - 1) / TB_BN);
   if constexpr (!W8) {
-    // Three tile widths, 256, 128 and 64 features (a workgroup of 128 does half the MFMAs of 256 in
+    // Fewer rows than a tile, or hardly more: launch_few_rows where its tiles fill one round (three quarters of
+    // the CUs with 256 x 256, a quarter with 128 x 128 tiles).  Else
+    // three tile widths, 256, 128 and 64 features (a workgroup of 128 does half the MFMAs of 256 in
     // about 0.8 of the time, one of 64 a quarter in about 0.55), and two ways to take a ragged
     // bottom of at most 128 rows: as one more, moved-up row of tiles, or through the streaming
     // kernel (one sweep over the weights per 64 rows).  The combinations are priced in rounds of
@@ -1869,6 +1912,10 @@ void launch_tiled(const void* x, const void* W, const void* scales, int64_t M, i
     if (K % 64 == 0 && K >= 128 && M > 64) {
       const int64_t cus = num_cus(), rem = M % TQ_BM;
       const int64_t cols[3] = {(N + 255) / 256, (N + 127) / 128, (N + 63) / 64};
+      if (M < TQ_BM && cols[0] <= cus && cols[0] * 4 >= cus * 3)
+        return launch_few_rows<MODE, 8, 8>(x, W, M, N, K, epi, s);
+      if (M > 128 && M <= TQ_BM && cols[1] * 2 <= cus && cols[1] * 8 >= cus)
+        return launch_few_rows<MODE, 4, 4>(x, W, M, N, K, epi, s);
       const double factor[3] = {1.0, 0.8, 0.55};
       const double unit = 63.0 * K / 4096;  // us per round of wide tiles
       const double sweep = (double)N * K * 2 / 5e6 + 4;  // us per streaming launch

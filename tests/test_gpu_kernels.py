@@ -442,6 +442,37 @@ def test_linear_f16(lib, M, N, K, epi):
             assert torch.equal(unpack_act(y3.cpu(), M, N), y2.cpu())
 
 
+# 128 x 128 tiles (129 .. 256 rows; from a quarter of the chip to all of it, ragged edges, K of the ring's length
+# and less) and 256 x 256 tiles of fewer rows under a wide output
+@pytest.mark.parametrize("M,N,K", [(129, 4096, 128), (160, 4112, 192), (255, 12304, 320), (256, 16384, 640),
+                                   (200, 12288, 4096), (65, 50272, 128), (130, 50000, 192), (255, 49168, 576),
+                                   (250, 65536, 128)])
+@pytest.mark.parametrize("epi", ["plain", "bias_relu", "bias_res"])
+def test_linear_f16_few_rows(lib, M, N, K, epi):
+    print("few rows", M, N, K, epi, flush=True)
+    x, W = G(rnd(M, K, seed=M)), G(rnd(N, K, seed=N, std=0.05))
+    b = G(rnd(N, seed=9, std=0.1)) if epi != "plain" else None
+    res = G(rnd(M, N, seed=10)) if epi == "bias_res" else None
+    y = torch.full((M, N), float("nan"), dtype=torch.float16, device=DEV)
+    ok(lib.msa_linear_f16(P(x), P(pack_w(lib, W)), P(b), P(res), P(y), M, N, K, int(epi == "bias_relu"), None), lib)
+    torch.cuda.synchronize()
+    want = x.float() @ W.float().t()
+    # at the magnitude of the largest of the terms: an ulp (at most 2^-10 of it) for each rounding in front of the
+    # last, which two sums of other order may take to either side (with a residual two of them, the sum's and the
+    # bias's), half an ulp for the last, and the K-term sum itself
+    size = want.abs()
+    if b is not None:
+        want = want.half().float() + b.float()
+        size = torch.maximum(size, want.abs())
+    if epi == "bias_relu":
+        want = want.relu()
+    if res is not None:
+        want = want.half().float() + res.float()
+        size = torch.maximum(size, want.abs())
+    bound = 5 * size * 2.0 ** -11 + 8 * 2.0 ** -24 * K ** 0.5 * float(size.square().mean().sqrt()) + 2.0 ** -24
+    assert bool(((y.float() - want).abs() <= bound).all())
+
+
 # more than 64 columns of tiles, which are taken in panels of 16: full and partial 16 x 16 blocks, a last
 # panel of one column and of several, a ragged bottom and right edge
 @pytest.mark.parametrize("M,N", [(4096, 16640), (8400, 16400), (700, 20500 // 16 * 16), (4500, 20480), (256, 24592)])
