@@ -23,6 +23,23 @@ typedef float float16_t __attribute__((ext_vector_type(16)));
 
 void msa_set_error(const char* fmt, ...);
 
+// What a product of few rows can take in front of itself (gemm_kernels.h): x = round(round(round(sum of the S
+// slices) + bias) + x) and LayerNorm(x); the new x goes to x_out, which is not x.
+struct LnTail {
+  const float* part;  // [S][M][D]
+  const half_t *bias, *x;
+  half_t* x_out;
+  const half_t *gamma, *beta;
+  float eps;
+};
+// whether a product behind M rows of D in S slices takes their tail in front of itself
+bool msa_ln_folds(int M, int D, int S, bool int8);
+int msa_ln_qkv_proj(const LnTail& ln, int S, const void* W, const void* scales, const void* bias, void* q_out,
+                    void* Kc, void* Vc, int M, int H, int hd, int S0, int S_cap, int K, const int32_t* len_dev,
+                    hipStream_t stream);
+int msa_ln_linear_relu(const LnTail& ln, int S, const void* W, const void* scales, const void* bias, void* y_packed,
+                       int M, int N, int K, hipStream_t stream);
+
 // MFMA flash-style causal attention for T > 1 new queries (attention_prefill.hip)
 int msa_launch_prefill_attention(const void* q, const void* Kc, const void* Vc,
                                  const uint8_t* key_pad_mask, int64_t mask_stride, void* out,

@@ -25,9 +25,13 @@ namespace {
 
 int64_t align256(int64_t n) { return (n + 255) & ~(int64_t)255; }
 
+bool folds(const msa_decoder* d, int B, int S) {
+  return msa_ln_folds(B, d->cfg.d_model, S, d->cfg.int8 != 0);
+}
+
 // workspace layout for B rows
 struct StepBuffers {
-  char *x, *q, *h, *o, *u, *part, *positions, *step_len, *select_ws, *attn_ws, *logits;
+  char *x, *x2, *q, *h, *o, *u, *part, *positions, *step_len, *select_ws, *attn_ws, *logits;
   int64_t attn_keys;  // key positions per (b, h) that attn_ws holds scores for (0: none)
   int64_t bytes;
 };
@@ -67,6 +71,7 @@ StepBuffers carve(const msa_decoder* d, int B, const Splits& sp, char* base) {
     return p;
   };
   w.x = take(B * D * 2);
+  w.x2 = take(B * D * 2);  // (at any B: a workspace for more rows serves fewer)
   w.q = take(B * D * 2);
   w.h = take(MP * D * 2);
   w.o = take(MP * D * 2);
@@ -181,11 +186,29 @@ extern "C" int msa_decoder_step(msa_decoder* d, const msa_step_args* a, void* st
   const int keys_bound = a->len_dev && a->S0 == 0 ? a->S_cap : a->S0 + 1;
   const bool split_attention =
       a->S_cap <= w.attn_keys && msa_attention_prefers_split(B, H, hd, keys_bound);
+  // Of few rows the product behind out_proj and fc2 takes their tail in front of itself and writes the residual
+  // stream to the other of two buffers.
+  const bool fold_out = folds(d, B, sp.out), fold_fc2 = folds(d, B, sp.fc2);
+  char *x = w.x, *x_other = w.x2;
+  auto tail = [&](const void* bias, const void* gamma, const void* beta) {
+    return LnTail{(const float*)w.part, (const half_t*)bias, (const half_t*)x, (half_t*)x_other,
+                  (const half_t*)gamma, (const half_t*)beta, eps};
+  };
+  auto swap_x = [&] {
+    char* t = x;
+    x = x_other;
+    x_other = t;
+  };
   for (int i = 0; i < c.layers; ++i) {
     const msa_layer_weights& l = d->layers[i];
     void* kc = a->k_cache[i];
     void* vc = a->v_cache[i];
-    if (c.int8)
+    if (i > 0 && fold_fc2) {
+      rc = msa_ln_qkv_proj(tail(d->layers[i - 1].fc2_bias, l.ln1_gamma, l.ln1_beta), sp.fc2, l.qkv_weight,
+                           c.int8 ? l.qkv_scales : nullptr, l.qkv_bias, w.q, kc, vc, B, H, hd, a->S0, a->S_cap, D,
+                           len, (hipStream_t)stream);
+      swap_x();
+    } else if (c.int8)
       rc = msa_qkv_proj_w8a16(w.h, (const int8_t*)l.qkv_weight, l.qkv_scales, l.qkv_bias, w.q, kc,
                               vc, B, 1, H, hd, a->S0, a->S_cap, D, IN, len, stream);
     else
@@ -206,10 +229,16 @@ extern "C" int msa_decoder_step(msa_decoder* d, const msa_step_args* a, void* st
       rc = msa_linear_partial_f16(w.o, l.out_weight, (float*)w.part, B, D, D, sp.out, IN,
                                   stream);
     if (rc) return rc;
-    rc = msa_residual_layernorm_f16((const float*)w.part, sp.out, l.out_bias, w.x,
-                                    l.ln2_gamma, l.ln2_beta, w.h, B, D, eps, OUT, stream);
-    if (rc) return rc;
-    if (c.int8)
+    if (!fold_out) {
+      rc = msa_residual_layernorm_f16((const float*)w.part, sp.out, l.out_bias, x, l.ln2_gamma, l.ln2_beta, w.h, B,
+                                      D, eps, OUT, stream);
+      if (rc) return rc;
+    }
+    if (fold_out) {
+      rc = msa_ln_linear_relu(tail(l.out_bias, l.ln2_gamma, l.ln2_beta), sp.out, l.fc1_weight,
+                              c.int8 ? l.fc1_scales : nullptr, l.fc1_bias, w.u, B, F, D, (hipStream_t)stream);
+      swap_x();
+    } else if (c.int8)
       rc = msa_linear_w8a16(w.h, (const int8_t*)l.fc1_weight, l.fc1_scales, l.fc1_bias, nullptr,
                             w.u, B, F, D, MSA_EPI_RELU | IN | OUT, stream);
     else
@@ -224,7 +253,8 @@ extern "C" int msa_decoder_step(msa_decoder* d, const msa_step_args* a, void* st
                                   stream);
     if (rc) return rc;
     const bool last = i + 1 == c.layers;
-    rc = msa_residual_layernorm_f16((const float*)w.part, sp.fc2, l.fc2_bias, w.x,
+    if (fold_fc2 && !last) continue;
+    rc = msa_residual_layernorm_f16((const float*)w.part, sp.fc2, l.fc2_bias, x,
                                     last ? d->final_ln_gamma : d->layers[i + 1].ln1_gamma,
                                     last ? d->final_ln_beta : d->layers[i + 1].ln1_beta, w.h, B, D,
                                     eps, OUT, stream);

@@ -69,7 +69,7 @@ __global__ __launch_bounds__(256) void expand_w8_kernel(const uint8_t* __restric
 template <bool W8>
 int linear_entry(const char* name, const void* x, const void* W, const void* scales,
                  const void* bias, const void* residual, void* y, int64_t M, int N, int K,
-                 unsigned flags, void* stream) {
+                 unsigned flags, void* stream, const LnTail* ln = nullptr, int ln_slices = 0) {
   int rc = check_linear_args(name, x, W, y, M, N, K, W8, flags,
                              MSA_EPI_RELU | MSA_IN_PACKED | MSA_OUT_PACKED);
   if (rc) return rc;
@@ -84,7 +84,10 @@ int linear_entry(const char* name, const void* x, const void* W, const void* sca
   e.N = N;
   e.flags = flags & MSA_EPI_RELU;
   e.out_mb = (flags & MSA_OUT_PACKED) ? packed_row_blocks(M) : 0;
-  if (flags & MSA_IN_PACKED)
+  if (ln) {
+    MSA_REQUIRE((launch_stream_ln<W8, MODE_PLAIN>(*ln, ln_slices, W, scales, (int)M, N, K, e, (hipStream_t)stream)),
+                MSA_ERR_HIP, "%s: %d bytes of LDS refused", name, LN_MAX_K * 32);
+  } else if (flags & MSA_IN_PACKED)
     launch_stream<W8, MODE_PLAIN>(x, W, scales, nullptr, 1, (int)M, N, K, e, (hipStream_t)stream);
   else
     launch_tiled<W8, MODE_PLAIN>(x, W, scales, M, N, K, e, (hipStream_t)stream);
@@ -135,7 +138,8 @@ int partial_entry(const char* name, const void* x, const void* W, const void* sc
 template <bool W8>
 int qkv_entry(const char* name, const void* x, const void* W, const void* scales, const void* bqkv,
               void* q_out, void* Kc, void* Vc, int B, int T, int H, int hd, int S0, int S_cap,
-              int K, unsigned flags, const int32_t* len_dev, void* stream) {
+              int K, unsigned flags, const int32_t* len_dev, void* stream, const LnTail* ln = nullptr,
+              int ln_slices = 0) {
   MSA_REQUIRE(!len_dev || T == 1, MSA_ERR_INVALID_ARG, "%s: a device-side length needs T == 1",
               name);
   MSA_REQUIRE(q_out && Kc && Vc, MSA_ERR_INVALID_ARG, "%s: null pointer", name);
@@ -162,7 +166,10 @@ int qkv_entry(const char* name, const void* x, const void* W, const void* scales
   e.len_dev = len_dev;
   e.S_cap = S_cap;
   e.qscale = (float)pow((double)hd, -0.5);  // the reference's head_dim ** -0.5, cast to fp32
-  if (flags & MSA_IN_PACKED)
+  if (ln) {
+    MSA_REQUIRE((launch_stream_ln<W8, MODE_QKV>(*ln, ln_slices, W, scales, (int)M, N, K, e, (hipStream_t)stream)),
+                MSA_ERR_HIP, "%s: %d bytes of LDS refused", name, LN_MAX_K * 32);
+  } else if (flags & MSA_IN_PACKED)
     launch_stream<W8, MODE_QKV>(x, W, scales, nullptr, 1, (int)M, N, K, e, (hipStream_t)stream);
   else
     launch_tiled<W8, MODE_QKV>(x, W, scales, M, N, K, e, (hipStream_t)stream);
@@ -188,6 +195,28 @@ int pack_entry(const char* name, const void* src, void* dst, int N, int K, bool 
 }
 
 }  // namespace
+
+// Measured, a whole step without and with the fold, us: 12 layers of 768 one row 356 and 310, eight rows 406 and 329;
+// 24 of 1024 714 and 616, 758 and 662; 24 of 2048 1008 and 968, 1036 and 1028.  The int8 products are
+// shorter and have less to hide it behind: 8 layers of 2048 one row 322 and 317, four 327 and 325, six 331
+// and 334, eight 331 and 339.  More rows than waves or a longer row would not fit the registers.
+bool msa_ln_folds(int M, int D, int S, bool int8) {
+  return M >= 1 && M <= LN_MAX_ROWS && D <= LN_MAX_K && D % 64 == 0 && (S == 1 || S == 2 || S == 4) &&
+         (!int8 || M * D <= 8192);
+}
+int msa_ln_qkv_proj(const LnTail& ln, int S, const void* W, const void* scales, const void* bias, void* q_out,
+                    void* Kc, void* Vc, int M, int H, int hd, int S0, int S_cap, int K, const int32_t* len_dev,
+                    hipStream_t stream) {
+  auto entry = scales ? qkv_entry<true> : qkv_entry<false>;
+  return entry("qkv_proj behind a LayerNorm", ln.x, W, scales, bias, q_out, Kc, Vc, M, 1, H, hd, S0, S_cap, K,
+               MSA_IN_PACKED, len_dev, stream, &ln, S);
+}
+int msa_ln_linear_relu(const LnTail& ln, int S, const void* W, const void* scales, const void* bias, void* y_packed,
+                       int M, int N, int K, hipStream_t stream) {
+  auto entry = scales ? linear_entry<true> : linear_entry<false>;
+  return entry("linear behind a LayerNorm", ln.x, W, scales, bias, nullptr, y_packed, M, N, K,
+               MSA_EPI_RELU | MSA_IN_PACKED | MSA_OUT_PACKED, stream, &ln, S);
+}
 
 extern "C" int msa_pack_weight_f16(const void* src, void* dst, int N, int K, void* stream) {
   return pack_entry("msa_pack_weight_f16", src, dst, N, K, false, false, stream);

@@ -284,6 +284,84 @@ __device__ __forceinline__ half8_t dequant8(uint32_t lo, uint32_t hi, half_t sca
   return r;
 }
 
+// ---- the tail of a split-K product and the LayerNorm behind it, in front of the next product ----
+// Of a few rows every workgroup of the product that follows recomputes x = round(round(round(sum of slices) +
+// bias) + x) and LayerNorm(x) for itself, one wave per row, with layernorm_f16_kernel's arithmetic in its
+// order (the same bits), while its first weights are on their way.  Bound: a launch of the tail's own costs 3.3 us
+// of boundary and a chain of two block-wide sums; here the chain is one wave's, and its operands come out
+// of L2.  The first workgroup stores the new residual stream, to another buffer than the one that all read.
+constexpr int LN_MAX_ROWS = 8;     // one per wave
+constexpr int LN_MAX_K = 2048;     // four 16-byte chunks per lane
+template <int S>
+struct LnRow {
+  static constexpr int C = LN_MAX_K / 512;
+  float4_t p[S][C][2];
+  half8_t x[C], b[C], g[C], be[C];
+  __device__ __forceinline__ void fetch(const LnTail& t, int row, int M, int K, int lane) {
+    const int last = (K >> 3) - 1;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      if (c > 0 && c * 64 > last) continue;  // uniform
+      const int at = min(c * 64 + lane, last) * 8;
+#pragma unroll
+      for (int i = 0; i < S; ++i) {
+        const float* src = t.part + ((int64_t)i * M + row) * K + at;
+        p[i][c][0] = *reinterpret_cast<const float4_t*>(src);
+        p[i][c][1] = *reinterpret_cast<const float4_t*>(src + 4);
+      }
+      x[c] = *reinterpret_cast<const half8_t*>(t.x + (int64_t)row * K + at);
+      b[c] = *reinterpret_cast<const half8_t*>(t.bias + at);
+      g[c] = *reinterpret_cast<const half8_t*>(t.gamma + at);
+      be[c] = *reinterpret_cast<const half8_t*>(t.beta + at);
+    }
+  }
+  __device__ __forceinline__ void finish(const LnTail& t, int row, int M, int K, int lane, bool store,
+                                         half_t* rows) {
+    const int chunks = K >> 3;
+    float total = 0.f;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      float s = 0.f;
+      if (c > 0 && c * 64 >= chunks) continue;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        float v = p[0][c][i >> 2][i & 3];
+#pragma unroll
+        for (int k = 1; k < S; ++k) v += p[k][c][i >> 2][i & 3];
+        v = round_h(round_h(v) + (float)b[c][i]);
+        x[c][i] = (half_t)(v + (float)x[c][i]);
+        s += (float)x[c][i];
+      }
+      total += wave_sum(c * 64 + lane < chunks ? s : 0.f);
+    }
+    const float mean = total / (float)K;
+    float var = 0.f;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      float q = 0.f;
+      if (c > 0 && c * 64 >= chunks) continue;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float d = (float)x[c][i] - mean;
+        q += d * d;
+      }
+      var += wave_sum(c * 64 + lane < chunks ? q : 0.f);
+    }
+    const float rstd = rsqrtf(var / (float)K + t.eps);
+    if (row >= M) return;  // uniform
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      const int idx = c * 64 + lane;
+      if (idx >= chunks) continue;
+      if (store) *reinterpret_cast<half8_t*>(t.x_out + (int64_t)row * K + idx * 8) = x[c];
+      half8_t o;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) o[i] = (half_t)(((float)x[c][i] - mean) * rstd * (float)g[c][i] + (float)be[c][i]);
+      *reinterpret_cast<half8_t*>(rows + packed_act_offset(row, idx * 8, 1)) = o;
+    }
+  }
+};
+
 // ---- stream kernel (M <= 64) --------------------------------------------------------------
 // MFMA fragments: lane l supplies 8 consecutive K elements (offset 8*(l>>4)) of row (l&15) of
 // its operand; A rows are output features n, B rows are activation rows m.  The accumulator
@@ -300,15 +378,17 @@ constexpr int ST_RN = 4;  // tiles reduced across the waves per pass through LDS
 // tiles share each fragment and buffers fewer K steps to stay inside the register file (the
 // int8 kernel, whose stage also holds the raw bytes of two K steps, would spill).
 template <int MB, bool W8, int MODE, bool XR = false, int KG = ST_KG,
-          int NT = (MB <= 2 || W8 ? ST_NT : 2 * ST_NT), int U = (MB <= 2 ? 4 : (NT > ST_NT ? 1 : 2))>
+          int NT = (MB <= 2 || W8 ? ST_NT : 2 * ST_NT), int U = (MB <= 2 ? 4 : (NT > ST_NT ? 1 : 2)), int LN = 0>
 __global__ __launch_bounds__(KG * 64) void linear_stream_kernel(
     const half_t* __restrict__ xp, const void* __restrict__ Wp, const half_t* __restrict__ scales,
     float* __restrict__ part, int M, int N, int K, int tiles_per_wg, int ks_per_split,
-    Epilogue epi, int64_t m_off) {
+    Epilogue epi, int64_t m_off, LnTail ln = LnTail{}) {
+  static_assert(LN == 0 || (MB == 1 && !XR && KG == LN_MAX_ROWS), "one wave per row");
   // U = K steps (32 wide) buffered per stage; an int8 block covers two steps
   constexpr int UA = W8 ? U / 2 : U;  // weight loads per stage and tile
   constexpr int RN = NT < ST_RN ? NT : ST_RN;  // NT is a multiple of RN
   __shared__ float4_t red[KG][RN * MB][64];
+  extern __shared__ __attribute__((aligned(16))) half_t ln_rows[];  // LN: the normed rows, packed (one row block)
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int ntiles = N >> 4;
   const int nks = K >> 5;  // 32-wide steps in a row
@@ -346,6 +426,7 @@ __global__ __launch_bounds__(KG * 64) void linear_stream_kernel(
         s.a[u][j] = __builtin_nontemporal_load(
             reinterpret_cast<const half8_t*>((const half_t*)Wp + blk * 512 + lane * 8));
       }
+      if constexpr (LN > 0) continue;  // the activations are in LDS
 #pragma unroll
       for (int h = 0; h < (W8 ? 2 : 1); ++h) {
         const int kk = min(ks + h, ks_end - 1);
@@ -388,6 +469,8 @@ __global__ __launch_bounds__(KG * 64) void linear_stream_kernel(
     for (int u = 0; u < U; ++u) {
       const int ks = W8 ? ks_begin + 2 * (wave + KG * (st * UA + u / 2)) + (u & 1)
                         : ks_begin + wave + KG * (st * U + u);
+      if constexpr (LN > 0)
+        s.b[u][0] = *reinterpret_cast<const half8_t*>(ln_rows + (min(ks, ks_end - 1) * 64 + lane) * 8);
       if (ks >= ks_end) {
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) s.b[u][mb] = zero8();
@@ -454,7 +537,16 @@ __global__ __launch_bounds__(KG * 64) void linear_stream_kernel(
     clear();
   };
   clear();
-  load(s0, 0);
+  if constexpr (LN > 0) {
+    // Requested in this order, the tail's operands arrive while the first weights are on their way.
+    LnRow<LN> row;
+    row.fetch(ln, min(wave, M - 1), M, K, lane);
+    load(s0, 0);
+    row.finish(ln, wave, M, K, lane, blockIdx.x == 0, ln_rows);
+    __syncthreads();
+  } else {
+    load(s0, 0);
+  }
   int idx = 0;
   for (; idx + 2 < total; idx += 2) {  // steady state: every load is of a real stage
     load(s1, idx + 1);
@@ -1633,7 +1725,7 @@ void launch_stream_mb(const void* xp, const void* W, const void* scales, float* 
       auto kernel = tiles_per_wg == 1 ? linear_stream_kernel<MB, W8, MODE, false, ST_KG, 1, 4>
                                       : linear_stream_kernel<MB, W8, MODE, false, ST_KG, 2, 4>;
       hipLaunchKernelGGL(kernel, dim3(gx, S), dim3(ST_KG * 64), 0, s, (const half_t*)xp, W, (const half_t*)scales,
-                         part, M, N, K, tiles_per_wg, ks_per_split, epi, m_off);
+                         part, M, N, K, tiles_per_wg, ks_per_split, epi, m_off, LnTail{});
       return;
     }
   }
@@ -1752,6 +1844,35 @@ void launch_wide(const void* xp, const void* W, const void* scales, float* part,
   else
     launch_share_cfg<8, W8, MODE, 2, 4, 3, 2, 2>(xp, W, scales, part, S, M, N, K, tiles_per_wg, gx,
                                                  ks_per_split, epi, s);
+}
+
+// the tail in front of a product of at most LN_MAX_ROWS rows (S = 1, 2 or 4 slices); false: the LDS was refused
+template <bool W8, int MODE, int S>
+bool launch_stream_ln(const LnTail& ln, const void* W, const void* scales, int M, int N, int K, const Epilogue& epi,
+                      hipStream_t s) {
+  const int ntiles = N / 16, tpw = (ntiles + num_cus() - 1) / num_cus(), gx = (ntiles + tpw - 1) / tpw;
+  const int nks = K / 32, per = W8 ? (nks + 1) & ~1 : nks, bytes = K * 32;
+#define LN_RUN(NT)                                                                                            \
+  do {                                                                                                        \
+    auto kernel = linear_stream_kernel<1, W8, MODE, false, ST_KG, NT, 4, S>;                                  \
+    static std::atomic<uint64_t> allowed{0};                                                                  \
+    if (!allow_lds((const void*)kernel, LN_MAX_K * 32, allowed)) return false;                                \
+    hipLaunchKernelGGL(kernel, dim3(gx), dim3(ST_KG * 64), bytes, s, (const half_t*)nullptr, W,               \
+                       (const half_t*)scales, (float*)nullptr, M, N, K, tpw, per, epi, (int64_t)0, ln);       \
+  } while (0)
+  if (tpw == 1) LN_RUN(1);
+  else if (tpw == 2) LN_RUN(2);
+  else if (tpw == 3 || tpw == 6) LN_RUN(3);
+  else LN_RUN(4);
+#undef LN_RUN
+  return true;
+}
+template <bool W8, int MODE>
+bool launch_stream_ln(const LnTail& ln, int S, const void* W, const void* scales, int M, int N, int K,
+                      const Epilogue& epi, hipStream_t s) {
+  return S == 1   ? launch_stream_ln<W8, MODE, 1>(ln, W, scales, M, N, K, epi, s)
+         : S == 2 ? launch_stream_ln<W8, MODE, 2>(ln, W, scales, M, N, K, epi, s)
+                  : launch_stream_ln<W8, MODE, 4>(ln, W, scales, M, N, K, epi, s);
 }
 
 template <bool W8, int MODE, bool XR = false>
@@ -2014,7 +2135,10 @@ int pick_splits(int64_t M, int N, int K, int wbytes) {
   const int stage = MB > 2 ? 16 : ST_KG * 4;
   int best = 1;
   double best_cost = 0;
-  for (int S = 1; S <= 8; S *= 2) {
+  // Up to eight fp16 rows stop at four slices, which the next product can sum itself (msa_ln_folds): 2048 x 8192
+  // takes 7.8 us in four and 7.9 in eight, and a 1.3b step of one row without the fold 1020 us and 1008.
+  const int most = M <= LN_MAX_ROWS && wbytes == 2 ? 4 : 8;
+  for (int S = 1; S <= most; S *= 2) {
     const int G = num_cus() / S;
     if (G < 1 || nks / S < stage) break;  // every wave needs a full stage of K steps
     const int tpw = (ntiles + G - 1) / G;

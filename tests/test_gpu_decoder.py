@@ -396,6 +396,33 @@ def test_one_call_decode_step_equals_the_step_driven_entry_point_by_entry_point(
         assert a[6] == b[6]
 
 
+@pytest.mark.parametrize("dim,heads,rows,int8", [
+    (64, 1, 1, False), (64, 1, 8, True), (576, 9, 3, False), (768, 12, 8, False), (768, 12, 1, True),
+    (1024, 16, 5, False), (1600, 25, 7, False), (2048, 32, 8, False), (2048, 32, 1, False),
+    (2048, 16, 4, True), (2048, 32, 5, True), (2112, 33, 2, False), (768, 12, 9, False)])
+def test_one_call_step_of_few_rows_takes_the_layernorm_into_the_next_product(dim, heads, rows, int8):
+    """The bits of the Python-driven sequence, whose LayerNorms are launches of their own: one lane group of a
+    chunk to all four chunks of a row, one to eight rows, one to four slices; and just outside of it."""
+    cfg = OPTConfig(decoder_layers=3, decoder_embed_dim=dim, decoder_attention_heads=heads,
+                    decoder_ffn_embed_dim=4 * dim, vocab_size=512, max_target_positions=64)
+    model, _ = build(cfg, seed=dim + rows, int8=int8)
+    dec = model.decoder
+    prompt = random_prompts(cfg, rows, 6, seed=2).to(DEV)
+    nxt = torch.randint(4, cfg.vocab_size, (rows, 3), generator=torch.Generator().manual_seed(3)).to(DEV)
+    outs = []
+    for native in (True, False):
+        dec.native_step = native
+        inc, toks, steps = {}, prompt, []
+        model(prompt, incremental_state=inc)
+        for t in range(3):
+            toks = torch.cat([toks, nxt[:, t:t + 1]], 1)
+            steps.append(dec(toks, incremental_state=inc)[0].clone())
+        outs.append(steps)
+    dec.native_step = True
+    for x, y in zip(*outs):
+        assert bool(torch.isfinite(x).all()) and torch.equal(x, y)
+
+
 def test_one_call_step_with_split_attention_equals_the_one_launch_form():
     """One request over a history of more than 4096 positions at head_dim 128:
     msa_decoder_step takes the two-launch attention, the Python-driven step the one-launch
