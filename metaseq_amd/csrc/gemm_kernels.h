@@ -1258,11 +1258,10 @@ struct GroupTiles {
 // PART: split-K.  Workgroup (bx, by, z) sums over the K range of ``part_stages`` 64-wide stages
 // that starts at stage z * part_stages and stores its fp32 sums, with no epilogue, as slice z of
 // ``part`` ([gridDim.z][M][N]); a later launch adds the slices in slice order.
-template <int MODE, int WF, bool PART = false, bool GROUPED = false, int RF = 8, bool FEW = false>
-__global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
-    const half_t* __restrict__ x, const void* __restrict__ Wp, int64_t M, int N, int K,
-    int rm_a, int rm_b, int rm_r, Epilogue epi, float* __restrict__ part, int part_stages,
-    GroupTiles gt = GroupTiles{}) {
+template <int MODE, int WF, bool PART, bool GROUPED, int RF, bool FEW>
+__device__ __forceinline__ void quad_tile(const half_t* __restrict__ x, const void* __restrict__ Wp, int64_t M, int N,
+                                          int K, int bx, int by, int bz, int64_t g_first, const Epilogue& epi,
+                                          float* __restrict__ part, int part_stages, const GroupTiles& gt) {
   extern __shared__ __attribute__((aligned(16))) char tq_lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 15, lg = lane >> 4;
@@ -1271,40 +1270,6 @@ __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
   constexpr int TQ_RX = tq_rx(RF), TQ_RW = tq_rw(RF), TQ_WOFF = TQ_RX * TQ_XBYTES;
   constexpr int WL = WF / 2;  // weight load instructions per wave and step
   constexpr int XL = RF;      // activation load instructions per wave and stage
-  int bx = blockIdx.x, by = blockIdx.y;
-  int64_t g_first = 0;
-  if constexpr (GROUPED) {
-    const int ncol = gridDim.x, L = by * ncol + bx, total = *gt.n_tiles * ncol;
-    const int per = (total + 7) / 8, t = (L & 7) * per + (L >> 3);
-    if ((L >> 3) >= per || t >= total) return;
-    by = t / ncol;
-    bx = t - by * ncol;
-    const int g = gt.tile_group[by];
-    g_first = gt.tile_row[by];
-    M = min((int64_t)gt.group_end[g], g_first + TQ_BM);
-    Wp = (const char*)Wp + (int64_t)g * N * K * 2;
-  } else if (rm_a < 0) {
-    // panels of 16 columns, one after the other over all rows: 16 x 16 tiles of a panel at a time as eight
-    // 4 x 8 blocks, one per XCD, the panel's last rows and a narrower last panel row by row
-    const int ncol = gridDim.x, nrow = gridDim.y, L = by * ncol + bx;
-    const int p = L / (TQ_PANEL * nrow), w = min(TQ_PANEL, ncol - p * TQ_PANEL), idx = L - p * TQ_PANEL * nrow;
-    const int i = idx & 255, round = idx >> 8;
-    if (w == TQ_PANEL && (round + 1) * 16 <= nrow) {
-      const int xcd = i & 7, k = i >> 3;
-      bx = p * TQ_PANEL + (xcd & 3) * 4 + (k & 3);
-      by = round * 16 + (xcd >> 2) * 8 + (k >> 2);
-    } else {
-      bx = p * TQ_PANEL + idx % w;
-      by = idx / w;
-    }
-  } else if (rm_a > 0) {
-    const int ncol = gridDim.x, L = by * ncol + bx, round = L >> 8, i = L & 255;
-    if ((round + 1) * rm_r <= (int)gridDim.y) {  // a full round of 256 tiles
-      const int xcd = i & 7, k = i >> 3, gx = ncol / rm_a;
-      bx = (xcd % gx) * rm_a + k % rm_a;
-      by = round * rm_r + (xcd / gx) * rm_b + k / rm_a;
-    }
-  }
   // The narrowest form (WF = 2) also serves fewer than 256 rows: it does not move a ragged tile up
   // but repeats the last row in its loads and drops the rows past it in the epilogue.  So does
   // the split-K form of WF = 4 (decode batches of 129 .. 255 rows cut K eight ways over it).
@@ -1314,7 +1279,7 @@ __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
   const int n0 = bx * TQ_BN;
   // the stages this workgroup sums over: all of K, or its slice (the operand bases below move
   // to the slice's first stage, so that stage and step numbers count from 0 either way)
-  const int st_first = PART ? (int)blockIdx.z * part_stages : 0;
+  const int st_first = PART ? bz * part_stages : 0;
   const int nst = PART ? part_stages : K / 64, nks = 2 * nst;
   const int ntiles = N / 16;
 
@@ -1515,6 +1480,10 @@ __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
     });
   };
   int xs = 0, ws = 0;
+  // The loop begins at (or 4 bytes past) a 128-byte line of instructions: with one wave per SIMD its fetches show
+  // wherever it happens to lie (1500 x 3072 x 4096 on 256 x 128 tiles 51 us, 60 bytes past a line 52.6).  The
+  // fill covers, with the few scalar instructions the compiler puts behind it, one line.
+  asm volatile(".p2align 7\n\t.fill 25, 4, 0xbf800000" ::"s"(nks), "s"(xs), "s"(ws) : "memory");
   for (int t = 0; t < nks; t += 2) {
     step(t, xs, ws, std::integral_constant<int, 0>{});
     ws = ws == TQ_RW - 1 ? 0 : ws + 1;
@@ -1536,7 +1505,7 @@ __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
   if constexpr (PART) {
     // the sums as the lanes hold them: D tile (i, j) = activation row 16 * i + lr of the wave's
     // 128, features 16 * j + 4 * lg .. + 3 of the wave's 16 WF (16 bytes per lane, 64 per row)
-    float* slice = part + (int64_t)blockIdx.z * M * N;
+    float* slice = part + (int64_t)bz * M * N;
 #pragma unroll
     for (int i = 0; i < RF; ++i) {
       const int64_t m = m0 + wm * (TQ_BM / 2) + i * 16 + lr;
@@ -1670,6 +1639,84 @@ __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
       }
     }
     if (i + TQ_RES_AHEAD < RF) load_res(i + TQ_RES_AHEAD, res8[i % TQ_RES_AHEAD]);
+  }
+}
+
+// Tile t of ncol x nrow in the order of launch (see above: rm_a > 0 regrouped rounds, < 0 panels, 0 row by row).
+__device__ __forceinline__ void quad_place(int t, int ncol, int nrow, int rm_a, int rm_b, int rm_r, int& bx, int& by) {
+  by = t / ncol;
+  bx = t - by * ncol;
+  if (rm_a < 0) {
+    // panels of 16 columns, one after the other over all rows: 16 x 16 tiles of a panel at a time as eight
+    // 4 x 8 blocks, one per XCD, the panel's last rows and a narrower last panel row by row
+    const int p = t / (TQ_PANEL * nrow), w = min(TQ_PANEL, ncol - p * TQ_PANEL), idx = t - p * TQ_PANEL * nrow;
+    const int i = idx & 255, round = idx >> 8;
+    if (w == TQ_PANEL && (round + 1) * 16 <= nrow) {
+      const int xcd = i & 7, k = i >> 3;
+      bx = p * TQ_PANEL + (xcd & 3) * 4 + (k & 3);
+      by = round * 16 + (xcd >> 2) * 8 + (k >> 2);
+    } else {
+      bx = p * TQ_PANEL + idx % w;
+      by = idx / w;
+    }
+  } else if (rm_a > 0) {
+    const int round = t >> 8, i = t & 255;
+    if ((round + 1) * rm_r <= nrow) {  // a full round of 256 tiles
+      const int xcd = i & 7, k = i >> 3, gx = ncol / rm_a;
+      bx = (xcd % gx) * rm_a + k % rm_a;
+      by = round * rm_r + (xcd / gx) * rm_b + k / rm_a;
+    }
+  }
+}
+
+template <int MODE, int WF, bool PART = false, bool GROUPED = false, int RF = 8, bool FEW = false>
+__global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
+    const half_t* __restrict__ x, const void* __restrict__ Wp, int64_t M, int N, int K,
+    int rm_a, int rm_b, int rm_r, Epilogue epi, float* __restrict__ part, int part_stages,
+    GroupTiles gt = GroupTiles{}) {
+  int bx = blockIdx.x, by = blockIdx.y;
+  int64_t g_first = 0;
+  if constexpr (GROUPED) {
+    const int ncol = gridDim.x, L = by * ncol + bx, total = *gt.n_tiles * ncol;
+    const int per = (total + 7) / 8, t = (L & 7) * per + (L >> 3);
+    if ((L >> 3) >= per || t >= total) return;
+    by = t / ncol;
+    bx = t - by * ncol;
+    const int g = gt.tile_group[by];
+    g_first = gt.tile_row[by];
+    M = min((int64_t)gt.group_end[g], g_first + tq_bm(RF));
+    Wp = (const char*)Wp + (int64_t)g * N * K * 2;
+  } else if (rm_a != 0) {
+    quad_place(by * gridDim.x + bx, gridDim.x, gridDim.y, rm_a, rm_b, rm_r, bx, by);
+  }
+  quad_tile<MODE, WF, PART, GROUPED, RF, FEW>(x, Wp, M, N, K, bx, by, blockIdx.z, g_first, epi, part, part_stages, gt);
+}
+
+// Tiles that would begin a round without filling half of it, in pieces: the first n_full tiles (of all K slices, whole
+// rounds) are 256 x 256, the others PIECES = 2 of 256 x 128 or 4 of 128 x 128, side by side on one XCD.
+template <int MODE, bool PART, int PIECES>
+__global__ __launch_bounds__(TQ_THREADS) void linear_quad_pieces_kernel(
+    const half_t* __restrict__ x, const void* __restrict__ Wp, int64_t M, int N, int K, int ncol, int nrow,
+    int slices, int n_full, int rm_a, int rm_b, int rm_r, Epilogue epi, float* __restrict__ part, int part_stages) {
+  const int tiles = ncol * nrow, j = (int)blockIdx.x - n_full;
+  int unit = blockIdx.x, piece = 0, bx, by;
+  if (j >= 0) {  // the first pieces of eight tiles, then their second ones, ...
+    const int q = j / (8 * PIECES), w = min(8, tiles * slices - n_full - 8 * q), r = j % (8 * PIECES);
+    unit = n_full + 8 * q + r % w;
+    piece = r / w;
+  }
+  const int bz = PART ? unit / tiles : 0;
+  quad_place(unit - bz * tiles, ncol, nrow, rm_a, rm_b, rm_r, bx, by);
+  const GroupTiles none{};
+  if (j < 0) return quad_tile<MODE, 8, PART, false, 8, false>(x, Wp, M, N, K, bx, by, bz, 0, epi, part, part_stages, none);
+  bx = 2 * bx + (piece & 1);
+  if (bx * tq_bn(4) >= N) return;
+  if constexpr (PIECES == 2) {
+    quad_tile<MODE, 4, PART, false, 8, false>(x, Wp, M, N, K, bx, by, bz, 0, epi, part, part_stages, none);
+  } else {
+    by = 2 * by + (piece >> 1);
+    if ((int64_t)by * tq_bm(4) < M)
+      quad_tile<MODE, 4, PART, false, 4, false>(x, Wp, M, N, K, bx, by, bz, 0, epi, part, part_stages, none);
   }
 }
 
@@ -1912,39 +1959,87 @@ void launch_stream(const void* xp, const void* W, const void* scales, float* par
 // rows 600 -> 502; 6038 x 21888 x 4096 (86 columns) 960 -> 918; 48 and 64 columns are the same either way.
 bool wide_panels(int ncol) { return ncol > 64; }
 
-// One launch of the four-wave kernel (WF = 8: 256 x 256 tiles, WF = 4: 256 x 128) on rows
-// 0 .. M_main - 1 (a ragged last row tile is moved up) plus the streaming kernel on the rows from
-// M_main on (at most 128).
-template <int MODE, int WF>
-void launch_quad(const void* x, const void* W, const void* scales, int64_t M, int64_t M_main, int N,
-                 int K, const Epilogue& epi, hipStream_t s) {
-  static std::atomic<uint64_t> lds_allowed_q{0};
-  if (!allow_lds((const void*)linear_quad_kernel<MODE, WF>, tq_lds_bytes(WF), lds_allowed_q)) return;
-  const int ncol = (N + tq_bn(WF) - 1) / tq_bn(WF);
-  const int nrow = (int)((M_main + TQ_BM - 1) / TQ_BM);
-  // regrouping of a round's 256 tiles: a x b per XCD with a * b = 32, (ncol / a) * (r / b) = 8
-  // for r = 256 / ncol rows per round; taken when it beats the default strip (ncol / 8) x r
-  int rm_a = 0, rm_b = 0, rm_r = 0;
-  if (ncol >= 8 && 256 % ncol == 0) {
+// regrouping of a round's 256 tiles: a x b per XCD with a * b = 32, (ncol / a) * (r / b) = 8 for r = 256 / ncol
+// rows per round; taken when it beats the default strip (ncol / 8) x r.  a < 0: panels, a = 0: row by row
+struct TileOrder {
+  int a, b, r;
+};
+TileOrder tile_order(int ncol) {
+  TileOrder o{0, 0, 0};
+  if (wide_panels(ncol)) {
+    o.a = -TQ_PANEL;
+  } else if (ncol >= 8 && 256 % ncol == 0) {
     const int r = 256 / ncol;
     int best = ncol / 8 + r;
     for (int a = 1; a <= 32; a *= 2) {
       const int b = 32 / a;
       if (ncol % a || r % b || (ncol / a) * (r / b) != 8) continue;
-      if (a + b < best) best = a + b, rm_a = a, rm_b = b, rm_r = r;
+      if (a + b < best) best = a + b, o = TileOrder{a, b, r};
     }
   }
-  if (wide_panels(ncol)) rm_a = -TQ_PANEL;
-  hipLaunchKernelGGL((linear_quad_kernel<MODE, WF>), dim3(ncol, nrow), dim3(TQ_THREADS),
-                     tq_lds_bytes(WF), s, (const half_t*)x, W, M_main, N, K, rm_a, rm_b, rm_r, epi,
-                     (float*)nullptr, 0);
+  return o;
+}
+
+// Time of a round of tiles, in rounds of 256 x 256 ones (103 us of K = 4096): 256 x 128 63 us, 256 x 64 45, 128 x 128 37.
+constexpr double TQ_ROUND_US = 103.0 / 4096, TQ_COST_4 = 0.61, TQ_COST_2 = 0.43, TQ_COST_Q = 0.36;
+int64_t quad_rounds(int64_t tiles) { return (tiles + num_cus() - 1) / num_cus(); }
+// Into how many pieces the tiles are cut that are left after whole rounds of 256 x 256 ones (1: they are not): as many
+// as still run in one round.  Without and with, K = 4096, us: 2005 x 9216 (32 tiles left) 170 -> 130 in quarters,
+// 147 in halves; 2005 x 10240 (64) 171 -> 136, 149; 1500 x 14848 (92) 198 -> 171; 2005 x 12288 (128) 179 ->
+// 162, 171 in quarters; 6038 x 5888 (two rounds and 40) 272 -> 233; 2005 x 50272 (six and 40) 677 -> 638.
+// More than half a round is not cut: 1500 x 50272 (four and 158) 490 and 502.
+int quad_pieces(int64_t tiles) {
+  const int64_t left = tiles % num_cus();
+  return tiles < num_cus() || left == 0 || left * 2 > num_cus() ? 1 : left * 4 > num_cus() ? 2 : 4;
+}
+double quad_cost(int64_t tiles) {
+  const int pieces = quad_pieces(tiles);
+  return pieces == 1 ? (double)quad_rounds(tiles)
+                     : (double)(tiles / num_cus()) + (pieces == 2 ? TQ_COST_4 : TQ_COST_Q);
+}
+
+template <int MODE, bool PART, int PIECES>
+void launch_quad_pieces(const void* x, const void* W, int64_t M, int N, int K, int S, const Epilogue& epi, float* part,
+                        hipStream_t s) {
+  static std::atomic<uint64_t> lds_allowed_h{0};
+  auto kernel = linear_quad_pieces_kernel<MODE, PART, PIECES>;
+  if (!allow_lds((const void*)kernel, tq_lds_bytes(8), lds_allowed_h)) return;
+  const int ncol = (N + tq_bn(8) - 1) / tq_bn(8), nrow = (int)((M + TQ_BM - 1) / TQ_BM), units = ncol * nrow * S;
+  const int n_full = units / num_cus() * num_cus();
+  const TileOrder o = tile_order(ncol);
+  hipLaunchKernelGGL(kernel, dim3(n_full + PIECES * (units - n_full)), dim3(TQ_THREADS), tq_lds_bytes(8), s,
+                     (const half_t*)x, W, M, N, K, ncol, nrow, S, n_full, o.a, o.b, o.r, epi, part, K / 64 / S);
+}
+
+// One launch of the four-wave kernel (WF = 8: 256 x 256 tiles, the last of them in pieces where that pays; WF = 4:
+// 256 x 128, WF = 2: 256 x 64) on rows 0 .. M_main - 1 (a ragged last row tile is moved up) plus the streaming kernel on the rows from
+// M_main on (at most 128).
+template <int MODE, int WF>
+void launch_quad(const void* x, const void* W, const void* scales, int64_t M, int64_t M_main, int N,
+                 int K, const Epilogue& epi, hipStream_t s) {
+  const int ncol = (N + tq_bn(WF) - 1) / tq_bn(WF);
+  const int nrow = (int)((M_main + TQ_BM - 1) / TQ_BM);
+  const int pieces = WF == 8 ? quad_pieces((int64_t)ncol * nrow) : 1;
+  if (pieces == 4) {
+    launch_quad_pieces<MODE, false, 4>(x, W, M_main, N, K, 1, epi, nullptr, s);
+  } else if (pieces == 2) {
+    launch_quad_pieces<MODE, false, 2>(x, W, M_main, N, K, 1, epi, nullptr, s);
+  } else {
+    static std::atomic<uint64_t> lds_allowed_q{0};
+    if (!allow_lds((const void*)linear_quad_kernel<MODE, WF>, tq_lds_bytes(WF), lds_allowed_q)) return;
+    const TileOrder o = tile_order(ncol);
+    hipLaunchKernelGGL((linear_quad_kernel<MODE, WF>), dim3(ncol, nrow), dim3(TQ_THREADS),
+                       tq_lds_bytes(WF), s, (const half_t*)x, W, M_main, N, K, o.a, o.b, o.r, epi,
+                       (float*)nullptr, 0);
+  }
   for (int64_t m0 = M_main; m0 < M; m0 += 64)
     launch_stream<false, MODE, true>(x, W, scales, nullptr, 1, (int)min((int64_t)64, M - m0), N,
                                      K, epi, s, m0);
 }
 
 // One round of tiles over fewer rows than a 256-row tile holds, or a little more than one of 128.
-//   RF = 4: 128 x 128 tiles, two rows of them side by side on one XCD.  Of 129 .. 256 rows a CU then reads half as
+//   RF = 4: 128 x 128 tiles, two rows of them side by side on one XCD (also of more rows, where one round of them
+//   is cheapest: 2048 x 2048 x 4096 44.9 us on 256 x 64 tiles -> 39.6).  Of 129 .. 256 rows a CU then reads half as
 //   many activations as with the 256 x 64 form, its weights once more from L2: 200 x 12288 x 4096 44.3 ->
 //   39.5 us, 200 x 16384 x 4096 48.4 -> 46.8, 129 x 8192 x 2048 22.5 -> 19.3.  (As split-K sums they
 //   gained nothing: 200 x 4096 x 16384 49.8 -> 53.5.)
@@ -1972,24 +2067,29 @@ void launch_quad_partial_w(const void* x, const void* W, float* part, int64_t M,
   const int ncol = (N + tq_bn(WF) - 1) / tq_bn(WF);
   const int nrow = (int)((M + TQ_BM - 1) / TQ_BM);
   Epilogue e{};
-  const int rm_a = wide_panels(ncol) ? -TQ_PANEL : 0;
+  const TileOrder o = tile_order(ncol);
   hipLaunchKernelGGL(kernel, dim3(ncol, nrow, S), dim3(TQ_THREADS), tq_lds_bytes(WF), s,
-                     (const half_t*)x, W, M, N, K, rm_a, 0, 0, e, part, K / 64 / S, GroupTiles{});
+                     (const half_t*)x, W, M, N, K, o.a, o.b, o.r, e, part, K / 64 / S, GroupTiles{});
 }
 
-// 256 x 64 tiles while their S slices fit the chip in one round; an S beyond that means 256 x 128
-// tiles.
+// fp16: 256 x 64 tiles while their S slices fit the chip in one round; an S beyond that means 256 x 128
+// tiles.  bf16 (prefill-sized products whose sums leave as fp32): the cheapest of all widths.
 template <int MODE>
 void launch_quad_partial(const void* x, const void* W, float* part, int64_t M, int N, int K, int S,
                          hipStream_t s) {
-  const int64_t tiles2 = ((M + TQ_BM - 1) / TQ_BM) * ((N + tq_bn(2) - 1) / tq_bn(2));
+  const int64_t rows = (M + TQ_BM - 1) / TQ_BM;
+  const int64_t tiles2 = rows * ((N + 63) / 64) * S, tiles4 = rows * ((N + 127) / 128) * S;
   if constexpr (is_bf<MODE>) {
-    // prefill-sized products whose sums leave as fp32: 256 x 256 tiles once they fill the chip
-    const int64_t tiles8 = ((M + TQ_BM - 1) / TQ_BM) * ((N + tq_bn(8) - 1) / tq_bn(8));
-    if (M >= TQ_BM && tiles8 * S * 4 >= num_cus() * 3)
+    const int64_t tiles8 = rows * ((N + 255) / 256) * S;
+    const double narrow = fmin(quad_rounds(tiles4) * TQ_COST_4, quad_rounds(tiles2) * TQ_COST_2);
+    if (M >= TQ_BM && quad_cost(tiles8) <= narrow) {
+      const int pieces = quad_pieces(tiles8);
+      if (pieces == 4) return launch_quad_pieces<MODE, true, 4>(x, W, M, N, K, S, Epilogue{}, part, s);
+      if (pieces == 2) return launch_quad_pieces<MODE, true, 2>(x, W, M, N, K, S, Epilogue{}, part, s);
       return launch_quad_partial_w<MODE, 8>(x, W, part, M, N, K, S, s);
+    }
   }
-  if (tiles2 * S > num_cus())
+  if (tiles2 > num_cus())
     return launch_quad_partial_w<MODE, 4>(x, W, part, M, N, K, S, s);
   launch_quad_partial_w<MODE, 2>(x, W, part, M, N, K, S, s);
 }
@@ -2033,43 +2133,44 @@ void launch_tiled(const void* x, const void* W, const void* scales, int64_t M, i
   const int64_t big_tiles = ((M + TB_BM - 1) / TB_BM) * ((N + TB_BN - 1) / TB_BN);
   if constexpr (!W8) {
     // Fewer rows than a tile, or hardly more: launch_few_rows where its tiles fill one round (three quarters of
-    // the CUs with 256 x 256, a quarter with 128 x 128 tiles).  Else
-    // three tile widths, 256, 128 and 64 features (a workgroup of 128 does half the MFMAs of 256 in
-    // about 0.8 of the time, one of 64 a quarter in about 0.55), and two ways to take a ragged
-    // bottom of at most 128 rows: as one more, moved-up row of tiles, or through the streaming
-    // kernel (one sweep over the weights per 64 rows).  The combinations are priced in rounds of
-    // workgroups and the cheapest is taken.  The two wider forms go down to 3/8 of a tile per CU:
-    // below that a single round of their tiles no longer beats the narrowest form, which is taken
-    // down to 1/8 of a tile per CU and also serves 65 .. 255 rows (it repeats the last row instead
-    // of moving a tile up); below that the 128 x 128 kernel runs.
+    // the CUs with 256 x 256, a quarter with 128 x 128 tiles).  Else four tiles, 256 x 256 (the last of
+    // them in pieces), 256 x 128, 256 x 64 and 128 x 128, and two ways to take a ragged bottom of at
+    // most 128 rows: as one more, moved-up row of tiles, or through the streaming kernel (one sweep
+    // over the weights per 64 rows).  The combinations are priced in rounds of workgroups and the
+    // cheapest is taken.  The 256 x 64 tiles also serve 65 .. 255 rows (they repeat the last row instead of
+    // moving up); where even they would fill less than an eighth of the chip the 128 x 128 kernel
+    // of eight waves runs.
     if (K % 64 == 0 && K >= 128 && M > 64) {
-      const int64_t cus = num_cus(), rem = M % TQ_BM;
+      const int64_t cus = num_cus(), rem = M % TQ_BM, rows = (M + TQ_BM - 1) / TQ_BM;
       const int64_t cols[3] = {(N + 255) / 256, (N + 127) / 128, (N + 63) / 64};
       if (M < TQ_BM && cols[0] <= cus && cols[0] * 4 >= cus * 3)
         return launch_few_rows<MODE, 8, 8>(x, W, M, N, K, epi, s);
       if (M > 128 && M <= TQ_BM && cols[1] * 2 <= cus && cols[1] * 8 >= cus)
         return launch_few_rows<MODE, 4, 4>(x, W, M, N, K, epi, s);
-      const double factor[3] = {1.0, 0.8, 0.55};
-      const double unit = 63.0 * K / 4096;  // us per round of wide tiles
-      const double sweep = (double)N * K * 2 / 5e6 + 4;  // us per streaming launch
-      double best = 1e30;
-      int best_w = -1;
-      int64_t best_main = M;
-      for (int opt = 0; opt < 6; ++opt) {
-        const int w = opt >> 1;
-        const bool stream = opt & 1;
-        if (w < 2 && M < TQ_BM) continue;
-        if (stream && !(w < 2 && rem > 0 && rem <= 128 && M - rem >= TQ_BM)) continue;
-        const int64_t m_main = stream ? M - rem : M;
-        const int64_t tiles = ((m_main + TQ_BM - 1) / TQ_BM) * cols[w];
-        if (tiles * 8 < (w == 2 ? cus : cus * 3)) continue;
-        const double cost = (double)((tiles + cus - 1) / cus) * factor[w] * unit +
-                            (stream ? (double)((rem + 63) / 64) * sweep : 0.0);
-        if (cost < best) best = cost, best_w = w, best_main = m_main;
+      if (rows * cols[2] * 8 >= cus) {
+        const double unit = TQ_ROUND_US * K;                  // us per round of 256 x 256 tiles
+        const double sweep = (double)N * K * 2 / 5e6 + 4;  // us per streaming launch
+        double best = (double)quad_rounds(rows * cols[2]) * TQ_COST_2 * unit;
+        int best_w = 2;
+        int64_t best_main = M;
+        auto offer = [&](double cost, int w, int64_t m_main) {
+          if (cost < best) best = cost, best_w = w, best_main = m_main;
+        };
+        if (M > TQ_BM) offer((double)quad_rounds((M + 127) / 128 * cols[1]) * TQ_COST_Q * unit, 3, M);
+        if (M >= TQ_BM) {
+          offer((double)quad_rounds(rows * cols[1]) * TQ_COST_4 * unit, 1, M);
+          offer(quad_cost(rows * cols[0]) * unit, 0, M);
+        }
+        if (rem > 0 && rem <= 128 && M - rem >= TQ_BM) {
+          const double below = (double)((rem + 63) / 64) * sweep;
+          offer((double)quad_rounds((rows - 1) * cols[1]) * TQ_COST_4 * unit + below, 1, M - rem);
+          offer(quad_cost((rows - 1) * cols[0]) * unit + below, 0, M - rem);
+        }
+        if (best_w == 0) return launch_quad<MODE, 8>(x, W, scales, M, best_main, N, K, epi, s);
+        if (best_w == 1) return launch_quad<MODE, 4>(x, W, scales, M, best_main, N, K, epi, s);
+        if (best_w == 2) return launch_quad<MODE, 2>(x, W, scales, M, best_main, N, K, epi, s);
+        return launch_few_rows<MODE, 4, 4>(x, W, M, N, K, epi, s);
       }
-      if (best_w == 0) return launch_quad<MODE, 8>(x, W, scales, M, best_main, N, K, epi, s);
-      if (best_w == 1) return launch_quad<MODE, 4>(x, W, scales, M, best_main, N, K, epi, s);
-      if (best_w == 2) return launch_quad<MODE, 2>(x, W, scales, M, best_main, N, K, epi, s);
     }
   }
   if constexpr (!is_bf<MODE>) if (K % (2 * TB_BK) == 0 && big_tiles >= num_cus()) {

@@ -107,6 +107,28 @@ def test_linear_partial_bf16_wide_panels(M, N):
         close(part.sum(0).cpu(), ref.cpu(), 1e-5, "partial sums, S=%d" % S)
 
 
+@pytest.mark.parametrize("M,N", [(1500, 6032), (1500, 6912), (2305, 7168), (3000, 7680)])
+def test_linear_bf16_pieces(M, N):
+    """A few tiles past whole rounds, cut in four or in two: sums of one and two slices (288 and 324 tiles of
+    them), a gated activation with fp32 columns behind it."""
+    lib, K = _capi.load_hybrid(), 256
+    g = torch.Generator("cuda").manual_seed(M)
+    x = torch.randn(M, K, generator=g, device="cuda").to(BF16)
+    w = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).to(BF16)
+    wp, ref = pack_tiles(w), (x.float() @ w.float().t()).cpu()
+    for S in (1, 2):
+        part = torch.full((S, M, N), float("nan"), device="cuda")
+        check(lib.msa_linear_partial_bf16(ptr(x), ptr(wp), ptr(part), M, N, K, S, 0, _capi.stream_ptr()), lib)
+        close(part.sum(0).cpu(), ref, 1e-5, "partial sums, S=%d" % S)
+    n32 = N // 2 // 32 * 32
+    y = torch.zeros(M, n32 // 2, dtype=BF16, device="cuda")
+    y32 = torch.zeros(M, N - n32, device="cuda")
+    check(lib.msa_linear_bf16(ptr(x), ptr(wp), ptr(y), ptr(y32), M, N, K, n32, _capi.MSA_GLU_CLAMPED, 0.7, 0,
+                              _capi.stream_ptr()), lib)
+    close(y.cpu(), glu(_capi.MSA_GLU_CLAMPED, ref[:, 0:n32:2], ref[:, 1:n32:2], 0.7), 6e-3, "glu")
+    close(y32.cpu(), ref[:, n32:], 1e-5, "fp32 columns beside glu")
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 16, 32), (70, 80, 96), (200, 144, 128)])
 def test_linear_f32(M, N, K):
     lib = _capi.load_hybrid()

@@ -473,6 +473,30 @@ def test_linear_f16_few_rows(lib, M, N, K, epi):
     assert bool(((y.float() - want).abs() <= bound).all())
 
 
+# Whole rounds of 256 x 256 tiles and a few left, which are cut in four (280, 276 and 1060 tiles) or in two (360 and
+# 1122): pieces past the last row or column, of one row and of a few columns, a last group of fewer
+# than eight tiles; and 128 x 128 tiles of more than 256 rows
+@pytest.mark.parametrize("M,N", [(2305, 7168), (2825, 5728), (5000, 13328), (2945, 7520), (3000, 7680), (4352, 16656),
+                                 (2048, 2048), (641, 4112)])
+def test_linear_f16_pieces(lib, M, N):
+    K = 128
+    print("pieces", M, N, flush=True)
+    x, W, b = G(rnd(M, K, seed=M)), G(rnd(N, K, seed=N, std=0.05)), G(rnd(N, seed=9, std=0.1))
+    y = G(rnd(M, N, seed=10))
+    res = y.float()
+    ok(lib.msa_linear_f16(P(x), P(pack_w(lib, W)), P(b), P(y), P(y), M, N, K, 0, None), lib)   # in place
+    torch.cuda.synchronize()
+    want = x.float() @ W.float().t()
+    size = want.abs()
+    want = want.half().float() + b.float()
+    size = torch.maximum(size, want.abs())
+    want = want.half().float() + res
+    size = torch.maximum(size, want.abs())
+    # the bound of test_linear_f16_few_rows
+    bound = 5 * size * 2.0 ** -11 + 8 * 2.0 ** -24 * K ** 0.5 * float(size.square().mean().sqrt()) + 2.0 ** -24
+    assert bool(((y.float() - want).abs() <= bound).all())
+
+
 # more than 64 columns of tiles, which are taken in panels of 16: full and partial 16 x 16 blocks, a last
 # panel of one column and of several, a ragged bottom and right edge
 @pytest.mark.parametrize("M,N", [(4096, 16640), (8400, 16400), (700, 20500 // 16 * 16), (4500, 20480), (256, 24592)])
