@@ -208,6 +208,16 @@ int msa_qkv_proj_w8a16(const void* x, const int8_t* Wq, const void* scales, cons
                        int S0, int S_cap, int K, unsigned flags, const int32_t* len_dev,
                        void* stream);
 
+/* The same for M rows each of which appends to a cache row and at a position of its own (device arrays of M; a
+ * negative position or one past S_cap: neither key nor value is stored; every rows[m] names a row of the cache):
+ * several prompts back to back, each into its slot. */
+int msa_qkv_proj_rows_f16(const void* x, const void* Wqkv, const void* bqkv, void* q_out, void* Kcache, void* Vcache,
+                          const int32_t* rows, const int32_t* positions, int M, int H, int hd, int S_cap, int K,
+                          unsigned flags, void* stream);
+int msa_qkv_proj_rows_w8a16(const void* x, const int8_t* Wq, const void* scales, const void* bqkv, void* q_out,
+                            void* Kcache, void* Vcache, const int32_t* rows, const int32_t* positions, int M, int H,
+                            int hd, int S_cap, int K, unsigned flags, void* stream);
+
 /* Causal attention of T new queries (already scaled, q[B*T, H*hd]) over the cache, whose
  * positions 0 .. S0+T-1 are valid: query t sees keys 0 .. S0+t.
  *   s = round(q . k);  s = -inf where key_pad_mask[b, key] != 0;
@@ -222,6 +232,11 @@ int msa_attention_f16(const void* q, const void* Kcache, const void* Vcache,
                       const uint8_t* key_pad_mask, int64_t mask_stride, void* out, int B, int H,
                       int hd, int T, int S0, int S_cap, unsigned flags, const int32_t* len_dev,
                       void* stream);
+
+/* Causal attention of several whole prompts back to back: segment i is rows starts[i] .. starts[i + 1] - 1 of q and out
+ * (device, segments + 1 ascending entries; at most `longest` rows each) over the first positions of cache row rows[i]. */
+int msa_attention_rows_f16(const void* q, const void* Kcache, const void* Vcache, void* out, const int32_t* starts,
+                           const int32_t* rows, int segments, int longest, int H, int hd, int S_cap, void* stream);
 
 /* EXPERIMENTAL: pays only beyond OPT's 2048 positions (no benchmark configuration selects it;
  * msa_decoder_step takes it for a single request over more than 4096 keys at head_dim 128).

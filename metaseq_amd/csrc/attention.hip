@@ -343,6 +343,22 @@ __global__ __launch_bounds__(16 * (64 / (HD / 8)) * 4) void attention_values_ker
 
 }  // namespace
 
+extern "C" int msa_attention_rows_f16(const void* q, const void* Kcache, const void* Vcache, void* out,
+                                      const int32_t* starts, const int32_t* rows, int segments, int longest, int H,
+                                      int hd, int S_cap, void* stream) {
+  const char* name = "msa_attention_rows_f16";
+  MSA_REQUIRE(q && Kcache && Vcache && out && starts && rows, MSA_ERR_INVALID_ARG, "%s: null pointer", name);
+  MSA_REQUIRE(segments > 0 && H > 0 && longest > 0 && (int64_t)segments * H <= 0x7fffffff, MSA_ERR_INVALID_ARG,
+              "%s: bad shape segments=%d H=%d longest=%d", name, segments, H, longest);
+  MSA_REQUIRE(hd == 64 || hd == 128, MSA_ERR_INVALID_ARG, "%s: head_dim %d not supported (64 or 128)", name, hd);
+  MSA_REQUIRE(longest <= S_cap && longest <= 8192, MSA_ERR_CAPACITY,
+              "%s: %d positions exceed the cache capacity %d or 8192", name, longest, S_cap);
+  msa_launch_prefill_attention(q, Kcache, Vcache, nullptr, 0, out, segments, H, hd, longest, 0, S_cap,
+                               (hipStream_t)stream, starts, rows);
+  MSA_CHECK_LAUNCH(name);
+  return MSA_OK;
+}
+
 extern "C" int msa_attention_f16(const void* q, const void* Kcache, const void* Vcache,
                                  const uint8_t* key_pad_mask, int64_t mask_stride, void* out, int B,
                                  int H, int hd, int T, int S0, int S_cap, unsigned flags,

@@ -45,7 +45,8 @@ template <int HD>
 __global__ __launch_bounds__(PF_THREADS) void prefill_attention_kernel(
     const half_t* __restrict__ q, const half_t* __restrict__ Kc, const half_t* __restrict__ Vc,
     const uint8_t* __restrict__ key_pad_mask, int64_t mask_stride, half_t* __restrict__ out,
-    int BH, int n_qt, int grouped, int H, int T, int S0, int S_cap) {
+    int BH, int n_qt, int grouped, int H, int T, int S0, int S_cap, const int32_t* __restrict__ seg_start,
+    const int32_t* __restrict__ seg_row) {
   constexpr int KSTEPS = HD / 16;           // MFMA k steps over the head dimension
   constexpr int DBLK = HD / 32;             // 32-row blocks of O^T
   constexpr int ROWB = HD * 2;              // bytes of a key row
@@ -74,6 +75,15 @@ __global__ __launch_bounds__(PF_THREADS) void prefill_attention_kernel(
   }
   if (bh >= BH) return;  // the last group of 8 may be incomplete (uniform per workgroup)
   const int b = bh / H, h = bh - b * H;
+  // segments of their own lengths, back to back: the launch has the longest one's tiles for all
+  int64_t row0 = (int64_t)b * T;
+  int cache_row = b;
+  if (seg_start) {
+    row0 = seg_start[b];
+    T = seg_start[b + 1] - (int)row0;
+    cache_row = seg_row[b];
+    if (qt * PF_BM >= T) return;
+  }
   const int D = H * HD;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -86,14 +96,14 @@ __global__ __launch_bounds__(PF_THREADS) void prefill_attention_kernel(
   const int wg_last_q = qt * PF_BM - lead + PF_BM - 1;
   const int n_keys = S0 + wg_last_q + 1;  // keys this workgroup needs
   const int ntiles = (n_keys + PF_BN - 1) / PF_BN;
-  const half_t* kbase = Kc + (int64_t)bh * S_cap * HD;
-  const half_t* vbase = Vc + (int64_t)bh * S_cap * HD;
+  const half_t* kbase = Kc + ((int64_t)cache_row * H + h) * S_cap * HD;
+  const half_t* vbase = Vc + ((int64_t)cache_row * H + h) * S_cap * HD;
   const uint8_t* mrow = key_pad_mask ? key_pad_mask + (int64_t)b * mask_stride : nullptr;
 
   // Q^T fragments (B operand): query j, 8 consecutive d at 16*ks + 8*hl
   half8_t qf[KSTEPS];
   {
-    const half_t* qrow = q + ((int64_t)b * T + tqc) * D + h * HD + hl * 8;
+    const half_t* qrow = q + (row0 + tqc) * D + h * HD + hl * 8;
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks)
       qf[ks] = *reinterpret_cast<const half8_t*>(qrow + ks * 16);
@@ -278,7 +288,7 @@ __global__ __launch_bounds__(PF_THREADS) void prefill_attention_kernel(
   }
   // O^T accumulator: lane holds query j and d = 32*db + 8*blk + 4*hl + r
   if (tq >= 0) {
-    half_t* orow = out + ((int64_t)b * T + tq) * D + h * HD;
+    half_t* orow = out + (row0 + tq) * D + h * HD;
 #pragma unroll
     for (int db = 0; db < DBLK; ++db)
 #pragma unroll
@@ -296,7 +306,8 @@ __global__ __launch_bounds__(PF_THREADS) void prefill_attention_kernel(
 int msa_launch_prefill_attention(const void* q, const void* Kc, const void* Vc,
                                  const uint8_t* key_pad_mask, int64_t mask_stride, void* out,
                                  int B, int H, int hd, int T, int S0, int S_cap,
-                                 hipStream_t stream) {
+                                 hipStream_t stream, const int32_t* seg_start,
+                                 const int32_t* seg_row) {
   const int n_qt = (T + PF_BM - 1) / PF_BM, BH = B * H;
   const dim3 grid((unsigned)(((BH + 7) / 8) * 8 * n_qt));
   // K and V rows of all (row, head) pairs against the 32 MB of L2 + part of the memory-side cache
@@ -304,10 +315,12 @@ int msa_launch_prefill_attention(const void* q, const void* Kc, const void* Vc,
   if (hd == 64)
     hipLaunchKernelGGL(prefill_attention_kernel<64>, grid, dim3(PF_THREADS), 0, stream,
                        (const half_t*)q, (const half_t*)Kc, (const half_t*)Vc, key_pad_mask,
-                       mask_stride, (half_t*)out, BH, n_qt, grouped, H, T, S0, S_cap);
+                       mask_stride, (half_t*)out, BH, n_qt, grouped, H, T, S0, S_cap,
+                       seg_start, seg_row);
   else
     hipLaunchKernelGGL(prefill_attention_kernel<128>, grid, dim3(PF_THREADS), 0, stream,
                        (const half_t*)q, (const half_t*)Kc, (const half_t*)Vc, key_pad_mask,
-                       mask_stride, (half_t*)out, BH, n_qt, grouped, H, T, S0, S_cap);
+                       mask_stride, (half_t*)out, BH, n_qt, grouped, H, T, S0, S_cap,
+                       seg_start, seg_row);
   return 0;
 }

@@ -139,7 +139,7 @@ template <bool W8>
 int qkv_entry(const char* name, const void* x, const void* W, const void* scales, const void* bqkv,
               void* q_out, void* Kc, void* Vc, int B, int T, int H, int hd, int S0, int S_cap,
               int K, unsigned flags, const int32_t* len_dev, void* stream, const LnTail* ln = nullptr,
-              int ln_slices = 0) {
+              int ln_slices = 0, const int32_t* row_dev = nullptr) {
   MSA_REQUIRE(!len_dev || T == 1, MSA_ERR_INVALID_ARG, "%s: a device-side length needs T == 1",
               name);
   MSA_REQUIRE(q_out && Kc && Vc, MSA_ERR_INVALID_ARG, "%s: null pointer", name);
@@ -164,6 +164,7 @@ int qkv_entry(const char* name, const void* x, const void* W, const void* scales
   e.hd_shift = (hd & (hd - 1)) == 0 ? __builtin_ctz((unsigned)hd) : -1;
   e.S0 = S0;
   e.len_dev = len_dev;
+  e.row_dev = row_dev;
   e.S_cap = S_cap;
   e.qscale = (float)pow((double)hd, -0.5);  // the reference's head_dim ** -0.5, cast to fp32
   if (ln) {
@@ -209,7 +210,7 @@ int msa_ln_qkv_proj(const LnTail& ln, int S, const void* W, const void* scales, 
                     hipStream_t stream) {
   auto entry = scales ? qkv_entry<true> : qkv_entry<false>;
   return entry("qkv_proj behind a LayerNorm", ln.x, W, scales, bias, q_out, Kc, Vc, M, 1, H, hd, S0, S_cap, K,
-               MSA_IN_PACKED, len_dev, stream, &ln, S);
+               MSA_IN_PACKED, len_dev, stream, &ln, S, nullptr);
 }
 int msa_ln_linear_relu(const LnTail& ln, int S, const void* W, const void* scales, const void* bias, void* y_packed,
                        int M, int N, int K, hipStream_t stream) {
@@ -425,4 +426,23 @@ extern "C" int msa_qkv_proj_w8a16(const void* x, const int8_t* Wq, const void* s
                                   const int32_t* len_dev, void* stream) {
   return qkv_entry<true>("msa_qkv_proj_w8a16", x, Wq, scales, bqkv, q_out, Kcache, Vcache, B, T, H,
                          hd, S0, S_cap, K, flags, len_dev, stream);
+}
+
+extern "C" int msa_qkv_proj_rows_f16(const void* x, const void* Wqkv, const void* bqkv, void* q_out, void* Kcache,
+                                     void* Vcache, const int32_t* rows, const int32_t* positions, int M, int H,
+                                     int hd, int S_cap, int K, unsigned flags, void* stream) {
+  const char* name = "msa_qkv_proj_rows_f16";
+  MSA_REQUIRE(rows && positions, MSA_ERR_INVALID_ARG, "%s: null pointer", name);
+  return qkv_entry<false>(name, x, Wqkv, nullptr, bqkv, q_out, Kcache, Vcache, M, 1, H, hd, 0, S_cap, K, flags,
+                          positions, stream, nullptr, 0, rows);
+}
+
+extern "C" int msa_qkv_proj_rows_w8a16(const void* x, const int8_t* Wq, const void* scales, const void* bqkv,
+                                       void* q_out, void* Kcache, void* Vcache, const int32_t* rows,
+                                       const int32_t* positions, int M, int H, int hd, int S_cap, int K,
+                                       unsigned flags, void* stream) {
+  const char* name = "msa_qkv_proj_rows_w8a16";
+  MSA_REQUIRE(rows && positions, MSA_ERR_INVALID_ARG, "%s: null pointer", name);
+  return qkv_entry<true>(name, x, Wq, scales, bqkv, q_out, Kcache, Vcache, M, 1, H, hd, 0, S_cap, K, flags,
+                         positions, stream, nullptr, 0, rows);
 }

@@ -58,6 +58,7 @@ struct Epilogue {
   int T, H, hd, S0, S_cap;
   int hd_shift;  // log2(hd) if hd is a power of two, else -1
   const int32_t* len_dev;  // if set (T == 1): per-row append positions on the device (< 0: skip)
+  const int32_t* row_dev;  // if set (with len_dev): the row of the cache that each row appends to
   float qscale;
   // MODE_SELECT: greedy selection over the output row instead of (or besides) storing it
   SelectPartial* partials;  // [M][gridDim.x]
@@ -251,7 +252,7 @@ __device__ __forceinline__ void epilogue4(const Epilogue& e, int64_t m, int n, f
       const int s0 = e.len_dev ? e.len_dev[b] : e.S0;  // per-row lengths: T == 1, b = row
       if (s0 >= 0 && s0 + tt < e.S_cap) {
         half_t* dst = (part == 0 ? e.Kc : e.Vc) +
-                      (((int64_t)b * e.H + h) * e.S_cap + s0 + tt) * e.hd + d;
+                      (((int64_t)(e.row_dev ? e.row_dev[b] : b) * e.H + h) * e.S_cap + s0 + tt) * e.hd + d;
         *reinterpret_cast<half4_t*>(dst) = o;
       }
     }
@@ -1197,10 +1198,10 @@ __device__ __forceinline__ void tq_static_for(F&& f) {
 
 // 8 consecutive output columns n..n+7 of row m; v holds the accumulators rounded to fp16, b the
 // bias and r the residual values of those columns (read only where the epilogue has them)
-// (QKV mode: qb, qt = the row's batch row and position, m = qb * T + qt)
+// (QKV mode: qb, qt = the row's batch row and its position behind the cache's first s0)
 template <int MODE>
 __device__ __forceinline__ void epilogue8(const Epilogue& e, int64_t m, int n, half8_t v,
-                                          half8_t b, half8_t r, int qb, int qt) {
+                                          half8_t b, half8_t r, int qb, int qt, int s0) {
   float t[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) t[i] = (float)v[i];
@@ -1235,7 +1236,6 @@ __device__ __forceinline__ void epilogue8(const Epilogue& e, int64_t m, int n, h
 #pragma unroll
       for (int i = 0; i < 8; ++i) o[i] = (half_t)t[i];
       const int h = e.hd_shift >= 0 ? c >> e.hd_shift : c / e.hd, d = c - h * e.hd;
-      const int s0 = e.len_dev ? e.len_dev[qb] : e.S0;
       if (s0 >= 0 && s0 + qt < e.S_cap) {
         half_t* dst = (part == 0 ? e.Kc : e.Vc) +
                       (((int64_t)qb * e.H + h) * e.S_cap + s0 + qt) * e.hd + d;
@@ -1614,6 +1614,19 @@ __device__ __forceinline__ void quad_tile(const half_t* __restrict__ x, const vo
     qb = epi.T == 1 ? mf : mf / epi.T;
     qt = mf - qb * epi.T;
   }
+  // rows with positions (and cache rows) of their own: all of the lane's are read in front of its first store, behind
+  // which none would be in flight
+  int own_at[MODE == MODE_QKV ? RF : 1][ENR], own_row[MODE == MODE_QKV ? RF : 1][ENR];
+  if (MODE == MODE_QKV && epi.len_dev) {
+#pragma unroll
+    for (int i = 0; i < (MODE == MODE_QKV ? RF : 0); ++i)
+#pragma unroll
+      for (int r = 0; r < ENR; ++r) {
+        const int m = (int)min(m0 + wm * (TQ_BM / 2) + i * 16 + ERPI * r + erow, M - 1);
+        own_at[i][r] = epi.len_dev[m];
+        own_row[i][r] = epi.row_dev ? epi.row_dev[m] : m;
+      }
+  }
 #pragma unroll
   for (int i = 0; i < RF; ++i) {
     char* buf = mine + (i & 1) * 4096;
@@ -1631,8 +1644,13 @@ __device__ __forceinline__ void quad_tile(const half_t* __restrict__ x, const vo
       const half8_t v = *reinterpret_cast<const half8_t*>(buf + row * ERB +
                                                           ((ec ^ (row & (ECH - 1))) * 16));
       const int64_t m = m0 + wm * (TQ_BM / 2) + i * 16 + row;
-      if (col_ok && m >= m_own && m < M)
-        epilogue8<MODE>(epi, m, en, v, bias8, res8[i % TQ_RES_AHEAD][r], qb, qt);
+      if (col_ok && m >= m_own && m < M) {
+        if (MODE == MODE_QKV && epi.len_dev)
+          epilogue8<MODE>(epi, m, en, v, bias8, bias8, own_row[MODE == MODE_QKV ? i : 0][r], 0,
+                          own_at[MODE == MODE_QKV ? i : 0][r]);
+        else
+          epilogue8<MODE>(epi, m, en, v, bias8, res8[i % TQ_RES_AHEAD][r], qb, qt, epi.S0);
+      }
       if (MODE == MODE_QKV) {
         qt += ERPI;
         while (qt >= epi.T) qt -= epi.T, ++qb;

@@ -11,6 +11,7 @@ import ctypes
 import uuid
 from typing import Any, Dict, Optional
 
+import numpy as np
 import torch
 from torch import nn
 
@@ -368,7 +369,18 @@ class TransformerDecoder(IncrementalDecoder):
             check(lib.msa_linear_partial_f16(ptr(x), ptr(lin.weight), ptr(part), M, N, K, S,
                                              MSA_IN_PACKED, stream))
 
-    def _qkv(self, lib, stream, h, qkv, q, kc, vc, B, T, H, hd, S0, cap, D, flags, len_dev=None):
+    def _qkv(self, lib, stream, h, qkv, q, kc, vc, B, T, H, hd, S0, cap, D, flags, len_dev=None,
+             prompts=None):
+        if prompts is not None:
+            to = (ptr(q), ptr(kc), ptr(vc), ptr(prompts.row), ptr(prompts.position), B * T, H, hd, cap, D,
+                  flags, stream)
+            if qkv.qweight is not None and not self._expands(B * T, 3 * D):
+                check(lib.msa_qkv_proj_rows_w8a16(ptr(h), ptr(qkv.qweight), ptr(qkv.scales), ptr(qkv.bias),
+                                                  *to))
+            else:
+                w = self._expanded(lib, stream, qkv) if qkv.qweight is not None else ptr(qkv.weight)
+                check(lib.msa_qkv_proj_rows_f16(ptr(h), w, ptr(qkv.bias), *to))
+            return
         if qkv.qweight is not None and self._expands(B * T, 3 * D):
             check(lib.msa_qkv_proj_f16(ptr(h), self._expanded(lib, stream, qkv), ptr(qkv.bias),
                                        ptr(q), ptr(kc), ptr(vc), B, T, H, hd, S0, cap, D, flags,
@@ -746,7 +758,7 @@ class TransformerDecoder(IncrementalDecoder):
         return features, packed, (B, T), {"inner_states": inner_states}
 
     def _rows_core(self, lib, stream, tokens, B, n, T, S0, kv, mask, token_embeddings=None,
-                   len_dev=None, step_len=None):
+                   len_dev=None, step_len=None, prompts=None):
         """Prefill (or a decode batch above 128 rows): the last T columns of ``tokens[B, n]``
         through embedding, L layers and the final LayerNorm on row-major activations and the
         tiled MFMA kernels, keys and values written at positions S0 .. S0 + T - 1 of ``kv``
@@ -754,7 +766,9 @@ class TransformerDecoder(IncrementalDecoder):
         [B * T, D] and the inner-states list.  With ``len_dev`` (T == 1; int32 [B] device
         tensor: positions each row already holds, negative = inactive row) every row appends at
         and attends up to its own length; ``step_len`` (int32 [B]) receives the lengths the
-        step used (-1 for the rows that sat it out)."""
+        step used (-1 for the rows that sat it out).  With ``prompts`` (_Prompts; S0 == 0) the
+        pads are dropped behind the embedding: everything runs over the prompts' own rows, one
+        after the other, and their keys and values go to the cache rows they name."""
         cfg = self.cfg
         D = cfg.decoder_embed_dim
         dev = tokens.device
@@ -771,12 +785,16 @@ class TransformerDecoder(IncrementalDecoder):
         if step_len is not None:
             len_dev = step_len
         inner_states = [{"tok": None, "pos": positions, "emb": None}]
+        if prompts is not None:
+            x = x.index_select(0, prompts.index)
+            M = B = x.shape[0]
+            T = 1
         if self.return_inner_states:
             inner_states[0]["emb"] = x.view(B, T, D).transpose(0, 1).clone()
         work = self._rows_buffers(M, dev)
         for i, layer in enumerate(self.layers):
             self._rows_layer(lib, stream, layer, x, work, B, T, S0, kv.k(i), kv.v(i),
-                             kv.capacity, mask, len_dev)
+                             kv.capacity, mask, len_dev, prompts)
             if self.layer_probe is not None:
                 self.layer_probe(i, x)
         if self.return_inner_states:
@@ -826,7 +844,17 @@ class TransformerDecoder(IncrementalDecoder):
         return {"q": torch.empty(M, D, **f16), "h": torch.empty(M, D, **f16),
                 "o": torch.empty(M, D, **f16), "u": torch.empty(M, F, **f16)}
 
-    def _rows_layer(self, lib, stream, layer, x, work, B, T, S0, kc, vc, cap, mask, len_dev=None):
+    def _rows_attention(self, lib, stream, q, kc, vc, mask, o, B, H, hd, T, S0, cap, len_dev, prompts):
+        if prompts is not None:
+            check(lib.msa_attention_rows_f16(ptr(q), ptr(kc), ptr(vc), ptr(o), ptr(prompts.start),
+                                             ptr(prompts.slot), prompts.count, prompts.longest, H, hd, cap,
+                                             stream))
+            return
+        check(lib.msa_attention_f16(ptr(q), ptr(kc), ptr(vc), ptr(mask), mask.stride(0) if mask is not None else 0,
+                                    ptr(o), B, H, hd, T, S0, cap, 0, ptr(len_dev), stream))
+
+    def _rows_layer(self, lib, stream, layer, x, work, B, T, S0, kc, vc, cap, mask, len_dev=None,
+                    prompts=None):
         """One layer over B * T row-major rows (transformer_decoder_layer.py:233-284): ``x`` is
         the residual stream, updated in place; keys and values of the T new positions of every
         row go to positions S0 .. S0 + T - 1 of ``kc`` / ``vc``."""
@@ -836,14 +864,12 @@ class TransformerDecoder(IncrementalDecoder):
         M = B * T
         if M <= self.PACKED_MAX_ROWS:
             return self._rows_layer_short(lib, stream, layer, x, work, B, T, S0, kc, vc, cap, mask,
-                                          len_dev)
+                                          len_dev, prompts)
         q, h, o, u = work["q"], work["h"], work["o"], work["u"]
-        mask_stride = mask.stride(0) if mask is not None else 0
         self._layernorm(lib, stream, x, layer.self_attn_layer_norm, M, D, h)
         self._qkv(lib, stream, h, layer.self_attn.qkv_proj, q, kc, vc, B, T, H, hd, S0, cap, D, 0,
-                  len_dev)
-        check(lib.msa_attention_f16(ptr(q), ptr(kc), ptr(vc), ptr(mask), mask_stride, ptr(o), B,
-                                    H, hd, T, S0, cap, 0, ptr(len_dev), stream))
+                  len_dev, prompts)
+        self._rows_attention(lib, stream, q, kc, vc, mask, o, B, H, hd, T, S0, cap, len_dev, prompts)
         # x = round(round(o Wo^T + bo) + x)   (transformer_decoder_layer.py:222-230)
         ln2 = layer.final_layer_norm
         if not self._linear_split(lib, stream, o, layer.self_attn.out_proj, x, work, M, D, D,
@@ -855,7 +881,7 @@ class TransformerDecoder(IncrementalDecoder):
             self._linear(lib, stream, u, layer.fc2, M, D, F, residual=x, out=x)
 
     def _rows_layer_short(self, lib, stream, layer, x, work, B, T, S0, kc, vc, cap, mask,
-                          len_dev=None):
+                          len_dev=None, prompts=None):
         """``_rows_layer`` for at most 128 rows (a short prompt): the layer's GEMM inputs are
         produced in the packed activation layout by the kernels in front of them, so that qkv,
         fc1 and fc2 run on the weight-streaming kernels of the decode step (56 rows, OPT-6.7B
@@ -876,12 +902,10 @@ class TransformerDecoder(IncrementalDecoder):
             splits = lib.msa_linear_default_splits_w8a16 if int8 else lib.msa_linear_default_splits
             work["S_f"] = splits(M, D, F)
         hp, up, S_f = work["hp"], work["up"], work["S_f"]
-        mask_stride = mask.stride(0) if mask is not None else 0
         self._layernorm(lib, stream, x, layer.self_attn_layer_norm, M, D, hp, OUT)
         self._qkv(lib, stream, hp, layer.self_attn.qkv_proj, q, kc, vc, B, T, H, hd, S0, cap, D, IN,
-                  len_dev)
-        check(lib.msa_attention_f16(ptr(q), ptr(kc), ptr(vc), ptr(mask), mask_stride, ptr(o), B,
-                                    H, hd, T, S0, cap, 0, ptr(len_dev), stream))
+                  len_dev, prompts)
+        self._rows_attention(lib, stream, q, kc, vc, mask, o, B, H, hd, T, S0, cap, len_dev, prompts)
         ln2 = layer.final_layer_norm
         if not self._linear_split(lib, stream, o, layer.self_attn.out_proj, x, work, M, D, D,
                                   ln=ln2, ln_out=hp, ln_flags=OUT):
@@ -963,10 +987,10 @@ class TransformerDecoder(IncrementalDecoder):
 
     def prefill_slots(self, cache: KVCache, slots, prompts):
         """One prefill for several prompts (1-D id tensors on the device, as for
-        ``prefill_slot``) into the rows ``slots`` of ``cache``: the prompts run as one
-        right-padded batch, so the weights are read once for all of them - under the causal
-        mask no real position sees a pad, and the pads' own rows are dropped - and every
-        prompt's keys and values are then copied to its slot.  Returns the logits of every
+        ``prefill_slot``) into the rows ``slots`` of ``cache``: the prompts' rows run back to
+        back, so the weights are read once for all of them, nothing is computed for padding (only the
+        embedding sees a right-padded batch), and every prompt's keys and values are written to its
+        slot as they are made.  Returns the logits of every
         prompt's positions, a list of ``[T_i, V]`` fp16 tensors.  The products run on other
         tile shapes than a prompt's own prefill would, so results can differ from
         ``prefill_slot``'s in the last bit."""
@@ -993,15 +1017,12 @@ class TransformerDecoder(IncrementalDecoder):
         toks = torch.full((k, Tmax), self.padding_idx, dtype=torch.long, device=dev)
         for r, t in enumerate(prompts):
             toks[r, :lens[r]] = t
-        tmp = KVCache(cfg.decoder_layers, k, cfg.decoder_attention_heads, cfg.head_dim, Tmax, dev)
-        h, _ = self._rows_core(lib, _capi.stream_ptr(), toks, k, Tmax, Tmax, 0, tmp, None)
-        # one copy per layer: whole padded rows (what lies past a prompt's length is never read)
-        where = upload(slots, torch.long, dev)
-        for mine, theirs in zip(cache.layers, tmp.layers):
-            mine[:, :, :, :Tmax].index_copy_(1, where, theirs)
-        cache.lens[where] = upload(lens, torch.int32, dev)
-        logits = self._project(h, False, k, Tmax)
-        return [logits[r, :lens[r]] for r in range(k)]
+        packed = _Prompts(slots, lens, dev)
+        h, _ = self._rows_core(lib, _capi.stream_ptr(), toks, k, Tmax, Tmax, 0, cache, None,
+                               prompts=packed)
+        cache.lens[upload(slots, torch.long, dev)] = upload(lens, torch.int32, dev)
+        logits = self._project(h, False, 1, sum(lens))[0]
+        return list(logits.split(lens))
 
     def decode_slots(self, cache: KVCache, last_tokens: torch.Tensor, *, temperature=1.0,
                      banned=(), stop=(), eos=2, row_mode=None, tok_out=None, score_out=None,
@@ -1165,6 +1186,22 @@ class TransformerDecoder(IncrementalDecoder):
             ptr(f), ptr(self._lm_head), ptr(logits_out), ptr(ws), B, V, D, float(temperature), ba,
             len(banned), sa, len(stop), ptr(finished), ptr(row_mode), int(force_eos), int(eos),
             ptr(tok_out), tok_stride, ptr(score_out), score_stride, None, _capi.stream_ptr()))
+
+
+class _Prompts:
+    """Where the rows of several prompts back to back come from and go to: ``index`` into the right-padded batch,
+    ``row`` and ``position`` in the cache (int32, one per row), and per prompt its ``start`` and ``slot``."""
+
+    def __init__(self, slots, lens, device):
+        self.count, self.longest = len(lens), max(lens)
+        n = np.asarray(lens, dtype=np.int32)
+        start = np.concatenate([[0], np.cumsum(n)]).astype(np.int32)
+        of = np.repeat(np.arange(len(lens), dtype=np.int32), n)
+        position = np.arange(start[-1], dtype=np.int32) - start[of]
+        parts = [of * np.int32(self.longest) + position, np.asarray(slots, dtype=np.int32)[of], position, start,
+                 np.asarray(slots, dtype=np.int32)]
+        flat = torch.from_numpy(np.concatenate(parts)).pin_memory().to(device, non_blocking=True)
+        self.index, self.row, self.position, self.start, self.slot = flat.split([p.size for p in parts])
 
 
 class _SlotView:

@@ -527,6 +527,35 @@ def test_shared_prefill_of_several_prompts_matches_their_own_prefills(int8):
         dec.prefill_slots(shared, [2, 2], prompts[:2])
 
 
+@pytest.mark.parametrize("dim,heads,int8,lens", [
+    (256, 2, False, [1, 1]), (256, 2, False, [128, 1, 127]), (128, 2, False, [129, 300, 128, 5, 256]),
+    (256, 2, True, [40, 30, 7]), (128, 2, True, [200, 1, 131]), (2048, 16, False, [1, 511, 300, 2])])
+def test_prompts_back_to_back_match_their_own_prefills(dim, heads, int8, lens):
+    """Lengths around the query tile's 128, one row and many, into slots in no order of a cache that holds NaN:
+    logits, keys and values as each prompt's own prefill leaves them, nothing else written."""
+    cfg = tiny_cfg(layers=2, dim=dim, heads=heads, vocab=96, max_pos=600)
+    model, _ = build(cfg, seed=22, int8=int8)
+    dec = model.decoder
+    g = torch.Generator().manual_seed(4)
+    slots = [(3 * i + 2) % 7 for i in range(len(lens))]
+    prompts = [torch.cat([torch.tensor([2]), torch.randint(4, 96, (n - 1,), generator=g)]).to(DEV) for n in lens]
+    shared, alone = dec.new_slot_cache(7, 520), dec.new_slot_cache(7, 520)
+    for layer in shared.layers:
+        layer.fill_(float("nan"))
+    got = dec.prefill_slots(shared, slots, prompts)
+    want = [dec.prefill_slot(alone, s, p) for s, p in zip(slots, prompts)]
+    assert shared.lens.tolist() == alone.lens.tolist()
+    for g_l, w_l, n in zip(got, want, lens):
+        assert g_l.shape == (n, 96)
+        check_logits(g_l, w_l, "back to back, %d positions" % n)
+    for a, b in zip(shared.layers, alone.layers):
+        for s in range(7):
+            n = lens[slots.index(s)] if s in slots else 0
+            if n:   # (the tolerance of the test above)
+                assert float((a[:, s, :, :n].float() - b[:, s, :, :n].float()).abs().nan_to_num(9.0).max()) < 2e-2
+            assert bool(torch.isnan(a[:, s, :, n:]).all())
+
+
 @pytest.mark.parametrize("kw", [dict(), dict(temperature=0.7), dict(need_logprobs=True),
                                 dict(alpha_presence=0.4, alpha_frequency=0.1)],
                          ids=["fused greedy", "fused, scaled", "distributions kept",
