@@ -85,61 +85,80 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const float* __restrict_
   if (shared_gate && lane == 0) shared_gate[m] = sigmoidf(row[E]);
 }
 
-// One workgroup per expert: counts all pairs, then writes its own expert's rows in pair order.
-__global__ __launch_bounds__(256) void moe_plan_kernel(const int32_t* __restrict__ ids, int P, int E,
-                                                       int tile_rows, int32_t* __restrict__ perm,
-                                                       int32_t* __restrict__ inverse,
-                                                       int32_t* __restrict__ group_end,
-                                                       int32_t* __restrict__ tile_group,
-                                                       int32_t* __restrict__ tile_row,
-                                                       int32_t* __restrict__ n_tiles,
-                                                       int max_tiles) {
+// One workgroup per expert: counts all pairs, then writes its own expert's rows in pair order.  Bound: a chain of loads
+// per wave.  Every wave owns one run of the pairs and goes over it twice without a barrier, first to count its
+// expert's pairs, then to place them behind those of the waves in front of it; eight loads in
+// flight.  48304 pairs, 64 experts: 17 us (a barrier pair per 256 pairs: 114), 256 pairs 4.7 (5.7).
+constexpr int MP_THREADS = 1024, MP_WAVES = MP_THREADS / 64, MP_AHEAD = 8;
+__global__ __launch_bounds__(MP_THREADS) void moe_plan_kernel(const int32_t* __restrict__ ids, int P, int E,
+                                                              int tile_rows, int32_t* __restrict__ perm,
+                                                              int32_t* __restrict__ inverse,
+                                                              int32_t* __restrict__ group_end,
+                                                              int32_t* __restrict__ tile_group,
+                                                              int32_t* __restrict__ tile_row,
+                                                              int32_t* __restrict__ n_tiles, int max_tiles) {
   __shared__ int hist[512];
-  __shared__ int sh_row, sh_tile, wcount[4];
+  __shared__ int sh_row, sh_tile, wcount[MP_WAVES];
   const int e = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  for (int i = tid; i < E; i += 256) hist[i] = 0;
+  for (int i = tid; i < E; i += MP_THREADS) hist[i] = 0;
   __syncthreads();
-  for (int p = tid; p < P; p += 256) atomicAdd(&hist[ids[p]], 1);
+  const int run = ((P + MP_WAVES - 1) / MP_WAVES + 63) / 64 * 64;  // pairs per wave
+  const int first = min(wave * run, P), last = min(first + run, P);
+  auto walk = [&](auto&& each) {
+    for (int p0 = first; p0 < last; p0 += 64 * MP_AHEAD) {
+      int id[MP_AHEAD];
+#pragma unroll
+      for (int i = 0; i < MP_AHEAD; ++i) {
+        const int p = p0 + i * 64 + lane;
+        id[i] = p < last ? ids[p] : -1;
+      }
+#pragma unroll
+      for (int i = 0; i < MP_AHEAD; ++i) each(p0 + i * 64 + lane, id[i]);
+    }
+  };
+  int own = 0;
+  walk([&](int, int id) {
+    own += __popcll(__ballot(id == e));
+    if (id >= 0) atomicAdd(&hist[id], 1);
+  });
+  if (lane == 0) wcount[wave] = own;
   __syncthreads();
-  if (tid == 0) {
+  if (wave == 0) {
     int row = 0, tile = 0;
-    for (int i = 0; i < e; ++i) {
+    for (int i = lane; i < e; i += 64) {
       row += hist[i];
       tile += (hist[i] + tile_rows - 1) / tile_rows;
     }
-    sh_row = row;
-    sh_tile = tile;
-    group_end[e] = row + hist[e];
-    if (e == E - 1) *n_tiles = min(max_tiles, tile + (hist[e] + tile_rows - 1) / tile_rows);
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) {
+      row += __shfl_xor(row, d, MSA_WAVE);
+      tile += __shfl_xor(tile, d, MSA_WAVE);
+    }
+    if (lane == 0) {
+      sh_row = row;
+      sh_tile = tile;
+      group_end[e] = row + hist[e];
+      if (e == E - 1) *n_tiles = min(max_tiles, tile + (hist[e] + tile_rows - 1) / tile_rows);
+    }
   }
   __syncthreads();
   const int mine = hist[e], row0 = sh_row, tile0 = sh_tile;
-  for (int t = tid; t < (mine + tile_rows - 1) / tile_rows; t += 256)
+  for (int t = tid; t < (mine + tile_rows - 1) / tile_rows; t += MP_THREADS)
     if (tile0 + t < max_tiles) {
       tile_group[tile0 + t] = e;
       tile_row[tile0 + t] = row0 + t * tile_rows;
     }
   int at = row0;
-  for (int p0 = 0; p0 < P; p0 += 256) {
-    const int p = p0 + tid;
-    const bool hit = p < P && ids[p] == e;
-    const unsigned long long b = __ballot(hit);
-    if (lane == 0) wcount[wave] = __popcll(b);
-    __syncthreads();
-    int before = at + __popcll(b & ((1ull << lane) - 1));
-    int total = 0;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      if (w < wave) before += wcount[w];
-      total += wcount[w];
+  for (int w = 0; w < wave; ++w) at += wcount[w];
+  walk([&](int p, int id) {
+    const unsigned long long b = __ballot(id == e);
+    if (id == e) {
+      const int to = at + __popcll(b & ((1ull << lane) - 1));
+      perm[to] = p;
+      inverse[p] = to;
     }
-    if (hit) {
-      perm[before] = p;
-      inverse[p] = before;
-    }
-    at += total;
-    __syncthreads();
-  }
+    at += __popcll(b);
+  });
 }
 
 }  // namespace
@@ -173,7 +192,7 @@ extern "C" int msa_moe_plan(const int32_t* ids, int P, int E, int tile_rows, int
                   max_tiles >= P / tile_rows + (E < P ? E : P),
               MSA_ERR_INVALID_ARG, "%s: P=%d E=%d tile_rows=%d max_tiles=%d", name, P, E, tile_rows,
               max_tiles);
-  hipLaunchKernelGGL(moe_plan_kernel, dim3(E), dim3(256), 0, (hipStream_t)stream, ids, P, E,
+  hipLaunchKernelGGL(moe_plan_kernel, dim3(E), dim3(MP_THREADS), 0, (hipStream_t)stream, ids, P, E,
                      tile_rows, perm, inverse, group_end, tile_group, tile_row, n_tiles, max_tiles);
   MSA_CHECK_LAUNCH(name);
   return MSA_OK;

@@ -421,6 +421,27 @@ def test_route_and_plan(E, groups, keep, top):
         assert list(zip(tg.cpu().tolist(), tr.cpu().tolist()))[:len(tiles)] == tiles
 
 
+@pytest.mark.parametrize("P,E", [(1, 3), (64, 2), (1025, 512), (8192, 7), (8256, 64), (48304, 64)])
+def test_plan_of_many_pairs(P, E):
+    """Runs of pairs per wave of one load, of several and of a few left over; waves without any."""
+    lib = _capi.load_hybrid()
+    flat = torch.randint(0, E, (P,), generator=gen(P))
+    rows, n_max = 256, P // 256 + min(E, P)
+    ids = flat.int().cuda()
+    perm, inv = (torch.full((P,), -1, dtype=torch.int32, device="cuda") for _ in range(2))
+    end = torch.zeros(E, dtype=torch.int32, device="cuda")
+    tg, tr = (torch.full((n_max,), -1, dtype=torch.int32, device="cuda") for _ in range(2))
+    n = torch.zeros(1, dtype=torch.int32, device="cuda")
+    check(lib.msa_moe_plan(ptr(ids), P, E, rows, ptr(perm), ptr(inv), ptr(end), ptr(tg), ptr(tr), ptr(n), n_max,
+                           _capi.stream_ptr()), lib)
+    order, counts = torch.sort(flat, stable=True).indices, torch.bincount(flat, minlength=E)
+    assert torch.equal(perm.cpu().long(), order)
+    assert torch.equal(inv.cpu().long()[order], torch.arange(P))
+    assert torch.equal(end.cpu().long(), counts.cumsum(0))
+    tiles = [(e, int(counts[:e].sum()) + r) for e in range(E) for r in range(0, int(counts[e]), rows)]
+    assert list(zip(tg.cpu().tolist(), tr.cpu().tolist()))[:int(n)] == tiles
+
+
 @pytest.mark.parametrize("hd", [32, 64, 96, 128, 192, 256])
 @pytest.mark.parametrize("T,pos0", [(1, 0), (17, 3), (64, 64), (130, 0), (33, 400), (300, 100)])
 def test_flash_attention(hd, T, pos0):
