@@ -64,7 +64,7 @@ extern "C" int msa_linear_bf16(const void* x, const void* W, void* y, float* y32
 }
 
 extern "C" int msa_linear_bf16_splits(int64_t M, int N, int K, int packed) {
-  return packed ? pick_splits(M, N, K, 2) : pick_row_splits(M, N, K);
+  return packed ? pick_splits(M, N, K, 2) : pick_row_splits_f32(M, N, K);
 }
 
 extern "C" int msa_linear_partial_bf16(const void* x, const void* W, float* part, int64_t M, int N,

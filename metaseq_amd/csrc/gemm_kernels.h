@@ -2129,6 +2129,21 @@ int pick_row_splits(int64_t M, int N, int K) {
   return best;
 }
 
+// The same for sums that leave as fp32 from any width of tile (bf16): also two slices of prompts' products whose
+// 256 x 256 tiles fill half of the chip or less, priced with what the second slice costs to write and read (5
+// TB/s).  1500 x 4096 x 16384: one slice of 256 x 128 tiles 194 us, two of 256 x 256 165 and 5 in the tail; 1500 x
+// 4096 x 4096 stays at one, 54 against 53 and 5.
+int pick_row_splits_f32(int64_t M, int N, int K) {
+  const int few = pick_row_splits(M, N, K);
+  if (few > 1 || M < TQ_BM || N % 16 || K % 128 || K < 1024) return few;
+  const int64_t rows = (M + TQ_BM - 1) / TQ_BM, cols8 = (N + 255) / 256, cols4 = (N + 127) / 128;
+  auto cost = [&](int S) {
+    const double rounds = fmin(quad_cost(rows * cols8 * S), quad_rounds(rows * cols4 * S) * TQ_COST_4);
+    return rounds * TQ_ROUND_US * K / S + (S - 1) * (double)M * N * 8 / 5e6;
+  };
+  return rows * cols8 * 2 <= num_cus() && cost(2) < 0.95 * cost(1) ? 2 : 1;
+}
+
 template <bool W8, int MODE>
 void launch_tiled(const void* x, const void* W, const void* scales, int64_t M, int N, int K,
                   const Epilogue& epi, hipStream_t s) {

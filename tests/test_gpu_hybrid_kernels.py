@@ -107,6 +107,19 @@ def test_linear_partial_bf16_wide_panels(M, N):
         close(part.sum(0).cpu(), ref.cpu(), 1e-5, "partial sums, S=%d" % S)
 
 
+@pytest.mark.parametrize("M,N,K", [(700, 4096, 2048), (2048, 4096, 8192), (1500, 4096, 16384)])
+def test_linear_partial_bf16_in_two_slices(M, N, K):
+    """Prompts whose tiles fill half of the chip or less: two slices are suggested, and sum to the product."""
+    lib = _capi.load_hybrid()
+    g = torch.Generator("cuda").manual_seed(M)
+    x = torch.randn(M, K, generator=g, device="cuda").to(BF16)
+    w = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).to(BF16)
+    assert lib.msa_linear_bf16_splits(M, N, K, 0) == 2 and lib.msa_linear_bf16_splits(M, N, K - 64, 0) == 1
+    part = torch.full((2, M, N), float("nan"), device="cuda")
+    check(lib.msa_linear_partial_bf16(ptr(x), ptr(pack_tiles(w)), ptr(part), M, N, K, 2, 0, _capi.stream_ptr()), lib)
+    close(part.sum(0).cpu(), (x.float() @ w.float().t()).cpu(), 1e-5, "two slices")
+
+
 @pytest.mark.parametrize("M,N", [(1500, 6032), (1500, 6912), (2305, 7168), (3000, 7680)])
 def test_linear_bf16_pieces(M, N):
     """A few tiles past whole rounds, cut in four or in two: sums of one and two slices (288 and 324 tiles of
