@@ -16,7 +16,7 @@
 // dots, a sum over lanes and the update takes 500 cycles per token whatever the machine has idle; a
 // chunk's chain takes 2800 (3800 with decays per channel, which are multiplied up while staging) per sixteen.
 // Measured, both kernels against the scan, 32 heads of 128 x 128: one segment of 1500 tokens 132 us against 368
-// (decays per channel 184 against 370), 8 x 1024 tokens 300 against 839 (332 against 1018).
+// (decays per channel 184 against 370), 8 x 1024 tokens 309 against 840 (329 against 1040).
 #include <math.h>
 
 #include <type_traits>
