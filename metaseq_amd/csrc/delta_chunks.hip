@@ -37,6 +37,8 @@ constexpr int DC_T = 0, DC_A = 256, DC_FK = 512, DC_FQ = 528, DC_FU = 544, DC_GC
 // (DC_GC holds sixteen copies: one address for all lanes would be a scalar load, whose latency every LDS
 // barrier waits for)
 
+__device__ __forceinline__ bool finite(float v) { return fabsf(v) <= 3.4028234663852886e38f; }
+
 // records of a segment start here: chunks are counted from each segment's own start, and
 // ceil(n / 16) <= floor((first + n) / 16) - floor(first / 16) + 1
 __device__ __forceinline__ int64_t record_of(int first, int seg, int chunk, int heads, int h) {
@@ -187,13 +189,21 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(
       x[i] = i < lane ? 0.f : beta[i] * ((i == lane ? 1.f : 0.f) - fk[i] * d);
       rec[DC_T + i * DC_TOK + lane] = x[i];
     });
+    // A row of T that is not finite (a beta, decay or key that is not) would reach the chunk's earlier tokens as a U
+    // that is 0 x NaN in A U.  Its factor of K' S0 says so: right_hand_side() takes every column out from there on.
+    int bad = DC_TOK;
+#pragma unroll
+    for (int i = DC_TOK - 1; i >= 0; --i)
+      if (!finite(x[i])) bad = i;
+#pragma unroll
+    for (int d = 1; d < DC_TOK; d *= 2) bad = min(bad, __shfl_xor(bad, d, MSA_WAVE));
     float before = 1.f, after = 1.f;
     if constexpr (!CH) {
 #pragma unroll
       for (int i = 0; i < DC_TOK; ++i) (i <= lane ? before : after) *= gs[i];
       rec[DC_GC + lane] = before * after;
     }
-    rec[DC_FK + lane] = fk[lane] * before;
+    rec[DC_FK + lane] = lane == bad ? __builtin_nanf("") : fk[lane] * before;
     rec[DC_FQ + lane] = fq[lane] * before;
     rec[DC_FU + lane] = fk[lane] * after;
   }
@@ -344,7 +354,6 @@ __device__ __forceinline__ float4_t decayed_plus(float4_t s, float4_t g, float4_
   for (int r = 0; r < 4; ++r) s[r] = fmaf(s[r], g[r], add[r]);
   return s;
 }
-__device__ __forceinline__ bool finite(float v) { return fabsf(v) <= 3.4028234663852886e38f; }
 
 // A lane's part of a record: tokens 4 lg .., and row lm of T
 struct Factors {

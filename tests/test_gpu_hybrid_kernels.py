@@ -723,6 +723,49 @@ def test_delta_chunks_keep_a_nan_from_earlier_tokens(heads, channels):
     assert float((scan - chunks)[fine].abs().max()) <= 2e-6 * float(scan[fine].abs().max())
     del alive
 
+def _scan_and_chunks(qkv, ba, decays, state, heads, dp, vp, channels, segments=None):
+    """Outputs and state of the scan and of the chunks over the same inputs."""
+    lib = _capi.load_hybrid()
+    M, C = qkv.shape
+    b, alive = _batch(segments or [(0, 12, M)], M)
+    out = []
+    for chunked in (False, True):
+        qd, bd, dd, sd = qkv.cuda(), ba.cuda(), decays.cuda(), state.cuda()
+        o, rd = torch.zeros(M, heads * vp, device="cuda"), torch.ones(heads, device="cuda")
+        a = _capi.DeltaArgs()
+        a.dtype, a.heads, a.kv_heads, a.dim, a.dp, a.vp = int(qkv.dtype == F32), heads, heads, dp, dp, vp
+        a.qkv, a.ld, a.ba, a.ldba, a.state, a.o = ptr(qd), C, ptr(bd), ba.shape[1], ptr(sd), ptr(o)
+        if channels:
+            a.decay = ptr(dd)
+        else:
+            a.decay_rate, a.dt_bias = ptr(rd), ptr(rd)
+        if chunked:
+            scratch = torch.empty(lib.msa_delta_scratch_floats(ctypes.byref(a), ctypes.byref(b)), device="cuda")
+            a.scratch, a.scratch_floats = ptr(scratch), scratch.numel()
+        check(lib.msa_delta_scan(ctypes.byref(a), ctypes.byref(b), _capi.stream_ptr()), lib)
+        out.append((o.cpu(), sd.cpu()))
+    del alive
+    return out
+
+
+@pytest.mark.parametrize("channels", [False, True])
+@pytest.mark.parametrize("heads", [3, 64])
+@pytest.mark.parametrize("bad", [37, 111])
+def test_delta_chunks_keep_a_nan_of_the_gates_from_earlier_tokens(bad, heads, channels):
+    """A beta that is NaN (head 0), or a decay (head 1), spoils its head from its token on and nothing else."""
+    g, M, dp, vp = gen(4), 112, 32, 128
+    qkv = torch.randn(M, 2 * heads * dp + heads * vp, generator=g).to(BF16)
+    ba, decays = torch.randn(M, 2 * heads, generator=g), torch.rand(M, heads, dp, generator=g)
+    ba[bad, 0] = ba[bad, heads + 1] = decays[bad, 1] = float("nan")
+    (scan, s_scan), (chunks, s_chunks) = _scan_and_chunks(qkv, ba, decays, torch.randn(1, heads, vp, dp, generator=g),
+                                                          heads, dp, vp, channels)
+    fine = torch.isfinite(scan)
+    assert bool(fine[:bad].all()) and not bool(fine[bad:, :2 * vp].any()) and bool(fine[:, 2 * vp:].all())
+    assert torch.equal(torch.isfinite(chunks), fine)
+    assert torch.equal(torch.isfinite(s_chunks), torch.isfinite(s_scan))
+    assert float((scan - chunks)[fine].abs().max()) <= 2e-6 * float(scan[fine].abs().max())
+
+
 def test_selection_over_fp32_logits():
     """The fp32 forms of selection, scoring and sampling agree with plain PyTorch, at row strides
     and vocabulary sizes that are no multiple of 8."""
