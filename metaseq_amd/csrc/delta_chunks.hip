@@ -29,11 +29,14 @@ namespace {
 
 constexpr int DC_TOK = 16;
 constexpr int DC_WIDE = 128;  // workgroups of several column tiles from which on they take over
-// A record: T and A (16 x 16, row-major), then per token the factors that are one number for all channels,
-// which the loops below apply to 16 x 16 results and not to the operands: of K' S0 (1 / |k|), Q' S0
-// (scale / |q|) and U (1 / |k|), each times the token's product of decays where a head has one decay, and that
-// product over the chunk.  Past the segment's end the factors are 0.
-constexpr int DC_T = 0, DC_A = 256, DC_FK = 512, DC_FQ = 528, DC_FU = 544, DC_GC = 560, DC_REC = 576;
+// A record: T and A (16 x 16, row-major), then per token the factors that are one number for all channels.
+// The norms are divided out in two steps.  Operands are multiplied by a power of two (SK of k, SQ of q), which is exact
+// and brings them near unit length, so that no product overflows that the scan's unit vectors would not; a vector whose
+// squared norm overflows has the factor 0, as in the scan.  The rest, between 1 and 2, the loops below apply to 16 x 16
+// results: of K' S0 (1 / |k|), Q' S0 (scale / |q|) and U (1 / |k|), each times the token's product of decays where a
+// head has one decay, and that product over the chunk.  Past the segment's end the factors are 0.
+constexpr int DC_T = 0, DC_A = 256, DC_FK = 512, DC_FQ = 528, DC_FU = 544, DC_GC = 560, DC_SK = 576, DC_SQ = 592,
+              DC_REC = 608;
 // (DC_GC holds sixteen copies: one address for all lanes would be a scalar load, whose latency every LDS
 // barrier waits for)
 
@@ -84,10 +87,11 @@ __device__ __forceinline__ float transposed_sums(float (&v)[64], int lane) {
   return v[0];
 }
 
-// Place of a sum in the order the loops below form them: per token j first |k_j|^2, q_j . k_j and |q_j|^2, then
-// for every later token i the sums of L_ij and A_ij.
-constexpr int sum_at(int j) { return 34 * j - j * j; }
-constexpr int DC_SUMS = sum_at(DC_TOK);  // 288
+// Place of a sum in the order the loops below form them: per token j first q_j . k_j, then for every later token i
+// the sums of L_ij and A_ij.
+constexpr int sum_at(int j) { return 32 * j - j * j; }
+constexpr int DC_SUMS = sum_at(DC_TOK);  // 256
+static_assert(DC_SUMS % 64 == 0, "whole groups of sums");
 
 // One wave per (chunk, head).  Bound: the vector ALU (for 128 channels some 800 multiply-adds and
 // 700 steps of the sums per chunk and lane).  The decays between two tokens are multiplied up as j's row moves from token to token.
@@ -98,7 +102,7 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(
     const float* __restrict__ decay, int heads, int kv_heads, float q_scale, float* __restrict__ records,
     const int32_t* __restrict__ seg_start, const int32_t* __restrict__ seg_pos) {
   constexpr int CE = (DP + 63) / 64;  // channels per lane
-  __shared__ float sums[4][(DC_SUMS + 63) / 64 * 64], tok[4][4][DC_TOK];
+  __shared__ float sums[4][DC_SUMS], tok[4][6][DC_TOK];  // tok: beta, rest of 1 / |k| and of scale / |q|, decay, SK, SQ
   const int s = blockIdx.z, t0 = blockIdx.x * DC_TOK;
   const int first = seg_start[s], n = seg_start[s + 1] - first;
   if (t0 >= n || seg_pos[s] < 0) return;
@@ -124,10 +128,33 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(
       }
     }
   }
+  auto dot = [&](const float (&a)[CE], const float (&b)[CE]) {
+    float d = a[0] * b[0];
+#pragma unroll
+    for (int e = 1; e < CE; ++e) d = fmaf(a[e], b[e], d);
+    return d;
+  };
+  float v[64];
+#pragma unroll
+  for (int t = 0; t < DC_TOK; ++t) {
+    v[t] = dot(k[t], k[t]);
+    v[DC_TOK + t] = dot(q[t], q[t]);
+    v[2 * DC_TOK + t] = v[3 * DC_TOK + t] = 0.f;
+  }
+  const float square = transposed_sums(v, lane);  // of k (lanes 0 .. 15) or q (16 .. 31)
+  if (lane < 2 * DC_TOK) {
+    // (the few factors per token in 64 bits: one rounding each, and no time that shows beside the sums)
+    const int t = lane & 15;
+    const bool of_q = lane >> 4, in = t0 + t < n;
+    const double norm = sqrt((double)square + 1e-6), scale = of_q ? q_scale : 1.f;
+    int e = 0;
+    const double rest = isfinite(norm) ? frexp(norm, &e) : norm;
+    tok[wave][of_q ? 5 : 4][t] = in && isfinite(norm) ? ldexpf(1.f, -e) : 0.f;
+    tok[wave][of_q ? 2 : 1][t] = in ? (float)(scale / rest) : 0.f;
+  }
   if (lane < DC_TOK) {
     const bool in = t0 + lane < n;
     const float* z = ba + (int64_t)(first + min(t0 + lane, n - 1)) * ldba;
-    // (the few factors per token in 64 bits: one rounding each, and no time that shows beside the sums)
     tok[wave][0][lane] = in ? (float)(1.0 / (1.0 + exp(-(double)z[h]))) : 0.f;
     if (!CH) tok[wave][3][lane] = in ? decay_of(z[heads + h] + dt_bias[h], decay_rate[h]) : 1.f;
   }
@@ -137,23 +164,21 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(
 #pragma unroll
     for (int t = 0; t < DC_TOK; ++t) gs[t] = tok[wave][3][t];
   }
-  float v[64];
+#pragma unroll
+  for (int t = 0; t < DC_TOK; ++t)
+#pragma unroll
+    for (int e = 0; e < CE; ++e) {
+      k[t][e] *= tok[wave][4][t];
+      q[t][e] *= tok[wave][5][t];
+    }
   auto emit = [&](auto at, float x) {
     constexpr int A = decltype(at)::value;
     v[A & 63] = x;
     if constexpr ((A & 63) == 63) sums[wave][A - 63 + lane] = transposed_sums(v, lane);
   };
-  auto dot = [&](const float (&a)[CE], const float (&b)[CE]) {
-    float d = a[0] * b[0];
-#pragma unroll
-    for (int e = 1; e < CE; ++e) d = fmaf(a[e], b[e], d);
-    return d;
-  };
   each<DC_TOK>([&](auto jc) {
     constexpr int j = decltype(jc)::value, at = sum_at(j);
-    emit(std::integral_constant<int, at>{}, dot(k[j], k[j]));
-    emit(std::integral_constant<int, at + 1>{}, dot(q[j], k[j]));
-    emit(std::integral_constant<int, at + 2>{}, dot(q[j], q[j]));
+    emit(std::integral_constant<int, at>{}, dot(q[j], k[j]));
     float w[CE];
 #pragma unroll
     for (int e = 0; e < CE; ++e) w[e] = k[j][e];
@@ -161,21 +186,12 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(
       constexpr int i = j + 1 + decltype(ic)::value;
 #pragma unroll
       for (int e = 0; e < CE; ++e) w[e] *= CH ? g[CH ? i : 0][e] : gs[CH ? 0 : i];
-      emit(std::integral_constant<int, at + 1 + 2 * (i - j)>{}, dot(k[i], w));
-      emit(std::integral_constant<int, at + 2 + 2 * (i - j)>{}, dot(q[i], w));
+      emit(std::integral_constant<int, at + 2 * (i - j) - 1>{}, dot(k[i], w));
+      emit(std::integral_constant<int, at + 2 * (i - j)>{}, dot(q[i], w));
     });
   });
-  constexpr int rest = (DC_SUMS + 63) / 64 * 64 - DC_SUMS;
-  each<rest>([&](auto c) { emit(std::integral_constant<int, DC_SUMS + decltype(c)::value>{}, 0.f); });
   __syncthreads();
   const float* sm = sums[wave];
-  if (lane < DC_TOK) {
-    const bool in = t0 + lane < n;
-    const int a = 34 * lane - lane * lane;
-    tok[wave][1][lane] = in ? (float)(1.0 / sqrt((double)sm[a] + 1e-6)) : 0.f;
-    tok[wave][2][lane] = in ? (float)(q_scale / sqrt((double)sm[a + 2] + 1e-6)) : 0.f;
-  }
-  __syncthreads();
   if (h_own >= heads) return;
   float* rec = records + record_of(first, s, blockIdx.x, heads, h);
   const float *beta = tok[wave][0], *fk = tok[wave][1], *fq = tok[wave][2];
@@ -185,7 +201,7 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(
       constexpr int i = decltype(ic)::value;
       float d = 0.f;
 #pragma unroll
-      for (int j = 0; j < i; ++j) d = fmaf(sm[34 * j - j * j + 1 + 2 * (i - j)] * fk[j], x[j], d);
+      for (int j = 0; j < i; ++j) d = fmaf(sm[sum_at(j) + 2 * (i - j) - 1] * fk[j], x[j], d);
       x[i] = i < lane ? 0.f : beta[i] * ((i == lane ? 1.f : 0.f) - fk[i] * d);
       rec[DC_T + i * DC_TOK + lane] = x[i];
     });
@@ -206,12 +222,13 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(
     rec[DC_FK + lane] = lane == bad ? __builtin_nanf("") : fk[lane] * before;
     rec[DC_FQ + lane] = fq[lane] * before;
     rec[DC_FU + lane] = fk[lane] * after;
+    rec[DC_SK + lane] = tok[wave][4][lane];
+    rec[DC_SQ + lane] = tok[wave][5][lane];
   }
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const int i = (lane >> 4) * 4 + e, j = lane & 15;
-    const int a = 34 * j - j * j;
-    const float raw = sm[i == j ? a + 1 : i > j ? a + 2 + 2 * (i - j) : 0];
+    const float raw = sm[i >= j ? sum_at(j) + 2 * (i - j) : 0];
     rec[DC_A + i * DC_TOK + j] = i >= j ? fq[i] * fk[j] * raw : 0.f;
   }
 }
@@ -238,7 +255,7 @@ struct Operands {
 // the chunk's tokens and multiplies the decays up; the lane 32 away has the other half.
 // Chunks are requested two ahead.  The loops of these kernels take chunks in pairs and without conditions
 // around their loads, so that each wait is for the oldest chunk alone; an odd number of chunks is made even
-// by one past the end, whose factors are set to 0 and its decays to 1, which changes nothing.
+// by one past the end, whose k, q and U are set to 0 and its decays to 1, which changes nothing.
 template <typename T, int DP, bool CH>
 struct Stager {
   typedef T t4 __attribute__((ext_vector_type(4), aligned(8)));
@@ -248,16 +265,17 @@ struct Stager {
     t4 x[CH ? 1 : 4];       // one decay per head: 8 of k, 8 of q
     t2 y[CH ? 8 : 1];
     f2 g[CH ? 8 : 1];
+    float f[CH ? 8 : 2];    // SK or SQ of the thread's tokens; one decay per head: SK and SQ of its token
   };
   const T *ksrc, *qsrc;      // uniform: the head's first channel of the segment's first token
-  const float* dsrc;
-  int64_t ld, ldd;
+  const float *dsrc, *fsrc;
+  int64_t ld, ldd, ldf;
   int n, t, half;
   unsigned at;               // first channel of the thread
   bool is_k, live;
 
   __device__ Stager(int t_, const T* rows, int64_t ld_, const float* decay, int first, int heads, int kv_heads,
-                    int h, int n_) {
+                    int h, int n_, const float* rec0) {
     t = t_;
     n = n_;
     ld = ld_;
@@ -272,9 +290,18 @@ struct Stager {
     const int pair = (wave & 1) * 32 + (t & 31);
     live = CH ? pair < DP / 2 : t < 2 * DP;
     at = CH ? min(pair, DP / 2 - 1) * 2 : min(t, 2 * DP - 1) % (DP / 8) * 8;
+    ldf = (int64_t)heads * DC_REC;
+    fsrc = rec0 + (CH ? (is_k ? DC_SK : DC_SQ) + half * 8 : DC_SK + min(t, 2 * DP - 1) / (DP / 8));
   }
   __device__ __forceinline__ void fetch(Raw& a, int c) const {
+    const float* fac = fsrc + min(c, (n - 1) / DC_TOK) * ldf;
     if constexpr (CH) {
+#pragma unroll
+      for (int i = 0; i < 8; i += 4) {
+        const float4_t f = *reinterpret_cast<const float4_t*>(fac + i);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) a.f[CH ? i + j : 0] = f[j];
+      }
       const T* src = is_k ? ksrc : qsrc;
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
@@ -288,17 +315,22 @@ struct Stager {
       a.x[1] = *reinterpret_cast<const t4*>(ksrc + row + 4);
       a.x[2] = *reinterpret_cast<const t4*>(qsrc + row);
       a.x[3] = *reinterpret_cast<const t4*>(qsrc + row + 4);
+      a.f[0] = fac[0];
+      a.f[1] = fac[DC_SQ - DC_SK];
     }
   }
   __device__ __forceinline__ void stage(Operands<DP, CH>& L, const Raw& a, int c) const {
     const int b = c & 1;
+    const bool past = c * DC_TOK >= n;
     if constexpr (!CH) {
       if (!live) return;
       const int tok = t / (DP / 8);
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < 4; ++i) {
+        const float f = past ? 0.f : a.f[i >> 1];
         *reinterpret_cast<float4_t*>(&(i < 2 ? L.k : L.q)[b][tok][at + (i & 1) * 4]) =
-            float4_t{(float)a.x[i][0], (float)a.x[i][1], (float)a.x[i][2], (float)a.x[i][3]};
+            float4_t{(float)a.x[i][0], (float)a.x[i][1], (float)a.x[i][2], (float)a.x[i][3]} * f;
+      }
       return;
     }
     f2 g[8], p = {1.f, 1.f};
@@ -316,7 +348,7 @@ struct Stager {
     f2 x[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      x[i] = f2{(float)a.y[CH ? i : 0][0], (float)a.y[CH ? i : 0][1]};
+      x[i] = f2{(float)a.y[CH ? i : 0][0], (float)a.y[CH ? i : 0][1]} * (past ? 0.f : a.f[CH ? i : 0]);
       m[0] *= g[i][0], m[1] *= g[i][1];
       *reinterpret_cast<f2*>(&(is_k ? L.k : L.q)[b][tok + i][at]) = f2{x[i][0] * m[0], x[i][1] * m[1]};
     }
@@ -367,8 +399,11 @@ struct Factors {
     u = *reinterpret_cast<const float4_t*>(rec + DC_FU + lg * 4);
     gc = ch ? 1.f : rec[DC_GC + lm];
   }
-  __device__ __forceinline__ void end(int c, int nch) {  // a chunk past the end changes nothing
-    if (c >= nch) u = float4_t{0.f, 0.f, 0.f, 0.f}, gc = 1.f;
+  // U on its way to the state; a chunk past the end changes nothing, whatever its U is
+  __device__ __forceinline__ void finish(float4_t& x, int bad, int lg, int c, int nch) {
+    if (c >= nch) gc = 1.f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) x[r] = c >= nch ? 0.f : lg * 4 + r >= bad ? __builtin_nanf("") : x[r] * u[r];
   }
 };
 
@@ -408,8 +443,9 @@ struct FewLds {
 // Few segments: a workgroup owns one segment, one head and 16 of its columns for all of the segment's chunks.
 // Waves 0 .. 3 hold the state, a quarter of its rows each, as MFMA accumulators (a lane: four rows of one
 // column), which are the B operands of the next chunk's products as they lie; they sum K' S0 through
-// LDS, form U redundantly and update their rows.  Waves 4 .. 7 run beside them: they stage the next chunk and
-// finish the previous chunk's outputs.  Two barriers per chunk.
+// LDS, form U redundantly and update their rows.  Waves 4 .. 7 run beside them, between the two barriers of a chunk:
+// they finish the previous chunk's outputs and stage the next chunk (before the first barrier, beside the short
+// product K' S0, 1500 tokens took 124 us, here 115).
 template <typename T, int DP, bool CH>
 __global__ __launch_bounds__(512) void delta_chunk_kernel(
     const T* __restrict__ qkv, int64_t ld, const float* __restrict__ decay, int heads, int kv_heads, int vp,
@@ -483,9 +519,7 @@ __global__ __launch_bounds__(512) void delta_chunk_kernel(
         L.u[b][lane] = u;
         if (lane < 16) L.bad[b][lane] = bad;
       }
-      a.f.end(c, nch);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) u[r] = lg * 4 + r >= bad ? __builtin_nanf("") : u[r] * a.f.u[r];
+      a.f.finish(u, bad, lg, c, nch);
       const float gc = a.f.gc;
       fetch(a, c + 2);
       float4_t kh[TPW], us[TPW], g[TPW], add[TPW];
@@ -519,7 +553,7 @@ __global__ __launch_bounds__(512) void delta_chunk_kernel(
 
   typedef Stager<T, DP, CH> St;
   const int ht = tid - 256;
-  const St stager(ht, rows, ld, decay, first, heads, kv_heads, h, n);
+  const St stager(ht, rows, ld, decay, first, heads, kv_heads, h, n, rec0);
   struct Raw {
     typename St::Raw r;
     float a;  // element ht of A
@@ -553,10 +587,10 @@ __global__ __launch_bounds__(512) void delta_chunk_kernel(
   fetch(raw[0], 2);
   lds_barrier();
   auto beside = [&](Raw& x, int c) {  // x holds chunk c + 1
-    stage(x, c + 1);
     lds_barrier();  // A
-    fetch(x, c + 3);
     finish(c - 1);
+    stage(x, c + 1);
+    fetch(x, c + 3);
     lds_barrier();  // B
   };
   for (int c = 0; c < nch; c += 2) {
@@ -593,7 +627,7 @@ __global__ __launch_bounds__((CT + 4) * 64) void delta_chunk_wide_kernel(
   const int64_t rec_step = (int64_t)heads * DC_REC;
   if (wave >= CT) {
     typedef Stager<T, DP, CH> St;
-    const St stager(tid - CT * 64, rows, ld, decay, first, heads, kv_heads, h, n);
+    const St stager(tid - CT * 64, rows, ld, decay, first, heads, kv_heads, h, n, rec0);
     typename St::Raw raw[2];
     stager.fetch(raw[0], 0);
     stager.fetch(raw[1], 1);
@@ -601,7 +635,7 @@ __global__ __launch_bounds__((CT + 4) * 64) void delta_chunk_wide_kernel(
     stager.fetch(raw[0], 2);
     lds_barrier();
     auto beside = [&](typename St::Raw& x, int c) {
-      stager.stage(L, x, c + 1);  // (past the last chunk: zeros that nothing, or a surplus chunk, reads)
+      stager.stage(L, x, c + 1);  // (past the last chunk: zeros, which a surplus chunk reads)
       stager.fetch(x, c + 3);
       lds_barrier();
     };
@@ -654,12 +688,10 @@ __global__ __launch_bounds__((CT + 4) * 64) void delta_chunk_wide_kernel(
     for (int r = 0; r < 4; ++r)
       if (lg * 4 + r >= bad) u[r] = 0.f;
     y = mfma4(x.a, u, y);
-    x.f.end(c, nch);
+    x.f.finish(u, bad, lg, c, nch);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      u[r] = lg * 4 + r >= bad ? __builtin_nanf("") : u[r] * x.f.u[r];
+    for (int r = 0; r < 4; ++r)
       if (lg * 4 + r >= bad) y[r] = __builtin_nanf("");
-    }
     const float gc = x.f.gc;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {

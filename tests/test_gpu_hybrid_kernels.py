@@ -766,6 +766,50 @@ def test_delta_chunks_keep_a_nan_of_the_gates_from_earlier_tokens(bad, heads, ch
     assert float((scan - chunks)[fine].abs().max()) <= 2e-6 * float(scan[fine].abs().max())
 
 
+@pytest.mark.parametrize("channels", [False, True])
+@pytest.mark.parametrize("heads", [3, 64])
+@pytest.mark.parametrize("M", [112, 121])
+def test_delta_chunks_of_huge_and_tiny_keys(M, heads, channels):
+    """Keys and queries far from unit length, values and a state of up to 1e25: products of the raw vectors would
+    overflow where the scan, which divides by the norms first, stays finite.  Vectors whose squared norm itself
+    overflows count as zeros in both.  Seven and eight chunks; the last tokens are huge ones."""
+    g, dp, vp = gen(5), 64, 128
+    qk = torch.randn(M, 2 * heads, dp, generator=g)
+    qk *= 10.0 ** torch.randint(-3, 19, (M, 2 * heads, 1), generator=g)
+    qk[-1], qk[40] = 1e18 * torch.sign(qk[-1]), 3e25 * torch.sign(qk[40])
+    v = torch.randn(M, heads * vp, generator=g) * 10.0 ** torch.randint(0, 26, (1, heads * vp), generator=g)
+    qkv = torch.cat([qk.view(M, -1), v], dim=1)
+    ba, decays = torch.randn(M, 2 * heads, generator=g), torch.rand(M, heads, dp, generator=g) ** 0.25
+    state = torch.randn(1, heads, vp, dp, generator=g) * 10.0 ** torch.randint(0, 26, (vp, 1), generator=g)
+    unit = lambda t: t / torch.sqrt((t * t).sum(-1, keepdim=True) + 1e-6)
+    for x in (qkv, qkv.to(BF16)):
+        d = x.double()
+        q, k = (unit(t.view(M, heads, dp)) for t in (d[:, :heads * dp], d[:, heads * dp:2 * heads * dp]))
+        q, k, v = q * dp ** -0.5, k.clone(), d[:, 2 * heads * dp:].view(M, heads, vp)
+        q[40] = k[40] = 0.0
+        beta = torch.sigmoid(ba[:, :heads].double())
+        one = torch.exp(-torch.nn.functional.softplus(ba[:, heads:].double() + 1.0))
+        s, want = state[0].double(), []
+        size, most = s.norm(dim=-1), torch.zeros(heads, vp, dtype=torch.float64)  # of what is summed, per column
+        for m in range(M):
+            g = decays[m].double().unsqueeze(1) if channels else one[m].view(-1, 1, 1)
+            s = s * g
+            add = beta[m].unsqueeze(1) * (v[m] - (s * k[m].unsqueeze(1)).sum(-1))
+            s = s + add.unsqueeze(2) * k[m].unsqueeze(1)
+            want.append((s * q[m].unsqueeze(1)).sum(-1))
+            size = torch.maximum(torch.maximum(size * g.amax(-1), add.abs()), s.norm(dim=-1))
+            most = torch.maximum(most, size * dp ** -0.5)
+        want = torch.stack(want)
+        for o, end in _scan_and_chunks(x, ba, decays, state, heads, dp, vp, channels):
+            assert bool(torch.isfinite(o).all()) and bool(torch.isfinite(end).all()) and not bool(o[40].any())
+            off = float(((o.view(M, heads, vp).double() - want).abs().amax(0) / most).max())
+            end_off = float(((end[0].double() - s).norm(dim=-1) / size).max())
+            print(off, end_off, flush=True)
+            # sums of dp + 32 terms of random sign, rounded each: 10 * 2^-24 of what is summed, and three times that
+            # for the worst of thousands
+            assert off <= 30 * 2.0 ** -24 and end_off <= 30 * 2.0 ** -24, (off, end_off)
+
+
 def test_selection_over_fp32_logits():
     """The fp32 forms of selection, scoring and sampling agree with plain PyTorch, at row strides
     and vocabulary sizes that are no multiple of 8."""
