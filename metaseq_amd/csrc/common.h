@@ -151,6 +151,13 @@ __device__ __forceinline__ void lse_merge(float& m, float& s, float om, float os
   }
 }
 
+// A segment of no tokens leaves its state as it is; one that begins its sequence leaves zeros.  ``st``: the floats that
+// the workgroup owns, whole and in a row.
+__device__ __forceinline__ void empty_segment(float* st, int count, int pos) {
+  if (pos == 0)
+    for (int i = threadIdx.x; i < count; i += blockDim.x) st[i] = 0.f;
+}
+
 // Barrier of a workgroup for data exchanged through LDS: waits for this wave's LDS operations but, other
 // than __syncthreads(), not for its global loads, which stay in flight across it.
 __device__ __forceinline__ void lds_barrier() {

@@ -464,6 +464,7 @@ __global__ __launch_bounds__(512) void delta_chunk_kernel(
     for (int i = tid; i < n * 16; i += 512) out[(int64_t)(i >> 4) * heads * vp + (i & 15)] = 0.f;
     return;
   }
+  if (n <= 0) return empty_segment(state + (((int64_t)seg_slot[s] * heads + h) * vp + col0) * DP, 16 * DP, pos);
   const int nch = (n + DC_TOK - 1) / DC_TOK;
   const T* rows = qkv + (int64_t)first * ld;
   const float* rec0 = records + record_of(first, s, 0, heads, h);
@@ -621,6 +622,7 @@ __global__ __launch_bounds__((CT + 4) * 64) void delta_chunk_wide_kernel(
       o[(int64_t)(first + i / (CT * 16)) * heads * vp + h * vp + col0 + i % (CT * 16)] = 0.f;
     return;
   }
+  if (n <= 0) return empty_segment(state + (((int64_t)seg_slot[s] * heads + h) * vp + col0) * DP, CT * 16 * DP, pos);
   const int nch = (n + DC_TOK - 1) / DC_TOK;
   const T* rows = qkv + (int64_t)first * ld;
   const float* rec0 = records + record_of(first, s, 0, heads, h);

@@ -248,6 +248,7 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(
       o[(int64_t)(first + i / CW) * heads * vp + h * vp + col0 + i % CW] = 0.f;
     return;
   }
+  if (n <= 0) return empty_segment(state + (((int64_t)seg_slot[s] * heads + h) * vp + col0) * DP, CW * DP, pos);
   const int cl = tid / LPC, rl = tid % LPC;  // column of the workgroup's, row group
   float* st = state + (((int64_t)seg_slot[s] * heads + h) * vp + col0 + cl) * DP + rl * R;
   float S[R];

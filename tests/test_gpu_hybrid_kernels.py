@@ -768,6 +768,24 @@ def test_delta_chunks_keep_a_nan_of_the_gates_from_earlier_tokens(bad, heads, ch
 
 @pytest.mark.parametrize("channels", [False, True])
 @pytest.mark.parametrize("heads", [3, 64])
+def test_delta_segments_without_tokens(heads, channels):
+    """In front, between and behind others: they change nothing, but one that begins its sequence leaves a state of
+    zeros."""
+    g, M, dp, vp = gen(6), 160, 32, 128
+    qkv = torch.randn(M, 2 * heads * dp + heads * vp, generator=g).to(BF16)
+    ba, decays = torch.randn(M, 2 * heads, generator=g), torch.rand(M, heads, dp, generator=g)
+    state = torch.randn(6, heads, vp, dp, generator=g)
+    run = lambda segs: _scan_and_chunks(qkv, ba, decays, state, heads, dp, vp, channels, segs)
+    plain = run([(1, 12, 48), (4, 0, 112)])
+    gaps = run([(0, 7, 0), (1, 12, 48), (2, 0, 0), (4, 0, 112), (3, 5, 0), (5, 0, 0)])
+    for (o, s), (o2, s2) in zip(plain, gaps):
+        assert torch.equal(o, o2)
+        s[2] = s[5] = 0.0
+        assert torch.equal(s, s2)
+
+
+@pytest.mark.parametrize("channels", [False, True])
+@pytest.mark.parametrize("heads", [3, 64])
 @pytest.mark.parametrize("M", [112, 121])
 def test_delta_chunks_of_huge_and_tiny_keys(M, heads, channels):
     """Keys and queries far from unit length, values and a state of up to 1e25: products of the raw vectors would
