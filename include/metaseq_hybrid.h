@@ -176,12 +176,14 @@ typedef struct {
   const void* gate; int64_t ld_gate;   /* heads * vp columns, activation format */
   const float* w; float eps;           /* the output's norm over vdim, weight [vp] */
   void* out; int64_t ld_out; int out_mb;
-  float* scratch; int64_t scratch_floats;  /* msa_delta_scan: at least msa_delta_scratch_floats, or NULL */
 } msa_delta_args;
-/* Scratch with which msa_delta_scan takes sixteen tokens at a time on the matrix cores (fp32); 0 where it
- * goes token by token anyway (short segments, keys beyond 128), as it does without scratch. */
-int64_t msa_delta_scratch_floats(const msa_delta_args* a, const msa_batch* b);
 int msa_delta_scan(const msa_delta_args* a, const msa_batch* b, void* stream);
+/* The same with scratch of at least msa_delta_scratch_floats, with which it takes sixteen tokens at a time on the
+ * matrix cores (fp32); 0 where that does not pay (short segments) or does not exist (keys beyond 128): then it
+ * needs no scratch and goes token by token. */
+int64_t msa_delta_scratch_floats(const msa_delta_args* a, const msa_batch* b);
+int msa_delta_scan_chunks(const msa_delta_args* a, const msa_batch* b, float* scratch, int64_t scratch_floats,
+                          void* stream);
 /* out = rmsnorm over vdim of every head's o, times w, times silu(gate) or sigmoid(gate) (gate_act) */
 int msa_delta_output(const msa_delta_args* a, int M, void* stream);
 /* Both in one launch where every segment holds one token. */

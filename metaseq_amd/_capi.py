@@ -151,8 +151,7 @@ DeltaArgs = _struct(
     "DeltaArgs", "msa_delta_args", (c_int, "dtype heads kv_heads dim dp vdim vp gate_act"),
     (c_void_p, "qkv"), (c_int64, "ld"), (c_void_p, "ba"), (c_int, "ldba"),
     (c_void_p, "decay_rate dt_bias decay state o gate"), (c_int64, "ld_gate"), (c_void_p, "w"),
-    (c_float, "eps"), (c_void_p, "out"), (c_int64, "ld_out"), (c_int, "out_mb"),
-    (c_void_p, "scratch"), (c_int64, "scratch_floats"))
+    (c_float, "eps"), (c_void_p, "out"), (c_int64, "ld_out"), (c_int, "out_mb"))
 GroupedArgs = _struct(
     "GroupedArgs", "msa_grouped_args", (c_int, "dtype heads kv_heads hd vd chunk rot_dims rows"),
     (c_float, "scale"), (c_void_p, "inv_freq q k v"), (c_int64, "ld"),
@@ -203,6 +202,7 @@ HYBRID_SIGNATURES = {
     "msa_rglru_scan": [c_int, _P, _P, _P, _P, c_int64, _P, c_int64, _P, c_int, _P, _P, _P, c_int64,
                        c_int, _BP, _P],
     "msa_delta_scan": [ctypes.POINTER(DeltaArgs), _BP, _P],
+    "msa_delta_scan_chunks": [ctypes.POINTER(DeltaArgs), _BP, _P, c_int64, _P],
     "msa_delta_output": [ctypes.POINTER(DeltaArgs), c_int, _P],
     "msa_delta_step": [ctypes.POINTER(DeltaArgs), _BP, _P],
     "msa_grouped_rotate": [ctypes.POINTER(GroupedArgs), _BP, _P],

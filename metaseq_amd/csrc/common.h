@@ -50,7 +50,7 @@ int msa_launch_prefill_attention(const void* q, const void* Kc, const void* Vc,
 // routed products over 256-row tiles, bf16 (gemm_bf16.hip)
 bool msa_launch_group_quad(const msa_group_linear_args& a, hipStream_t stream);
 // the delta rule sixteen tokens at a time, for calls with scratch (delta_chunks.hip)
-int msa_launch_delta_chunks(const msa_delta_args& a, const msa_batch* b, hipStream_t stream);
+int msa_launch_delta_chunks(const msa_delta_args& a, const msa_batch* b, float* scratch, hipStream_t stream);
 int msa_launch_linear_post(const msa_linear_args& a, hipStream_t stream);
 
 #define MSA_REQUIRE(cond, code, ...) \

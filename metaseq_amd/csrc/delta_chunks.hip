@@ -721,20 +721,20 @@ __global__ __launch_bounds__((CT + 4) * 64) void delta_chunk_wide_kernel(
 }
 
 template <typename T, int DP, bool CH>
-int run_chunks(const msa_delta_args& a, const msa_batch* b, hipStream_t s) {
+int run_chunks(const msa_delta_args& a, const msa_batch* b, float* scratch, hipStream_t s) {
   const unsigned chunks = (unsigned)((b->max_count + DC_TOK - 1) / DC_TOK);
   hipLaunchKernelGGL((delta_prepare_kernel<T, DP, CH>), dim3(chunks, (a.heads + 3) / 4, b->nseg), dim3(256), 0,
                      s, (const T*)a.qkv, a.ld, a.ba, a.ldba, a.decay_rate, a.dt_bias, a.decay, a.heads,
-                     a.kv_heads, (float)pow((double)a.dim, -0.5), a.scratch, b->seg_start, b->seg_pos);
+                     a.kv_heads, (float)pow((double)a.dim, -0.5), scratch, b->seg_start, b->seg_pos);
 #define DC_RUN(KERNEL, COLS, THREADS, BYTES)                                                           \
   do {                                                                                                 \
     static std::atomic<uint64_t> raised{0};                                                            \
     if (!raise_lds((const void*)KERNEL, BYTES, raised)) {                                              \
-      msa_set_error("msa_delta_scan: %d bytes of LDS refused", BYTES);                                 \
+      msa_set_error("msa_delta_scan_chunks: %d bytes of LDS refused", BYTES);                                 \
       return MSA_ERR_HIP;                                                                              \
     }                                                                                                  \
     hipLaunchKernelGGL(KERNEL, dim3(a.vp / (COLS), a.heads, b->nseg), dim3(THREADS), BYTES, s,         \
-                       (const T*)a.qkv, a.ld, a.decay, a.heads, a.kv_heads, a.vp, a.state, a.scratch,  \
+                       (const T*)a.qkv, a.ld, a.decay, a.heads, a.kv_heads, a.vp, a.state, scratch,  \
                        a.o, b->seg_start, b->seg_slot, b->seg_pos);                                    \
   } while (0)
   const int64_t units = (int64_t)b->nseg * a.heads;
@@ -750,10 +750,10 @@ int run_chunks(const msa_delta_args& a, const msa_batch* b, hipStream_t s) {
 }
 
 template <typename T>
-int pick_chunks(const msa_delta_args& a, const msa_batch* b, hipStream_t s) {
+int pick_chunks(const msa_delta_args& a, const msa_batch* b, float* scratch, hipStream_t s) {
 #define DC_CASE(DP) \
   case DP:          \
-    return a.decay ? run_chunks<T, DP, true>(a, b, s) : run_chunks<T, DP, false>(a, b, s);
+    return a.decay ? run_chunks<T, DP, true>(a, b, scratch, s) : run_chunks<T, DP, false>(a, b, scratch, s);
   switch (a.dp) {
     DC_CASE(32)
     DC_CASE(64)
@@ -778,6 +778,6 @@ extern "C" int64_t msa_delta_scratch_floats(const msa_delta_args* a, const msa_b
   return ((int64_t)b->M / DC_TOK + b->nseg) * a->heads * DC_REC;
 }
 
-int msa_launch_delta_chunks(const msa_delta_args& a, const msa_batch* b, hipStream_t s) {
-  return a.dtype == MSA_BF16 ? pick_chunks<bf16_t>(a, b, s) : pick_chunks<float>(a, b, s);
+int msa_launch_delta_chunks(const msa_delta_args& a, const msa_batch* b, float* scratch, hipStream_t s) {
+  return a.dtype == MSA_BF16 ? pick_chunks<bf16_t>(a, b, scratch, s) : pick_chunks<float>(a, b, scratch, s);
 }

@@ -288,8 +288,8 @@ int Run::delta_core(const msa_hybrid_layer& l, const msa_hybrid_state& st, char*
   t.o = step ? nullptr : (float*)alloc((int64_t)M * l.heads * l.vp * 4);
   t.heads = l.heads;
   t.dp = l.dp;
-  t.scratch_floats = step ? 0 : msa_delta_scratch_floats(&t, &b);
-  if (t.scratch_floats > 0) t.scratch = (float*)alloc(t.scratch_floats * 4);
+  const int64_t scratch_floats = step ? 0 : msa_delta_scratch_floats(&t, &b);
+  float* scratch = scratch_floats > 0 ? (float*)alloc(scratch_floats * 4) : nullptr;
   if (!dry) {
     HY(msa_short_conv(d->cfg.dtype, in, ld, C, l.taps, nullptr, l.conv_w, nullptr, 1, qkv, C, st.conv, &b,
                       stream));
@@ -310,7 +310,7 @@ int Run::delta_core(const msa_hybrid_layer& l, const msa_hybrid_state& st, char*
     if (step) {
       HY(msa_delta_step(&t, &b, stream));
     } else {
-      HY(msa_delta_scan(&t, &b, stream));
+      HY(msa_delta_scan_chunks(&t, &b, scratch, scratch_floats, stream));
       HY(msa_delta_output(&t, M, stream));
     }
   }

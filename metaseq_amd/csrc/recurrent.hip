@@ -702,17 +702,26 @@ extern "C" int msa_delta_scan(const msa_delta_args* a, const msa_batch* b, void*
   int rc = check_delta(name, a, b);
   if (rc) return rc;
   MSA_REQUIRE(a->o, MSA_ERR_INVALID_ARG, "%s: null pointer", name);
-  const int64_t scratch = a->scratch ? msa_delta_scratch_floats(a, b) : 0;
-  MSA_REQUIRE(scratch == 0 || a->scratch_floats >= scratch, MSA_ERR_CAPACITY,
-              "%s: scratch of %lld floats, %lld needed", name, (long long)a->scratch_floats,
-              (long long)scratch);
-  if (scratch > 0) {
-    rc = msa_launch_delta_chunks(*a, b, (hipStream_t)stream);
-    if (rc) return rc;
-  } else if (a->dtype == MSA_BF16)
+  if (a->dtype == MSA_BF16)
     dispatch_delta<bf16_t>(*a, b, false, (hipStream_t)stream);
   else
     dispatch_delta<float>(*a, b, false, (hipStream_t)stream);
+  MSA_CHECK_LAUNCH(name);
+  return MSA_OK;
+}
+
+extern "C" int msa_delta_scan_chunks(const msa_delta_args* a, const msa_batch* b, float* scratch,
+                                     int64_t scratch_floats, void* stream) {
+  const int64_t need = msa_delta_scratch_floats(a, b);
+  if (need == 0) return msa_delta_scan(a, b, stream);
+  const char* name = "msa_delta_scan_chunks";
+  int rc = check_delta(name, a, b);
+  if (rc) return rc;
+  MSA_REQUIRE(a->o && scratch, MSA_ERR_INVALID_ARG, "%s: null pointer", name);
+  MSA_REQUIRE(scratch_floats >= need, MSA_ERR_CAPACITY, "%s: scratch of %lld floats, %lld needed", name,
+              (long long)scratch_floats, (long long)need);
+  rc = msa_launch_delta_chunks(*a, b, scratch, (hipStream_t)stream);
+  if (rc) return rc;
   MSA_CHECK_LAUNCH(name);
   return MSA_OK;
 }

@@ -674,12 +674,13 @@ def test_delta_chunks(heads, kv_heads, dim, dp, vp, counts, dtype, channels):
             a.decay_rate, a.dt_bias = ptr(rd), ptr(td)
         need = lib.msa_delta_scratch_floats(ctypes.byref(a), ctypes.byref(b))
         assert need > 0
+        to = ctypes.byref(a), ctypes.byref(b)
         if chunked:
             scratch = torch.full((need,), float("nan"), device="cuda")
-            a.scratch, a.scratch_floats = ptr(scratch), need - 1
-            assert lib.msa_delta_scan(ctypes.byref(a), ctypes.byref(b), _capi.stream_ptr()) == -2
-            a.scratch_floats = need
-        check(lib.msa_delta_scan(ctypes.byref(a), ctypes.byref(b), _capi.stream_ptr()), lib)
+            assert lib.msa_delta_scan_chunks(*to, ptr(scratch), need - 1, _capi.stream_ptr()) == -2
+            check(lib.msa_delta_scan_chunks(*to, ptr(scratch), need, _capi.stream_ptr()), lib)
+        else:
+            check(lib.msa_delta_scan(*to, _capi.stream_ptr()), lib)
         errors.append((rel(o, want), rel(sd, S)))
     print(errors, flush=True)
     # fp32 throughout, some 2 dp + 32 roundings behind every output, of random sign; the scan shows 1 to 3e-7
@@ -712,10 +713,12 @@ def test_delta_chunks_keep_a_nan_from_earlier_tokens(heads, channels):
             a.decay = ptr(dd)
         else:
             a.decay_rate, a.dt_bias = ptr(rd), ptr(rd)
+        to = ctypes.byref(a), ctypes.byref(b)
         if chunked:
-            scratch = torch.empty(lib.msa_delta_scratch_floats(ctypes.byref(a), ctypes.byref(b)), device="cuda")
-            a.scratch, a.scratch_floats = ptr(scratch), scratch.numel()
-        check(lib.msa_delta_scan(ctypes.byref(a), ctypes.byref(b), _capi.stream_ptr()), lib)
+            scratch = torch.empty(lib.msa_delta_scratch_floats(*to), device="cuda")
+            check(lib.msa_delta_scan_chunks(*to, ptr(scratch), scratch.numel(), _capi.stream_ptr()), lib)
+        else:
+            check(lib.msa_delta_scan(*to, _capi.stream_ptr()), lib)
         out.append((torch.isfinite(o).cpu(), o.cpu()))
     (fine, scan), (kept, chunks) = out
     assert not fine[bad, 5] and not fine[bad, vp] and bool(fine[:bad].all())
@@ -739,10 +742,12 @@ def _scan_and_chunks(qkv, ba, decays, state, heads, dp, vp, channels, segments=N
             a.decay = ptr(dd)
         else:
             a.decay_rate, a.dt_bias = ptr(rd), ptr(rd)
+        to = ctypes.byref(a), ctypes.byref(b)
         if chunked:
-            scratch = torch.empty(lib.msa_delta_scratch_floats(ctypes.byref(a), ctypes.byref(b)), device="cuda")
-            a.scratch, a.scratch_floats = ptr(scratch), scratch.numel()
-        check(lib.msa_delta_scan(ctypes.byref(a), ctypes.byref(b), _capi.stream_ptr()), lib)
+            scratch = torch.empty(lib.msa_delta_scratch_floats(*to), device="cuda")
+            check(lib.msa_delta_scan_chunks(*to, ptr(scratch), scratch.numel(), _capi.stream_ptr()), lib)
+        else:
+            check(lib.msa_delta_scan(*to, _capi.stream_ptr()), lib)
         out.append((o.cpu(), sd.cpu()))
     del alive
     return out

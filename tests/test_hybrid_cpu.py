@@ -232,6 +232,24 @@ def test_structures_match_the_header(tmp_path):
     assert [int(x) for x in out.split()] == want
 
 
+def test_delta_arguments_keep_their_layout():
+    """A caller built against an earlier header passes 160 bytes: what the chunks need comes beside them."""
+    assert ctypes.sizeof(_capi.DeltaArgs) == 160
+    lib = _capi.load_hybrid()
+    b, d = _capi.Batch(), _capi.DeltaArgs()
+    b.M = b.max_count = 1000
+    b.nseg = 1
+    d.qkv = d.ba = d.decay_rate = d.dt_bias = d.state = d.o = 4096
+    d.ld, d.ldba, d.heads, d.kv_heads, d.dim, d.dp, d.vp = 96 * 32, 64, 32, 32, 128, 128, 128
+    to = ctypes.byref(d), ctypes.byref(b)
+    need = lib.msa_delta_scratch_floats(*to)
+    assert need > 0
+    assert lib.msa_delta_scan_chunks(*to, None, need, None) == -1
+    assert lib.msa_delta_scan_chunks(*to, ctypes.c_void_p(4096), need - 1, None) == -2
+    d.ldba = 32
+    assert lib.msa_delta_scan_chunks(*to, ctypes.c_void_p(4096), need, None) == -1
+
+
 def test_arguments_are_checked_before_anything_is_launched():
     lib = _capi.load_hybrid()
     one = ctypes.c_void_p(4096)
