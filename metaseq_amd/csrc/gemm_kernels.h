@@ -2259,8 +2259,8 @@ int check_linear_args(const char* name, const void* x, const void* W, const void
 // Split count that minimises what one workgroup moves through its L1: its weight tiles over
 // its K range, the activation fragments of that K range once per tile group, and its fp32
 // partial sums (written here, read back by the LayerNorm tail).  More splits mean more tiles
-// per workgroup over a shorter K range, i.e. fewer activation bytes per weight byte.
-int pick_splits(int64_t M, int N, int K, int wbytes) {
+// per workgroup over a shorter K range, i.e. fewer activation bytes per weight byte.  At most `most` slices.
+int pick_splits(int64_t M, int N, int K, int wbytes, int most = 8) {
   if (M < 1 || M > MSA_PACKED_MAX_ROWS || N % 16 || K % 64) return 1;
   const int MB = packed_row_blocks(M), ntiles = N / 16, nks = K / 32;
   // tiles that share one sweep over the activations (int8 has a 2 x 6 x 3 shape of the
@@ -2269,9 +2269,6 @@ int pick_splits(int64_t M, int N, int K, int wbytes) {
   const int stage = MB > 2 ? 16 : ST_KG * 4;
   int best = 1;
   double best_cost = 0;
-  // Up to eight fp16 rows stop at four slices, which the next product can sum itself (msa_ln_folds): 2048 x 8192
-  // takes 7.8 us in four and 7.9 in eight, and a 1.3b step of one row without the fold 1020 us and 1008.
-  const int most = M <= LN_MAX_ROWS && wbytes == 2 ? 4 : 8;
   for (int S = 1; S <= most; S *= 2) {
     const int G = num_cus() / S;
     if (G < 1 || nks / S < stage) break;  // every wave needs a full stage of K steps

@@ -96,3 +96,19 @@ def test_decoder_handle_is_host_only_bookkeeping():
     bad = _capi.DecoderConfig(2, 160, 2, 512, 64, 40, 1, 0)            # head_dim 80
     assert lib.msa_decoder_create(ctypes.byref(bad), one, one, one, one, one, table,
                                   ctypes.byref(h)) == -1
+
+
+@pytest.mark.parametrize("N,K,rows,fp16,bf16", [
+    (2048, 8192, (1, 4, 8), 4, 8),     # the next product of an fp16 step sums four slices itself
+    (2048, 8192, (9, 16), 8, 8),       # but not of more rows,
+    (2560, 10240, (1, 8, 16), 8, 8),   # nor of a wider model
+    (5120, 20480, (1, 4), 8, 8),
+    (5120, 20480, (8, 16), 4, 4),
+    (1024, 4096, (1, 8, 16), 4, 4),
+])
+def test_only_products_that_fold_stop_at_four_slices(N, K, rows, fp16, bf16):
+    """(256 compute units: also where there is no device)"""
+    core, hybrid = _capi.load(), _capi.load_hybrid()
+    for M in rows:
+        assert core.msa_linear_default_splits(M, N, K) == fp16, M
+        assert hybrid.msa_linear_bf16_splits(M, N, K, 1) == bf16, M
