@@ -13,7 +13,7 @@ bool run_grouped(const msa_group_linear_args& a, const Epilogue& e, hipStream_t 
   // the shares of the eight XCDs are rounded up: up to 7 workgroups beyond the tiles
   const GroupTiles gt{a.perm, a.tile_group, a.tile_row, a.n_tiles, a.group_end, a.rows_per_x};
   hipLaunchKernelGGL(kernel, dim3(ncol, a.max_tiles + (7 + ncol - 1) / ncol), dim3(TQ_THREADS),
-                     tq_lds_bytes(8), s, (const half_t*)a.x, a.W, (int64_t)0, a.N, a.K, 0, 0, 0, e,
+                     tq_lds_bytes(8), s, (const half_t*)a.x, a.W, (int64_t)0, a.N, a.K, 0, 0, e,
                      (float*)nullptr, 0, gt);
   return true;
 }

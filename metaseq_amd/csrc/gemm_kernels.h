@@ -1158,7 +1158,7 @@ __global__ __launch_bounds__(TB_THREADS) void linear_tiled_big_kernel(
 // 256-byte row pieces per 16 lanes.
 // Workgroup -> tile: consecutive workgroups land on consecutive XCDs; where the default order would
 // give an XCD a long thin strip of a round's tiles, the 256 tiles of a round are regrouped so that
-// every XCD's L2 serves a compact a x b block (rm_a, rm_b, rm_r from the host; rm_a < 0: by panels).
+// every XCD's L2 serves a compact a x b block (rm_a, rm_r from the host; rm_a < 0: by panels).
 // Three widths of the workgroup's tile, by the number WF of 16-feature weight fragments per wave:
 // 8 -> 256 x 256 (as described), 4 -> 256 x 128, 2 -> 256 x 64 (fewer accumulators, weight loads and
 // MFMAs per step; the same activation stages).  The two wider forms need M >= 256: a ragged last
@@ -1480,10 +1480,12 @@ __device__ __forceinline__ void quad_tile(const half_t* __restrict__ x, const vo
     });
   };
   int xs = 0, ws = 0;
-  // The loop begins at (or 4 bytes past) a 128-byte line of instructions: with one wave per SIMD its fetches show
-  // wherever it happens to lie (1500 x 3072 x 4096 on 256 x 128 tiles 51 us, 60 bytes past a line 52.6).  The
-  // fill covers, with the few scalar instructions the compiler puts behind it, one line.
-  asm volatile(".p2align 7\n\t.fill 25, 4, 0xbf800000" ::"s"(nks), "s"(xs), "s"(ws) : "memory");
+  // Where the loop begins shows: with one wave per SIMD its fetches have nothing beside them.  The wider forms begin at
+  // (or 4 bytes past) a 128-byte line of instructions (1500 x 3072 x 4096 on 256 x 128 tiles 51 us, 60 bytes past
+  // a line 52.6; 2005 x 4096 x 16384 224 us, 32 past 230), the narrowest 32 or 36 bytes past one (200 x 2048
+  // x 1024 12.5 us, at a line or 24 past 12.9).  The fills leave room for the few scalar instructions that the
+  // compiler puts behind them.
+  asm volatile(".p2align 7\n\t.fill %3, 4, 0xbf800000" ::"s"(nks), "s"(xs), "s"(ws), "n"(WF > 2 ? 25 : 2) : "memory");
   for (int t = 0; t < nks; t += 2) {
     step(t, xs, ws, std::integral_constant<int, 0>{});
     ws = ws == TQ_RW - 1 ? 0 : ws + 1;
@@ -1660,37 +1662,53 @@ __device__ __forceinline__ void quad_tile(const half_t* __restrict__ x, const vo
   }
 }
 
+// Panels of 16 columns of tiles, one after the other over all rows: 16 x 16 tiles of a panel at a time as eight
+// 4 x 8 blocks, one per XCD, the panel's last rows and a narrower last panel row by row.  False: past the last tile.
+__device__ __forceinline__ bool quad_panel(int p, int idx, int ncol, int nrow, int& bx, int& by) {
+  const int w = min(TQ_PANEL, ncol - p * TQ_PANEL), i = idx & 255, round = idx >> 8;
+  if (w < TQ_PANEL) {
+    by = idx / w;
+    bx = p * TQ_PANEL + idx - by * w;
+    return by < nrow;
+  }
+  if ((round + 1) * 16 <= nrow) {
+    const int xcd = i & 7, k = i >> 3;
+    bx = p * TQ_PANEL + (xcd & 3) * 4 + (k & 3);
+    by = round * 16 + (xcd >> 2) * 8 + (k >> 2);
+  } else {
+    bx = p * TQ_PANEL + (idx & (TQ_PANEL - 1));
+    by = idx / TQ_PANEL;
+  }
+  return true;
+}
+// Tile t of a round of 256 regrouped (ncol, a and b are powers of two); the rows below the last whole round row by row.
+__device__ __forceinline__ void quad_regroup(int t, int ncol, int nrow, int rm_a, int rm_r, int& bx, int& by) {
+  const int cs = __builtin_ctz(ncol), as = __builtin_ctz(rm_a), round = t >> 8, i = t & 255;
+  by = t >> cs;
+  bx = t & (ncol - 1);
+  if ((round + 1) * rm_r <= nrow) {  // a full round of 256 tiles
+    const int xcd = i & 7, k = i >> 3, gs = cs - as;
+    bx = ((xcd & ((1 << gs) - 1)) << as) + (k & (rm_a - 1));
+    by = round * rm_r + (xcd >> gs) * (32 >> as) + (k >> as);
+  }
+}
 // Tile t of ncol x nrow in the order of launch (see above: rm_a > 0 regrouped rounds, < 0 panels, 0 row by row).
-__device__ __forceinline__ void quad_place(int t, int ncol, int nrow, int rm_a, int rm_b, int rm_r, int& bx, int& by) {
-  by = t / ncol;
-  bx = t - by * ncol;
+__device__ __forceinline__ void quad_place(int t, int ncol, int nrow, int rm_a, int rm_r, int& bx, int& by) {
   if (rm_a < 0) {
-    // panels of 16 columns, one after the other over all rows: 16 x 16 tiles of a panel at a time as eight
-    // 4 x 8 blocks, one per XCD, the panel's last rows and a narrower last panel row by row
-    const int p = t / (TQ_PANEL * nrow), w = min(TQ_PANEL, ncol - p * TQ_PANEL), idx = t - p * TQ_PANEL * nrow;
-    const int i = idx & 255, round = idx >> 8;
-    if (w == TQ_PANEL && (round + 1) * 16 <= nrow) {
-      const int xcd = i & 7, k = i >> 3;
-      bx = p * TQ_PANEL + (xcd & 3) * 4 + (k & 3);
-      by = round * 16 + (xcd >> 2) * 8 + (k >> 2);
-    } else {
-      bx = p * TQ_PANEL + idx % w;
-      by = idx / w;
-    }
+    const int p = t / (TQ_PANEL * nrow);
+    quad_panel(p, t - p * TQ_PANEL * nrow, ncol, nrow, bx, by);
   } else if (rm_a > 0) {
-    const int round = t >> 8, i = t & 255;
-    if ((round + 1) * rm_r <= nrow) {  // a full round of 256 tiles
-      const int xcd = i & 7, k = i >> 3, gx = ncol / rm_a;
-      bx = (xcd % gx) * rm_a + k % rm_a;
-      by = round * rm_r + (xcd / gx) * rm_b + k / rm_a;
-    }
+    quad_regroup(t, ncol, nrow, rm_a, rm_r, bx, by);
+  } else {
+    by = t / ncol;
+    bx = t - by * ncol;
   }
 }
 
 template <int MODE, int WF, bool PART = false, bool GROUPED = false, int RF = 8, bool FEW = false>
 __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
     const half_t* __restrict__ x, const void* __restrict__ Wp, int64_t M, int N, int K,
-    int rm_a, int rm_b, int rm_r, Epilogue epi, float* __restrict__ part, int part_stages,
+    int rm_a, int rm_r, Epilogue epi, float* __restrict__ part, int part_stages,
     GroupTiles gt = GroupTiles{}) {
   int bx = blockIdx.x, by = blockIdx.y;
   int64_t g_first = 0;
@@ -1704,8 +1722,11 @@ __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
     g_first = gt.tile_row[by];
     M = min((int64_t)gt.group_end[g], g_first + tq_bm(RF));
     Wp = (const char*)Wp + (int64_t)g * N * K * 2;
-  } else if (rm_a != 0) {
-    quad_place(by * gridDim.x + bx, gridDim.x, gridDim.y, rm_a, rm_b, rm_r, bx, by);
+  } else if (WF > 2 && rm_a < 0) {  // a row of the grid is a panel
+    const int ncol = (N + tq_bn(WF) - 1) / tq_bn(WF), nrow = (int)((M + tq_bm(RF) - 1) / tq_bm(RF));
+    if (!quad_panel(by, bx, ncol, nrow, bx, by)) return;
+  } else if (rm_a > 0) {
+    quad_regroup(by * gridDim.x + bx, gridDim.x, gridDim.y, rm_a, rm_r, bx, by);
   }
   quad_tile<MODE, WF, PART, GROUPED, RF, FEW>(x, Wp, M, N, K, bx, by, blockIdx.z, g_first, epi, part, part_stages, gt);
 }
@@ -1715,7 +1736,7 @@ __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
 template <int MODE, bool PART, int PIECES>
 __global__ __launch_bounds__(TQ_THREADS) void linear_quad_pieces_kernel(
     const half_t* __restrict__ x, const void* __restrict__ Wp, int64_t M, int N, int K, int ncol, int nrow,
-    int slices, int n_full, int rm_a, int rm_b, int rm_r, Epilogue epi, float* __restrict__ part, int part_stages) {
+    int slices, int n_full, int rm_a, int rm_r, Epilogue epi, float* __restrict__ part, int part_stages) {
   const int tiles = ncol * nrow, j = (int)blockIdx.x - n_full;
   int unit = blockIdx.x, piece = 0, bx, by;
   if (j >= 0) {  // the first pieces of eight tiles, then their second ones, ...
@@ -1724,7 +1745,7 @@ __global__ __launch_bounds__(TQ_THREADS) void linear_quad_pieces_kernel(
     piece = r / w;
   }
   const int bz = PART ? unit / tiles : 0;
-  quad_place(unit - bz * tiles, ncol, nrow, rm_a, rm_b, rm_r, bx, by);
+  quad_place(unit - bz * tiles, ncol, nrow, rm_a, rm_r, bx, by);
   const GroupTiles none{};
   if (j < 0) return quad_tile<MODE, 8, PART, false, 8, false>(x, Wp, M, N, K, bx, by, bz, 0, epi, part, part_stages, none);
   bx = 2 * bx + (piece & 1);
@@ -1978,24 +1999,31 @@ void launch_stream(const void* xp, const void* W, const void* scales, float* par
 bool wide_panels(int ncol) { return ncol > 64; }
 
 // regrouping of a round's 256 tiles: a x b per XCD with a * b = 32, (ncol / a) * (r / b) = 8 for r = 256 / ncol
-// rows per round; taken when it beats the default strip (ncol / 8) x r.  a < 0: panels, a = 0: row by row
+// rows per round; taken when it beats the default strip (ncol / 8) x r.  a < 0: panels, a = 0: row by row, which is
+// also the order of a single row and of less than one round
 struct TileOrder {
-  int a, b, r;
+  int a, r;
 };
-TileOrder tile_order(int ncol) {
-  TileOrder o{0, 0, 0};
-  if (wide_panels(ncol)) {
+// (256 x 64 tiles, rarely more than a round, are not taken in panels: code in front of the first load shows in
+// products of 5 us)
+TileOrder tile_order(int ncol, int nrow, int WF) {
+  TileOrder o{0, 0};
+  if (nrow == 1) return o;
+  if (WF > 2 && wide_panels(ncol)) {
     o.a = -TQ_PANEL;
-  } else if (ncol >= 8 && 256 % ncol == 0) {
+  } else if (ncol >= 8 && 256 % ncol == 0 && 256 / ncol <= nrow) {
     const int r = 256 / ncol;
     int best = ncol / 8 + r;
     for (int a = 1; a <= 32; a *= 2) {
       const int b = 32 / a;
       if (ncol % a || r % b || (ncol / a) * (r / b) != 8) continue;
-      if (a + b < best) best = a + b, o = TileOrder{a, b, r};
+      if (a + b < best) best = a + b, o = TileOrder{a, r};
     }
   }
   return o;
+}
+dim3 quad_grid(int ncol, int nrow, const TileOrder& o, int slices = 1) {
+  return o.a < 0 ? dim3(TQ_PANEL * nrow, (ncol + TQ_PANEL - 1) / TQ_PANEL, slices) : dim3(ncol, nrow, slices);
 }
 
 // Time of a round of tiles, in rounds of 256 x 256 ones (103 us of K = 4096): 256 x 128 63 us, 256 x 64 45, 128 x 128 37.
@@ -2024,9 +2052,9 @@ void launch_quad_pieces(const void* x, const void* W, int64_t M, int N, int K, i
   if (!allow_lds((const void*)kernel, tq_lds_bytes(8), lds_allowed_h)) return;
   const int ncol = (N + tq_bn(8) - 1) / tq_bn(8), nrow = (int)((M + TQ_BM - 1) / TQ_BM), units = ncol * nrow * S;
   const int n_full = units / num_cus() * num_cus();
-  const TileOrder o = tile_order(ncol);
+  const TileOrder o = tile_order(ncol, nrow, 8);
   hipLaunchKernelGGL(kernel, dim3(n_full + PIECES * (units - n_full)), dim3(TQ_THREADS), tq_lds_bytes(8), s,
-                     (const half_t*)x, W, M, N, K, ncol, nrow, S, n_full, o.a, o.b, o.r, epi, part, K / 64 / S);
+                     (const half_t*)x, W, M, N, K, ncol, nrow, S, n_full, o.a, o.r, epi, part, K / 64 / S);
 }
 
 // One launch of the four-wave kernel (WF = 8: 256 x 256 tiles, the last of them in pieces where that pays; WF = 4:
@@ -2045,9 +2073,9 @@ void launch_quad(const void* x, const void* W, const void* scales, int64_t M, in
   } else {
     static std::atomic<uint64_t> lds_allowed_q{0};
     if (!allow_lds((const void*)linear_quad_kernel<MODE, WF>, tq_lds_bytes(WF), lds_allowed_q)) return;
-    const TileOrder o = tile_order(ncol);
-    hipLaunchKernelGGL((linear_quad_kernel<MODE, WF>), dim3(ncol, nrow), dim3(TQ_THREADS),
-                       tq_lds_bytes(WF), s, (const half_t*)x, W, M_main, N, K, o.a, o.b, o.r, epi,
+    const TileOrder o = tile_order(ncol, nrow, WF);
+    hipLaunchKernelGGL((linear_quad_kernel<MODE, WF>), quad_grid(ncol, nrow, o), dim3(TQ_THREADS),
+                       tq_lds_bytes(WF), s, (const half_t*)x, W, M_main, N, K, o.a, o.r, epi,
                        (float*)nullptr, 0);
   }
   for (int64_t m0 = M_main; m0 < M; m0 += 64)
@@ -2069,8 +2097,9 @@ void launch_few_rows(const void* x, const void* W, int64_t M, int N, int K, cons
   auto kernel = linear_quad_kernel<MODE, WF, false, false, RF, true>;
   if (!allow_lds((const void*)kernel, tq_lds_bytes(WF, RF), lds_allowed_s)) return;
   const int ncol = (N + tq_bn(WF) - 1) / tq_bn(WF), nrow = (int)((M + tq_bm(RF) - 1) / tq_bm(RF));
-  hipLaunchKernelGGL(kernel, dim3(ncol, nrow), dim3(TQ_THREADS), tq_lds_bytes(WF, RF), s, (const half_t*)x, W, M,
-                     N, K, -TQ_PANEL, 0, 0, epi, (float*)nullptr, 0, GroupTiles{});
+  const TileOrder o{nrow == 1 ? 0 : -TQ_PANEL, 0};
+  hipLaunchKernelGGL(kernel, quad_grid(ncol, nrow, o), dim3(TQ_THREADS), tq_lds_bytes(WF, RF), s, (const half_t*)x, W,
+                     M, N, K, o.a, o.r, epi, (float*)nullptr, 0, GroupTiles{});
 }
 
 // Split-K launch of a narrow four-wave form (WF = 2: 256 x 64 tiles, WF = 4: 256 x 128) on
@@ -2085,9 +2114,9 @@ void launch_quad_partial_w(const void* x, const void* W, float* part, int64_t M,
   const int ncol = (N + tq_bn(WF) - 1) / tq_bn(WF);
   const int nrow = (int)((M + TQ_BM - 1) / TQ_BM);
   Epilogue e{};
-  const TileOrder o = tile_order(ncol);
-  hipLaunchKernelGGL(kernel, dim3(ncol, nrow, S), dim3(TQ_THREADS), tq_lds_bytes(WF), s,
-                     (const half_t*)x, W, M, N, K, o.a, o.b, o.r, e, part, K / 64 / S, GroupTiles{});
+  const TileOrder o = tile_order(ncol, nrow, WF);
+  hipLaunchKernelGGL(kernel, quad_grid(ncol, nrow, o, S), dim3(TQ_THREADS), tq_lds_bytes(WF), s,
+                     (const half_t*)x, W, M, N, K, o.a, o.r, e, part, K / 64 / S, GroupTiles{});
 }
 
 // fp16: 256 x 64 tiles while their S slices fit the chip in one round; an S beyond that means 256 x 128
