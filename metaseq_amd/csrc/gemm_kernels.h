@@ -2088,7 +2088,9 @@ void launch_quad(const void* x, const void* W, const void* scales, int64_t M, in
 //   is cheapest: 2048 x 2048 x 4096 44.9 us on 256 x 64 tiles -> 39.6).  Of 129 .. 256 rows a CU then reads half as
 //   many activations as with the 256 x 64 form, its weights once more from L2: 200 x 12288 x 4096 44.3 ->
 //   39.5 us, 200 x 16384 x 4096 48.4 -> 46.8, 129 x 8192 x 2048 22.5 -> 19.3.  (As split-K sums they
-//   gained nothing: 200 x 4096 x 16384 49.8 -> 53.5.)
+//   gained nothing: 200 x 4096 x 16384 49.8 -> 53.5.)  Of 129 .. 256 rows its longer fill of the rings is paid back from
+//   K = 512 on (200 x 4096: K = 256 7.0 -> 7.1 us, 512 9.0 -> 8.6), with more than 192 tiles from K = 4096 on (160 x
+//   16384: K = 2048 26.1 -> 27.1, 4096 47 -> 42).
 //   RF = 8: 256 x 256 tiles that repeat the last row, for outputs wide enough that one row of them fills
 //   the chip (the vocabulary): 200 x 50272 x 4096 171 -> 115 us.
 template <int MODE, int WF, int RF>
@@ -2207,7 +2209,8 @@ void launch_tiled(const void* x, const void* W, const void* scales, int64_t M, i
       const int64_t cols[3] = {(N + 255) / 256, (N + 127) / 128, (N + 63) / 64};
       if (M < TQ_BM && cols[0] <= cus && cols[0] * 4 >= cus * 3)
         return launch_few_rows<MODE, 8, 8>(x, W, M, N, K, epi, s);
-      if (M > 128 && M <= TQ_BM && cols[1] * 2 <= cus && cols[1] * 8 >= cus)
+      if (M > 128 && M <= TQ_BM && cols[1] * 2 <= cus && cols[1] * 8 >= cus &&
+          K >= (cols[1] * 8 <= cus * 3 ? 512 : 4096))
         return launch_few_rows<MODE, 4, 4>(x, W, M, N, K, epi, s);
       if (rows * cols[2] * 8 >= cus) {
         const double unit = TQ_ROUND_US * K;                  // us per round of 256 x 256 tiles
@@ -2218,7 +2221,16 @@ void launch_tiled(const void* x, const void* W, const void* scales, int64_t M, i
         auto offer = [&](double cost, int w, int64_t m_main) {
           if (cost < best) best = cost, best_w = w, best_main = m_main;
         };
-        if (M > TQ_BM) offer((double)quad_rounds((M + 127) / 128 * cols[1]) * TQ_COST_Q * unit, 3, M);
+        if (M > TQ_BM) {
+          const int64_t tiles = (M + 127) / 128 * cols[1];
+          // An odd number of 128 rows, the last of them nearly full (a 256-row tile would repeat its last row
+          // there, from the CU's own cache): 384 x 4096 x 16384 (96 tiles) 139 us against 133 on 256 x 64, 640
+          // 140 against 136, but 384 x 7168 x 28672 (168) 248 against 297; of more than a round bf16 352 x
+          // 50272 x 768 55 against 51 on 256 x 256, 384 x 50272 x 4096 197 against 186, 300 rows 173 against 184.
+          const bool full = rem >= 96 && rem <= 128;
+          const double more = !full ? 1.0 : K > 8192 && tiles * 8 <= cus * 5 ? 1.25 : 1.12;
+          offer((double)quad_rounds(tiles) * TQ_COST_Q * more * unit, 3, M);
+        }
         if (M >= TQ_BM) {
           offer((double)quad_rounds(rows * cols[1]) * TQ_COST_4 * unit, 1, M);
           offer(quad_cost(rows * cols[0]) * unit, 0, M);

@@ -443,9 +443,10 @@ def test_linear_f16(lib, M, N, K, epi):
 
 
 # 128 x 128 tiles (129 .. 256 rows; from a quarter of the chip to all of it, ragged edges, K of the ring's length
-# and less) and 256 x 256 tiles of fewer rows under a wide output
+# and more), shapes beside them whose K is too short for those, and 256 x 256 tiles of fewer rows under a wide output
 @pytest.mark.parametrize("M,N,K", [(129, 4096, 128), (160, 4112, 192), (255, 12304, 320), (256, 16384, 640),
-                                   (200, 12288, 4096), (65, 50272, 128), (130, 50000, 192), (255, 49168, 576),
+                                   (200, 12288, 4096), (129, 4096, 512), (160, 4112, 576), (255, 12288, 640),
+                                   (256, 16384, 4096), (65, 50272, 128), (130, 50000, 192), (255, 49168, 576),
                                    (250, 65536, 128)])
 @pytest.mark.parametrize("epi", ["plain", "bias_relu", "bias_res"])
 def test_linear_f16_few_rows(lib, M, N, K, epi):
