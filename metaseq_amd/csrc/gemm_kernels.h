@@ -2163,13 +2163,19 @@ int pick_row_splits(int64_t M, int N, int K) {
 // The same for sums that leave as fp32 from any width of tile (bf16): also two slices of prompts' products whose
 // 256 x 256 tiles fill half of the chip or less, priced with what the second slice costs to write and read (5
 // TB/s).  1500 x 4096 x 16384: one slice of 256 x 128 tiles 194 us, two of 256 x 256 165 and 5 in the tail; 1500 x
-// 4096 x 4096 stays at one, 54 against 53 and 5.
+// 4096 x 4096 stays at one, 54 against 53 and 5, and so do 1000 x 4096 x 1024 (15.0 against 16.8 and 3) and 3000 x 1024
+// x 1024 (14.3, 17.3 and 2.5), whose one slice is taken in 256 x 64 tiles; 1000 x 4096 x 4096 43 against 37 and 3.
+// Where those tiles leave more than a quarter of the chip idle the clock is higher than the price's: up to K = 8192
+// one slice (2048 x 1408 x 4096 36 against 40 and 2; 1000 x 2560 x 10240 99 against 68 and 2).
 int pick_row_splits_f32(int64_t M, int N, int K) {
   const int few = pick_row_splits(M, N, K);
   if (few > 1 || M < TQ_BM || N % 16 || K % 128 || K < 1024) return few;
-  const int64_t rows = (M + TQ_BM - 1) / TQ_BM, cols8 = (N + 255) / 256, cols4 = (N + 127) / 128;
+  const int64_t rows = (M + TQ_BM - 1) / TQ_BM, cols8 = (N + 255) / 256, cols4 = (N + 127) / 128,
+                cols2 = (N + 63) / 64;
+  if (K < 8192 && rows * cols2 * 4 < num_cus() * 3) return few;
   auto cost = [&](int S) {
-    const double rounds = fmin(quad_cost(rows * cols8 * S), quad_rounds(rows * cols4 * S) * TQ_COST_4);
+    const double narrow = fmin(quad_rounds(rows * cols4 * S) * TQ_COST_4, quad_rounds(rows * cols2 * S) * TQ_COST_2);
+    const double rounds = fmin(quad_cost(rows * cols8 * S), narrow);
     return rounds * TQ_ROUND_US * K / S + (S - 1) * (double)M * N * 8 / 5e6;
   };
   return rows * cols8 * 2 <= num_cus() && cost(2) < 0.95 * cost(1) ? 2 : 1;
