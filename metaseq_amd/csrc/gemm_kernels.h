@@ -249,10 +249,14 @@ __device__ __forceinline__ void epilogue4(const Epilogue& e, int64_t m, int n, f
       const int h = e.hd_shift >= 0 ? c >> e.hd_shift : c / e.hd, d = c - h * e.hd;
       const int mi = (int)m;
       const int b = e.T == 1 ? mi : mi / e.T, tt = mi - b * e.T;
-      const int s0 = e.len_dev ? e.len_dev[b] : e.S0;  // per-row lengths: T == 1, b = row
+      int s0 = e.S0, row = b;
+      if (e.len_dev) {  // per-row lengths: T == 1, b = row
+        s0 = e.len_dev[b];
+        if (e.row_dev) row = e.row_dev[b];
+      }
       if (s0 >= 0 && s0 + tt < e.S_cap) {
         half_t* dst = (part == 0 ? e.Kc : e.Vc) +
-                      (((int64_t)(e.row_dev ? e.row_dev[b] : b) * e.H + h) * e.S_cap + s0 + tt) * e.hd + d;
+                      (((int64_t)row * e.H + h) * e.S_cap + s0 + tt) * e.hd + d;
         *reinterpret_cast<half4_t*>(dst) = o;
       }
     }
