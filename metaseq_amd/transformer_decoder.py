@@ -144,8 +144,9 @@ class TransformerDecoder(IncrementalDecoder):
         self.inference = True
         self.return_inner_states = False
         # instrumentation: called as layer_probe(i, x) with the residual stream [B * T, D] after
-        # layer i of a pass over row-major activations (prefill); the tensor is overwritten by
-        # the next layer, so a probe that keeps it must copy
+        # layer i of a pass over row-major activations (prefill; several prompts into their slots:
+        # one row per position of each prompt, one prompt after the other); the tensor is
+        # overwritten by the next layer, so a probe that keeps it must copy
         self.layer_probe = None
         # decode steps of at most 128 rows go through msa_decoder_step (one C call per token);
         # False drives the same kernels entry point by entry point from Python

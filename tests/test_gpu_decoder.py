@@ -485,8 +485,8 @@ def test_given_token_embeddings_replace_the_lookup():
 
 @pytest.mark.parametrize("int8", [False, True])
 def test_shared_prefill_of_several_prompts_matches_their_own_prefills(int8):
-    """prefill_slots: prompts of different lengths run as one right-padded batch (no real
-    position sees a pad under the causal mask) and land in their slots.  Logits, keys and
+    """prefill_slots: prompts of different lengths run back to back, each over its own positions,
+    and land in their slots.  Logits, keys and
     values agree with each prompt's own prefill to the kernels' tolerance (other tile shapes:
     not to the bit), the lengths are the prompts' own, other slots stay empty, and a decode
     step over the slots agrees likewise."""

@@ -477,11 +477,12 @@ def test_linear_f16_few_rows(lib, M, N, K, epi):
 # Whole rounds of 256 x 256 tiles and a few left, which are cut in four (280, 276 and 1060 tiles) or in two (360 and
 # 1122): pieces past the last row or column, of one row and of a few columns, a last group of fewer
 # than eight tiles; and 128 x 128 tiles of more than 256 rows
-@pytest.mark.parametrize("M,N", [(2305, 7168), (2825, 5728), (5000, 13328), (2945, 7520), (3000, 7680), (4352, 16656),
-                                 (2048, 2048), (641, 4112)])
-def test_linear_f16_pieces(lib, M, N):
-    K = 128
-    print("pieces", M, N, flush=True)
+@pytest.mark.parametrize("M,N,K", [(2305, 7168, 128), (2825, 5728, 128), (5000, 13328, 128), (2945, 7520, 128),
+                                   (3000, 7680, 128), (4352, 16656, 128), (2048, 2048, 128), (641, 4112, 128),
+                                   (2305, 7168, 704), (2945, 7520, 704)])
+def test_linear_f16_pieces(lib, M, N, K):
+    """(K = 704: the quarters' five stages of activations are gone through twice)"""
+    print("pieces", M, N, K, flush=True)
     x, W, b = G(rnd(M, K, seed=M)), G(rnd(N, K, seed=N, std=0.05)), G(rnd(N, seed=9, std=0.1))
     y = G(rnd(M, N, seed=10))
     res = y.float()
@@ -813,6 +814,62 @@ def test_qkv_proj_wide_decode_batch_with_row_lengths(lib, B):
     assert_fp16_close(Kh, wantK, atol=atol, what="K cache")
     assert_fp16_close(Vh, wantV, atol=atol, what="V cache")
     assert float(Kh[7].abs().sum()) == 0 and float(Vh[7].abs().sum()) == 0
+
+
+# packed rows, a tile of few rows, the four-wave tiles, and a ragged bottom of 20 rows on the streaming kernel
+@pytest.mark.parametrize("M,H,K,packed,w8", [
+    (9, 2, 256, True, False), (100, 2, 256, True, True), (70, 3, 256, False, True), (150, 16, 512, False, False),
+    (300, 16, 256, False, False), (1300, 32, 2048, False, False)])
+def test_qkv_proj_rows_into_cache_rows_and_positions_of_their_own(lib, M, H, K, packed, w8):
+    """Every row's key and value go to the cache row and position it names, and nowhere where the position is
+    negative or past the capacity; the numbers are those of the one-row-per-sequence form."""
+    print("qkv rows", M, H, K, packed, w8, flush=True)
+    hd, S_cap, slots = 128, 20, M // 20 + 2
+    D, flags = H * hd, IN_PACKED if packed else 0
+    x, W, b = rnd(M, K, seed=1), rnd(3 * D, K, seed=2, std=0.05), rnd(3 * D, seed=3, std=0.1)
+    xin = G(pack_act(x)) if packed else G(x)
+    weight = (pack_w8(lib, G(O.quantize_int8(W)[0])), G(O.quantize_int8(W)[1])) if w8 else (pack_w(lib, G(W)),)
+    at = torch.randperm(slots * S_cap, generator=torch.Generator().manual_seed(6))[:M]
+    rows, positions = (at // S_cap).int(), (at % S_cap).int()
+    positions[3], positions[M - 1], positions[M // 2] = -1, S_cap, S_cap + 100
+    new = lambda *shape: torch.full(shape, 7.0, dtype=torch.float16, device=DEV)
+    want_q, want_k, want_v = new(M, D), new(M, H, 1, hd), new(M, H, 1, hd)
+    got_q, Kc, Vc = new(M, D), new(slots, H, S_cap, hd), new(slots, H, S_cap, hd)
+    name = "w8a16" if w8 else "f16"
+    ok(getattr(lib, "msa_qkv_proj_" + name)(P(xin), *map(P, weight), P(G(b)), P(want_q), P(want_k), P(want_v), M, 1, H, hd,
+                                            0, 1, K, flags, P(G(torch.zeros(M, dtype=torch.int32))), None), lib)
+    ok(getattr(lib, "msa_qkv_proj_rows_" + name)(P(xin), *map(P, weight), P(G(b)), P(got_q), P(Kc), P(Vc), P(G(rows)),
+                                                 P(G(positions)), M, H, hd, S_cap, K, flags, None), lib)
+    torch.cuda.synchronize()
+    assert torch.equal(got_q, want_q) and bool((want_q != 7.0).any())
+    inside = (positions >= 0) & (positions < S_cap)
+    for cache, mine in ((Kc, want_k), (Vc, want_v)):
+        want = torch.full((slots, H, S_cap, hd), 7.0, dtype=torch.float16)
+        want[rows[inside].long(), :, positions[inside].long()] = mine[:, :, 0].cpu()[inside]
+        assert torch.equal(cache.cpu(), want)
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+def test_attention_of_prompts_back_to_back(lib, hd):
+    """Segments of their own lengths give the bits that each gives by itself; a single position sees its own value."""
+    H, S_cap, lens, slots = 3, 320, [129, 1, 128, 2, 300], [4, 0, 5, 2, 1]
+    print("attention rows", hd, flush=True)
+    D, M = H * hd, sum(lens)
+    starts = torch.tensor([0] + lens).cumsum(0)
+    q, Kc, Vc = G(rnd(M, D, seed=1)), G(rnd(6, H, S_cap, hd, seed=2)), G(rnd(6, H, S_cap, hd, seed=3))
+    out = torch.full((M, D), float("nan"), dtype=torch.float16, device=DEV)
+    ok(lib.msa_attention_rows_f16(P(q), P(Kc), P(Vc), P(out), P(G(starts.int())), P(G(torch.tensor(slots).int())),
+                                  len(lens), max(lens), H, hd, S_cap, None), lib)
+    for i, (n, slot) in enumerate(zip(lens, slots)):
+        mine = slice(int(starts[i]), int(starts[i + 1]))
+        if n == 1:
+            want = Vc[slot, :, 0].reshape(1, D)
+        else:
+            want = torch.empty(n, D, dtype=torch.float16, device=DEV)
+            ok(lib.msa_attention_f16(P(q[mine]), P(Kc[slot]), P(Vc[slot]), None, 0, P(want), 1, H, hd, n, 0, S_cap, 0,
+                                     None, None), lib)
+        torch.cuda.synchronize()
+        assert torch.equal(out[mine], want), n
 
 
 def test_qkv_proj_capacity_error(lib):
