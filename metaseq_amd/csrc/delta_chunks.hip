@@ -14,9 +14,11 @@
 // heads at once, a wave each, and left in a scratch record (20 us for 1500 tokens x 32 heads); then the
 // chunks of a (segment, head, some columns) are walked one after the other.  A scan step's chain of LDS reads, two
 // dots, a sum over lanes and the update takes 500 cycles per token whatever the machine has idle; a
-// chunk's chain takes 2800 (3800 with decays per channel, which are multiplied up while staging) per sixteen.
-// Measured, both kernels against the scan, 32 heads of 128 x 128: one segment of 1500 tokens 132 us against 368
-// (decays per channel 184 against 370), 8 x 1024 tokens 309 against 840 (329 against 1040).
+// chunk's chain takes 2800 (3800 with decays per channel, which are multiplied up while staging) per sixteen
+// where few segments leave a workgroup a CU of its own.  Where many fill the chip the matrix cores are the bound: 104
+// fp32 products of 32 cycles per wave and chunk, two such waves per SIMD, 6650 cycles of the 11000 a chunk takes.
+// Measured, both kernels against the scan, 32 heads of 128 x 128: one segment of 1500 tokens 128 us against 349
+// (decays per channel 174 against 354), 8 x 1024 tokens 322 against 788 (362 against 1003).
 #include <math.h>
 
 #include <type_traits>
@@ -637,7 +639,7 @@ __global__ __launch_bounds__((CT + 4) * 64) void delta_chunk_wide_kernel(
     stager.fetch(raw[0], 2);
     lds_barrier();
     auto beside = [&](typename St::Raw& x, int c) {
-      stager.stage(L, x, c + 1);  // (past the last chunk: zeros, which a surplus chunk reads)
+      stager.stage(L, x, c + 1);  // (past the last chunk: copies of the last row times 0)
       stager.fetch(x, c + 3);
       lds_barrier();
     };
@@ -767,9 +769,9 @@ int pick_chunks(const msa_delta_args& a, const msa_batch* b, float* scratch, hip
 }  // namespace
 
 // The scan stays faster for few short segments (both kernels cost some 15 us before the first token; one segment of
-// 64 / 96 / 128 tokens: 21.0 / 23.4 / 25.6 us against 20.1 / 27.8 / 35.3, with decays per channel 24.3 /
-// 28.1 / 32.1 against 20.1 / 28.0 / 36.8); where the segments fill the chip the chunks win from the first length
-// tried (8 x 64 tokens 37 us against 62, seven segments of 20 and one of 64 35 against 40).
+// 96 / 112 / 128 tokens: 21.2 / 23.2 / 23.2 us against 24.1 / 27.6 / 31.1, with decays per channel 25.3 /
+// 28.6 / 28.9 against 24.1 / 27.9 / 33.0; of 64 tokens 16.7 by the scan); where the segments fill the chip the chunks
+// win from the first length tried (8 x 48 tokens 32 us against 44, seven segments of 20 and one of 64 32 against 36).
 constexpr int DC_FROM = 96, DC_FROM_WIDE = 48;
 
 extern "C" int64_t msa_delta_scratch_floats(const msa_delta_args* a, const msa_batch* b) {

@@ -197,10 +197,11 @@ int pack_entry(const char* name, const void* src, void* dst, int N, int K, bool 
 
 }  // namespace
 
-// Measured, a whole step without and with the fold, us: 12 layers of 768 one row 356 and 310, eight rows 406 and 329;
-// 24 of 1024 714 and 616, 758 and 662; 24 of 2048 1008 and 968, 1036 and 1028.  The int8 products are
-// shorter and have less to hide it behind: 8 layers of 2048 one row 322 and 317, four 327 and 325, six 331
-// and 334, eight 331 and 339.  More rows than waves or a longer row would not fit the registers.
+// Measured, a whole step over 48 positions without and with the fold, us (medians of seven, which lie within 2 % with
+// it): 12 layers of 768 one row 385 and 311, eight rows 387 and 329; 24 of 1024 767 and 615, 780 and 660; 24 of 2048
+// 1015 and 965, four rows 1045 and 991, eight 1055 and 1031 (over 576 positions 1159 and 1150).  The int8 products
+// are shorter and have less to hide it behind: 8 layers of 2048 one row 326 and 316, four 331 and 325; with the fold
+// six took 334 for 331 and eight 339 for 331.  More rows than waves or a longer row would not fit the registers.
 bool msa_ln_folds(int M, int D, int S, bool int8) {
   return M >= 1 && M <= LN_MAX_ROWS && D <= LN_MAX_K && D % 64 == 0 && (S == 1 || S == 2 || S == 4) &&
          (!int8 || M * D <= 8192);
@@ -375,7 +376,7 @@ extern "C" int msa_lm_head_greedy_select_noalloc_f16(
 
 // Rows and widths whose sum the next product of a decode step can take in front of itself stop at the four
 // slices that it takes: 2048 x 8192 in four 7.8 us and in eight 7.9, and a step of 24 such layers, one row,
-// without the fold 1020 us and 1008 (with it, in four, 968).
+// without the fold 1020 us and 1008 (with it, in four, 965).
 extern "C" int msa_linear_default_splits(int64_t M, int N, int K) {
   return pick_splits(M, N, K, 2, M <= LN_MAX_ROWS && msa_ln_folds((int)M, N, 4, false) ? 4 : 8);
 }
