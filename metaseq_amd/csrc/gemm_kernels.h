@@ -1786,7 +1786,8 @@ int num_cus() {  // compute units of the current device
 }
 
 // Raises a kernel's dynamic LDS limit once per device (one mask per kernel instantiation; a
-// second thread that gets here at the same time only repeats the call).
+// second thread that gets here at the same time only repeats the call).  False: nothing may be launched; the
+// runtime keeps the refusal as its last error, which every entry point reads behind its launches.
 bool allow_lds(const void* kernel, int bytes, std::atomic<uint64_t>& done) {
   const int dev = current_device();
   const uint64_t bit = dev >= 0 ? 1ull << dev : 0;
@@ -2090,13 +2091,13 @@ void launch_quad(const void* x, const void* W, const void* scales, int64_t M, in
 // One round of tiles over fewer rows than a 256-row tile holds, or a little more than one of 128.
 //   RF = 4: 128 x 128 tiles, two rows of them side by side on one XCD (also of more rows, where one round of them
 //   is cheapest: 2048 x 2048 x 4096 44.9 us on 256 x 64 tiles -> 39.6).  Of 129 .. 256 rows a CU then reads half as
-//   many activations as with the 256 x 64 form, its weights once more from L2: 200 x 12288 x 4096 44.3 ->
-//   39.5 us, 200 x 16384 x 4096 48.4 -> 46.8, 129 x 8192 x 2048 22.5 -> 19.3.  (As split-K sums they
+//   many activations as with the 256 x 64 form, its weights once more from L2: 200 x 12288 x 4096 43.3 ->
+//   37.5 us, 200 x 16384 x 4096 48.1 -> 41.2, 130 x 8192 x 2048 21.8 -> 18.7.  (As split-K sums they
 //   gained nothing: 200 x 4096 x 16384 49.8 -> 53.5.)  Of 129 .. 256 rows its longer fill of the rings is paid back from
 //   K = 512 on (200 x 4096: K = 256 7.0 -> 7.1 us, 512 9.0 -> 8.6), with more than 192 tiles from K = 4096 on (160 x
 //   16384: K = 2048 26.1 -> 27.1, 4096 47 -> 42).
 //   RF = 8: 256 x 256 tiles that repeat the last row, for outputs wide enough that one row of them fills
-//   the chip (the vocabulary): 200 x 50272 x 4096 171 -> 115 us.
+//   the chip (the vocabulary): bf16 200 x 50272 x 4096 168 -> 101 us.
 template <int MODE, int WF, int RF>
 void launch_few_rows(const void* x, const void* W, int64_t M, int N, int K, const Epilogue& epi, hipStream_t s) {
   static std::atomic<uint64_t> lds_allowed_s{0};
