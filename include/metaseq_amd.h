@@ -238,6 +238,12 @@ int msa_attention_f16(const void* q, const void* Kcache, const void* Vcache,
 int msa_attention_rows_f16(const void* q, const void* Kcache, const void* Vcache, void* out, const int32_t* starts,
                            const int32_t* rows, int segments, int longest, int H, int hd, int S_cap, void* stream);
 
+/* Either of the two over M <= 128 rows in all, its output in the packed activation layout: with `starts` and `rows` as
+ * msa_attention_rows_f16 (B segments of at most T rows), without (NULL) as msa_attention_f16 over B x T = M rows. */
+int msa_attention_packed_f16(const void* q, const void* Kcache, const void* Vcache, const uint8_t* key_pad_mask,
+                             int64_t mask_stride, void* out, const int32_t* starts, const int32_t* rows, int M, int B,
+                             int H, int hd, int T, int S0, int S_cap, void* stream);
+
 /* EXPERIMENTAL: pays only beyond OPT's 2048 positions (no benchmark configuration selects it;
  * msa_decoder_step takes it for a single request over more than 4096 keys at head_dim 128).
  * The decode step's attention (T == 1) in two launches, for few (batch row, head) pairs over long

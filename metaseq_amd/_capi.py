@@ -84,6 +84,8 @@ SIGNATURES = {
     "msa_qkv_proj_rows_w8a16": [_P, _P, _P, _P, _P, _P, _P, _P, _P, c_int, c_int, c_int, c_int,
                                 c_int, c_uint, _P],
     "msa_attention_rows_f16": [_P, _P, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, _P],
+    "msa_attention_packed_f16": [_P, _P, _P, _P, c_int64, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
+                                 _P],
     "msa_attention_f16": [_P, _P, _P, _P, c_int64, _P, c_int, c_int, c_int, c_int, c_int, c_int,
                           c_uint, _P, _P],
     "msa_attention_split_f16": [_P, _P, _P, _P, c_int64, _P, _P, c_int, c_int, c_int, c_int, c_int,

@@ -392,6 +392,28 @@ extern "C" int msa_attention_rows_f16(const void* q, const void* Kcache, const v
   return MSA_OK;
 }
 
+extern "C" int msa_attention_packed_f16(const void* q, const void* Kcache, const void* Vcache,
+                                        const uint8_t* key_pad_mask, int64_t mask_stride, void* out,
+                                        const int32_t* starts, const int32_t* rows, int M, int B, int H, int hd, int T,
+                                        int S0, int S_cap, void* stream) {
+  const char* name = "msa_attention_packed_f16";
+  MSA_REQUIRE(q && Kcache && Vcache && out && (starts == nullptr) == (rows == nullptr), MSA_ERR_INVALID_ARG,
+              "%s: null pointer", name);
+  MSA_REQUIRE(B > 0 && H > 0 && T > 0 && S0 >= 0 && M > 0 && M <= MSA_PACKED_MAX_ROWS, MSA_ERR_INVALID_ARG,
+              "%s: bad shape B=%d H=%d T=%d S0=%d M=%d", name, B, H, T, S0, M);
+  MSA_REQUIRE(starts ? !key_pad_mask && S0 == 0 && T <= M && B <= M : (int64_t)B * T == M, MSA_ERR_INVALID_ARG,
+              "%s: %d rows of %d x %d", name, M, B, T);
+  MSA_REQUIRE(hd == 64 || hd == 128, MSA_ERR_INVALID_ARG, "%s: head_dim %d not supported (64 or 128)", name, hd);
+  MSA_REQUIRE((int64_t)S0 + T <= S_cap && S0 + T <= 8192, MSA_ERR_CAPACITY,
+              "%s: %d positions exceed the cache capacity %d or 8192", name, S0 + T, S_cap);
+  MSA_REQUIRE(!key_pad_mask || mask_stride >= S0 + T, MSA_ERR_INVALID_ARG, "%s: mask_stride %lld shorter than %d keys",
+              name, (long long)mask_stride, S0 + T);
+  msa_launch_prefill_attention(q, Kcache, Vcache, key_pad_mask, mask_stride, out, B, H, hd, T, S0, S_cap,
+                               (hipStream_t)stream, starts, rows, packed_row_blocks(M));
+  MSA_CHECK_LAUNCH(name);
+  return MSA_OK;
+}
+
 extern "C" int msa_attention_f16(const void* q, const void* Kcache, const void* Vcache,
                                  const uint8_t* key_pad_mask, int64_t mask_stride, void* out, int B,
                                  int H, int hd, int T, int S0, int S_cap, unsigned flags,

@@ -46,7 +46,7 @@ __global__ __launch_bounds__(PF_THREADS) void prefill_attention_kernel(
     const half_t* __restrict__ q, const half_t* __restrict__ Kc, const half_t* __restrict__ Vc,
     const uint8_t* __restrict__ key_pad_mask, int64_t mask_stride, half_t* __restrict__ out,
     int BH, int n_qt, int grouped, int H, int T, int S0, int S_cap, const int32_t* __restrict__ seg_start,
-    const int32_t* __restrict__ seg_row) {
+    const int32_t* __restrict__ seg_row, int out_mb) {
   constexpr int KSTEPS = HD / 16;           // MFMA k steps over the head dimension
   constexpr int DBLK = HD / 32;             // 32-row blocks of O^T
   constexpr int ROWB = HD * 2;              // bytes of a key row
@@ -288,6 +288,7 @@ __global__ __launch_bounds__(PF_THREADS) void prefill_attention_kernel(
   }
   // O^T accumulator: lane holds query j and d = 32*db + 8*blk + 4*hl + r
   if (tq >= 0) {
+    const int row = (int)(row0 + tq);  // (packed rows: at most 128 of them)
     half_t* orow = out + (row0 + tq) * D + h * HD;
 #pragma unroll
     for (int db = 0; db < DBLK; ++db)
@@ -296,7 +297,8 @@ __global__ __launch_bounds__(PF_THREADS) void prefill_attention_kernel(
         half4_t v;
 #pragma unroll
         for (int r = 0; r < 4; ++r) v[r] = (half_t)o[db][4 * blk + r];
-        *reinterpret_cast<half4_t*>(orow + db * 32 + blk * 8 + hl * 4) = v;
+        const int d = db * 32 + blk * 8 + hl * 4;
+        *reinterpret_cast<half4_t*>(out_mb > 0 ? out + packed_act_offset(row, h * HD + d, out_mb) : orow + d) = v;
       }
   }
 }
@@ -307,7 +309,7 @@ int msa_launch_prefill_attention(const void* q, const void* Kc, const void* Vc,
                                  const uint8_t* key_pad_mask, int64_t mask_stride, void* out,
                                  int B, int H, int hd, int T, int S0, int S_cap,
                                  hipStream_t stream, const int32_t* seg_start,
-                                 const int32_t* seg_row) {
+                                 const int32_t* seg_row, int out_mb) {
   const int n_qt = (T + PF_BM - 1) / PF_BM, BH = B * H;
   const dim3 grid((unsigned)(((BH + 7) / 8) * 8 * n_qt));
   // K and V rows of all (row, head) pairs against the 32 MB of L2 + part of the memory-side cache
@@ -316,11 +318,11 @@ int msa_launch_prefill_attention(const void* q, const void* Kc, const void* Vc,
     hipLaunchKernelGGL(prefill_attention_kernel<64>, grid, dim3(PF_THREADS), 0, stream,
                        (const half_t*)q, (const half_t*)Kc, (const half_t*)Vc, key_pad_mask,
                        mask_stride, (half_t*)out, BH, n_qt, grouped, H, T, S0, S_cap,
-                       seg_start, seg_row);
+                       seg_start, seg_row, out_mb);
   else
     hipLaunchKernelGGL(prefill_attention_kernel<128>, grid, dim3(PF_THREADS), 0, stream,
                        (const half_t*)q, (const half_t*)Kc, (const half_t*)Vc, key_pad_mask,
                        mask_stride, (half_t*)out, BH, n_qt, grouped, H, T, S0, S_cap,
-                       seg_start, seg_row);
+                       seg_start, seg_row, out_mb);
   return 0;
 }

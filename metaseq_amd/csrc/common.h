@@ -45,7 +45,7 @@ int msa_launch_prefill_attention(const void* q, const void* Kc, const void* Vc,
                                  const uint8_t* key_pad_mask, int64_t mask_stride, void* out,
                                  int B, int H, int hd, int T, int S0, int S_cap,
                                  hipStream_t stream, const int32_t* seg_start = nullptr,
-                                 const int32_t* seg_row = nullptr);
+                                 const int32_t* seg_row = nullptr, int out_mb = 0);
 
 // routed products over 256-row tiles, bf16 (gemm_bf16.hip)
 bool msa_launch_group_quad(const msa_group_linear_args& a, hipStream_t stream);

@@ -794,8 +794,12 @@ class TransformerDecoder(IncrementalDecoder):
             inner_states[0]["emb"] = x.view(B, T, D).transpose(0, 1).clone()
         work = self._rows_buffers(M, dev)
         for i, layer in enumerate(self.layers):
+            # (a probe may change the stream in front of the next LayerNorm)
+            last = i + 1 == len(self.layers)
+            after = (None if self.layer_probe is not None else self.layer_norm if last
+                     else self.layers[i + 1].self_attn_layer_norm)
             self._rows_layer(lib, stream, layer, x, work, B, T, S0, kv.k(i), kv.v(i),
-                             kv.capacity, mask, len_dev, prompts)
+                             kv.capacity, mask, len_dev, prompts, after, last)
             if self.layer_probe is not None:
                 self.layer_probe(i, x)
         if self.return_inner_states:
@@ -803,7 +807,8 @@ class TransformerDecoder(IncrementalDecoder):
         else:
             inner_states.append(None)
         h = work["h"]
-        self._layernorm(lib, stream, x, self.layer_norm, M, D, h)
+        if not work["normed"]:
+            self._layernorm(lib, stream, x, self.layer_norm, M, D, h)
         return h, inner_states
 
     def _decode_chunks(self, lib, stream, tokens, n, B, cache, mask, lens, S0,
@@ -839,11 +844,12 @@ class TransformerDecoder(IncrementalDecoder):
                 torch.cat(positions))
 
     def _rows_buffers(self, M, dev):
-        """Work buffers of ``_rows_layer`` for M row-major activation rows."""
+        """Work buffers of ``_rows_layer`` for M row-major activation rows.  ``normed``: the tail of the
+        layer before has already written the LayerNorm that comes next."""
         D, F = self.cfg.decoder_embed_dim, self.cfg.decoder_ffn_embed_dim
         f16 = dict(dtype=torch.float16, device=dev)
         return {"q": torch.empty(M, D, **f16), "h": torch.empty(M, D, **f16),
-                "o": torch.empty(M, D, **f16), "u": torch.empty(M, F, **f16)}
+                "o": torch.empty(M, D, **f16), "u": torch.empty(M, F, **f16), "normed": False}
 
     def _rows_attention(self, lib, stream, q, kc, vc, mask, o, B, H, hd, T, S0, cap, len_dev, prompts):
         if prompts is not None:
@@ -855,19 +861,22 @@ class TransformerDecoder(IncrementalDecoder):
                                     ptr(o), B, H, hd, T, S0, cap, 0, ptr(len_dev), stream))
 
     def _rows_layer(self, lib, stream, layer, x, work, B, T, S0, kc, vc, cap, mask, len_dev=None,
-                    prompts=None):
+                    prompts=None, after=None, last=False):
         """One layer over B * T row-major rows (transformer_decoder_layer.py:233-284): ``x`` is
         the residual stream, updated in place; keys and values of the T new positions of every
-        row go to positions S0 .. S0 + T - 1 of ``kc`` / ``vc``."""
+        row go to positions S0 .. S0 + T - 1 of ``kc`` / ``vc``.  Where fc2 runs as partial sums, the launch
+        that adds them up also writes the LayerNorm ``after`` that follows (``last``: the decoder's own,
+        row-major): per layer 200 rows 6.6 + 5.4 -> 6.7 us, 57 rows 4.9 + 4.7 -> 4.9."""
         cfg = self.cfg
         D, H, hd, F = (cfg.decoder_embed_dim, cfg.decoder_attention_heads, cfg.head_dim,
                        cfg.decoder_ffn_embed_dim)
         M = B * T
         if M <= self.PACKED_MAX_ROWS:
             return self._rows_layer_short(lib, stream, layer, x, work, B, T, S0, kc, vc, cap, mask,
-                                          len_dev, prompts)
+                                          len_dev, prompts, after, last)
         q, h, o, u = work["q"], work["h"], work["o"], work["u"]
-        self._layernorm(lib, stream, x, layer.self_attn_layer_norm, M, D, h)
+        if not work["normed"]:
+            self._layernorm(lib, stream, x, layer.self_attn_layer_norm, M, D, h)
         self._qkv(lib, stream, h, layer.self_attn.qkv_proj, q, kc, vc, B, T, H, hd, S0, cap, D, 0,
                   len_dev, prompts)
         self._rows_attention(lib, stream, q, kc, vc, mask, o, B, H, hd, T, S0, cap, len_dev, prompts)
@@ -878,45 +887,59 @@ class TransformerDecoder(IncrementalDecoder):
             self._linear(lib, stream, o, layer.self_attn.out_proj, M, D, D, residual=x, out=x)
             self._layernorm(lib, stream, x, ln2, M, D, h)
         self._linear(lib, stream, h, layer.fc1, M, F, D, relu=True, out=u)
-        if not self._linear_split(lib, stream, u, layer.fc2, x, work, M, D, F):
+        work["normed"] = self._linear_split(lib, stream, u, layer.fc2, x, work, M, D, F, ln=after,
+                                            ln_out=h if after is not None else None)
+        if not work["normed"]:
             self._linear(lib, stream, u, layer.fc2, M, D, F, residual=x, out=x)
+        work["normed"] = work["normed"] and after is not None
 
     def _rows_layer_short(self, lib, stream, layer, x, work, B, T, S0, kc, vc, cap, mask,
-                          len_dev=None, prompts=None):
+                          len_dev=None, prompts=None, after=None, last=False):
         """``_rows_layer`` for at most 128 rows (a short prompt): the layer's GEMM inputs are
         produced in the packed activation layout by the kernels in front of them, so that qkv,
-        fc1 and fc2 run on the weight-streaming kernels of the decode step (56 rows, OPT-6.7B
-        shapes: 25 / 30 / 30 us against 32 / 45 / 52 on row-major rows).  The attention output
-        stays row-major (the prefill attention kernel writes no packed rows), so out_proj runs
-        as in ``_rows_layer``."""
+        out_proj, fc1 and fc2 run on the weight-streaming kernels of the decode step (56 rows, OPT-6.7B
+        shapes: 25 / 12.6 / 30 / 30 us against 32 / 15 / 45 / 52 on row-major rows)."""
         cfg = self.cfg
         D, H, hd, F = (cfg.decoder_embed_dim, cfg.decoder_attention_heads, cfg.head_dim,
                        cfg.decoder_ffn_embed_dim)
         M = B * T
         IN, OUT = MSA_IN_PACKED, MSA_OUT_PACKED
-        q, o = work["q"], work["o"]
+        q = work["q"]
         if "hp" not in work:
             MP = self._packed_rows(M)
             work["hp"] = torch.empty(MP * D, dtype=torch.float16, device=x.device)
+            work["op"] = torch.empty(MP * D, dtype=torch.float16, device=x.device)
             work["up"] = torch.empty(MP * F, dtype=torch.float16, device=x.device)
             int8 = layer.fc2.qweight is not None
             splits = lib.msa_linear_default_splits_w8a16 if int8 else lib.msa_linear_default_splits
-            work["S_f"] = splits(M, D, F)
-        hp, up, S_f = work["hp"], work["up"], work["S_f"]
-        self._layernorm(lib, stream, x, layer.self_attn_layer_norm, M, D, hp, OUT)
+            work["S_o"], work["S_f"] = splits(M, D, D), splits(M, D, F)
+        hp, op, up, S_o, S_f = (work[k] for k in ("hp", "op", "up", "S_o", "S_f"))
+        if not work["normed"]:
+            self._layernorm(lib, stream, x, layer.self_attn_layer_norm, M, D, hp, OUT)
         self._qkv(lib, stream, hp, layer.self_attn.qkv_proj, q, kc, vc, B, T, H, hd, S0, cap, D, IN,
                   len_dev, prompts)
-        self._rows_attention(lib, stream, q, kc, vc, mask, o, B, H, hd, T, S0, cap, len_dev, prompts)
-        ln2 = layer.final_layer_norm
-        if not self._linear_split(lib, stream, o, layer.self_attn.out_proj, x, work, M, D, D,
-                                  ln=ln2, ln_out=hp, ln_flags=OUT):
-            self._linear(lib, stream, o, layer.self_attn.out_proj, M, D, D, residual=x, out=x)
-            self._layernorm(lib, stream, x, ln2, M, D, hp, OUT)
+        mask_stride = mask.stride(0) if mask is not None else 0
+        if prompts is not None:
+            check(lib.msa_attention_packed_f16(ptr(q), ptr(kc), ptr(vc), None, 0, ptr(op), ptr(prompts.start),
+                                               ptr(prompts.slot), M, prompts.count, H, hd, prompts.longest, 0, cap,
+                                               stream))
+        elif T > 1:
+            check(lib.msa_attention_packed_f16(ptr(q), ptr(kc), ptr(vc), ptr(mask), mask_stride, ptr(op), None, None,
+                                               M, B, H, hd, T, S0, cap, stream))
+        else:
+            check(lib.msa_attention_f16(ptr(q), ptr(kc), ptr(vc), ptr(mask), mask_stride, ptr(op), B, H, hd, 1, S0,
+                                        cap, OUT, ptr(len_dev), stream))
+        ln2, out_proj = layer.final_layer_norm, layer.self_attn.out_proj
+        part = self._part(work, max(S_o, S_f) * M * D, x.device)
+        self._linear_partial(lib, stream, op, out_proj, part, M, D, D, S_o)
+        check(lib.msa_residual_layernorm_f16(ptr(part), S_o, ptr(out_proj.bias), ptr(x), ptr(ln2.weight),
+                                             ptr(ln2.bias), ptr(hp), M, D, 1e-5, OUT, stream))
         self._linear(lib, stream, hp, layer.fc1, M, F, D, relu=True, out=up, flags=IN | OUT)
-        part = self._part(work, S_f * M * D, x.device)
         self._linear_partial(lib, stream, up, layer.fc2, part, M, D, F, S_f)
-        check(lib.msa_residual_layernorm_f16(ptr(part), S_f, ptr(layer.fc2.bias), ptr(x), None,
-                                             None, None, M, D, 1e-5, 0, stream))
+        work["normed"] = after is not None
+        g, b, to = (after.weight, after.bias, work["h"] if last else hp) if after is not None else (None,) * 3
+        check(lib.msa_residual_layernorm_f16(ptr(part), S_f, ptr(layer.fc2.bias), ptr(x), ptr(g),
+                                             ptr(b), ptr(to), M, D, 1e-5, 0 if last else OUT, stream))
 
     @staticmethod
     def _part(work, n, dev):

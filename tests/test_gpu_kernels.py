@@ -872,6 +872,37 @@ def test_attention_of_prompts_back_to_back(lib, hd):
         assert torch.equal(out[mine], want), n
 
 
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("lens,S0,masked", [([57], 0, False), ([1, 2, 61, 64], 0, False), ([1], 0, False),
+                                            ([3] * 5, 40, True), ([128], 129, True)])
+def test_packed_attention_output_holds_the_rows_of_the_plain_one(lib, hd, lens, S0, masked):
+    """The same bits in the packed layout, whole and in segments; rows past the last are left alone."""
+    H, S_cap, slots = 4, 320, list(range(len(lens)))[::-1]
+    print("packed attention", hd, lens, flush=True)
+    D, M, B, T = H * hd, sum(lens), len(lens), max(lens)
+    q, Kc, Vc = G(rnd(M, D, seed=1)), G(rnd(B, H, S_cap, hd, seed=2)), G(rnd(B, H, S_cap, hd, seed=3))
+    mask = torch.zeros(B, S_cap, dtype=torch.uint8, device=DEV)
+    mask[:, :2] = masked
+    pm = P(mask) if masked else None
+    MB = 8 if M > 64 else (M + 15) // 16
+    got = torch.full((MB * 16 * D,), 7.0, dtype=torch.float16, device=DEV)
+    want = torch.empty(M, D, dtype=torch.float16, device=DEV)
+    if len(set(lens)) == 1 and T > 1:
+        ok(lib.msa_attention_f16(P(q), P(Kc), P(Vc), pm, S_cap, P(want), B, H, hd, T, S0, S_cap, 0, None, None), lib)
+        ok(lib.msa_attention_packed_f16(P(q), P(Kc), P(Vc), pm, S_cap, P(got), None, None, M, B, H, hd, T, S0, S_cap,
+                                        None), lib)
+    else:
+        to = P(G(torch.tensor([0] + lens).cumsum(0).int())), P(G(torch.tensor(slots).int()))
+        ok(lib.msa_attention_rows_f16(P(q), P(Kc), P(Vc), P(want), *to, B, T, H, hd, S_cap, None), lib)
+        ok(lib.msa_attention_packed_f16(P(q), P(Kc), P(Vc), None, 0, P(got), *to, M, B, H, hd, T, 0, S_cap, None), lib)
+    torch.cuda.synchronize()
+    rows = got.view(D // 32, MB, 4, 16, 8).permute(1, 3, 0, 2, 4).reshape(MB * 16, D)
+    assert torch.equal(rows[:M], want) and bool((rows[M:] == 7.0).all())
+    for bad in ((None, None, M, B, H, hd, T + 1, S0, S_cap), (None, None, 129, 129, H, hd, 1, S0, S_cap),
+                (None, P(mask), M, B, H, hd, T, S0, S_cap)):
+        assert lib.msa_attention_packed_f16(P(q), P(Kc), P(Vc), None, 0, P(got), *bad, None) == -1
+
+
 def test_qkv_proj_capacity_error(lib):
     x = torch.zeros(2, 128, dtype=torch.float16, device=DEV)
     rc = lib.msa_qkv_proj_f16(P(x), P(x), P(x), P(x), P(x), P(x), 2, 1, 2, 64, 10, 10, 128, 0,
