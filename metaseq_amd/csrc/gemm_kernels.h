@@ -645,7 +645,7 @@ __global__ __launch_bounds__(KL * NG * 64) void linear_share_kernel(
     const half_t* __restrict__ xp, const void* __restrict__ Wp, const half_t* __restrict__ scales,
     float* __restrict__ part, int M, int N, int K, int tiles_per_wg, int ks_per_split,
     Epilogue epi) {
-  static_assert(MODE != MODE_SELECT, "selection runs in the plain stream kernel");
+  static_assert(MODE != MODE_SELECT || (KL == 1 && NT == 1), "a wave that selects owns its tiles' sums");
   using C = ShareCfg<MB, W8, KL, NG, NT, U>;
   constexpr int SK = C::SK, UA = C::UA, XH = C::XH, XP = C::XP, THREADS = C::THREADS;
   constexpr int PIECES = C::PIECES;
@@ -773,8 +773,20 @@ __global__ __launch_bounds__(KL * NG * 64) void linear_share_kernel(
       }
     }
   };
+  SelectState sel[MODE == MODE_SELECT ? MB : 1];  // of row lane % 16 of each block
   auto finish = [&](int idx) {  // after the last stage of a tile group
     const int grp = idx / nstages;
+    if constexpr (MODE == MODE_SELECT) {
+      const int t = tile_begin + grp * NG + ng;
+      if (t < tile_end) {
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+          if (mb * 16 + (lane & 15) < M)
+            select_update4(sel[mb], epi, mb * 16 + (lane & 15), t * 16 + ((lane >> 4) << 2), acc[0][mb]);
+      }
+      clear();
+      return;
+    }
     float4_t* red = red_own;
     if constexpr (C::RED_ALIAS) {  // the stage just consumed, once every wave is done reading it
       red = reinterpret_cast<float4_t*>(lx_share + (idx & 1) * XH);
@@ -801,7 +813,7 @@ __global__ __launch_bounds__(KL * NG * 64) void linear_share_kernel(
           if (part)
             *reinterpret_cast<float4_t*>(part + ((int64_t)blockIdx.y * M + m) * N + n) = sum;
           else
-            epilogue4<MODE>(epi, m, n, sum);
+            epilogue4<MODE == MODE_SELECT ? MODE_PLAIN : MODE>(epi, m, n, sum);
         }
       }
       if (j + 1 < NT) __syncthreads();  // the buffer is rewritten by the next slot
@@ -834,6 +846,36 @@ __global__ __launch_bounds__(KL * NG * 64) void linear_share_kernel(
       compute(w[st], i);
       if (i < total && (i + 1) % nstages == 0) finish(i);
       __syncthreads();
+    }
+  }
+  if constexpr (MODE == MODE_SELECT) {  // the row's lanes through shuffles, the waves through LDS, as in the stream kernel
+    static_assert(NG * MB * 16 * sizeof(SelectPartial) <= C::LDS_BYTES, "the states take the stages' place");
+    SelectPartial* sp = reinterpret_cast<SelectPartial*>(lx_share);  // [NG][MB * 16]
+    auto partial_of = [](const SelectState& st) {
+      SelectPartial p;
+      p.m = st.m, p.s = st.s, p.best = st.best, p.bidx = st.bidx, p.nan = st.nan ? 1.f : 0.f;
+      p.pad[0] = p.pad[1] = p.pad[2] = 0.f;
+      return p;
+    };
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+      SelectState st = sel[mb];
+#pragma unroll
+      for (int o = 16; o <= 32; o <<= 1)
+        select_merge(st, __shfl_xor(st.m, o, MSA_WAVE), __shfl_xor(st.s, o, MSA_WAVE),
+                     __shfl_xor(st.best, o, MSA_WAVE), __shfl_xor(st.bidx, o, MSA_WAVE),
+                     (bool)__shfl_xor((int)st.nan, o, MSA_WAVE));
+      if (lane < 16) sp[ng * (MB * 16) + mb * 16 + lane] = partial_of(st);
+    }
+    __syncthreads();
+    const int m = threadIdx.x;
+    if (m < MB * 16 && m < M) {
+      SelectState st;
+      for (int w = 0; w < NG; ++w) {
+        const SelectPartial p = sp[w * (MB * 16) + m];
+        select_merge(st, p.m, p.s, p.best, p.bidx, p.nan > 0.f);
+      }
+      epi.partials[(int64_t)m * gridDim.x + blockIdx.x] = partial_of(st);
     }
   }
 }
@@ -1849,6 +1891,12 @@ void launch_stream_mb(const void* xp, const void* W, const void* scales, float* 
 
 constexpr int SH_GROUP = 12;  // most tiles per pass of the shared-activation kernel (4 lanes x 3)
 constexpr int SH_GROUP_W8 = 18;  // int8 only: 6 lanes x 3
+// A vocabulary of 16-bit weights (13 or 14 tiles per workgroup) is one pass of a wave per tile over all of K: no
+// sums between waves, the fewest registers and so the most loads in flight.  Measured, 50272 x 4096, us: 8 rows 69
+// -> 64, 32 rows 75 -> 65 (6.3 TB/s; both on the stream kernel before), 40 rows 75 -> 66, 64 rows 95 -> 66, 100 rows
+// 116 -> 93; K = 2048, 64 rows 48 -> 36; K = 9216, 64 rows 199 -> 138.  A third weight stage in flight costs as much as
+// it gives (69 at 64 rows), eight K steps to a stage spill (89).
+constexpr bool vocabulary_tiles(int tiles_per_wg) { return tiles_per_wg == 13 || tiles_per_wg == 14; }
 
 // The shared-activation kernel sweeps K once per pass of SH_GROUP tiles: it is used when the
 // workgroup's tiles fill their passes to at least three quarters.
@@ -1876,7 +1924,10 @@ void launch_share_cfg(const void* xp, const void* W, const void* scales, float* 
                      (const half_t*)scales, part, M, N, K, tiles_per_wg, ks_per_split, epi);
 }
 
-// 33 .. 64 packed rows, no selection: the shared-activation kernel
+// 33 .. 64 packed rows (a vocabulary: from one row on, selections too): the shared-activation kernel.  16-bit weights of
+// one to three tiles per workgroup take a wave per tile and K lane: 12288 x 4096 (three tiles) at 40 / 64 rows 23.7 /
+// 25.6 us on 2 x 4 waves, 21.7 / 23.7 on 4 x 3; 8192 x 2048 (two) 13.0 / 14.0 and 10.7 / 12.0 on 4 x 2; 3072 x 768 and
+// 3072 x 1024 (one) 7.9 / 8.3 and 6.1 / 7.0 on 8 x 1.  Four tiles are as fast either way, int8 weights slower.
 template <int MB, bool W8, int MODE>
 void launch_share(const void* xp, const void* W, const void* scales, float* part, int S, int M,
                   int N, int K, const Epilogue& epi, hipStream_t s) {
@@ -1898,8 +1949,20 @@ void launch_share(const void* xp, const void* W, const void* scales, float* part
     if (tiles_per_wg > 12 && tiles_per_wg <= 18)
       return launch_share_cfg<MB, W8, MODE, 2, 6, 3, 2, 3>(xp, W, scales, part, S, M, N, K,
                                                         tiles_per_wg, gx, ks_per_split, epi, s);
+  } else {
+#define SH_RUN(...)                                                                                           \
+  return launch_share_cfg<MB, W8, MODE, __VA_ARGS__>(xp, W, scales, part, S, M, N, K, tiles_per_wg, gx, \
+                                                     ks_per_split, epi, s)
+    if (vocabulary_tiles(tiles_per_wg)) SH_RUN(1, 14, 1, 4);
+    if constexpr (MB > 2 && MODE != MODE_SELECT) {
+      if (tiles_per_wg == 1) SH_RUN(8, 1, 1, 2);
+      if (tiles_per_wg == 2) SH_RUN(4, 2, 1, 4);
+      if (tiles_per_wg == 3) SH_RUN(4, 3, 1, 2);
+    }
+#undef SH_RUN
   }
-  if (tiles_per_wg <= 4)
+  if constexpr (MB <= 2 || MODE == MODE_SELECT) return;  // (not reached)
+  else if (tiles_per_wg <= 4)
     launch_share_cfg<MB, W8, MODE, 2, 4, 1, 8>(xp, W, scales, part, S, M, N, K, tiles_per_wg, gx,
                                                ks_per_split, epi, s);
   else if (tiles_per_wg <= 8)
@@ -1915,7 +1978,8 @@ void launch_share(const void* xp, const void* W, const void* scales, float* part
 // reduction buffer make 96 KB of LDS).  With so many rows per weight fragment the tiles of a
 // workgroup are few per wave, so more weight stages are kept in flight instead (PF).  Measured
 // at 128 x 12288 x 4096 (38.6 us as built): four K lanes x two tile lanes x two tiles 45.8 us,
-// stages of eight K steps 43.0, six weight stages in flight instead of four 44.3.
+// stages of eight K steps 43.0, six weight stages in flight instead of four 44.3.  16-bit weights: a vocabulary a
+// wave per tile (50272 x 4096 at 128 rows 116 -> 95); four tiles in stages of four K steps (16384 x 4096 38.3 -> 36.3).
 template <bool W8, int MODE>
 void launch_wide(const void* xp, const void* W, const void* scales, float* part, int S, int M,
                  int N, int K, const Epilogue& epi, hipStream_t s) {
@@ -1926,6 +1990,16 @@ void launch_wide(const void* xp, const void* W, const void* scales, float* part,
   const int gx = (ntiles + tiles_per_wg - 1) / tiles_per_wg;
   int ks_per_split = (nks + S - 1) / S;
   if (W8) ks_per_split = (ks_per_split + 1) & ~1;  // int8 blocks cover two steps
+  if constexpr (!W8) {
+    if (vocabulary_tiles(tiles_per_wg))
+      return tiles_per_wg == 13 ? launch_share_cfg<8, W8, MODE, 1, 13, 1, 2>(xp, W, scales, part, S, M, N, K,
+                                                                             tiles_per_wg, gx, ks_per_split, epi, s)
+                                : launch_share_cfg<8, W8, MODE, 1, 14, 1, 2>(xp, W, scales, part, S, M, N, K,
+                                                                             tiles_per_wg, gx, ks_per_split, epi, s);
+    if (tiles_per_wg == 4)
+      return launch_share_cfg<8, W8, MODE, 2, 4, 1, 4>(xp, W, scales, part, S, M, N, K, tiles_per_wg, gx,
+                                                       ks_per_split, epi, s);
+  }
   if (tiles_per_wg <= 4)
     launch_share_cfg<8, W8, MODE, 2, 4, 1, 2, 4>(xp, W, scales, part, S, M, N, K, tiles_per_wg, gx,
                                                  ks_per_split, epi, s);
@@ -1971,6 +2045,15 @@ void launch_stream(const void* xp, const void* W, const void* scales, float* par
                    int N, int K, const Epilogue& epi, hipStream_t s, int64_t m_off = 0) {
   if constexpr (!XR && MODE != MODE_SELECT) {
     if (M > 64) return launch_wide<W8, MODE>(xp, W, scales, part, S, M, N, K, epi, s);
+  }
+  if constexpr (!XR && !W8) {
+    const int G = num_cus() / S < 1 ? 1 : num_cus() / S;
+    if (M <= 64 && vocabulary_tiles((N / 16 + G - 1) / G)) {
+      if (M > 48) return launch_share<4, W8, MODE>(xp, W, scales, part, S, M, N, K, epi, s);
+      if (M > 32) return launch_share<3, W8, MODE>(xp, W, scales, part, S, M, N, K, epi, s);
+      if (M > 16) return launch_share<2, W8, MODE>(xp, W, scales, part, S, M, N, K, epi, s);
+      return launch_share<1, W8, MODE>(xp, W, scales, part, S, M, N, K, epi, s);
+    }
   }
   if (!XR && MODE != MODE_SELECT && M > 32 && share_fits(N, S, W8)) {
     constexpr int PM = MODE == MODE_SELECT ? MODE_PLAIN : MODE;

@@ -749,17 +749,17 @@ class TransformerDecoder(IncrementalDecoder):
                 incremental_state[self._state_key] = cache
             inner = [{"tok": None, "pos": positions, "emb": None}, x_last]
             return feat.view(B, T, D), False, (B, T), {"inner_states": inner}
+        packed = want_packed and M <= 64 and native_out is None
         h, inner_states = self._rows_core(lib, stream, tokens, B, n, T, S0, cache, mask,
-                                          token_embeddings)
-        packed = False
-        features = h.view(B, T, D)
+                                          token_embeddings, want_packed=packed)
+        features = h if packed else h.view(B, T, D)
         cache.length = S0 + T
         if incremental_state is not None:
             incremental_state[self._state_key] = cache
         return features, packed, (B, T), {"inner_states": inner_states}
 
     def _rows_core(self, lib, stream, tokens, B, n, T, S0, kv, mask, token_embeddings=None,
-                   len_dev=None, step_len=None, prompts=None):
+                   len_dev=None, step_len=None, prompts=None, want_packed=False):
         """Prefill (or a decode batch above 128 rows): the last T columns of ``tokens[B, n]``
         through embedding, L layers and the final LayerNorm on row-major activations and the
         tiled MFMA kernels, keys and values written at positions S0 .. S0 + T - 1 of ``kv``
@@ -769,7 +769,8 @@ class TransformerDecoder(IncrementalDecoder):
         and attends up to its own length; ``step_len`` (int32 [B]) receives the lengths the
         step used (-1 for the rows that sat it out).  With ``prompts`` (_Prompts; S0 == 0) the
         pads are dropped behind the embedding: everything runs over the prompts' own rows, one
-        after the other, and their keys and values go to the cache rows they name."""
+        after the other, and their keys and values go to the cache rows they name.  ``want_packed``
+        (at most 64 rows): the features leave in the packed activation layout."""
         cfg = self.cfg
         D = cfg.decoder_embed_dim
         dev = tokens.device
@@ -799,16 +800,16 @@ class TransformerDecoder(IncrementalDecoder):
             after = (None if self.layer_probe is not None else self.layer_norm if last
                      else self.layers[i + 1].self_attn_layer_norm)
             self._rows_layer(lib, stream, layer, x, work, B, T, S0, kv.k(i), kv.v(i),
-                             kv.capacity, mask, len_dev, prompts, after, last)
+                             kv.capacity, mask, len_dev, prompts, after, last and not want_packed)
             if self.layer_probe is not None:
                 self.layer_probe(i, x)
         if self.return_inner_states:
             inner_states.append(x.view(B, T, D).transpose(0, 1).clone())
         else:
             inner_states.append(None)
-        h = work["h"]
+        h = work["hp" if want_packed else "h"]
         if not work["normed"]:
-            self._layernorm(lib, stream, x, self.layer_norm, M, D, h)
+            self._layernorm(lib, stream, x, self.layer_norm, M, D, h, MSA_OUT_PACKED if want_packed else 0)
         return h, inner_states
 
     def _decode_chunks(self, lib, stream, tokens, n, B, cache, mask, lens, S0,
@@ -865,8 +866,8 @@ class TransformerDecoder(IncrementalDecoder):
         """One layer over B * T row-major rows (transformer_decoder_layer.py:233-284): ``x`` is
         the residual stream, updated in place; keys and values of the T new positions of every
         row go to positions S0 .. S0 + T - 1 of ``kc`` / ``vc``.  Where fc2 runs as partial sums, the launch
-        that adds them up also writes the LayerNorm ``after`` that follows (``last``: the decoder's own,
-        row-major): per layer 200 rows 6.6 + 5.4 -> 6.7 us, 57 rows 4.9 + 4.7 -> 4.9."""
+        that adds them up also writes the LayerNorm ``after`` that follows (``last``: row-major whatever the
+        number of rows): per layer 200 rows 6.6 + 5.4 -> 6.7 us, 57 rows 4.9 + 4.7 -> 4.9."""
         cfg = self.cfg
         D, H, hd, F = (cfg.decoder_embed_dim, cfg.decoder_attention_heads, cfg.head_dim,
                        cfg.decoder_ffn_embed_dim)
@@ -1005,9 +1006,9 @@ class TransformerDecoder(IncrementalDecoder):
             raise ValueError("not a slot cache, or slot %d outside 0..%d" % (slot, cache.batch - 1))
         toks = tokens.long().contiguous().view(1, T)
         h, _ = self._rows_core(lib, _capi.stream_ptr(), toks, 1, T, T, 0, _SlotView(cache, slot),
-                               None)
+                               None, want_packed=T <= 64)
         cache.lens[slot:slot + 1].fill_(T)   # (an element assignment waits for the stream)
-        return self._project(h, False, 1, T)[0]
+        return self._project(h, T <= 64, 1, T)[0]
 
     def prefill_slots(self, cache: KVCache, slots, prompts):
         """One prefill for several prompts (1-D id tensors on the device, as for
@@ -1042,10 +1043,11 @@ class TransformerDecoder(IncrementalDecoder):
         for r, t in enumerate(prompts):
             toks[r, :lens[r]] = t
         packed = _Prompts(slots, lens, dev)
+        few = sum(lens) <= 64
         h, _ = self._rows_core(lib, _capi.stream_ptr(), toks, k, Tmax, Tmax, 0, cache, None,
-                               prompts=packed)
+                               prompts=packed, want_packed=few)
         cache.lens[upload(slots, torch.long, dev)] = upload(lens, torch.int32, dev)
-        logits = self._project(h, False, 1, sum(lens))[0]
+        logits = self._project(h, few, 1, sum(lens))[0]
         return list(logits.split(lens))
 
     def decode_slots(self, cache: KVCache, last_tokens: torch.Tensor, *, temperature=1.0,

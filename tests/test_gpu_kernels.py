@@ -1093,6 +1093,42 @@ def test_target_logprob(lib):
     assert torch.allclose(out.cpu(), want, atol=2e-5)
 
 
+@pytest.mark.parametrize("M,N,K", [
+    # 13 and 14 tiles per workgroup: a wave per tile, every number of row blocks, K that ends inside a stage
+    (1, 50272, 96), (16, 54000, 160), (17, 50272, 32), (33, 54000, 64), (48, 50272, 288), (64, 54000, 416),
+    (65, 54000, 96), (128, 50272, 160),
+    # one, two and three tiles per workgroup of 33 to 64 rows, four of more; the last workgroup's tiles run out
+    (33, 4096, 1056), (64, 2304, 96), (48, 8176, 416), (64, 6160, 32), (33, 12272, 224), (64, 12288, 96),
+    (65, 16368, 160), (128, 16384, 96)])
+def test_products_of_a_wave_per_tile(lib, M, N, K):
+    """Against fp32 within one rounding to fp16 and the error of fp32 sums in any order; the greedy choice of a
+    vocabulary is made from the same bits."""
+    print("wave per tile", M, N, K, flush=True)
+    x, w = rnd(M, K, seed=1, std=1.0), rnd(N, K, seed=2, std=K ** -0.5)
+    xp, wp = G(pack_act(x)), pack_w(lib, G(w))
+    y = torch.full((M, N), float("nan"), dtype=torch.float16, device=DEV)
+    ok(lib.msa_linear_f16(P(xp), P(wp), None, None, P(y), M, N, K, IN_PACKED, None), lib)
+    torch.cuda.synchronize()
+    xf, wf = x.double(), w.double()
+    want = xf @ wf.t()
+    bound = 2.0 ** -11 * want.abs() + K * 2.0 ** -23 * (xf.abs() @ wf.abs().t()) + 2.0 ** -25
+    assert bool(((y.cpu().double() - want).abs() <= bound).all())
+    if M > 64 or N < 50000:
+        return
+    logits = torch.empty_like(y)
+    tok, score = torch.zeros(M, dtype=torch.long, device=DEV), torch.zeros(M, device=DEV)
+    ban = (ctypes.c_int32 * 1)(int(y[0].argmax()))
+    ok(lib.msa_lm_head_greedy_select_noalloc_f16(P(xp), P(wp), P(logits), M, N, K, 1.0, ban, 1, ban, 0, None, None, 0,
+                                                 2, P(tok), 1, P(score), 1, None, None), lib)
+    torch.cuda.synchronize()
+    assert torch.equal(logits, y)
+    lp = torch.log_softmax(y.float(), -1)
+    lp[:, ban[0]] = -float("inf")
+    best, at = lp.max(-1)
+    assert torch.equal(lp.gather(1, tok.view(-1, 1)).view(-1), best) and bool((tok <= at).all())
+    assert torch.allclose(score, best, atol=2e-5)
+
+
 @pytest.mark.parametrize("M,V,K", [(1, 96, 64), (17, 2048, 256), (32, 50272, 768), (64, 4000, 128),
                                    (48, 50272, 256)])
 def test_lm_head_fused_selection_matches_projection_then_select(lib, M, V, K):
