@@ -246,6 +246,18 @@ int msa_flash_attention_bf16(const void* q, int64_t ldq, const void* kv, int64_t
                              int64_t ldo, int out_mb, int row0, int heads, int hd, int T, int pos0,
                              float scale, void* stream);
 
+/* The same for up to 32 segments in one launch: segment i is rows row0[i] .. + counts[i] - 1 of q and out, behind pos0[i]
+ * tokens; the expanded rows of its pos0[i] + counts[i] positions follow those of segment i - 1 in kv.  The arrays are
+ * host memory. */
+int msa_flash_attention_segments_bf16(const void* q, int64_t ldq, const void* kv, int64_t ldkv, void* out,
+                                      int64_t ldo, int out_mb, int heads, int hd, int nseg, const int32_t* row0,
+                                      const int32_t* counts, const int32_t* pos0, float scale, void* stream);
+
+/* The first counts[i] latents of cache row slots[i] ([slots, capacity, rp]; at most 32 segments, host arrays), one
+ * segment's behind the other's: [sum of counts, rp]. */
+int msa_gather_latents_bf16(const void* cache, int capacity, int rp, int nseg, const int32_t* slots,
+                            const int32_t* counts, void* out, void* stream);
+
 /* clears columns c0 .. c1 - 1 of an activation matrix */
 int msa_zero_columns(int dtype, void* y, int64_t M, int64_t ld, int mb, int c0, int c1, void* stream);
 /* rows `rows[i]` of an activation matrix (layout src_mb / ld) to row i of another (dst_mb) */

@@ -219,6 +219,9 @@ HYBRID_SIGNATURES = {
                              c_int, _P],
     "msa_flash_attention_bf16": [_P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, c_int, c_int,
                                  c_int, c_int, c_float, _P],
+    "msa_flash_attention_segments_bf16": [_P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, c_int, c_int, _P, _P, _P,
+                                          c_float, _P],
+    "msa_gather_latents_bf16": [_P, c_int, c_int, c_int, _P, _P, _P, _P],
     "msa_zero_columns": [c_int, _P, c_int64, c_int64, c_int, c_int, c_int, _P],
     "msa_gather_rows": [c_int, _P, c_int, _P, c_int, c_int, _P, c_int, _P],
     "msa_step_positions": [_P, _P, c_int64, c_int64, c_int, _P, _P],

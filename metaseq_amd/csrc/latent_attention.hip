@@ -276,8 +276,17 @@ __global__ __launch_bounds__(128) void latent_combine_kernel(const float* __rest
 // online softmax.  Everything is transposed (S^T = K Q^T, O^T = V^T P^T) so that a query's scores lie
 // in one lane (and its partner 32 lanes away) and P^T is the B operand as it stands.  Tiles go
 // through registers into LDS rows padded by 16 bytes, one tile ahead, double buffered.  The query
-// tiles of one head run on one XCD, the longest first.
+// tiles of one head run on one XCD, the longest first.  Several segments share a launch, the longest first: one alone
+// has 160 to 256 workgroups, of which the longest is the launch's time (eight of 530 to 1024 tokens, 32 heads of 128:
+// 240 us one by one, 107 together).
 constexpr int FA_BM = 128, FA_BN = 64;
+constexpr int FA_SEGS = 32;
+struct FlashSegments {
+  int n;
+  int first[FA_SEGS];  // workgroups / 8 before the segment's
+  int row0[FA_SEGS], T[FA_SEGS], pos0[FA_SEGS];  // its rows of q and out; new tokens; tokens before them
+  int kv0[FA_SEGS];    // its first row of kv
+};
 template <int HD>
 constexpr int fa_pitch = HD * 2 + 16;
 template <int HD>
@@ -286,12 +295,15 @@ constexpr int fa_lds_bytes = 2 * 2 * FA_BN * fa_pitch<HD>;
 template <int HD>
 __global__ __launch_bounds__(256) void flash_attention_kernel(
     const bf16_t* __restrict__ q, int64_t ldq, const bf16_t* __restrict__ kv, int64_t ldkv,
-    bf16_t* __restrict__ out, int64_t ldo, int out_mb, int row0, int heads, int T, int pos0,
-    float scale_log2, int n_qt) {
+    bf16_t* __restrict__ out, int64_t ldo, int out_mb, int heads, float scale_log2, FlashSegments segs) {
   constexpr int KSTEPS = HD / 16, DBLK = HD / 32, PITCH = fa_pitch<HD>, TILE = FA_BN * PITCH;
   constexpr int CH = HD / 8, LD = FA_BN * CH / 256;  // chunks per row; loads per thread and tile
   extern __shared__ __attribute__((aligned(16))) char lds[];  // [2][K, V][TILE]
-  const int L = blockIdx.x, xcd = L & 7, seq = L >> 3;
+  const int L = blockIdx.x, xcd = L & 7;
+  int seg = 0;
+  while (seg + 1 < segs.n && (L >> 3) >= segs.first[seg + 1]) ++seg;
+  const int row0 = segs.row0[seg], T = segs.T[seg], pos0 = segs.pos0[seg];
+  const int seq = (L >> 3) - segs.first[seg], n_qt = (T + FA_BM - 1) / FA_BM;
   const int h = (seq / n_qt) * 8 + xcd, qt = n_qt - 1 - seq % n_qt;
   if (h >= heads) return;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -301,12 +313,12 @@ __global__ __launch_bounds__(256) void flash_attention_kernel(
   const int tq = q0 + j, tqc = min(tq, T - 1), pq = pos0 + tqc;
   const int n_keys = pos0 + min(T, qt * FA_BM + FA_BM);
   const int ntiles = (n_keys + FA_BN - 1) / FA_BN;
-  const bf16_t* kb = kv + (int64_t)h * HD;
-  const bf16_t* vb = kv + (int64_t)(heads + h) * HD;
+  const bf16_t* kb = kv + segs.kv0[seg] * ldkv + (int64_t)h * HD;
+  const bf16_t* vb = kb + (int64_t)heads * HD;
 
   bf16x8_t qf[KSTEPS];
   {
-    const bf16_t* qr = q + (int64_t)tqc * ldq + (int64_t)h * HD + hl * 8;
+    const bf16_t* qr = q + (int64_t)(row0 + tqc) * ldq + (int64_t)h * HD + hl * 8;
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks) qf[ks] = *reinterpret_cast<const bf16x8_t*>(qr + ks * 16);
   }
@@ -455,15 +467,30 @@ bool has_decode_kernel(int dtype, int rp) {
   return dtype == MSA_BF16 && (rp == 128 || rp == 192 || rp == 256 || rp == 384 || rp == 512);
 }
 
+// rows of the cache, one segment's behind the other's; 16 bytes per thread
+struct GatherSegments {
+  int n;
+  int first[FA_SEGS], slot[FA_SEGS];  // first row of the result; row of the cache
+};
+__global__ __launch_bounds__(256) void gather_latents_kernel(const bf16_t* __restrict__ cache, int64_t slot_stride,
+                                                             int rp, int rows, GatherSegments segs,
+                                                             bf16_t* __restrict__ out) {
+  const int q = rp / 8, i = blockIdx.x * 256 + threadIdx.x, r = i / q, c = (i - r * q) * 8;
+  if (r >= rows) return;
+  int seg = 0;
+  while (seg + 1 < segs.n && r >= segs.first[seg + 1]) ++seg;
+  *reinterpret_cast<half8_t*>(out + (int64_t)r * rp + c) = *reinterpret_cast<const half8_t*>(
+      cache + segs.slot[seg] * slot_stride + (int64_t)(r - segs.first[seg]) * rp + c);
+}
+
 template <int HD>
 bool run_flash(const void* q, int64_t ldq, const void* kv, int64_t ldkv, void* out, int64_t ldo,
-               int out_mb, int row0, int heads, int T, int pos0, float scale, hipStream_t s) {
+               int out_mb, int heads, float scale, const FlashSegments& segs, int groups, hipStream_t s) {
   static std::atomic<uint64_t> raised{0};
   if (!raise_lds((const void*)flash_attention_kernel<HD>, fa_lds_bytes<HD>, raised)) return false;
-  const int n_qt = (T + FA_BM - 1) / FA_BM;
-  hipLaunchKernelGGL(flash_attention_kernel<HD>, dim3((unsigned)((heads + 7) / 8 * 8 * n_qt)),
-                     dim3(256), fa_lds_bytes<HD>, s, (const bf16_t*)q, ldq, (const bf16_t*)kv, ldkv,
-                     (bf16_t*)out, ldo, out_mb, row0, heads, T, pos0, scale * LOG2E, n_qt);
+  hipLaunchKernelGGL(flash_attention_kernel<HD>, dim3((unsigned)(8 * groups)), dim3(256), fa_lds_bytes<HD>, s,
+                     (const bf16_t*)q, ldq, (const bf16_t*)kv, ldkv, (bf16_t*)out, ldo, out_mb, heads, scale * LOG2E,
+                     segs);
   return true;
 }
 
@@ -534,15 +561,72 @@ extern "C" int msa_flash_attention_bf16(const void* q, int64_t ldq, const void* 
                                         void* out, int64_t ldo, int out_mb, int row0, int heads, int hd,
                                         int T, int pos0, float scale, void* stream) {
   const char* name = "msa_flash_attention_bf16";
-  MSA_REQUIRE(q && kv && out, MSA_ERR_INVALID_ARG, "%s: null pointer", name);
-  MSA_REQUIRE(T > 0 && pos0 >= 0 && row0 >= 0 && heads > 0 && ldq % 8 == 0 && ldkv % 8 == 0 &&
-                  ldkv >= 2 * (int64_t)heads * hd && ldq >= (int64_t)heads * hd && scale > 0.f &&
-                  (out_mb == 0 || row0 + T <= out_mb * 16),
-              MSA_ERR_INVALID_ARG, "%s: T=%d pos0=%d heads=%d hd=%d", name, T, pos0, heads, hd);
+  MSA_REQUIRE(row0 >= 0, MSA_ERR_INVALID_ARG, "%s: row0=%d", name, row0);
+  // (q is the segment's first row there, its own row `row0` here)
+  return msa_flash_attention_segments_bf16(q ? (const bf16_t*)q - row0 * ldq : nullptr, ldq, kv, ldkv, out, ldo, out_mb,
+                                           heads, hd, 1, &row0, &T, &pos0, scale, stream);
+}
+
+extern "C" int msa_gather_latents_bf16(const void* cache, int capacity, int rp, int nseg, const int32_t* slots,
+                                       const int32_t* counts, void* out, void* stream) {
+  const char* name = "msa_gather_latents_bf16";
+  MSA_REQUIRE(cache && out && slots && counts, MSA_ERR_INVALID_ARG, "%s: null pointer", name);
+  MSA_REQUIRE(nseg > 0 && nseg <= FA_SEGS && capacity > 0 && rp > 0 && rp % 8 == 0, MSA_ERR_INVALID_ARG,
+              "%s: nseg=%d capacity=%d rp=%d", name, nseg, capacity, rp);
+  GatherSegments segs{};
+  segs.n = nseg;
+  int64_t rows = 0;
+  for (int i = 0; i < nseg; ++i) {
+    MSA_REQUIRE(slots[i] >= 0 && counts[i] > 0 && counts[i] <= capacity, MSA_ERR_INVALID_ARG,
+                "%s: %d rows of slot %d", name, counts[i], slots[i]);
+    segs.first[i] = (int)rows;
+    segs.slot[i] = slots[i];
+    rows += counts[i];
+    MSA_REQUIRE(rows * (rp / 8) <= 0x7fffff00, MSA_ERR_INVALID_ARG, "%s: too many rows", name);
+  }
+  hipLaunchKernelGGL(gather_latents_kernel, dim3((unsigned)((rows * (rp / 8) + 255) / 256)), dim3(256), 0,
+                     (hipStream_t)stream, (const bf16_t*)cache, (int64_t)capacity * rp, rp, (int)rows, segs,
+                     (bf16_t*)out);
+  MSA_CHECK_LAUNCH(name);
+  return MSA_OK;
+}
+
+extern "C" int msa_flash_attention_segments_bf16(const void* q, int64_t ldq, const void* kv, int64_t ldkv, void* out,
+                                                 int64_t ldo, int out_mb, int heads, int hd, int nseg,
+                                                 const int32_t* row0, const int32_t* counts, const int32_t* pos0,
+                                                 float scale, void* stream) {
+  const char* name = "msa_flash_attention_segments_bf16";
+  MSA_REQUIRE(q && kv && out && row0 && counts && pos0, MSA_ERR_INVALID_ARG, "%s: null pointer", name);
+  MSA_REQUIRE(heads > 0 && hd > 0 && nseg > 0 && nseg <= FA_SEGS && ldq % 8 == 0 && ldkv % 8 == 0 &&
+                  ldkv >= 2 * (int64_t)heads * hd && ldq >= (int64_t)heads * hd && scale > 0.f,
+              MSA_ERR_INVALID_ARG, "%s: nseg=%d heads=%d hd=%d", name, nseg, heads, hd);
+  int order[FA_SEGS], kv0[FA_SEGS];
+  int64_t rows = 0, groups = 0;
+  for (int i = 0; i < nseg; ++i) {
+    MSA_REQUIRE(counts[i] > 0 && pos0[i] >= 0 && row0[i] >= 0 && (out_mb == 0 || row0[i] + counts[i] <= out_mb * 16),
+                MSA_ERR_INVALID_ARG, "%s: T=%d pos0=%d", name, counts[i], pos0[i]);
+    kv0[i] = (int)rows;
+    rows += (int64_t)pos0[i] + counts[i];
+    groups += (int64_t)((heads + 7) / 8) * ((counts[i] + FA_BM - 1) / FA_BM);
+    MSA_REQUIRE(rows <= 0x7fffffff && groups <= 0x7ffffff, MSA_ERR_INVALID_ARG, "%s: too many rows", name);
+    // the segment whose last tile sees most keys first
+    int at = i;
+    for (; at > 0 && pos0[order[at - 1]] + counts[order[at - 1]] < pos0[i] + counts[i]; --at) order[at] = order[at - 1];
+    order[at] = i;
+  }
+  FlashSegments segs{};
+  segs.n = nseg;
+  groups = 0;
+  for (int i = 0; i < nseg; ++i) {
+    const int k = order[i];
+    segs.first[i] = (int)groups;
+    segs.row0[i] = row0[k], segs.T[i] = counts[k], segs.pos0[i] = pos0[k], segs.kv0[i] = kv0[k];
+    groups += (int64_t)((heads + 7) / 8) * ((counts[k] + FA_BM - 1) / FA_BM);
+  }
   bool ok = false;
 #define FA_CASE(HD)                                                                                \
   case HD:                                                                                         \
-    ok = run_flash<HD>(q, ldq, kv, ldkv, out, ldo, out_mb, row0, heads, T, pos0, scale,            \
+    ok = run_flash<HD>(q, ldq, kv, ldkv, out, ldo, out_mb, heads, scale, segs, (int)groups,        \
                        (hipStream_t)stream);                                                       \
     break;
   switch (hd) {

@@ -122,6 +122,10 @@ def test_batch_of_unequal_requests_equals_each_alone(lens, dtype):
         case.check(torch.cat(got[i]), want[i], "request %d of %s" % (i, (lens,)))
 
 
+def test_more_long_requests_than_one_launch_of_attention_takes():
+    test_batch_of_unequal_requests_equals_each_alone(tuple(17 + i % 5 for i in range(34)), BF16)
+
+
 @DTYPES
 def test_slots_are_reused_without_a_trace_of_the_last_request(dtype):
     case = H.Case(H.mixed(dtype), seed=13, dtype=dtype)

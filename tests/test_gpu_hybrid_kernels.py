@@ -477,6 +477,51 @@ def test_flash_attention(hd, T, pos0):
     close(out, ref, 1e-2, "flash %d" % hd)
 
 
+@pytest.mark.parametrize("hd,heads,segs", [
+    (128, 9, [(130, 0), (1, 500), (128, 64), (17, 3), (300, 100)]), (64, 3, [(33, 0)]),
+    (32, 8, [(17 + 3 * i, (5 * i) % 70) for i in range(32)])])
+@pytest.mark.parametrize("packed", [False, True])
+def test_flash_attention_of_several_segments(hd, heads, segs, packed):
+    """The bits that each segment gives by itself, wherever its rows lie."""
+    lib = _capi.load_hybrid()
+    g = gen(hd)
+    gap = 5                     # rows between the segments
+    row0, kv0 = [], [0]
+    for n, p in segs:
+        row0.append(gap + (row0[-1] + segs[len(row0) - 1][0] if row0 else 0))
+        kv0.append(kv0[-1] + n + p)
+    M, D, scale = row0[-1] + segs[-1][0], heads * hd, 1.5 * hd ** -0.5
+    mb = (M + 15) // 16 if packed else 0
+    q = torch.randn(M, D, generator=g).to(BF16).cuda()
+    kv = torch.randn(kv0[-1], 2 * D, generator=g).to(BF16).cuda()
+    out, want = (torch.full((max(M, 16 * mb) * D,), 7.0, dtype=BF16, device="cuda") for _ in range(2))
+    ints = lambda x: (ctypes.c_int32 * len(x))(*x)
+    n, p = zip(*segs)
+    check(lib.msa_flash_attention_segments_bf16(ptr(q), D, ptr(kv), 2 * D, ptr(out), D, mb, heads, hd, len(segs),
+                                                ints(row0), ints(n), ints(p), scale, _capi.stream_ptr()), lib)
+    for i, (n, p) in enumerate(segs):
+        check(lib.msa_flash_attention_bf16(ptr(q[row0[i]:]), D, ptr(kv[kv0[i]:]), 2 * D, ptr(want), D, mb, row0[i],
+                                           heads, hd, n, p, scale, _capi.stream_ptr()), lib)
+    torch.cuda.synchronize()
+    assert torch.equal(out, want) and bool((out != 7.0).any())
+    one = ints([1] * 33)
+    assert lib.msa_flash_attention_segments_bf16(ptr(q), D, ptr(kv), 2 * D, ptr(out), D, mb, heads, hd, 33, one, one,
+                                                 one, scale, _capi.stream_ptr()) == -1
+
+
+def test_gathered_latents():
+    lib = _capi.load_hybrid()
+    for rp, slots, counts in ((512, [3, 0, 2], [70, 1, 33]), (24, [1], [7]), (80, list(range(32)), [9] * 32)):
+        c = torch.randn(32, 70, rp).to(BF16).cuda()
+        out = torch.full((sum(counts) + 1, rp), 7.0, dtype=BF16, device="cuda")
+        ints = lambda x: (ctypes.c_int32 * len(x))(*x)
+        check(lib.msa_gather_latents_bf16(ptr(c), 70, rp, len(slots), ints(slots), ints(counts), ptr(out),
+                                          _capi.stream_ptr()), lib)
+        want = torch.cat([c[s, :n] for s, n in zip(slots, counts)])
+        assert torch.equal(out[:-1], want) and bool((out[-1] == 7.0).all())
+        assert lib.msa_gather_latents_bf16(ptr(c), 70, rp, 1, ints([0]), ints([71]), ptr(out), _capi.stream_ptr()) == -1
+
+
 @pytest.mark.parametrize("dtype", [BF16, F32], ids=["bf16", "f32"])
 @pytest.mark.parametrize("rp", [128, 192, 256, 384, 512, 640])
 def test_latent_attention(rp, dtype):
