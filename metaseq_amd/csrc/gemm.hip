@@ -386,7 +386,7 @@ extern "C" int msa_linear_default_splits_w8a16(int64_t M, int N, int K) {
 }
 
 extern "C" int msa_linear_default_splits_rows(int64_t M, int N, int K) {
-  return pick_row_splits(M, N, K);
+  return pick_row_splits_f16(M, N, K);
 }
 
 extern "C" int msa_linear_f16(const void* x, const void* Wp, const void* bias,

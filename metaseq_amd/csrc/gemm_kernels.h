@@ -2210,7 +2210,7 @@ void launch_quad_partial_w(const void* x, const void* W, float* part, int64_t M,
 }
 
 // fp16: 256 x 64 tiles while their S slices fit the chip in one round; an S beyond that means 256 x 128
-// tiles.  bf16 (prefill-sized products whose sums leave as fp32): the cheapest of all widths.
+// tiles, and one for which those do not fit either 256 x 256 (pick_row_splits).  bf16 (prefill-sized products whose sums leave as fp32): the cheapest of all widths.
 template <int MODE>
 void launch_quad_partial(const void* x, const void* W, float* part, int64_t M, int N, int K, int S,
                          hipStream_t s) {
@@ -2226,6 +2226,7 @@ void launch_quad_partial(const void* x, const void* W, float* part, int64_t M, i
       return launch_quad_partial_w<MODE, 8>(x, W, part, M, N, K, S, s);
     }
   }
+  if (!is_bf<MODE> && M >= TQ_BM && tiles4 > num_cus()) return launch_quad_partial_w<MODE, 8>(x, W, part, M, N, K, S, s);
   if (tiles2 > num_cus())
     return launch_quad_partial_w<MODE, 4>(x, W, part, M, N, K, S, s);
   launch_quad_partial_w<MODE, 2>(x, W, part, M, N, K, S, s);
@@ -2246,6 +2247,18 @@ int pick_row_splits(int64_t M, int N, int K) {
     if (tiles * S <= num_cus() && K % (64 * S) == 0 && K / S >= 512) best = S;
   if (best > 1 && best < 8 && M > 128 && K / best >= 4096 && K % (128 * best) == 0) best *= 2;
   return best;
+}
+
+// The same for fp16 prompts whose tail adds the slices: two of a long sum (K of 8192 or more) whose 256 x 256 tiles
+// fill half of the chip or less.  One slice takes 256 x 128 tiles there, at 0.61 of the wide tiles' time for half of
+// their work.  Product, tail and LayerNorm, cold weights, one slice and two: 4096 x 16384 over 1025 rows 233 and 190 us,
+// 1607 218 and 196, 2048 243 and 224; 2048 x 8192 over 2100 rows 109 and 99, 3000 112 and 108, 3584 121 and 120, 4096 132
+// and 136: the shorter sum up to three quarters of the chip.
+int pick_row_splits_f16(int64_t M, int N, int K) {
+  const int few = pick_row_splits(M, N, K);
+  if (few > 1 || M < TQ_BM || N % 16 || K % 128 || K < 8192) return few;
+  const int64_t rows = (M + TQ_BM - 1) / TQ_BM, tiles8 = rows * ((N + 255) / 256), tiles4 = rows * ((N + 127) / 128);
+  return tiles8 * 2 <= num_cus() * (K >= 16384 ? 4 : 3) / 4 && tiles4 * 2 > num_cus() ? 2 : 1;
 }
 
 // The same for sums that leave as fp32 from any width of tile (bf16): also two slices of prompts' products whose

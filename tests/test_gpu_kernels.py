@@ -665,6 +665,19 @@ def test_split_k_partials_of_row_major_rows(lib, M, N, K, S):
     assert_fp16_close(h, want_h, max_ulp=2, max_frac=2e-2, atol=4 * atol, what="fused LN")
 
 
+@pytest.mark.parametrize("M,N,K", [(1025, 4096, 256), (1100, 4112, 384), (2048, 4080, 512), (257, 16384, 256)])
+def test_two_slices_of_wide_tiles(lib, M, N, K):
+    """Slices that do not fit one round of 256 x 128 tiles: 256 x 256 ones, the last row of them moved up."""
+    test_split_k_partials_of_row_major_rows(lib, M, N, K, 2)
+
+
+def test_which_sums_of_prompts_are_cut_in_two(lib):
+    f = lib.msa_linear_default_splits_rows
+    assert [f(M, 4096, 16384) for M in (1025, 1607, 2048, 2049)] == [2, 2, 2, 1]
+    assert [f(M, 2048, 8192) for M in (2100, 3072, 3073, 4096)] == [2, 2, 1, 1]
+    assert f(1607, 4096, 4096) == 1
+
+
 def test_split_k_of_row_major_rows_rejects_and_suggestion(lib):
     x = torch.zeros(256, 4096, dtype=torch.float16, device=DEV)
     part = torch.zeros(8 * 256 * 64, dtype=torch.float32, device=DEV)
