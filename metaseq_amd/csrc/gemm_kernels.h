@@ -1244,51 +1244,32 @@ __device__ __forceinline__ void tq_static_for(F&& f) {
 
 // 8 consecutive output columns n..n+7 of row m; v holds the accumulators rounded to fp16, b the
 // bias and r the residual values of those columns (read only where the epilogue has them)
-// (QKV mode: qb, qt = the row's batch row and its position behind the cache's first s0)
-template <int MODE>
-__device__ __forceinline__ void epilogue8(const Epilogue& e, int64_t m, int n, half8_t v,
-                                          half8_t b, half8_t r, int qb, int qt, int s0) {
-  float t[8];
+__device__ __forceinline__ void biased8(const Epilogue& e, half8_t v, half8_t b, float (&t)[8]) {
 #pragma unroll
   for (int i = 0; i < 8; ++i) t[i] = (float)v[i];
   if (e.bias) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) t[i] = round_h(t[i] + (float)b[i]);
   }
+}
+__device__ __forceinline__ void epilogue8(const Epilogue& e, int64_t m, int n, half8_t v, half8_t b, half8_t r) {
+  float t[8];
+  biased8(e, v, b, t);
   half8_t o;
-  if (MODE == MODE_PLAIN) {
-    if (e.flags & MSA_EPI_RELU) {
+  if (e.flags & MSA_EPI_RELU) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) t[i] = fmaxf(t[i], 0.f);
-    }
-    if (e.residual) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) t[i] = round_h(t[i] + (float)r[i]);
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) o[i] = (half_t)t[i];
-    if (e.out_mb > 0)
-      *reinterpret_cast<half8_t*>(e.y + packed_act_offset((int)m, n, e.out_mb)) = o;
-    else
-      *reinterpret_cast<half8_t*>(e.y + m * e.N + n) = o;
-  } else {
-    const int D = e.H * e.hd;
-    const int part = (n >= D) + (n >= 2 * D), c = n - part * D;  // 0 = K, 1 = V, 2 = Q
-    if (part == 2) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) o[i] = (half_t)(t[i] * e.qscale);
-      *reinterpret_cast<half8_t*>(e.q_out + m * D + c) = o;
-    } else {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) o[i] = (half_t)t[i];
-      const int h = e.hd_shift >= 0 ? c >> e.hd_shift : c / e.hd, d = c - h * e.hd;
-      if (s0 >= 0 && s0 + qt < e.S_cap) {
-        half_t* dst = (part == 0 ? e.Kc : e.Vc) +
-                      (((int64_t)qb * e.H + h) * e.S_cap + s0 + qt) * e.hd + d;
-        *reinterpret_cast<half8_t*>(dst) = o;
-      }
-    }
+    for (int i = 0; i < 8; ++i) t[i] = fmaxf(t[i], 0.f);
   }
+  if (e.residual) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) t[i] = round_h(t[i] + (float)r[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) o[i] = (half_t)t[i];
+  if (e.out_mb > 0)
+    *reinterpret_cast<half8_t*>(e.y + packed_act_offset((int)m, n, e.out_mb)) = o;
+  else
+    *reinterpret_cast<half8_t*>(e.y + m * e.N + n) = o;
 }
 
 // Row tiles of a grouped product (routed experts): tile t holds rows tile_row[t] .. of group
@@ -1654,26 +1635,35 @@ __device__ __forceinline__ void quad_tile(const half_t* __restrict__ x, const vo
   };
 #pragma unroll
   for (int i = 0; i < TQ_RES_AHEAD; ++i) load_res(i, res8[i]);
-  // QKV mode: the lane's rows come ERPI apart, so (batch row, position) of a row follow from the
-  // previous row's without a division
-  int qb = 0, qt = 0;
-  if (MODE == MODE_QKV) {
-    const int mf = (int)(m0 + wm * (TQ_BM / 2) + erow);
-    qb = epi.T == 1 ? mf : mf / epi.T;
-    qt = mf - qb * epi.T;
-  }
-  // rows with positions (and cache rows) of their own: all of the lane's are read in front of its first store, behind
-  // which none would be in flight
-  int own_at[MODE == MODE_QKV ? RF : 1][ENR], own_row[MODE == MODE_QKV ? RF : 1][ENR];
-  if (MODE == MODE_QKV && epi.len_dev) {
+  // QKV mode: where a row's keys and values go (elements in front of its first head's, -1: nowhere) is worked out
+  // once per row, two rows to a lane, and kept in LDS; the lane's columns are the same in every iteration, so their part
+  // and head are constants.  (Kept in registers instead, positions, cache rows and divisions spilled 196 of
+  // them: 1607 x 12288 x 4096 into cache rows of their own 179 us, now 156, as the plain product; 3000 rows 277 and 243.)
+  const int64_t* place = reinterpret_cast<const int64_t*>(tq_lds + 32768 + wave * (TQ_BM / 2 * 8));
+  half_t* to = nullptr;
+  int qkv_part = 0;
+  if constexpr (MODE == MODE_QKV) {
+    int64_t* fill = reinterpret_cast<int64_t*>(tq_lds + 32768 + wave * (TQ_BM / 2 * 8));
 #pragma unroll
-    for (int i = 0; i < (MODE == MODE_QKV ? RF : 0); ++i)
-#pragma unroll
-      for (int r = 0; r < ENR; ++r) {
-        const int m = (int)min(m0 + wm * (TQ_BM / 2) + i * 16 + ERPI * r + erow, M - 1);
-        own_at[i][r] = epi.len_dev[m];
-        own_row[i][r] = epi.row_dev ? epi.row_dev[m] : m;
+    for (int k = 0; k < TQ_BM / 2; k += 64) {
+      const int m = (int)min(m0 + wm * (TQ_BM / 2) + k + lane, M - 1);
+      int b = m, at = epi.S0;
+      bool ok = epi.S0 >= 0;
+      if (epi.len_dev) {
+        at = epi.len_dev[m];
+        if (epi.row_dev) b = epi.row_dev[m];
+        ok = at >= 0;
+      } else if (epi.T > 1) {
+        b = m / epi.T;
+        at += m - b * epi.T;
       }
+      fill[k + lane] = ok && at < epi.S_cap ? ((int64_t)b * epi.H * epi.S_cap + at) * epi.hd : -1;
+    }
+    const int D = epi.H * epi.hd;
+    qkv_part = (en >= D) + (en >= 2 * D);  // 0 = K, 1 = V, 2 = Q
+    const int c = en - qkv_part * D, h = epi.hd_shift >= 0 ? c >> epi.hd_shift : c / epi.hd;
+    to = qkv_part == 2 ? epi.q_out + c
+                       : (qkv_part == 0 ? epi.Kc : epi.Vc) + (int64_t)h * epi.S_cap * epi.hd + (c - h * epi.hd);
   }
 #pragma unroll
   for (int i = 0; i < RF; ++i) {
@@ -1693,15 +1683,20 @@ __device__ __forceinline__ void quad_tile(const half_t* __restrict__ x, const vo
                                                           ((ec ^ (row & (ECH - 1))) * 16));
       const int64_t m = m0 + wm * (TQ_BM / 2) + i * 16 + row;
       if (col_ok && m >= m_own && m < M) {
-        if (MODE == MODE_QKV && epi.len_dev)
-          epilogue8<MODE>(epi, m, en, v, bias8, bias8, own_row[MODE == MODE_QKV ? i : 0][r], 0,
-                          own_at[MODE == MODE_QKV ? i : 0][r]);
-        else
-          epilogue8<MODE>(epi, m, en, v, bias8, res8[i % TQ_RES_AHEAD][r], qb, qt, epi.S0);
-      }
-      if (MODE == MODE_QKV) {
-        qt += ERPI;
-        while (qt >= epi.T) qt -= epi.T, ++qb;
+        if constexpr (MODE == MODE_QKV) {
+          const int64_t at = qkv_part == 2 ? m * (epi.H * epi.hd) : place[i * 16 + row];
+          if (at >= 0) {
+            float t[8];
+            biased8(epi, v, bias8, t);
+            half8_t o;
+            const float scale = qkv_part == 2 ? epi.qscale : 1.f;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) o[k] = (half_t)(t[k] * scale);
+            *reinterpret_cast<half8_t*>(to + at) = o;
+          }
+        } else {
+          epilogue8(epi, m, en, v, bias8, res8[i % TQ_RES_AHEAD][r]);
+        }
       }
     }
     if (i + TQ_RES_AHEAD < RF) load_res(i + TQ_RES_AHEAD, res8[i % TQ_RES_AHEAD]);
