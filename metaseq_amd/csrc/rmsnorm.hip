@@ -83,10 +83,28 @@ __global__ __launch_bounds__(NT) void embed_kernel(
   if (w) norm_out<T, NV, NT>(v, m, D, Dp, eps, w, h, mb, red);
 }
 
-// b += the sum of S slices of row m; four slices at a time, their loads in flight together
+// b += the sum of S slices of row m; four slices at a time, their loads in flight together.  One or two slices (prompts)
+// are read without a condition of their own around any load.
 template <int NV, int NT>
 __device__ __forceinline__ void sum_slices(const float* part, int S, int M, int64_t m, int Dp,
                                            float4_t (&b)[NV]) {
+  if (S <= 2) {
+    float4_t v[2][NV];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      if (s == S) break;  // uniform
+      const float* p = part + ((int64_t)s * M + m) * Dp;
+#pragma unroll
+      for (int i = 0; i < NV; ++i)
+        v[s][i] = *reinterpret_cast<const float4_t*>(p + min((int)(threadIdx.x + i * NT) * 4, Dp - 4));
+    }
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      if (S == 2) v[0][i] += v[1][i];
+      b[i] += (int)(threadIdx.x + i * NT) * 4 < Dp ? v[0][i] : float4_t{0.f, 0.f, 0.f, 0.f};
+    }
+    return;
+  }
   for (int s0 = 0; s0 < S; s0 += 4) {
     float4_t v[4][NV];
 #pragma unroll
@@ -308,6 +326,19 @@ constexpr auto tail_two = tail_kernel<T, NV, NT, true>;
     else RN_RUN(KERNEL, T, 4, 1024, M, __VA_ARGS__);                                        \
   } while (0)
 
+// The tail of many rows takes twice the threads: half of a row's operands per thread, all in flight (and four routed
+// terms at a time), so that more rows share a compute unit.  6038 x 4096, us: one fp32 slice 90 -> 70, eight routed
+// terms 172 -> 118; 1500 x 4096 in two slices 28 -> 23, two sublayers of two slices 38 -> 27.  1024 threads are slower (93
+// on average against 81); rows of 2048 (two operands per thread of 256) and the embedding have nothing to gain (40.7
+// against 43.0; 59 and 61).
+#define RN_DISPATCH_TAIL(KERNEL, T, M, Dp, ...)                                             \
+  do {                                                                                      \
+    const int q_ = (Dp) / 4;                                                                \
+    if ((M) > RN_FEW_ROWS && q_ > 512 && q_ <= 1024) RN_RUN(KERNEL, T, 2, 512, M, __VA_ARGS__); \
+    else if ((M) > RN_FEW_ROWS && q_ > 1024 && q_ <= 2048) RN_RUN(KERNEL, T, 2, 1024, M, __VA_ARGS__); \
+    else RN_DISPATCH(KERNEL, T, M, Dp, __VA_ARGS__);                                        \
+  } while (0)
+
 }  // namespace
 
 extern "C" int msa_embed_rmsnorm(int dtype, const int64_t* tokens, const int32_t* tok_pos, int M,
@@ -344,13 +375,13 @@ extern "C" int msa_residual_rmsnorm_tail(const msa_tail_args* a, void* stream) {
   MSA_REQUIRE(!a->bias || a->part, MSA_ERR_INVALID_ARG, "%s: a bias without a product", name);
   if (a->part2) {
     if (a->dtype == MSA_BF16)
-      RN_DISPATCH(tail_two, bf16_t, a->M, a->Dp, *a);
+      RN_DISPATCH_TAIL(tail_two, bf16_t, a->M, a->Dp, *a);
     else
-      RN_DISPATCH(tail_two, float, a->M, a->Dp, *a);
+      RN_DISPATCH_TAIL(tail_two, float, a->M, a->Dp, *a);
   } else if (a->dtype == MSA_BF16) {
-    RN_DISPATCH(tail_one, bf16_t, a->M, a->Dp, *a);
+    RN_DISPATCH_TAIL(tail_one, bf16_t, a->M, a->Dp, *a);
   } else {
-    RN_DISPATCH(tail_one, float, a->M, a->Dp, *a);
+    RN_DISPATCH_TAIL(tail_one, float, a->M, a->Dp, *a);
   }
   MSA_CHECK_LAUNCH(name);
   return MSA_OK;

@@ -264,6 +264,35 @@ def test_tail_of_two_sides_with_loop_terms(M, D, dtype):
         close(hd[:, :D], h, 6e-3 if dtype == BF16 else 3e-6, "normed")
 
 
+@pytest.mark.parametrize("D", [3000, 4096, 4104])
+def test_tail_of_many_wide_rows(D):
+    test_tail_of_two_sides_with_loop_terms(1030, D, BF16)
+
+
+@pytest.mark.parametrize("M,D,top", [(1025, 4000, 3), (1025, 4096, 8), (1030, 8000, 5), (7, 4096, 5)])
+def test_tail_of_routed_terms(M, D, top):
+    """A gated sum and the routed terms, wherever their rows lie."""
+    lib = _capi.load_hybrid()
+    g = gen(M + top)
+    Dp, eps = (D + 63) // 64 * 64, 1e-5
+    x, part, pairs = (torch.zeros(n, Dp) for n in (M, M, M * top))
+    for t in (x, part, pairs):
+        t[:, :D] = torch.randn(len(t), D, generator=g)
+    pairs = pairs.to(BF16)
+    weight, gate = torch.rand(M, top, generator=g), torch.rand(M, generator=g)
+    inverse = torch.randperm(M * top, generator=g).view(M, top)
+    want = x.double() + part.double() * gate.double().view(M, 1)
+    for k in range(top):
+        want += weight[:, k:k + 1].double() * pairs[inverse[:, k]].double()
+    dev = [t.cuda() for t in (x, part, pairs, weight, gate, inverse.int())]
+    a = _capi.TailArgs()
+    a.dtype, a.M, a.D, a.Dp, a.S, a.eps = 0, M, D, Dp, 1, eps
+    a.x, a.part, a.pair_y, a.pair_w, a.gate, a.inverse = (ptr(t) for t in dev)
+    a.top = top
+    check(lib.msa_residual_rmsnorm_tail(ctypes.byref(a), _capi.stream_ptr()), lib)
+    close(dev[0], want, 2e-6, "stream")
+
+
 def _grouped(lib, dtype, heads, kv_heads, hd, vd, chunk, rot, segments, capacity, seed, fused=None):
     """One step of grouped attention over ``segments`` ((slot, first position, tokens)) through the
     three calls; returns its outputs and the caches with what they should be."""
