@@ -304,7 +304,11 @@ __global__ __launch_bounds__(256) void flash_attention_kernel(
   while (seg + 1 < segs.n && (L >> 3) >= segs.first[seg + 1]) ++seg;
   const int row0 = segs.row0[seg], T = segs.T[seg], pos0 = segs.pos0[seg];
   const int seq = (L >> 3) - segs.first[seg], n_qt = (T + FA_BM - 1) / FA_BM;
-  const int h = (seq / n_qt) * 8 + xcd, qt = n_qt - 1 - seq % n_qt;
+  // few workgroups: the longest tiles of all heads first (one segment of 1500 tokens 72 us -> 60); many: head by head, one
+  // head's rows in L2
+  const bool spread = gridDim.x <= 1024;
+  const int hg = (heads + 7) / 8, h = (spread ? seq % hg : seq / n_qt) * 8 + xcd;
+  const int qt = n_qt - 1 - (spread ? seq / hg : seq % n_qt);
   if (h >= heads) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
