@@ -264,6 +264,36 @@ def test_tail_of_two_sides_with_loop_terms(M, D, dtype):
         close(hd[:, :D], h, 6e-3 if dtype == BF16 else 3e-6, "normed")
 
 
+@pytest.mark.parametrize("dtype", [BF16, F32], ids=["bf16", "f32"])
+@pytest.mark.parametrize("M,heads,vdim,off", [(1, 1, 5, 0), (17, 3, 40, 0), (5, 7, 64, 0), (33, 5, 100, 0),
+                                              (40, 9, 128, 0), (3, 2, 200, 0), (9, 3, 256, 0), (5, 3, 300, 0),
+                                              (2, 1, 512, 0), (17, 3, 40, 1), (6, 2, 300, 2)])
+def test_delta_output(M, heads, vdim, off, dtype):
+    """Norm and gate of every head's outputs, row-major and packed; gates that lie `off` elements off alignment."""
+    lib = _capi.load_hybrid()
+    g = gen(M + vdim)
+    vp, eps = (vdim + 15) // 16 * 16, 1e-4
+    o, w = torch.zeros(M, heads, vp), torch.zeros(vp)
+    o[..., :vdim], w[:vdim] = torch.randn(M, heads, vdim, generator=g), torch.randn(vdim, generator=g)
+    z = torch.randn(M, heads * vp + 8, generator=g).to(dtype)
+    gate = z[:, off:off + heads * vp].double().view(M, heads, vp)
+    od, wd, zd = o.cuda(), w.cuda(), z.cuda()
+    for act, packed in ((0, False), (1, False), (0, True)):
+        if packed and (dtype == F32 or heads * vp % 32 or M > 128):
+            continue
+        want = o.double() * torch.rsqrt((o.double() ** 2).sum(-1, keepdim=True) / vdim + eps) * w.double()
+        want = (want * (torch.sigmoid(gate) if act else torch.nn.functional.silu(gate))).view(M, -1)
+        mb = (M + 15) // 16 if packed else 0
+        out = torch.full((mb * 16 if packed else M, heads * vp), 7.0, dtype=dtype, device="cuda")
+        a = _capi.DeltaArgs()
+        a.dtype, a.heads, a.vdim, a.vp, a.eps, a.gate_act = int(dtype == F32), heads, vdim, vp, eps, act
+        a.o, a.w, a.gate, a.ld_gate = ptr(od), ptr(wd), ptr(zd[:, off:]), z.shape[1]
+        a.out, a.ld_out, a.out_mb = ptr(out), heads * vp, mb
+        check(lib.msa_delta_output(ctypes.byref(a), M, _capi.stream_ptr()), lib)
+        got = unpack_rows(out.view(-1).cpu(), M, heads * vp) if packed else out
+        close(got, want, 6e-3 if dtype == BF16 else 3e-6, "act %d packed %d" % (act, packed))
+
+
 @pytest.mark.parametrize("D", [3000, 4096, 4104])
 def test_tail_of_many_wide_rows(D):
     test_tail_of_two_sides_with_loop_terms(1030, D, BF16)
