@@ -289,7 +289,7 @@ int lm_head_select_impl(const char* name, const void* x, const void* Ep, void* l
   IdList stop{};
   stop.n = n_stop;
   for (int i = 0; i < n_stop; ++i) stop.id[i] = stop_host[i];
-  // same decomposition as launch_stream_mb at S = 1: the partial stride is its grid size
+  // same decomposition as launch_stream_mb and launch_share at S = 1: the partial stride is the grid size
   const int ntiles = V / 16;
   const int tiles_per_wg = (ntiles + num_cus() - 1) / num_cus();
   const int gx = (ntiles + tiles_per_wg - 1) / tiles_per_wg;

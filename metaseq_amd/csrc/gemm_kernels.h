@@ -8,15 +8,17 @@
 //
 // Five kernels:
 //   * stream (M <= 32 packed rows, the decode step; also the fused vocabulary projection +
-//     selection up to 64 rows): HBM-bound.  A workgroup of 8 waves owns a contiguous range of
-//     16-row tiles (and, with split-K, one K range); it walks the tiles 3 or 4 at a time, the
-//     waves taking interleaved K steps.  Activations come in the matching packed fragment
-//     layout from L2 and every activation fragment is reused for the tiles of the group.
-//     Fragments are double buffered several steps deep and the prefetch runs across tile-group
-//     boundaries, so the memory pipe never drains while a finished group is reduced across
-//     the waves through LDS (fixed order: results are run-to-run deterministic).
-//   * shared-activation stream (33 .. 64 packed rows): the same weight streaming, with the
-//     activation fragments staged once per workgroup in LDS and shared by four waves.
+//     selection of up to 64 rows where the next kernel does not take it): HBM-bound.  A
+//     workgroup of 8 waves owns a contiguous range of 16-row tiles (and, with split-K, one K
+//     range); it walks the tiles 3 or 4 at a time (1 or 2 where it has no more), the waves taking
+//     interleaved K steps.  Activations come in the matching packed fragment layout from L2 and
+//     every activation fragment is reused for the tiles of the group.  Fragments are double
+//     buffered several steps deep and the prefetch runs across tile-group boundaries, so the
+//     memory pipe never drains while a finished group is reduced across the waves through LDS
+//     (fixed order: results are run-to-run deterministic).
+//   * shared-activation stream (33 .. 128 packed rows; vocabularies of 16-bit weights and their
+//     selection from one row on): the same weight streaming, with the activation fragments staged
+//     once per workgroup in LDS and shared by its waves.
 //   * large tiled, fp16 weights (prefill-sized M): 256 x 256 per workgroup of four waves of
 //     128 x 128 with their accumulators in the AGPR bank, both operands global -> LDS directly.
 //   * large tiled, int8 weights: 256 x 256 x 64 per workgroup of eight waves, weights straight
@@ -610,10 +612,10 @@ __global__ __launch_bounds__(KG * 64) void linear_stream_kernel(
   }
 }
 
-// ---- shared-activation stream kernel (33 .. 64 rows) ------------------------------------------
+// ---- shared-activation stream kernel (33 .. 128 rows; vocabularies from one row on) ------------
 // With more than 32 activation rows a wave that loads its own activation fragments moves more
 // bytes of activations (from L2) than of weights (from HBM) through the L1, and the L1 fill rate
-// becomes the limit.  Here the 8 waves form KL K lanes x NG tile lanes: the NG waves of a K lane
+// becomes the limit.  Here the waves form KL K lanes x NG tile lanes: the NG waves of a K lane
 // work on different weight tiles over the same K steps and read their activation fragments from
 // LDS, which the whole workgroup fills once per stage (SK = KL * U consecutive K steps, one
 // contiguous piece of the packed activations).  Weights still go from HBM straight to registers.
