@@ -180,7 +180,8 @@ typedef struct {
 int msa_delta_scan(const msa_delta_args* a, const msa_batch* b, void* stream);
 /* The same with scratch of at least msa_delta_scratch_floats, with which it takes sixteen tokens at a time on the
  * matrix cores (fp32); 0 where that does not pay (short segments) or does not exist (keys beyond 128): then it
- * needs no scratch and goes token by token. */
+ * needs no scratch and goes token by token.  The size follows from heads, dp, vp (not set yet: enough for any) and
+ * whether decay is NULL, and from M, nseg and max_count of the batch. */
 int64_t msa_delta_scratch_floats(const msa_delta_args* a, const msa_batch* b);
 int msa_delta_scan_chunks(const msa_delta_args* a, const msa_batch* b, float* scratch, int64_t scratch_floats,
                           void* stream);

@@ -821,7 +821,8 @@ constexpr int DC_FROM = 96, DC_FROM_WIDE = 48;
 extern "C" int64_t msa_delta_scratch_floats(const msa_delta_args* a, const msa_batch* b) {
   if (!a || !b || a->heads <= 0 || a->dp > 128) return 0;
   if (b->max_count < ((int64_t)b->nseg * a->heads >= DC_WIDE ? DC_FROM_WIDE : DC_FROM)) return 0;
-  const int ready = wide_tiles(*a, b) ? 0 : 3 * DC_TOK * a->dp + (a->decay ? a->dp : 0);
+  // (a caller that has not set vp gets enough for any)
+  const int ready = a->vp > 0 && wide_tiles(*a, b) ? 0 : 3 * DC_TOK * a->dp + (a->decay ? a->dp : 0);
   return ((int64_t)b->M / DC_TOK + b->nseg) * a->heads * (DC_REC + ready);
 }
 

@@ -312,28 +312,28 @@ int Run::delta_core(const msa_hybrid_layer& l, const msa_hybrid_state& st, char*
   const int C = 2 * l.kv_heads * l.dp + l.heads * l.vp;
   void* qkv = alloc((int64_t)M * C * es);
   const bool step = b.max_count == 1;
-  t.o = step ? nullptr : (float*)alloc((int64_t)M * l.heads * l.vp * 4);
+  t.dtype = d->cfg.dtype;
   t.heads = l.heads;
+  t.kv_heads = l.kv_heads;
+  t.dim = l.dim;
   t.dp = l.dp;
-  const int64_t scratch_floats = step ? 0 : msa_delta_scratch_floats(&t, &b);
+  t.vdim = l.vdim;
+  t.vp = l.vp;
+  t.qkv = qkv;
+  t.ld = C;
+  t.state = st.rec;
+  t.o = step ? nullptr : (float*)alloc((int64_t)M * l.heads * l.vp * 4);
+  t.w = l.o_norm;
+  t.eps = d->cfg.eps;
+  t.out = out.p;
+  t.ld_out = out.ld;
+  t.out_mb = mb;
+  const int64_t scratch_floats = step ? 0 : msa_delta_scratch_floats(&t, &b);  // (reads the sizes set above)
   float* scratch = scratch_floats > 0 ? (float*)alloc(scratch_floats * 4) : nullptr;
   if (!dry) {
     HY(msa_short_conv(d->cfg.dtype, in, ld, C, l.taps, nullptr, l.conv_w, nullptr, 1, qkv, C, st.conv, &b,
                       stream));
     HY(msa_conv_state(d->cfg.dtype, in, ld, C, l.taps, st.conv, &b, stream));
-    t.dtype = d->cfg.dtype;
-    t.kv_heads = l.kv_heads;
-    t.dim = l.dim;
-    t.vdim = l.vdim;
-    t.vp = l.vp;
-    t.qkv = qkv;
-    t.ld = C;
-    t.state = st.rec;
-    t.w = l.o_norm;
-    t.eps = d->cfg.eps;
-    t.out = out.p;
-    t.ld_out = out.ld;
-    t.out_mb = mb;
     if (step) {
       HY(msa_delta_step(&t, &b, stream));
     } else {

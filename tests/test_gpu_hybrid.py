@@ -122,6 +122,27 @@ def test_batch_of_unequal_requests_equals_each_alone(lens, dtype):
         case.check(torch.cat(got[i]), want[i], "request %d of %s" % (i, (lens,)))
 
 
+@DTYPES
+@pytest.mark.parametrize("heads,vdim,lens", [(16, 96, (48, 60, 51, 49, 64, 48, 50, 100)), (16, 40, (48,) * 8),
+                                             (64, 24, (70, 33)), (128, 16, (50,))], ids=str)
+@pytest.mark.parametrize("kind", ["delta", "parallel"])
+def test_delta_heads_of_any_width_in_batches_that_fill_the_chip(kind, heads, vdim, lens, dtype):
+    """128 (segment, head) pairs or more, values that are not whole groups of 64 columns: prompts in one call and their
+    continuation in another, every row as if the request were alone."""
+    if kind == "delta":
+        cfg = H.config([(H.delta(heads=heads, kv_heads=2, dim=24, vdim=vdim, conv=2), None)])
+    else:
+        cfg = H.looped([(H.parallel(delta_heads=heads, delta_kv_heads=2, delta_dim=24, delta_vdim=vdim), None)])
+    case = H.Case(cfg, seed=13, dtype=dtype, tweak=H.steady if kind == "parallel" else None)
+    more = 49
+    toks = [case.tokens(n + more, seed=70 + i) for i, n in enumerate(lens)]
+    cache = case.decoder.new_slot_cache(len(lens), 256)
+    first = case.decoder.extend(cache, [(i, t[:n].cuda()) for i, (t, n) in enumerate(zip(toks, lens))], want_all=True)
+    then = case.decoder.extend(cache, [(i, t[n:].cuda()) for i, (t, n) in enumerate(zip(toks, lens))], want_all=True)
+    for i, (a, b) in enumerate(zip(first.split(list(lens)), then.split(more))):
+        case.check(torch.cat([a, b]), case.want(toks[i]), "%s, request %d" % (kind, i))
+
+
 def test_more_long_requests_than_one_launch_of_attention_takes():
     test_batch_of_unequal_requests_equals_each_alone(tuple(17 + i % 5 for i in range(34)), BF16)
 

@@ -250,6 +250,69 @@ def test_delta_arguments_keep_their_layout():
     assert lib.msa_delta_scan_chunks(*to, ctypes.c_void_p(4096), need, None) == -1
 
 
+def _delta_decoder(lib, heads, vdim, per_channel):
+    """A decoder of one layer without a feed-forward, its pointers never followed: a delta layer, or, with decays per
+    channel, one beside attention."""
+    t, cfg, h = _capi.HybridLayer(), _capi.HybridConfigC(), ctypes.c_void_p()
+    for s in (t, t.att, cfg):
+        for name, kind in s._fields_:
+            if kind is ctypes.c_void_p:
+                setattr(s, name, 4096)
+    vp = (vdim + 15) // 16 * 16
+    t.kind, t.heads, t.kv_heads, t.dim, t.dp = (3 if per_channel else 2), heads, 1, 128, 128
+    t.vdim, t.vp, t.taps, t.scale, t.ff_kind = vdim, vp, 3, 1.0, _capi.MSA_FF_NONE
+    t.ko = max(128, (heads * vp + 63) // 64 * 64)
+    C = 2 * t.dp + heads * vp
+    t.n_in = C + heads * vp + 2 * heads
+    if per_channel:
+        a = t.att
+        a.heads, a.kv_heads, a.hd, a.vd, a.chunk, a.rot_dims, a.ko, a.scale = 1, 1, 16, 16, 0, 0, 128, 1.0
+        t.lr = 128
+        t.n_in = 3 * 16 + C + 128 + 1 + heads
+    t.n_in = (t.n_in + 15) // 16 * 16
+    cfg.dtype, cfg.layers, cfg.D, cfg.Dp, cfg.vocab, cfg.Vp, cfg.eps = 0, 1, 128, 128, 16, 16, 1e-6
+    cfg.n_runs = 0
+    assert lib.msa_hybrid_create(ctypes.byref(cfg), (_capi.HybridLayer * 1)(t), ctypes.byref(h)) == 0, \
+        lib.msa_last_error()
+    return h, t
+
+
+def _batch_of(lens):
+    start = [sum(lens[:i]) for i in range(len(lens) + 1)]
+    b = _capi.Batch()
+    b.M, b.nseg, b.max_count, b.key_bound = sum(lens), len(lens), max(lens), max(lens)
+    held = [(ctypes.c_int32 * len(x))(*x) for x in (start, range(len(lens)), [0] * len(lens))]
+    b.host_start, b.host_slot, b.host_pos = held
+    return b, held
+
+
+@pytest.mark.parametrize("per_channel", [False, True], ids=["per head", "per channel"])
+@pytest.mark.parametrize("heads,vdim,short,long", [
+    # the longest segment one token below and at the length from which chunks are taken: all else is as large
+    (16, 96, [47, 47] + [40] * 6, [48, 46] + [40] * 6), (16, 40, [47, 47] + [40] * 6, [48, 46] + [40] * 6),
+    (16, 128, [47, 47] + [40] * 6, [48, 46] + [40] * 6), (128, 100, [47, 47], [48, 46]), (32, 16, [47] * 4, [48, 46, 47, 47]),
+    (32, 128, [95, 95], [96, 94]), (32, 96, [95, 95], [96, 94]), (3, 48, [95, 95], [96, 94])])
+def test_a_step_reserves_what_the_delta_rule_takes(heads, vdim, short, long, per_channel):
+    """The workspace grows by the chunks' scratch, as the launch will ask for it, and by no more."""
+    lib = _capi.load_hybrid()
+    h, t = _delta_decoder(lib, heads, vdim, per_channel)
+    need, args = [], _capi.DeltaArgs()
+    args.heads, args.dp, args.vp, args.decay = heads, t.dp, t.vp, 4096 if per_channel else None
+    total = []
+    for lens in (short, long):
+        a = _capi.HybridStepArgs()
+        a.batch, held = _batch_of(lens)
+        a.capacity = 4096
+        need.append(lib.msa_delta_scratch_floats(ctypes.byref(args), ctypes.byref(a.batch)))
+        total.append(lib.msa_hybrid_workspace_bytes(h, ctypes.byref(a)))
+        assert total[-1] > 0, lib.msa_last_error()
+    assert need[0] == 0 and need[1] > 0
+    assert need[1] * 4 <= total[1] - total[0] < need[1] * 4 + 256
+    args.vp = 0        # asked before vp is known: enough for any
+    assert lib.msa_delta_scratch_floats(ctypes.byref(args), ctypes.byref(a.batch)) >= need[1]
+    lib.msa_hybrid_destroy(h)
+
+
 def test_arguments_are_checked_before_anything_is_launched():
     lib = _capi.load_hybrid()
     one = ctypes.c_void_p(4096)
