@@ -10,15 +10,15 @@
 // multiplied up token by token, so a channel that forgets at once is as exact as in the scan.  All of
 // it is fp32, the products on v_mfma_f32_16x16x4_f32.
 //
-// Two kernels.  What does not depend on S0 (T, A, the norms of k and q; for few segments also K', Q' and K^) is
-// computed for all chunks of all heads at once, a wave each, and left in a scratch record; then the
+// Two kernels.  What does not depend on S0 (T, A, the norms of k and q; for few segments with decays per channel also
+// K', Q' and K^) is computed for all chunks of all heads at once, a wave each, and left in a scratch record; then the
 // chunks of a (segment, head, some columns) are walked one after the other.  A scan step's chain of LDS reads, two
 // dots, a sum over lanes and the update takes 500 cycles per token whatever the machine has idle; a
-// chunk's chain takes 2300 per sixteen (28 fp32 products of 32 cycles per wave, a barrier, the LDS reads behind it)
+// chunk's chain takes 2700 per sixteen with one decay per head and 2300 with decays per channel
 // where few segments leave a workgroup a CU of its own.  Where many fill the chip the matrix cores are the bound: 104
 // fp32 products of 32 cycles per wave and chunk, two such waves per SIMD, 6650 cycles of the 11000 a chunk takes.
-// Measured, both kernels against the scan, 32 heads of 128 x 128: one segment of 1500 tokens 141 us against 349
-// (decays per channel 149 against 354), 8 x 1024 tokens 322 against 788 (362 against 1003).
+// Measured, both kernels against the scan, 32 heads of 128 x 128: one segment of 1500 tokens 128 us against 349
+// (decays per channel 123 against 351), 8 x 1024 tokens 322 against 788 (362 against 1003).
 #include <math.h>
 
 #include <type_traits>
@@ -39,10 +39,10 @@ constexpr int DC_WIDE = 128;  // workgroups of several column tiles from which o
 // head has one decay, and that product over the chunk.  Past the segment's end the factors are 0.
 constexpr int DC_T = 0, DC_A = 256, DC_FK = 512, DC_FQ = 528, DC_FU = 544, DC_GC = 560, DC_SK = 576, DC_SQ = 592,
               DC_REC = 608;
-// For the kernel of few segments a record goes on with K', Q' and K^ (16 x DP each) in the order in which the lanes of
-// its MFMAs take them, 1 KB per 16 channels, and, with decays per channel, p_C.
-template <int DP, bool CH, bool READY>
-constexpr int rec_floats = DC_REC + (READY ? 3 * DC_TOK * DP + (CH ? DP : 0) : 0);
+// For few segments with decays per channel a record goes on with K', Q' and K^ (16 x DP each) in the order in which the
+// lanes of the MFMAs take them, 1 KB per 16 channels, and p_C.
+template <int DP, bool READY>
+constexpr int rec_floats = DC_REC + (READY ? 3 * DC_TOK * DP + DP : 0);
 // (DC_GC holds sixteen copies: one address for all lanes would be a scalar load, whose latency every LDS
 // barrier waits for)
 
@@ -107,6 +107,7 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(
     const float* __restrict__ decay_rate, const float* __restrict__ dt_bias,
     const float* __restrict__ decay, int heads, int kv_heads, float q_scale, float* __restrict__ records,
     const int32_t* __restrict__ seg_start, const int32_t* __restrict__ seg_pos) {
+  static_assert(CH || !READY, "records of whole operands are for decays per channel");
   constexpr int CE = (DP + 63) / 64;  // channels per lane
   __shared__ float sums[4][DC_SUMS], tok[4][6][DC_TOK];  // tok: beta, rest of 1 / |k| and of scale / |q|, decay, SK, SQ
   const int s = blockIdx.z, t0 = blockIdx.x * DC_TOK;
@@ -198,11 +199,11 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(
   });
   __syncthreads();
   const float* sm = sums[wave];
-  float* rec = records + record_of(first, s, blockIdx.x, heads, h, rec_floats<DP, CH, READY>);
+  float* rec = records + record_of(first, s, blockIdx.x, heads, h, rec_floats<DP, READY>);
   if constexpr (READY) {
     // K' and Q' go through LDS (rows padded: the lanes that write a token lie 68 floats apart), so that the stores
     // are whole lines; a channel's K^ is 16 bytes of four tokens as it lies.  75 MB for 1500 tokens of 32 heads:
-    // 23 -> 39 us with decays per channel, 22 -> 28 without.
+    // 23 -> 39 us.
     constexpr int TILES = DP / 16, PITCH = 68;
     __shared__ float turn[4][TILES * 4 * PITCH];
     float* tw = turn[wave];
@@ -214,9 +215,9 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(
       for (int t = 0; t < DC_TOK; ++t)
 #pragma unroll
         for (int e = 0; e < CE; ++e) {
-          if (CH) p[e] *= g[CH ? t : 0][e];
+          p[e] *= g[t][e];
           const int c = c0 + e;
-          if (live) tw[(c >> 2) * PITCH + t * 4 + (c & 3)] = CH ? x[t][e] * p[e] : x[t][e];
+          if (live) tw[(c >> 2) * PITCH + t * 4 + (c & 3)] = x[t][e] * p[e];
         }
       __syncthreads();
 #pragma unroll
@@ -235,17 +236,17 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(
         float* to = rec + DC_REC + 2 * DC_TOK * DP + (c >> 4) * 256 + (c & 15) * 4;
         float m = 1.f, late = 1.f, x[DC_TOK];
 #pragma unroll
-        for (int t = DC_TOK / 2; t < DC_TOK; ++t) late *= CH ? g[CH ? t : 0][e] : 1.f;
+        for (int t = DC_TOK / 2; t < DC_TOK; ++t) late *= g[t][e];
 #pragma unroll
         for (int t = DC_TOK - 1; t >= 0; --t) {
           if (t == DC_TOK / 2 - 1) m = late;
-          x[t] = CH ? k[t][e] * m : k[t][e];
-          if (CH) m *= g[CH ? t : 0][e];
+          x[t] = k[t][e] * m;
+          m *= g[t][e];
         }
 #pragma unroll
         for (int t = 0; t < DC_TOK; t += 4)
           *reinterpret_cast<float4_t*>(to + t * 16) = float4_t{x[t], x[t + 1], x[t + 2], x[t + 3]};
-        if (CH) rec[DC_REC + 3 * DC_TOK * DP + c] = p[e];
+        rec[DC_REC + 3 * DC_TOK * DP + c] = p[e];
       }
     }
   }
@@ -488,29 +489,196 @@ __device__ __forceinline__ int right_hand_side(const T (&v)[4], float4_t ks, flo
   return bad;
 }
 
-struct FewLds {
-  float4_t ks[2][4][64], qs[2][4][64], u[2][64];
+template <int DP>
+struct StagedLds {
+  Operands<DP, false> op;
+  float a[4][DC_TOK][DC_TOK + 4];            // A of the chunk being staged, used and finished
+  float4_t ks[4][64], qs[2][4][64], u[2][64];
   int bad[2][16];
 };
 
-// Few segments: a workgroup owns one segment, one head and 16 of its columns for all of the segment's chunks.
+// Few segments, one decay per head: a workgroup owns one segment, one head and 16 of its columns for all of the segment's
+// chunks.
 // Waves 0 .. 3 hold the state, a quarter of its rows each, as MFMA accumulators (a lane: four rows of one
 // column), which are the B operands of the next chunk's products as they lie; they sum K' S0 through
-// LDS, form U redundantly and update their rows.  K', Q' and K^ come from the chunk's record straight into
-// registers, two chunks ahead; the workgroups of a head run on one XCD and share its L2 lines.  Waves 4 .. 7
-// finish the outputs, a chunk each in turn.  One barrier per chunk, behind its K' S0: what the waves hand each
-// other is double buffered.  1500 tokens, 32 heads of 128: 109 us (174 with four waves that staged k, q and
-// decays in LDS for every 16 columns again and multiplied the decays up there, and a second barrier); with one decay
-// per head 114 (130).
-template <typename T, int DP, bool CH>
+// LDS, form U redundantly and update their rows.  Waves 4 .. 7 run beside them, between the two barriers of a chunk:
+// they finish the previous chunk's outputs and stage the next chunk (before the first barrier, beside the short
+// product K' S0, 1500 tokens took 124 us, here 115).
+template <typename T, int DP>
 __global__ __launch_bounds__(512) void delta_chunk_kernel(
     const T* __restrict__ qkv, int64_t ld, int heads, int kv_heads, int vp,
     float* __restrict__ state, const float* __restrict__ records, float* __restrict__ o,
     const int32_t* __restrict__ seg_start, const int32_t* __restrict__ seg_slot,
     const int32_t* __restrict__ seg_pos) {
   constexpr int TILES = DP / 16, TPW = (TILES + 3) / 4;  // 16-row tiles of the state, per wave
-  constexpr int REC = rec_floats<DP, CH, true>;
-  __shared__ FewLds L;
+  extern __shared__ __attribute__((aligned(16))) char dc_lds[];
+  StagedLds<DP>& L = *reinterpret_cast<StagedLds<DP>*>(dc_lds);
+  const int s = blockIdx.z, h = blockIdx.y, col0 = blockIdx.x * 16;
+  const int first = seg_start[s], n = seg_start[s + 1] - first, pos = seg_pos[s];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lm = lane & 15, lg = lane >> 4;
+  float* out = o + (int64_t)first * heads * vp + h * vp + col0;
+  if (pos < 0) {
+    for (int i = tid; i < n * 16; i += 512) out[(int64_t)(i >> 4) * heads * vp + (i & 15)] = 0.f;
+    return;
+  }
+  if (n <= 0) return empty_segment(state + (((int64_t)seg_slot[s] * heads + h) * vp + col0) * DP, 16 * DP, pos);
+  const int nch = (n + DC_TOK - 1) / DC_TOK;
+  const T* rows = qkv + (int64_t)first * ld;
+  const float* rec0 = records + record_of(first, s, 0, heads, h, DC_REC);
+  const int64_t rec_step = (int64_t)heads * DC_REC;
+
+  if (wave < 4) {
+    const int v_at = 2 * kv_heads * DP + h * vp + col0 + lm;
+    float* st = state + (((int64_t)seg_slot[s] * heads + h) * vp + col0 + lm) * DP + lg * 4;
+    float4_t S[TPW];
+#pragma unroll
+    for (int t = 0; t < TPW; ++t) {
+      S[t] = float4_t{0.f, 0.f, 0.f, 0.f};
+      if (pos > 0 && wave * TPW + t < TILES)
+        S[t] = *reinterpret_cast<const float4_t*>(st + (wave * TPW + t) * 16);
+    }
+    struct Ahead {
+      T v[4];
+      Factors f;
+    } ahead[2];
+    auto fetch = [&](Ahead& a, int c) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) a.v[r] = rows[(int64_t)min(c * DC_TOK + lg * 4 + r, n - 1) * ld + v_at];
+      a.f.fetch(rec0, rec_step, c, nch, lm, lg, false);
+    };
+    auto chunk = [&](Ahead& a, int c) {
+      const int b = c & 1;
+      auto times_state = [&](const float* x) {
+        // (tiles past the end: a state of zeros times some row in bounds)
+        float4_t sum[TPW], a[TPW];
+#pragma unroll
+        for (int t = 0; t < TPW; ++t) {
+          sum[t] = float4_t{0.f, 0.f, 0.f, 0.f};
+          a[t] = *reinterpret_cast<const float4_t*>(x + min(wave * TPW + t, TILES - 1) * 16);
+        }
+        mfma4(a, S, sum);
+#pragma unroll
+        for (int t = 1; t < TPW; ++t) sum[0] += sum[t];
+        return sum[0];
+      };
+      L.ks[wave][lane] = times_state(&L.op.k[b][lm][lg * 4]);
+      lds_barrier();  // A
+      float4_t ks = L.ks[0][lane];
+#pragma unroll
+      for (int w = 1; w < 4; ++w) ks += L.ks[w][lane];
+      L.qs[b][wave][lane] = times_state(&L.op.q[b][lm][lg * 4]) * a.f.q;
+      float4_t rhs;
+      const int bad = right_hand_side(a.v, ks, a.f.k, lg, rhs);
+      float4_t u = mfma4(a.f.t, rhs, float4_t{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (lg * 4 + r >= bad) u[r] = 0.f;
+      if (wave == 0) {
+        L.u[b][lane] = u;
+        if (lane < 16) L.bad[b][lane] = bad;
+      }
+      a.f.finish(u, bad, lg, c, nch);
+      const float gc = a.f.gc;
+      fetch(a, c + 2);
+      float4_t kh[TPW], us[TPW], add[TPW];
+#pragma unroll
+      for (int t = 0; t < TPW; ++t) {
+        const int row = min(wave * TPW + t, TILES - 1) * 16;
+        add[t] = float4_t{0.f, 0.f, 0.f, 0.f};
+        kh[t] = L.op.key_column(b, lg, row + lm);
+        us[t] = u;
+        if (wave * TPW + t >= TILES) kh[t] = us[t] = float4_t{0.f, 0.f, 0.f, 0.f};
+      }
+      mfma4(kh, us, add);
+#pragma unroll
+      for (int t = 0; t < TPW; ++t) S[t] = decayed_plus(S[t], float4_t{gc, gc, gc, gc}, add[t]);
+      lds_barrier();  // B
+    };
+    fetch(ahead[0], 0);
+    fetch(ahead[1], 1);
+    lds_barrier();  // chunk 0 is staged
+    for (int c = 0; c < nch; c += 2) {
+      chunk(ahead[0], c);
+      chunk(ahead[1], c + 1);
+    }
+#pragma unroll
+    for (int t = 0; t < TPW; ++t)
+      if (wave * TPW + t < TILES) *reinterpret_cast<float4_t*>(st + (wave * TPW + t) * 16) = S[t];
+    return;
+  }
+
+  typedef Stager<T, DP, false> St;
+  const int ht = tid - 256;
+  const St stager(ht, rows, ld, nullptr, first, heads, kv_heads, h, n, rec0);
+  struct Raw {
+    typename St::Raw r;
+    float a;  // element ht of A
+  } raw[2];
+  auto fetch = [&](Raw& x, int c) {
+    stager.fetch(x.r, c);
+    x.a = rec0[min(c, nch - 1) * rec_step + DC_A + ht];
+  };
+  auto stage = [&](const Raw& x, int c) {
+    L.a[c & 3][ht >> 4][ht & 15] = x.a;
+    stager.stage(L.op, x.r, c);
+  };
+  // outputs of chunk c, by one of the four waves in turn
+  auto finish = [&](int c) {
+    if (c < 0 || (c & 3) != wave - 4) return;
+    const int b = c & 1;
+    float4_t y = L.qs[b][0][lane];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) y += L.qs[b][w][lane];
+    y = mfma4(*reinterpret_cast<const float4_t*>(&L.a[c & 3][lm][lg * 4]), L.u[b][lane], y);
+    const int bad = L.bad[b][lm];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int t = c * DC_TOK + lg * 4 + r;
+      if (t < n) out[(int64_t)t * heads * vp + lm] = lg * 4 + r >= bad ? __builtin_nanf("") : y[r];
+    }
+  };
+  fetch(raw[0], 0);
+  fetch(raw[1], 1);
+  stage(raw[0], 0);
+  fetch(raw[0], 2);
+  lds_barrier();
+  auto beside = [&](Raw& x, int c) {  // x holds chunk c + 1
+    lds_barrier();  // A
+    finish(c - 1);
+    stage(x, c + 1);
+    fetch(x, c + 3);
+    lds_barrier();  // B
+  };
+  for (int c = 0; c < nch; c += 2) {
+    beside(raw[1], c);
+    beside(raw[0], c + 1);
+  }
+  finish((nch + 1) / 2 * 2 - 1);  // (the loop finished all chunks before that one)
+}
+
+struct ReadyLds {
+  float4_t ks[2][4][64], qs[2][4][64], u[2][64];
+  int bad[2][16];
+};
+
+// The same with decays per channel, which would be multiplied up again for every 16 columns: K', Q' and K^ come from the
+// chunk's record straight into the state waves' registers, two chunks ahead; the workgroups of a head run on one
+// XCD and share its L2 lines.  Waves 4 .. 7 finish the outputs, a chunk each in turn.  One barrier per chunk, behind
+// its K' S0: what the waves hand each other is double buffered.  Both kernels, 32 heads of 128, one segment of 128 / 512 /
+// 1500 / 16384 tokens: 25 / 50 / 123 / 1343 us (29 / 67 / 176 / 1820 staged); 16 heads of 128 x 96, 8 x 512 and 32 x 512 of
+// 80: 132 and 490 (189 and 641).  With one decay per head the staged one is the faster: there its staging is a copy, and the
+// operands' 27 KB per record cost more than they save (24 / 51 / 128 / 1285 staged, 26 / 54 / 122 / 1250 so; 117 and 351 against
+// 134 and 455).
+template <typename T, int DP>
+__global__ __launch_bounds__(512) void delta_chunk_ready_kernel(
+    const T* __restrict__ qkv, int64_t ld, int heads, int kv_heads, int vp,
+    float* __restrict__ state, const float* __restrict__ records, float* __restrict__ o,
+    const int32_t* __restrict__ seg_start, const int32_t* __restrict__ seg_slot,
+    const int32_t* __restrict__ seg_pos) {
+  constexpr int TILES = DP / 16, TPW = (TILES + 3) / 4;  // 16-row tiles of the state, per wave
+  constexpr int REC = rec_floats<DP, true>;
+  __shared__ ReadyLds L;
   const int s = blockIdx.z, h = blockIdx.x, col0 = blockIdx.y * 16;
   const int first = seg_start[s], n = seg_start[s + 1] - first, pos = seg_pos[s];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -537,7 +705,7 @@ __global__ __launch_bounds__(512) void delta_chunk_kernel(
         S[t] = *reinterpret_cast<const float4_t*>(st + (wave * TPW + t) * 16);
     }
     struct Ahead {
-      float4_t k[TPW], q[TPW], kh[TPW], g[CH ? TPW : 1];
+      float4_t k[TPW], q[TPW], kh[TPW], g[TPW];
       T v[4];
       Factors f;
     } ahead[2];
@@ -550,12 +718,11 @@ __global__ __launch_bounds__(512) void delta_chunk_kernel(
         a.k[t] = *reinterpret_cast<const float4_t*>(ready + tile * 256 + lane * 4);
         a.q[t] = *reinterpret_cast<const float4_t*>(ready + DC_TOK * DP + tile * 256 + lane * 4);
         a.kh[t] = *reinterpret_cast<const float4_t*>(ready + 2 * DC_TOK * DP + tile * 256 + lane * 4);
-        if constexpr (CH)
-          a.g[CH ? t : 0] = *reinterpret_cast<const float4_t*>(ready + 3 * DC_TOK * DP + tile * 16 + lg * 4);
+        a.g[t] = *reinterpret_cast<const float4_t*>(ready + 3 * DC_TOK * DP + tile * 16 + lg * 4);
       }
 #pragma unroll
       for (int r = 0; r < 4; ++r) a.v[r] = rows[(int64_t)min(c * DC_TOK + lg * 4 + r, n - 1) * ld + v_at];
-      a.f.fetch(rec0, rec_step, c, nch, lm, lg, CH);
+      a.f.fetch(rec0, rec_step, c, nch, lm, lg, true);
     };
     auto times_state = [&](const float4_t (&x)[TPW]) {
       float4_t sum[TPW];
@@ -595,10 +762,8 @@ __global__ __launch_bounds__(512) void delta_chunk_kernel(
         if (wave * TPW + t >= TILES) a.kh[t] = us[t] = float4_t{0.f, 0.f, 0.f, 0.f};
       }
       mfma4(a.kh, us, add);
-      const float gc = a.f.gc;
 #pragma unroll
-      for (int t = 0; t < TPW; ++t)
-        S[t] = decayed_plus(S[t], CH ? a.g[CH ? t : 0] : float4_t{gc, gc, gc, gc}, add[t]);
+      for (int t = 0; t < TPW; ++t) S[t] = decayed_plus(S[t], a.g[t], add[t]);
       fetch(a, c + 2);
       L.ks[b ^ 1][wave][lane] = times_state(next.k);
       lds_barrier();
@@ -772,26 +937,37 @@ template <typename T, int DP, bool CH>
 int run_chunks(const msa_delta_args& a, const msa_batch* b, float* scratch, hipStream_t s) {
   const unsigned chunks = (unsigned)((b->max_count + DC_TOK - 1) / DC_TOK);
   const int wide = wide_tiles(a, b);
-  auto prepare = wide ? delta_prepare_kernel<T, DP, CH, false> : delta_prepare_kernel<T, DP, CH, true>;
+  auto prepare = delta_prepare_kernel<T, DP, CH, false>;
+  if constexpr (CH) {
+    if (!wide) prepare = delta_prepare_kernel<T, DP, CH, true>;
+  }
   hipLaunchKernelGGL(prepare, dim3(chunks, (a.heads + 3) / 4, b->nseg), dim3(256), 0,
                      s, (const T*)a.qkv, a.ld, a.ba, a.ldba, a.decay_rate, a.dt_bias, a.decay, a.heads,
                      a.kv_heads, (float)pow((double)a.dim, -0.5), scratch, b->seg_start, b->seg_pos);
-  if (!wide) {
-    hipLaunchKernelGGL((delta_chunk_kernel<T, DP, CH>), dim3(a.heads, a.vp / 16, b->nseg), dim3(512), 0, s,
+  static std::atomic<uint64_t> raised[3];
+  auto lds = [&](auto kernel, int bytes, std::atomic<uint64_t>& done) {
+    if (raise_lds((const void*)kernel, bytes, done)) return true;
+    msa_set_error("msa_delta_scan_chunks: %d bytes of LDS refused", bytes);
+    return false;
+  };
+  if (wide) {
+    auto kernel = wide == 8 ? delta_chunk_wide_kernel<T, DP, CH, 8> : delta_chunk_wide_kernel<T, DP, CH, 4>;
+    const int bytes = (int)sizeof(Operands<DP, CH>);
+    if (!lds(kernel, bytes, raised[wide == 8])) return MSA_ERR_HIP;
+    hipLaunchKernelGGL(kernel, dim3(a.vp / (wide * 16), a.heads, b->nseg), dim3((wide + 4) * 64), bytes, s,
+                       (const T*)a.qkv, a.ld, a.decay, a.heads, a.kv_heads, a.vp, a.state, scratch, a.o, b->seg_start,
+                       b->seg_slot, b->seg_pos);
+  } else if constexpr (CH) {
+    hipLaunchKernelGGL((delta_chunk_ready_kernel<T, DP>), dim3(a.heads, a.vp / 16, b->nseg), dim3(512), 0, s,
                        (const T*)a.qkv, a.ld, a.heads, a.kv_heads, a.vp, a.state, scratch, a.o, b->seg_start,
                        b->seg_slot, b->seg_pos);
-    return MSA_OK;
+  } else {
+    auto kernel = delta_chunk_kernel<T, DP>;
+    const int bytes = (int)sizeof(StagedLds<DP>);
+    if (!lds(kernel, bytes, raised[2])) return MSA_ERR_HIP;
+    hipLaunchKernelGGL(kernel, dim3(a.vp / 16, a.heads, b->nseg), dim3(512), bytes, s, (const T*)a.qkv, a.ld, a.heads,
+                       a.kv_heads, a.vp, a.state, scratch, a.o, b->seg_start, b->seg_slot, b->seg_pos);
   }
-  auto kernel = wide == 8 ? delta_chunk_wide_kernel<T, DP, CH, 8> : delta_chunk_wide_kernel<T, DP, CH, 4>;
-  static std::atomic<uint64_t> raised[2];
-  const int bytes = (int)sizeof(Operands<DP, CH>);
-  if (!raise_lds((const void*)kernel, bytes, raised[wide == 8])) {
-    msa_set_error("msa_delta_scan_chunks: %d bytes of LDS refused", bytes);
-    return MSA_ERR_HIP;
-  }
-  hipLaunchKernelGGL(kernel, dim3(a.vp / (wide * 16), a.heads, b->nseg), dim3((wide + 4) * 64), bytes, s,
-                     (const T*)a.qkv, a.ld, a.decay, a.heads, a.kv_heads, a.vp, a.state, scratch, a.o, b->seg_start,
-                     b->seg_slot, b->seg_pos);
   return MSA_OK;
 }
 
@@ -813,8 +989,8 @@ int pick_chunks(const msa_delta_args& a, const msa_batch* b, float* scratch, hip
 }  // namespace
 
 // The scan stays faster for few short segments (both kernels cost some 15 us before the first token; one segment of
-// 96 / 112 / 128 tokens: 21.2 / 23.2 / 23.2 us against 24.1 / 27.6 / 31.1, with decays per channel 25.3 /
-// 28.6 / 28.9 against 24.1 / 27.9 / 33.0; of 64 tokens 16.7 by the scan); where the segments fill the chip the chunks
+// 96 / 112 / 128 tokens: 22.2 / 23.9 / 23.8 us against 25.5 / 28.6 / 31.5, with decays per channel 22.5 / 23.7 /
+// 25.0 against 25.1 / 30.1 / 34.2; of 64 tokens 17.9 and 17.2 by the scan); where the segments fill the chip the chunks
 // win from the first length tried (8 x 48 tokens 32 us against 44, seven segments of 20 and one of 64 32 against 36).
 constexpr int DC_FROM = 96, DC_FROM_WIDE = 48;
 
@@ -822,7 +998,7 @@ extern "C" int64_t msa_delta_scratch_floats(const msa_delta_args* a, const msa_b
   if (!a || !b || a->heads <= 0 || a->dp > 128) return 0;
   if (b->max_count < ((int64_t)b->nseg * a->heads >= DC_WIDE ? DC_FROM_WIDE : DC_FROM)) return 0;
   // (a caller that has not set vp gets enough for any)
-  const int ready = a->vp > 0 && wide_tiles(*a, b) ? 0 : 3 * DC_TOK * a->dp + (a->decay ? a->dp : 0);
+  const int ready = !a->decay || (a->vp > 0 && wide_tiles(*a, b)) ? 0 : 3 * DC_TOK * a->dp + a->dp;
   return ((int64_t)b->M / DC_TOK + b->nseg) * a->heads * (DC_REC + ready);
 }
 

@@ -308,6 +308,8 @@ def test_a_step_reserves_what_the_delta_rule_takes(heads, vdim, short, long, per
         assert total[-1] > 0, lib.msa_last_error()
     assert need[0] == 0 and need[1] > 0
     assert need[1] * 4 <= total[1] - total[0] < need[1] * 4 + 256
+    if not per_channel:   # T, A and six factors per token: whatever else a chunk needs is staged from its rows
+        assert need[1] == (sum(long) // 16 + len(long)) * heads * 608
     args.vp = 0        # asked before vp is known: enough for any
     assert lib.msa_delta_scratch_floats(ctypes.byref(args), ctypes.byref(a.batch)) >= need[1]
     lib.msa_hybrid_destroy(h)
