@@ -21,6 +21,7 @@
 // (decays per channel 123 against 351), 8 x 1024 tokens 322 against 788 (362 against 1003).
 #include <math.h>
 
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -31,6 +32,8 @@ namespace {
 
 constexpr int DC_TOK = 16;
 constexpr int DC_WIDE = 128;  // workgroups of several column tiles from which on they take over
+constexpr int DC_READY = 512;  // workgroups of one column tile up to which ready operands are the faster
+constexpr int64_t DC_LONG = 40 << 20;  // floats of long records kept at a time
 // A record: T and A (16 x 16, row-major), then per token the factors that are one number for all channels.
 // The norms are divided out in two steps.  Operands are multiplied by a power of two (SK of k, SQ of q), which is exact
 // and brings them near unit length, so that no product overflows that the scan's unit vectors would not; a vector whose
@@ -53,6 +56,26 @@ __device__ __forceinline__ bool finite(float v) { return fabsf(v) <= 3.402823466
 __device__ __forceinline__ int64_t record_of(int first, int seg, int chunk, int heads, int h, int floats) {
   return ((int64_t)(first / DC_TOK + seg + chunk) * heads + h) * floats;
 }
+// Long records are kept for `count` chunks of every segment at a time, from chunk `from` on (count 0: for all chunks, as
+// above): a launch sees that portion as the segment.  False: nothing of the segment lies in it.
+struct Portion {
+  int from, count;
+  __device__ __forceinline__ bool narrow(int& first, int& n, int& pos) const {
+    if (count == 0) return true;
+    if (from > 0) {
+      if (pos < 0 || n <= from * DC_TOK) return false;
+      first += from * DC_TOK;
+      n -= from * DC_TOK;
+      pos = 1;  // (behind tokens: the state goes on)
+    }
+    if (pos >= 0) n = min(n, count * DC_TOK);
+    return true;
+  }
+  __device__ __forceinline__ int64_t record(int first, int seg, int chunk, int heads, int h, int floats) const {
+    return count == 0 ? record_of(first, seg, chunk, heads, h, floats)
+                      : ((int64_t)(seg * count + chunk) * heads + h) * floats;
+  }
+};
 
 template <int N, int... I, class F>
 __device__ __forceinline__ void each(F&& f, std::integer_sequence<int, I...>) {
@@ -106,13 +129,14 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(
     const T* __restrict__ qkv, int64_t ld, const float* __restrict__ ba, int ldba,
     const float* __restrict__ decay_rate, const float* __restrict__ dt_bias,
     const float* __restrict__ decay, int heads, int kv_heads, float q_scale, float* __restrict__ records,
-    const int32_t* __restrict__ seg_start, const int32_t* __restrict__ seg_pos) {
+    const int32_t* __restrict__ seg_start, const int32_t* __restrict__ seg_pos, Portion portion) {
   static_assert(CH || !READY, "records of whole operands are for decays per channel");
   constexpr int CE = (DP + 63) / 64;  // channels per lane
   __shared__ float sums[4][DC_SUMS], tok[4][6][DC_TOK];  // tok: beta, rest of 1 / |k| and of scale / |q|, decay, SK, SQ
   const int s = blockIdx.z, t0 = blockIdx.x * DC_TOK;
-  const int first = seg_start[s], n = seg_start[s + 1] - first;
-  if (t0 >= n || seg_pos[s] < 0) return;
+  int first = seg_start[s], n = seg_start[s + 1] - first, pos = seg_pos[s];
+  if (READY && !portion.narrow(first, n, pos)) return;
+  if (t0 >= n || pos < 0) return;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int h_own = blockIdx.y * 4 + wave, h = min(h_own, heads - 1);
   const int hk = h / (heads / kv_heads), c0 = lane * CE;
@@ -199,7 +223,9 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(
   });
   __syncthreads();
   const float* sm = sums[wave];
-  float* rec = records + record_of(first, s, blockIdx.x, heads, h, rec_floats<DP, READY>);
+  constexpr int REC = rec_floats<DP, READY>;
+  float* rec = records + (READY ? portion.record(first, s, blockIdx.x, heads, h, REC)
+                                : record_of(first, s, blockIdx.x, heads, h, REC));
   if constexpr (READY) {
     // K' and Q' go through LDS (rows padded: the lanes that write a token lie 68 floats apart), so that the stores
     // are whole lines; a channel's K^ is 16 bytes of four tokens as it lies.  75 MB for 1500 tokens of 32 heads:
@@ -489,30 +515,29 @@ __device__ __forceinline__ int right_hand_side(const T (&v)[4], float4_t ks, flo
   return bad;
 }
 
-template <int DP>
+template <int DP, bool CH>
 struct StagedLds {
-  Operands<DP, false> op;
+  Operands<DP, CH> op;
   float a[4][DC_TOK][DC_TOK + 4];            // A of the chunk being staged, used and finished
   float4_t ks[4][64], qs[2][4][64], u[2][64];
   int bad[2][16];
 };
 
-// Few segments, one decay per head: a workgroup owns one segment, one head and 16 of its columns for all of the segment's
-// chunks.
+// Few segments: a workgroup owns one segment, one head and 16 of its columns for all of the segment's chunks.
 // Waves 0 .. 3 hold the state, a quarter of its rows each, as MFMA accumulators (a lane: four rows of one
 // column), which are the B operands of the next chunk's products as they lie; they sum K' S0 through
 // LDS, form U redundantly and update their rows.  Waves 4 .. 7 run beside them, between the two barriers of a chunk:
 // they finish the previous chunk's outputs and stage the next chunk (before the first barrier, beside the short
 // product K' S0, 1500 tokens took 124 us, here 115).
-template <typename T, int DP>
+template <typename T, int DP, bool CH>
 __global__ __launch_bounds__(512) void delta_chunk_kernel(
-    const T* __restrict__ qkv, int64_t ld, int heads, int kv_heads, int vp,
+    const T* __restrict__ qkv, int64_t ld, const float* __restrict__ decay, int heads, int kv_heads, int vp,
     float* __restrict__ state, const float* __restrict__ records, float* __restrict__ o,
     const int32_t* __restrict__ seg_start, const int32_t* __restrict__ seg_slot,
     const int32_t* __restrict__ seg_pos) {
   constexpr int TILES = DP / 16, TPW = (TILES + 3) / 4;  // 16-row tiles of the state, per wave
   extern __shared__ __attribute__((aligned(16))) char dc_lds[];
-  StagedLds<DP>& L = *reinterpret_cast<StagedLds<DP>*>(dc_lds);
+  StagedLds<DP, CH>& L = *reinterpret_cast<StagedLds<DP, CH>*>(dc_lds);
   const int s = blockIdx.z, h = blockIdx.y, col0 = blockIdx.x * 16;
   const int first = seg_start[s], n = seg_start[s + 1] - first, pos = seg_pos[s];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -545,7 +570,7 @@ __global__ __launch_bounds__(512) void delta_chunk_kernel(
     auto fetch = [&](Ahead& a, int c) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) a.v[r] = rows[(int64_t)min(c * DC_TOK + lg * 4 + r, n - 1) * ld + v_at];
-      a.f.fetch(rec0, rec_step, c, nch, lm, lg, false);
+      a.f.fetch(rec0, rec_step, c, nch, lm, lg, CH);
     };
     auto chunk = [&](Ahead& a, int c) {
       const int b = c & 1;
@@ -581,10 +606,12 @@ __global__ __launch_bounds__(512) void delta_chunk_kernel(
       a.f.finish(u, bad, lg, c, nch);
       const float gc = a.f.gc;
       fetch(a, c + 2);
-      float4_t kh[TPW], us[TPW], add[TPW];
+      float4_t kh[TPW], us[TPW], g[TPW], add[TPW];
 #pragma unroll
       for (int t = 0; t < TPW; ++t) {
         const int row = min(wave * TPW + t, TILES - 1) * 16;
+        if constexpr (CH) g[t] = *reinterpret_cast<const float4_t*>(&L.op.gc[CH ? b : 0][CH ? row + lg * 4 : 0]);
+        else g[t] = float4_t{gc, gc, gc, gc};
         add[t] = float4_t{0.f, 0.f, 0.f, 0.f};
         kh[t] = L.op.key_column(b, lg, row + lm);
         us[t] = u;
@@ -592,7 +619,7 @@ __global__ __launch_bounds__(512) void delta_chunk_kernel(
       }
       mfma4(kh, us, add);
 #pragma unroll
-      for (int t = 0; t < TPW; ++t) S[t] = decayed_plus(S[t], float4_t{gc, gc, gc, gc}, add[t]);
+      for (int t = 0; t < TPW; ++t) S[t] = decayed_plus(S[t], g[t], add[t]);
       lds_barrier();  // B
     };
     fetch(ahead[0], 0);
@@ -608,9 +635,9 @@ __global__ __launch_bounds__(512) void delta_chunk_kernel(
     return;
   }
 
-  typedef Stager<T, DP, false> St;
+  typedef Stager<T, DP, CH> St;
   const int ht = tid - 256;
-  const St stager(ht, rows, ld, nullptr, first, heads, kv_heads, h, n, rec0);
+  const St stager(ht, rows, ld, decay, first, heads, kv_heads, h, n, rec0);
   struct Raw {
     typename St::Raw r;
     float a;  // element ht of A
@@ -623,9 +650,9 @@ __global__ __launch_bounds__(512) void delta_chunk_kernel(
     L.a[c & 3][ht >> 4][ht & 15] = x.a;
     stager.stage(L.op, x.r, c);
   };
-  // outputs of chunk c, by one of the four waves in turn
+  // outputs of chunk c, by one of the four waves in turn (with decays per channel, of the two that stage q)
   auto finish = [&](int c) {
-    if (c < 0 || (c & 3) != wave - 4) return;
+    if (c < 0 || (CH ? (c & 1) != wave - 6 : (c & 3) != wave - 4)) return;
     const int b = c & 1;
     float4_t y = L.qs[b][0][lane];
 #pragma unroll
@@ -662,25 +689,25 @@ struct ReadyLds {
   int bad[2][16];
 };
 
-// The same with decays per channel, which would be multiplied up again for every 16 columns: K', Q' and K^ come from the
+// The same for decays per channel, which would be multiplied up again for every 16 columns: K', Q' and K^ come from the
 // chunk's record straight into the state waves' registers, two chunks ahead; the workgroups of a head run on one
 // XCD and share its L2 lines.  Waves 4 .. 7 finish the outputs, a chunk each in turn.  One barrier per chunk, behind
 // its K' S0: what the waves hand each other is double buffered.  Both kernels, 32 heads of 128, one segment of 128 / 512 /
-// 1500 / 16384 tokens: 25 / 50 / 123 / 1343 us (29 / 67 / 176 / 1820 staged); 16 heads of 128 x 96, 8 x 512 and 32 x 512 of
-// 80: 132 and 490 (189 and 641).  With one decay per head the staged one is the faster: there its staging is a copy, and the
-// operands' 27 KB per record cost more than they save (24 / 51 / 128 / 1285 staged, 26 / 54 / 122 / 1250 so; 117 and 351 against
-// 134 and 455).
+// 1500 / 16384 tokens: 25 / 50 / 123 / 1333 us (staged 29 / 67 / 176 / 1820).  With one decay per head staging is a copy,
+// and the longer records cost more than they save (128 / 512 tokens 23.8 / 51.0 us staged, 25.7 / 53.7 so; 16 heads of 128 x
+// 96, 8 x 512 tokens 117 and 134).
 template <typename T, int DP>
 __global__ __launch_bounds__(512) void delta_chunk_ready_kernel(
     const T* __restrict__ qkv, int64_t ld, int heads, int kv_heads, int vp,
     float* __restrict__ state, const float* __restrict__ records, float* __restrict__ o,
     const int32_t* __restrict__ seg_start, const int32_t* __restrict__ seg_slot,
-    const int32_t* __restrict__ seg_pos) {
+    const int32_t* __restrict__ seg_pos, Portion portion) {
   constexpr int TILES = DP / 16, TPW = (TILES + 3) / 4;  // 16-row tiles of the state, per wave
   constexpr int REC = rec_floats<DP, true>;
   __shared__ ReadyLds L;
   const int s = blockIdx.z, h = blockIdx.x, col0 = blockIdx.y * 16;
-  const int first = seg_start[s], n = seg_start[s + 1] - first, pos = seg_pos[s];
+  int first = seg_start[s], n = seg_start[s + 1] - first, pos = seg_pos[s];
+  if (!portion.narrow(first, n, pos)) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lm = lane & 15, lg = lane >> 4;
   float* out = o + (int64_t)first * heads * vp + h * vp + col0;
@@ -691,7 +718,7 @@ __global__ __launch_bounds__(512) void delta_chunk_ready_kernel(
   if (n <= 0) return empty_segment(state + (((int64_t)seg_slot[s] * heads + h) * vp + col0) * DP, 16 * DP, pos);
   const int nch = (n + DC_TOK - 1) / DC_TOK;
   const T* rows = qkv + (int64_t)first * ld;
-  const float* rec0 = records + record_of(first, s, 0, heads, h, REC);
+  const float* rec0 = records + portion.record(first, s, 0, heads, h, REC);
   const int64_t rec_step = (int64_t)heads * REC;
 
   if (wave < 4) {
@@ -823,12 +850,14 @@ __global__ __launch_bounds__((CT + 4) * 64) void delta_chunk_wide_kernel(
   const int first = seg_start[s], n = seg_start[s + 1] - first, pos = seg_pos[s];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lm = lane & 15, lg = lane >> 4;
+  const int cols = min(CT * 16, vp - col0);  // the last group of a width that is not whole groups has fewer
   if (pos < 0) {
     for (int i = tid; i < n * CT * 16; i += (CT + 4) * 64)
-      o[(int64_t)(first + i / (CT * 16)) * heads * vp + h * vp + col0 + i % (CT * 16)] = 0.f;
+      if (i % (CT * 16) < cols)
+        o[(int64_t)(first + i / (CT * 16)) * heads * vp + h * vp + col0 + i % (CT * 16)] = 0.f;
     return;
   }
-  if (n <= 0) return empty_segment(state + (((int64_t)seg_slot[s] * heads + h) * vp + col0) * DP, CT * 16 * DP, pos);
+  if (n <= 0) return empty_segment(state + (((int64_t)seg_slot[s] * heads + h) * vp + col0) * DP, cols * DP, pos);
   const int nch = (n + DC_TOK - 1) / DC_TOK;
   const T* rows = qkv + (int64_t)first * ld;
   const float* rec0 = records + record_of(first, s, 0, heads, h, DC_REC);
@@ -850,6 +879,14 @@ __global__ __launch_bounds__((CT + 4) * 64) void delta_chunk_wide_kernel(
     for (int c = 0; c < nch; c += 2) {
       beside(raw[1], c);
       beside(raw[0], c + 1);
+    }
+    return;
+  }
+  if (wave * 16 >= cols) {  // no columns: the barriers of the others
+    lds_barrier();
+    for (int c = 0; c < nch; c += 2) {
+      lds_barrier();
+      lds_barrier();
     }
     return;
   }
@@ -926,48 +963,74 @@ __global__ __launch_bounds__((CT + 4) * 64) void delta_chunk_wide_kernel(
   for (int t = 0; t < TILES; ++t) *reinterpret_cast<float4_t*>(st + t * 16) = S[t];
 }
 
-// Waves that own all rows of a head's state, and how many of them to a workgroup; 0: the kernel of few segments.
-int wide_tiles(const msa_delta_args& a, const msa_batch* b) {
+// Which kernel walks the chunks: wide workgroups of 64 or 128 columns, or sixteen columns each (few segments), the operands
+// staged from the rows or ready in the records.  Ready ones spare every column tile the staging, which with decays per
+// channel is most of the work, until their 27 KB per chunk and head are what is waited for: then the wide kernel, whose
+// staging serves four tiles, is the better one for any width, and a single tile stages for itself.  128 keys, decays per
+// channel, us staged / ready / wide of 64, 1000 tokens of one segment: 64 heads of 96 columns (384 workgroups) 236 / 158 /
+// 186, 96 of 80 (480) 245 / 185 / 196, 128 of 48 (384) 254 / 215 / 201, 128 of 80 (640) 358 / 277 / 207; 500 tokens, 256 of
+// 32 (512) 153 / 165 / 125; 8 x 1024 tokens, 16 of 96 (768) 359 / 285 / 208; one tile, 128 heads 150 / 148 / 199, 256 heads
+// 195 / 268 / 239.
+enum Form { STAGED, READY, WIDE_64, WIDE_128 };
+Form form_of(const msa_delta_args& a, const msa_batch* b) {
   const int64_t units = (int64_t)b->nseg * a.heads;
-  if (a.vp % 128 == 0 && units >= DC_WIDE) return 8;
-  return a.vp % 64 == 0 && units * (a.vp / 64) >= DC_WIDE ? 4 : 0;
+  if (a.vp % 128 == 0 && units >= DC_WIDE) return WIDE_128;
+  if (a.vp % 64 == 0 && units * (a.vp / 64) >= DC_WIDE) return WIDE_64;
+  if (!a.decay) return STAGED;
+  if (a.vp == 16) return units <= DC_WIDE ? READY : STAGED;
+  return a.vp % 64 != 0 && units * (a.vp / 16) >= DC_READY ? WIDE_64 : READY;
+}
+
+// Chunks of every segment whose long records are kept at a time, all portions alike; 0: all.  32 heads of 128, one segment
+// of 4096 / 16384 tokens: all at once (226 and 903 MB) 355 / 1368 us, in portions of 64 / 32 / 16 / 8 Mi floats - / 1420, 333 /
+// 1332, 342 / 1447, 405 / 1635: up to some 160 MB the records are still in the memory-side cache when they are read,
+// and a portion costs two launches and the loads in front of its first chunk.
+int portion_chunks(const msa_delta_args& a, const msa_batch* b) {
+  const int64_t layer = (int64_t)a.heads * (DC_REC + (3 * DC_TOK + 1) * a.dp);
+  if (((int64_t)b->M / DC_TOK + b->nseg) * layer <= DC_LONG) return 0;
+  const int chunks = (b->max_count + DC_TOK - 1) / DC_TOK;
+  const int most = (int)std::max<int64_t>(1, DC_LONG / (layer * b->nseg));
+  const int portions = (chunks + most - 1) / most;
+  return (chunks + portions - 1) / portions;
 }
 
 template <typename T, int DP, bool CH>
 int run_chunks(const msa_delta_args& a, const msa_batch* b, float* scratch, hipStream_t s) {
-  const unsigned chunks = (unsigned)((b->max_count + DC_TOK - 1) / DC_TOK);
-  const int wide = wide_tiles(a, b);
-  auto prepare = delta_prepare_kernel<T, DP, CH, false>;
-  if constexpr (CH) {
-    if (!wide) prepare = delta_prepare_kernel<T, DP, CH, true>;
-  }
-  hipLaunchKernelGGL(prepare, dim3(chunks, (a.heads + 3) / 4, b->nseg), dim3(256), 0,
-                     s, (const T*)a.qkv, a.ld, a.ba, a.ldba, a.decay_rate, a.dt_bias, a.decay, a.heads,
-                     a.kv_heads, (float)pow((double)a.dim, -0.5), scratch, b->seg_start, b->seg_pos);
-  static std::atomic<uint64_t> raised[3];
-  auto lds = [&](auto kernel, int bytes, std::atomic<uint64_t>& done) {
-    if (raise_lds((const void*)kernel, bytes, done)) return true;
-    msa_set_error("msa_delta_scan_chunks: %d bytes of LDS refused", bytes);
-    return false;
+  const int chunks = (b->max_count + DC_TOK - 1) / DC_TOK;
+  const Form form = form_of(a, b);
+  auto prepare = [&](auto kernel, int count, Portion p) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)count, (a.heads + 3) / 4, b->nseg), dim3(256), 0, s, (const T*)a.qkv,
+                       a.ld, a.ba, a.ldba, a.decay_rate, a.dt_bias, a.decay, a.heads, a.kv_heads,
+                       (float)pow((double)a.dim, -0.5), scratch, b->seg_start, b->seg_pos, p);
   };
-  if (wide) {
-    auto kernel = wide == 8 ? delta_chunk_wide_kernel<T, DP, CH, 8> : delta_chunk_wide_kernel<T, DP, CH, 4>;
-    const int bytes = (int)sizeof(Operands<DP, CH>);
-    if (!lds(kernel, bytes, raised[wide == 8])) return MSA_ERR_HIP;
-    hipLaunchKernelGGL(kernel, dim3(a.vp / (wide * 16), a.heads, b->nseg), dim3((wide + 4) * 64), bytes, s,
-                       (const T*)a.qkv, a.ld, a.decay, a.heads, a.kv_heads, a.vp, a.state, scratch, a.o, b->seg_start,
-                       b->seg_slot, b->seg_pos);
-  } else if constexpr (CH) {
-    hipLaunchKernelGGL((delta_chunk_ready_kernel<T, DP>), dim3(a.heads, a.vp / 16, b->nseg), dim3(512), 0, s,
-                       (const T*)a.qkv, a.ld, a.heads, a.kv_heads, a.vp, a.state, scratch, a.o, b->seg_start,
-                       b->seg_slot, b->seg_pos);
-  } else {
-    auto kernel = delta_chunk_kernel<T, DP>;
-    const int bytes = (int)sizeof(StagedLds<DP>);
-    if (!lds(kernel, bytes, raised[2])) return MSA_ERR_HIP;
-    hipLaunchKernelGGL(kernel, dim3(a.vp / 16, a.heads, b->nseg), dim3(512), bytes, s, (const T*)a.qkv, a.ld, a.heads,
-                       a.kv_heads, a.vp, a.state, scratch, a.o, b->seg_start, b->seg_slot, b->seg_pos);
+  if constexpr (CH) {
+    if (form == READY) {
+      const int at_once = portion_chunks(a, b), step = at_once > 0 ? at_once : chunks;
+      for (int from = 0; from < chunks; from += step) {
+        const Portion p{from, at_once};
+        prepare(delta_prepare_kernel<T, DP, CH, true>, std::min(step, chunks - from), p);
+        hipLaunchKernelGGL((delta_chunk_ready_kernel<T, DP>), dim3(a.heads, a.vp / 16, b->nseg), dim3(512), 0, s,
+                           (const T*)a.qkv, a.ld, a.heads, a.kv_heads, a.vp, a.state, scratch, a.o, b->seg_start,
+                           b->seg_slot, b->seg_pos, p);
+      }
+      return MSA_OK;
+    }
   }
+  prepare(delta_prepare_kernel<T, DP, CH, false>, chunks, Portion{});
+  auto kernel = form == WIDE_128  ? delta_chunk_wide_kernel<T, DP, CH, 8>
+                : form == WIDE_64 ? delta_chunk_wide_kernel<T, DP, CH, 4>
+                                  : delta_chunk_kernel<T, DP, CH>;
+  const int cols = form == WIDE_128 ? 128 : form == WIDE_64 ? 64 : 16;
+  const int threads = form == WIDE_128 ? 768 : 512;
+  const int bytes = form == STAGED ? (int)sizeof(StagedLds<DP, CH>) : (int)sizeof(Operands<DP, CH>);
+  static std::atomic<uint64_t> raised[WIDE_128 + 1];
+  if (!raise_lds((const void*)kernel, bytes, raised[form])) {
+    msa_set_error("msa_delta_scan_chunks: %d bytes of LDS refused", bytes);
+    return MSA_ERR_HIP;
+  }
+  hipLaunchKernelGGL(kernel, dim3((a.vp + cols - 1) / cols, a.heads, b->nseg), dim3(threads), bytes, s,
+                     (const T*)a.qkv, a.ld, a.decay, a.heads, a.kv_heads, a.vp, a.state, scratch, a.o, b->seg_start,
+                     b->seg_slot, b->seg_pos);
   return MSA_OK;
 }
 
@@ -997,9 +1060,12 @@ constexpr int DC_FROM = 96, DC_FROM_WIDE = 48;
 extern "C" int64_t msa_delta_scratch_floats(const msa_delta_args* a, const msa_batch* b) {
   if (!a || !b || a->heads <= 0 || a->dp > 128) return 0;
   if (b->max_count < ((int64_t)b->nseg * a->heads >= DC_WIDE ? DC_FROM_WIDE : DC_FROM)) return 0;
+  const int64_t all = ((int64_t)b->M / DC_TOK + b->nseg) * a->heads, staged = all * DC_REC;
   // (a caller that has not set vp gets enough for any)
-  const int ready = !a->decay || (a->vp > 0 && wide_tiles(*a, b)) ? 0 : 3 * DC_TOK * a->dp + a->dp;
-  return ((int64_t)b->M / DC_TOK + b->nseg) * a->heads * (DC_REC + ready);
+  if (!a->decay || (a->vp > 0 && form_of(*a, b) != READY)) return staged;
+  const int at_once = portion_chunks(*a, b);
+  const int64_t ready = (at_once > 0 ? (int64_t)at_once * b->nseg * a->heads : all) * (DC_REC + (3 * DC_TOK + 1) * a->dp);
+  return a->vp > 0 ? ready : std::max(ready, staged);
 }
 
 int msa_launch_delta_chunks(const msa_delta_args& a, const msa_batch* b, float* scratch, hipStream_t s) {

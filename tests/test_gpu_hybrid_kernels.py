@@ -937,6 +937,47 @@ def test_delta_chunks_of_huge_and_tiny_keys(M, heads, channels):
             assert off <= 30 * 2.0 ** -24 and end_off <= 30 * 2.0 ** -24, (off, end_off)
 
 
+@pytest.mark.parametrize("heads,kv_heads,dim,dp,vp,counts", [
+    # a last group of one to three column tiles, in batches that fill the chip; one tile of many heads
+    (16, 4, 24, 32, 80, [50, 3, 64, 17, 48, 1, 30, 50]), (64, 1, 64, 64, 144, [49, 48]), (43, 43, 90, 96, 112, [33, 20, 48]),
+    (128, 2, 128, 128, 176, [49]), (64, 2, 120, 128, 16, [50, 48])])
+def test_delta_chunks_of_any_number_of_column_tiles(heads, kv_heads, dim, dp, vp, counts):
+    for channels in (False, True):
+        test_delta_chunks(heads, kv_heads, dim, dp, vp, counts, BF16, channels)
+
+
+@pytest.mark.parametrize("heads,vp,segs", [
+    (31, 16, [(0, 12, 1700), (2, -1, 90), (3, 5, 1400), (1, 0, 10)]), (61, 48, [(1, 0, 1), (0, 3, 1601)])])
+def test_delta_operands_kept_for_a_portion_of_the_chunks(heads, vp, segs):
+    """More chunks than the scratch holds: segments that end before, in and behind a portion, a state carried across
+    their borders."""
+    g, dp, M = gen(9), 128, sum(n for _, _, n in segs)
+    a, b = _capi.DeltaArgs(), _capi.Batch()
+    a.heads, a.dp, a.vp, a.decay, b.M, b.nseg, b.max_count = heads, dp, vp, 4096, M, len(segs), max(n for _, _, n in segs)
+    need = _capi.load_hybrid().msa_delta_scratch_floats(ctypes.byref(a), ctypes.byref(b))
+    assert need <= 40 << 20 and need < (M // 16 + len(segs)) * heads * 6880
+    qkv = torch.randn(M, 2 * heads * dp + heads * vp, generator=g).to(BF16)
+    ba, decays = torch.randn(M, heads, generator=g), torch.rand(M, heads, dp, generator=g) ** 0.125
+    state = torch.randn(4, heads, vp, dp, generator=g)
+    (o, s), (o2, s2) = _scan_and_chunks(qkv, ba, decays, state, heads, dp, vp, True, segs)
+    # both sum in fp32 what 2 dp + 32 products add, of random sign: some 3e-7 each
+    assert float((o - o2).norm() / o.norm()) <= 1e-6 and float((s - s2).norm() / s.norm()) <= 1e-6
+
+
+@pytest.mark.parametrize("channels", [False, True])
+def test_delta_segments_without_tokens_beside_a_last_group_of_columns(channels):
+    g, M, heads, dp, vp = gen(6), 160, 43, 32, 80
+    qkv = torch.randn(M, 2 * heads * dp + heads * vp, generator=g).to(BF16)
+    ba, decays = torch.randn(M, 2 * heads, generator=g), torch.rand(M, heads, dp, generator=g)
+    state = torch.randn(6, heads, vp, dp, generator=g)
+    out = _scan_and_chunks(qkv, ba, decays, state, heads, dp, vp, channels,
+                           [(0, 7, 0), (1, 12, 48), (3, -1, 12), (2, 0, 0), (4, 0, 100)])
+    (o, s), (o2, s2) = out
+    assert torch.equal(s[[0, 2, 3, 5]], s2[[0, 2, 3, 5]]) and not bool(s2[2].any())
+    assert torch.equal(s2[0], state[0]) and not bool(o2[48:60].any())
+    assert float((o - o2).norm() / o.norm()) <= 1e-6 and float((s - s2).norm() / s.norm()) <= 1e-6
+
+
 def test_selection_over_fp32_logits():
     """The fp32 forms of selection, scoring and sampling agree with plain PyTorch, at row strides
     and vocabulary sizes that are no multiple of 8."""

@@ -315,6 +315,24 @@ def test_a_step_reserves_what_the_delta_rule_takes(heads, vdim, short, long, per
     lib.msa_hybrid_destroy(h)
 
 
+@pytest.mark.parametrize("vp", [16, 48, 64, 80, 96, 128, 256])
+@pytest.mark.parametrize("dp", [32, 64, 96, 128])
+def test_scratch_of_the_delta_rule_is_bounded(dp, vp):
+    """Records of 608 floats, or at most 160 MB of records with whole operands: a batch that fills the chip, or one of
+    16384 tokens, keeps no more."""
+    lib = _capi.load_hybrid()
+    a, b = _capi.DeltaArgs(), _capi.Batch()
+    a.dp, a.vp, a.decay = dp, vp, 4096
+    for a.heads in (1, 16, 31, 32, 127, 128, 500):
+        for b.nseg, b.max_count in ((1, 96), (1, 1500), (1, 65535), (3, 16384), (8, 100), (8, 2047), (256, 64), (256, 255)):
+            b.M = min(65535, b.nseg * b.max_count)
+            need = lib.msa_delta_scratch_floats(ctypes.byref(a), ctypes.byref(b))
+            records = (b.M // 16 + b.nseg) * a.heads
+            assert need == records * 608 or 0 < need <= 40 << 20, (a.heads, b.nseg, b.max_count, need)
+            if b.nseg * a.heads >= 128 and vp % 64 == 0:
+                assert need == records * 608
+
+
 def test_arguments_are_checked_before_anything_is_launched():
     lib = _capi.load_hybrid()
     one = ctypes.c_void_p(4096)
