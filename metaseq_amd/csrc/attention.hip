@@ -66,11 +66,12 @@ __global__ void attention_kernel(const half_t* __restrict__ q, const half_t* __r
   // U rows per lane group are requested before the first is used, also in the last (or only)
   // round, where rows past the end re-read the last key and are not scored: a short history
   // (few rounds, or less than one) is one memory latency, not one per row.
-  // A history of at most U rows per lane group takes as many loads as it has rows: a surplus load of the last
-  // row costs the L1 as much as a real one.  Up to four rows the values are requested with the keys, before
-  // anything is waited for; from five on they would only hold up the keys of the other waves.
-  // Per launch, 16 waves, heads of 64: 12 heads over 49 keys 6.5 -> 6.0 us, 192 over 99 keys 7.1 -> 6.3, 256 over
-  // 577 keys 11.8 -> 11.5 (12.7 with the values requested first).
+  // A history of fewer than U rows per lane group takes as many loads as it has rows: a surplus load of the last
+  // row costs the L1 as much as a real one.  Up to three rows the values are requested with the keys, before
+  // anything is waited for; from four on they would only hold up the keys of the other waves.
+  // Per launch, heads of 64: 16 waves, 12 heads over 50 keys 5.5 -> 5.0 us, 192 over 99 keys 7.0 -> 6.2, over 577
+  // keys (five rows) 9.6 -> 9.1, over 900 (eight) 12.0; four waves, 512 over 99 keys (four rows) 5.9 -> 5.7 (6.3 with the
+  // values requested first), 1024 8.1 -> 7.6 (8.4).
   const int last = n_keys - 1;
   const int vkey0 = wave * RPW + rsel;
   half8_t vpre[U];
@@ -84,16 +85,16 @@ __global__ void attention_kernel(const half_t* __restrict__ q, const half_t* __r
     constexpr int R = decltype(rows)::value;
     half8_t kv[R];
     request(kbase, kv, rows);
-    if (R <= 4) request(vbase, vpre, rows);
+    if (R <= 3) request(vbase, vpre, rows);
 #pragma unroll
     for (int u = 0; u < R; ++u)
       if (u + 1 < R || vkey0 + u * kstride < n_keys) score(kv[u], vkey0 + u * kstride);
-    if (R > 4) request(vbase, vpre, rows);
+    if (R > 3) request(vbase, vpre, rows);
   };
   const int rows = (last + kstride) / kstride;  // of the lane group that has most
   int key = vkey0;
   static_assert(U == 8, "the cases below");
-  if (rows <= U) {
+  if (rows < U) {
     switch (rows) {
       case 1: short_history(std::integral_constant<int, 1>{}); break;
       case 2: short_history(std::integral_constant<int, 2>{}); break;
@@ -101,8 +102,7 @@ __global__ void attention_kernel(const half_t* __restrict__ q, const half_t* __r
       case 4: short_history(std::integral_constant<int, 4>{}); break;
       case 5: short_history(std::integral_constant<int, 5>{}); break;
       case 6: short_history(std::integral_constant<int, 6>{}); break;
-      case 7: short_history(std::integral_constant<int, 7>{}); break;
-      default: short_history(std::integral_constant<int, 8>{}); break;
+      default: short_history(std::integral_constant<int, 7>{}); break;
     }
   } else {
     for (; key + (U - 1) * kstride < n_keys; key += U * kstride) {  // whole rounds
@@ -153,9 +153,14 @@ __global__ void attention_kernel(const half_t* __restrict__ q, const half_t* __r
       for (int i = 0; i < 8; ++i) acc[i] = fmaf(p, (float)vv[i], acc[i]);
     }
   };
+  if (rows < U) {  // (apart: the checks cost a long history 1 %, their absence a short one 4 %)
 #pragma unroll
-  for (int u = 0; u < U; ++u)
-    if (u < rows) weigh(vpre[u], vkey0 + u * kstride);  // uniform
+    for (int u = 0; u + 1 < U; ++u)
+      if (u < rows) weigh(vpre[u], vkey0 + u * kstride);  // uniform
+  } else {
+#pragma unroll
+    for (int u = 0; u < U; ++u) weigh(vpre[u], vkey0 + u * kstride);
+  }
   for (key = vkey0 + U * kstride; key + (U - 1) * kstride < n_keys; key += U * kstride) {
     half8_t vv[U];
 #pragma unroll

@@ -981,6 +981,16 @@ def test_attention(lib, B, H, hd, T, S0, masked):
                       what="attention")
 
 
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("rows", [1, 2, 3, 4, 6, 7, 8])
+def test_attention_of_histories_around_whole_rows_per_lane_group(lib, rows, hd):
+    """One key short of, at and past a history of `rows` keys to a lane group, in workgroups of sixteen and of four waves."""
+    for B, H, waves in ((1, 3, 16), (8, 64, 4)):
+        stride = waves * 512 // hd
+        for n in (stride * rows - 1, stride * rows, stride * rows + 1):
+            test_attention(lib, B, H, hd, 1, n - 1, rows == 3)
+
+
 @pytest.mark.parametrize("B,H,hd,S0,mode", [
     (1, 12, 64, 1100, "plain"), (1, 12, 64, 37, "plain"), (2, 5, 128, 700, "mask"),
     (3, 7, 128, 2049, "lens"), (2, 9, 64, 1500, "lens"), (1, 32, 128, 4, "plain"),
