@@ -281,29 +281,36 @@ __global__ __launch_bounds__(128) void latent_combine_kernel(const float* __rest
 // 240 us one by one, 107 together).
 constexpr int FA_BM = 128, FA_BN = 64;
 constexpr int FA_SEGS = 32;
+struct FlashSegment {
+  int first;          // workgroups / 8 before the segment's
+  int row0, T, pos0;  // its rows of q and out; new tokens; tokens before them
+  int kv0;            // its first row of kv
+};
+// (a launch of one segment carries one: 640 bytes of arguments are 0.4 us)
+template <int SEGS>
 struct FlashSegments {
   int n;
-  int first[FA_SEGS];  // workgroups / 8 before the segment's
-  int row0[FA_SEGS], T[FA_SEGS], pos0[FA_SEGS];  // its rows of q and out; new tokens; tokens before them
-  int kv0[FA_SEGS];    // its first row of kv
+  FlashSegment at[SEGS];
 };
 template <int HD>
 constexpr int fa_pitch = HD * 2 + 16;
 template <int HD>
 constexpr int fa_lds_bytes = 2 * 2 * FA_BN * fa_pitch<HD>;
 
-template <int HD>
+template <int HD, int SEGS>
 __global__ __launch_bounds__(256) void flash_attention_kernel(
     const bf16_t* __restrict__ q, int64_t ldq, const bf16_t* __restrict__ kv, int64_t ldkv,
-    bf16_t* __restrict__ out, int64_t ldo, int out_mb, int heads, float scale_log2, FlashSegments segs) {
+    bf16_t* __restrict__ out, int64_t ldo, int out_mb, int heads, float scale_log2, FlashSegments<SEGS> segs) {
   constexpr int KSTEPS = HD / 16, DBLK = HD / 32, PITCH = fa_pitch<HD>, TILE = FA_BN * PITCH;
   constexpr int CH = HD / 8, LD = FA_BN * CH / 256;  // chunks per row; loads per thread and tile
   extern __shared__ __attribute__((aligned(16))) char lds[];  // [2][K, V][TILE]
   const int L = blockIdx.x, xcd = L & 7;
   int seg = 0;
-  while (seg + 1 < segs.n && (L >> 3) >= segs.first[seg + 1]) ++seg;
-  const int row0 = segs.row0[seg], T = segs.T[seg], pos0 = segs.pos0[seg];
-  const int seq = (L >> 3) - segs.first[seg], n_qt = (T + FA_BM - 1) / FA_BM;
+  if constexpr (SEGS > 1)
+    while (seg + 1 < segs.n && (L >> 3) >= segs.at[seg + 1].first) ++seg;
+  const FlashSegment own = segs.at[seg];
+  const int row0 = own.row0, T = own.T, pos0 = own.pos0, kv0 = own.kv0;
+  const int seq = (L >> 3) - own.first, n_qt = (T + FA_BM - 1) / FA_BM;
   // few workgroups: the longest tiles of all heads first (one segment of 1500 tokens 72 us -> 60); many: head by head, one
   // head's rows in L2
   const bool spread = gridDim.x <= 1024;
@@ -317,7 +324,7 @@ __global__ __launch_bounds__(256) void flash_attention_kernel(
   const int tq = q0 + j, tqc = min(tq, T - 1), pq = pos0 + tqc;
   const int n_keys = pos0 + min(T, qt * FA_BM + FA_BM);
   const int ntiles = (n_keys + FA_BN - 1) / FA_BN;
-  const bf16_t* kb = kv + segs.kv0[seg] * ldkv + (int64_t)h * HD;
+  const bf16_t* kb = kv + kv0 * ldkv + (int64_t)h * HD;
   const bf16_t* vb = kb + (int64_t)heads * HD;
 
   bf16x8_t qf[KSTEPS];
@@ -487,12 +494,12 @@ __global__ __launch_bounds__(256) void gather_latents_kernel(const bf16_t* __res
       cache + segs.slot[seg] * slot_stride + (int64_t)(r - segs.first[seg]) * rp + c);
 }
 
-template <int HD>
+template <int HD, int SEGS>
 bool run_flash(const void* q, int64_t ldq, const void* kv, int64_t ldkv, void* out, int64_t ldo,
-               int out_mb, int heads, float scale, const FlashSegments& segs, int groups, hipStream_t s) {
+               int out_mb, int heads, float scale, const FlashSegments<SEGS>& segs, int groups, hipStream_t s) {
   static std::atomic<uint64_t> raised{0};
-  if (!raise_lds((const void*)flash_attention_kernel<HD>, fa_lds_bytes<HD>, raised)) return false;
-  hipLaunchKernelGGL(flash_attention_kernel<HD>, dim3((unsigned)(8 * groups)), dim3(256), fa_lds_bytes<HD>, s,
+  if (!raise_lds((const void*)flash_attention_kernel<HD, SEGS>, fa_lds_bytes<HD>, raised)) return false;
+  hipLaunchKernelGGL((flash_attention_kernel<HD, SEGS>), dim3((unsigned)(8 * groups)), dim3(256), fa_lds_bytes<HD>, s,
                      (const bf16_t*)q, ldq, (const bf16_t*)kv, ldkv, (bf16_t*)out, ldo, out_mb, heads, scale * LOG2E,
                      segs);
   return true;
@@ -618,20 +625,21 @@ extern "C" int msa_flash_attention_segments_bf16(const void* q, int64_t ldq, con
     for (; at > 0 && pos0[order[at - 1]] + counts[order[at - 1]] < pos0[i] + counts[i]; --at) order[at] = order[at - 1];
     order[at] = i;
   }
-  FlashSegments segs{};
+  FlashSegments<FA_SEGS> segs{};
   segs.n = nseg;
   groups = 0;
   for (int i = 0; i < nseg; ++i) {
     const int k = order[i];
-    segs.first[i] = (int)groups;
-    segs.row0[i] = row0[k], segs.T[i] = counts[k], segs.pos0[i] = pos0[k], segs.kv0[i] = kv0[k];
+    segs.at[i] = {(int)groups, row0[k], counts[k], pos0[k], kv0[k]};
     groups += (int64_t)((heads + 7) / 8) * ((counts[k] + FA_BM - 1) / FA_BM);
   }
   bool ok = false;
 #define FA_CASE(HD)                                                                                \
   case HD:                                                                                         \
-    ok = run_flash<HD>(q, ldq, kv, ldkv, out, ldo, out_mb, heads, scale, segs, (int)groups,        \
-                       (hipStream_t)stream);                                                       \
+    ok = nseg > 1 ? run_flash<HD>(q, ldq, kv, ldkv, out, ldo, out_mb, heads, scale, segs, (int)groups,                \
+                                  (hipStream_t)stream)                                                             \
+                  : run_flash<HD>(q, ldq, kv, ldkv, out, ldo, out_mb, heads, scale,                                \
+                                  FlashSegments<1>{1, {segs.at[0]}}, (int)groups, (hipStream_t)stream);            \
     break;
   switch (hd) {
     FA_CASE(32)
