@@ -309,7 +309,7 @@ __global__ __launch_bounds__(SM_THREADS) void log_softmax_kernel(
 // some hundred to a few thousand such ids.  A longer list, or topp = 1, takes the same steps over the
 // whole row.  V = 50272, 6 rows, topp 0.9, us per launch:
 // a clear choice 121 -> 63 (49 in a generation, 129 before), logits of deviation 3 155 -> 89, Zipf 143 -> 85, nearly
-// flat logits (a list of more than SP_LIST) 170 -> 161; topp 1: 129 -> 107; greedy with penalties 58 -> 51.
+// flat logits (a list of more than SP_LIST) 170 -> 161; topp 1: 129 -> 107; greedy with penalties 68 -> 61.
 // The draw is an exponential race: arg-max of p / noise over the nucleus, noise ~ Exp(1) per id,
 // which picks id v with probability p[v] / mass(nucleus).
 constexpr int SP_THREADS = 1024;
@@ -420,15 +420,13 @@ __global__ __launch_bounds__(SP_THREADS) void sample_topp_kernel(
       for (int t = 0; t < stop.n; ++t) ok &= (stop.id[t] != id);
     return ok;
   };
+  auto less_by = [](float z, float cnt, float frequency, float presence) {
+    return z - (cnt * frequency + (cnt > 0.f ? presence : 0.f));
+  };
   auto penalised = [&](int id, float z) {
-    if (pen.counts) {
-      const float cnt = (float)pen.counts[(int64_t)b * V + id];
-      z -= cnt * pen.frequency + (cnt > 0.f ? pen.presence : 0.f);
-    }
-    if (pen.counts_src) {
-      const float cnt = (float)pen.counts_src[(int64_t)b * V + id];
-      z -= cnt * pen.frequency_src + (cnt > 0.f ? pen.presence_src : 0.f);
-    }
+    if (pen.counts) z = less_by(z, (float)pen.counts[(int64_t)b * V + id], pen.frequency, pen.presence);
+    if (pen.counts_src)
+      z = less_by(z, (float)pen.counts_src[(int64_t)b * V + id], pen.frequency_src, pen.presence_src);
     return z;
   };
   // e(id) = z - penalties for an eligible id, -inf otherwise
@@ -452,9 +450,22 @@ __global__ __launch_bounds__(SP_THREADS) void sample_topp_kernel(
       }
     }
     if (pen.counts || pen.counts_src) {
+      float cnt[2][SP_BATCH];
+      auto request = [&](const int64_t* counts, float* to) {
 #pragma unroll
-      for (int j = 0; j < SP_BATCH; ++j)
-        v.e[j] = penalised(min(from + j * SP_THREADS + (int)threadIdx.x, V - 1), v.e[j]);
+        for (int j = 0; j < SP_BATCH; ++j)
+          to[j] = (float)counts[(int64_t)b * V + min(from + j * SP_THREADS + (int)threadIdx.x, V - 1)];
+      };
+      if (pen.counts) request(pen.counts, cnt[0]);
+      if (pen.counts_src) request(pen.counts_src, cnt[1]);
+      if (pen.counts) {
+#pragma unroll
+        for (int j = 0; j < SP_BATCH; ++j) v.e[j] = less_by(v.e[j], cnt[0][j], pen.frequency, pen.presence);
+      }
+      if (pen.counts_src) {
+#pragma unroll
+        for (int j = 0; j < SP_BATCH; ++j) v.e[j] = less_by(v.e[j], cnt[1][j], pen.frequency_src, pen.presence_src);
+      }
     }
     const int k = from / SP_THREADS;
     if (k + SP_BATCH > 63 || ((masked_rounds >> k) & ((1u << SP_BATCH) - 1))) {
@@ -496,9 +507,13 @@ __global__ __launch_bounds__(SP_THREADS) void sample_topp_kernel(
   if (!dead) {
     for (int from = 0; from < V; from += SP_BATCH * SP_THREADS) {
       Batch v;
-      if (!need_all && min(from + SP_BATCH * SP_THREADS, V) <= cap) {
+      if (min(from + SP_BATCH * SP_THREADS, V) <= cap) {  // (the masks and penalties are in what the cache holds)
 #pragma unroll
-        for (int j = 0; j < SP_BATCH; ++j) v.e[j] = e_cache[min(from + j * SP_THREADS + tid, V - 1)];
+        for (int j = 0; j < SP_BATCH; ++j) {
+          const int id = min(from + j * SP_THREADS + tid, V - 1);
+          if (need_all) v.raw[j] = (float)row[id];
+          v.e[j] = e_cache[id];
+        }
       } else {
         load(v, from);
       }

@@ -1377,6 +1377,25 @@ def test_sampling_kernel_per_row_temperature_and_skipped_rows(lib):
             assert int(tok[r]) == int(lp.argmax()) and abs(float(sc[r]) - float(lp.max())) < 2e-5
 
 
+@pytest.mark.parametrize("V", [5119, 35840, 35841, 50272])
+def test_greedy_choice_and_its_distribution_with_penalties(lib, V):
+    """Without noise: values kept from the first pass (up to 35840 of them) and values formed again give one distribution."""
+    B, g = 3, torch.Generator().manual_seed(V)
+    logits = (torch.randn(B, V, generator=g) * 2.0).half()
+    counts, counts_src = (torch.randint(0, 3, (B, V), generator=g) for _ in range(2))
+    alphas = (0.7, 0.2, 0.4, 0.1)
+    for temperature in (1.0, 0.8):
+        lp = _reference_lprobs(logits, temperature, [1], None, [False] * B, 2, counts, counts_src, alphas)
+        stored = torch.empty(B, V, device=DEV)
+        tok, sc = _sample(lib, G(logits), temperature=temperature, counts=G(counts.clone()), counts_src=G(counts_src),
+                          alphas=alphas, lprobs=stored)
+        best = lp.max(-1).values
+        assert torch.allclose(sc, best, atol=2e-5) and torch.allclose(lp.gather(1, tok.view(-1, 1)).view(-1), best, atol=2e-5)
+        fine = torch.isfinite(lp)
+        assert torch.equal(torch.isfinite(stored.cpu()), fine)
+        assert torch.allclose(stored.cpu()[fine], lp[fine], atol=1e-5, rtol=1e-6)
+
+
 def test_log_softmax_rows_into_a_strided_buffer(lib):
     """msa_log_softmax_f16 against torch's fp32 log_softmax: rows (b, t), t < T - 1, of logits
     [B, T, V] land at out[b, t + 1], as the generator stores the prompt's distributions."""
