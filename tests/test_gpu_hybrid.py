@@ -143,6 +143,23 @@ def test_delta_heads_of_any_width_in_batches_that_fill_the_chip(kind, heads, vdi
         case.check(torch.cat([a, b]), case.want(toks[i]), "%s, request %d" % (kind, i))
 
 
+def test_requests_that_hold_more_than_is_expanded_at_a_time():
+    """Continuations of five long contexts (16384 positions are expanded at a time), one of them too short to expand,
+    against each alone."""
+    case = H.Case(H.config([(H.latent(heads=2, dim=16, vdim=16, kv_rank=32, q_rank=16), None)] * 2), seed=21, dtype=BF16)
+    d, held, more = case.decoder, (4030, 3900, 4100, 4077, 3333), (40, 17, 33, 5, 129)
+    toks = [case.tokens(a + b, seed=90 + i) for i, (a, b) in enumerate(zip(held, more))]
+    got = []
+    for together in (False, True):
+        cache = d.new_slot_cache(5, 4240)
+        for i, n in enumerate(held):
+            d.extend(cache, [(i, toks[i][:n].cuda())])
+        entries = [(i, toks[i][n:].cuda()) for i, n in enumerate(held)]
+        got.append(d.extend(cache, entries, want_all=True) if together else
+                   torch.cat([d.extend(cache, [e], want_all=True) for e in entries]))
+    case.check(got[1], got[0], "together")
+
+
 def test_more_long_requests_than_one_launch_of_attention_takes():
     test_batch_of_unequal_requests_equals_each_alone(tuple(17 + i % 5 for i in range(34)), BF16)
 

@@ -93,6 +93,15 @@ def test_linear_bf16(M, N, K):
         close(part.sum(0), ref, 1e-5, "partial sums, S=%d" % S)
 
 
+@pytest.mark.parametrize("M,N,K", [
+    # a wave per tile: vocabularies (13 and 14 tiles per workgroup) from one row on, one to three tiles of 33 to 64 rows,
+    # four of more; the last workgroup's tiles run out
+    (1, 50272, 160), (17, 54000, 96), (33, 54000, 160), (64, 50272, 96), (65, 54000, 96), (128, 50272, 160),
+    (40, 3088, 160), (50, 8176, 96), (64, 12272, 224), (33, 12288, 96), (100, 16368, 160)])
+def test_linear_bf16_of_a_wave_per_tile(M, N, K):
+    test_linear_bf16(M, N, K)
+
+
 @pytest.mark.parametrize("M,N", [(4352, 16656), (600, 24576)])
 def test_linear_partial_bf16_wide_panels(M, N):
     """More than 64 columns of tiles, taken in panels of 16; sums of one and two slices."""
@@ -566,6 +575,39 @@ def test_flash_attention_of_several_segments(hd, heads, segs, packed):
     one = ints([1] * 33)
     assert lib.msa_flash_attention_segments_bf16(ptr(q), D, ptr(kv), 2 * D, ptr(out), D, mb, heads, hd, 33, one, one,
                                                  one, scale, _capi.stream_ptr()) == -1
+
+
+def test_flash_attention_of_more_than_1024_workgroups():
+    """Head by head, where few workgroups take the longest query tiles of all heads first."""
+    test_flash_attention_of_several_segments(64, 9, [(257 + 4 * i, 37 * i % 300) for i in range(32)], False)
+
+
+@pytest.mark.parametrize("kv_heads,chunk", [(8, 0), (2, 0), (8, 100)])
+def test_grouped_prompts_of_more_than_1024_workgroups(kv_heads, chunk):
+    """Head by head, where few workgroups take the longest query tiles of all heads first: every segment holds the bits
+    that it gets alone."""
+    lib = _capi.load_hybrid()
+    heads, hd, rows, g = 16, 64, 400, gen(kv_heads)
+    segs = [(i, -1 if i == 7 else 3 * i % 50, 130 + 5 * i) for i in range(33)]
+    M, D = sum(n for _, _, n in segs), (heads + 2 * kv_heads) * hd
+    b, alive = _batch(segs, M)
+    x = torch.randn(M, D, generator=g).to(BF16).cuda()
+    kc, vc = (torch.randn(33, kv_heads, rows, hd, generator=g).to(BF16).cuda() for _ in range(2))
+    out, want = (torch.full((M, heads * hd), 7.0, dtype=BF16, device="cuda") for _ in range(2))
+    a = _capi.GroupedArgs()
+    a.dtype, a.heads, a.kv_heads, a.hd, a.vd, a.chunk, a.rows, a.scale, a.splits = 0, heads, kv_heads, hd, hd, chunk, rows, 0.2, 1
+    a.q, a.k, a.v, a.ld = ptr(x), ptr(x[:, heads * hd:]), ptr(x[:, (heads + kv_heads) * hd:]), D
+    a.k_cache, a.v_cache, a.out, a.ldo = ptr(kc), ptr(vc), ptr(out), heads * hd
+    to = ctypes.byref(a), ctypes.byref(b)
+    assert heads * 3 * len(segs) > 1024
+    check(lib.msa_grouped_attention(*to, 0, len(segs), max(n for _, _, n in segs), _capi.stream_ptr()), lib)
+    a.out = ptr(want)
+    for i, (_, _, n) in enumerate(segs):
+        check(lib.msa_grouped_attention(*to, i, i + 1, n, _capi.stream_ptr()), lib)
+    torch.cuda.synchronize()
+    at = sum(n for _, _, n in segs[:7])
+    assert torch.equal(out, want) and bool((out[:at] != 7.0).any(1).all()) and bool((out[at:at + segs[7][2]] == 7.0).all())
+    del alive
 
 
 def test_gathered_latents():
