@@ -845,12 +845,18 @@ class TransformerDecoder(IncrementalDecoder):
                 torch.cat(positions))
 
     def _rows_buffers(self, M, dev):
-        """Work buffers of ``_rows_layer`` for M row-major activation rows.  ``normed``: the tail of the
-        layer before has already written the LayerNorm that comes next."""
+        """Work buffers of ``_rows_layer`` for M row-major activation rows; ``hp``, ``op``, ``up``: of at most 128,
+        in the packed layout.  ``normed``: the tail of the layer before has already written the LayerNorm that
+        comes next."""
         D, F = self.cfg.decoder_embed_dim, self.cfg.decoder_ffn_embed_dim
         f16 = dict(dtype=torch.float16, device=dev)
-        return {"q": torch.empty(M, D, **f16), "h": torch.empty(M, D, **f16),
-                "o": torch.empty(M, D, **f16), "u": torch.empty(M, F, **f16), "normed": False}
+        work = {"q": torch.empty(M, D, **f16), "h": torch.empty(M, D, **f16), "normed": False}
+        if M > self.PACKED_MAX_ROWS:
+            work.update(o=torch.empty(M, D, **f16), u=torch.empty(M, F, **f16))
+        else:
+            MP = self._packed_rows(M)
+            work.update(hp=torch.empty(MP * D, **f16), op=torch.empty(MP * D, **f16), up=torch.empty(MP * F, **f16))
+        return work
 
     def _rows_attention(self, lib, stream, q, kc, vc, mask, o, B, H, hd, T, S0, cap, len_dev, prompts):
         if prompts is not None:
@@ -906,11 +912,7 @@ class TransformerDecoder(IncrementalDecoder):
         M = B * T
         IN, OUT = MSA_IN_PACKED, MSA_OUT_PACKED
         q = work["q"]
-        if "hp" not in work:
-            MP = self._packed_rows(M)
-            work["hp"] = torch.empty(MP * D, dtype=torch.float16, device=x.device)
-            work["op"] = torch.empty(MP * D, dtype=torch.float16, device=x.device)
-            work["up"] = torch.empty(MP * F, dtype=torch.float16, device=x.device)
+        if "S_o" not in work:
             int8 = layer.fc2.qweight is not None
             splits = lib.msa_linear_default_splits_w8a16 if int8 else lib.msa_linear_default_splits
             work["S_o"], work["S_f"] = splits(M, D, D), splits(M, D, F)

@@ -584,3 +584,17 @@ def test_generation_that_ends_early_leaves_nothing_behind(kw):
     assert float(got["scores"][:, 0, ended:].abs().max()) == 0.0
     if kw.get("need_logprobs"):
         assert float(got["distributions"][:, 0, ended:].abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("n", [4, 70, 200])
+def test_a_decoder_without_layers_projects_its_embedding(n):
+    """Short prompts (packed features up to 64 rows), and longer ones: no layer has made their work buffers."""
+    cfg = OPTConfig(0, 256, 4, vocab_size=512, max_target_positions=256)
+    model, sd = build(cfg)
+    d = model.decoder
+    toks = torch.randint(4, 512, (n,), generator=torch.Generator().manual_seed(n))
+    got = d.prefill_slot(d.new_slot_cache(1, 256), 0, toks.to(DEV))
+    w = {k: v.float().to(DEV) for k, v in sd.items()}
+    x = w["decoder.embed_tokens.weight"][toks.to(DEV)] + w["decoder.embed_positions.weight"][torch.arange(n, device=DEV) + 2]
+    x = torch.nn.functional.layer_norm(x.half().float(), (256,), w["decoder.layer_norm.weight"], w["decoder.layer_norm.bias"])
+    check_logits(got, x.half().float() @ w["decoder.embed_tokens.weight"].t(), "no layers, %d tokens" % n)
