@@ -1892,7 +1892,11 @@ constexpr int SH_GROUP_W8 = 18;  // int8 only: 6 lanes x 3
 // sums between waves, the fewest registers and so the most loads in flight.  Measured, 50272 x 4096, us: 8 rows 69
 // -> 64, 32 rows 75 -> 65 (6.3 TB/s; both on the stream kernel before), 40 rows 75 -> 66, 64 rows 95 -> 66, 100 rows
 // 116 -> 93; K = 2048, 64 rows 48 -> 36; K = 9216, 64 rows 199 -> 138.  A third weight stage in flight costs as much as
-// it gives (69 at 64 rows), eight K steps to a stage spill (89).
+// it gives (69 at 64 rows), eight K steps to a stage spill (89).  These are the numbers of tiles that gain at every number
+// of rows.  A wave per tile for others, as they run now and so (K = 4096): 9 tiles, 1 row 44 and 46, 64 rows 53 and 50,
+// 100 rows 67 and 71; 12 tiles 60 and 66, 70 and 69, 71 and 78; 15 tiles 73 and 76, 106 and 80, 129 and 99; 16 tiles 78
+// and 90, 108 and 91, 127 and 102: less work in flight per CU below 13, and from 15 on four or more waves to a SIMD whose
+// registers hold fewer loads each.
 constexpr bool vocabulary_tiles(int tiles_per_wg) { return tiles_per_wg == 13 || tiles_per_wg == 14; }
 
 // The shared-activation kernel sweeps K once per pass of SH_GROUP tiles: it is used when the
@@ -1950,7 +1954,8 @@ void launch_share(const void* xp, const void* W, const void* scales, float* part
 #define SH_RUN(...)                                                                                           \
   return launch_share_cfg<MB, W8, MODE, __VA_ARGS__>(xp, W, scales, part, S, M, N, K, tiles_per_wg, gx, \
                                                      ks_per_split, epi, s)
-    if (vocabulary_tiles(tiles_per_wg)) SH_RUN(1, 14, 1, 4);
+    // (few rows and selections come here for vocabularies only; any number of tiles is right, in as many passes)
+    if (MB <= 2 || MODE == MODE_SELECT || vocabulary_tiles(tiles_per_wg)) SH_RUN(1, 14, 1, 4);
     if constexpr (MB > 2 && MODE != MODE_SELECT) {
       if (tiles_per_wg == 1) SH_RUN(8, 1, 1, 2);
       if (tiles_per_wg == 2) SH_RUN(4, 2, 1, 4);
@@ -1958,16 +1963,19 @@ void launch_share(const void* xp, const void* W, const void* scales, float* part
     }
 #undef SH_RUN
   }
-  if constexpr (MB <= 2 || MODE == MODE_SELECT) return;  // (not reached)
-  else if (tiles_per_wg <= 4)
-    launch_share_cfg<MB, W8, MODE, 2, 4, 1, 8>(xp, W, scales, part, S, M, N, K, tiles_per_wg, gx,
-                                               ks_per_split, epi, s);
-  else if (tiles_per_wg <= 8)
-    launch_share_cfg<MB, W8, MODE, 2, 4, 2, 4>(xp, W, scales, part, S, M, N, K, tiles_per_wg, gx,
-                                               ks_per_split, epi, s);
-  else
-    launch_share_cfg<MB, W8, MODE, 2, 4, 3, 4>(xp, W, scales, part, S, M, N, K, tiles_per_wg, gx,
-                                               ks_per_split, epi, s);
+  if constexpr (MB > 2 && MODE != MODE_SELECT) {
+    if (tiles_per_wg <= 4)
+      launch_share_cfg<MB, W8, MODE, 2, 4, 1, 8>(xp, W, scales, part, S, M, N, K, tiles_per_wg, gx,
+                                                 ks_per_split, epi, s);
+    else if (tiles_per_wg <= 8)
+      launch_share_cfg<MB, W8, MODE, 2, 4, 2, 4>(xp, W, scales, part, S, M, N, K, tiles_per_wg, gx,
+                                                 ks_per_split, epi, s);
+    else
+      launch_share_cfg<MB, W8, MODE, 2, 4, 3, 4>(xp, W, scales, part, S, M, N, K, tiles_per_wg, gx,
+                                                 ks_per_split, epi, s);
+  } else {
+    static_assert(!W8, "int8 weights of so few rows stream");
+  }
 }
 
 // 65 .. 128 packed rows (eight row blocks): the shared-activation kernel as 2 K lanes x 4 tile
@@ -1976,7 +1984,8 @@ void launch_share(const void* xp, const void* W, const void* scales, float* part
 // workgroup are few per wave, so more weight stages are kept in flight instead (PF).  Measured
 // at 128 x 12288 x 4096 (38.6 us as built): four K lanes x two tile lanes x two tiles 45.8 us,
 // stages of eight K steps 43.0, six weight stages in flight instead of four 44.3.  16-bit weights: a vocabulary a
-// wave per tile (50272 x 4096 at 128 rows 116 -> 95); four tiles in stages of four K steps (16384 x 4096 38.3 -> 36.3).
+// wave per tile (50272 x 4096 at 128 rows 116 -> 95); four tiles in stages of eight K steps, two weight stages in
+// flight and all 160 KB (16384 x 4096 38.3 -> 36.3).
 template <bool W8, int MODE>
 void launch_wide(const void* xp, const void* W, const void* scales, float* part, int S, int M,
                  int N, int K, const Epilogue& epi, hipStream_t s) {
@@ -2189,8 +2198,8 @@ void launch_few_rows(const void* x, const void* W, int64_t M, int N, int K, cons
                      M, N, K, o.a, o.r, epi, (float*)nullptr, 0, GroupTiles{});
 }
 
-// Split-K launch of a narrow four-wave form (WF = 2: 256 x 64 tiles, WF = 4: 256 x 128) on
-// row-major activations: S slices of K, each a whole number of 64-wide stages (at least two),
+// Split-K launch of a four-wave form (WF = 2: 256 x 64 tiles, WF = 4: 256 x 128, WF = 8: 256 x 256, of at least
+// 256 rows) on row-major activations: S slices of K, each a whole number of 64-wide stages (at least two),
 // fp32 sums into part[S][M][N].
 template <int MODE, int WF>
 void launch_quad_partial_w(const void* x, const void* W, float* part, int64_t M, int N, int K,
@@ -2206,8 +2215,9 @@ void launch_quad_partial_w(const void* x, const void* W, float* part, int64_t M,
                      (const half_t*)x, W, M, N, K, o.a, o.r, e, part, K / 64 / S, GroupTiles{});
 }
 
-// fp16: 256 x 64 tiles while their S slices fit the chip in one round; an S beyond that means 256 x 128
-// tiles, and one for which those do not fit either 256 x 256 (pick_row_splits).  bf16 (prefill-sized products whose sums leave as fp32): the cheapest of all widths.
+// fp16: 256 x 64 tiles while their S slices fit the chip in one round; an S beyond that means 256 x 128 tiles
+// (pick_row_splits), and one for which those do not fit either 256 x 256 (pick_row_splits_f16).  bf16
+// (prefill-sized products whose sums leave as fp32): the cheapest of all widths.
 template <int MODE>
 void launch_quad_partial(const void* x, const void* W, float* part, int64_t M, int N, int K, int S,
                          hipStream_t s) {
@@ -2248,9 +2258,13 @@ int pick_row_splits(int64_t M, int N, int K) {
 
 // The same for fp16 prompts whose tail adds the slices: two of a long sum (K of 8192 or more) whose 256 x 256 tiles
 // fill half of the chip or less.  One slice takes 256 x 128 tiles there, at 0.61 of the wide tiles' time for half of
-// their work.  Product, tail and LayerNorm, cold weights, one slice and two: 4096 x 16384 over 1025 rows 233 and 190 us,
-// 1607 218 and 196, 2048 243 and 224; 2048 x 8192 over 2100 rows 109 and 99, 3000 112 and 108, 3584 121 and 120, 4096 132
-// and 136: the shorter sum up to three quarters of the chip.
+// their work.  Product, tail and LayerNorm, cold weights, one slice and two, us: 4096 x 16384 over 1180 rows 205 and 166,
+// 1692 225 and 200, 2048 250 and 224; 5120 x 20480 over 1024 257 and 215, 1536 289 and 263; 7168 x 28672 over 768 380 and
+// 305, 1024 396 and 344; 9216 x 36864 over 512 481 and 370, 768 503 and 433; 9216 x 9216 over 512 128 and 108; 2560 x
+// 10240 over 1692 135 and 113, 2304 141 and 123.  A sum shorter than 16384 stops at three quarters of that half: 2048
+// x 8192 over 3072 rows (96 tiles) 120 and 109, 3328 122 and 116, 3584 125 and 122, 3840 128 and 129, 4096 135 and 133.
+// (The line is drawn for K = 8192; between it and 16384 two slices stay ahead past it: 9216 x 9216 over 768 rows, 108
+// tiles, 137 and 126, 2560 x 10240 over 3072, 120 tiles, 156 and 148.)
 int pick_row_splits_f16(int64_t M, int N, int K) {
   const int few = pick_row_splits(M, N, K);
   if (few > 1 || M < TQ_BM || N % 16 || K % 128 || K < 8192) return few;
