@@ -394,8 +394,10 @@ __global__ __launch_bounds__(256) void grouped_flash_kernel(msa_grouped_args a,
   const int seg = seg0 + blockIdx.y, first = seg_start[seg], T = seg_start[seg + 1] - first;
   const int pos0 = seg_pos[seg];
   const int L = blockIdx.x, xcd = L & 7, seq = L >> 3;
-  // Few workgroups: the longest query tiles of all heads first, so that none of them begins late or shares its compute
-  // unit with another (1500 tokens, 32 heads of 128: 72 us head by head, 60).  Many: head by head, one head's rows in L2.
+  // Up to 1024 workgroups: the longest query tiles of all heads first, so that none of them begins late or shares its
+  // compute unit with another (32 heads of 128, 1500 tokens 60 us head by head, 50; 4096 225 and 186).  Beyond: head by
+  // head, one head's rows in L2 (there the first order is ahead by less, 6000 tokens 385 and 364, 8192 676 and 647, but 8 x
+  // 1024 150 and 127; as the only order it is scheduled 3 % slower for the few, 1500 tokens 51, 2048 70 against 68).
   const bool spread = gridDim.x * gridDim.y <= 1024;
   const int hg = (a.heads + 7) / 8, hi = spread ? seq % hg : seq / n_qt;
   const int qt = n_qt - 1 - (spread ? seq / hg : seq % n_qt);

@@ -329,9 +329,11 @@ constexpr auto tail_two = tail_kernel<T, NV, NT, true>;
 
 // The tail of many rows takes twice the threads: half of a row's operands per thread, all in flight (and four routed
 // terms at a time), so that more rows share a compute unit.  6038 x 4096, us: one fp32 slice 90 -> 70, eight routed
-// terms 172 -> 118; 1500 x 4096 in two slices 28 -> 23, two sublayers of two slices 38 -> 27.  1024 threads are slower (93
-// on average against 81); rows of 2048 (two operands per thread of 256) and the embedding have nothing to gain (40.7
-// against 43.0; 59 and 61).
+// terms 172 -> 118; 1500 x 4096 in two slices 28 -> 23, two sublayers of two slices 38 -> 27.  Rows of 4097 to 8192 take
+// 1024 threads in place of 512 for the same reason, operands still in the caches: 6038 x 5120 one slice 102 -> 68, eight
+// terms 257 -> 179, two sublayers 193 -> 164; 8192 161 -> 124, 333 -> 286, 301 -> 257; 1025 x 8192 25 -> 20, 51 -> 37,
+// 52 -> 44.  Rows up to 4096 are slower with 1024 (93 on average against 81); rows of 2048 (two operands per thread of
+// 256) and the embedding have nothing to gain (40.7 against 43.0; 59 and 61).
 #define RN_DISPATCH_TAIL(KERNEL, T, M, Dp, ...)                                             \
   do {                                                                                      \
     const int q_ = (Dp) / 4;                                                                \
