@@ -723,12 +723,32 @@ __global__ __launch_bounds__(KL * NG * 64) void linear_share_kernel(
     }
   };
 
-  float4_t acc[NT][MB];
+  // A wave that owns all of its tiles' K sums every stage by itself and then the stages, where the sums leave in 32 bits:
+  // one chain over all of K had two to three times the error of sums over eight waves (bf16 of K = 768 / 2048 / 4096 /
+  // 9216: 1.6 / 2.7 / 3.9 / 6.1e-7, eight waves 0.8 / 1.0 / 1.4 / 2.0e-7, so 0.8 / 1.0 / 1.2 / 1.7e-7, at no cost in time).
+  // Results of 16 bits are the same to five digits either way.  More row blocks leave no registers for it (launch_wide).
+  constexpr bool LEVELS = KL == 1 && MB <= 4 && MODE != MODE_SELECT;
+  float4_t acc[NT][MB], done[LEVELS ? NT : 1][LEVELS ? MB : 1];
   auto clear = [&]() {
 #pragma unroll
     for (int j = 0; j < NT; ++j)
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb) acc[j][mb] = float4_t{0.f, 0.f, 0.f, 0.f};
+      for (int mb = 0; mb < MB; ++mb) {
+        acc[j][mb] = float4_t{0.f, 0.f, 0.f, 0.f};
+        if (LEVELS) done[LEVELS ? j : 0][LEVELS ? mb : 0] = acc[j][mb];
+      }
+  };
+  auto settle = [&]() {
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) {
+        done[LEVELS ? j : 0][LEVELS ? mb : 0] += acc[j][mb];
+        acc[j][mb] = float4_t{0.f, 0.f, 0.f, 0.f};
+      }
+  };
+  auto sum_of = [&](int j, int mb) {
+    return LEVELS ? done[LEVELS ? j : 0][LEVELS ? mb : 0] + acc[j][mb] : acc[j][mb];
   };
   auto compute = [&](const Wst& w, int idx) {
     const half_t* l = lx_share + (idx & 1) * XH + kl * U * MB * 512 + lane * 8;
@@ -784,7 +804,7 @@ __global__ __launch_bounds__(KL * NG * 64) void linear_share_kernel(
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
           if (mb * 16 + (lane & 15) < M)
-            select_update4(sel[mb], epi, mb * 16 + (lane & 15), t * 16 + ((lane >> 4) << 2), acc[0][mb]);
+            select_update4(sel[mb], epi, mb * 16 + (lane & 15), t * 16 + ((lane >> 4) << 2), sum_of(0, mb));
       }
       clear();
       return;
@@ -806,7 +826,7 @@ __global__ __launch_bounds__(KL * NG * 64) void linear_share_kernel(
       if (kl == 0 && t < tile_end) {
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) {
-          float4_t sum = acc[j][mb];
+          float4_t sum = sum_of(j, mb);
 #pragma unroll
           for (int k = 1; k < KL; ++k) sum += red[(((k - 1) * NG + ng) * MB + mb) * 64 + lane];
           const int m = mb * 16 + (lane & 15);
@@ -846,6 +866,7 @@ __global__ __launch_bounds__(KL * NG * 64) void linear_share_kernel(
       gload_x(i + 2);
       gload_w(w[(st + PF - 1) % PF], i + PF - 1);
       compute(w[st], i);
+      if (LEVELS && (is_bf<MODE> || part)) settle();
       if (i < total && (i + 1) % nstages == 0) finish(i);
       __syncthreads();
     }
@@ -1997,11 +2018,15 @@ void launch_wide(const void* xp, const void* W, const void* scales, float* part,
   int ks_per_split = (nks + S - 1) / S;
   if (W8) ks_per_split = (ks_per_split + 1) & ~1;  // int8 blocks cover two steps
   if constexpr (!W8) {
-    if (vocabulary_tiles(tiles_per_wg))
-      return tiles_per_wg == 13 ? launch_share_cfg<8, W8, MODE, 1, 13, 1, 2>(xp, W, scales, part, S, M, N, K,
-                                                                             tiles_per_wg, gx, ks_per_split, epi, s)
-                                : launch_share_cfg<8, W8, MODE, 1, 14, 1, 2>(xp, W, scales, part, S, M, N, K,
-                                                                             tiles_per_wg, gx, ks_per_split, epi, s);
+    // (results of 16 bits only: its one chain over K has 1.4 times the error of two K lanes, K = 4096 3.9e-7 and 2.7e-7.
+    // fp32 results of 128 rows by two K lanes: 50272 x 4096 114 us, by the chain 99.)
+    if constexpr (!is_bf<MODE>) {
+      if (vocabulary_tiles(tiles_per_wg) && !part)
+        return tiles_per_wg == 13 ? launch_share_cfg<8, W8, MODE, 1, 13, 1, 2>(xp, W, scales, part, S, M, N, K,
+                                                                               tiles_per_wg, gx, ks_per_split, epi, s)
+                                  : launch_share_cfg<8, W8, MODE, 1, 14, 1, 2>(xp, W, scales, part, S, M, N, K,
+                                                                               tiles_per_wg, gx, ks_per_split, epi, s);
+    }
     if (tiles_per_wg == 4)
       return launch_share_cfg<8, W8, MODE, 2, 4, 1, 4>(xp, W, scales, part, S, M, N, K, tiles_per_wg, gx,
                                                        ks_per_split, epi, s);

@@ -102,6 +102,21 @@ def test_linear_bf16_of_a_wave_per_tile(M, N, K):
     test_linear_bf16(M, N, K)
 
 
+@pytest.mark.parametrize("M,K,most", [(1, 768, 1.0e-7), (33, 4096, 1.8e-7), (64, 9216, 2.5e-7), (100, 4096, 3.3e-7)])
+def test_fp32_logits_of_a_vocabulary_are_no_single_chain_over_k(M, K, most):
+    """The error of fp32 sums grows with the root of the additions behind each: K / 128 stages of four steps up to 64 rows,
+    K / 64 steps beyond.  One chain of K / 32 steps has 1.6, 3.9, 6.1 and 3.9e-7 here."""
+    lib, N = _capi.load_hybrid(), 50272
+    g = torch.Generator("cuda").manual_seed(K)
+    x = torch.randn(M, K, generator=g, device="cuda").to(BF16)
+    w = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).to(BF16)
+    y = torch.empty(M, N, device="cuda")
+    check(lib.msa_linear_partial_bf16(ptr(pack_rows(x.cpu()).cuda()), ptr(pack_tiles(w)), ptr(y), M, N, K, 1,
+                                      _capi.MSA_IN_PACKED, _capi.stream_ptr()), lib)
+    want = x.double() @ w.double().t()
+    assert float((y.double() - want).norm() / want.norm()) <= most
+
+
 @pytest.mark.parametrize("M,N", [(4352, 16656), (600, 24576)])
 def test_linear_partial_bf16_wide_panels(M, N):
     """More than 64 columns of tiles, taken in panels of 16; sums of one and two slices."""
