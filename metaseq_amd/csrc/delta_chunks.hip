@@ -837,7 +837,10 @@ __global__ __launch_bounds__(512) void delta_chunk_ready_kernel(
 // Many segments: a workgroup owns CT x 16 columns of a head, one wave 16 of them with all rows of the state, so
 // that nothing is summed between waves and k, q and decays are staged for CT column tiles at once; four
 // more waves stage.  One barrier per chunk.
-template <typename T, int DP, bool CH, int CT>
+// CHAINS: accumulators of K' S0 and Q' S0.  Two are enough to keep the matrix cores busy; widths with a last partial
+// group, which few segments' kernels would take otherwise, get one per tile of the state as there (error of the outputs
+// against 64 bits, 8 x 300 tokens, 16 heads of 96 columns: two 1.76e-7, one per tile 1.58e-7 as staged; 208 and 211 us).
+template <typename T, int DP, bool CH, int CT, int CHAINS>
 __global__ __launch_bounds__((CT + 4) * 64) void delta_chunk_wide_kernel(
     const T* __restrict__ qkv, int64_t ld, const float* __restrict__ decay, int heads, int kv_heads, int vp,
     float* __restrict__ state, const float* __restrict__ records, float* __restrict__ o,
@@ -913,16 +916,26 @@ __global__ __launch_bounds__((CT + 4) * 64) void delta_chunk_wide_kernel(
   };
   auto chunk = [&](Ahead& x, int c) {
     const int b = c & 1;
-    auto times_state = [&](const float* p) {  // two chains
-      float4_t sum[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    auto times_state = [&](const float* p) {
+      float4_t sum[CHAINS];
 #pragma unroll
-      for (int t = 0; t < TILES; t += 2) {
-        const float4_t a[2] = {*reinterpret_cast<const float4_t*>(p + t * 16),
-                               *reinterpret_cast<const float4_t*>(p + t * 16 + 16)};
-        const float4_t x2[2] = {S[t], S[t + 1]};
-        mfma4(a, x2, sum);
+      for (int i = 0; i < CHAINS; ++i) sum[i] = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int t = 0; t < TILES; t += CHAINS) {
+        float4_t a[CHAINS], x[CHAINS];
+#pragma unroll
+        for (int i = 0; i < CHAINS; ++i) {
+          a[i] = *reinterpret_cast<const float4_t*>(p + (t + i) * 16);
+          x[i] = S[t + i];
+        }
+        mfma4(a, x, sum);
       }
-      return sum[0] + sum[1];
+#pragma unroll
+      for (int i = 0; i < CHAINS; i += 2) {
+        if (i + 1 < CHAINS) sum[i] += sum[i + 1];
+        if (i > 0) sum[0] += sum[i];
+      }
+      return sum[0];
     };
     const float4_t ks = times_state(&L.k[b][lm][lg * 4]);
     float4_t y = times_state(&L.q[b][lm][lg * 4]) * x.f.q;
@@ -968,17 +981,17 @@ __global__ __launch_bounds__((CT + 4) * 64) void delta_chunk_wide_kernel(
 // channel is most of the work, until their 27 KB per chunk and head are what is waited for: then the wide kernel, whose
 // staging serves four tiles, is the better one for any width, and a single tile stages for itself.  128 keys, decays per
 // channel, us staged / ready / wide of 64, 1000 tokens of one segment: 64 heads of 96 columns (384 workgroups) 236 / 158 /
-// 186, 96 of 80 (480) 245 / 185 / 196, 128 of 48 (384) 254 / 215 / 201, 128 of 80 (640) 358 / 277 / 207; 500 tokens, 256 of
-// 32 (512) 153 / 165 / 125; 8 x 1024 tokens, 16 of 96 (768) 359 / 285 / 208; one tile, 128 heads 150 / 148 / 199, 256 heads
+// 186, 96 of 80 (480) 245 / 185 / 196, 128 of 48 (384) 254 / 215 / 201, 128 of 80 (640) 358 / 277 / 211; 500 tokens, 256 of
+// 32 (512) 153 / 165 / 127; 8 x 1024 tokens, 16 of 96 (768) 359 / 285 / 211; one tile, 128 heads 150 / 148 / 199, 256 heads
 // 195 / 268 / 239.
-enum Form { STAGED, READY, WIDE_64, WIDE_128 };
+enum Form { STAGED, READY, WIDE_64, WIDE_128, WIDE_ANY, FORMS };
 Form form_of(const msa_delta_args& a, const msa_batch* b) {
   const int64_t units = (int64_t)b->nseg * a.heads;
   if (a.vp % 128 == 0 && units >= DC_WIDE) return WIDE_128;
   if (a.vp % 64 == 0 && units * (a.vp / 64) >= DC_WIDE) return WIDE_64;
   if (!a.decay) return STAGED;
   if (a.vp == 16) return units <= DC_WIDE ? READY : STAGED;
-  return a.vp % 64 != 0 && units * (a.vp / 16) >= DC_READY ? WIDE_64 : READY;
+  return a.vp % 64 != 0 && units * (a.vp / 16) >= DC_READY ? WIDE_ANY : READY;
 }
 
 // Chunks of every segment whose long records are kept at a time, all portions alike; 0: all.  32 heads of 128, one segment
@@ -1017,13 +1030,16 @@ int run_chunks(const msa_delta_args& a, const msa_batch* b, float* scratch, hipS
     }
   }
   prepare(delta_prepare_kernel<T, DP, CH, false>, chunks, Portion{});
-  auto kernel = form == WIDE_128  ? delta_chunk_wide_kernel<T, DP, CH, 8>
-                : form == WIDE_64 ? delta_chunk_wide_kernel<T, DP, CH, 4>
+  auto kernel = form == WIDE_128  ? delta_chunk_wide_kernel<T, DP, CH, 8, 2>
+                : form == WIDE_64 ? delta_chunk_wide_kernel<T, DP, CH, 4, 2>
                                   : delta_chunk_kernel<T, DP, CH>;
-  const int cols = form == WIDE_128 ? 128 : form == WIDE_64 ? 64 : 16;
+  if constexpr (CH) {
+    if (form == WIDE_ANY) kernel = delta_chunk_wide_kernel<T, DP, CH, 4, DP / 16>;
+  }
+  const int cols = form == WIDE_128 ? 128 : form == STAGED ? 16 : 64;
   const int threads = form == WIDE_128 ? 768 : 512;
   const int bytes = form == STAGED ? (int)sizeof(StagedLds<DP, CH>) : (int)sizeof(Operands<DP, CH>);
-  static std::atomic<uint64_t> raised[WIDE_128 + 1];
+  static std::atomic<uint64_t> raised[FORMS];
   if (!raise_lds((const void*)kernel, bytes, raised[form])) {
     msa_set_error("msa_delta_scan_chunks: %d bytes of LDS refused", bytes);
     return MSA_ERR_HIP;
