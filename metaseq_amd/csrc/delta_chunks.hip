@@ -14,7 +14,7 @@
 // K', Q' and K^) is computed for all chunks of all heads at once, a wave each, and left in a scratch record; then the
 // chunks of a (segment, head, some columns) are walked one after the other.  A scan step's chain of LDS reads, two
 // dots, a sum over lanes and the update takes 500 cycles per token whatever the machine has idle; a
-// chunk's chain takes 2700 per sixteen with one decay per head and 2300 with decays per channel
+// chunk's chain takes 2900 per sixteen with one decay per head and 2400 with decays per channel
 // where few segments leave a workgroup a CU of its own.  Where many fill the chip the matrix cores are the bound: 104
 // fp32 products of 32 cycles per wave and chunk, two such waves per SIMD, 6650 cycles of the 11000 a chunk takes.
 // Measured, both kernels against the scan, 32 heads of 128 x 128: one segment of 1500 tokens 128 us against 349
