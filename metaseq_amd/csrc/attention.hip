@@ -153,14 +153,13 @@ __global__ void attention_kernel(const half_t* __restrict__ q, const half_t* __r
       for (int i = 0; i < 8; ++i) acc[i] = fmaf(p, (float)vv[i], acc[i]);
     }
   };
-  if (rows < U) {  // (apart: the checks cost a long history 1 %, their absence a short one 4 %)
+  do {  // (uniform: a short history leaves behind its last row; a check in front of every row cost long ones 1 to 2 %)
 #pragma unroll
-    for (int u = 0; u + 1 < U; ++u)
-      if (u < rows) weigh(vpre[u], vkey0 + u * kstride);  // uniform
-  } else {
-#pragma unroll
-    for (int u = 0; u < U; ++u) weigh(vpre[u], vkey0 + u * kstride);
-  }
+    for (int u = 0; u < U; ++u) {
+      weigh(vpre[u], vkey0 + u * kstride);
+      if (u + 1 == rows) break;
+    }
+  } while (false);
   for (key = vkey0 + U * kstride; key + (U - 1) * kstride < n_keys; key += U * kstride) {
     half8_t vv[U];
 #pragma unroll
