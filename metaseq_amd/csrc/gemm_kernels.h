@@ -1256,6 +1256,17 @@ __device__ __forceinline__ void tq_mfma(float4_t& acc, const half8_t& a, const h
     asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
 }
 
+// Which of a step's RF x WF MFMAs (row * WF + column) is the q-th: two rows side by side, column after column, back and
+// forth.  What an MFMA draws depends on the operands of the one before it, and the part lowers its clock by that:
+// MFMAs alone, random operands, 1.91 PFLOP/s row by row, 1.96 so (one operand new each time, a snake of rows, 1.93;
+// both new 1.84; four rows side by side 1.90).  32768 x 16384 x 4096 3118 -> 3075 us, 2048 x 16384 x 4096 206 -> 200.
+constexpr int tq_order(int RF, int WF, int q) {
+  const int g = q / (2 * WF), w = q % (2 * WF);
+  if (2 * g + 1 >= RF) return 2 * g * WF + (g & 1 ? WF - 1 - w : w);
+  const int c = w / 2;
+  return (2 * g + (w & 1)) * WF + (g & 1 ? WF - 1 - c : c);
+}
+
 template <int... I, class F>
 __device__ __forceinline__ void tq_static_for_impl(std::integer_sequence<int, I...>, F&& f) {
   (f(std::integral_constant<int, I>{}), ...);
@@ -1482,7 +1493,8 @@ __device__ __forceinline__ void quad_tile(const half_t* __restrict__ x, const vo
       constexpr int i = decltype(ic)::value;
       tq_static_for<WF>([&](auto jc) {
         constexpr int j = decltype(jc)::value;
-        tq_mfma<MODE>(acc[i][j], wf[H][j], xf[H][i]);
+        constexpr int o = tq_order(RF, WF, i * WF + j);
+        tq_mfma<MODE>(acc[o / WF][o % WF], wf[H][o % WF], xf[H][o / WF]);
         if constexpr (RF == 4) {
           if (j == 1) xf[H ^ 1][i] = H == 0 ? xfrag(xs, 1, i) : xfrag(xnext, 0, i);
           if (j == 3) wf[H ^ 1][i] = wfrag(wnext, i);
