@@ -1238,13 +1238,14 @@ __global__ __launch_bounds__(TB_THREADS) void linear_tiled_big_kernel(
 constexpr int TQ_BM = 256, TQ_THREADS = 256;  // (rows of a tile unless RF is given)
 constexpr int TQ_PANEL = 16;  // columns of tiles taken together where many lie across
 constexpr int tq_bm(int RF) { return 32 * RF; }
-constexpr int tq_rx(int RF) { return RF == 8 ? 3 : 5; }    // stages of activations in the ring
-constexpr int tq_rw(int RF) { return RF == 8 ? 4 : 8; }    // steps of weights
+// stages of activations and steps of weights in the rings: as many as 160 KB hold, steps for all but one stage
+constexpr int tq_rx(int RF, int WF) { return RF == 4 && WF == 4 ? 5 : RF == 4 || (RF < 8 && WF == 4) ? 4 : 3; }
+constexpr int tq_rw(int RF, int WF) { return 2 * (tq_rx(RF, WF) - 1); }
 constexpr int tq_xbytes(int RF) { return tq_bm(RF) * 64 * 2; }  // one 64-wide stage of activations
 constexpr int tq_bn(int WF) { return 32 * WF; }
 constexpr int tq_wbytes(int WF) { return 2 * WF * 1024; }  // one 32-wide step of weights
 constexpr int tq_lds_bytes(int WF, int RF = 8) {  // 160 / 128 / 112 KB; 144 KB with RF = 4
-  return tq_rx(RF) * tq_xbytes(RF) + tq_rw(RF) * tq_wbytes(WF);
+  return tq_rx(RF, WF) * tq_xbytes(RF) + tq_rw(RF, WF) * tq_wbytes(WF);
 }
 typedef __attribute__((address_space(3))) void tq_lds_void;
 
@@ -1320,22 +1321,22 @@ struct GroupTiles {
 // that starts at stage z * part_stages and stores its fp32 sums, with no epilogue, as slice z of
 // ``part`` ([gridDim.z][M][N]); a later launch adds the slices in slice order.
 template <int MODE, int WF, bool PART, bool GROUPED, int RF, bool FEW>
+// (m_own: the first row that this tile owns)
 __device__ __forceinline__ void quad_tile(const half_t* __restrict__ x, const void* __restrict__ Wp, int64_t M, int N,
-                                          int K, int bx, int by, int bz, int64_t g_first, const Epilogue& epi,
+                                          int K, int bx, int64_t m_own, int bz, const Epilogue& epi,
                                           float* __restrict__ part, int part_stages, const GroupTiles& gt) {
   extern __shared__ __attribute__((aligned(16))) char tq_lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 15, lg = lane >> 4;
   const int wm = wave >> 1, wn = wave & 1;
   constexpr int TQ_BN = tq_bn(WF), TQ_WBYTES = tq_wbytes(WF), TQ_BM = tq_bm(RF), TQ_XBYTES = tq_xbytes(RF);
-  constexpr int TQ_RX = tq_rx(RF), TQ_RW = tq_rw(RF), TQ_WOFF = TQ_RX * TQ_XBYTES;
+  constexpr int TQ_RX = tq_rx(RF, WF), TQ_RW = tq_rw(RF, WF), TQ_WOFF = TQ_RX * TQ_XBYTES;
   constexpr int WL = WF / 2;  // weight load instructions per wave and step
   constexpr int XL = RF;      // activation load instructions per wave and stage
   // The narrowest form (WF = 2) also serves fewer than 256 rows: it does not move a ragged tile up
   // but repeats the last row in its loads and drops the rows past it in the epilogue.  So does
   // the split-K form of WF = 4 (decode batches of 129 .. 255 rows cut K eight ways over it).
-  constexpr bool CLAMP = WF == 2 || (WF == 4 && PART) || GROUPED || RF == 4 || FEW;
-  const int64_t m_own = GROUPED ? g_first : (int64_t)by * TQ_BM;  // first row this tile owns
+  constexpr bool CLAMP = WF == 2 || (WF == 4 && PART) || GROUPED || (RF == 4 && WF == 4) || FEW;
   const int64_t m0 = !CLAMP && m_own + TQ_BM > M ? M - TQ_BM : m_own;
   const int n0 = bx * TQ_BN;
   // the stages this workgroup sums over: all of K, or its slice (the operand bases below move
@@ -1365,6 +1366,9 @@ __device__ __forceinline__ void quad_tile(const half_t* __restrict__ x, const vo
   const uint32_t xrow = (uint32_t)(lane >> 3) * (uint32_t)K * 2;
   const uint32_t xlane0 = xrow + (((lane & 7) ^ (lane >> 4)) * 16);
   const uint32_t xlane1 = xrow + (((lane & 7) ^ (4 + (lane >> 4))) * 16);
+  // (an odd RF: the second and the fourth wave's rows begin at an odd multiple of eight)
+  const bool swap = RF % 2 && (wave & 1);
+  const uint32_t xeven = swap ? xlane1 : xlane0, xodd = swap ? xlane0 : xlane1;
   const uint32_t wlane = lane * 16;
   // CLAMP: per instruction, the lane's row offset from the (clamped) scalar base row
   uint32_t xl[CLAMP ? XL : 1];
@@ -1378,7 +1382,7 @@ __device__ __forceinline__ void quad_tile(const half_t* __restrict__ x, const vo
       } else {
         d -= min(r, M - 1);
       }
-      xl[i] = (uint32_t)d * (uint32_t)K * 2 + ((i & 1 ? xlane1 : xlane0) - xrow);
+      xl[i] = (uint32_t)d * (uint32_t)K * 2 + ((i & 1 ? xodd : xeven) - xrow);
     }
   }
   const uint32_t lds0 = (uint32_t)(uintptr_t)(tq_lds_void*)tq_lds;
@@ -1390,8 +1394,8 @@ __device__ __forceinline__ void quad_tile(const half_t* __restrict__ x, const vo
   auto set_x = [&](int slot, int st) {
     st = min(st, nst - 1);
     xst = st * 128;
-    xv0 = xlane0 + st * 128;
-    xv1 = xlane1 + st * 128;
+    xv0 = xeven + st * 128;
+    xv1 = xodd + st * 128;
     xm0 = lds0 + slot * TQ_XBYTES + wave * (TQ_BM / 4 * 128) + XL / 2 * 1024;
   };
   auto set_w = [&](int slot, int ks) {
@@ -1452,7 +1456,7 @@ __device__ __forceinline__ void quad_tile(const half_t* __restrict__ x, const vo
   // prologue: activation stages 0 and 1, weight steps 0..3 requested; stages 0, 1 and steps 0, 1
   // landed
   half8_t xf[2][RF], wf[2][WF];
-  if constexpr (RF == 8) {
+  if constexpr (TQ_RX == 3) {
     group_x(0, 0);
     group_w(0, 0);
     group_x(1, 1);
@@ -1495,7 +1499,27 @@ __device__ __forceinline__ void quad_tile(const half_t* __restrict__ x, const vo
         constexpr int j = decltype(jc)::value;
         constexpr int o = tq_order(RF, WF, i * WF + j);
         tq_mfma<MODE>(acc[o / WF][o % WF], wf[H][o % WF], xf[H][o / WF]);
-        if constexpr (RF == 4) {
+        if constexpr (RF < 8 && !(RF == 4 && WF == 4)) {
+          // one instruction behind an MFMA: fragments of step t + 1, then a row's load of activations (even steps)
+          // and one of weights
+          if (j == 1) xf[H ^ 1][i] = H == 0 ? xfrag(xs, 1, i) : xfrag(xnext, 0, i);
+          if constexpr (WF == 8) {
+            if constexpr (j == 5) wf[H ^ 1][i] = wfrag(wnext, i);
+            if constexpr (j == 7 && RF + i < WF) wf[H ^ 1][(RF + i) % WF] = wfrag(wnext, (RF + i) % WF);
+          } else {
+            if constexpr (j == 3 && i < WF) wf[H ^ 1][i % WF] = wfrag(wnext, i % WF);
+          }
+          if constexpr (H == 0) {
+            if (i == 0 && j == 0) set_x(xfree, S + TQ_RX - 1);
+            if constexpr (j == 0) issue_x(ic);
+          }
+          if (i == 0 && j == 1) set_w(ws, t + TQ_RW);
+          if constexpr (WF == 8) {
+            if constexpr (j == 3 && i < WL) issue_w(std::integral_constant<int, i % WL>{});
+          } else {
+            if constexpr (j == 2 && (i == 1 || i == 3)) issue_w(std::integral_constant<int, (i >> 1) % WL>{});
+          }
+        } else if constexpr (RF == 4) {
           if (j == 1) xf[H ^ 1][i] = H == 0 ? xfrag(xs, 1, i) : xfrag(xnext, 0, i);
           if (j == 3) wf[H ^ 1][i] = wfrag(wnext, i);
           if constexpr (H == 0) {
@@ -1692,7 +1716,8 @@ __device__ __forceinline__ void quad_tile(const half_t* __restrict__ x, const vo
         b = m / epi.T;
         at += m - b * epi.T;
       }
-      fill[k + lane] = ok && at < epi.S_cap ? ((int64_t)b * epi.H * epi.S_cap + at) * epi.hd : -1;
+      if (TQ_BM / 2 % 64 == 0 || k + lane < TQ_BM / 2)
+        fill[k + lane] = ok && at < epi.S_cap ? ((int64_t)b * epi.H * epi.S_cap + at) * epi.hd : -1;
     }
     const int D = epi.H * epi.hd;
     qkv_part = (en >= D) + (en >= 2 * D);  // 0 = K, 1 = V, 2 = Q
@@ -1804,7 +1829,8 @@ __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
   } else if (rm_a > 0) {
     quad_regroup(by * gridDim.x + bx, gridDim.x, gridDim.y, rm_a, rm_r, bx, by);
   }
-  quad_tile<MODE, WF, PART, GROUPED, RF, FEW>(x, Wp, M, N, K, bx, by, blockIdx.z, g_first, epi, part, part_stages, gt);
+  const int64_t m_own = GROUPED ? g_first : (int64_t)by * tq_bm(RF);
+  quad_tile<MODE, WF, PART, GROUPED, RF, FEW>(x, Wp, M, N, K, bx, m_own, blockIdx.z, epi, part, part_stages, gt);
 }
 
 // Tiles that would begin a round without filling half of it, in pieces: the first n_full tiles (of all K slices, whole
@@ -1823,16 +1849,36 @@ __global__ __launch_bounds__(TQ_THREADS) void linear_quad_pieces_kernel(
   const int bz = PART ? unit / tiles : 0;
   quad_place(unit - bz * tiles, ncol, nrow, rm_a, rm_r, bx, by);
   const GroupTiles none{};
-  if (j < 0) return quad_tile<MODE, 8, PART, false, 8, false>(x, Wp, M, N, K, bx, by, bz, 0, epi, part, part_stages, none);
+  const int64_t m_own = (int64_t)by * TQ_BM;
+  if (j < 0) return quad_tile<MODE, 8, PART, false, 8, false>(x, Wp, M, N, K, bx, m_own, bz, epi, part, part_stages, none);
   bx = 2 * bx + (piece & 1);
   if (bx * tq_bn(4) >= N) return;
   if constexpr (PIECES == 2) {
-    quad_tile<MODE, 4, PART, false, 8, false>(x, Wp, M, N, K, bx, by, bz, 0, epi, part, part_stages, none);
+    quad_tile<MODE, 4, PART, false, 8, false>(x, Wp, M, N, K, bx, m_own, bz, epi, part, part_stages, none);
   } else {
-    by = 2 * by + (piece >> 1);
-    if ((int64_t)by * tq_bm(4) < M)
-      quad_tile<MODE, 4, PART, false, 4, false>(x, Wp, M, N, K, bx, by, bz, 0, epi, part, part_stages, none);
+    const int64_t m = m_own + (piece >> 1) * tq_bm(4);
+    if (m < M) quad_tile<MODE, 4, PART, false, 4, false>(x, Wp, M, N, K, bx, m, bz, epi, part, part_stages, none);
   }
+}
+
+// Rows cut evenly instead of by 256: the first n_tall rows of tiles are 32 RF high, the others 32 less (RF = 5 .. 8), at
+// least 256 rows in all.
+template <int MODE, int WF, bool PART, int RF>
+__global__ __launch_bounds__(TQ_THREADS) void linear_quad_even_kernel(
+    const half_t* __restrict__ x, const void* __restrict__ Wp, int64_t M, int N, int K, int nrow, int n_tall, int rm_a,
+    int rm_r, Epilogue epi, float* __restrict__ part, int part_stages) {
+  int bx = blockIdx.x, by = blockIdx.y;
+  if (rm_a < 0) {
+    if (!quad_panel(by, bx, (N + tq_bn(WF) - 1) / tq_bn(WF), nrow, bx, by)) return;
+  } else if (rm_a > 0) {
+    quad_regroup(by * gridDim.x + bx, gridDim.x, nrow, rm_a, rm_r, bx, by);
+  }
+  const GroupTiles none{};
+  const int64_t m_own = (int64_t)(by * RF - max(by - n_tall, 0)) * 32;
+  if (by < n_tall)
+    quad_tile<MODE, WF, PART, false, RF, false>(x, Wp, M, N, K, bx, m_own, blockIdx.z, epi, part, part_stages, none);
+  else
+    quad_tile<MODE, WF, PART, false, RF - 1, false>(x, Wp, M, N, K, bx, m_own, blockIdx.z, epi, part, part_stages, none);
 }
 
 // ---- host side ------------------------------------------------------------------------------
@@ -2157,22 +2203,108 @@ dim3 quad_grid(int ncol, int nrow, const TileOrder& o, int slices = 1) {
   return o.a < 0 ? dim3(TQ_PANEL * nrow, (ncol + TQ_PANEL - 1) / TQ_PANEL, slices) : dim3(ncol, nrow, slices);
 }
 
-// Time of a round of tiles, in rounds of 256 x 256 ones (103 us of K = 4096): 256 x 128 63 us, 256 x 64 45, 128 x 128 37.
-constexpr double TQ_ROUND_US = 103.0 / 4096, TQ_COST_4 = 0.61, TQ_COST_2 = 0.43, TQ_COST_Q = 0.36;
-int64_t quad_rounds(int64_t tiles) { return (tiles + num_cus() - 1) / num_cus(); }
+// Time of a tile of 32 RF rows and 32 WF columns while the whole chip computes such tiles, us; of a round that
+// fills a part of it: the clock rises as CUs fall idle (K = 16384, 256 x 256 tiles on 256, 192 and 128 CUs 382, 325 and
+// 277 us).  Fitted to 1200 products of 260 .. 6038 rows (K = 768 .. 16384), which it meets within 5 % (rms).
+double quad_tile_us(int WF, int RF, int K) {
+  if (WF == 2) return 4.3 + 0.0088 * K;
+  return WF == 8 ? 1.0 + 1.45 * RF + (0.0063 + 0.00165 * RF) * K : 0.8 + 0.75 * RF + (0.0024 + 0.00127 * RF) * K;
+}
+double quad_part_round(int tiles, int cus) { return 0.75 + 0.25 * tiles / cus; }
+double quad_rounds_us(int64_t tiles, double tile_us, int cus) {
+  const int left = (int)(tiles % cus);
+  return tile_us * ((double)(tiles / cus) + (left ? quad_part_round(left, cus) : 0.0));
+}
 // Into how many pieces the tiles are cut that are left after whole rounds of 256 x 256 ones (1: they are not): as many
 // as still run in one round.  Without and with, K = 4096, us: 2005 x 9216 (32 tiles left) 170 -> 130 in quarters,
 // 147 in halves; 2005 x 10240 (64) 171 -> 136, 149; 1500 x 14848 (92) 198 -> 171; 2005 x 12288 (128) 179 ->
 // 162, 171 in quarters; 6038 x 5888 (two rounds and 40) 272 -> 233; 2005 x 50272 (six and 40) 677 -> 638.
 // More than half a round is not cut: 1500 x 50272 (four and 158) 490 and 502.
-int quad_pieces(int64_t tiles) {
-  const int64_t left = tiles % num_cus();
-  return tiles < num_cus() || left == 0 || left * 2 > num_cus() ? 1 : left * 4 > num_cus() ? 2 : 4;
+int quad_pieces(int64_t tiles, int cus) {
+  const int64_t left = tiles % cus;
+  return tiles < cus || left == 0 || left * 2 > cus ? 1 : left * 4 > cus ? 2 : 4;
 }
-double quad_cost(int64_t tiles) {
-  const int pieces = quad_pieces(tiles);
-  return pieces == 1 ? (double)quad_rounds(tiles)
-                     : (double)(tiles / num_cus()) + (pieces == 2 ? TQ_COST_4 : TQ_COST_Q);
+double quad_cost(int64_t tiles, int K, int cus) {  // 256 x 256 tiles, us
+  const int pieces = quad_pieces(tiles, cus);
+  if (pieces == 1) return quad_rounds_us(tiles, quad_tile_us(8, 8, K), cus);
+  return (double)(tiles / cus) * quad_tile_us(8, 8, K) +
+         quad_rounds_us(tiles % cus * pieces, quad_tile_us(4, pieces == 2 ? 8 : 4, K), cus);
+}
+
+// The cheapest even cut of at least 256 rows (linear_quad_even_kernel): as many rows of tiles as fill whole rounds,
+// each of the height that is left for it, so that neither a round is left half empty nor a row of tiles.
+// Against tiles of one height (256 rows, or 128 x 128), us: 300 x 16384 x 4096 68 -> 50, 640 x 12288 x 4096 80 -> 67, 900 x
+// 16384 x 4096 110 -> 97, 1100 x 4096 x 4096 53 -> 40, 1260 x 4096 x 16384 201 -> 167, 1607 x 16384 x 4096 in a model 211 ->
+// 180, 2140 x 2048 x 8192 101 -> 75, 2460 x 4096 x 16384 328 -> 252, 1390 x 6144 x 2048 61 -> 37; 360 products of 66 ..
+// 8300 rows (K = 768 .. 16384) 4 % on average, none slower than the runs of one side differ.
+struct QuadPlan {
+  double us = 1e30;
+  int wf = 0, rf = 0, nrow = 0, n_tall = 0;
+};
+QuadPlan quad_plan(int64_t M, int N, int K, int S, int cus) {
+  QuadPlan best;
+  if (M < TQ_BM || M > 16384) return best;
+  const int units = (int)((M + 31) / 32), most = 24 * cus;
+  for (int wf = 4; wf <= 8; wf += 4) {
+    const int ncol = (N + tq_bn(wf) - 1) / tq_bn(wf);
+    // (128 columns: 256-row tiles among lower ones are never the cheapest)
+    for (int nrow = (units + wf / 4 + 5) / (wf / 4 + 6); nrow * 4 < units + 4; ++nrow) {
+      const int rf = nrow * 4 < units ? (units + nrow - 1) / nrow : 5;  // (the last: all rows 128 high)
+      const int n_tall = nrow * 4 < units ? units - nrow * (rf - 1) : 0, slice = nrow * ncol, tiles = slice * S;
+      if (tiles > most) break;
+      const double tall = quad_tile_us(wf, rf, K / S), low = quad_tile_us(wf, rf - 1, K / S);
+      double us = 0;
+      for (int t = 0; t < tiles && us < best.us; t += cus) {  // a round takes as long as its tallest tile
+        const int n = tiles - t < cus ? tiles - t : cus, at = S == 1 ? t : t % slice;
+        us += (at < n_tall * ncol || (n_tall && at + n > slice) ? tall : low) * (n < cus ? quad_part_round(n, cus) : 1.0);
+      }
+      if (us < best.us) best = QuadPlan{us, wf, rf, nrow, n_tall};
+    }
+  }
+  return best;
+}
+// The cheapest form of S sums over at least 256 rows: 256 x 256 tiles, the last of them in pieces (w = 8), 256 x
+// 128 (4), 256 x 64 (2), or an even cut.
+constexpr int QUAD_EVEN = 1;
+struct QuadPrice {
+  double us;
+  int w;
+  QuadPlan even;
+};
+QuadPrice quad_price(int64_t M, int N, int K, int S, int cus) {
+  const int64_t rows = (M + TQ_BM - 1) / TQ_BM * S;
+  QuadPrice best{quad_cost(rows * ((N + 255) / 256), K / S, cus), 8, quad_plan(M, N, K, S, cus)};
+  const double four = quad_rounds_us(rows * ((N + 127) / 128), quad_tile_us(4, 8, K / S), cus);
+  const double two = quad_rounds_us(rows * ((N + 63) / 64), quad_tile_us(2, 8, K / S), cus);
+  if (four < best.us) best.us = four, best.w = 4;
+  if (two < best.us) best.us = two, best.w = 2;
+  if (best.even.us < best.us) best.us = best.even.us, best.w = QUAD_EVEN;
+  return best;
+}
+template <int MODE, int WF, bool PART, int RF>
+void launch_quad_even(const void* x, const void* W, int64_t M, int N, int K, int S, const QuadPlan& p,
+                      const Epilogue& epi, float* part, hipStream_t s) {
+  static std::atomic<uint64_t> lds_allowed_e{0};
+  constexpr int lds = tq_lds_bytes(WF, RF) > tq_lds_bytes(WF, RF - 1) ? tq_lds_bytes(WF, RF) : tq_lds_bytes(WF, RF - 1);
+  auto kernel = linear_quad_even_kernel<MODE, WF, PART, RF>;
+  if (!allow_lds((const void*)kernel, lds, lds_allowed_e)) return;
+  const int ncol = (N + tq_bn(WF) - 1) / tq_bn(WF);
+  const TileOrder o = tile_order(ncol, p.nrow, WF);
+  hipLaunchKernelGGL(kernel, quad_grid(ncol, p.nrow, o, S), dim3(TQ_THREADS), lds, s, (const half_t*)x, W, M, N, K,
+                     p.nrow, p.n_tall, o.a, o.r, epi, part, K / 64 / S);
+}
+template <int MODE, bool PART>
+void launch_quad_plan(const void* x, const void* W, int64_t M, int N, int K, int S, const QuadPlan& p,
+                      const Epilogue& epi, float* part, hipStream_t s) {
+  if (p.wf == 8) {
+    if (p.rf == 8) return launch_quad_even<MODE, 8, PART, 8>(x, W, M, N, K, S, p, epi, part, s);
+    if (p.rf == 7) return launch_quad_even<MODE, 8, PART, 7>(x, W, M, N, K, S, p, epi, part, s);
+    if (p.rf == 6) return launch_quad_even<MODE, 8, PART, 6>(x, W, M, N, K, S, p, epi, part, s);
+    return launch_quad_even<MODE, 8, PART, 5>(x, W, M, N, K, S, p, epi, part, s);
+  }
+  if (p.rf == 7) return launch_quad_even<MODE, 4, PART, 7>(x, W, M, N, K, S, p, epi, part, s);
+  if (p.rf == 6) return launch_quad_even<MODE, 4, PART, 6>(x, W, M, N, K, S, p, epi, part, s);
+  return launch_quad_even<MODE, 4, PART, 5>(x, W, M, N, K, S, p, epi, part, s);
 }
 
 template <int MODE, bool PART, int PIECES>
@@ -2196,7 +2328,7 @@ void launch_quad(const void* x, const void* W, const void* scales, int64_t M, in
                  int K, const Epilogue& epi, hipStream_t s) {
   const int ncol = (N + tq_bn(WF) - 1) / tq_bn(WF);
   const int nrow = (int)((M_main + TQ_BM - 1) / TQ_BM);
-  const int pieces = WF == 8 ? quad_pieces((int64_t)ncol * nrow) : 1;
+  const int pieces = WF == 8 ? quad_pieces((int64_t)ncol * nrow, num_cus()) : 1;
   if (pieces == 4) {
     launch_quad_pieces<MODE, false, 4>(x, W, M_main, N, K, 1, epi, nullptr, s);
   } else if (pieces == 2) {
@@ -2259,21 +2391,60 @@ template <int MODE>
 void launch_quad_partial(const void* x, const void* W, float* part, int64_t M, int N, int K, int S,
                          hipStream_t s) {
   const int64_t rows = (M + TQ_BM - 1) / TQ_BM;
-  const int64_t tiles2 = rows * ((N + 63) / 64) * S, tiles4 = rows * ((N + 127) / 128) * S;
-  if constexpr (is_bf<MODE>) {
-    const int64_t tiles8 = rows * ((N + 255) / 256) * S;
-    const double narrow = fmin(quad_rounds(tiles4) * TQ_COST_4, quad_rounds(tiles2) * TQ_COST_2);
-    if (M >= TQ_BM && quad_cost(tiles8) <= narrow) {
-      const int pieces = quad_pieces(tiles8);
+  const int64_t tiles2 = rows * ((N + 63) / 64) * S;
+  if (M >= TQ_BM) {
+    const QuadPrice price = quad_price(M, N, K, S, num_cus());
+    if (price.w == QUAD_EVEN) return launch_quad_plan<MODE, true>(x, W, M, N, K, S, price.even, Epilogue{}, part, s);
+    if (price.w == 8) {
+      const int pieces = quad_pieces(rows * ((N + 255) / 256) * S, num_cus());
       if (pieces == 4) return launch_quad_pieces<MODE, true, 4>(x, W, M, N, K, S, Epilogue{}, part, s);
       if (pieces == 2) return launch_quad_pieces<MODE, true, 2>(x, W, M, N, K, S, Epilogue{}, part, s);
       return launch_quad_partial_w<MODE, 8>(x, W, part, M, N, K, S, s);
     }
+    if (price.w == 4) return launch_quad_partial_w<MODE, 4>(x, W, part, M, N, K, S, s);
+    return launch_quad_partial_w<MODE, 2>(x, W, part, M, N, K, S, s);
   }
-  if (!is_bf<MODE> && M >= TQ_BM && tiles4 > num_cus()) return launch_quad_partial_w<MODE, 8>(x, W, part, M, N, K, S, s);
-  if (tiles2 > num_cus())
-    return launch_quad_partial_w<MODE, 4>(x, W, part, M, N, K, S, s);
+  if (tiles2 > num_cus()) return launch_quad_partial_w<MODE, 4>(x, W, part, M, N, K, S, s);
   launch_quad_partial_w<MODE, 2>(x, W, part, M, N, K, S, s);
+}
+
+// How a product of more than 64 row-major rows is taken: the forms of quad_price, 128 x 128 tiles (w = 0), and two ways
+// to take a ragged bottom of at most 128 rows: as one more, moved-up row of tiles, or (main < M) through the
+// streaming kernel, a sweep over the weights per 64 rows.
+struct TileChoice {
+  double us;
+  int w;
+  int64_t main;
+  QuadPlan even;
+};
+TileChoice tile_choice(int64_t M, int N, int K, int cus) {
+  const int64_t rows = (M + TQ_BM - 1) / TQ_BM, rem = M % TQ_BM;
+  const int64_t cols[3] = {(N + 255) / 256, (N + 127) / 128, (N + 63) / 64};
+  TileChoice best{quad_rounds_us(rows * cols[2], quad_tile_us(2, 8, K), cus), 2, M, QuadPlan{}};
+  auto offer = [&](double us, int w, int64_t m_main) {
+    if (us < best.us) best.us = us, best.w = w, best.main = m_main;
+  };
+  if (M > TQ_BM) {
+    const int64_t tiles = (M + 127) / 128 * cols[1];
+    // An odd number of 128 rows, the last of them nearly full (a 256-row tile would repeat its last row
+    // there, from the CU's own cache): 384 x 4096 x 16384 (96 tiles) 139 us against 133 on 256 x 64, 640
+    // 140 against 136, but 384 x 7168 x 28672 (168) 248 against 297; of more than a round bf16 352 x
+    // 50272 x 768 55 against 51 on 256 x 256, 384 x 50272 x 4096 197 against 186, 300 rows 173 against 184.
+    const bool full = rem >= 96 && rem <= 128;
+    const double more = !full ? 1.0 : K > 8192 && tiles * 8 <= cus * 5 ? 1.25 : 1.12;
+    offer(quad_rounds_us(tiles, quad_tile_us(4, 4, K), cus) * more, 0, M);
+  }
+  if (M >= TQ_BM) {
+    const QuadPrice p = quad_price(M, N, K, 1, cus);
+    best.even = p.even;
+    offer(p.us, p.w, M);
+  }
+  if (rem > 0 && rem <= 128 && M - rem >= TQ_BM) {
+    const double below = (double)((rem + 63) / 64) * ((double)N * K * 2 / 5e6 + 4);  // us of the streaming launches
+    offer(quad_rounds_us((rows - 1) * cols[1], quad_tile_us(4, 8, K), cus) + below, 4, M - rem);
+    offer(quad_cost((rows - 1) * cols[0], K, cus) + below, 8, M - rem);
+  }
+  return best;
 }
 
 // Slices for a product of M row-major rows whose tiles alone leave most of the chip idle (a
@@ -2301,12 +2472,17 @@ int pick_row_splits(int64_t M, int N, int K) {
 // 10240 over 1692 135 and 113, 2304 141 and 123.  A sum shorter than 16384 stops at three quarters of that half: 2048
 // x 8192 over 3072 rows (96 tiles) 120 and 109, 3328 122 and 116, 3584 125 and 122, 3840 128 and 129, 4096 135 and 133.
 // (The line is drawn for K = 8192; between it and 16384 two slices stay ahead past it: 9216 x 9216 over 768 rows, 108
-// tiles, 137 and 126, 2560 x 10240 over 3072, 120 tiles, 156 and 148.)
+// tiles, 137 and 126, 2560 x 10240 over 3072, 120 tiles, 156 and 148.)  Where one slice would fit as 256 x 128 or 128 x 128
+// tiles, two are taken if their price with what the second slice costs to write and read is the lower: 4096 x 16384, product
+// alone, 520 rows 104 and 79, 700 118 and 90, 1000 144 and 117; 2048 x 8192 over 1100 rows 59 and 44, 1500 67 and 48.
 int pick_row_splits_f16(int64_t M, int N, int K) {
   const int few = pick_row_splits(M, N, K);
   if (few > 1 || M < TQ_BM || N % 16 || K % 128 || K < 8192) return few;
   const int64_t rows = (M + TQ_BM - 1) / TQ_BM, tiles8 = rows * ((N + 255) / 256), tiles4 = rows * ((N + 127) / 128);
-  return tiles8 * 2 <= num_cus() * (K >= 16384 ? 4 : 3) / 4 && tiles4 * 2 > num_cus() ? 2 : 1;
+  if (tiles8 * 2 > num_cus() * (K >= 16384 ? 4 : 3) / 4) return 1;
+  if (tiles4 * 2 > num_cus()) return 2;
+  const double one = tile_choice(M, N, K, num_cus()).us, two = quad_price(M, N, K, 2, num_cus()).us;
+  return two + (double)M * N * 8 / 5e6 < 0.95 * one ? 2 : 1;
 }
 
 // The same for sums that leave as fp32 from any width of tile (bf16): also two slices of prompts' products whose
@@ -2323,9 +2499,13 @@ int pick_row_splits_f32(int64_t M, int N, int K) {
                 cols2 = (N + 63) / 64;
   if (K < 8192 && rows * cols2 * 4 < num_cus() * 3) return few;
   auto cost = [&](int S) {
-    const double narrow = fmin(quad_rounds(rows * cols4 * S) * TQ_COST_4, quad_rounds(rows * cols2 * S) * TQ_COST_2);
-    const double rounds = fmin(quad_cost(rows * cols8 * S), narrow);
-    return rounds * TQ_ROUND_US * K / S + (S - 1) * (double)M * N * 8 / 5e6;
+    // in rounds of 256 x 256 tiles (103 us of K = 4096), of which 256 x 128 ones take 0.61 and 256 x 64 0.43
+    auto full = [](int64_t tiles) { return (double)((tiles + num_cus() - 1) / num_cus()); };
+    const int64_t tiles = rows * cols8 * S;
+    const int pieces = quad_pieces(tiles, num_cus());
+    const double wide = pieces == 1 ? full(tiles) : (double)(tiles / num_cus()) + (pieces == 2 ? 0.61 : 0.36);
+    const double rounds = fmin(wide, fmin(full(rows * cols4 * S) * 0.61, full(rows * cols2 * S) * 0.43));
+    return rounds * 103.0 / 4096 * K / S + (S - 1) * (double)M * N * 8 / 5e6;
   };
   return rows * cols8 * 2 <= num_cus() && cost(2) < 0.95 * cost(1) ? 2 : 1;
 }
@@ -2352,54 +2532,23 @@ void launch_tiled(const void* x, const void* W, const void* scales, int64_t M, i
   const int64_t big_tiles = ((M + TB_BM - 1) / TB_BM) * ((N + TB_BN - 1) / TB_BN);
   if constexpr (!W8) {
     // Fewer rows than a tile, or hardly more: launch_few_rows where its tiles fill one round (three quarters of
-    // the CUs with 256 x 256, a quarter with 128 x 128 tiles).  Else four tiles, 256 x 256 (the last of
-    // them in pieces), 256 x 128, 256 x 64 and 128 x 128, and two ways to take a ragged bottom of at
-    // most 128 rows: as one more, moved-up row of tiles, or through the streaming kernel (one sweep
-    // over the weights per 64 rows).  The combinations are priced in rounds of workgroups and the
-    // cheapest is taken.  The 256 x 64 tiles also serve 65 .. 255 rows (they repeat the last row instead of
-    // moving up); where even they would fill less than an eighth of the chip the 128 x 128 kernel
-    // of eight waves runs.
+    // the CUs with 256 x 256 tiles).  Else the cheapest form of tile_choice; the 256 x 64 tiles also serve 65 .. 255
+    // rows (they repeat the last row instead of moving up).  The 128 x 128 kernel of eight waves is left with what is no
+    // multiple of 64 deep: a few tiles of the four-wave forms are ahead of it too (us: 100 x 768 x 768 17.0 and 10.1, 200
+    // x 1024 x 4096 60 and 28, 300 x 768 x 3072 58 and 22, 500 x 256 x 1024 20.5 and 11.2, 65 x 16 x 2048 29.8 and 18.5, 65
+    // x 128 x 128 8.0 and 7.6).
     if (K % 64 == 0 && K >= 128 && M > 64) {
-      const int64_t cus = num_cus(), rem = M % TQ_BM, rows = (M + TQ_BM - 1) / TQ_BM;
-      const int64_t cols[3] = {(N + 255) / 256, (N + 127) / 128, (N + 63) / 64};
+      const int64_t cus = num_cus(), cols[2] = {(N + 255) / 256, (N + 127) / 128};
       if (M < TQ_BM && cols[0] <= cus && cols[0] * 4 >= cus * 3)
         return launch_few_rows<MODE, 8, 8>(x, W, M, N, K, epi, s);
-      if (M > 128 && M <= TQ_BM && cols[1] * 2 <= cus && cols[1] * 8 >= cus &&
-          K >= (cols[1] * 8 <= cus * 3 ? 512 : 4096))
+      if (M > 128 && M <= TQ_BM && cols[1] * 2 <= cus && K >= (cols[1] * 8 <= cus * 3 ? 512 : 4096))
         return launch_few_rows<MODE, 4, 4>(x, W, M, N, K, epi, s);
-      if (rows * cols[2] * 8 >= cus) {
-        const double unit = TQ_ROUND_US * K;                  // us per round of 256 x 256 tiles
-        const double sweep = (double)N * K * 2 / 5e6 + 4;  // us per streaming launch
-        double best = (double)quad_rounds(rows * cols[2]) * TQ_COST_2 * unit;
-        int best_w = 2;
-        int64_t best_main = M;
-        auto offer = [&](double cost, int w, int64_t m_main) {
-          if (cost < best) best = cost, best_w = w, best_main = m_main;
-        };
-        if (M > TQ_BM) {
-          const int64_t tiles = (M + 127) / 128 * cols[1];
-          // An odd number of 128 rows, the last of them nearly full (a 256-row tile would repeat its last row
-          // there, from the CU's own cache): 384 x 4096 x 16384 (96 tiles) 139 us against 133 on 256 x 64, 640
-          // 140 against 136, but 384 x 7168 x 28672 (168) 248 against 297; of more than a round bf16 352 x
-          // 50272 x 768 55 against 51 on 256 x 256, 384 x 50272 x 4096 197 against 186, 300 rows 173 against 184.
-          const bool full = rem >= 96 && rem <= 128;
-          const double more = !full ? 1.0 : K > 8192 && tiles * 8 <= cus * 5 ? 1.25 : 1.12;
-          offer((double)quad_rounds(tiles) * TQ_COST_Q * more * unit, 3, M);
-        }
-        if (M >= TQ_BM) {
-          offer((double)quad_rounds(rows * cols[1]) * TQ_COST_4 * unit, 1, M);
-          offer(quad_cost(rows * cols[0]) * unit, 0, M);
-        }
-        if (rem > 0 && rem <= 128 && M - rem >= TQ_BM) {
-          const double below = (double)((rem + 63) / 64) * sweep;
-          offer((double)quad_rounds((rows - 1) * cols[1]) * TQ_COST_4 * unit + below, 1, M - rem);
-          offer(quad_cost((rows - 1) * cols[0]) * unit + below, 0, M - rem);
-        }
-        if (best_w == 0) return launch_quad<MODE, 8>(x, W, scales, M, best_main, N, K, epi, s);
-        if (best_w == 1) return launch_quad<MODE, 4>(x, W, scales, M, best_main, N, K, epi, s);
-        if (best_w == 2) return launch_quad<MODE, 2>(x, W, scales, M, best_main, N, K, epi, s);
-        return launch_few_rows<MODE, 4, 4>(x, W, M, N, K, epi, s);
-      }
+      const TileChoice c = tile_choice(M, N, K, (int)cus);
+      if (c.w == QUAD_EVEN) return launch_quad_plan<MODE, false>(x, W, M, N, K, 1, c.even, epi, nullptr, s);
+      if (c.w == 8) return launch_quad<MODE, 8>(x, W, scales, M, c.main, N, K, epi, s);
+      if (c.w == 4) return launch_quad<MODE, 4>(x, W, scales, M, c.main, N, K, epi, s);
+      if (c.w == 2) return launch_quad<MODE, 2>(x, W, scales, M, c.main, N, K, epi, s);
+      return launch_few_rows<MODE, 4, 4>(x, W, M, N, K, epi, s);
     }
   }
   if constexpr (!is_bf<MODE>) if (K % (2 * TB_BK) == 0 && big_tiles >= num_cus()) {

@@ -166,6 +166,12 @@ def test_linear_bf16_pieces(M, N):
     close(y32.cpu(), ref[:, n32:], 1e-5, "fp32 columns beside glu")
 
 
+@pytest.mark.parametrize("M,N", [(289, 6144), (387, 6144), (481, 8224), (577, 8224), (898, 8224), (1345, 8224), (2465, 8224)])
+def test_linear_bf16_rows_cut_evenly(M, N):
+    """Rows of tiles of 128 .. 256 rows in one launch, 128 and 256 columns wide, the last of them ragged."""
+    test_linear_bf16_pieces(M, N)
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 16, 32), (70, 80, 96), (200, 144, 128)])
 def test_linear_f32(M, N, K):
     lib = _capi.load_hybrid()
@@ -242,6 +248,12 @@ def test_linear_with_bias_activation_and_decays(M, N, K, dtype):
                 slow = z > 0.999
                 off = ((1 - y32.cpu().double()) - (1 - z)).abs()[slow]
                 assert off.numel() == 0 or float(off.max()) < 3e-7, what
+
+
+@pytest.mark.parametrize("M,N,K", [(385, 8208, 256), (577, 8208, 256), (1345, 8208, 128)])
+def test_linear_with_bias_rows_cut_evenly(M, N, K):
+    test_linear_with_bias_activation_and_decays(M, N, K, BF16)
+
 
 
 @pytest.mark.parametrize("dtype", [BF16, F32], ids=["bf16", "f32"])

@@ -499,6 +499,45 @@ def test_linear_f16_pieces(lib, M, N, K):
     assert bool(((y.float() - want).abs() <= bound).all())
 
 
+# rows cut evenly: tiles of 128 and of 256 columns, 160, 192, 224 and 256 rows high, alone and above lower ones, the
+# last of them ragged; all rows 128 high; panels of columns
+EVEN = [(289, 12288, 192), (352, 528, 192), (257, 12288, 192), (353, 12288, 128), (321, 12288, 192), (417, 12288, 128),
+        (385, 12288, 192), (449, 16400, 192), (257, 16400, 192), (385, 16400, 128), (545, 16400, 192), (481, 16400, 128),
+        (641, 16400, 128), (577, 16400, 128), (1569, 16400, 128), (1000, 768, 704)]
+
+
+@pytest.mark.parametrize("M,N,K", EVEN)
+def test_linear_f16_rows_cut_evenly(lib, M, N, K):
+    test_linear_f16_pieces(lib, M, N, K)
+
+
+@pytest.mark.parametrize("M,N", [(289, 6144), (387, 6144), (385, 8208), (577, 8208), (898, 8208), (1345, 8208), (2465, 8208)])
+def test_split_k_partials_of_rows_cut_evenly(lib, M, N):
+    K = 256
+    print("even partials", M, N, flush=True)
+    x, W = G(rnd(M, K, seed=M)), G(rnd(N, K, seed=N, std=0.05))
+    for S in (1, 2):
+        part = torch.full((S + 1, M, N), float("nan"), dtype=torch.float32, device=DEV)
+        ok(lib.msa_linear_partial_f16(P(x), P(pack_w(lib, W)), P(part), M, N, K, S, 0, None), lib)
+        torch.cuda.synchronize()
+        assert bool(torch.isnan(part[S]).all()), "wrote past the last slice"
+        for xs, ws, got in zip(x.float().chunk(S, 1), W.float().chunk(S, 1), part):
+            want = xs @ ws.t()
+            # a sum of K / S fp32 terms
+            assert float((got - want).abs().max()) <= 8 * 2.0 ** -24 * K ** 0.5 * float(want.abs().max())
+
+
+@pytest.mark.parametrize("M,H,K", [(385, 32, 256), (577, 43, 256), (1569, 43, 128)])
+def test_qkv_proj_rows_cut_evenly(lib, M, H, K):
+    test_qkv_proj_rows_into_cache_rows_and_positions_of_their_own(lib, M, H, K, False, False)
+
+
+# fewer tiles than an eighth of the chip
+@pytest.mark.parametrize("M,N,K", [(65, 16, 128), (128, 80, 192), (129, 48, 512), (200, 272, 704), (300, 128, 128)])
+def test_linear_f16_few_tiles(lib, M, N, K):
+    test_linear_f16_pieces(lib, M, N, K)
+
+
 # more than 64 columns of tiles, which are taken in panels of 16: full and partial 16 x 16 blocks, a last
 # panel of one column and of several, a ragged bottom and right edge
 @pytest.mark.parametrize("M,N", [(4096, 16640), (8400, 16400), (700, 20500 // 16 * 16), (4500, 20480), (256, 24592)])
