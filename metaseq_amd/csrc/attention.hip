@@ -13,12 +13,14 @@
 
 namespace {
 
+// (The first 14 words of a kernel's arguments are in registers when a wave starts; the others are a read of memory, some
+// 0.3 us in front of whatever waits for it.  Nothing up to the first keys and values needs more than those, the
+// mask's pointer least of all: `waves` is their number, 256 more where there is a mask.)
 template <int HD>
 __global__ void attention_kernel(const half_t* __restrict__ q, const half_t* __restrict__ Kc,
-                                 const half_t* __restrict__ Vc,
-                                 const uint8_t* __restrict__ key_pad_mask, int64_t mask_stride,
-                                 half_t* __restrict__ out, int H, int T, int S0, int S_cap,
-                                 int out_mb, const int32_t* __restrict__ len_dev) {
+                                 const half_t* __restrict__ Vc, const int32_t* __restrict__ len_dev, int H, int S0,
+                                 int S_cap, int T, int waves, int out_mb, half_t* __restrict__ out,
+                                 const uint8_t* __restrict__ key_pad_mask, int64_t mask_stride) {
   constexpr int LPR = HD / 8;    // lanes per key row (16 bytes each)
   constexpr int RPW = 64 / LPR;  // key rows per wave instruction
   extern __shared__ float smem[];
@@ -28,7 +30,7 @@ __global__ void attention_kernel(const half_t* __restrict__ q, const half_t* __r
 
   const int bh = blockIdx.x, t = blockIdx.y;
   const int b = bh / H, h = bh - b * H;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = waves & 255, threads = nw * 64;
   const int sub = lane % LPR, rsel = lane / LPR;
   if (len_dev) {  // per-row cache lengths kept on the device (ragged batches, graph replay)
     S0 = len_dev[b];
@@ -40,10 +42,10 @@ __global__ void attention_kernel(const half_t* __restrict__ q, const half_t* __r
 
   const half_t* kbase = Kc + (int64_t)bh * S_cap * HD + sub * 8;
   const half_t* vbase = Vc + (int64_t)bh * S_cap * HD + sub * 8;
-  const uint8_t* mrow = key_pad_mask ? key_pad_mask + (int64_t)b * mask_stride : nullptr;
 
-  const half8_t qv =
-      *reinterpret_cast<const half8_t*>(q + ((int64_t)b * T + t) * D + h * HD + sub * 8);
+  // (of one new position the row and the head are not needed yet: a division less in front of the first load)
+  const int64_t q_at = T == 1 ? (int64_t)bh * HD : ((int64_t)b * T + t) * D + h * HD;
+  const half8_t qv = *reinterpret_cast<const half8_t*>(q + q_at + sub * 8);
   float qf[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) qf[i] = (float)qv[i];
@@ -59,7 +61,7 @@ __global__ void attention_kernel(const half_t* __restrict__ q, const half_t* __r
 #pragma unroll
     for (int o = LPR / 2; o > 0; o >>= 1) d += __shfl_xor(d, o, MSA_WAVE);
     float s = round_h(d);
-    if (mrow && mrow[kk]) s = -INFINITY;
+    if (waves >= 256 && key_pad_mask[(int64_t)b * mask_stride + kk]) s = -INFINITY;
     if (sub == 0) sc[kk] = s;
     lmax = fmaxf(lmax, s);
   };
@@ -91,7 +93,7 @@ __global__ void attention_kernel(const half_t* __restrict__ q, const half_t* __r
       if (u + 1 < R || vkey0 + u * kstride < n_keys) score(kv[u], vkey0 + u * kstride);
     if (R > 3) request(vbase, vpre, rows);
   };
-  const int rows = (last + kstride) / kstride;  // of the lane group that has most
+  const int rows = (last + kstride) >> __builtin_ctz(kstride);  // of the lane group that has most (4 or 16 waves)
   int key = vkey0;
   static_assert(U == 8, "the cases below");
   if (rows < U) {
@@ -131,13 +133,13 @@ __global__ void attention_kernel(const half_t* __restrict__ q, const half_t* __r
 
   // ---- softmax in fp32, probabilities rounded to fp16 ----
   float lsum = 0.f;
-  for (int i = threadIdx.x; i < n_keys; i += blockDim.x) {
+  for (int i = threadIdx.x; i < n_keys; i += threads) {
     const float e = expf(sc[i] - m);
     sc[i] = e;
     lsum += e;
   }
   const float denom = block_sum(lsum, red);
-  for (int i = threadIdx.x; i < n_keys; i += blockDim.x) sc[i] = round_h(sc[i] / denom);
+  for (int i = threadIdx.x; i < n_keys; i += threads) sc[i] = round_h(sc[i] / denom);
   __syncthreads();
 
   // ---- weighted sum of V rows ----
@@ -192,7 +194,7 @@ __global__ void attention_kernel(const half_t* __restrict__ q, const half_t* __r
     for (int i = 0; i < 8; ++i) oacc[wave][sub * 8 + i] = acc[i];
   }
   __syncthreads();
-  for (int d = threadIdx.x; d < HD; d += blockDim.x) {
+  for (int d = threadIdx.x; d < HD; d += threads) {
     float s = 0.f;
     for (int w = 0; w < nw; ++w) s += oacc[w][d];
     if (out_mb > 0)  // packed activation layout of the decode GEMMs (T == 1: row = b)
@@ -458,15 +460,16 @@ extern "C" int msa_attention_f16(const void* q, const void* Kcache, const void* 
   const int threads = (T == 1 && BH < 512) ? 1024 : 256;
   const size_t lds = (size_t)(len_dev ? S_cap : S0 + T) * sizeof(float);
   const dim3 grid((unsigned)BH, (unsigned)T);
+  const int waves = threads / 64 + (key_pad_mask ? 256 : 0);
   hipStream_t s = (hipStream_t)stream;
   if (hd == 64)
     hipLaunchKernelGGL(attention_kernel<64>, grid, dim3(threads), lds, s, (const half_t*)q,
-                       (const half_t*)Kcache, (const half_t*)Vcache, key_pad_mask, mask_stride,
-                       (half_t*)out, H, T, S0, S_cap, out_mb, len_dev);
+                       (const half_t*)Kcache, (const half_t*)Vcache, len_dev, H, S0, S_cap, T, waves, out_mb,
+                       (half_t*)out, key_pad_mask, mask_stride);
   else
     hipLaunchKernelGGL(attention_kernel<128>, grid, dim3(threads), lds, s, (const half_t*)q,
-                       (const half_t*)Kcache, (const half_t*)Vcache, key_pad_mask, mask_stride,
-                       (half_t*)out, H, T, S0, S_cap, out_mb, len_dev);
+                       (const half_t*)Kcache, (const half_t*)Vcache, len_dev, H, S0, S_cap, T, waves, out_mb,
+                       (half_t*)out, key_pad_mask, mask_stride);
   MSA_CHECK_LAUNCH("msa_attention_f16");
   return MSA_OK;
 }

@@ -28,6 +28,7 @@ HEADERS = ["common.h", "gemm_kernels.h", "attention_tiles.h",
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17", "-Wall", "-Wno-unused-function",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    "-mllvm", "-amdgpu-kernarg-preload-count=16",
 ]
 
 

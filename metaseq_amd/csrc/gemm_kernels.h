@@ -384,12 +384,11 @@ constexpr int ST_RN = 4;  // tiles reduced across the waves per pass through LDS
 // group) outweigh the weights in cache-fill traffic, so the fp16 kernel lets twice as many
 // tiles share each fragment and buffers fewer K steps to stay inside the register file (the
 // int8 kernel, whose stage also holds the raw bytes of two K steps, would spill).
-template <int MB, bool W8, int MODE, bool XR = false, int KG = ST_KG,
-          int NT = (MB <= 2 || W8 ? ST_NT : 2 * ST_NT), int U = (MB <= 2 ? 4 : (NT > ST_NT ? 1 : 2)), int LN = 0>
-__global__ __launch_bounds__(KG * 64) void linear_stream_kernel(
-    const half_t* __restrict__ xp, const void* __restrict__ Wp, const half_t* __restrict__ scales,
-    float* __restrict__ part, int M, int N, int K, int tiles_per_wg, int ks_per_split,
-    Epilogue epi, int64_t m_off, LnTail ln = LnTail{}) {
+template <int MB, bool W8, int MODE, bool XR, int KG, int NT, int U, int LN>
+__device__ __forceinline__ void stream_tiles(const half_t* __restrict__ xp, const void* __restrict__ Wp,
+                                             const half_t* __restrict__ scales, float* __restrict__ part, int M, int N,
+                                             int K, int tiles_per_wg, int ks_per_split, const Epilogue& epi,
+                                             int64_t m_off, const LnTail& ln) {
   static_assert(LN == 0 || (MB == 1 && !XR && KG == LN_MAX_ROWS), "one wave per row");
   // U = K steps (32 wide) buffered per stage; an int8 block covers two steps
   constexpr int UA = W8 ? U / 2 : U;  // weight loads per stage and tile
@@ -610,6 +609,28 @@ __global__ __launch_bounds__(KG * 64) void linear_stream_kernel(
       }
     }
   }
+}
+
+template <int MB, bool W8, int MODE, bool XR = false, int KG = ST_KG,
+          int NT = (MB <= 2 || W8 ? ST_NT : 2 * ST_NT), int U = (MB <= 2 ? 4 : (NT > ST_NT ? 1 : 2))>
+__global__ __launch_bounds__(KG * 64) void linear_stream_kernel(
+    const half_t* __restrict__ xp, const void* __restrict__ Wp, const half_t* __restrict__ scales,
+    float* __restrict__ part, int M, int N, int K, int tiles_per_wg, int ks_per_split, Epilogue epi, int64_t m_off) {
+  stream_tiles<MB, W8, MODE, XR, KG, NT, U, 0>(xp, Wp, scales, part, M, N, K, tiles_per_wg, ks_per_split, epi, m_off,
+                                               LnTail{});
+}
+
+// LN slices' tail and the LayerNorm in front.  What the first loads need is in the first 14 words of the arguments, which
+// a wave finds in its registers (nk: N / 16 above 8 bits of K / 32; mt: tiles per workgroup above 8 bits of M).
+template <bool W8, int MODE, int NT, int LN>
+__global__ __launch_bounds__(ST_KG * 64) void linear_stream_ln_kernel(
+    const float* __restrict__ ln_part, const half_t* __restrict__ ln_x, const void* __restrict__ Wp,
+    const half_t* __restrict__ ln_bias, const half_t* __restrict__ gamma, const half_t* __restrict__ beta, uint32_t nk,
+    uint32_t mt, half_t* __restrict__ x_out, const half_t* __restrict__ scales, float eps, Epilogue epi) {
+  const int nks = nk & 255;
+  stream_tiles<1, W8, MODE, false, ST_KG, NT, 4, LN>(nullptr, Wp, scales, nullptr, mt & 255, (int)(nk >> 8) * 16, nks * 32,
+                                                     mt >> 8, W8 ? (nks + 1) & ~1 : nks, epi, 0,
+                                                     LnTail{ln_part, ln_bias, ln_x, x_out, gamma, beta, eps});
 }
 
 // ---- shared-activation stream kernel (33 .. 128 rows; vocabularies from one row on) ------------
@@ -1934,7 +1955,7 @@ void launch_stream_mb(const void* xp, const void* W, const void* scales, float* 
       auto kernel = tiles_per_wg == 1 ? linear_stream_kernel<MB, W8, MODE, false, ST_KG, 1, 4>
                                       : linear_stream_kernel<MB, W8, MODE, false, ST_KG, 2, 4>;
       hipLaunchKernelGGL(kernel, dim3(gx, S), dim3(ST_KG * 64), 0, s, (const half_t*)xp, W, (const half_t*)scales,
-                         part, M, N, K, tiles_per_wg, ks_per_split, epi, m_off, LnTail{});
+                         part, M, N, K, tiles_per_wg, ks_per_split, epi, m_off);
       return;
     }
   }
@@ -2105,14 +2126,16 @@ template <bool W8, int MODE, int S>
 bool launch_stream_ln(const LnTail& ln, const void* W, const void* scales, int M, int N, int K, const Epilogue& epi,
                       hipStream_t s) {
   const int ntiles = N / 16, tpw = (ntiles + num_cus() - 1) / num_cus(), gx = (ntiles + tpw - 1) / tpw;
-  const int nks = K / 32, per = W8 ? (nks + 1) & ~1 : nks, bytes = K * 32;
+  const int bytes = K * 32;
+  static_assert(LN_MAX_K / 32 < 256 && LN_MAX_ROWS < 256, "packed below");
 #define LN_RUN(NT)                                                                                            \
   do {                                                                                                        \
-    auto kernel = linear_stream_kernel<1, W8, MODE, false, ST_KG, NT, 4, S>;                                  \
+    auto kernel = linear_stream_ln_kernel<W8, MODE, NT, S>;                                                   \
     static std::atomic<uint64_t> allowed{0};                                                                  \
     if (!allow_lds((const void*)kernel, LN_MAX_K * 32, allowed)) return false;                                \
-    hipLaunchKernelGGL(kernel, dim3(gx), dim3(ST_KG * 64), bytes, s, (const half_t*)nullptr, W,               \
-                       (const half_t*)scales, (float*)nullptr, M, N, K, tpw, per, epi, (int64_t)0, ln);       \
+    hipLaunchKernelGGL(kernel, dim3(gx), dim3(ST_KG * 64), bytes, s, ln.part, ln.x, W, ln.bias, ln.gamma,     \
+                       ln.beta, (uint32_t)ntiles << 8 | K / 32, (uint32_t)tpw << 8 | M, ln.x_out,             \
+                       (const half_t*)scales, ln.eps, epi);                                                   \
   } while (0)
   if (tpw == 1) LN_RUN(1);
   else if (tpw == 2) LN_RUN(2);

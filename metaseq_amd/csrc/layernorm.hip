@@ -18,9 +18,9 @@ constexpr int LN_MAX_CHUNKS = 4;  // 8 halves per chunk per thread -> D <= 512*8
 // rows) narrow ones so that several rows share a compute unit.
 template <int ST, int THREADS = LN_THREADS>
 __global__ __launch_bounds__(THREADS) void layernorm_f16_kernel(
-    const half_t* x, const float* __restrict__ part, int S,
-    const half_t* __restrict__ bias, half_t* x_out, const half_t* __restrict__ gamma,
-    const half_t* __restrict__ beta, half_t* __restrict__ y, int M, int D, float eps, int out_mb) {
+    const half_t* x, const float* __restrict__ part, const half_t* __restrict__ bias,
+    const half_t* __restrict__ gamma, const half_t* __restrict__ beta, int M, int D, half_t* __restrict__ y, half_t* x_out,
+    int S, float eps, int out_mb) {
   __shared__ float red[16];
   const int row = blockIdx.x;
   const int nchunk = D >> 3;  // 16-byte chunks in the row
@@ -239,9 +239,8 @@ extern "C" int msa_layernorm_f16(const void* x, const void* gamma, const void* b
                 : threads == 256      ? layernorm_f16_kernel<0, 256>
                                       : layernorm_f16_kernel<0, 128>;
   hipLaunchKernelGGL(kernel, dim3((unsigned)rows), dim3(threads), 0, (hipStream_t)stream,
-                     (const half_t*)x, (const float*)nullptr, 0, (const half_t*)nullptr,
-                     (half_t*)nullptr, (const half_t*)gamma, (const half_t*)beta, (half_t*)y,
-                     (int)rows, D, eps, out_mb);
+                     (const half_t*)x, (const float*)nullptr, (const half_t*)nullptr, (const half_t*)gamma,
+                     (const half_t*)beta, (int)rows, D, (half_t*)y, (half_t*)nullptr, 0, eps, out_mb);
   MSA_CHECK_LAUNCH("msa_layernorm_f16");
   return MSA_OK;
 }
@@ -265,9 +264,8 @@ extern "C" int msa_residual_layernorm_f16(const float* part, int S, const void* 
                 : S == 8 ? layernorm_f16_kernel<8>
                          : layernorm_f16_kernel<0>;
   hipLaunchKernelGGL(kernel, dim3((unsigned)rows), dim3(LN_THREADS), 0, (hipStream_t)stream,
-                     (const half_t*)x, part, S, (const half_t*)bias, (half_t*)x,
-                     (const half_t*)gamma, (const half_t*)beta, (half_t*)y, (int)rows, D, eps,
-                     out_mb);
+                     (const half_t*)x, part, (const half_t*)bias, (const half_t*)gamma, (const half_t*)beta, (int)rows,
+                     D, (half_t*)y, (half_t*)x, S, eps, out_mb);
   MSA_CHECK_LAUNCH("msa_residual_layernorm_f16");
   return MSA_OK;
 }
