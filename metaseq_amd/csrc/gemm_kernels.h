@@ -184,11 +184,39 @@ __device__ __forceinline__ void select_merge(SelectState& a, float om, float os,
   a.nan |= onan;
 }
 
-// 4 consecutive output columns n..n+3 of row m
+// What the epilogue of columns n .. n + 3 of row m reads.  A kernel of a few us requests it with its first weights: behind
+// its last sum it is a round trip to memory with nothing beside it (qkv and fc1 of a decode step).
 template <int MODE>
-__device__ __forceinline__ void epilogue4(const Epilogue& e, int64_t m, int n, float4_t acc) {
+struct Ahead {
+  half4_t bias, res;
+  int at, row;  // MODE_QKV: position and row of the cache
+  PostVectors post;
+};
+template <int MODE>
+__device__ __forceinline__ Ahead<MODE> epilogue_ahead(const Epilogue& e, int64_t m, int n) {
+  Ahead<MODE> a{};
+  if constexpr (MODE == MODE_BF_POST) a.post = post_vectors(e, n);
+  if constexpr (is_bf<MODE>) return a;
+  if (e.bias) a.bias = *reinterpret_cast<const half4_t*>(e.bias + n);
+  if constexpr (MODE == MODE_PLAIN)
+    if (e.residual) a.res = *reinterpret_cast<const half4_t*>(e.residual + m * e.N + n);
+  if constexpr (MODE == MODE_QKV) {
+    const int mi = (int)m;
+    a.row = e.T == 1 ? mi : mi / e.T;
+    a.at = e.S0;
+    if (e.len_dev) {  // per-row lengths: T == 1, row = mi
+      a.at = e.len_dev[mi];
+      if (e.row_dev) a.row = e.row_dev[mi];
+    }
+  }
+  return a;
+}
+
+// 4 consecutive output columns n..n+3 of row m (GIVEN: what it reads is in `a`)
+template <int MODE, bool GIVEN = false>
+__device__ __forceinline__ void epilogue4(const Epilogue& e, int64_t m, int n, float4_t acc, const Ahead<MODE>& a = {}) {
   if constexpr (is_bf<MODE>) {
-    if constexpr (MODE == MODE_BF_POST) acc = post4(e, n, acc, post_vectors(e, n));
+    if constexpr (MODE == MODE_BF_POST) acc = post4(e, n, acc, GIVEN ? a.post : post_vectors(e, n));
     if (n >= e.n32) {
       *reinterpret_cast<float4_t*>(e.y32 + m * (e.N - e.n32) + (n - e.n32)) = acc;
     } else if constexpr (MODE != MODE_BF_GLU) {
@@ -214,7 +242,7 @@ __device__ __forceinline__ void epilogue4(const Epilogue& e, int64_t m, int n, f
 #pragma unroll
   for (int i = 0; i < 4; ++i) t[i] = round_h(acc[i]);
   if (e.bias) {
-    const half4_t b = *reinterpret_cast<const half4_t*>(e.bias + n);
+    const half4_t b = GIVEN ? a.bias : *reinterpret_cast<const half4_t*>(e.bias + n);
 #pragma unroll
     for (int i = 0; i < 4; ++i) t[i] = round_h(t[i] + (float)b[i]);
   }
@@ -224,7 +252,7 @@ __device__ __forceinline__ void epilogue4(const Epilogue& e, int64_t m, int n, f
       for (int i = 0; i < 4; ++i) t[i] = fmaxf(t[i], 0.f);
     }
     if (e.residual) {
-      const half4_t r = *reinterpret_cast<const half4_t*>(e.residual + m * e.N + n);
+      const half4_t r = GIVEN ? a.res : *reinterpret_cast<const half4_t*>(e.residual + m * e.N + n);
 #pragma unroll
       for (int i = 0; i < 4; ++i) t[i] = round_h(t[i] + (float)r[i]);
     }
@@ -251,8 +279,8 @@ __device__ __forceinline__ void epilogue4(const Epilogue& e, int64_t m, int n, f
       const int h = e.hd_shift >= 0 ? c >> e.hd_shift : c / e.hd, d = c - h * e.hd;
       const int mi = (int)m;
       const int b = e.T == 1 ? mi : mi / e.T, tt = mi - b * e.T;
-      int s0 = e.S0, row = b;
-      if (e.len_dev) {  // per-row lengths: T == 1, b = row
+      int s0 = GIVEN ? a.at : e.S0, row = GIVEN ? a.row : b;
+      if (!GIVEN && e.len_dev) {  // per-row lengths: T == 1, b = row
         s0 = e.len_dev[b];
         if (e.row_dev) row = e.row_dev[b];
       }
@@ -406,6 +434,14 @@ __device__ __forceinline__ void stream_tiles(const half_t* __restrict__ xp, cons
   const int ngroups = (tile_end - tile_begin + NT - 1) / NT;
   const int nstages = (ks_end - ks_begin + KG * U - 1) / (KG * U);
   const int total = ngroups * nstages;
+  // (a stage is followed, not found by division: 30 scalar instructions each time, in kernels of a few us)
+  struct At {
+    int grp, st, nstages;
+    __device__ void next() {
+      if (++st == nstages) st = 0, ++grp;
+    }
+    __device__ bool last() const { return st + 1 == nstages; }
+  };
 
   struct Stage {
     half8_t a[UA][NT];  // fp16: one A fragment; int8: 16 raw bytes = two A fragments
@@ -416,9 +452,8 @@ __device__ __forceinline__ void stream_tiles(const half_t* __restrict__ xp, cons
   // load inside a branch makes the compiler wait for every outstanding load before the MFMAs).
   // Steps and tiles past the end read a clamped, valid address: a surplus tile is dropped in
   // finish(), a surplus step gets its activation fragment zeroed in mma().
-  auto load = [&](Stage& s, int idx) {
-    const int grp = idx / nstages, st = idx - grp * nstages;
-    const int t0 = tile_begin + grp * NT;
+  auto load = [&](Stage& s, const At& at) {
+    const int st = at.st, t0 = tile_begin + at.grp * NT;
 #pragma unroll
     for (int u = 0; u < UA; ++u) {
       // first 32-wide step covered by this load (wave-uniform)
@@ -461,8 +496,8 @@ __device__ __forceinline__ void stream_tiles(const half_t* __restrict__ xp, cons
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) acc[j][mb] = float4_t{0.f, 0.f, 0.f, 0.f};
   };
-  auto mma = [&](Stage& s, int idx) {
-    const int grp = idx / nstages, st = idx - grp * nstages;
+  auto mma = [&](Stage& s, const At& at) {
+    const int grp = at.grp, st = at.st;
     half_t sc[NT];
     if (W8) {
       const int t0 = tile_begin + grp * NT;
@@ -507,8 +542,18 @@ __device__ __forceinline__ void stream_tiles(const half_t* __restrict__ xp, cons
         }
       }
   };
-  auto finish = [&](int idx) {  // after the last stage of a tile group
-    const int grp = idx / nstages;
+  // the epilogue's operands of the group that comes next, where a thread has one slot of it
+  constexpr bool AHEAD = MB <= 2 && !XR && MODE != MODE_SELECT;
+  static_assert(!AHEAD || (SEL_IT == 1 && NT == RN), "one slot");
+  constexpr int EMODE = MODE == MODE_SELECT ? MODE_PLAIN : MODE;
+  Ahead<EMODE> ahead{};
+  auto look_ahead = [&](int grp) {
+    if (!AHEAD || part) return;
+    const int jm = min((int)threadIdx.x >> 6, RN * MB - 1), jj = jm / MB, mb = jm - jj * MB;
+    ahead = epilogue_ahead<EMODE>(epi, min(mb * 16 + (lane & 15), M - 1),
+                                  min(tile_begin + grp * NT + jj, tile_end - 1) * 16 + ((lane >> 4) << 2));
+  };
+  auto finish = [&](int grp) {  // after the last stage of a tile group
     const int t0 = tile_begin + grp * NT;
 #pragma unroll
     for (int p = 0; p < NT / RN; ++p) {  // RN tiles per pass through the LDS buffer
@@ -534,43 +579,52 @@ __device__ __forceinline__ void stream_tiles(const half_t* __restrict__ xp, cons
             *reinterpret_cast<float4_t*>(part + ((int64_t)blockIdx.y * M + m) * N + n) = sum;
           else if (MODE == MODE_SELECT)
             select_update4(sel[it], epi, m, n, sum);
+          else if constexpr (AHEAD)
+            epilogue4<EMODE, true>(epi, m_off + m, n, sum, ahead);
           else
-            epilogue4<MODE == MODE_SELECT ? MODE_PLAIN : MODE>(epi, m_off + m, n, sum);
+            epilogue4<EMODE>(epi, m_off + m, n, sum);
         }
       }
       __syncthreads();
     }
     clear();
+    if (grp + 1 < ngroups) look_ahead(grp + 1);
   };
   clear();
+  At la{0, 0, nstages}, ma{0, 0, nstages};  // the stages loaded and multiplied next
   if constexpr (LN > 0) {
     // Requested in this order, the tail's operands arrive while the first weights are on their way.
     LnRow<LN> row;
     row.fetch(ln, min(wave, M - 1), M, K, lane);
-    load(s0, 0);
+    load(s0, la);
+    look_ahead(0);
     row.finish(ln, wave, M, K, lane, blockIdx.x == 0, ln_rows);
     __syncthreads();
   } else {
-    load(s0, 0);
+    load(s0, la);
+    look_ahead(0);
   }
+  auto take = [&](Stage& s) {
+    mma(s, ma);
+    if (ma.last()) finish(ma.grp);
+    ma.next();
+  };
   int idx = 0;
   for (; idx + 2 < total; idx += 2) {  // steady state: every load is of a real stage
-    load(s1, idx + 1);
-    mma(s0, idx);
-    if ((idx + 1) % nstages == 0) finish(idx);
-    load(s0, idx + 2);
-    mma(s1, idx + 1);
-    if ((idx + 2) % nstages == 0) finish(idx + 1);
+    la.next();
+    load(s1, la);
+    take(s0);
+    la.next();
+    load(s0, la);
+    take(s1);
   }
   if (idx + 1 < total) {  // two stages left
-    load(s1, idx + 1);
-    mma(s0, idx);
-    if ((idx + 1) % nstages == 0) finish(idx);
-    mma(s1, idx + 1);
-    finish(idx + 1);
+    la.next();
+    load(s1, la);
+    take(s0);
+    take(s1);
   } else {  // one stage left
-    mma(s0, idx);
-    finish(idx);
+    take(s0);
   }
   if (MODE == MODE_SELECT) {
     // The 16 threads that hold one row (4 lane groups x RN tile slots of one row block) merge
