@@ -196,7 +196,12 @@ __global__ void attention_kernel(const half_t* __restrict__ q, const half_t* __r
   __syncthreads();
   for (int d = threadIdx.x; d < HD; d += threads) {
     float s = 0.f;
-    for (int w = 0; w < nw; ++w) s += oacc[w][d];
+    if (nw == 16) {  // read together, added in turn
+#pragma unroll
+      for (int w = 0; w < 16; ++w) s += oacc[w][d];
+    } else {
+      for (int w = 0; w < nw; ++w) s += oacc[w][d];
+    }
     if (out_mb > 0)  // packed activation layout of the decode GEMMs (T == 1: row = b)
       out[packed_act_offset(b, h * HD + d, out_mb)] = (half_t)s;
     else
