@@ -106,6 +106,15 @@ __global__ __launch_bounds__(SM_THREADS) void greedy_select_kernel(
   if ((reinterpret_cast<uintptr_t>(row) & 15) == 0) {
     const int nv = V >> 3;
     constexpr int UNR = 4;  // chunks requested together: one memory round trip per UNR chunks
+    // Of a chunk that holds none of the ids that may not be chosen only the values are compared (a thread's ids ascend,
+    // so the first of equals stays).  200 rows of 50272 27.7 -> 18.3 us.
+    auto special = [&](int c) {
+      bool any = only_eos || (ban_early && (eos >> 3) == c);
+      for (int j = 0; j < banned.n; ++j) any |= (banned.id[j] >> 3) == c;
+      if (ban_early)
+        for (int j = 0; j < stop.n; ++j) any |= (stop.id[j] >> 3) == c;
+      return any;
+    };
     for (int c0 = threadIdx.x; c0 < nv; c0 += blockDim.x * UNR) {
       typedef typename Logits8<LT>::type lt8;
       lt8 vv[UNR];
@@ -122,7 +131,20 @@ __global__ __launch_bounds__(SM_THREADS) void greedy_select_kernel(
           z[i] = (float)vv[u][i];
           if (scale) z[i] = z[i] / temperature;
           cm = fmaxf(cm, z[i]);
-          visit((c << 3) + i, z[i]);
+          nan |= (z[i] != z[i]);
+        }
+        if (special(c)) {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) visit((c << 3) + i, z[i]);
+        } else {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            if (z[i] > best) {
+              best = z[i];
+              bidx = (c << 3) + i;
+            }
+          }
+          if (bidx == 0x7fffffff) bidx = c << 3;  // nothing but the lowest value so far
         }
         if (cm > m) {  // rescale once per 8 ids
           s *= __expf(m - cm);

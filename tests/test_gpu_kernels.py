@@ -121,6 +121,24 @@ def test_layernorm(lib, rows, D):
         assert torch.equal(unpack_act(yp.cpu(), rows, D), y.cpu())
 
 
+# workgroups of 128, 256 and 512 threads; two slices of many rows take 256 threads up to 6144 wide
+@pytest.mark.parametrize("rows,D,S", [(3, 1024, 4), (3, 1032, 1), (70, 2048, 8), (5, 2056, 2), (1025, 2056, 2), (1025, 4096, 2),
+                                      (1030, 6144, 2), (1025, 6152, 2), (1025, 4096, 3)])
+def test_residual_layernorm_of_slices(lib, rows, D, S):
+    print("tail", rows, D, S, flush=True)
+    part, x, b = torch.randn(S, rows, D, generator=torch.Generator().manual_seed(D)), rnd(rows, D, seed=1), rnd(D, seed=2)
+    g, be = (1 + rnd(D, seed=3, std=0.1).float()).half(), rnd(D, seed=4)
+    xd, y = G(x).clone(), torch.empty(rows, D, dtype=torch.float16, device=DEV)
+    ok(lib.msa_residual_layernorm_f16(P(G(part)), S, P(G(b)), P(xd), P(G(g)), P(G(be)), P(y), rows, D, 1e-5, 0, None), lib)
+    torch.cuda.synchronize()
+    total = part[0]
+    for p in part[1:]:
+        total = total + p
+    want = r16(r16(r16(total) + b.float()) + x.float())
+    assert torch.equal(xd.cpu(), want.half())
+    assert_fp16_close(y, O.layer_norm(want, g, be).half(), atol=2e-5, what="layernorm")
+
+
 def test_layernorm_rejects_bad_dim(lib):
     x = torch.zeros(4, 12, dtype=torch.float16, device=DEV)
     assert lib.msa_layernorm_f16(P(x), P(x), P(x), P(x), 4, 12, 1e-5, 0, None) == -1
@@ -497,6 +515,12 @@ def test_linear_f16_pieces(lib, M, N, K):
     # the bound of test_linear_f16_few_rows
     bound = 5 * size * 2.0 ** -11 + 8 * 2.0 ** -24 * K ** 0.5 * float(size.square().mean().sqrt()) + 2.0 ** -24
     assert bool(((y.float() - want).abs() <= bound).all())
+
+
+# a vocabulary of fewer rows than a tile: as high as the rows need
+@pytest.mark.parametrize("M", [66, 128, 129, 160, 161, 192, 193, 224, 225])
+def test_linear_f16_vocabulary_of_few_rows(lib, M):
+    test_linear_f16_pieces(lib, M, 50272, 192)
 
 
 # rows cut evenly: tiles of 128 and of 256 columns, 160, 192, 224 and 256 rows high, alone and above lower ones, the
@@ -1125,6 +1149,22 @@ def test_greedy_select_matches_reference_passes(lib, temperature):
     assert torch.equal(tok, want_t)
     assert torch.allclose(sc, want_s, atol=2e-5)
     assert tok[3] == 100
+
+
+def test_greedy_select_chunks_with_and_without_banned_ids(lib):
+    """Ties across chunks of eight, a best id that is banned, rows of nothing but the lowest value and of none to choose."""
+    V = 8192 * 2 + 40
+    logits = torch.full((6, V), -3.0, dtype=torch.float16)
+    logits[0, [16, 24, 9000]] = 5.0      # 16 is banned: the first of the others
+    logits[1, [8191, 8192, 16384]] = 2.0
+    logits[2] = float("-inf")
+    logits[3] = float("-inf")
+    logits[3, V - 1] = -7.0
+    logits[4, 17] = 9.0                  # in a chunk with banned ids
+    tok, sc = _select(lib, logits.to(DEV), 1.0, banned=[1, 16])
+    assert tok.tolist() == [24, 8191, 0, V - 1, 17, 0]
+    want = torch.log_softmax(logits.double(), -1)   # (in 32 bits 1e-4 off itself over 16424 ids)
+    assert torch.allclose(sc[[0, 1, 4, 5]].double(), want[[0, 1, 4, 5], tok[[0, 1, 4, 5]]], atol=2e-5)
 
 
 def test_greedy_select_finished_force_stop_nan(lib):
