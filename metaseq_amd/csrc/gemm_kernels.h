@@ -2436,8 +2436,9 @@ void launch_quad(const void* x, const void* W, const void* scales, int64_t M, in
 //   gained nothing: 200 x 4096 x 16384 49.8 -> 53.5.)  Of 129 .. 256 rows its longer fill of the rings is paid back from
 //   K = 512 on (200 x 4096: K = 256 7.0 -> 7.1 us, 512 9.0 -> 8.6), with more than 192 tiles from K = 4096 on (160 x
 //   16384: K = 2048 26.1 -> 27.1, 4096 47 -> 42).
-//   RF = 8: 256 x 256 tiles that repeat the last row, for outputs wide enough that one row of them fills
-//   the chip (the vocabulary): bf16 200 x 50272 x 4096 168 -> 101 us.
+//   WF = 8: 128 to 256 rows x 256 tiles that repeat the last row, for outputs wide enough that one row of them fills
+//   the chip (the vocabulary): bf16 200 x 50272 x 4096 168 -> 101 us.  As high as the rows need, fp16, against 256 rows: 66
+//   106 -> 86, 129 106 -> 89, 170 111 -> 95, 200 111 -> 101.
 template <int MODE, int WF, int RF>
 void launch_few_rows(const void* x, const void* W, int64_t M, int N, int K, const Epilogue& epi, hipStream_t s) {
   static std::atomic<uint64_t> lds_allowed_s{0};
@@ -2621,8 +2622,13 @@ void launch_tiled(const void* x, const void* W, const void* scales, int64_t M, i
     // x 128 x 128 8.0 and 7.6).
     if (K % 64 == 0 && K >= 128 && M > 64) {
       const int64_t cus = num_cus(), cols[2] = {(N + 255) / 256, (N + 127) / 128};
-      if (M < TQ_BM && cols[0] <= cus && cols[0] * 4 >= cus * 3)
+      if (M < TQ_BM && cols[0] <= cus && cols[0] * 4 >= cus * 3) {
+        if (M <= 128) return launch_few_rows<MODE, 8, 4>(x, W, M, N, K, epi, s);
+        if (M <= 160) return launch_few_rows<MODE, 8, 5>(x, W, M, N, K, epi, s);
+        if (M <= 192) return launch_few_rows<MODE, 8, 6>(x, W, M, N, K, epi, s);
+        if (M <= 224) return launch_few_rows<MODE, 8, 7>(x, W, M, N, K, epi, s);
         return launch_few_rows<MODE, 8, 8>(x, W, M, N, K, epi, s);
+      }
       if (M > 128 && M <= TQ_BM && cols[1] * 2 <= cus && K >= (cols[1] * 8 <= cus * 3 ? 512 : 4096))
         return launch_few_rows<MODE, 4, 4>(x, W, M, N, K, epi, s);
       const TileChoice c = tile_choice(M, N, K, (int)cus);
