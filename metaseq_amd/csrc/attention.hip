@@ -25,7 +25,7 @@ __global__ void attention_kernel(const half_t* __restrict__ q, const half_t* __r
   constexpr int RPW = 64 / LPR;  // key rows per wave instruction
   extern __shared__ float smem[];
   float* sc = smem;  // [n_keys] scores, then probabilities
-  __shared__ float red[16];
+  __shared__ __attribute__((aligned(16))) float red[16], red_sum[16];
   __shared__ float oacc[16][HD];
 
   const int bh = blockIdx.x, t = blockIdx.y;
@@ -129,7 +129,15 @@ __global__ void attention_kernel(const half_t* __restrict__ q, const half_t* __r
     // the first V rows are requested before the softmax so that HBM stays busy through it
     request(vbase, vpre, std::integral_constant<int, U>{});
   }
-  const float m = block_max(lmax, red);  // barriers inside also publish sc[]
+  // One barrier to a reduction (each has slots of its own), 4 or 16 waves; the first also publishes sc[].
+  const float wmax = wave_max(lmax);
+  if (lane == 0) red[wave] = wmax;
+  __syncthreads();
+  float m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  if (nw == 16) {
+#pragma unroll
+    for (int w = 4; w < 16; ++w) m = fmaxf(m, red[w]);
+  }
 
   // ---- softmax in fp32, probabilities rounded to fp16 ----
   float lsum = 0.f;
@@ -138,7 +146,14 @@ __global__ void attention_kernel(const half_t* __restrict__ q, const half_t* __r
     sc[i] = e;
     lsum += e;
   }
-  const float denom = block_sum(lsum, red);
+  const float wsum = wave_sum(lsum);
+  if (lane == 0) red_sum[wave] = wsum;
+  __syncthreads();
+  float denom = ((red_sum[0] + red_sum[1]) + red_sum[2]) + red_sum[3];
+  if (nw == 16) {
+#pragma unroll
+    for (int w = 4; w < 16; ++w) denom += red_sum[w];
+  }
   for (int i = threadIdx.x; i < n_keys; i += threads) sc[i] = round_h(sc[i] / denom);
   __syncthreads();
 

@@ -186,6 +186,26 @@ __device__ __forceinline__ float wave_sum(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
 }
 
+// several at once, step by step: their steps do not wait for one another
+template <int N>
+__device__ __forceinline__ void wave_sums(float (&v)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] += dpp_move<0xB1, 0xf>(0.f, v[i]);
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] += dpp_move<0x4E, 0xf>(0.f, v[i]);
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] += dpp_move<0x124, 0xf>(0.f, v[i]);
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] += dpp_move<0x128, 0xf>(0.f, v[i]);
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] += dpp_move<0x142, 0xa>(0.f, v[i]);
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] += dpp_move<0x143, 0xc>(0.f, v[i]);
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+    v[i] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v[i]), 63));
+}
+
 __device__ __forceinline__ float wave_max(float v) {
   v = fmaxf(v, dpp_move<0xB1, 0xf>(-INFINITY, v));
   v = fmaxf(v, dpp_move<0x4E, 0xf>(-INFINITY, v));

@@ -353,10 +353,12 @@ struct LnRow {
   __device__ __forceinline__ void finish(const LnTail& t, int row, int M, int K, int lane, bool store,
                                          half_t* rows) {
     const int chunks = K >> 3;
-    float total = 0.f;
+    // (the chunks' sums over the wave step by step together: one after the other each waits for itself)
+    float sums[C];
 #pragma unroll
     for (int c = 0; c < C; ++c) {
       float s = 0.f;
+      sums[c] = 0.f;
       if (c > 0 && c * 64 >= chunks) continue;
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
@@ -367,21 +369,29 @@ struct LnRow {
         x[c][i] = (half_t)(v + (float)x[c][i]);
         s += (float)x[c][i];
       }
-      total += wave_sum(c * 64 + lane < chunks ? s : 0.f);
+      sums[c] = c * 64 + lane < chunks ? s : 0.f;
     }
+    wave_sums(sums);
+    float total = 0.f;
+#pragma unroll
+    for (int c = 0; c < C; ++c) total += sums[c];
     const float mean = total / (float)K;
-    float var = 0.f;
 #pragma unroll
     for (int c = 0; c < C; ++c) {
       float q = 0.f;
+      sums[c] = 0.f;
       if (c > 0 && c * 64 >= chunks) continue;
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const float d = (float)x[c][i] - mean;
         q += d * d;
       }
-      var += wave_sum(c * 64 + lane < chunks ? q : 0.f);
+      sums[c] = c * 64 + lane < chunks ? q : 0.f;
     }
+    wave_sums(sums);
+    float var = 0.f;
+#pragma unroll
+    for (int c = 0; c < C; ++c) var += sums[c];
     const float rstd = rsqrtf(var / (float)K + t.eps);
     if (row >= M) return;  // uniform
 #pragma unroll
