@@ -234,6 +234,19 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
   return t;
 }
 
+// The same for blocks of NT threads, at the first use of `red` in a kernel: one barrier, and no more slots read than there are.
+template <int NT>
+__device__ __forceinline__ float block_sum_once(float v, float* red) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  v = wave_sum(v);
+  if (lane == 0) red[wave] = v;
+  __syncthreads();
+  float t = 0.f;
+#pragma unroll
+  for (int i = 0; i < NT / 64; ++i) t += red[i];
+  return t;
+}
+
 // two sums at once; `red` is >= 32 floats
 __device__ __forceinline__ void block_sum2(float& a, float& b, float* red) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;

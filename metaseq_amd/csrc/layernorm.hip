@@ -23,7 +23,7 @@ __global__ __launch_bounds__(THREADS) void layernorm_f16_kernel(
     const half_t* x, const float* __restrict__ part, const half_t* __restrict__ bias,
     const half_t* __restrict__ gamma, const half_t* __restrict__ beta, int M, int D, half_t* __restrict__ y, half_t* x_out,
     int S, float eps, int out_mb) {
-  __shared__ float red[16];
+  __shared__ float red[16], red2[16];
   const int row = blockIdx.x;
   const int nchunk = D >> 3;  // 16-byte chunks in the row
 
@@ -89,7 +89,7 @@ __global__ __launch_bounds__(THREADS) void layernorm_f16_kernel(
     }
   }
   if (!gamma) return;
-  const float mean = block_sum(s, red) / (float)D;
+  const float mean = block_sum_once<THREADS>(s, red) / (float)D;
   float q = 0.f;
 #pragma unroll
   for (int c = 0; c < LN_MAX_CHUNKS; ++c) {
@@ -102,7 +102,7 @@ __global__ __launch_bounds__(THREADS) void layernorm_f16_kernel(
       }
     }
   }
-  const float var = block_sum(q, red) / (float)D;
+  const float var = block_sum_once<THREADS>(q, red2) / (float)D;
   const float rstd = rsqrtf(var + eps);
 #pragma unroll
   for (int c = 0; c < LN_MAX_CHUNKS; ++c) {
