@@ -381,16 +381,20 @@ constexpr int GF_BM = 128, GF_BN = 64;
 template <int HD, int VD>
 constexpr int gf_lds_bytes = 2 * GF_BN * (HD * 2 + 16 + VD * 2 + 16);
 
-template <int HD, int VD>
-__global__ __launch_bounds__(256) void grouped_flash_kernel(msa_grouped_args a,
-                                                            const int32_t* __restrict__ seg_start,
-                                                            const int32_t* __restrict__ seg_slot,
-                                                            const int32_t* __restrict__ seg_pos,
-                                                            int seg0, float scale_log2, int n_qt) {
+// G = 2: two groups of four waves take every other key tile of the same queries, with tiles of their own in LDS, and
+// the second's sums are added to the first's at the end.  A tile is a chain of products, softmax and products
+// (some 2.2 us by itself) of which a SIMD with one wave hides nothing: where few workgroups share the chip the longest of
+// them is what counts.
+template <int HD, int VD, int G>
+__global__ __launch_bounds__(256 * G) void grouped_flash_kernel(msa_grouped_args a,
+                                                                const int32_t* __restrict__ seg_start,
+                                                                const int32_t* __restrict__ seg_slot,
+                                                                const int32_t* __restrict__ seg_pos,
+                                                                int seg0, float scale_log2, int n_qt) {
   constexpr int KSTEPS = HD / 16, DBLK = VD / 32, KP = HD * 2 + 16, VP = VD * 2 + 16;
   constexpr int KT = GF_BN * KP, TILE = KT + GF_BN * VP;
   constexpr int KCH = HD / 8, VCH = VD / 8, KLD = GF_BN * KCH / 256, VLD = GF_BN * VCH / 256;
-  extern __shared__ __attribute__((aligned(16))) char lds[];  // [2][K tile, V tile]
+  extern __shared__ __attribute__((aligned(16))) char all_lds[];  // [G][2][K tile, V tile]
   const int seg = seg0 + blockIdx.y, first = seg_start[seg], T = seg_start[seg + 1] - first;
   const int pos0 = seg_pos[seg];
   const int L = blockIdx.x, xcd = L & 7, seq = L >> 3;
@@ -407,8 +411,10 @@ __global__ __launch_bounds__(256) void grouped_flash_kernel(msa_grouped_args a,
   const int h = a.kv_heads % 8 == 0 ? ((hi / per) * 8 + xcd) * per + hi % per : hi * 8 + xcd;
   if (h >= a.heads) return;
   const int g = h / per;
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int tid = threadIdx.x & 255, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int group = G > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
+  char* lds = all_lds + group * 2 * TILE;
   const int j = lane & 31, hl = lane >> 5;
   const int q0 = qt * GF_BM + wave * 32;
   const int tq = q0 + j, tqc = min(tq, T - 1), pq = pos0 + tqc;
@@ -470,19 +476,21 @@ __global__ __launch_bounds__(256) void grouped_flash_kernel(msa_grouped_args a,
                             0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   // transposing read of V: key row 4 (lane / 32) + (lane % 16) / 4, columns 16 ((lane / 16) % 2) + 4 (lane % 4)
   const int vat = (4 * hl + ((lane & 15) >> 2)) * VP + ((lane >> 4) & 1) * 32 + (lane & 3) * 8;
-  fetch(0);
+  // (the group's tiles: group, group + G, ...; one past the last reads the last key and is not used)
+  const int rounds = (ntiles + G - 1) / G;
+  fetch(group);
   park(0);
-  if (ntiles > 1) fetch(1);
+  if (rounds > 1) fetch(group + G);
   lds_barrier();
-  for (int tile = 0; tile < ntiles; ++tile) {
-    const int buf = tile & 1;
+  for (int round = 0; round < rounds; ++round) {
+    const int buf = round & 1, tile = round * G + group;
     const char* kt = lds + buf * TILE;
     const char* vt = kt + KT;
-    if (tile + 1 < ntiles) park(buf ^ 1);
-    if (tile + 2 < ntiles) fetch(tile + 2);
+    if (round + 1 < rounds) park(buf ^ 1);
+    if (round + 2 < rounds) fetch(tile + 2 * G);
     const int kt0 = k_lo + tile * GF_BN;
     // wave-uniform: some query of this wave sees the tile
-    if (q0 < T && kt0 <= w_last && kt0 + GF_BN > any_lo) {
+    if (q0 < T && (G == 1 || tile < ntiles) && kt0 <= w_last && kt0 + GF_BN > any_lo) {
       float16_t s[2];
 #pragma unroll
       for (int ks = 0; ks < KSTEPS; ++ks)
@@ -540,6 +548,28 @@ __global__ __launch_bounds__(256) void grouped_flash_kernel(msa_grouped_args a,
       l += (t4[0] + t4[1]) + (t4[2] + t4[3]);
     }
     lds_barrier();
+  }
+  if constexpr (G == 2) {  // behind the last barrier no wave reads tiles
+    static_assert(4 * (DBLK * 16 + 2) * 64 * 4 <= G * 2 * TILE, "the second group's sums take the tiles' place");
+    float* sums = (float*)all_lds + wave * (DBLK * 16 + 2) * 64 + lane;
+    if (group == 1) {
+#pragma unroll
+      for (int d = 0; d < DBLK; ++d)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) sums[(d * 16 + v) * 64] = o[d][v];
+      sums[DBLK * 16 * 64] = mx;
+      sums[(DBLK * 16 + 1) * 64] = l;
+    }
+    lds_barrier();
+    if (group == 1) return;
+    const float mx1 = sums[DBLK * 16 * 64], mn = fmaxf(mx, mx1);
+    const float f0 = mx > -INFINITY ? __builtin_amdgcn_exp2f(mx - mn) : 0.f;
+    const float f1 = mx1 > -INFINITY ? __builtin_amdgcn_exp2f(mx1 - mn) : 0.f;
+    l = l * f0 + sums[(DBLK * 16 + 1) * 64] * f1;
+#pragma unroll
+    for (int d = 0; d < DBLK; ++d)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) o[d][v] = o[d][v] * f0 + sums[(d * 16 + v) * 64] * f1;
   }
   l += __shfl_xor(l, 32, MSA_WAVE);
   if (tq < T) {
@@ -640,6 +670,16 @@ bool run_decode(const msa_grouped_args& a, const msa_batch* b, int r0, int segs,
   return true;
 }
 
+template <int HD, int VD, int G>
+bool run_flash(const msa_grouped_args& a, const msa_batch* b, int seg0, int segs, int n_qt, hipStream_t s) {
+  static std::atomic<uint64_t> raised{0};
+  constexpr int bytes = G * gf_lds_bytes<HD, VD>;
+  if (!raise_lds((const void*)grouped_flash_kernel<HD, VD, G>, bytes, raised)) return false;
+  hipLaunchKernelGGL((grouped_flash_kernel<HD, VD, G>), dim3((unsigned)((a.heads + 7) / 8 * 8 * n_qt), segs),
+                     dim3(256 * G), bytes, s, a, b->seg_start, b->seg_slot, b->seg_pos, seg0, a.scale * LOG2E, n_qt);
+  return true;
+}
+
 template <int HD, int VD>
 bool run_tiles(const msa_grouped_args& a, const msa_batch* b, int r0, int seg0, int segs, int longest,
                hipStream_t s) {
@@ -651,14 +691,16 @@ bool run_tiles(const msa_grouped_args& a, const msa_batch* b, int r0, int seg0, 
       hipLaunchKernelGGL(grouped_combine_kernel, dim3((unsigned)(segs * a.heads)), dim3(64), 0, s, a, r0);
     return true;
   }
-  static std::atomic<uint64_t> raised{0};
-  constexpr int bytes = gf_lds_bytes<HD, VD>;
-  if (!raise_lds((const void*)grouped_flash_kernel<HD, VD>, bytes, raised)) return false;
   const int n_qt = (longest + GF_BM - 1) / GF_BM;
-  hipLaunchKernelGGL((grouped_flash_kernel<HD, VD>), dim3((unsigned)((a.heads + 7) / 8 * 8 * n_qt), segs),
-                     dim3(256), bytes, s, a, b->seg_start, b->seg_slot, b->seg_pos, seg0,
-                     a.scale * LOG2E, n_qt);
-  return true;
+  if constexpr (2 * gf_lds_bytes<HD, VD> <= 160 * 1024) {
+    // Two groups of waves where at most two workgroups share a CU, from 385 tokens on (32 heads of 128, 8 of keys, us: one segment
+    // of 300 tokens 13.6 and 12.6, 512 21.4 -> 17.7, 1000 36.7 -> 28.4, 1500 54.2 -> 38.9, 2048 75.6 -> 60.2).  More
+    // workgroups cover each other's chains, and there the LDS of two groups costs: 3000 tokens 112 and 122, 8 x 300 31 and
+    // 38, 8 x 1000 154 and 174.
+    const int64_t workgroups = (int64_t)a.heads * n_qt * segs;
+    if (longest > 384 && workgroups <= 512) return run_flash<HD, VD, 2>(a, b, seg0, segs, n_qt, s);
+  }
+  return run_flash<HD, VD, 1>(a, b, seg0, segs, n_qt, s);
 }
 
 template <int HD>
