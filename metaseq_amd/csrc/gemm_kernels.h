@@ -19,8 +19,9 @@
 //   * shared-activation stream (33 .. 128 packed rows; vocabularies of 16-bit weights and their
 //     selection from one row on): the same weight streaming, with the activation fragments staged
 //     once per workgroup in LDS and shared by its waves.
-//   * large tiled, fp16 weights (prefill-sized M): 256 x 256 per workgroup of four waves of
-//     128 x 128 with their accumulators in the AGPR bank, both operands global -> LDS directly.
+//   * large tiled, fp16 weights (from 65 row-major rows on): 256 x 256 per workgroup of four waves of
+//     128 x 128 with their accumulators in the AGPR bank, both operands global -> LDS directly; tiles of 128 to 256
+//     rows and of 64 to 256 columns where the rows are few or leave a round half empty.
 //   * large tiled, int8 weights: 256 x 256 x 64 per workgroup of eight waves, weights straight
 //     from the packed layout into registers (dequantised there), activations through LDS.
 //   * tiled (shapes in between): 128 x 128 x 32 LDS double-buffered tiles, 4 waves of 64 x 64,
@@ -1356,8 +1357,8 @@ __global__ __launch_bounds__(TB_THREADS) void linear_tiled_big_kernel(
 // MFMAs per step; the same activation stages).  The two wider forms need M >= 256: a ragged last
 // row tile is moved up to end at M and stores only the rows no other tile owns.  The narrowest
 // form repeats the last row in its loads instead and drops the rows past it, so it also serves
-// fewer than 256 rows, as does any form with FEW.  RF = 4 (16-row activation fragments per wave; else 8): tiles
-// of 128 rows, whose rings are five stages and eight steps deep.  All need K % 64 == 0, K >= 128.
+// fewer than 256 rows, as does any form with FEW.  RF = 4 .. 8 16-row activation fragments per wave: tiles of 32 RF
+// rows, whose rings are as deep as the LDS allows (128 x 128: five stages and eight steps).  All need K % 64 == 0, K >= 128.
 constexpr int TQ_BM = 256, TQ_THREADS = 256;  // (rows of a tile unless RF is given)
 constexpr int TQ_PANEL = 16;  // columns of tiles taken together where many lie across
 constexpr int tq_bm(int RF) { return 32 * RF; }
@@ -2658,13 +2659,13 @@ void launch_tiled(const void* x, const void* W, const void* scales, int64_t M, i
       return;
     }
   }
-  // the 256 x 256 kernel once it fills the chip; the 128 x 128 one for the shapes in between
+  // int8: the 256 x 256 kernel once it fills the chip; the 128 x 128 one for the shapes in between
   const int64_t big_tiles = ((M + TB_BM - 1) / TB_BM) * ((N + TB_BN - 1) / TB_BN);
   if constexpr (!W8) {
     // Fewer rows than a tile, or hardly more: launch_few_rows where its tiles fill one round (three quarters of
     // the CUs with 256 x 256 tiles).  Else the cheapest form of tile_choice; the 256 x 64 tiles also serve 65 .. 255
-    // rows (they repeat the last row instead of moving up).  The 128 x 128 kernel of eight waves is left with what is no
-    // multiple of 64 deep: a few tiles of the four-wave forms are ahead of it too (us: 100 x 768 x 768 17.0 and 10.1, 200
+    // rows (they repeat the last row instead of moving up).  linear_tiled_kernel is left with what is no
+    // multiple of 64 deep: a few tiles of the direct-to-LDS forms are ahead of it too (us: 100 x 768 x 768 17.0 and 10.1, 200
     // x 1024 x 4096 60 and 28, 300 x 768 x 3072 58 and 22, 500 x 256 x 1024 20.5 and 11.2, 65 x 16 x 2048 29.8 and 18.5, 65
     // x 128 x 128 8.0 and 7.6).
     if (K % 64 == 0 && K >= 128 && M > 64) {
@@ -2686,7 +2687,7 @@ void launch_tiled(const void* x, const void* W, const void* scales, int64_t M, i
       return launch_few_rows<MODE, 4, 4>(x, W, M, N, K, epi, s);
     }
   }
-  if constexpr (!is_bf<MODE>) if (K % (2 * TB_BK) == 0 && big_tiles >= num_cus()) {
+  if constexpr (W8) if (K % (2 * TB_BK) == 0 && big_tiles >= num_cus()) {
     static std::atomic<uint64_t> lds_allowed{0};  // one mask per instantiation
     if (!allow_lds((const void*)linear_tiled_big_kernel<W8, MODE>, TB_LDS_BYTES, lds_allowed))
       return;  // the launch check below reports the error
