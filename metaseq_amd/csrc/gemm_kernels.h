@@ -2380,8 +2380,9 @@ QuadPlan quad_plan(int64_t M, int N, int K, int S, int cus) {
     // (128 columns: 256-row tiles among lower ones are never the cheapest)
     for (int nrow = (units + wf / 4 + 5) / (wf / 4 + 6); nrow * 4 < units + 4; ++nrow) {
       const int rf = nrow * 4 < units ? (units + nrow - 1) / nrow : 5;  // (the last: all rows 128 high)
-      const int n_tall = nrow * 4 < units ? units - nrow * (rf - 1) : 0, slice = nrow * ncol, tiles = slice * S;
-      if (tiles > most) break;
+      const int n_tall = nrow * 4 < units ? units - nrow * (rf - 1) : 0;
+      if ((int64_t)nrow * ncol * S > most) break;
+      const int slice = nrow * ncol, tiles = slice * S;
       const double tall = quad_tile_us(wf, rf, K / S), low = quad_tile_us(wf, rf - 1, K / S);
       double us = 0;
       for (int t = 0; t < tiles && us < best.us; t += cus) {  // a round takes as long as its tallest tile
