@@ -216,6 +216,8 @@ int msa_grouped_rotate(const msa_grouped_args* a, const msa_batch* b, void* stre
 /* appends the keys and values of every segment's last chunk (nothing where msa_grouped_rotate did) */
 int msa_grouped_append(const msa_grouped_args* a, const msa_batch* b, void* stream);
 int msa_grouped_attention_splits(const msa_grouped_args* a, int M, int key_bound);
+/* how many groups of waves of a workgroup share the keys of a prompt's queries (1 or 2) in the call of the same arguments */
+int msa_grouped_attention_groups(const msa_grouped_args* a, const msa_batch* b, int seg0, int seg1, int longest);
 /* whether msa_grouped_attention can take rotation and appending over for this batch: with `fused` set, the
  * other two calls fall away */
 int msa_grouped_fuses(const msa_grouped_args* a, const msa_batch* b);

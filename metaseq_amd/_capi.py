@@ -210,6 +210,7 @@ HYBRID_SIGNATURES = {
     "msa_grouped_rotate": [ctypes.POINTER(GroupedArgs), _BP, _P],
     "msa_grouped_append": [ctypes.POINTER(GroupedArgs), _BP, _P],
     "msa_grouped_attention_splits": [ctypes.POINTER(GroupedArgs), c_int, c_int],
+    "msa_grouped_attention_groups": [ctypes.POINTER(GroupedArgs), _BP, c_int, c_int, c_int],
     "msa_grouped_fuses": [ctypes.POINTER(GroupedArgs), _BP],
     "msa_grouped_attention": [ctypes.POINTER(GroupedArgs), _BP, c_int, c_int, c_int, _P],
     "msa_latent_norm": [c_int, _P, c_int, c_int, c_int, c_int, c_int, _P, c_int, c_int, _P,

@@ -378,8 +378,9 @@ __global__ __launch_bounds__(64) void grouped_combine_kernel(msa_grouped_args a,
 
 // ---- several new tokens per sequence, bf16 ------------------------------------------------------
 constexpr int GF_BM = 128, GF_BN = 64;
+constexpr int gf_lds(int hd, int vd) { return 2 * GF_BN * (hd * 2 + 16 + vd * 2 + 16); }
 template <int HD, int VD>
-constexpr int gf_lds_bytes = 2 * GF_BN * (HD * 2 + 16 + VD * 2 + 16);
+constexpr int gf_lds_bytes = gf_lds(HD, VD);
 
 // G = 2: two groups of four waves take every other key tile of the same queries, with tiles of their own in LDS, and
 // the second's sums are added to the first's at the end.  A tile is a chain of products, softmax and products
@@ -670,6 +671,34 @@ bool run_decode(const msa_grouped_args& a, const msa_batch* b, int r0, int segs,
   return true;
 }
 
+// Groups of waves that share the key tiles of a tile of queries: two where a workgroup has a long list of key tiles and few
+// workgroups lie beside it, from 385 tokens on.  32 heads of 128, 8 of keys, one group and two, us: one segment of 512 tokens
+// 21.4 and 17.7, 1000 36.7 and 28.4, 2048 75.6 and 60.2.  More than two workgroups to a CU cover each other's
+// chains, and there the LDS of two groups costs: 3000 tokens 112 and 122, 8 x 300 31 and 38, 8 x 1000 154 and 174.
+// The list is what a tile of 128 queries sees, a chunk at most.  Heads whose two groups leave room for no second workgroup
+// on a CU need eight key tiles to be ahead past a workgroup per CU: 64 heads of 128 in chunks of 64, 640 tokens 13.1 and
+// 18.7; 32 in chunks of 256, 2000 tokens 20.3 and 25.3; 64, 2 x 400 tokens (seven tiles) 23.8 and 26.5, 500 and 60 (eight) 20.9
+// and 18.4, 640 in one chunk 21.1 and 18.0; 64 heads of 64 9.3 and 8.8, 13.1 and 13.3, 15.4 and 15.1, 14.2 and 12.2.  Up to a
+// workgroup per CU two groups are ahead from four tiles on (chunks of 256, 400 tokens 13.1 and 12.3), with three (chunks of 64
+// that the tiles of queries do not begin with) heads of 64 8.8 and 8.7, of 128 12.0 and 12.5, with two 7.3 and 6.8, 9.9
+// and 9.5, values of 192 10.4 and 10.5.
+constexpr int GF_MOST_LDS = 160 * 1024;
+int wave_groups(const msa_grouped_args& a, const msa_batch* b, int seg0, int seg1, int longest) {
+  if (longest <= 384) return 1;
+  const int wide = a.chunk > GF_BM ? a.chunk : GF_BM, step = a.chunk < GF_BM ? a.chunk : GF_BM;
+  bool aligned = a.chunk > 0 && wide % step == 0 && b->host_pos;  // query tiles begin with a chunk, or as many after one
+  int64_t workgroups = 0;                                         // that have queries
+  for (int i = seg0; i < seg1; ++i) {
+    if (b->host_pos && b->host_pos[i] < 0) continue;
+    if (aligned) aligned = b->host_pos[i] % step == 0;
+    workgroups += (int64_t)a.heads * ((b->host_start[i + 1] - b->host_start[i] + GF_BM - 1) / GF_BM);
+  }
+  const int64_t seen = a.chunk > 0 ? (int64_t)wide + (aligned ? 0 : step - 1) : longest;
+  const int tiles = (int)(((seen < longest ? seen : longest) + GF_BN - 1) / GF_BN);
+  if (tiles < 4 && (tiles == 2 ? a.vd > 128 : a.hd + a.vd > 192)) return 1;
+  return workgroups <= (tiles >= 8 || 4 * gf_lds(a.hd, a.vd) <= GF_MOST_LDS ? 512 : 256) ? 2 : 1;
+}
+
 template <int HD, int VD, int G>
 bool run_flash(const msa_grouped_args& a, const msa_batch* b, int seg0, int segs, int n_qt, hipStream_t s) {
   static std::atomic<uint64_t> raised{0};
@@ -692,13 +721,8 @@ bool run_tiles(const msa_grouped_args& a, const msa_batch* b, int r0, int seg0, 
     return true;
   }
   const int n_qt = (longest + GF_BM - 1) / GF_BM;
-  if constexpr (2 * gf_lds_bytes<HD, VD> <= 160 * 1024) {
-    // Two groups of waves where at most two workgroups share a CU, from 385 tokens on (32 heads of 128, 8 of keys, us: one segment
-    // of 300 tokens 13.6 and 12.6, 512 21.4 -> 17.7, 1000 36.7 -> 28.4, 1500 54.2 -> 38.9, 2048 75.6 -> 60.2).  More
-    // workgroups cover each other's chains, and there the LDS of two groups costs: 3000 tokens 112 and 122, 8 x 300 31 and
-    // 38, 8 x 1000 154 and 174.
-    const int64_t workgroups = (int64_t)a.heads * n_qt * segs;
-    if (longest > 384 && workgroups <= 512) return run_flash<HD, VD, 2>(a, b, seg0, segs, n_qt, s);
+  if constexpr (2 * gf_lds_bytes<HD, VD> <= GF_MOST_LDS) {
+    if (wave_groups(a, b, seg0, seg0 + segs, longest) == 2) return run_flash<HD, VD, 2>(a, b, seg0, segs, n_qt, s);
   }
   return run_flash<HD, VD, 1>(a, b, seg0, segs, n_qt, s);
 }
@@ -779,6 +803,14 @@ extern "C" int msa_grouped_attention_splits(const msa_grouped_args* a, int M, in
   // up to a workgroup per CU, at least 128 keys (a tile per wave) each
   while (s < 64 && groups * s * 2 <= 256 && (int64_t)keys >= 256 * s) s *= 2;
   return s;
+}
+
+extern "C" int msa_grouped_attention_groups(const msa_grouped_args* a, const msa_batch* b, int seg0, int seg1,
+                                            int longest) {
+  if (!a || !b || !b->host_start || !has_tiles(*a) || longest < 2 ||
+      2 * gf_lds(a->hd, a->vd) > GF_MOST_LDS)
+    return 1;
+  return wave_groups(*a, b, seg0, seg1, longest);
 }
 
 extern "C" int msa_grouped_fuses(const msa_grouped_args* a, const msa_batch* b) {

@@ -642,20 +642,23 @@ def test_grouped_prompts_of_more_than_1024_workgroups(kv_heads, chunk):
 @pytest.mark.parametrize("heads,kv_heads,hd,chunk,segs", [
     (4, 2, 64, 0, [(0, 0, 385)]), (8, 8, 128, 0, [(0, 0, 449)]), (3, 1, 128, 0, [(1, 37, 600), (0, 0, 130)]),
     (2, 1, 64, 300, [(0, 50, 700)]), (4, 1, 128, 0, [(0, 0, 385), (1, -1, 20), (2, 5, 512)]), (2, 2, 192, 0, [(0, 0, 400)])])
-def test_grouped_prompts_of_few_workgroups(heads, kv_heads, hd, chunk, segs):
+def test_grouped_prompts_of_few_workgroups(heads, kv_heads, hd, chunk, segs, vd=None, groups=None):
     lib = _capi.load_hybrid()
-    print("grouped", heads, kv_heads, hd, chunk, segs, flush=True)
+    vd = vd or hd
+    print("grouped", heads, kv_heads, hd, vd, chunk, segs, flush=True)
     rows, g, scale = 800, gen(hd), 0.15
-    M, D = sum(n for _, _, n in segs), (heads + 2 * kv_heads) * hd
+    M, D = sum(n for _, _, n in segs), heads * hd + kv_heads * (hd + vd)
     b, alive = _batch(segs, M)
     x = torch.randn(M, D, generator=g).to(BF16)
-    kc, vc = (torch.randn(len(segs), kv_heads, rows, hd, generator=g).to(BF16) for _ in range(2))
-    xd, kd, vd = x.cuda(), kc.cuda(), vc.cuda()
-    out = torch.full((M, heads * hd), 7.0, dtype=BF16, device="cuda")
+    kc, vc = (torch.randn(len(segs), kv_heads, rows, n, generator=g).to(BF16) for n in (hd, vd))
+    xd, kcd, vcd = x.cuda(), kc.cuda(), vc.cuda()
+    out = torch.full((M, heads * vd), 7.0, dtype=BF16, device="cuda")
     a = _capi.GroupedArgs()
-    a.dtype, a.heads, a.kv_heads, a.hd, a.vd, a.chunk, a.rows, a.scale, a.splits = 0, heads, kv_heads, hd, hd, chunk, rows, scale, 1
+    a.dtype, a.heads, a.kv_heads, a.hd, a.vd, a.chunk, a.rows, a.scale, a.splits = 0, heads, kv_heads, hd, vd, chunk, rows, scale, 1
     a.q, a.k, a.v, a.ld = ptr(xd), ptr(xd[:, heads * hd:]), ptr(xd[:, (heads + kv_heads) * hd:]), D
-    a.k_cache, a.v_cache, a.out, a.ldo = ptr(kd), ptr(vd), ptr(out), heads * hd
+    a.k_cache, a.v_cache, a.out, a.ldo = ptr(kcd), ptr(vcd), ptr(out), heads * vd
+    if groups:
+        assert lib.msa_grouped_attention_groups(ctypes.byref(a), ctypes.byref(b), 0, len(segs), b.max_count) == groups
     check(lib.msa_grouped_attention(ctypes.byref(a), ctypes.byref(b), 0, len(segs), max(n for _, _, n in segs),
                                     _capi.stream_ptr()), lib)
     torch.cuda.synchronize()
@@ -667,17 +670,26 @@ def test_grouped_prompts_of_few_workgroups(heads, kv_heads, hd, chunk, segs):
             assert bool((got == 7.0).all())
             continue
         start = pos // chunk * chunk if chunk else 0      # the cache holds the chunk that the first token is in
-        new = mine.view(n, -1, hd)
-        q, k, v = new[:, :heads], new[:, heads:heads + kv_heads], new[:, heads + kv_heads:]
+        q, k = mine[:, :(heads + kv_heads) * hd].view(n, -1, hd).split([heads, kv_heads], 1)
+        v = mine[:, (heads + kv_heads) * hd:].view(n, -1, vd)
         k = torch.cat([kc[slot, :, :pos - start].double().transpose(0, 1), k]).repeat_interleave(heads // kv_heads, 1)
         v = torch.cat([vc[slot, :, :pos - start].double().transpose(0, 1), v]).repeat_interleave(heads // kv_heads, 1)
         at, key = torch.arange(pos, pos + n)[:, None], torch.arange(start, pos + n)[None]
         seen = (key <= at) & (key >= (at // chunk * chunk if chunk else 0))
         s = (torch.einsum("qhd,khd->hqk", q, k) * scale).masked_fill(~seen, float("-inf"))
-        want = torch.einsum("hqk,khd->qhd", torch.softmax(s, -1), v).reshape(n, heads * hd)
+        want = torch.einsum("hqk,khd->qhd", torch.softmax(s, -1), v).reshape(n, heads * vd)
         # probabilities rounded to bf16 (2^-9 each, of either sign) and one rounding of the result
         assert float((got - want).norm() / want.norm()) < 2.0 ** -8
     del alive
+
+
+# values of another size than the keys; chunks that leave a tile of queries two, three and more key tiles, with both forms
+@pytest.mark.parametrize("heads,kv_heads,hd,vd,chunk,segs,groups", [
+    (4, 1, 64, 128, 0, [(0, 0, 500)], 2), (2, 2, 128, 64, 0, [(0, 20, 450)], 2), (2, 1, 192, 64, 0, [(0, 0, 385)], 2),
+    (2, 1, 64, 192, 0, [(0, 0, 400), (1, 0, 90)], 2), (2, 2, 64, 64, 64, [(0, 0, 400)], 2), (4, 2, 64, 128, 48, [(0, 100, 400)], 2),
+    (4, 2, 128, 128, 64, [(0, 30, 400)], 1), (4, 2, 128, 128, 64, [(0, 64, 400)], 2), (4, 2, 128, 128, 256, [(0, 200, 400)], 2), (64, 8, 128, 64, 64, [(0, 0, 640)], 1)])
+def test_grouped_prompts_of_chunks_and_value_sizes(heads, kv_heads, hd, vd, chunk, segs, groups):
+    test_grouped_prompts_of_few_workgroups(heads, kv_heads, hd, chunk, segs, vd, groups)
 
 
 def test_gathered_latents():

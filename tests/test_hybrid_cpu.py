@@ -375,6 +375,28 @@ def test_arguments_are_checked_before_anything_is_launched():
 
 
 # ---------------------------------------------------------------- oracle pins
+# two groups of waves: long lists of keys and few workgroups; not where a chunk cuts the lists short under many workgroups, and
+# segments count as they are, not as the longest
+@pytest.mark.parametrize("heads,hd,vd,chunk,segs,groups", [
+    (32, 128, 128, 0, [(0, 384)], 1), (32, 128, 128, 0, [(0, 385)], 2), (32, 128, 128, 0, [(0, 2048)], 2),
+    (32, 128, 128, 0, [(0, 2049)], 1), (64, 128, 128, 64, [(0, 640)], 1), (64, 64, 128, 256, [(0, 640)], 1),
+    (32, 128, 64, 256, [(0, 2000)], 1), (32, 128, 128, 256, [(0, 1000)], 2), (64, 128, 128, 1024, [(0, 640)], 2),
+    (64, 128, 128, 0, [(0, 400), (0, 400)], 1), (64, 64, 64, 64, [(0, 640)], 2), (16, 64, 128, 64, [(0, 640)], 2),
+    (16, 128, 128, 64, [(0, 640)], 2), (16, 128, 128, 64, [(30, 640)], 1), (16, 64, 64, 64, [(30, 640)], 2),
+    (16, 64, 192, 64, [(0, 640)], 1), (16, 128, 128, 48, [(0, 640)], 1), (32, 64, 192, 0, [(0, 640)], 2),
+    (32, 192, 192, 0, [(0, 640)], 1), (32, 128, 128, 0, [(0, 1000)] + [(0, 20)] * 7, 2),
+    (32, 128, 128, 0, [(0, 2000), (-1, 1000)], 2), (32, 128, 128, 0, [(0, 1100), (0, 1000)], 1)])
+def test_groups_of_waves_follow_the_keys_that_are_seen(heads, hd, vd, chunk, segs, groups):
+    lib = _capi.load_hybrid()
+    a, b = _capi.GroupedArgs(), _capi.Batch()
+    a.dtype, a.heads, a.kv_heads, a.hd, a.vd, a.chunk = 0, heads, heads // 4, hd, vd, chunk
+    starts = [sum(n for _, n in segs[:i]) for i in range(len(segs) + 1)]
+    b.M, b.nseg, b.max_count = starts[-1], len(segs), max(n for _, n in segs)
+    b.host_start = (ctypes.c_int32 * len(starts))(*starts)
+    b.host_pos = (ctypes.c_int32 * len(segs))(*[p for p, _ in segs])
+    assert lib.msa_grouped_attention_groups(ctypes.byref(a), ctypes.byref(b), 0, len(segs), b.max_count) == groups
+
+
 def test_oracle_convolution_by_hand():
     x = torch.tensor([[1.0], [2.0], [3.0]])
     w = torch.tensor([[10.0, 100.0]])     # previous, current
