@@ -1385,7 +1385,11 @@ __device__ __forceinline__ void tq_mfma(float4_t& acc, const half8_t& a, const h
 // forth.  What an MFMA draws depends on the operands of the one before it, and the part lowers its clock by that:
 // MFMAs alone, random operands, 1.91 PFLOP/s row by row, 1.96 so (one operand new each time, a snake of rows, 1.93;
 // both new 1.84; four rows side by side 1.90).  32768 x 16384 x 4096 3118 -> 3075 us, 2048 x 16384 x 4096 206 -> 200.
+// Not of 64 columns: those tiles draw less, and a step of 16 MFMAs waits for two rows of fragments in front of its first
+// pair (row by row and so, us: bf16 147 x 416 x 7104 50.2 and 54.1, 182 x 288 x 2944 14.2 and 14.8, fp16 83 x 7168 x 28672 in two
+// slices 133 and 137).
 constexpr int tq_order(int RF, int WF, int q) {
+  if (WF == 2) return q;
   const int g = q / (2 * WF), w = q % (2 * WF);
   if (2 * g + 1 >= RF) return 2 * g * WF + (g & 1 ? WF - 1 - w : w);
   const int c = w / 2;
