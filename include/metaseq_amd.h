@@ -193,6 +193,24 @@ int msa_linear_default_splits(int64_t M, int N, int K);
 int msa_linear_default_splits_w8a16(int64_t M, int N, int K);
 int msa_linear_default_splits_rows(int64_t M, int N, int K);
 
+/* The tiles that a product of M row-major rows and 16-bit weights (fp16 and bf16 alike) is cut into on a device of `cus`
+ * compute units (0: the current one): a whole product (S = 0), or S sums of msa_linear_partial_f16 / _bf16. */
+enum {
+  MSA_TILES_NONE = 0,   /* sweeps over the weights, 64 rows at a time */
+  MSA_TILES_WHOLE = 1,  /* 256 rows to a tile, a ragged last one (256 columns and 128) moved up */
+  MSA_TILES_FEW = 2,    /* tiles that repeat the last row: fewer rows than a tile, or tiles of 128 x 128 */
+  MSA_TILES_EVEN = 3,   /* the first n_tall rows of tiles are `rows` high, the others 32 less */
+  MSA_TILES_SIMPLE = 4  /* 128 x 128, K no multiple of 64 */
+};
+typedef struct {
+  int kind, rows, columns; /* rows and columns of a tile */
+  int n_rows, n_tall;      /* rows of tiles, and (MSA_TILES_EVEN) the taller ones among them */
+  int pieces;              /* 2 or 4: the tiles that would begin a round without half filling it are cut into as many */
+  int panels;              /* whether sixteen columns of tiles are taken at a time */
+  int64_t main;            /* rows taken in tiles; the rest as MSA_TILES_NONE */
+} msa_tile_form;
+int msa_linear_tiles(int64_t M, int N, int K, int S, int cus, msa_tile_form* out);
+
 /* Fused QKV projection: kvq = round(round(x . Wqkv^T) + bqkv) with rows of Wqkv ordered
  * K | V | Q; then for row m = b*T + t and head h:
  *   Kcache[b,h,S0+t,:] = k,  Vcache[b,h,S0+t,:] = v,  q_out[m, h*hd:(h+1)*hd] = round(q * hd^-0.5).

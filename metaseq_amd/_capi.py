@@ -55,6 +55,13 @@ class StepArgs(ctypes.Structure):
                 ("col_dev", c_void_p)]
 
 
+class TileForm(ctypes.Structure):
+    """msa_tile_form"""
+    _fields_ = [(n, c_int) for n in ("kind", "rows", "columns", "n_rows", "n_tall", "pieces", "panels")] + [("main", c_int64)]
+
+
+MSA_TILES_NONE, MSA_TILES_WHOLE, MSA_TILES_FEW, MSA_TILES_EVEN, MSA_TILES_SIMPLE = range(5)
+
 # name -> argtypes, in the order of include/metaseq_amd.h
 SIGNATURES = {
     "msa_pack_weight_f16": [_P, _P, c_int, c_int, _P],
@@ -75,6 +82,7 @@ SIGNATURES = {
     "msa_linear_default_splits": [c_int64, c_int, c_int],
     "msa_linear_default_splits_w8a16": [c_int64, c_int, c_int],
     "msa_linear_default_splits_rows": [c_int64, c_int, c_int],
+    "msa_linear_tiles": [c_int64, c_int, c_int, c_int, c_int, ctypes.POINTER(TileForm)],
     "msa_qkv_proj_f16": [_P, _P, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
                          c_uint, _P, _P],
     "msa_qkv_proj_w8a16": [_P, _P, _P, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int,

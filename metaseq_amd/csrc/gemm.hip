@@ -389,6 +389,26 @@ extern "C" int msa_linear_default_splits_rows(int64_t M, int N, int K) {
   return pick_row_splits_f16(M, N, K);
 }
 
+extern "C" int msa_linear_tiles(int64_t M, int N, int K, int S, int cus, msa_tile_form* out) {
+  const char* name = "msa_linear_tiles";
+  MSA_REQUIRE(out, MSA_ERR_INVALID_ARG, "%s: null pointer", name);
+  MSA_REQUIRE(M >= 1 && M < (1ll << 31) && N > 0 && N % 16 == 0 && K > 0 && K % 32 == 0 && S >= 0 && cus >= 0 &&
+                  (S == 0 || (K % (64 * S) == 0 && K / S >= 128)),
+              MSA_ERR_INVALID_ARG, "%s: M=%lld N=%d K=%d S=%d cus=%d", name, (long long)M, N, K, S, cus);
+  if (cus == 0) cus = num_cus();
+  const TileForm f = S == 0 ? tile_form(M, N, K, cus) : partial_form(M, N, K, S, cus);
+  *out = msa_tile_form{f.kind, 0, 0, 0, 0, f.pieces, 0, f.main};
+  if (f.kind == MSA_TILES_NONE) return MSA_OK;
+  out->rows = tq_bm(f.rf), out->columns = tq_bn(f.wf);
+  out->n_rows = f.kind == MSA_TILES_EVEN ? f.even.nrow : (int)((f.main + out->rows - 1) / out->rows);
+  if (f.kind == MSA_TILES_EVEN) out->n_tall = f.even.n_tall;
+  const int ncol = (N + out->columns - 1) / out->columns;
+  out->panels = f.kind == MSA_TILES_FEW && S == 0 ? out->n_rows > 1
+                : f.kind != MSA_TILES_SIMPLE      ? tile_order(ncol, out->n_rows, f.wf).a < 0
+                                                  : 0;
+  return MSA_OK;
+}
+
 extern "C" int msa_linear_f16(const void* x, const void* Wp, const void* bias,
                               const void* residual, void* y, int64_t M, int N, int K,
                               unsigned flags, void* stream) {

@@ -2460,10 +2460,9 @@ void launch_quad_pieces(const void* x, const void* W, int64_t M, int N, int K, i
 // M_main on (at most 128).
 template <int MODE, int WF>
 void launch_quad(const void* x, const void* W, const void* scales, int64_t M, int64_t M_main, int N,
-                 int K, const Epilogue& epi, hipStream_t s) {
+                 int K, int pieces, const Epilogue& epi, hipStream_t s) {
   const int ncol = (N + tq_bn(WF) - 1) / tq_bn(WF);
   const int nrow = (int)((M_main + TQ_BM - 1) / TQ_BM);
-  const int pieces = WF == 8 ? quad_pieces((int64_t)ncol * nrow, num_cus()) : 1;
   if (pieces == 4) {
     launch_quad_pieces<MODE, false, 4>(x, W, M_main, N, K, 1, epi, nullptr, s);
   } else if (pieces == 2) {
@@ -2520,30 +2519,6 @@ void launch_quad_partial_w(const void* x, const void* W, float* part, int64_t M,
                      (const half_t*)x, W, M, N, K, o.a, o.r, e, part, K / 64 / S, GroupTiles{});
 }
 
-// fp16: 256 x 64 tiles while their S slices fit the chip in one round; an S beyond that means 256 x 128 tiles
-// (pick_row_splits), and one for which those do not fit either 256 x 256 (pick_row_splits_f16).  bf16
-// (prefill-sized products whose sums leave as fp32): the cheapest of all widths.
-template <int MODE>
-void launch_quad_partial(const void* x, const void* W, float* part, int64_t M, int N, int K, int S,
-                         hipStream_t s) {
-  const int64_t rows = (M + TQ_BM - 1) / TQ_BM;
-  const int64_t tiles2 = rows * ((N + 63) / 64) * S;
-  if (M >= TQ_BM) {
-    const QuadPrice price = quad_price(M, N, K, S, num_cus());
-    if (price.w == QUAD_EVEN) return launch_quad_plan<MODE, true>(x, W, M, N, K, S, price.even, Epilogue{}, part, s);
-    if (price.w == 8) {
-      const int pieces = quad_pieces(rows * ((N + 255) / 256) * S, num_cus());
-      if (pieces == 4) return launch_quad_pieces<MODE, true, 4>(x, W, M, N, K, S, Epilogue{}, part, s);
-      if (pieces == 2) return launch_quad_pieces<MODE, true, 2>(x, W, M, N, K, S, Epilogue{}, part, s);
-      return launch_quad_partial_w<MODE, 8>(x, W, part, M, N, K, S, s);
-    }
-    if (price.w == 4) return launch_quad_partial_w<MODE, 4>(x, W, part, M, N, K, S, s);
-    return launch_quad_partial_w<MODE, 2>(x, W, part, M, N, K, S, s);
-  }
-  if (tiles2 > num_cus()) return launch_quad_partial_w<MODE, 4>(x, W, part, M, N, K, S, s);
-  launch_quad_partial_w<MODE, 2>(x, W, part, M, N, K, S, s);
-}
-
 // How a product of more than 64 row-major rows is taken: the forms of quad_price, 128 x 128 tiles (w = 0), and two ways
 // to take a ragged bottom of at most 128 rows: as one more, moved-up row of tiles, or (main < M) through the
 // streaming kernel, a sweep over the weights per 64 rows.
@@ -2581,6 +2556,77 @@ TileChoice tile_choice(int64_t M, int N, int K, int cus) {
     offer(quad_cost((rows - 1) * cols[0], K, cus) + below, 8, M - rem);
   }
   return best;
+}
+
+// What a product of row-major activations is taken with.
+struct TileForm {
+  int kind = MSA_TILES_SIMPLE, wf = 4, rf = 4, pieces = 1;
+  int64_t main = 0;  // rows in tiles; the others in sweeps over the weights
+  QuadPlan even;
+};
+// S sums to be stored as they are, of any number of rows: the cheapest form of quad_price.  Below 256 rows 256 x 64 tiles while
+// their slices fit the chip in one round; an S beyond that means 256 x 128 tiles (pick_row_splits).
+TileForm partial_form(int64_t M, int N, int K, int S, int cus) {
+  const int64_t rows = (M + TQ_BM - 1) / TQ_BM;
+  TileForm f;
+  f.main = M, f.rf = 8;
+  if (M < TQ_BM) {
+    f.kind = MSA_TILES_FEW;
+    f.wf = rows * ((N + 63) / 64) * S > cus ? 4 : 2;
+    return f;
+  }
+  const QuadPrice price = quad_price(M, N, K, S, cus);
+  f.kind = price.w == QUAD_EVEN ? MSA_TILES_EVEN : MSA_TILES_WHOLE;
+  f.even = price.even;
+  f.wf = price.w == QUAD_EVEN ? price.even.wf : price.w;
+  if (price.w == QUAD_EVEN) f.rf = price.even.rf;
+  if (price.w == 8) f.pieces = quad_pieces(rows * ((N + 255) / 256) * S, cus);
+  return f;
+}
+// A whole product.  Fewer rows than a tile, or hardly more: launch_few_rows where its tiles fill one round (three quarters of
+// the CUs with 256 x 256 tiles).  Else the cheapest form of tile_choice; the 256 x 64 tiles also serve 65 .. 255
+// rows (they repeat the last row instead of moving up).  linear_tiled_kernel is left with what is no
+// multiple of 64 deep: a few tiles of the direct-to-LDS forms are ahead of it too (us: 100 x 768 x 768 17.0 and 10.1, 200
+// x 1024 x 4096 60 and 28, 300 x 768 x 3072 58 and 22, 500 x 256 x 1024 20.5 and 11.2, 65 x 16 x 2048 29.8 and 18.5, 65
+// x 128 x 128 8.0 and 7.6).
+TileForm tile_form(int64_t M, int N, int K, int cus) {
+  TileForm f;
+  if (M <= 64) {
+    f.kind = MSA_TILES_NONE;
+    return f;
+  }
+  f.main = M;
+  if (K % 64 || K < 128) return f;
+  const int64_t cols[2] = {(N + 255) / 256, (N + 127) / 128};
+  if (M < TQ_BM && cols[0] <= cus && cols[0] * 4 >= cus * 3) {
+    f.kind = MSA_TILES_FEW;
+    f.wf = 8, f.rf = M <= 128 ? 4 : M <= 160 ? 5 : M <= 192 ? 6 : M <= 224 ? 7 : 8;
+    return f;
+  }
+  if (M > 128 && M <= TQ_BM && cols[1] * 2 <= cus && K >= (cols[1] * 8 <= cus * 3 ? 512 : 4096)) {
+    f.kind = MSA_TILES_FEW;
+    return f;
+  }
+  const TileChoice c = tile_choice(M, N, K, cus);
+  f.kind = c.w == QUAD_EVEN ? MSA_TILES_EVEN : c.w == 0 ? MSA_TILES_FEW : MSA_TILES_WHOLE;
+  f.even = c.even;
+  f.main = c.w == QUAD_EVEN || c.w == 0 ? M : c.main;
+  if (c.w == QUAD_EVEN) f.wf = c.even.wf, f.rf = c.even.rf;
+  if (c.w > 1) f.wf = c.w, f.rf = 8;
+  if (c.w == 8) f.pieces = quad_pieces((f.main + TQ_BM - 1) / TQ_BM * cols[0], cus);
+  return f;
+}
+
+template <int MODE>
+void launch_quad_partial(const void* x, const void* W, float* part, int64_t M, int N, int K, int S,
+                         hipStream_t s) {
+  const TileForm f = partial_form(M, N, K, S, num_cus());
+  if (f.kind == MSA_TILES_EVEN) return launch_quad_plan<MODE, true>(x, W, M, N, K, S, f.even, Epilogue{}, part, s);
+  if (f.pieces == 4) return launch_quad_pieces<MODE, true, 4>(x, W, M, N, K, S, Epilogue{}, part, s);
+  if (f.pieces == 2) return launch_quad_pieces<MODE, true, 2>(x, W, M, N, K, S, Epilogue{}, part, s);
+  if (f.wf == 8) return launch_quad_partial_w<MODE, 8>(x, W, part, M, N, K, S, s);
+  if (f.wf == 4) return launch_quad_partial_w<MODE, 4>(x, W, part, M, N, K, S, s);
+  launch_quad_partial_w<MODE, 2>(x, W, part, M, N, K, S, s);
 }
 
 // Slices for a product of M row-major rows whose tiles alone leave most of the chip idle (a
@@ -2667,29 +2713,20 @@ void launch_tiled(const void* x, const void* W, const void* scales, int64_t M, i
   // int8: the 256 x 256 kernel once it fills the chip; the 128 x 128 one for the shapes in between
   const int64_t big_tiles = ((M + TB_BM - 1) / TB_BM) * ((N + TB_BN - 1) / TB_BN);
   if constexpr (!W8) {
-    // Fewer rows than a tile, or hardly more: launch_few_rows where its tiles fill one round (three quarters of
-    // the CUs with 256 x 256 tiles).  Else the cheapest form of tile_choice; the 256 x 64 tiles also serve 65 .. 255
-    // rows (they repeat the last row instead of moving up).  linear_tiled_kernel is left with what is no
-    // multiple of 64 deep: a few tiles of the direct-to-LDS forms are ahead of it too (us: 100 x 768 x 768 17.0 and 10.1, 200
-    // x 1024 x 4096 60 and 28, 300 x 768 x 3072 58 and 22, 500 x 256 x 1024 20.5 and 11.2, 65 x 16 x 2048 29.8 and 18.5, 65
-    // x 128 x 128 8.0 and 7.6).
-    if (K % 64 == 0 && K >= 128 && M > 64) {
-      const int64_t cus = num_cus(), cols[2] = {(N + 255) / 256, (N + 127) / 128};
-      if (M < TQ_BM && cols[0] <= cus && cols[0] * 4 >= cus * 3) {
-        if (M <= 128) return launch_few_rows<MODE, 8, 4>(x, W, M, N, K, epi, s);
-        if (M <= 160) return launch_few_rows<MODE, 8, 5>(x, W, M, N, K, epi, s);
-        if (M <= 192) return launch_few_rows<MODE, 8, 6>(x, W, M, N, K, epi, s);
-        if (M <= 224) return launch_few_rows<MODE, 8, 7>(x, W, M, N, K, epi, s);
-        return launch_few_rows<MODE, 8, 8>(x, W, M, N, K, epi, s);
-      }
-      if (M > 128 && M <= TQ_BM && cols[1] * 2 <= cus && K >= (cols[1] * 8 <= cus * 3 ? 512 : 4096))
-        return launch_few_rows<MODE, 4, 4>(x, W, M, N, K, epi, s);
-      const TileChoice c = tile_choice(M, N, K, (int)cus);
-      if (c.w == QUAD_EVEN) return launch_quad_plan<MODE, false>(x, W, M, N, K, 1, c.even, epi, nullptr, s);
-      if (c.w == 8) return launch_quad<MODE, 8>(x, W, scales, M, c.main, N, K, epi, s);
-      if (c.w == 4) return launch_quad<MODE, 4>(x, W, scales, M, c.main, N, K, epi, s);
-      if (c.w == 2) return launch_quad<MODE, 2>(x, W, scales, M, c.main, N, K, epi, s);
-      return launch_few_rows<MODE, 4, 4>(x, W, M, N, K, epi, s);
+    const TileForm f = tile_form(M, N, K, num_cus());
+    if (f.kind == MSA_TILES_EVEN) return launch_quad_plan<MODE, false>(x, W, M, N, K, 1, f.even, epi, nullptr, s);
+    if (f.kind == MSA_TILES_WHOLE) {
+      if (f.wf == 8) return launch_quad<MODE, 8>(x, W, scales, M, f.main, N, K, f.pieces, epi, s);
+      if (f.wf == 4) return launch_quad<MODE, 4>(x, W, scales, M, f.main, N, K, 1, epi, s);
+      return launch_quad<MODE, 2>(x, W, scales, M, f.main, N, K, 1, epi, s);
+    }
+    if (f.kind == MSA_TILES_FEW) {
+      if (f.wf == 4) return launch_few_rows<MODE, 4, 4>(x, W, M, N, K, epi, s);
+      if (f.rf == 4) return launch_few_rows<MODE, 8, 4>(x, W, M, N, K, epi, s);
+      if (f.rf == 5) return launch_few_rows<MODE, 8, 5>(x, W, M, N, K, epi, s);
+      if (f.rf == 6) return launch_few_rows<MODE, 8, 6>(x, W, M, N, K, epi, s);
+      if (f.rf == 7) return launch_few_rows<MODE, 8, 7>(x, W, M, N, K, epi, s);
+      return launch_few_rows<MODE, 8, 8>(x, W, M, N, K, epi, s);
     }
   }
   if constexpr (W8) if (K % (2 * TB_BK) == 0 && big_tiles >= num_cus()) {

@@ -112,3 +112,51 @@ def test_only_products_that_fold_stop_at_four_slices(N, K, rows, fp16, bf16):
     for M in rows:
         assert core.msa_linear_default_splits(M, N, K) == fp16, M
         assert hybrid.msa_linear_bf16_splits(M, N, K, 1) == bf16, M
+
+
+def tiles(M, N, K, S=0, cus=256):
+    f = _capi.TileForm()
+    assert _capi.load().msa_linear_tiles(M, N, K, S, cus, ctypes.byref(f)) == 0
+    return f
+
+
+@pytest.mark.parametrize("M,N,K,S,want", [
+    (64, 4096, 4096, 0, dict(kind=_capi.MSA_TILES_NONE, main=0)),
+    (65, 768, 96, 0, dict(kind=_capi.MSA_TILES_SIMPLE, rows=128, columns=128)),
+    (65, 768, 768, 0, dict(kind=_capi.MSA_TILES_WHOLE, columns=64, n_rows=1)),
+    (200, 12288, 4096, 0, dict(kind=_capi.MSA_TILES_FEW, rows=128, columns=128, n_rows=2)),
+    (66, 50272, 4096, 0, dict(kind=_capi.MSA_TILES_FEW, rows=128, columns=256)),
+    (129, 50272, 4096, 0, dict(kind=_capi.MSA_TILES_FEW, rows=160, columns=256)),
+    (193, 50272, 4096, 0, dict(kind=_capi.MSA_TILES_FEW, rows=224, columns=256)),
+    (2005, 9216, 4096, 0, dict(kind=_capi.MSA_TILES_WHOLE, columns=256, pieces=4, main=2005)),
+    (32800, 16384, 4096, 0, dict(kind=_capi.MSA_TILES_WHOLE, columns=256, pieces=1, main=32768)),
+    (1607, 16384, 4096, 0, dict(kind=_capi.MSA_TILES_EVEN)),
+    (2005, 4096, 16384, 2, dict(columns=256)),
+    (200, 4096, 16384, 8, dict(kind=_capi.MSA_TILES_FEW, rows=256, columns=128)),
+    (200, 4096, 4096, 4, dict(kind=_capi.MSA_TILES_FEW, rows=256, columns=64))])
+def test_tiles_of_a_product(M, N, K, S, want):
+    f = tiles(M, N, K, S)
+    assert {k: getattr(f, k) for k in want} == want
+
+
+def test_even_cuts_cover_the_rows():
+    seen = set()
+    for M in list(range(256, 2100, 7)) + [3000, 5555, 8200]:
+        for N, K, S in ((4096, 4096, 0), (12288, 4096, 0), (16384, 4096, 0), (4096, 16384, 1), (2048, 8192, 2), (11392, 1984, 0)):
+            f = tiles(M, N, K, S)
+            if f.kind != _capi.MSA_TILES_EVEN:
+                continue
+            low = f.rows - 32
+            rows = f.n_tall * f.rows + (f.n_rows - f.n_tall) * low
+            last = f.rows if f.n_tall == f.n_rows else low
+            assert rows - last < M <= rows and 0 <= f.n_tall <= f.n_rows and 160 <= f.rows <= 32 * (8 if f.columns == 256 else 7)
+            assert f.main == M and f.pieces == 1
+            seen.add((f.columns, f.rows))
+    assert len(seen) > 4
+
+
+def test_tiles_refuses_what_the_products_refuse():
+    lib, f = _capi.load(), _capi.TileForm()
+    for bad in ((0, 64, 64, 0, 256), (4, 8, 64, 0, 256), (4, 64, 48, 0, 256), (300, 64, 256, 4, 256), (300, 64, 256, -1, 256)):
+        assert lib.msa_linear_tiles(*bad, ctypes.byref(f)) == -1, bad
+    assert lib.msa_linear_tiles(300, 64, 256, 0, 256, None) == -1
