@@ -155,6 +155,16 @@ def test_even_cuts_cover_the_rows():
     assert len(seen) > 4
 
 
+@pytest.mark.parametrize("M,N,K,S,panels", [
+    (516, 11392, 1984, 0, 1), (516, 11392, 1984, 1, 1), (1143, 2160, 1856, 0, 1), (669, 12480, 512, 0, 1),
+    (1436, 3552, 448, 0, 0),       # columns in fours
+    (778, 1600, 14720, 2, 0),      # slices
+    (640, 12288, 4096, 0, 0), (545, 16400, 704, 0, 1)])
+def test_even_cuts_of_odd_columns_are_taken_in_panels(M, N, K, S, panels):
+    f = tiles(M, N, K, S)
+    assert (f.kind, f.panels) == (_capi.MSA_TILES_EVEN, panels), (f.kind, f.columns, f.n_rows)
+
+
 def test_tiles_refuses_what_the_products_refuse():
     lib, f = _capi.load(), _capi.TileForm()
     for bad in ((0, 64, 64, 0, 256), (4, 8, 64, 0, 256), (4, 64, 48, 0, 256), (300, 64, 256, 4, 256), (300, 64, 256, -1, 256)):

@@ -556,6 +556,14 @@ def test_qkv_proj_rows_cut_evenly(lib, M, H, K):
     test_qkv_proj_rows_into_cache_rows_and_positions_of_their_own(lib, M, H, K, False, False)
 
 
+# an odd number of columns below 64, in panels: of one and of more columns at the end
+@pytest.mark.parametrize("M,N,K", [(1143, 2160, 704), (516, 11392, 704), (669, 12480, 192), (1200, 4240, 128)])
+def test_linear_f16_rows_cut_evenly_of_odd_columns(lib, M, N, K):
+    from tests.test_capi_cpu import tiles
+    assert tiles(M, N, K).kind == 3 and tiles(M, N, K).panels
+    test_linear_f16_pieces(lib, M, N, K)
+
+
 # fewer tiles than an eighth of the chip
 @pytest.mark.parametrize("M,N,K", [(65, 16, 128), (128, 80, 192), (129, 48, 512), (200, 272, 704), (300, 128, 128)])
 def test_linear_f16_few_tiles(lib, M, N, K):
