@@ -404,7 +404,7 @@ extern "C" int msa_linear_tiles(int64_t M, int N, int K, int S, int cus, msa_til
   if (f.kind == MSA_TILES_EVEN) out->n_tall = f.even.n_tall;
   const int ncol = (N + out->columns - 1) / out->columns;
   out->panels = f.kind == MSA_TILES_FEW && S == 0 ? out->n_rows > 1
-                : f.kind == MSA_TILES_EVEN        ? even_order(ncol, out->n_rows, f.wf, S > 1 ? S : 1).a < 0
+                : f.kind == MSA_TILES_EVEN        ? even_order(ncol, out->n_rows, f.wf, S > 1 ? S : 1, cus).a < 0
                 : f.kind != MSA_TILES_SIMPLE      ? tile_order(ncol, out->n_rows, f.wf).a < 0
                                                   : 0;
   return MSA_OK;

@@ -2419,11 +2419,12 @@ QuadPrice quad_price(int64_t M, int N, int K, int S, int cus) {
 // Row by row, a number of columns that 4 does not divide moves a column on to another XCD in each row of tiles, and each of
 // them reads its weights from beyond its own L2; an even cut has many rows.  In panels a column keeps to one XCD: 516 x
 // 11392 x 1984 (45 columns, five rows) 40.3 -> 35.5 us, 1143 x 2160 x 1856 (17, nine) 19.2 -> 16.9, 669 x 12480 x 512 21.1 ->
-// 16.2.  28 columns, two XCDs to each, are as well row by row (1436 x 3552 x 448 10.0 and 10.7), and so are slices, of which
-// the empty places behind each leave the XCDs unequal shares (778 x 1600 x 14720 64 and 76).
-TileOrder even_order(int ncol, int nrow, int WF, int S) {
+// 16.2.  28 columns, two XCDs to each, are as well row by row (1436 x 3552 x 448 10.0 and 10.7).  The empty places behind the
+// tiles of a slice leave the XCDs unequal shares: slices are taken so where all tiles still run at once (in two slices, 600 x
+// 3424 x 9600 55.4 -> 51.1; 778 x 1600 x 14720 64 and 76).
+TileOrder even_order(int ncol, int nrow, int WF, int S, int cus) {
   TileOrder o = tile_order(ncol, nrow, WF);
-  if (o.a == 0 && S == 1 && ncol % 4 && ncol > TQ_PANEL && nrow > 1) o.a = -TQ_PANEL;
+  if (o.a == 0 && ncol % 4 && ncol > TQ_PANEL && nrow > 1 && (S == 1 || (ncol * nrow + 7) / 8 * 8 * S <= cus)) o.a = -TQ_PANEL;
   return o;
 }
 template <int MODE, int WF, bool PART, int RF>
@@ -2434,7 +2435,7 @@ void launch_quad_even(const void* x, const void* W, int64_t M, int N, int K, int
   auto kernel = linear_quad_even_kernel<MODE, WF, PART, RF>;
   if (!allow_lds((const void*)kernel, lds, lds_allowed_e)) return;
   const int ncol = (N + tq_bn(WF) - 1) / tq_bn(WF);
-  const TileOrder o = even_order(ncol, p.nrow, WF, S);
+  const TileOrder o = even_order(ncol, p.nrow, WF, S, num_cus());
   hipLaunchKernelGGL(kernel, quad_grid(ncol, p.nrow, o, S), dim3(TQ_THREADS), lds, s, (const half_t*)x, W, M, N, K,
                      p.nrow, p.n_tall, o.a, o.r, epi, part, K / 64 / S);
 }

@@ -158,7 +158,7 @@ def test_even_cuts_cover_the_rows():
 @pytest.mark.parametrize("M,N,K,S,panels", [
     (516, 11392, 1984, 0, 1), (516, 11392, 1984, 1, 1), (1143, 2160, 1856, 0, 1), (669, 12480, 512, 0, 1),
     (1436, 3552, 448, 0, 0),       # columns in fours
-    (778, 1600, 14720, 2, 0),      # slices
+    (600, 3424, 9600, 2, 1), (778, 1600, 14720, 2, 0), (1110, 3296, 8576, 2, 0),      # slices
     (640, 12288, 4096, 0, 0), (545, 16400, 704, 0, 1)])
 def test_even_cuts_of_odd_columns_are_taken_in_panels(M, N, K, S, panels):
     f = tiles(M, N, K, S)

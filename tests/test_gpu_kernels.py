@@ -536,9 +536,8 @@ def test_linear_f16_rows_cut_evenly(lib, M, N, K):
 
 
 @pytest.mark.parametrize("M,N", [(289, 6144), (387, 6144), (385, 8208), (577, 8208), (898, 8208), (1345, 8208), (2465, 8208)])
-def test_split_k_partials_of_rows_cut_evenly(lib, M, N):
-    K = 256
-    print("even partials", M, N, flush=True)
+def test_split_k_partials_of_rows_cut_evenly(lib, M, N, K=256):
+    print("even partials", M, N, K, flush=True)
     x, W = G(rnd(M, K, seed=M)), G(rnd(N, K, seed=N, std=0.05))
     for S in (1, 2):
         part = torch.full((S + 1, M, N), float("nan"), dtype=torch.float32, device=DEV)
@@ -549,6 +548,13 @@ def test_split_k_partials_of_rows_cut_evenly(lib, M, N):
             want = xs @ ws.t()
             # a sum of K / S fp32 terms
             assert float((got - want).abs().max()) <= 8 * 2.0 ** -24 * K ** 0.5 * float(want.abs().max())
+
+
+@pytest.mark.parametrize("M,N", [(372, 3424), (385, 6288), (1100, 2128)])
+def test_split_k_partials_of_rows_cut_evenly_of_odd_columns(lib, M, N):
+    from tests.test_capi_cpu import tiles
+    assert all(tiles(M, N, 1408, S).kind == 3 and tiles(M, N, 1408, S).panels for S in (1, 2))
+    test_split_k_partials_of_rows_cut_evenly(lib, M, N, 1408)
 
 
 @pytest.mark.parametrize("M,H,K", [(385, 32, 256), (577, 43, 256), (1569, 43, 128)])
