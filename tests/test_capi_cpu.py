@@ -165,6 +165,34 @@ def test_even_cuts_of_odd_columns_are_taken_in_panels(M, N, K, S, panels):
     assert (f.kind, f.panels) == (_capi.MSA_TILES_EVEN, panels), (f.kind, f.columns, f.n_rows)
 
 
+def test_sizes_of_the_kernel_tests_reach_the_kernels_that_they_name():
+    from tests import test_gpu_hybrid_kernels as H, test_gpu_kernels as C
+
+    def of(M, N, K, S=0):
+        f = tiles(M, N, K, S)
+        return f.kind, f.columns, f.rows
+    for M, N, K, pieces in C.PIECES:
+        assert tiles(M, N, K).pieces == pieces, (M, N, K)
+    for M, K, rows in C.FEW_ROWS:
+        assert of(M, 50272, K) == (_capi.MSA_TILES_FEW, 256, rows), M
+    for M, N, columns, rows, tall in C.EVEN_DEEP:
+        assert of(M, N, 704) + (tiles(M, N, 704).n_tall,) == (_capi.MSA_TILES_EVEN, columns, rows, tall), (M, N)
+    for M, N, K in C.EVEN_ODD:
+        assert tiles(M, N, K).kind == _capi.MSA_TILES_EVEN and tiles(M, N, K).panels, (M, N, K)
+    for M, N in C.PARTIALS_ODD:
+        assert all(tiles(M, N, 1408, S).kind == _capi.MSA_TILES_EVEN and tiles(M, N, 1408, S).panels for S in (1, 2)), (M, N)
+    for M, N, columns, rows in C.PARTIALS_DEEP:
+        assert of(M, N, 1408, 2) == (_capi.MSA_TILES_EVEN, columns, rows), (M, N)
+    for M, heads, columns, rows in C.QKV_DEEP:
+        assert of(M, 384 * heads, 704) == (_capi.MSA_TILES_EVEN, columns, rows), (M, heads)
+    for M, N, pieces in H.BF16_PIECES:
+        assert tuple(tiles(M, N, 1408, S).pieces for S in (0, 1, 2)) == pieces, (M, N)
+    for M, N, columns, rows in H.BF16_EVEN:
+        assert of(M, N, 1408) == (_capi.MSA_TILES_EVEN, columns, rows), (M, N)
+    assert {r[2:4] for r in C.EVEN_DEEP} == {(128, 160), (128, 192), (128, 224), (256, 160), (256, 192), (256, 224), (256, 256)}
+    assert {r[2:4] for r in C.PARTIALS_DEEP} == {r[2:4] for r in C.EVEN_DEEP}
+
+
 def test_tiles_refuses_what_the_products_refuse():
     lib, f = _capi.load(), _capi.TileForm()
     for bad in ((0, 64, 64, 0, 256), (4, 8, 64, 0, 256), (4, 64, 48, 0, 256), (300, 64, 256, 4, 256), (300, 64, 256, -1, 256)):

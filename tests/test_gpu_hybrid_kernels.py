@@ -145,10 +145,10 @@ def test_linear_partial_bf16_in_two_slices(M, N, K):
 
 
 @pytest.mark.parametrize("M,N", [(1500, 6032), (1500, 6912), (2305, 7168), (3000, 7680)])
-def test_linear_bf16_pieces(M, N):
-    """A few tiles past whole rounds, cut in four or in two: sums of one and two slices (288 and 324 tiles of
-    them), a gated activation with fp32 columns behind it."""
-    lib, K = _capi.load_hybrid(), 256
+def test_linear_bf16_pieces(M, N, K=256):
+    """More than a round of tiles: sums of one and two slices, a gated activation with fp32 columns behind it."""
+    lib = _capi.load_hybrid()
+    print("rows", M, N, K, flush=True)
     g = torch.Generator("cuda").manual_seed(M)
     x = torch.randn(M, K, generator=g, device="cuda").to(BF16)
     w = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).to(BF16)
@@ -164,6 +164,26 @@ def test_linear_bf16_pieces(M, N):
                               _capi.stream_ptr()), lib)
     close(y.cpu(), glu(_capi.MSA_GLU_CLAMPED, ref[:, 0:n32:2], ref[:, 1:n32:2], 0.7), 6e-3, "glu")
     close(y32.cpu(), ref[:, n32:], 1e-5, "fp32 columns beside glu")
+
+
+# the pieces that the last tiles are cut into as a whole product, as sums of one slice and of two (of eleven stages and more)
+BF16_PIECES = [(3000, 5632, (4, 4, 4)), (2817, 6400, (4, 4, 1)), (3000, 7488, (2, 2, 1)), (3000, 6304, (4, 4, 2)),
+               (1500, 6912, (1, 1, 2))]
+
+
+@pytest.mark.parametrize("M,N,pieces", BF16_PIECES)
+def test_linear_bf16_pieces_of_the_last_round(M, N, pieces):
+    test_linear_bf16_pieces(M, N, 1408)
+
+
+# (columns and rows of the taller tiles of the whole product)
+BF16_EVEN = [(481, 8224, 128, 192), (577, 8224, 128, 224), (385, 8224, 128, 160), (898, 8224, 256, 160), (1345, 8224, 256, 224),
+             (2465, 8224, 256, 192)]
+
+
+@pytest.mark.parametrize("M,N,columns,rows", BF16_EVEN)
+def test_linear_bf16_rows_cut_evenly_over_more_stages(M, N, columns, rows):
+    test_linear_bf16_pieces(M, N, 1408)
 
 
 @pytest.mark.parametrize("M,N", [(289, 6144), (387, 6144), (481, 8224), (577, 8224), (898, 8224), (1345, 8224), (2465, 8224)])
@@ -255,6 +275,9 @@ def test_linear_with_bias_rows_cut_evenly(M, N, K):
     test_linear_with_bias_activation_and_decays(M, N, K, BF16)
 
 
+@pytest.mark.parametrize("M,N,K", [(385, 8208, 704), (577, 8208, 704), (1345, 8208, 704)])
+def test_linear_with_bias_rows_cut_evenly_over_more_stages(M, N, K):
+    test_linear_with_bias_activation_and_decays(M, N, K, BF16)
 
 @pytest.mark.parametrize("dtype", [BF16, F32], ids=["bf16", "f32"])
 @pytest.mark.parametrize("M,D", [(1, 72), (5, 4096), (40, 1000), (130, 2100), (1100, 300),

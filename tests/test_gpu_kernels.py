@@ -492,15 +492,13 @@ def test_linear_f16_few_rows(lib, M, N, K, epi):
     assert bool(((y.float() - want).abs() <= bound).all())
 
 
-# Whole rounds of 256 x 256 tiles and a few left, which are cut in four (280, 276 and 1060 tiles) or in two (360 and
-# 1122): pieces past the last row or column, of one row and of a few columns, a last group of fewer
-# than eight tiles; and 128 x 128 tiles of more than 256 rows
+# Products of more than a round: 3000 x 7680 and 4352 x 16656 leave tiles that are cut in two, the others are cut evenly
+# or take 128 x 128 tiles (more pieces: PIECES below)
 @pytest.mark.parametrize("M,N,K", [(2305, 7168, 128), (2825, 5728, 128), (5000, 13328, 128), (2945, 7520, 128),
                                    (3000, 7680, 128), (4352, 16656, 128), (2048, 2048, 128), (641, 4112, 128),
                                    (2305, 7168, 704), (2945, 7520, 704)])
 def test_linear_f16_pieces(lib, M, N, K):
-    """(K = 704: the quarters' five stages of activations are gone through twice)"""
-    print("pieces", M, N, K, flush=True)
+    print("rows", M, N, K, flush=True)
     x, W, b = G(rnd(M, K, seed=M)), G(rnd(N, K, seed=N, std=0.05)), G(rnd(N, seed=9, std=0.1))
     y = G(rnd(M, N, seed=10))
     res = y.float()
@@ -517,10 +515,31 @@ def test_linear_f16_pieces(lib, M, N, K):
     assert bool(((y.float() - want).abs() <= bound).all())
 
 
+# Whole rounds of 256 x 256 tiles and a few left, which are cut in two or in four: pieces past the last row or column, of one
+# row and of a few columns, a last group of fewer than eight tiles.  From K = 704 on, eleven stages, every ring (of three to
+# five stages of activations) is gone through twice and more, here and below.
+PIECES = [(3000, 5632, 704, 4), (2817, 6400, 1536, 4), (1000, 16400, 128, 4), (4096, 16640, 128, 4), (3000, 7488, 704, 2),
+          (2945, 8080, 704, 2), (3000, 7680, 128, 2), (4352, 16656, 128, 2)]
+
+
+@pytest.mark.parametrize("M,N,K,pieces", PIECES)
+def test_linear_f16_pieces_of_the_last_round(lib, M, N, K, pieces):
+    test_linear_f16_pieces(lib, M, N, K)
+
+
 # a vocabulary of fewer rows than a tile: as high as the rows need
 @pytest.mark.parametrize("M", [66, 128, 129, 160, 161, 192, 193, 224, 225])
 def test_linear_f16_vocabulary_of_few_rows(lib, M):
     test_linear_f16_pieces(lib, M, 50272, 192)
+
+
+# (M, K, rows of the tile)
+FEW_ROWS = [(M, 704, rows) for M, rows in ((66, 128), (128, 128), (130, 160), (161, 192), (200, 224), (225, 256))]
+
+
+@pytest.mark.parametrize("M,K,rows", FEW_ROWS)
+def test_linear_f16_vocabulary_of_few_rows_and_more_stages(lib, M, K, rows):
+    test_linear_f16_pieces(lib, M, 50272, K)
 
 
 # rows cut evenly: tiles of 128 and of 256 columns, 160, 192, 224 and 256 rows high, alone and above lower ones, the
@@ -550,11 +569,38 @@ def test_split_k_partials_of_rows_cut_evenly(lib, M, N, K=256):
             assert float((got - want).abs().max()) <= 8 * 2.0 ** -24 * K ** 0.5 * float(want.abs().max())
 
 
-@pytest.mark.parametrize("M,N", [(372, 3424), (385, 6288), (1100, 2128)])
-def test_split_k_partials_of_rows_cut_evenly_of_odd_columns(lib, M, N):
-    from tests.test_capi_cpu import tiles
-    assert all(tiles(M, N, 1408, S).kind == 3 and tiles(M, N, 1408, S).panels for S in (1, 2))
+PARTIALS_ODD = [(372, 3424), (385, 6288), (1100, 2128)]   # in panels, of one and of two slices
+# (M, N, columns and rows of the taller tiles in two slices of eleven stages)
+PARTIALS_DEEP = [(289, 8208, 256, 160), (577, 8208, 256, 224), (1345, 8208, 256, 224), (2465, 8208, 256, 256),
+                 (700, 4096, 128, 192), (400, 6144, 128, 224), (270, 8192, 128, 160), (536, 8208, 256, 192)]
+
+
+@pytest.mark.parametrize("M,N", PARTIALS_ODD + [a[:2] for a in PARTIALS_DEEP])
+def test_split_k_partials_of_rows_cut_evenly_over_more_stages(lib, M, N):
     test_split_k_partials_of_rows_cut_evenly(lib, M, N, 1408)
+
+
+# (M, heads of 128, columns and rows of the taller tiles)
+QKV_DEEP = [(385, 32, 128, 224), (289, 32, 128, 160), (449, 43, 256, 160), (577, 43, 256, 224)]
+
+
+@pytest.mark.parametrize("M,H,columns,rows", QKV_DEEP)
+def test_qkv_proj_rows_cut_evenly_over_more_stages(lib, M, H, columns, rows):
+    """One position to a row: keys, values and queries against the plain product."""
+    K, D = 704, H * 128
+    print("qkv deep", M, H, flush=True)
+    x, W, b = G(rnd(M, K, seed=M)), G(rnd(3 * D, K, seed=H, std=0.05)), G(rnd(3 * D, seed=3, std=0.1))
+    k, v, q = (torch.full((M, D), float("nan"), dtype=torch.float16, device=DEV) for _ in range(3))
+    ok(lib.msa_qkv_proj_f16(P(x), P(pack_w(lib, W)), P(b), P(q), P(k), P(v), M, 1, H, 128, 0, 1, K, 0, None, None), lib)
+    torch.cuda.synchronize()
+    sums = x.float() @ W.float().t()
+    want = sums.half().float() + b.float()
+    # roundings of the sum and of the biased sum, which a sum of other order may take to either side, and the sum itself
+    size = torch.maximum(sums.abs(), want.abs())
+    bound = 4 * size * 2.0 ** -11 + 8 * 2.0 ** -24 * K ** 0.5 * float(size.square().mean().sqrt()) + 2.0 ** -24
+    for got, i, scale in ((k, 0, 1.0), (v, 1, 1.0), (q, 2, 128 ** -0.5)):
+        of = slice(i * D, (i + 1) * D)
+        assert bool(((got.float() - want[:, of] * scale).abs() <= bound[:, of] * scale + (scale < 1) * 2.0 ** -11 * want[:, of].abs() * scale).all()), i
 
 
 @pytest.mark.parametrize("M,H,K", [(385, 32, 256), (577, 43, 256), (1569, 43, 128)])
@@ -562,11 +608,24 @@ def test_qkv_proj_rows_cut_evenly(lib, M, H, K):
     test_qkv_proj_rows_into_cache_rows_and_positions_of_their_own(lib, M, H, K, False, False)
 
 
+# every height with the one below it, and alone: (M, N, columns and rows of the taller tiles, rows of tiles of that height)
+EVEN_DEEP = [(289, 12288, 128, 160, 2), (257, 12288, 128, 160, 1), (352, 528, 128, 160, 0), (353, 12288, 128, 192, 2),
+             (321, 12288, 128, 192, 1), (417, 12288, 128, 224, 2), (385, 12288, 128, 224, 1), (449, 16400, 256, 160, 3),
+             (257, 16400, 256, 160, 0), (385, 16400, 256, 160, 1), (545, 16400, 256, 192, 3), (481, 16400, 256, 192, 1),
+             (641, 16400, 256, 224, 3), (577, 16400, 256, 224, 1), (1569, 16400, 256, 256, 1)]
+
+
+@pytest.mark.parametrize("M,N,columns,rows,tall", EVEN_DEEP)
+def test_linear_f16_rows_cut_evenly_over_more_stages(lib, M, N, columns, rows, tall):
+    test_linear_f16_pieces(lib, M, N, 704)
+
+
 # an odd number of columns below 64, in panels: of one and of more columns at the end
-@pytest.mark.parametrize("M,N,K", [(1143, 2160, 704), (516, 11392, 704), (669, 12480, 192), (1200, 4240, 128)])
+EVEN_ODD = [(1143, 2160, 704), (516, 11392, 704), (669, 12480, 192), (1200, 4240, 128)]
+
+
+@pytest.mark.parametrize("M,N,K", EVEN_ODD)
 def test_linear_f16_rows_cut_evenly_of_odd_columns(lib, M, N, K):
-    from tests.test_capi_cpu import tiles
-    assert tiles(M, N, K).kind == 3 and tiles(M, N, K).panels
     test_linear_f16_pieces(lib, M, N, K)
 
 
