@@ -514,6 +514,48 @@ def test_group_linear_dense(M, dtype):
             close(y, ref, tol, "groups %s" % ((G, N, K, share),))
 
 
+# tiles of 256 rows and a last one of 128, 192 or 256: groups of no row, of one, at each edge and past a whole tile
+@pytest.mark.parametrize("N,K", [(544, 704), (256, 128), (1056, 192)])
+@pytest.mark.parametrize("kind", [-1, _capi.MSA_GLU_GELU, _capi.MSA_GLU_CLAMPED])
+def test_group_linear_routed_tiles_as_high_as_the_rows(N, K, kind):
+    lib = _capi.load_hybrid()
+    print("routed", N, K, kind, flush=True)
+    g, top = gen(N + kind), 2
+    counts = [1, 128, 129, 0, 192, 193, 256, 257, 384, 385, 448, 449, 300, 100]
+    E, P = len(counts), sum(counts)
+    flat = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(P, generator=g)]
+    x = torch.randn((P + top - 1) // top, K, generator=g).to(BF16)
+    w = (torch.randn(E, N, K, generator=g) * K ** -0.5).to(BF16)
+    n_max = P // 256 + E
+    ids = flat.int().cuda()
+    perm, inv = (torch.full((P,), -1, dtype=torch.int32, device="cuda") for _ in range(2))
+    end, n = torch.zeros(E, dtype=torch.int32, device="cuda"), torch.zeros(1, dtype=torch.int32, device="cuda")
+    tg, tr = (torch.full((n_max,), -1, dtype=torch.int32, device="cuda") for _ in range(2))
+    check(lib.msa_moe_plan(ptr(ids), P, E, 256, ptr(perm), ptr(inv), ptr(end), ptr(tg), ptr(tr), ptr(n), n_max,
+                           _capi.stream_ptr()), lib)
+    cols = N // 2 if kind >= 0 else N
+    xd, wd = x.cuda(), pack_tiles(w.view(E * N, K)).cuda()
+    y = torch.full((P + 1, cols), 7.0, dtype=BF16, device="cuda")
+    a = _capi.GroupLinearArgs()
+    a.dtype, a.glu, a.limit = 0, kind, 0.7
+    a.x, a.ldx, a.W, a.y, a.ldy = ptr(xd), K, ptr(wd), ptr(y), cols
+    a.N, a.K, a.groups, a.M = N, K, E, P
+    a.perm, a.tile_group, a.tile_row, a.n_tiles, a.group_end = ptr(perm), ptr(tg), ptr(tr), ptr(n), ptr(end)
+    a.rows_per_x, a.max_tiles, a.tile_rows = top, n_max, 256
+    check(lib.msa_group_linear(ctypes.byref(a), _capi.stream_ptr()), lib)
+    torch.cuda.synchronize()
+    assert bool((y[P] == 7.0).all()), "wrote past the last row"
+    first = 0
+    order = torch.sort(flat, stable=True).indices
+    for e, count in enumerate(counts):
+        ref = x[order[first:first + count] // top].double() @ w[e].double().T
+        if kind >= 0:
+            ref = glu(kind, ref[:, 0::2], ref[:, 1::2], 0.7)
+        if count:
+            close(y[first:first + count], ref, 6e-3, "group of %d" % count)
+        first += count
+
+
 @pytest.mark.parametrize("E,groups,keep,top", [(1, 1, 1, 1), (12, 1, 1, 5), (12, 4, 2, 3),
                                                (96, 8, 3, 10), (512, 16, 16, 8), (300, 100, 1, 3)])
 def test_route_and_plan(E, groups, keep, top):
