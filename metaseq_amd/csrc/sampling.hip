@@ -106,10 +106,11 @@ __global__ __launch_bounds__(SM_THREADS) void greedy_select_kernel(
   if ((reinterpret_cast<uintptr_t>(row) & 15) == 0) {
     const int nv = V >> 3;
     constexpr int UNR = 4;  // chunks requested together: one memory round trip per UNR chunks
-    // Of a chunk that holds none of the ids that may not be chosen only the values are compared (a thread's ids ascend,
-    // so the first of equals stays).  200 rows of 50272 27.7 -> 18.3 us.
+    // Of a chunk that holds none of the ids that are treated apart only the values are compared (a thread's ids ascend,
+    // so the first of equals stays), or, in a row that may only end, nothing.  200 rows of 50272 27.7 -> 18.3 us, finished
+    // ones 24.5 -> 17.8.
     auto special = [&](int c) {
-      bool any = only_eos || (ban_early && (eos >> 3) == c);
+      bool any = (only_eos || ban_early) && (eos >> 3) == c;
       for (int j = 0; j < banned.n; ++j) any |= (banned.id[j] >> 3) == c;
       if (ban_early)
         for (int j = 0; j < stop.n; ++j) any |= (stop.id[j] >> 3) == c;
@@ -136,7 +137,7 @@ __global__ __launch_bounds__(SM_THREADS) void greedy_select_kernel(
         if (special(c)) {
 #pragma unroll
           for (int i = 0; i < 8; ++i) visit((c << 3) + i, z[i]);
-        } else {
+        } else if (!only_eos) {
 #pragma unroll
           for (int i = 0; i < 8; ++i) {
             if (z[i] > best) {
@@ -144,7 +145,6 @@ __global__ __launch_bounds__(SM_THREADS) void greedy_select_kernel(
               bidx = (c << 3) + i;
             }
           }
-          if (bidx == 0x7fffffff) bidx = c << 3;  // nothing but the lowest value so far
         }
         if (cm > m) {  // rescale once per 8 ids
           s *= __expf(m - cm);

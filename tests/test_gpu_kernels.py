@@ -1256,6 +1256,22 @@ def test_greedy_select_finished_force_stop_nan(lib):
     assert tok[:3].tolist() == [2, 2, 2]
 
 
+@pytest.mark.parametrize("eos", [2, 16383, 16384, 16424 + 4])
+def test_greedy_select_rows_that_may_only_end(lib, eos):
+    """The end's id in the first chunk, at the edges of a thread's chunks and among the last ids that fill none."""
+    V = 8192 * 2 + 45
+    logits = rnd(4, V, seed=eos)
+    logits[1, eos] = float("-inf")
+    logits[2, 7] = float("nan")
+    fin = torch.tensor([1, 1, 1, 0], dtype=torch.uint8, device=DEV)
+    lp = torch.log_softmax(logits.double(), -1)
+    tok, sc = _select(lib, logits.to(DEV), banned=[1], finished=fin, eos=eos)
+    assert tok.tolist() == [eos, 0, 0, int(lp[3].masked_fill(torch.arange(V) == 1, -1e9).argmax())]
+    assert abs(float(sc[0]) - float(lp[0, eos])) < 2e-5 and sc[1:3].tolist() == [float("-inf")] * 2
+    tok, sc = _select(lib, logits.to(DEV), banned=[eos], force=1, eos=eos)
+    assert tok.tolist() == [0] * 4 and sc.tolist() == [float("-inf")] * 4
+
+
 def test_target_logprob(lib):
     R, V = 37, 50272
     logits = rnd(R, V, seed=9, std=1.2)
