@@ -449,13 +449,19 @@ __device__ __forceinline__ void stream_tiles(const half_t* __restrict__ xp, cons
   const int ngroups = (tile_end - tile_begin + NT - 1) / NT;
   const int nstages = (ks_end - ks_begin + KG * U - 1) / (KG * U);
   const int total = ngroups * nstages;
-  // (a stage is followed, not found by division: 30 scalar instructions each time, in kernels of a few us)
+  // A stage is followed, not found by division: 30 scalar instructions each time, in kernels of a few us (int8, one row, 6144
+  // x 2048 5.0 and 4.8 us).  Of three or four int8 tiles to a group the division is ahead, whose operands take fewer
+  // registers through the loop: 36864 x 9216 59.2 and 57.5, 28672 x 7168 38.2 and 37.2, 15360 x 5120 15.7 and 15.0.
+  constexpr bool BY_INDEX = W8 && NT > 2;
   struct At {
-    int grp, st, nstages;
+    int n, st, nstages;  // n: the group, or (BY_INDEX) the stage counted over all groups
     __device__ void next() {
-      if (++st == nstages) st = 0, ++grp;
+      if (BY_INDEX)
+        ++n;
+      else if (++st == nstages)
+        st = 0, ++n;
     }
-    __device__ bool last() const { return st + 1 == nstages; }
+    __device__ bool last() const { return BY_INDEX ? (n + 1) % nstages == 0 : st + 1 == nstages; }
   };
 
   // In the last row block the lanes of rows past M read row M - 1 (what they add is not stored): half as many lines to fetch
@@ -473,7 +479,8 @@ __device__ __forceinline__ void stream_tiles(const half_t* __restrict__ xp, cons
   // Steps and tiles past the end read a clamped, valid address: a surplus tile is dropped in
   // finish(), a surplus step gets its activation fragment zeroed in mma().
   auto load = [&](Stage& s, const At& at) {
-    const int st = at.st, t0 = tile_begin + at.grp * NT;
+    const int grp = BY_INDEX ? at.n / nstages : at.n, st = BY_INDEX ? at.n - grp * nstages : at.st;
+    const int t0 = tile_begin + grp * NT;
 #pragma unroll
     for (int u = 0; u < UA; ++u) {
       // first 32-wide step covered by this load (wave-uniform)
@@ -517,7 +524,7 @@ __device__ __forceinline__ void stream_tiles(const half_t* __restrict__ xp, cons
       for (int mb = 0; mb < MB; ++mb) acc[j][mb] = float4_t{0.f, 0.f, 0.f, 0.f};
   };
   auto mma = [&](Stage& s, const At& at) {
-    const int grp = at.grp, st = at.st;
+    const int grp = BY_INDEX ? at.n / nstages : at.n, st = BY_INDEX ? at.n - grp * nstages : at.st;
     half_t sc[NT];
     if (W8) {
       const int t0 = tile_begin + grp * NT;
@@ -562,8 +569,9 @@ __device__ __forceinline__ void stream_tiles(const half_t* __restrict__ xp, cons
         }
       }
   };
-  // the epilogue's operands of the group that comes next, where a thread has one slot of it
-  constexpr bool AHEAD = MB <= 2 && !XR && MODE != MODE_SELECT;
+  // the epilogue's operands of the group that comes next, where a thread has one slot of it (not of int8 weights, whose
+  // expansion fills the registers: one row, 12288 x 4096 11.3 and 10.8 us, 5120 x 20480 29.7 and 28.4)
+  constexpr bool AHEAD = MB <= 2 && !XR && MODE != MODE_SELECT && (!W8 || LN > 0);
   static_assert(!AHEAD || (SEL_IT == 1 && NT == RN), "one slot");
   constexpr int EMODE = MODE == MODE_SELECT ? MODE_PLAIN : MODE;
   Ahead<EMODE> ahead{};
@@ -631,7 +639,7 @@ __device__ __forceinline__ void stream_tiles(const half_t* __restrict__ xp, cons
   }
   auto take = [&](Stage& s) {
     mma(s, ma);
-    if (ma.last()) finish(ma.grp);
+    if (ma.last()) finish(BY_INDEX ? ma.n / nstages : ma.n);
     ma.next();
   };
   // stage idx is in `a`; steady state: every load is of a real stage
