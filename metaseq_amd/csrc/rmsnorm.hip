@@ -27,7 +27,9 @@ __device__ __forceinline__ float dot4(float4_t v) {
   return v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
 }
 
-// A row's weights are requested with the row: behind its sum over the workgroup they are a round trip with nothing beside it.
+// A row's weights are requested with the row where that is one float4 to a thread: behind its sum over the workgroup they are a
+// round trip with nothing beside it.  Of two and more they are read where they are used: kept through the
+// sums they take registers that are not there (a tail of two sublayers, 700 x 9216 146 -> 311 us, 700 x 8192 in fp32 18.7 -> 20.2).
 template <int NV, int NT>
 __device__ __forceinline__ void row_weights(const float* w, int Dp, float4_t (&to)[NV]) {
   if (!w) return;  // uniform
@@ -36,10 +38,10 @@ __device__ __forceinline__ void row_weights(const float* w, int Dp, float4_t (&t
     to[i] = *reinterpret_cast<const float4_t*>(w + min((int)(threadIdx.x + i * NT) * 4, Dp - 4));
 }
 
-// x (registers) -> h = x / rms(x) * w
-template <typename T, int NV, int NT>
-__device__ __forceinline__ void norm_out(const float4_t (&x)[NV], int64_t m, int D, int Dp, float eps,
-                                         const float4_t (&w)[NV], void* h, int mb, float* red) {
+// x (registers) -> h = x / rms(x) * w (GIVEN: the row's weights)
+template <typename T, int NV, int NT, bool GIVEN>
+__device__ __forceinline__ void norm_out(const float4_t (&x)[NV], int64_t m, int D, int Dp, float eps, const float* w,
+                                         const float4_t (&given)[NV], void* h, int mb, float* red) {
   float ss = 0.f;
 #pragma unroll
   for (int i = 0; i < NV; ++i) ss += dot4(x[i]);
@@ -48,7 +50,7 @@ __device__ __forceinline__ void norm_out(const float4_t (&x)[NV], int64_t m, int
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const int c = (threadIdx.x + i * NT) * 4;
-    if (c < Dp) store_act4<T>(h, m, Dp, mb, c, x[i] * r * w[i]);
+    if (c < Dp) store_act4<T>(h, m, Dp, mb, c, x[i] * r * (GIVEN ? given[i] : *reinterpret_cast<const float4_t*>(w + c)));
   }
 }
 
@@ -87,8 +89,7 @@ __global__ __launch_bounds__(NT) void embed_kernel(
     if (step) v[i] += *reinterpret_cast<const float4_t*>(step + c);
     *reinterpret_cast<float4_t*>(x + m * Dp + c) = v[i];
   }
-  if constexpr (NV > 1) row_weights<NV, NT>(w, Dp, wv);
-  if (w) norm_out<T, NV, NT>(v, m, D, Dp, eps, wv, h, mb, red);
+  if (w) norm_out<T, NV, NT, NV == 1>(v, m, D, Dp, eps, w, wv, h, mb, red);
 }
 
 // b += the sum of S slices of row m; four slices at a time, their loads in flight together.  One or two slices (prompts)
@@ -140,9 +141,11 @@ __global__ __launch_bounds__(NT) void tail_kernel(msa_tail_args a) {
   const int64_t m = blockIdx.x;
   const int D = a.D, Dp = a.Dp;
   float4_t b[NV], x[NV], w_post[NV], w_next[NV];
-  // (few rows, 32 x 4096: 6.3 -> 6.0 us.  Of many rows, two float4 to a thread, they only hold up the slices: 1500 x 4096 in two
-  // slices 22.9 and 23.4, two sublayers 26.3 and 27.9.)
-  constexpr bool AHEAD = NV == 1;
+  // (few rows, 32 x 4096: 6.3 -> 6.0 us.  Two and four float4 to a thread only hold up the slices, 1500 x 4096 in two slices 22.9
+  // and 23.4: they are requested behind those, in front of the sums (16 x 8192 4.2 -> 4.1), but for what that costs more: two of
+  // one fp32 sublayer (700 x 8192 18.5 and 20.5), four of two sublayers (above).  A second sublayer's sums take the
+  // registers of the first form: 16 x 4096 4.3 and 4.5.)
+  constexpr bool AHEAD = NV == 1 && !TWO, BEHIND = NV == 2 ? TWO || sizeof(T) == 2 : NV == 4 && !TWO, GIVEN = AHEAD || BEHIND;
   if constexpr (AHEAD) {
     row_weights<NV, NT>(a.w_post, Dp, w_post);
     row_weights<NV, NT>(a.w_next, Dp, w_next);
@@ -222,12 +225,12 @@ __global__ __launch_bounds__(NT) void tail_kernel(msa_tail_args a) {
     ss = block_sum_once<NT>(ss, red);
     r = 1.f / sqrtf(ss / (float)D + a.eps);
   }
-  if constexpr (!AHEAD) row_weights<NV, NT>(a.w_post, Dp, w_post);
+  if constexpr (BEHIND) row_weights<NV, NT>(a.w_post, Dp, w_post);
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const int c = (threadIdx.x + i * NT) * 4;
     if (c < Dp) {
-      if (a.w_post) b[i] = b[i] * r * w_post[i];
+      if (a.w_post) b[i] = b[i] * r * (GIVEN ? w_post[i] : *reinterpret_cast<const float4_t*>(a.w_post + c));
       x[i] += b[i];
       if (a.probe) *reinterpret_cast<float4_t*>(a.probe + m * Dp + c) = x[i];
       if (a.add) x[i] += *reinterpret_cast<const float4_t*>(a.add + m * Dp + c);
@@ -235,8 +238,8 @@ __global__ __launch_bounds__(NT) void tail_kernel(msa_tail_args a) {
       *reinterpret_cast<float4_t*>(a.x + m * Dp + c) = x[i];
     }
   }
-  if constexpr (!AHEAD) row_weights<NV, NT>(a.w_next, Dp, w_next);
-  if (a.w_next) norm_out<T, NV, NT>(x, m, D, Dp, a.eps, w_next, a.h, a.h_mb, red_next);
+  if constexpr (BEHIND) row_weights<NV, NT>(a.w_next, Dp, w_next);
+  if (a.w_next) norm_out<T, NV, NT, GIVEN>(x, m, D, Dp, a.eps, a.w_next, w_next, a.h, a.h_mb, red_next);
 }
 
 // Down-projected latents: one workgroup per token, the two norms by different halves of it.
