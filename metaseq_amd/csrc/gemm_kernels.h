@@ -1169,7 +1169,7 @@ __global__ __launch_bounds__(TL_THREADS) void linear_tiled_kernel(
     }
 }
 
-// ---- large tiled kernel -------------------------------------------------------------------
+// ---- large tiled kernel, int8 weights --------------------------------------------------------
 // 256 x 256 x 64 per workgroup of 8 waves on v_mfma_f32_16x16x32_f16; every wave owns 32 output
 // features (two weight tiles) for all 256 activation rows.  Weight fragments come straight from
 // the packed layout in global memory into registers (one KB per wave instruction, no LDS round
@@ -1189,12 +1189,11 @@ constexpr int TB_NT = TB_BN / 8 / 16;   // weight tiles per wave
 constexpr int TB_PD = 4;                // LDS fragment reads in flight
 constexpr int TB_LDS_BYTES = 2 * TB_BM * TB_LD * (int)sizeof(half_t);
 
-template <bool W8>
-struct BigW {  // the weight fragments of one 64-wide stage; int8: the raw 16 bytes per tile
-  half8_t f[W8 ? 1 : 2][TB_NT];
+struct BigW {  // one 64-wide stage of weights: 16 raw bytes per tile, the fragments of two steps
+  half8_t f[TB_NT];
 };
 
-template <bool W8, int MODE>
+template <int MODE>
 __global__ __launch_bounds__(TB_THREADS) void linear_tiled_big_kernel(
     const half_t* __restrict__ x, const void* __restrict__ Wp, const half_t* __restrict__ scales,
     int64_t M, int N, int K, Epilogue epi) {
@@ -1222,9 +1221,8 @@ __global__ __launch_bounds__(TB_THREADS) void linear_tiled_big_kernel(
 #pragma unroll
   for (int j = 0; j < TB_NT; ++j) {
     const int t = min(n0 / 16 + j, ntiles - 1);
-    // a tile's K sweep is K * 16 elements: K * 32 bytes in fp16, K * 16 bytes in int8
-    wsrc[j] = (const char*)Wp + (int64_t)t * K * (W8 ? 16 : 32) + lane * 16;
-    wscale[j] = W8 ? scales[t * 16 + lr] : (half_t)0.f;
+    wsrc[j] = (const char*)Wp + (int64_t)t * K * 16 + lane * 16;
+    wscale[j] = scales[t * 16 + lr];
   }
 
   auto gload_x = [&](half8_t(&xr)[4], int kt) {
@@ -1232,17 +1230,10 @@ __global__ __launch_bounds__(TB_THREADS) void linear_tiled_big_kernel(
 #pragma unroll
     for (int i = 0; i < 4; ++i) xr[i] = *reinterpret_cast<const half8_t*>(xsrc[i] + kt * TB_BK);
   };
-  auto gload_w = [&](BigW<W8>& w, int kt) {
+  auto gload_w = [&](BigW& w, int kt) {
     kt = min(kt, nkt - 1);
 #pragma unroll
-    for (int j = 0; j < TB_NT; ++j) {
-      if (W8) {
-        w.f[0][j] = *reinterpret_cast<const half8_t*>(wsrc[j] + (int64_t)kt * 1024);
-      } else {
-        w.f[0][j] = *reinterpret_cast<const half8_t*>(wsrc[j] + (int64_t)kt * 2048);
-        w.f[W8 ? 0 : 1][j] = *reinterpret_cast<const half8_t*>(wsrc[j] + (int64_t)kt * 2048 + 1024);
-      }
-    }
+    for (int j = 0; j < TB_NT; ++j) w.f[j] = *reinterpret_cast<const half8_t*>(wsrc[j] + (int64_t)kt * 1024);
   };
   auto lstore = [&](const half8_t(&xr)[4], int buf) {
     half_t* l = lx_big + buf * (TB_BM * TB_LD);
@@ -1256,7 +1247,7 @@ __global__ __launch_bounds__(TB_THREADS) void linear_tiled_big_kernel(
 #pragma unroll
     for (int b = 0; b < TB_NT; ++b) acc[a][b] = float4_t{0.f, 0.f, 0.f, 0.f};
 
-  auto compute = [&](const BigW<W8>& w, int buf) {
+  auto compute = [&](const BigW& w, int buf) {
     // fragment f = 32-wide step f / TB_MF, row block f % TB_MF: chunk 4 * step + lg of row
     // 16 * block + lr, whose swizzle is (lr / 2) % 8 for every block
     const half_t* lb = lx_big + buf * (TB_BM * TB_LD) + lr * TB_LD;
@@ -1272,20 +1263,16 @@ __global__ __launch_bounds__(TB_THREADS) void linear_tiled_big_kernel(
     for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
       for (int j = 0; j < TB_NT; ++j) {
-        if (W8) {
-          const uint4 q = __builtin_bit_cast(uint4, w.f[0][j]);
-          a[ks][j] = ks == 0 ? dequant8(q.x, q.y, wscale[j]) : dequant8(q.z, q.w, wscale[j]);
-        } else {
-          a[ks][j] = w.f[W8 ? 0 : ks][j];
-        }
+        const uint4 q = __builtin_bit_cast(uint4, w.f[j]);
+        a[ks][j] = ks == 0 ? dequant8(q.x, q.y, wscale[j]) : dequant8(q.z, q.w, wscale[j]);
       }
     half8_t bx[TB_PD];
 #pragma unroll
     for (int p = 0; p < TB_PD; ++p)
       bx[p] = frag(p);
-    __builtin_amdgcn_sched_group_barrier(0x200, 4, 0);                         // LDS stores
-    __builtin_amdgcn_sched_group_barrier(0x020, 4 + (W8 ? 1 : 2) * TB_NT, 0);  // global loads
-    __builtin_amdgcn_sched_group_barrier(0x100, TB_PD, 0);                     // leading LDS reads
+    __builtin_amdgcn_sched_group_barrier(0x200, 4, 0);          // LDS stores
+    __builtin_amdgcn_sched_group_barrier(0x020, 4 + TB_NT, 0);  // global loads
+    __builtin_amdgcn_sched_group_barrier(0x100, TB_PD, 0);      // leading LDS reads
 #pragma unroll
     for (int f = 0; f < F; ++f) {
       const int ks = f / TB_MF, mf = f % TB_MF;
@@ -1302,7 +1289,7 @@ __global__ __launch_bounds__(TB_THREADS) void linear_tiled_big_kernel(
   };
 
   half8_t xr[4];
-  BigW<W8> w0, w1;
+  BigW w0, w1;
   gload_x(xr, 0);
   gload_w(w0, 0);
   lstore(xr, 0);
@@ -2752,7 +2739,7 @@ void launch_tiled(const void* x, const void* W, const void* scales, int64_t M, i
   }
   if constexpr (W8) if (K % (2 * TB_BK) == 0 && big_tiles >= num_cus()) {
     static std::atomic<uint64_t> lds_allowed{0};  // one mask per instantiation
-    if (!allow_lds((const void*)linear_tiled_big_kernel<W8, MODE>, TB_LDS_BYTES, lds_allowed))
+    if (!allow_lds((const void*)linear_tiled_big_kernel<MODE>, TB_LDS_BYTES, lds_allowed))
       return;  // the launch check below reports the error
     // A ragged bottom block would cost a full extra round of workgroups for a few rows (a
     // prompt of 2^k tokens plus the leading end-of-sentence token always has one): up to 128
@@ -2761,7 +2748,7 @@ void launch_tiled(const void* x, const void* W, const void* scales, int64_t M, i
     const int64_t rem = M % TB_BM;
     if (rem > 0 && rem <= 128 && M > rem) M_main = M - rem;
     const dim3 grid((N + TB_BN - 1) / TB_BN, (unsigned)((M_main + TB_BM - 1) / TB_BM));
-    hipLaunchKernelGGL((linear_tiled_big_kernel<W8, MODE>), grid, dim3(TB_THREADS), TB_LDS_BYTES,
+    hipLaunchKernelGGL((linear_tiled_big_kernel<MODE>), grid, dim3(TB_THREADS), TB_LDS_BYTES,
                        s, (const half_t*)x, W, (const half_t*)scales, M_main, N, K, epi);
     for (int64_t m0 = M_main; m0 < M; m0 += 64)
       launch_stream<W8, MODE, true>(x, W, scales, nullptr, 1, (int)min((int64_t)64, M - m0), N, K,
