@@ -1332,10 +1332,10 @@ __global__ __launch_bounds__(TB_THREADS) void linear_tiled_big_kernel(
 // address = scalar base + lane offset + the same instruction offset), so no load ever targets a
 // register and the only hand-placed waits are the vmcnt before each barrier:
 //   * activations in 64-wide stages (whole 128-byte lines), rows unpadded with their eight 16-byte
-//     chunks XOR-swizzled by (row / 2) % 8, ring of 3 x 32 KB;
+//     chunks XOR-swizzled by (row / 2) % 8, ring of 3 x 32 KB (256 rows);
 //   * weights in 32-wide steps, the packed 16 x 32 blocks as they lie in memory (lane order, so the
-//     fragment reads are linear), ring of 4 x 16 KB.
-// A group of loads (the 8 of a wave's share of a stage, the 4 of its share of a step) shares one
+//     fragment reads are linear), ring of 4 x 16 KB (256 columns).
+// A group of loads (the RF of a wave's share of a stage, the WF / 2 of its share of a step) shares one
 // M0 and one lane offset; the instruction offset picks the 1 KB piece, and the scalar bases, which
 // are loop invariant, are moved back by it.
 // One barrier per 32-wide step.  Behind the barrier of step t the weights of step t+1 (and, every
@@ -1365,9 +1365,17 @@ constexpr int tq_rw(int RF, int WF) { return 2 * (tq_rx(RF, WF) - 1); }
 constexpr int tq_xbytes(int RF) { return tq_bm(RF) * 64 * 2; }  // one 64-wide stage of activations
 constexpr int tq_bn(int WF) { return 32 * WF; }
 constexpr int tq_wbytes(int WF) { return 2 * WF * 1024; }  // one 32-wide step of weights
-constexpr int tq_lds_bytes(int WF, int RF = 8) {  // 160 / 128 / 112 KB; 144 KB with RF = 4
+// KB of columns x rows: 256 x 256 160, x 224 148, x 192 136, x 160 124, x 128 160; 128 x 256 128, x 224 160, x 192 144, x 160
+// 128, x 128 144; 64 x 256 112
+constexpr int tq_lds_bytes(int WF, int RF = 8) {
   return tq_rx(RF, WF) * tq_xbytes(RF) + tq_rw(RF, WF) * tq_wbytes(WF);
 }
+constexpr bool tq_lds_fits(int WF, int lo) {
+  for (int rf = lo; rf <= 8; ++rf)
+    if (tq_lds_bytes(WF, rf) > 160 * 1024) return false;
+  return true;
+}
+static_assert(tq_lds_fits(8, 4) && tq_lds_fits(4, 4) && tq_lds_fits(2, 8), "a CU has 160 KB of LDS");
 typedef __attribute__((address_space(3))) void tq_lds_void;
 
 template <int MODE>
@@ -1445,8 +1453,8 @@ struct GroupTiles {
 // PART: split-K.  Workgroup (bx, by, z) sums over the K range of ``part_stages`` 64-wide stages
 // that starts at stage z * part_stages and stores its fp32 sums, with no epilogue, as slice z of
 // ``part`` ([gridDim.z][M][N]); a later launch adds the slices in slice order.
+// m_own: the first row that the tile owns.
 template <int MODE, int WF, bool PART, bool GROUPED, int RF, bool FEW>
-// (m_own: the first row that this tile owns)
 __device__ __forceinline__ void quad_tile(const half_t* __restrict__ x, const void* __restrict__ Wp, int64_t M, int N,
                                           int K, int bx, int64_t m_own, int bz, const Epilogue& epi,
                                           float* __restrict__ part, int part_stages, const GroupTiles& gt) {
@@ -1470,11 +1478,11 @@ __device__ __forceinline__ void quad_tile(const half_t* __restrict__ x, const vo
   const int nst = PART ? part_stages : K / 64, nks = 2 * nst;
   const int ntiles = N / 16;
 
-  // direct loads.  Activations, per stage: instruction i (0..7) of the wave fills rows
-  // 64 * wave + 8 * i .. + 7 (lane l: row l / 8, chunk position l % 8, which must hold chunk
-  // (l % 8) ^ ((row / 2) % 8) = (l % 8) ^ (4 * (i % 2) + l / 16)), with M0 at the wave's piece
-  // + 4 KB and instruction offset 1024 * (i - 4).  Weights, per step: the wave copies the blocks
-  // of tiles 4 * wave .. 4 * wave + 3, instruction offset 1024 * j.
+  // direct loads.  Activations, per stage: instruction i (0 .. RF - 1) of the wave fills rows
+  // 8 RF * wave + 8 * i .. + 7 (lane l: row l / 8, chunk position l % 8, which must hold chunk
+  // (l % 8) ^ ((row / 2) % 8) = (l % 8) ^ (4 * (i % 2) + l / 16), or 4 * ((i + 1) % 2) where RF * wave is
+  // odd), with M0 at the wave's piece + RF / 2 KB and instruction offset 1024 * (i - RF / 2).  Weights, per
+  // step: the wave copies the blocks of tiles WL * wave .. WL * wave + WL - 1, instruction offset 1024 * j.
   const char* xb[XL];
   const char* wb[WL];
 #pragma unroll
@@ -1555,8 +1563,8 @@ __device__ __forceinline__ void quad_tile(const half_t* __restrict__ x, const vo
     tq_static_for<WL>([&](auto jc) { issue_w(jc); });
   };
 
-  // fragment reads.  Activation fragment i of half h of a stage: row 128 * wm + 16 * i + lr, chunk
-  // 4 * h + lg at position (4 * h + lg) ^ ((lr / 2) % 8); weight fragment j: tile 8 * wn + j.
+  // fragment reads.  Activation fragment i of half h of a stage: row 16 RF * wm + 16 * i + lr, chunk
+  // 4 * h + lg at position (4 * h + lg) ^ ((lr / 2) % 8); weight fragment j: tile WF * wn + j.
   const int sw = (lr >> 1) & 7;
   const uint32_t xoff0 = (uint32_t)(wm * (TQ_BM / 2) + lr) * 128 + ((lg ^ sw) * 16);
   const uint32_t xoff1 = (uint32_t)(wm * (TQ_BM / 2) + lr) * 128 + ((lg ^ sw ^ 4) * 16);
@@ -1578,8 +1586,8 @@ __device__ __forceinline__ void quad_tile(const half_t* __restrict__ x, const vo
       asm volatile("" : "+a"(acc[i][j]));
     }
 
-  // prologue: activation stages 0 and 1, weight steps 0..3 requested; stages 0, 1 and steps 0, 1
-  // landed
+  // prologue.  A ring of three stages: activation stages 0 and 1, weight steps 0..3 requested; stages 0, 1 and steps 0,
+  // 1 landed
   half8_t xf[2][RF], wf[2][WF];
   if constexpr (TQ_RX == 3) {
     group_x(0, 0);
@@ -1603,13 +1611,13 @@ __device__ __forceinline__ void quad_tile(const half_t* __restrict__ x, const vo
 #pragma unroll
   for (int j = 0; j < WF; ++j) wf[0][j] = wfrag(0, j);
 
-  // step t = 2 S + H; xs, ws: ring slots of stage S and step t.  An even step issues 8 + WL loads
-  // (stage S + 2, then step t + 4), an odd one WL (step t + 4).  Loads complete in order; the
-  // weights of step t + 1 were requested in step t - 3, and the 8 + 2 WL loads of steps t - 2 and
-  // t - 1 may still be outstanding at the barrier.  The activations an odd step starts to read
-  // (stage S + 1) were requested in step t - 3 as well, ahead of that step's weights.
-  // The 8 x WF MFMAs of a step carry, one each: the 8 + WF fragment reads of step t + 1 and the
-  // loads (even steps: activations under rows 0..3, weights under rows 4..7).
+  // step t = 2 S + H; xs, ws: ring slots of stage S and step t.  An even step issues RF + WL loads
+  // (stage S + TQ_RX - 1, then step t + TQ_RW), an odd one WL (step t + TQ_RW).  Loads complete in order; the weights
+  // of step t + 1 were requested TQ_RW - 1 steps ago, and the loads of the TQ_RW - 2 steps since may still be
+  // outstanding at the barrier, half of them with activations.  The activations an odd step starts to read
+  // (stage S + 1) were requested in the same step as its weights, ahead of them.
+  // The RF x WF MFMAs of a step carry, one each: the RF + WF fragment reads of step t + 1 and the
+  // loads (RF = 8, even steps: activations under rows 0..3, weights under rows 4..7).
   auto step = [&](int t, int xs, int ws, auto hc) {
     constexpr int H = decltype(hc)::value;
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"((TQ_RW - 2) / 2 * XL + (TQ_RW - 2) * WL) : "memory");
@@ -2363,7 +2371,11 @@ double quad_cost(int64_t tiles, int K, int cus) {  // 256 x 256 tiles, us
 }
 
 // The cheapest even cut of at least 256 rows (linear_quad_even_kernel): as many rows of tiles as fill whole rounds,
-// each of the height that is left for it, so that neither a round is left half empty nor a row of tiles.
+// each of the height that is left for it, so that neither a round is left half empty nor a row of tiles.  Up to 24 rounds
+// (100 of them are 0.01 % better) and 16384 rows (beyond, 0.7 % on average, for a choice of 3 us and more on the host;
+// 0.06 us at 300 rows, 0.2 at 2000, 0.5 at 5000).  Of 19200 products of eight widths from 768 to 9216 and 256 to 16384
+// rows 56 % are cut evenly; by columns x rows of the taller tiles, how often and what the price loses without them, on average and at most: 128
+// x 160 13 % (2.2, 53), x 192 3 (0.4, 24), x 224 3 (0.2, 12), 256 x 160 8 (0.8, 20), x 192 7 (0.6, 22), x 224 10 (0.6, 15), x 256 11 (0.2, 7).
 // Against tiles of one height (256 rows, or 128 x 128), us: 300 x 16384 x 4096 68 -> 50, 640 x 12288 x 4096 80 -> 67, 900 x
 // 16384 x 4096 110 -> 97, 1100 x 4096 x 4096 53 -> 40, 1260 x 4096 x 16384 201 -> 167, 1607 x 16384 x 4096 in a model 211 ->
 // 180, 2140 x 2048 x 8192 101 -> 75, 2460 x 4096 x 16384 328 -> 252, 1390 x 6144 x 2048 61 -> 37; 360 products of 66 ..

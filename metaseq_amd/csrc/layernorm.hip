@@ -265,7 +265,7 @@ extern "C" int msa_residual_layernorm_f16(const float* part, int S, const void* 
   if (rc) return rc;
   if (rows == 0) return MSA_OK;
   const int out_mb = (flags & MSA_OUT_PACKED) ? packed_row_blocks(rows) : 0;
-  // Two slices of more than 1024 rows, two chunks to a thread: eight rows to a CU at a time instead of four, us: 1030 x 4096
+  // Two slices of more than 1024 rows, two or three chunks to a thread: eight rows to a CU at a time instead of four, us: 1030 x 4096
   // 13.9 -> 12.6, 1607 21.6 -> 19.4, 2300 29.2 -> 26.7, 1607 x 5120 27.1 -> 25.6; x 7168 33.9 and 34.9.
   const bool many = rows > 1024 && S == 2 && D > 2048 && D <= 6144;
   auto pick = [&](auto threads) {
