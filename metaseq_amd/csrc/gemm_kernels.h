@@ -2694,6 +2694,8 @@ int pick_row_splits_f16(int64_t M, int N, int K) {
 // x 1024 (14.3, 17.3 and 2.5), whose one slice is taken in 256 x 64 tiles; 1000 x 4096 x 4096 43 against 37 and 3.
 // Where those tiles leave more than a quarter of the chip idle the clock is higher than the price's: up to K = 8192
 // one slice (2048 x 1408 x 4096 36 against 40 and 2; 1000 x 2560 x 10240 99 against 68 and 2).
+// (Rounds of whole tiles and of their pieces, at the costs below; the launch of either number of slices then takes the
+// cheapest form of quad_price, even cuts among them: 520 to 800 x 4096 x 4096 stay at one slice, 31 us, where two would take 28.)
 int pick_row_splits_f32(int64_t M, int N, int K) {
   const int few = pick_row_splits(M, N, K);
   if (few > 1 || M < TQ_BM || N % 16 || K % 128 || K < 1024) return few;
