@@ -807,7 +807,7 @@ extern "C" int msa_grouped_attention_splits(const msa_grouped_args* a, int M, in
 
 extern "C" int msa_grouped_attention_groups(const msa_grouped_args* a, const msa_batch* b, int seg0, int seg1,
                                             int longest) {
-  if (!a || !b || !b->host_start || !has_tiles(*a) || longest < 2 ||
+  if (!a || !b || !b->host_start || seg0 < 0 || seg1 > b->nseg || !has_tiles(*a) || longest < 2 ||
       2 * gf_lds(a->hd, a->vd) > GF_MOST_LDS)
     return 1;
   return wave_groups(*a, b, seg0, seg1, longest);

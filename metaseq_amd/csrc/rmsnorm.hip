@@ -28,8 +28,8 @@ __device__ __forceinline__ float dot4(float4_t v) {
 }
 
 // A row's weights are requested with the row where that is one float4 to a thread: behind its sum over the workgroup they are a
-// round trip with nothing beside it.  Of two and more they are read where they are used: kept through the
-// sums they take registers that are not there (a tail of two sublayers, 700 x 9216 146 -> 311 us, 700 x 8192 in fp32 18.7 -> 20.2).
+// round trip with nothing beside it.  Of more to a thread they hold up what is needed first, and kept through the sums they
+// can take registers that are not there (a tail of two sublayers, 700 x 9216 146 -> 311 us).
 template <int NV, int NT>
 __device__ __forceinline__ void row_weights(const float* w, int Dp, float4_t (&to)[NV]) {
   if (!w) return;  // uniform
@@ -142,9 +142,9 @@ __global__ __launch_bounds__(NT) void tail_kernel(msa_tail_args a) {
   const int D = a.D, Dp = a.Dp;
   float4_t b[NV], x[NV], w_post[NV], w_next[NV];
   // (few rows, 32 x 4096: 6.3 -> 6.0 us.  Two and four float4 to a thread only hold up the slices, 1500 x 4096 in two slices 22.9
-  // and 23.4: they are requested behind those, in front of the sums (16 x 8192 4.2 -> 4.1), but for what that costs more: two of
-  // one fp32 sublayer (700 x 8192 18.5 and 20.5), four of two sublayers (above).  A second sublayer's sums take the
-  // registers of the first form: 16 x 4096 4.3 and 4.5.)
+  // and 23.4: BEHIND requests them all at once behind those, the next norm's in front of its sum (16 x 8192 4.2 -> 4.1).
+  // Read where they are used: two of one fp32 sublayer (700 x 8192 18.5, so 20.5), four of two sublayers (above), and one
+  // of two sublayers, whose sums take its registers (16 x 4096 4.3, AHEAD 4.5).)
   constexpr bool AHEAD = NV == 1 && !TWO, BEHIND = NV == 2 ? TWO || sizeof(T) == 2 : NV == 4 && !TWO, GIVEN = AHEAD || BEHIND;
   if constexpr (AHEAD) {
     row_weights<NV, NT>(a.w_post, Dp, w_post);
