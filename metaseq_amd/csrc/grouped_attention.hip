@@ -674,7 +674,8 @@ bool run_decode(const msa_grouped_args& a, const msa_batch* b, int r0, int segs,
 // Groups of waves that share the key tiles of a tile of queries: two where a workgroup has a long list of key tiles and few
 // workgroups lie beside it, from 385 tokens on.  32 heads of 128, 8 of keys, one group and two, us: one segment of 512 tokens
 // 21.4 and 17.7, 1000 36.7 and 28.4, 2048 75.6 and 60.2.  More than two workgroups to a CU cover each other's
-// chains, and there the LDS of two groups costs: 3000 tokens 112 and 122, 8 x 300 31 and 38, 8 x 1000 154 and 174.
+// chains, and there the LDS of two groups costs: 3000 tokens 112 and 122, 8 x 300 31 and 38, 8 x 1000 154 and 174.  So it does
+// where most of them are those of short segments, which only begin and end: 1000 tokens beside 7 x 20 35 and 45.
 // The list is what a tile of 128 queries sees, a chunk at most.  Heads whose two groups leave room for no second workgroup
 // on a CU need eight key tiles to be ahead past a workgroup per CU: 64 heads of 128 in chunks of 64, 640 tokens 13.1 and
 // 18.7; 32 in chunks of 256, 2000 tokens 20.3 and 25.3; 64, 2 x 400 tokens (seven tiles) 23.8 and 26.5, 500 and 60 (eight) 20.9
@@ -684,7 +685,7 @@ bool run_decode(const msa_grouped_args& a, const msa_batch* b, int r0, int segs,
 // and 9.5, values of 192 10.4 and 10.5.
 constexpr int GF_MOST_LDS = 160 * 1024;
 int wave_groups(const msa_grouped_args& a, const msa_batch* b, int seg0, int seg1, int longest) {
-  if (longest <= 384) return 1;
+  if (longest <= 384 || (int64_t)a.heads * ((longest + GF_BM - 1) / GF_BM) * (seg1 - seg0) > 512) return 1;
   const int wide = a.chunk > GF_BM ? a.chunk : GF_BM, step = a.chunk < GF_BM ? a.chunk : GF_BM;
   bool aligned = a.chunk > 0 && wide % step == 0 && b->host_pos;  // query tiles begin with a chunk, or as many after one
   int64_t workgroups = 0;                                         // that have queries
@@ -696,7 +697,7 @@ int wave_groups(const msa_grouped_args& a, const msa_batch* b, int seg0, int seg
   const int64_t seen = a.chunk > 0 ? (int64_t)wide + (aligned ? 0 : step - 1) : longest;
   const int tiles = (int)(((seen < longest ? seen : longest) + GF_BN - 1) / GF_BN);
   if (tiles < 4 && (tiles == 2 ? a.vd > 128 : a.hd + a.vd > 192)) return 1;
-  return workgroups <= (tiles >= 8 || 4 * gf_lds(a.hd, a.vd) <= GF_MOST_LDS ? 512 : 256) ? 2 : 1;
+  return workgroups <= 256 || tiles >= 8 || 4 * gf_lds(a.hd, a.vd) <= GF_MOST_LDS ? 2 : 1;
 }
 
 template <int HD, int VD, int G>

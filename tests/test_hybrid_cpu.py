@@ -375,8 +375,8 @@ def test_arguments_are_checked_before_anything_is_launched():
 
 
 # ---------------------------------------------------------------- oracle pins
-# two groups of waves: long lists of keys and few workgroups; not where a chunk cuts the lists short under many workgroups, and
-# segments count as they are, not as the longest
+# two groups of waves: long lists of keys and few workgroups, those of short segments that begin and end at once among them; not
+# where the lists are short and more than a workgroup per CU has queries
 @pytest.mark.parametrize("heads,hd,vd,chunk,segs,groups", [
     (32, 128, 128, 0, [(0, 384)], 1), (32, 128, 128, 0, [(0, 385)], 2), (32, 128, 128, 0, [(0, 2048)], 2),
     (32, 128, 128, 0, [(0, 2049)], 1), (64, 128, 128, 64, [(0, 640)], 1), (64, 64, 128, 256, [(0, 640)], 1),
@@ -384,8 +384,10 @@ def test_arguments_are_checked_before_anything_is_launched():
     (64, 128, 128, 0, [(0, 400), (0, 400)], 1), (64, 64, 64, 64, [(0, 640)], 2), (16, 64, 128, 64, [(0, 640)], 2),
     (16, 128, 128, 64, [(0, 640)], 2), (16, 128, 128, 64, [(30, 640)], 1), (16, 64, 64, 64, [(30, 640)], 2),
     (16, 64, 192, 64, [(0, 640)], 1), (16, 128, 128, 48, [(0, 640)], 1), (32, 64, 192, 0, [(0, 640)], 2),
-    (32, 192, 192, 0, [(0, 640)], 1), (32, 128, 128, 0, [(0, 1000)] + [(0, 20)] * 7, 2),
-    (32, 128, 128, 0, [(0, 2000), (-1, 1000)], 2), (32, 128, 128, 0, [(0, 1100), (0, 1000)], 1)])
+    (32, 192, 192, 0, [(0, 640)], 1), (32, 128, 128, 0, [(0, 1000)] + [(0, 20)] * 7, 1),
+    (8, 128, 128, 0, [(0, 1000)] + [(0, 20)] * 7, 2), (32, 128, 128, 256, [(0, 1000), (-1, 1000)], 2),
+    (32, 128, 128, 0, [(0, 390)] + [(0, 20)] * 3, 2), (32, 128, 128, 0, [(0, 390)] * 3, 1),
+    (32, 128, 128, 0, [(0, 1100), (0, 1000)], 1)])
 def test_groups_of_waves_follow_the_keys_that_are_seen(heads, hd, vd, chunk, segs, groups):
     lib = _capi.load_hybrid()
     a, b = _capi.GroupedArgs(), _capi.Batch()
