@@ -412,7 +412,8 @@ __global__ __launch_bounds__(256 * G) void grouped_flash_kernel(msa_grouped_args
   const int h = a.kv_heads % 8 == 0 ? ((hi / per) * 8 + xcd) * per + hi % per : hi * 8 + xcd;
   if (h >= a.heads) return;
   const int g = h / per;
-  const int tid = threadIdx.x & 255, lane = tid & 63;
+  // (of one group the thread's number as it is: the mask alone changes the registers of the loop, 1000 tokens x 16 heads 34.1 -> 35.3 us)
+  const int tid = G > 1 ? threadIdx.x & 255 : threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int group = G > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
   char* lds = all_lds + group * 2 * TILE;
