@@ -933,10 +933,10 @@ __global__ __launch_bounds__(KL * NG * 64) void linear_share_kernel(
     constexpr int EMODE = MODE == MODE_SELECT ? MODE_PLAIN : MODE;
     // What the epilogue reads is requested for all row blocks at once, in front of the reduction (row by row behind it,
     // each block is a round trip; 57 rows x 12288 x 4096 24.0 and 23.6 us, 40 x 3072 x 1024 7.4 and 6.6).  Where there are
-    // registers for it and a reduction, one tile to a wave of up to four row blocks: of eight they spill, of two and three tiles they are
-    // taken from the loads in flight (int8, 40 rows in slices, 7168 x 28672 52.7 without and 56.8 with it, fp16 59 x 27648 x
-    // 9216 84.5 and 87.9).
-    constexpr bool AHEAD = MB <= 4 && !is_bf<EMODE> && NT == 1 && KL > 1;
+    // registers for it: of eight row blocks they spill; with two and three tiles to a wave, int8 weights or a cache to write to, they are
+    // taken from the loads in flight (int8, 40 rows in slices, 7168 x 28672 52.7 without and 56.8 with it, fp16 keys, values and
+    // queries of 59 x 9216 84.5 and 87.9), and fourteen waves of a tile each spill for the cache's places.
+    constexpr bool AHEAD = MB <= 4 && !is_bf<EMODE> && ((NT == 1 && KL > 1) || (EMODE == MODE_PLAIN && !W8));
     Ahead<EMODE> ahead[AHEAD ? MB : 1];
     auto look_ahead = [&](int t) {
       if (!AHEAD || part || kl > 0) return;
