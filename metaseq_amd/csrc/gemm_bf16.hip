@@ -6,9 +6,13 @@ namespace {
 
 template <int MODE>
 bool run_grouped(const msa_group_linear_args& a, const Epilogue& e, hipStream_t s) {
-  static std::atomic<uint64_t> lds_allowed{0};
-  auto kernel = linear_quad_kernel<MODE, 8, false, true>;
-  if (!allow_lds((const void*)kernel, tq_lds_bytes(8), lds_allowed)) return false;
+  static std::atomic<uint64_t> lds_allowed[2] = {};
+  // up to 64 rows to an expert on average: nearly all have one tile (320 tokens of 8 in 64 experts of 1408, width 4096, 274 ->
+  // 261 and 149 -> 144 us; 512 tokens 275 -> 276 and 160 -> 151)
+  const bool once = a.M <= (int64_t)a.groups * 64;
+  auto kernel = once ? linear_quad_kernel<MODE, 8, false, true, 8, false, true>
+                     : linear_quad_kernel<MODE, 8, false, true, 8, false, false>;
+  if (!allow_lds((const void*)kernel, tq_lds_bytes(8), lds_allowed[once])) return false;
   const int ncol = (a.N + tq_bn(8) - 1) / tq_bn(8);
   // the shares of the eight XCDs are rounded up: up to 7 workgroups beyond the tiles
   const GroupTiles gt{a.perm, a.tile_group, a.tile_row, a.n_tiles, a.group_end, a.rows_per_x};

@@ -1454,7 +1454,10 @@ struct GroupTiles {
 // that starts at stage z * part_stages and stores its fp32 sums, with no epilogue, as slice z of
 // ``part`` ([gridDim.z][M][N]); a later launch adds the slices in slice order.
 // m_own: the first row that the tile owns.
-template <int MODE, int WF, bool PART, bool GROUPED, int RF, bool FEW>
+// ONCE: one row of tiles (or experts of mostly one tile), so that a weight is read by one workgroup: its loads leave nothing in
+// the caches and are served faster (us: 200 x 50272 x 4096 101 -> 96, 100 x 50272 x 4096 84 -> 73, 70 x 16384 x 4096 43.9 -> 41.8,
+// eight slices of 200 x 4096 x 16384 41.5 -> 39.5; two rows of tiles would lose by it, 129 x 12288 x 4096 33.3 -> 39.3).
+template <int MODE, int WF, bool PART, bool GROUPED, int RF, bool FEW, bool ONCE = false>
 __device__ __forceinline__ void quad_tile(const half_t* __restrict__ x, const void* __restrict__ Wp, int64_t M, int N,
                                           int K, int bx, int64_t m_own, int bz, const Epilogue& epi,
                                           float* __restrict__ part, int part_stages, const GroupTiles& gt) {
@@ -1550,9 +1553,14 @@ __device__ __forceinline__ void quad_tile(const half_t* __restrict__ x, const vo
     const uint32_t vo = wv;
     const char* sb = wb[j];
     const uint32_t base = wm0;
-    asm volatile("global_load_lds_dwordx4 %0, %1 offset:%2" ::"v"(vo), "s"(sb), "n"(j * 1024),
-                 "{m0}"(base)
-                 : "memory");
+    if constexpr (ONCE)
+      asm volatile("global_load_lds_dwordx4 %0, %1 offset:%2 nt" ::"v"(vo), "s"(sb), "n"(j * 1024),
+                   "{m0}"(base)
+                   : "memory");
+    else
+      asm volatile("global_load_lds_dwordx4 %0, %1 offset:%2" ::"v"(vo), "s"(sb), "n"(j * 1024),
+                   "{m0}"(base)
+                   : "memory");
   };
   auto group_x = [&](int slot, int st) {
     set_x(slot, st);
@@ -1939,7 +1947,7 @@ __device__ __forceinline__ void quad_place(int t, int ncol, int nrow, int rm_a, 
   }
 }
 
-template <int MODE, int WF, bool PART = false, bool GROUPED = false, int RF = 8, bool FEW = false>
+template <int MODE, int WF, bool PART = false, bool GROUPED = false, int RF = 8, bool FEW = false, bool ONCE = false>
 __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
     const half_t* __restrict__ x, const void* __restrict__ Wp, int64_t M, int N, int K,
     int rm_a, int rm_r, Epilogue epi, float* __restrict__ part, int part_stages,
@@ -1964,10 +1972,10 @@ __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
   }
   const int64_t m_own = GROUPED ? g_first : (int64_t)by * tq_bm(RF);
   if constexpr (GROUPED) {  // a group's last tile is as high as its rows need (48304 rows in 64 groups x 2816 x 4096 1154 -> 1125 us)
-    if (M - m_own <= 128) return quad_tile<MODE, WF, PART, true, 4, FEW>(x, Wp, M, N, K, bx, m_own, 0, epi, part, 0, gt);
-    if (M - m_own <= 192) return quad_tile<MODE, WF, PART, true, 6, FEW>(x, Wp, M, N, K, bx, m_own, 0, epi, part, 0, gt);
+    if (M - m_own <= 128) return quad_tile<MODE, WF, PART, true, 4, FEW, ONCE>(x, Wp, M, N, K, bx, m_own, 0, epi, part, 0, gt);
+    if (M - m_own <= 192) return quad_tile<MODE, WF, PART, true, 6, FEW, ONCE>(x, Wp, M, N, K, bx, m_own, 0, epi, part, 0, gt);
   }
-  quad_tile<MODE, WF, PART, GROUPED, RF, FEW>(x, Wp, M, N, K, bx, m_own, blockIdx.z, epi, part, part_stages, gt);
+  quad_tile<MODE, WF, PART, GROUPED, RF, FEW, ONCE>(x, Wp, M, N, K, bx, m_own, blockIdx.z, epi, part, part_stages, gt);
 }
 
 // Tiles that would begin a round without filling half of it, in pieces: the first n_full tiles (of all K slices, whole
@@ -2488,12 +2496,14 @@ void launch_quad(const void* x, const void* W, const void* scales, int64_t M, in
   } else if (pieces == 2) {
     launch_quad_pieces<MODE, false, 2>(x, W, M_main, N, K, 1, epi, nullptr, s);
   } else {
-    static std::atomic<uint64_t> lds_allowed_q{0};
-    if (!allow_lds((const void*)linear_quad_kernel<MODE, WF>, tq_lds_bytes(WF), lds_allowed_q)) return;
+    static std::atomic<uint64_t> lds_allowed_q[2] = {};
+    auto kernel = nrow == 1 ? linear_quad_kernel<MODE, WF, false, false, 8, false, true>
+                            : linear_quad_kernel<MODE, WF, false, false, 8, false, false>;
+    if (!allow_lds((const void*)kernel, tq_lds_bytes(WF), lds_allowed_q[nrow == 1])) return;
     const TileOrder o = tile_order(ncol, nrow, WF);
-    hipLaunchKernelGGL((linear_quad_kernel<MODE, WF>), quad_grid(ncol, nrow, o), dim3(TQ_THREADS),
+    hipLaunchKernelGGL(kernel, quad_grid(ncol, nrow, o), dim3(TQ_THREADS),
                        tq_lds_bytes(WF), s, (const half_t*)x, W, M_main, N, K, o.a, o.r, epi,
-                       (float*)nullptr, 0);
+                       (float*)nullptr, 0, GroupTiles{});
   }
   for (int64_t m0 = M_main; m0 < M; m0 += 64)
     launch_stream<false, MODE, true>(x, W, scales, nullptr, 1, (int)min((int64_t)64, M - m0), N,
@@ -2513,10 +2523,11 @@ void launch_quad(const void* x, const void* W, const void* scales, int64_t M, in
 //   106 -> 86, 129 106 -> 89, 170 111 -> 95, 200 111 -> 101.
 template <int MODE, int WF, int RF>
 void launch_few_rows(const void* x, const void* W, int64_t M, int N, int K, const Epilogue& epi, hipStream_t s) {
-  static std::atomic<uint64_t> lds_allowed_s{0};
-  auto kernel = linear_quad_kernel<MODE, WF, false, false, RF, true>;
-  if (!allow_lds((const void*)kernel, tq_lds_bytes(WF, RF), lds_allowed_s)) return;
+  static std::atomic<uint64_t> lds_allowed_s[2] = {};
   const int ncol = (N + tq_bn(WF) - 1) / tq_bn(WF), nrow = (int)((M + tq_bm(RF) - 1) / tq_bm(RF));
+  auto kernel = nrow == 1 ? linear_quad_kernel<MODE, WF, false, false, RF, true, true>
+                          : linear_quad_kernel<MODE, WF, false, false, RF, true, false>;
+  if (!allow_lds((const void*)kernel, tq_lds_bytes(WF, RF), lds_allowed_s[nrow == 1])) return;
   const TileOrder o{nrow == 1 ? 0 : -TQ_PANEL, 0};
   hipLaunchKernelGGL(kernel, quad_grid(ncol, nrow, o), dim3(TQ_THREADS), tq_lds_bytes(WF, RF), s, (const half_t*)x, W,
                      M, N, K, o.a, o.r, epi, (float*)nullptr, 0, GroupTiles{});
@@ -2528,11 +2539,12 @@ void launch_few_rows(const void* x, const void* W, int64_t M, int N, int K, cons
 template <int MODE, int WF>
 void launch_quad_partial_w(const void* x, const void* W, float* part, int64_t M, int N, int K,
                            int S, hipStream_t s) {
-  static std::atomic<uint64_t> lds_allowed_p{0};
-  auto kernel = linear_quad_kernel<MODE, WF, true>;
-  if (!allow_lds((const void*)kernel, tq_lds_bytes(WF), lds_allowed_p)) return;
+  static std::atomic<uint64_t> lds_allowed_p[2] = {};
   const int ncol = (N + tq_bn(WF) - 1) / tq_bn(WF);
   const int nrow = (int)((M + TQ_BM - 1) / TQ_BM);
+  auto kernel = nrow == 1 ? linear_quad_kernel<MODE, WF, true, false, 8, false, true>
+                          : linear_quad_kernel<MODE, WF, true, false, 8, false, false>;
+  if (!allow_lds((const void*)kernel, tq_lds_bytes(WF), lds_allowed_p[nrow == 1])) return;
   Epilogue e{};
   const TileOrder o = tile_order(ncol, nrow, WF);
   hipLaunchKernelGGL(kernel, quad_grid(ncol, nrow, o, S), dim3(TQ_THREADS), tq_lds_bytes(WF), s,

@@ -68,7 +68,11 @@ __device__ __forceinline__ void store4(const msa_group_linear_args& a, int group
 
 // MT row blocks of 16 per workgroup, NT column tiles per wave, KW waves share a column range and
 // split K, U 32-wide steps per stage.
-template <int MT, int NT, int KW, int U, bool GLU>
+// Bound: the weights' way from memory.  ONCE: hardly a weight is read by two workgroups, and loads that leave nothing in the
+// caches are served faster (64 experts of 1408, width 4096, 16 rows to an expert's tile, us: 1 token 33.4 -> 29.7 and 16.2 ->
+// 15.4, 16 tokens 198 -> 179 and 101 -> 90, which is 6.9 TB/s; 128 tokens, where every second expert has two such tiles, would
+// take 464 for 398).  Routed tiles are taken for that while the groups' mean is half a tile.
+template <int MT, int NT, int KW, int U, bool GLU, bool ONCE>
 __global__ __launch_bounds__(256) void group_linear_bf16_kernel(msa_group_linear_args a) {
   constexpr int NW = 4 / KW;  // waves side by side over the columns
   __shared__ float4_t red[KW > 1 ? KW : 1][KW > 1 ? NW * MT * NT : 1][64];
@@ -107,8 +111,10 @@ __global__ __launch_bounds__(256) void group_linear_bf16_kernel(msa_group_linear
     for (int u = 0; u < U; ++u) {
       const int ks = min((idx * U + u) * KW + kw, nks - 1);
 #pragma unroll
-      for (int j = 0; j < NT; ++j)
-        st.w[u][j] = *reinterpret_cast<const half8_t*>(wp[j] + (int64_t)ks * 512);
+      for (int j = 0; j < NT; ++j) {
+        const half8_t* w = reinterpret_cast<const half8_t*>(wp[j] + (int64_t)ks * 512);
+        st.w[u][j] = ONCE ? __builtin_nontemporal_load(w) : *w;
+      }
 #pragma unroll
       for (int i = 0; i < MT; ++i)
         st.x[u][i] = *reinterpret_cast<const half8_t*>(xp[i] + ks * kstep);
@@ -176,10 +182,12 @@ template <int MT, int NT, int KW, int U>
 void launch_bf16(const msa_group_linear_args& a, int row_tiles, hipStream_t s) {
   constexpr int NB = 4 / KW * NT;
   const dim3 grid((a.N / 16 + NB - 1) / NB, row_tiles, a.tile_group ? 1 : a.groups);
-  if (a.glu == MSA_GLU_NONE)
-    hipLaunchKernelGGL((group_linear_bf16_kernel<MT, NT, KW, U, false>), grid, dim3(256), 0, s, a);
-  else
-    hipLaunchKernelGGL((group_linear_bf16_kernel<MT, NT, KW, U, true>), grid, dim3(256), 0, s, a);
+  const bool glu = a.glu != MSA_GLU_NONE, once = a.tile_group ? a.M * 2 <= (int64_t)a.groups * a.tile_rows : row_tiles == 1;
+  auto kernel = once ? (glu ? group_linear_bf16_kernel<MT, NT, KW, U, true, true>
+                            : group_linear_bf16_kernel<MT, NT, KW, U, false, true>)
+                     : (glu ? group_linear_bf16_kernel<MT, NT, KW, U, true, false>
+                            : group_linear_bf16_kernel<MT, NT, KW, U, false, false>);
+  hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, a);
 }
 
 // ---- fp32 -----------------------------------------------------------------------------------
@@ -292,7 +300,13 @@ extern "C" int msa_group_linear(const msa_group_linear_args* args, void* stream)
                                                routed ? 1 : a.groups),
                        dim3(256), 0, s, a, (float*)nullptr, a.N, PostF32{});
   } else if (rows <= 16) {
-    launch_bf16<1, 2, 4, 4>(a, (int)row_tiles, s);
+    // a stage is 16 steps of K, or 8 where those leave fewer empty ones of a short sum (K = 704, 64 experts, 64 rows of 2048
+    // columns each 40.6 -> 29.4 us)
+    const int nks = a.K / 32;
+    if (a.K < 1024 && (nks + 7) / 8 * 8 < (nks + 15) / 16 * 16)
+      launch_bf16<1, 2, 4, 2>(a, (int)row_tiles, s);
+    else
+      launch_bf16<1, 2, 4, 4>(a, (int)row_tiles, s);
   } else if (rows <= 32) {
     launch_bf16<2, 2, 4, 2>(a, (int)row_tiles, s);
   } else if (a.N <= 128 || (!routed && a.M <= 128)) {

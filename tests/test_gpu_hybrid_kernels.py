@@ -556,6 +556,45 @@ def test_group_linear_routed_tiles_as_high_as_the_rows(N, K, kind):
         first += count
 
 
+# groups whose mean is up to half a tile (their weights pass by the caches) and beyond, some of two tiles, in all heights of tiles;
+# sums whose last stage of 16 or 8 steps is full, nearly empty or the only one
+@pytest.mark.parametrize("rows", [16, 32, 64, 256])
+@pytest.mark.parametrize("dense", [False, True])
+@pytest.mark.parametrize("N,K", [(288, 704), (160, 128), (96, 1088)])
+def test_group_linear_routed_tiles_read_once_or_often(rows, dense, N, K):
+    lib = _capi.load_hybrid()
+    print("routed", rows, dense, N, K, flush=True)
+    g = gen(N + rows)
+    counts = [0, 1, rows - 1, rows, rows + 1] + [2] * 9 + [rows] * (20 if dense else 0)
+    E, P = len(counts), sum(counts)
+    limit = 64 if rows == 256 else rows / 2
+    assert (P > E * limit) == dense
+    flat = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(P, generator=g)]
+    x = torch.randn(P, K, generator=g).to(BF16)
+    w = (torch.randn(E, N, K, generator=g) * K ** -0.5).to(BF16)
+    n_max = P // rows + E
+    ids = flat.int().cuda()
+    perm, inv = (torch.full((P,), -1, dtype=torch.int32, device="cuda") for _ in range(2))
+    end, n = torch.zeros(E, dtype=torch.int32, device="cuda"), torch.zeros(1, dtype=torch.int32, device="cuda")
+    tg, tr = (torch.full((n_max,), -1, dtype=torch.int32, device="cuda") for _ in range(2))
+    check(lib.msa_moe_plan(ptr(ids), P, E, rows, ptr(perm), ptr(inv), ptr(end), ptr(tg), ptr(tr), ptr(n), n_max,
+                           _capi.stream_ptr()), lib)
+    xd, wd = x.cuda(), pack_tiles(w.view(E * N, K)).cuda()
+    y = torch.full((P + 1, N), 7.0, dtype=BF16, device="cuda")
+    a = _capi.GroupLinearArgs()
+    a.dtype, a.glu = 0, -1
+    a.x, a.ldx, a.W, a.y, a.ldy = ptr(xd), K, ptr(wd), ptr(y), N
+    a.N, a.K, a.groups, a.M = N, K, E, P
+    a.perm, a.tile_group, a.tile_row, a.n_tiles, a.group_end = ptr(perm), ptr(tg), ptr(tr), ptr(n), ptr(end)
+    a.rows_per_x, a.max_tiles, a.tile_rows = 1, n_max, rows
+    check(lib.msa_group_linear(ctypes.byref(a), _capi.stream_ptr()), lib)
+    torch.cuda.synchronize()
+    assert bool((y[P] == 7.0).all()), "wrote past the last row"
+    order = torch.sort(flat, stable=True).indices
+    ref = torch.stack([x[p].double() @ w[flat[p]].double().T for p in order.tolist()])
+    close(y[:P], ref, 6e-3, "rows %d" % rows)
+
+
 @pytest.mark.parametrize("E,groups,keep,top", [(1, 1, 1, 1), (12, 1, 1, 5), (12, 4, 2, 3),
                                                (96, 8, 3, 10), (512, 16, 16, 8), (300, 100, 1, 3)])
 def test_route_and_plan(E, groups, keep, top):
