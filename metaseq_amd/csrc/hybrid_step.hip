@@ -49,6 +49,28 @@ struct Act {
   int ld, n;
 };
 
+// Rows to a tile of the routed products (bf16; P pairs over E experts, hidden size ff).  What counts is that hardly an
+// expert has two tiles, whose weights are then read twice, and how fast a tile's kernel reads them: tiles of 16 rows at 6.9
+// TB/s, of 64 at 5 to 6, the 256-row kernel, whose tiles are as high as an expert's rows need, at 5.5 to 5.8.  Both products of
+// 64 experts of 1408, width 4096, us, by tokens of which each has eight experts: 48 tokens in tiles of 16 rows 346, of 64 383; 64
+// tokens 374, 393; 96 tokens 459, 412; 128 tokens 543 (of 32 rows 537), 437; 160 tokens of 32 rows 445, 64 413, 256 389; 256
+// tokens of 32 rows 583, 64 462, 256 395; 320 tokens of 64 506, 256 404; 512 tokens 760, 427.  (Packed rows are no input of the
+// 256-row kernel, and 16 of them gathered into a fragment are four times the lines of row-major ones: tiles of 32 gain nothing.)
+// Up to 2048 wide an expert's product is short, and row-major tiles of 32 are ahead for longer: 150 tokens 109, of 256 120; 200
+// tokens 121, 121; 260 tokens 150, 122.
+// Where there are fewer tiles than compute units (256 columns each from 64 rows on), low tiles have more workgroups to
+// spread the rows over: experts of 128, width 512, 140 tokens 11.2 in tiles of 16, 23 of 64 and 26 of 256.
+int routed_rows(int P, int E, int width, int ff, bool packed) {
+  const int avg = P / E;
+  if ((int64_t)(E < P ? E : P) * ((2 * ff + 255) / 256) < 256)
+    return avg <= 16 ? 16 : avg <= 32 ? 32 : avg <= 64 || packed ? 64 : 256;
+  if (P <= 8 * (int64_t)E) return 16;
+  if (packed) return 64;
+  if (width <= 2048 && avg <= 24) return 32;
+  const int64_t K = width > ff ? width : ff;
+  return avg <= 16 || (avg <= 64 && P * K * 2 >= (1ll << 32)) ? 64 : 256;
+}
+
 struct Run {
   const msa_hybrid* d;
   const msa_hybrid_step_args* a;
@@ -465,8 +487,7 @@ int Run::feed_forward(const msa_hybrid_layer& l, msa_tail_args& t) {
   // the shared expert's hidden layer, the router logits and the shared gate's logit in one product
   HY(linear(h, l.w_ff_in, u.p, true, z, l.n_ff_in, n32, shared ? MSA_GLU_CLAMPED : MSA_GLU_NONE,
             l.limit_shared));
-  const int avg = P / E, tile_rows = f32 ? 64 : avg <= 16 ? 16 : avg <= 32 ? 32
-                                                 : avg <= 64 || mb > 0 ? 64 : 256;
+  const int tile_rows = f32 ? 64 : routed_rows(P, E, c.Dp, l.ff_expert, mb > 0);
   const int max_tiles = P / tile_rows + (E < P ? E : P);
   int32_t* ids = (int32_t*)alloc((int64_t)P * 4);
   float* w = (float*)alloc((int64_t)P * 4);
