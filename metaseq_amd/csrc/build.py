@@ -16,13 +16,13 @@ LIBS = {"core": os.path.join(HERE, "libmetaseq_amd.so"),
         "hybrid": os.path.join(HERE, "libmetaseq_hybrid.so")}
 LIB = LIBS["core"]
 SOURCES = {
-    "core": ["capi.hip", "layernorm.hip", "embed.hip", "gemm.hip", "attention.hip",
+    "core": ["capi.hip", "layernorm.hip", "embed.hip", "gemm.hip", "gemm_queue_f16.hip", "gemm_queue_i8.hip", "attention.hip",
              "attention_prefill.hip", "sampling.hip", "probe.hip", "decoder_step.hip"],
-    "hybrid": ["capi.hip", "gemm_bf16.hip", "gemm_bf16_post.hip", "group_linear.hip", "moe.hip",
+    "hybrid": ["capi.hip", "gemm_bf16.hip", "gemm_bf16_post.hip", "gemm_queue_bf16.hip", "group_linear.hip", "moe.hip",
                "rmsnorm.hip", "recurrent.hip", "delta_chunks.hip", "latent_attention.hip",
                "grouped_attention.hip", "hybrid_step.hip"],
 }
-HEADERS = ["common.h", "gemm_kernels.h", "attention_tiles.h",
+HEADERS = ["common.h", "gemm_kernels.h", "gemm_queue.h", "attention_tiles.h",
            os.path.join("..", "..", "include", "metaseq_amd.h"),
            os.path.join("..", "..", "include", "metaseq_hybrid.h")]
 # (the last flag: a kernel's first fourteen argument words are in registers when a wave starts, where it would read them

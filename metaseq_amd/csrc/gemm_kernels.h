@@ -37,8 +37,6 @@
 
 #include "common.h"
 
-namespace {
-
 enum { MODE_PLAIN = 0, MODE_QKV = 1, MODE_SELECT = 2, MODE_BF = 3, MODE_BF_GLU = 4, MODE_BF_POST = 5 };
 // The bf16 modes: operands are bf16 bit patterns (the kernels only move them; what differs is the
 // MFMA instruction and the epilogue).  Columns below Epilogue::n32 are stored as bf16, the columns
@@ -83,6 +81,8 @@ struct Epilogue {
   bf16_t* y2;               // bf16 columns from n2 on: row-major with stride ld2, or packed (out2_mb)
   int act, n2, ld2, out2_mb;
 };
+
+namespace {
 
 // what MODE_BF_POST does to the sums of columns n .. n + 3, and the vectors it takes for them
 struct PostVectors {
@@ -2149,10 +2149,29 @@ void launch_share_cfg(const void* xp, const void* W, const void* scales, float* 
                      (const half_t*)scales, part, M, N, K, tiles_per_wg, ks_per_split, epi);
 }
 
-// 33 .. 64 packed rows (a vocabulary: from one row on, selections too): the shared-activation kernel.  16-bit weights of
-// one to three tiles per workgroup take a wave per tile and K lane: 12288 x 4096 (three tiles) at 40 / 64 rows 23.7 /
-// 25.6 us on 2 x 4 waves, 21.7 / 23.7 on 4 x 3; 8192 x 2048 (two) 13.0 / 14.0 and 10.7 / 12.0 on 4 x 2; 3072 x 768 and
-// 3072 x 1024 (one) 7.9 / 8.3 and 6.1 / 7.0 on 8 x 1.  Four tiles are as fast either way, int8 weights slower.
+// Tiles of a workgroup that the queue kernel takes: up to nine, as many as fit its sums beside their rows.  Up to 32 rows only from five
+// tiles on, of int8 weights or two row blocks: the stream kernel loads four tiles' operands in one pass and does not go through
+// LDS (us, stream and queue: 16384 x 4096, 32 rows 24.5 and 25, int8 17.3 and 18.2, 8 rows int8 16.9 and 18.1; five tiles int8
+// 8 x 20480 x 5120 23.0 and 18.6; fp16 of one row block, seven tiles, 62.0 and 62.6).
+constexpr int QUEUE_TILES = 9;
+constexpr int queue_rows(int M) {  // row blocks that it multiplies: 65 .. 96 rows leave two of the eight out
+  return M > 96 ? 8 : M > 64 ? 6 : (M + 15) / 16;
+}
+constexpr bool queue_takes(int M, bool w8, int tiles_per_wg) {
+  const int mb = queue_rows(M);
+  if (tiles_per_wg > QUEUE_TILES || mb * tiles_per_wg > 64) return false;  // 64: QueueCfg::OK
+  return mb > 2 || (tiles_per_wg >= 5 && (w8 || mb == 2));
+}
+
+}  // namespace
+// (gemm_queue.h; compiled in files of its own, gemm_queue_*.hip)
+template <bool W8, int MODE>
+void launch_queue(const void* xp, const void* W, const void* scales, float* part, int S, int M, int N, int K,
+                  int tiles_per_wg, const Epilogue& epi, hipStream_t s);
+namespace {
+
+// The shared-activation kernel: 33 .. 64 packed rows of more tiles than the queue kernel takes, and vocabularies from one row on,
+// selections too (any number of tiles is right, in as many passes).
 template <int MB, bool W8, int MODE>
 void launch_share(const void* xp, const void* W, const void* scales, float* part, int S, int M,
                   int N, int K, const Epilogue& epi, hipStream_t s) {
@@ -2163,53 +2182,26 @@ void launch_share(const void* xp, const void* W, const void* scales, float* part
   const int gx = (ntiles + tiles_per_wg - 1) / tiles_per_wg;
   int ks_per_split = (nks + S - 1) / S;
   if (W8) ks_per_split = (ks_per_split + 1) & ~1;  // int8 blocks cover two steps
-  // the wave grid and tiles per wave whose slots the workgroup's tiles fill best in one pass
-  if constexpr (W8) {
-    if (tiles_per_wg == 5 || tiles_per_wg == 6)
-      return launch_share_cfg<MB, W8, MODE, 4, 3, 2, 2, 2>(xp, W, scales, part, S, M, N, K,
-                                                        tiles_per_wg, gx, ks_per_split, epi, s);
-    if (tiles_per_wg == 9)
-      return launch_share_cfg<MB, W8, MODE, 4, 3, 3, 2, 2>(xp, W, scales, part, S, M, N, K,
-                                                        tiles_per_wg, gx, ks_per_split, epi, s);
-    if (tiles_per_wg > 12 && tiles_per_wg <= 18)
-      return launch_share_cfg<MB, W8, MODE, 2, 6, 3, 2, 3>(xp, W, scales, part, S, M, N, K,
-                                                        tiles_per_wg, gx, ks_per_split, epi, s);
-  } else {
-#define SH_RUN(...)                                                                                           \
-  return launch_share_cfg<MB, W8, MODE, __VA_ARGS__>(xp, W, scales, part, S, M, N, K, tiles_per_wg, gx, \
-                                                     ks_per_split, epi, s)
-    // (few rows and selections come here for vocabularies only; any number of tiles is right, in as many passes)
-    if (MB <= 2 || MODE == MODE_SELECT || vocabulary_tiles(tiles_per_wg)) SH_RUN(1, 14, 1, 4);
-    if constexpr (MB > 2 && MODE != MODE_SELECT) {
-      if (tiles_per_wg == 1) SH_RUN(8, 1, 1, 2);
-      if (tiles_per_wg == 2) SH_RUN(4, 2, 1, 4);
-      if (tiles_per_wg == 3) SH_RUN(4, 3, 1, 2);
-    }
-#undef SH_RUN
+  if constexpr (!W8) {
+    if (MB <= 2 || MODE == MODE_SELECT || vocabulary_tiles(tiles_per_wg))
+      return launch_share_cfg<MB, W8, MODE, 1, 14, 1, 4>(xp, W, scales, part, S, M, N, K, tiles_per_wg, gx, ks_per_split,
+                                                         epi, s);
   }
   if constexpr (MB > 2 && MODE != MODE_SELECT) {
-    if (tiles_per_wg <= 4)
-      launch_share_cfg<MB, W8, MODE, 2, 4, 1, 8>(xp, W, scales, part, S, M, N, K, tiles_per_wg, gx,
-                                                 ks_per_split, epi, s);
-    else if (tiles_per_wg <= 8)
-      launch_share_cfg<MB, W8, MODE, 2, 4, 2, 4>(xp, W, scales, part, S, M, N, K, tiles_per_wg, gx,
-                                                 ks_per_split, epi, s);
-    else
-      launch_share_cfg<MB, W8, MODE, 2, 4, 3, 4>(xp, W, scales, part, S, M, N, K, tiles_per_wg, gx,
-                                                 ks_per_split, epi, s);
+    if constexpr (W8) {
+      if (tiles_per_wg > 12 && tiles_per_wg <= 18)
+        return launch_share_cfg<MB, W8, MODE, 2, 6, 3, 2, 3>(xp, W, scales, part, S, M, N, K, tiles_per_wg, gx,
+                                                             ks_per_split, epi, s);
+    }
+    launch_share_cfg<MB, W8, MODE, 2, 4, 3, 4>(xp, W, scales, part, S, M, N, K, tiles_per_wg, gx, ks_per_split, epi, s);
   } else {
     static_assert(!W8, "int8 weights of so few rows stream");
   }
 }
 
-// 65 .. 128 packed rows (eight row blocks): the shared-activation kernel as 2 K lanes x 4 tile
-// lanes with stages of four K steps (32 KB of activations per stage; two stages and the
-// reduction buffer make 96 KB of LDS).  With so many rows per weight fragment the tiles of a
-// workgroup are few per wave, so more weight stages are kept in flight instead (PF).  Measured
-// at 128 x 12288 x 4096 (38.6 us as built): four K lanes x two tile lanes x two tiles 45.8 us,
-// stages of eight K steps 43.0, six weight stages in flight instead of four 44.3.  16-bit weights: a vocabulary a
-// wave per tile (50272 x 4096 at 128 rows 116 -> 95); four tiles in stages of eight K steps, two weight stages in
-// flight and all 160 KB (16384 x 4096 38.3 -> 36.3).
+// 65 .. 128 packed rows (eight row blocks) of more tiles than the queue kernel takes: the shared-activation kernel as 2 K
+// lanes x 4 tile lanes with stages of two K steps; a vocabulary of 16-bit weights a wave per tile (50272 x 4096 at 128 rows
+// 116 -> 95 us).
 template <bool W8, int MODE>
 void launch_wide(const void* xp, const void* W, const void* scales, float* part, int S, int M,
                  int N, int K, const Epilogue& epi, hipStream_t s) {
@@ -2230,19 +2222,8 @@ void launch_wide(const void* xp, const void* W, const void* scales, float* part,
                                   : launch_share_cfg<8, W8, MODE, 1, 14, 1, 2>(xp, W, scales, part, S, M, N, K,
                                                                                tiles_per_wg, gx, ks_per_split, epi, s);
     }
-    if (tiles_per_wg == 4)
-      return launch_share_cfg<8, W8, MODE, 2, 4, 1, 4>(xp, W, scales, part, S, M, N, K, tiles_per_wg, gx,
-                                                       ks_per_split, epi, s);
   }
-  if (tiles_per_wg <= 4)
-    launch_share_cfg<8, W8, MODE, 2, 4, 1, 2, 4>(xp, W, scales, part, S, M, N, K, tiles_per_wg, gx,
-                                                 ks_per_split, epi, s);
-  else if (tiles_per_wg <= 8)
-    launch_share_cfg<8, W8, MODE, 2, 4, 2, 2, 3>(xp, W, scales, part, S, M, N, K, tiles_per_wg, gx,
-                                                 ks_per_split, epi, s);
-  else
-    launch_share_cfg<8, W8, MODE, 2, 4, 3, 2, 2>(xp, W, scales, part, S, M, N, K, tiles_per_wg, gx,
-                                                 ks_per_split, epi, s);
+  launch_share_cfg<8, W8, MODE, 2, 4, 3, 2, 2>(xp, W, scales, part, S, M, N, K, tiles_per_wg, gx, ks_per_split, epi, s);
 }
 
 // the tail in front of a product of at most LN_MAX_ROWS rows (S = 1, 2 or 4 slices); false: the LDS was refused
@@ -2280,6 +2261,8 @@ template <bool W8, int MODE, bool XR = false>
 void launch_stream(const void* xp, const void* W, const void* scales, float* part, int S, int M,
                    int N, int K, const Epilogue& epi, hipStream_t s, int64_t m_off = 0) {
   if constexpr (!XR && MODE != MODE_SELECT) {
+    const int G = num_cus() / S < 1 ? 1 : num_cus() / S, tpw = (N / 16 + G - 1) / G;
+    if (queue_takes(M, W8, tpw)) return launch_queue<W8, MODE>(xp, W, scales, part, S, M, N, K, tpw, epi, s);
     if (M > 64) return launch_wide<W8, MODE>(xp, W, scales, part, S, M, N, K, epi, s);
   }
   if constexpr (!XR && !W8) {
@@ -2817,23 +2800,33 @@ int check_linear_args(const char* name, const void* x, const void* W, const void
 // its K range, the activation fragments of that K range once per tile group, and its fp32
 // partial sums (written here, read back by the LayerNorm tail).  More splits mean more tiles
 // per workgroup over a shorter K range, i.e. fewer activation bytes per weight byte.  At most `most` slices.
+// In the queue kernel activations, which come from L2, cost half of as many weights, and a tile's sums more than the bytes they
+// leave as: eight waves' go through LDS behind the loop.  Fitted to 130 products of 40 to 128 rows with their tails (us = 5 +
+// 0.0278 per KB of weights + 0.0126 per KB of activations + 0.18 per 16 x 16 sums + 0.14 per 1000 of slices x columns, to 4.5 %);
+// what it picks is 0.7 % slower than the best of 2, 4 and 8 slices on average.
 int pick_splits(int64_t M, int N, int K, int wbytes, int most = 8) {
   if (M < 1 || M > MSA_PACKED_MAX_ROWS || N % 16 || K % 64) return 1;
+  const bool w8 = wbytes == 1;
   const int MB = packed_row_blocks(M), ntiles = N / 16, nks = K / 32;
-  // tiles that share one sweep over the activations (int8 has a 2 x 6 x 3 shape of the
+  // elsewhere: tiles that share one sweep over the activations (int8 has a 2 x 6 x 3 shape of the
   // shared-activation kernel for up to 18), and K steps per stage of the workgroup
-  const int NT = MB > 2 ? (wbytes == 1 && MB <= 4 ? SH_GROUP_W8 : SH_GROUP) : ST_NT;
-  const int stage = MB > 2 ? 16 : ST_KG * 4;
+  const int NT = MB > 2 ? (w8 && MB <= 4 ? SH_GROUP_W8 : SH_GROUP) : ST_NT;
   int best = 1;
   double best_cost = 0;
   for (int S = 1; S <= most; S *= 2) {
     const int G = num_cus() / S;
-    if (G < 1 || nks / S < stage) break;  // every wave needs a full stage of K steps
+    if (G < 1) break;
     const int tpw = (ntiles + G - 1) / G;
+    const bool queue = queue_takes((int)M, w8, tpw);
+    const int stage = !queue ? (MB > 2 ? 16 : ST_KG * 4) : MB > 2 ? 8 * (w8 ? 2 : 1) : ST_KG * 4;
+    if (nks / S < stage) break;  // every wave needs a full stage of K steps
     const int groups = (tpw + NT - 1) / NT;
-    const double Ks = (double)K / S;
-    double cost = tpw * 16.0 * Ks * wbytes + groups * MB * 16.0 * Ks * 2 + 2.0 * tpw * 16 * M * 4;
-    cost *= 1.0 + 0.02 * S;  // ties go to fewer splits (fewer partial slices to sum)
+    const double Ks = (double)K / S, w = tpw * 16.0 * Ks * wbytes;
+    const int rows = queue_rows((int)M);
+    double cost = queue ? w + 0.45 * rows * 16.0 * Ks * 2 + 6500.0 * tpw * rows + 5.1 * S * N
+                        : w + groups * MB * 16.0 * Ks * 2 + 2.0 * tpw * 16 * M * 4;
+    if (!queue || MB <= 2) cost *= 1.0 + 0.02 * S;  // ties go to fewer splits (fewer partial slices to sum)
+    if (!queue && MB > 2) cost *= 2;                // the shared-activation kernel takes what is left
     if (S == 1 || cost < best_cost) {
       best = S;
       best_cost = cost;

@@ -460,6 +460,31 @@ def test_linear_f16(lib, M, N, K, epi):
             assert torch.equal(unpack_act(y3.cpu(), M, N), y2.cpu())
 
 
+# the queue kernel: every number of row blocks and of tiles to a workgroup (256 compute units), the last workgroup with fewer
+# tiles, fewer K steps than waves, one step more than a round of the waves, and more rounds than a queue holds
+@pytest.mark.parametrize("M,N,K", [(33, 16, 64), (48, 4080, 256), (49, 4112, 320), (64, 12320, 192), (65, 8208, 576),
+                                   (96, 12288, 1088), (97, 16400, 128), (128, 20400, 320), (40, 20496, 576),
+                                   (64, 24592, 320), (33, 28800, 128), (64, 32784, 1344), (128, 24800, 192),
+                                   (128, 28688, 320), (128, 32752, 128), (80, 36848, 192), (97, 36864, 64),
+                                   (17, 16400, 576), (32, 20512, 64), (24, 28688, 320), (18, 36864, 1344),
+                                   (1, 16400, 320), (16, 24608, 1344), (9, 32784, 64)])
+@pytest.mark.parametrize("w8", [False, True])
+def test_linear_packed_rows_in_queues(lib, M, N, K, w8):
+    print("queue", M, N, K, w8, flush=True)
+    x, W, b = rnd(M, K, seed=7), rnd(N, K, seed=8, std=0.05), rnd(N, seed=9, std=0.1)
+    xp = G(pack_act(x))
+    y = torch.full((M, N), float("nan"), dtype=torch.float16, device=DEV)
+    if w8:
+        q, sc = O.quantize_int8(W)
+        W = O.dequantize_int8(q, sc)
+        ok(lib.msa_linear_w8a16(P(xp), P(pack_w8(lib, G(q))), P(G(sc)), P(G(b)), None, P(y), M, N, K, IN_PACKED, None), lib)
+    else:
+        ok(lib.msa_linear_f16(P(xp), P(pack_w(lib, G(W))), P(G(b)), None, P(y), M, N, K, IN_PACKED, None), lib)
+    torch.cuda.synchronize()
+    want = _linear_want(x, W, b, None, False).half()
+    assert_fp16_close(y, want, atol=float(want.abs().max()) * 2 ** -10, what="queue")
+
+
 # 128 x 128 tiles (129 .. 256 rows; from a quarter of the chip to all of it, ragged edges, K of the ring's length
 # and more), shapes beside them whose K is too short for those, and 256 x 256 tiles of fewer rows under a wide output
 @pytest.mark.parametrize("M,N,K", [(129, 4096, 128), (160, 4112, 192), (255, 12304, 320), (256, 16384, 640),
