@@ -200,7 +200,8 @@ enum {
   MSA_TILES_WHOLE = 1,  /* 256 rows to a tile, a ragged last one (256 columns and 128) moved up */
   MSA_TILES_FEW = 2,    /* tiles that repeat the last row: fewer rows than a tile, or tiles of 128 x 128 */
   MSA_TILES_EVEN = 3,   /* the first n_tall rows of tiles are `rows` high, the others 32 less */
-  MSA_TILES_SIMPLE = 4  /* 128 x 128, K no multiple of 64 */
+  MSA_TILES_SIMPLE = 4, /* 128 x 128, K no multiple of 64 */
+  MSA_TILES_QUEUE = 5   /* two halves of 129 to 256 rows, up to 80 columns wide, a queue of loads to every wave */
 };
 typedef struct {
   int kind, rows, columns; /* rows and columns of a tile */

@@ -60,7 +60,7 @@ class TileForm(ctypes.Structure):
     _fields_ = [(n, c_int) for n in ("kind", "rows", "columns", "n_rows", "n_tall", "pieces", "panels")] + [("main", c_int64)]
 
 
-MSA_TILES_NONE, MSA_TILES_WHOLE, MSA_TILES_FEW, MSA_TILES_EVEN, MSA_TILES_SIMPLE = range(5)
+MSA_TILES_NONE, MSA_TILES_WHOLE, MSA_TILES_FEW, MSA_TILES_EVEN, MSA_TILES_SIMPLE, MSA_TILES_QUEUE = range(6)
 
 # name -> argtypes, in the order of include/metaseq_amd.h
 SIGNATURES = {

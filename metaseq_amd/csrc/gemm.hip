@@ -399,6 +399,10 @@ extern "C" int msa_linear_tiles(int64_t M, int N, int K, int S, int cus, msa_til
   const TileForm f = S == 0 ? tile_form(M, N, K, cus) : partial_form(M, N, K, S, cus);
   *out = msa_tile_form{f.kind, 0, 0, 0, 0, f.pieces, 0, f.main};
   if (f.kind == MSA_TILES_NONE) return MSA_OK;
+  if (f.kind == MSA_TILES_QUEUE) {
+    out->rows = 16 * queue_rows_blocks((int)M), out->columns = 16 * f.queue, out->n_rows = 2;
+    return MSA_OK;
+  }
   out->rows = tq_bm(f.rf), out->columns = tq_bn(f.wf);
   out->n_rows = f.kind == MSA_TILES_EVEN ? f.even.nrow : (int)((f.main + out->rows - 1) / out->rows);
   if (f.kind == MSA_TILES_EVEN) out->n_tall = f.even.n_tall;

@@ -2168,6 +2168,9 @@ constexpr bool queue_takes(int M, bool w8, int tiles_per_wg) {
 template <bool W8, int MODE>
 void launch_queue(const void* xp, const void* W, const void* scales, float* part, int S, int M, int N, int K,
                   int tiles_per_wg, const Epilogue& epi, hipStream_t s);
+template <int MODE>
+void launch_queue_rows(const void* x, const void* W, float* part, int S, int M, int N, int K, int tiles_per_wg,
+                       const Epilogue& epi, hipStream_t s);
 namespace {
 
 // The shared-activation kernel: 33 .. 64 packed rows of more tiles than the queue kernel takes, and vocabularies from one row on,
@@ -2577,14 +2580,32 @@ TileChoice tile_choice(int64_t M, int N, int K, int cus) {
 struct TileForm {
   int kind = MSA_TILES_SIMPLE, wf = 4, rf = 4, pieces = 1;
   int64_t main = 0;  // rows in tiles; the others in sweeps over the weights
+  int queue = 0;     // tiles of 16 columns to a workgroup of the queue kernel
   QuadPlan even;
 };
+// 129 .. 256 row-major rows in queues (gemm_queue.h): the tiles of a workgroup, 0 where there are more than five, or where
+// K is not in whole slots.  Two workgroups share a column of them.
+constexpr int QUEUE_ROWS_TILES = 5;
+constexpr int queue_rows_blocks(int M) { return M <= 160 ? 5 : M <= 192 ? 6 : M <= 224 ? 7 : 8; }
+int queue_rows_tiles(int64_t M, int N, int K, int S, int cus) {
+  if (M <= 128 || M > 256 || K % 64 || K < 128) return 0;
+  const int G = cus / (2 * S) < 1 ? 1 : cus / (2 * S), tiles = (N / 16 + G - 1) / G;
+  return tiles <= QUEUE_ROWS_TILES ? tiles : 0;
+}
 // S sums to be stored as they are, of any number of rows: the cheapest form of quad_price.  Below 256 rows 256 x 64 tiles while
 // their slices fit the chip in one round; an S beyond that means 256 x 128 tiles (pick_row_splits).
+// Of 129 .. 256 rows queues where those tiles would leave more than a quarter of the chip idle (us, 200 rows: 2560 x 2560 in four
+// slices, 160 tiles, 12.2 and 11.4 in queues, x 10240 30.2 and 23.3, 2048 x 2048 in four, 128 tiles, 10.1 and 8.9; 256 tiles:
+// 2048 x 8192 in eight 17.2, in four in queues 18.0, 4096 x 4096 in four 17.2, in two in queues 17.9).
 TileForm partial_form(int64_t M, int N, int K, int S, int cus) {
   const int64_t rows = (M + TQ_BM - 1) / TQ_BM;
   TileForm f;
   f.main = M, f.rf = 8;
+  f.queue = rows * ((N + 63) / 64) * S * 4 <= cus * 3 ? queue_rows_tiles(M, N, K, S, cus) : 0;
+  if (f.queue) {
+    f.kind = MSA_TILES_QUEUE;
+    return f;
+  }
   if (M < TQ_BM) {
     f.kind = MSA_TILES_FEW;
     f.wf = rows * ((N + 63) / 64) * S > cus ? 4 : 2;
@@ -2612,6 +2633,11 @@ TileForm tile_form(int64_t M, int N, int K, int cus) {
   }
   f.main = M;
   if (K % 64 || K < 128) return f;
+  f.queue = queue_rows_tiles(M, N, K, 1, cus);
+  if (f.queue) {
+    f.kind = MSA_TILES_QUEUE;
+    return f;
+  }
   const int64_t cols[2] = {(N + 255) / 256, (N + 127) / 128};
   if (M < TQ_BM && cols[0] <= cus && cols[0] * 4 >= cus * 3) {
     f.kind = MSA_TILES_FEW;
@@ -2636,6 +2662,7 @@ template <int MODE>
 void launch_quad_partial(const void* x, const void* W, float* part, int64_t M, int N, int K, int S,
                          hipStream_t s) {
   const TileForm f = partial_form(M, N, K, S, num_cus());
+  if (f.kind == MSA_TILES_QUEUE) return launch_queue_rows<MODE>(x, W, part, S, (int)M, N, K, f.queue, Epilogue{}, s);
   if (f.kind == MSA_TILES_EVEN) return launch_quad_plan<MODE, true>(x, W, M, N, K, S, f.even, Epilogue{}, part, s);
   if (f.pieces == 4) return launch_quad_pieces<MODE, true, 4>(x, W, M, N, K, S, Epilogue{}, part, s);
   if (f.pieces == 2) return launch_quad_pieces<MODE, true, 2>(x, W, M, N, K, S, Epilogue{}, part, s);
@@ -2657,6 +2684,11 @@ int pick_row_splits(int64_t M, int N, int K) {
   int best = 1;
   for (int S = 2; S <= 8; S *= 2)
     if (tiles * S <= num_cus() && K % (64 * S) == 0 && K / S >= 512) best = S;
+  // in queues, half as many are as fast from 2048 columns or 4096 of K on, and leave the tail half as much to add (us, 200 rows: 2048 x
+  // 2048 in four 8.9, in two 8.4, 2560 x 2560 11.4 and 11.1, 1024 x 4096 in eight 9.4, in four 8.4)
+  if (best >= 4 && partial_form(M, N, K, best, num_cus()).queue > 3 && partial_form(M, N, K, best / 2, num_cus()).queue &&
+      K / best <= 1024)
+    return best / 2;
   if (best > 1 && best < 8 && M > 128 && K / best >= 4096 && K % (128 * best) == 0) best *= 2;
   return best;
 }
@@ -2731,6 +2763,8 @@ void launch_tiled(const void* x, const void* W, const void* scales, int64_t M, i
   const int64_t big_tiles = ((M + TB_BM - 1) / TB_BM) * ((N + TB_BN - 1) / TB_BN);
   if constexpr (!W8) {
     const TileForm f = tile_form(M, N, K, num_cus());
+    if (f.kind == MSA_TILES_QUEUE)
+      return launch_queue_rows<MODE>(x, W, nullptr, 1, (int)M, N, K, f.queue, epi, s);
     if (f.kind == MSA_TILES_EVEN) return launch_quad_plan<MODE, false>(x, W, M, N, K, 1, f.even, epi, nullptr, s);
     if (f.kind == MSA_TILES_WHOLE) {
       if (f.wf == 8) return launch_quad<MODE, 8>(x, W, scales, M, f.main, N, K, f.pieces, epi, s);

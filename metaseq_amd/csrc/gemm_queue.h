@@ -1,5 +1,6 @@
 #pragma once
-// The queue kernel: products of packed rows, 33 .. 128 of them or fewer with many tiles to a workgroup (gemm_kernels.h chooses).
+// The queue kernels: products of packed rows, 33 .. 128 of them or fewer with many tiles to a workgroup, and of 129 .. 256
+// row-major rows (gemm_kernels.h chooses).
 #include "gemm_kernels.h"
 
 namespace {
@@ -180,6 +181,150 @@ __global__ __launch_bounds__((QueueCfg<MB, W8, NT>::KL * 64)) void linear_queue_
   }
 }
 
+// ---- the same for 129 .. 256 row-major rows ----
+// Two workgroups share a column of NT tiles, each with half of the rows (MB blocks of 16, the last row repeated), next to each
+// other on one XCD, so that the weights come from HBM once.  A slot is 64 deep: a load takes a 128-byte line of each of eight
+// rows, chunk c of row r at position c ^ (r / 2) % 8, as in the tile kernels, whose fragment reads then meet no bank conflicts;
+// a tile's two 1 KB blocks follow each other in memory.
+//
+// The tile kernels' four waves wait for each other at every 32-wide step, and cut so few rows and columns into few tiles.  us,
+// tiles and this, 129 / 200 / 256 rows: 3072 x 768 10.5 / 11.3 / 12.3 and 6.5 / 7.3 / 7.7; 6144 x 2048 18.4 / 20.3 / 22.6 and
+// 12.6 / 15.4 / 16.5; 4096 x 4096 29.7 / 33.9 / 39.0 and 16.9 / 20.3 / 22.4; 8192 x 4096 32.3 / 36.2 / 41.0 and 24.5 / 28.5 /
+// 31.2; 10240 x 2560 (five tiles) 24.3 / 26.7 / 30.6 and 19.8 / 24.2 / 26.1.  With six tiles or more a CU receives as many bytes as
+// with 128 x 128 tiles, and its one wave per SIMD has no second slot to wait with: 12288 x 2048 22.5 / 23.2 / 25.0 and 19.7 / 24.8
+// / 25.8, 200 x 16384 x 4096 42.6 and 49.
+template <int MB, int NT>
+struct QueueRowsCfg {
+  static constexpr int LOADS = 2 * (MB + NT), SLOT = LOADS * 1024;
+  static constexpr int REGS = 4 * (MB * NT + LOADS) + 40;
+  static constexpr int KL = REGS <= 256 && 8 * SLOT <= 160 * 1024 ? 8 : 4;
+  static constexpr int FIT = 160 * 1024 / (KL * SLOT), R = FIT > 4 ? 4 : FIT;
+  static constexpr int JFIT = 160 * 1024 / (KL * MB * 1024), J = JFIT > NT ? NT : JFIT;
+  static constexpr int RING = KL * R * SLOT, RED = KL * J * MB * 1024;
+  static constexpr int LDS_BYTES = RING > RED ? RING : RED;
+  static_assert(R >= 1 && J >= 1, "a CU has 160 KB of LDS");
+};
+
+// blockIdx.x: eight columns' upper halves, their lower halves, the next eight columns' ..; blockIdx.y: the slice of K
+template <int MB, int MODE, int NT>
+__global__ __launch_bounds__((QueueRowsCfg<MB, NT>::KL * 64)) void linear_queue_rows_kernel(
+    const half_t* __restrict__ x, const void* __restrict__ Wp, float* __restrict__ part, int M, int N, int K,
+    int tiles_per_wg, int stages_per_split, Epilogue epi) {
+  using C = QueueRowsCfg<MB, NT>;
+  constexpr int R = C::R, L = C::LOADS, KL = C::KL;
+  extern __shared__ __attribute__((aligned(16))) char lds_queue[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int half = (blockIdx.x >> 3) & 1, col = (blockIdx.x >> 4) * 8 + (blockIdx.x & 7);
+  const int ntiles = N >> 4, nst = K >> 6;
+  const int tile_begin = col * tiles_per_wg;
+  if (tile_begin >= ntiles) return;
+  const int tile_end = min(ntiles, tile_begin + tiles_per_wg);
+  const int m0 = half * (MB * 16);
+  const int s_begin = blockIdx.y * stages_per_split, s_end = min(nst, s_begin + stages_per_split);
+  const int n = s_begin + wave < s_end ? (s_end - s_begin - wave + KL - 1) / KL : 0;
+  const char* wb[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+    wb[j] = (const char*)Wp + (int64_t)min(tile_begin + j, tile_end - 1) * nst * 2048 - (j % 2) * 2048;
+  // (activations: load i takes rows 8 i .. 8 i + 7)
+  uint32_t xo[2 * MB];
+#pragma unroll
+  for (int i = 0; i < 2 * MB; ++i) {
+    const int row = min(m0 + i * 8 + (lane >> 3), M - 1);
+    xo[i] = (uint32_t)row * (uint32_t)K * 2u + (uint32_t)(((lane & 7) ^ (4 * (i & 1) + (lane >> 4))) * 16);
+  }
+  const char* xb[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) xb[q] = (const char*)x - q * 1024;
+  const char* ring = lds_queue + wave * (R * C::SLOT);
+  const uint32_t ring_at = (uint32_t)(uintptr_t)(tq_lds_void*)lds_queue + wave * (R * C::SLOT);
+  auto request = [&](int slot, int i) {
+    const uint32_t st = (uint32_t)(s_begin + wave + KL * i);
+    const uint32_t at = ring_at + slot * C::SLOT;
+    const uint32_t wv = (uint32_t)lane * 16u + st * 2048u;
+    tq_static_for<2 * NT>([&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      queue_load<(j % 4) * 1024, false>(wv, wb[j / 2], at + (j / 4) * 4096);
+    });
+    tq_static_for<2 * MB>([&](auto ic) {
+      constexpr int f = decltype(ic)::value;
+      queue_load<(f % 4) * 1024, false>(xo[f] + st * 128u, xb[f % 4], at + 2 * NT * 1024 + (f / 4) * 4096);
+    });
+  };
+  float4_t acc[NT][MB];
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) acc[j][mb] = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+    if (r < n) request(r, r);
+  const int lr = lane & 15, lg = lane >> 4;
+  const uint32_t x0 = lr * 128 + ((lg ^ (lr >> 1)) * 16), x1 = lr * 128 + (((4 + lg) ^ (lr >> 1)) * 16);
+  int slot = 0;
+  for (int i = 0; i < n; ++i) {
+    if (i + R - 1 < n)
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((R - 1) * L) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const char* from = ring + slot * C::SLOT;
+    half8_t w[2][NT], xf[2][MB];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+#pragma unroll
+      for (int j = 0; j < NT; ++j) w[u][j] = *reinterpret_cast<const half8_t*>(from + (2 * j + u) * 1024 + lane * 16);
+#pragma unroll
+      for (int f = 0; f < MB; ++f) xf[u][f] = *reinterpret_cast<const half8_t*>(from + (2 * NT + 2 * f) * 1024 + (u ? x1 : x0));
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (i + R < n) request(slot, i + R);
+    slot = slot == R - 1 ? 0 : slot + 1;
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) acc[j][mb] = mfma_16x16x32<MODE>(w[u][j], xf[u][mb], acc[j][mb]);
+  }
+
+  float4_t* red = reinterpret_cast<float4_t*>(lds_queue);
+  constexpr int TOT = C::J * MB, PER = (TOT + KL - 1) / KL;
+  constexpr bool AHEAD = PER <= (KL == 4 ? 10 : 4) && (!is_bf<MODE> || MODE == MODE_BF_POST);
+#pragma unroll
+  for (int j0 = 0; j0 < NT; j0 += C::J) {
+    Ahead<MODE> ahead[AHEAD ? PER : 1];
+    if (AHEAD && !part) {
+#pragma unroll
+      for (int q = 0; q < (AHEAD ? PER : 0); ++q) {
+        const int p = min(wave + q * KL, TOT - 1);
+        const int t = min(tile_begin + j0 + p / MB, tile_end - 1);
+        ahead[q] = epilogue_ahead<MODE>(epi, min(m0 + p % MB * 16 + lr, M - 1), t * 16 + lg * 4);
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = j0; j < j0 + C::J && j < NT; ++j)
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) red[((wave * C::J + j - j0) * MB + mb) * 64 + lane] = acc[j][mb];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+      const int p = wave + q * KL, j = j0 + p / MB, mb = p % MB, t = tile_begin + j;
+      if (p >= TOT || j >= NT || t >= tile_end) continue;
+      float4_t sum = red[p * 64 + lane];
+#pragma unroll
+      for (int k = 1; k < KL; ++k) sum += red[(k * TOT + p) * 64 + lane];
+      const int m = m0 + mb * 16 + lr, c = t * 16 + lg * 4;
+      if (m >= M) continue;
+      if (part)
+        *reinterpret_cast<float4_t*>(part + ((int64_t)blockIdx.y * M + m) * N + c) = sum;
+      else
+        epilogue4<MODE, AHEAD>(epi, m, c, sum, ahead[AHEAD ? q : 0]);
+    }
+  }
+}
+
 template <int MB, bool W8, int MODE, int NT>
 void launch_queue_cfg(const void* xp, const void* W, const void* scales, float* part, int S, int M, int N, int K,
                       int tiles_per_wg, int gx, int ks_per_split, const Epilogue& epi, hipStream_t s) {
@@ -198,6 +343,20 @@ void launch_queue_mb(const void* xp, const void* W, const void* scales, float* p
       return launch_queue_cfg<MB, W8, MODE, NT>(xp, W, scales, part, S, M, N, K, tiles_per_wg, gx, ks_per_split, epi, s);
   if constexpr (NT < QUEUE_TILES)
     launch_queue_mb<MB, W8, MODE, NT + 1>(xp, W, scales, part, S, M, N, K, tiles_per_wg, gx, ks_per_split, epi, s);
+}
+template <int MB, int MODE, int NT = 1>
+void launch_queue_rows_mb(const void* x, const void* W, float* part, int S, int M, int N, int K, int tiles_per_wg,
+                          const Epilogue& epi, hipStream_t s) {
+  if constexpr (NT < QUEUE_ROWS_TILES)
+    if (tiles_per_wg > NT)
+      return launch_queue_rows_mb<MB, MODE, NT + 1>(x, W, part, S, M, N, K, tiles_per_wg, epi, s);
+  using C = QueueRowsCfg<MB, NT>;
+  static std::atomic<uint64_t> lds_allowed{0};
+  auto kernel = linear_queue_rows_kernel<MB, MODE, NT>;
+  if (!allow_lds((const void*)kernel, C::LDS_BYTES, lds_allowed)) return;  // the caller's launch check reports the error
+  const int columns = (N / 16 + tiles_per_wg - 1) / tiles_per_wg, stages = (K / 64 + S - 1) / S;
+  hipLaunchKernelGGL(kernel, dim3((columns + 7) / 8 * 16, S), dim3(C::KL * 64), C::LDS_BYTES, s, (const half_t*)x, W, part,
+                     M, N, K, tiles_per_wg, stages, epi);
 }
 }  // namespace
 
@@ -222,4 +381,15 @@ void launch_queue(const void* xp, const void* W, const void* scales, float* part
     Q_RUN(8);
   }
 #undef Q_RUN
+}
+
+template <int MODE>
+void launch_queue_rows(const void* x, const void* W, float* part, int S, int M, int N, int K, int tiles_per_wg,
+                       const Epilogue& epi, hipStream_t s) {
+  switch (queue_rows_blocks(M)) {
+    case 5: return launch_queue_rows_mb<5, MODE>(x, W, part, S, M, N, K, tiles_per_wg, epi, s);
+    case 6: return launch_queue_rows_mb<6, MODE>(x, W, part, S, M, N, K, tiles_per_wg, epi, s);
+    case 7: return launch_queue_rows_mb<7, MODE>(x, W, part, S, M, N, K, tiles_per_wg, epi, s);
+    default: return launch_queue_rows_mb<8, MODE>(x, W, part, S, M, N, K, tiles_per_wg, epi, s);
+  }
 }

@@ -7,3 +7,9 @@ template void launch_queue<false, MODE_BF_GLU>(const void*, const void*, const v
                                        const Epilogue&, hipStream_t);
 template void launch_queue<false, MODE_BF_POST>(const void*, const void*, const void*, float*, int, int, int, int, int,
                                        const Epilogue&, hipStream_t);
+template void launch_queue_rows<MODE_BF>(const void*, const void*, float*, int, int, int, int, int, const Epilogue&,
+                                     hipStream_t);
+template void launch_queue_rows<MODE_BF_GLU>(const void*, const void*, float*, int, int, int, int, int, const Epilogue&,
+                                     hipStream_t);
+template void launch_queue_rows<MODE_BF_POST>(const void*, const void*, float*, int, int, int, int, int, const Epilogue&,
+                                     hipStream_t);

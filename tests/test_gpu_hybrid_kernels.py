@@ -102,6 +102,13 @@ def test_linear_bf16_of_a_wave_per_tile(M, N, K):
     test_linear_bf16(M, N, K)
 
 
+# packed rows and 129 .. 256 row-major ones in queues: tiles to a workgroup and row blocks of either
+@pytest.mark.parametrize("M,N,K", [(40, 16400, 320), (64, 28688, 192), (90, 24592, 576), (128, 20496, 320), (20, 32784, 192),
+                                   (140, 6160, 576), (190, 10256, 320), (256, 8208, 1088)])
+def test_linear_bf16_in_queues(M, N, K):
+    test_linear_bf16(M, N, K)
+
+
 @pytest.mark.parametrize("M,K,most", [(1, 768, 1.0e-7), (33, 4096, 1.8e-7), (64, 9216, 2.5e-7), (100, 4096, 3.3e-7)])
 def test_fp32_logits_of_a_vocabulary_are_no_single_chain_over_k(M, K, most):
     """The error of fp32 sums grows with the root of the additions behind each: K / 128 stages of four steps up to 64 rows,

@@ -485,6 +485,29 @@ def test_linear_packed_rows_in_queues(lib, M, N, K, w8):
     assert_fp16_close(y, want, atol=float(want.abs().max()) * 2 ** -10, what="queue")
 
 
+# 129 .. 256 row-major rows in queues: every number of row blocks and of tiles to a workgroup (256 compute units), the last
+# columns' workgroup with fewer, blocks whose rows run out, fewer 64-wide stages than waves and more than a queue holds
+QUEUE_ROWS = [(129, 16, 128), (160, 2064, 192), (161, 3072, 768), (192, 4112, 576), (193, 6160, 1088), (224, 8192, 320),
+              (225, 8208, 576), (255, 10240, 192), (256, 6144, 1344), (256, 2048, 704), (130, 10224, 128), (200, 4000, 2048)]
+
+
+@pytest.mark.parametrize("M,N,K", QUEUE_ROWS)
+def test_linear_f16_rows_in_queues(lib, M, N, K):
+    """A whole product with bias and, in place, a residual; two slices."""
+    print("queue rows", M, N, K, flush=True)
+    x, W, b, res = rnd(M, K, seed=7), rnd(N, K, seed=8, std=0.05), rnd(N, seed=9, std=0.1), rnd(M, N, seed=10)
+    want = _linear_want(x, W, b, res, False).half()
+    Wp, y = pack_w(lib, G(W)), G(res).clone()
+    ok(lib.msa_linear_f16(P(G(x)), P(Wp), P(G(b)), P(y), P(y), M, N, K, 0, None), lib)
+    torch.cuda.synchronize()
+    assert_fp16_close(y, want, atol=float(want.abs().max()) * 2 ** -10, what="queue rows")
+    S = 2 if K % 128 == 0 and K >= 256 else 1
+    part = torch.full((S, M, N), float("nan"), dtype=torch.float32, device=DEV)
+    ok(lib.msa_linear_partial_f16(P(G(x)), P(Wp), P(part), M, N, K, S, 0, None), lib)
+    torch.cuda.synchronize()
+    assert (part.sum(0).cpu() - x.float() @ W.float().t()).abs().max() < 1e-3
+
+
 # 128 x 128 tiles (129 .. 256 rows; from a quarter of the chip to all of it, ragged edges, K of the ring's length
 # and more), shapes beside them whose K is too short for those, and 256 x 256 tiles of fewer rows under a wide output
 @pytest.mark.parametrize("M,N,K", [(129, 4096, 128), (160, 4112, 192), (255, 12304, 320), (256, 16384, 640),
