@@ -6,7 +6,7 @@
 // the order the 64 lanes read it, and the blocks of one 16-row tile follow each other along K.
 // A wave instruction therefore reads one whole KB and a tile's K sweep is one linear stream.
 //
-// Five kernels:
+// Six kernels:
 //   * stream (M <= 32 packed rows, the decode step; also the fused vocabulary projection +
 //     selection of up to 64 rows where the next kernel does not take it): HBM-bound.  A
 //     workgroup of 8 waves owns a contiguous range of 16-row tiles (and, with split-K, one K
@@ -16,8 +16,10 @@
 //     buffered several steps deep and the prefetch runs across tile-group boundaries, so the
 //     memory pipe never drains while a finished group is reduced across the waves through LDS
 //     (fixed order: results are run-to-run deterministic).
-//   * shared-activation stream (33 .. 128 packed rows; vocabularies of 16-bit weights and their
-//     selection from one row on): the same weight streaming, with the activation fragments staged
+//   * queues (gemm_queue.h; 33 .. 128 packed rows and 129 .. 256 row-major ones, int8 weights and two row blocks also where
+//     a workgroup has five to nine tiles): every wave a K lane with a queue of loads of its own in LDS.
+//   * shared-activation stream (vocabularies of 16-bit weights and their selection from one row on; 33 .. 128 packed rows of
+//     more tiles than queues take): the same weight streaming, with the activation fragments staged
 //     once per workgroup in LDS and shared by its waves.
 //   * large tiled, fp16 weights (from 65 row-major rows on): 256 x 256 per workgroup of four waves of
 //     128 x 128 with their accumulators in the AGPR bank, both operands global -> LDS directly; tiles of 128 to 256
@@ -728,7 +730,7 @@ __global__ __launch_bounds__(ST_KG * 64) void linear_stream_ln_kernel(
                                                      LnTail{ln_part, ln_bias, ln_x, x_out, gamma, beta, eps});
 }
 
-// ---- shared-activation stream kernel (33 .. 128 rows; vocabularies from one row on) ------------
+// ---- shared-activation stream kernel (vocabularies from one row on; more tiles than queues take) ----
 // With more than 32 activation rows a wave that loads its own activation fragments moves more
 // bytes of activations (from L2) than of weights (from HBM) through the L1, and the L1 fill rate
 // becomes the limit.  Here the waves form KL K lanes x NG tile lanes: the NG waves of a K lane
@@ -737,10 +739,7 @@ __global__ __launch_bounds__(ST_KG * 64) void linear_stream_ln_kernel(
 // contiguous piece of the packed activations).  Weights still go from HBM straight to registers.
 // A tile group is NG * NT tiles, dealt round robin to the tile lanes; one barrier per stage;
 // activations are fetched two stages ahead and parked in LDS one stage ahead, weights (and int8
-// scales) one stage ahead.  The K lanes are summed through LDS in fixed order.
-// KL K lanes x NG tile lanes of one wave each (8 waves as 2 x 4, or 12 waves as 4 x 3 for
-// workgroups whose tile count is a multiple of 3: nine tiles fill 4 x 3 slots only to three
-// quarters, but 3 x 3 exactly).
+// scales) PF - 1 stages ahead.  The K lanes are summed through LDS in fixed order.
 template <int MB, bool W8, int KL, int NG, int NT, int U>
 struct ShareCfg {
   static constexpr int THREADS = KL * NG * 64;
@@ -748,14 +747,11 @@ struct ShareCfg {
   static constexpr int XH = SK * MB * 512;  // halves of activations per stage
   static constexpr int PIECES = XH / 8;     // 16-byte pieces per stage
   static constexpr int XP = (PIECES + THREADS - 1) / THREADS;  // pieces per thread and stage
-  // activations double buffered, then one tile slot's partial sums of the other K lanes; where
-  // both do not fit the 160 KB of a compute unit the partial sums take the place of the stage
-  // that has just been consumed
+  // activations double buffered, then one tile slot's partial sums of the other K lanes
   static constexpr int RED_BYTES = (KL - 1) * NG * MB * 1024;
-  static constexpr bool RED_ALIAS = 2 * XH * 2 + RED_BYTES > 160 * 1024;
-  static constexpr int LDS_BYTES = 2 * XH * 2 + (RED_ALIAS ? 0 : RED_BYTES);
+  static constexpr int LDS_BYTES = 2 * XH * 2 + RED_BYTES;
+  static_assert(LDS_BYTES <= 160 * 1024, "a CU has 160 KB of LDS");
   static_assert(U % 2 == 0, "a stage holds whole int8 blocks");
-  static_assert(!RED_ALIAS || RED_BYTES <= XH * 2, "the partial sums must fit one stage");
 };
 
 template <int MB, bool W8, int MODE, int KL, int NG, int NT, int U, int PF>
@@ -768,7 +764,7 @@ __global__ __launch_bounds__(KL * NG * 64) void linear_share_kernel(
   constexpr int SK = C::SK, UA = C::UA, XH = C::XH, XP = C::XP, THREADS = C::THREADS;
   constexpr int PIECES = C::PIECES;
   extern __shared__ __attribute__((aligned(16))) half_t lx_share[];  // [2][XH], then red
-  float4_t* red_own = reinterpret_cast<float4_t*>(lx_share + 2 * XH);  // [KL-1][NG][MB][64]
+  float4_t* red = reinterpret_cast<float4_t*>(lx_share + 2 * XH);  // [KL-1][NG][MB][64]
   const int lane = threadIdx.x & 63;
   // the wave number as a scalar: everything derived from it stays out of the vector registers
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -925,18 +921,11 @@ __global__ __launch_bounds__(KL * NG * 64) void linear_share_kernel(
       clear();
       return;
     }
-    float4_t* red = red_own;
-    if constexpr (C::RED_ALIAS) {  // the stage just consumed, once every wave is done reading it
-      red = reinterpret_cast<float4_t*>(lx_share + (idx & 1) * XH);
-      __syncthreads();
-    }
     constexpr int EMODE = MODE == MODE_SELECT ? MODE_PLAIN : MODE;
-    // What the epilogue reads is requested for all row blocks at once, in front of the reduction (row by row behind it,
-    // each block is a round trip; 57 rows x 12288 x 4096 24.0 and 23.6 us, 40 x 3072 x 1024 7.4 and 6.6).  Where there are
-    // registers for it: of eight row blocks they spill; with two and three tiles to a wave, int8 weights or a cache to write to, they are
-    // taken from the loads in flight (int8, 40 rows in slices, 7168 x 28672 52.7 without and 56.8 with it, fp16 keys, values and
-    // queries of 59 x 9216 84.5 and 87.9), and fourteen waves of a tile each spill for the cache's places.
-    constexpr bool AHEAD = MB <= 4 && !is_bf<EMODE> && ((NT == 1 && KL > 1) || (EMODE == MODE_PLAIN && !W8));
+    // What the epilogue reads is requested for all row blocks at once, in front of the reduction (row by row behind it, each
+    // block is a round trip), where there are registers for it: of eight row blocks they spill; int8 weights and a cache to
+    // write to lose the loads in flight by it (int8, 40 rows in slices, 7168 x 28672 52.7 without and 56.8 us with it).
+    constexpr bool AHEAD = MB <= 4 && EMODE == MODE_PLAIN && !W8;
     Ahead<EMODE> ahead[AHEAD ? MB : 1];
     auto look_ahead = [&](int t) {
       if (!AHEAD || part || kl > 0) return;
@@ -2063,10 +2052,8 @@ bool allow_lds(const void* kernel, int bytes, std::atomic<uint64_t>& done) {
 
 template <int MB, bool W8, int MODE, bool XR = false>
 void launch_stream_mb(const void* xp, const void* W, const void* scales, float* part, int S, int M,
-                      int N, int K, const Epilogue& epi, hipStream_t s, int64_t m_off = 0) {
+                      int N, int K, int G, const Epilogue& epi, hipStream_t s, int64_t m_off = 0) {
   const int ntiles = N / 16, nks = K / 32;
-  int G = num_cus() / S;
-  if (G < 1) G = 1;
   const int tiles_per_wg = (ntiles + G - 1) / G;
   const int gx = (ntiles + tiles_per_wg - 1) / tiles_per_wg;
   int ks_per_split = (nks + S - 1) / S;
@@ -2125,10 +2112,7 @@ constexpr bool vocabulary_tiles(int tiles_per_wg) { return tiles_per_wg == 13 ||
 
 // The shared-activation kernel sweeps K once per pass of SH_GROUP tiles: it is used when the
 // workgroup's tiles fill their passes to at least three quarters.
-bool share_fits(int N, int S, bool w8) {
-  int G = num_cus() / S;
-  if (G < 1) G = 1;
-  const int tpw = (N / 16 + G - 1) / G;
+bool share_fits(int tpw, bool w8) {
   if (tpw <= SH_GROUP) return true;  // one pass, with the tile count per wave chosen to fit
   if (w8 && tpw <= SH_GROUP_W8 && 4 * tpw >= 3 * SH_GROUP_W8) return true;  // one pass of 18
   const int passes = (tpw + SH_GROUP - 1) / SH_GROUP;
@@ -2154,9 +2138,7 @@ void launch_share_cfg(const void* xp, const void* W, const void* scales, float* 
 // LDS (us, stream and queue: 16384 x 4096, 32 rows 24.5 and 25, int8 17.3 and 18.2, 8 rows int8 16.9 and 18.1; five tiles int8
 // 8 x 20480 x 5120 23.0 and 18.6; fp16 of one row block, seven tiles, 62.0 and 62.6).
 constexpr int QUEUE_TILES = 9;
-constexpr int queue_rows(int M) {  // row blocks that it multiplies: 65 .. 96 rows leave two of the eight out
-  return M > 96 ? 8 : M > 64 ? 6 : (M + 15) / 16;
-}
+constexpr int queue_rows(int M) { return (M + 15) / 16; }  // row blocks that it multiplies, of eight from 65 rows on
 constexpr bool queue_takes(int M, bool w8, int tiles_per_wg) {
   const int mb = queue_rows(M);
   if (tiles_per_wg > QUEUE_TILES || mb * tiles_per_wg > 64) return false;  // 64: QueueCfg::OK
@@ -2177,10 +2159,8 @@ namespace {
 // selections too (any number of tiles is right, in as many passes).
 template <int MB, bool W8, int MODE>
 void launch_share(const void* xp, const void* W, const void* scales, float* part, int S, int M,
-                  int N, int K, const Epilogue& epi, hipStream_t s) {
+                  int N, int K, int G, const Epilogue& epi, hipStream_t s) {
   const int ntiles = N / 16, nks = K / 32;
-  int G = num_cus() / S;
-  if (G < 1) G = 1;
   const int tiles_per_wg = (ntiles + G - 1) / G;
   const int gx = (ntiles + tiles_per_wg - 1) / tiles_per_wg;
   int ks_per_split = (nks + S - 1) / S;
@@ -2207,10 +2187,8 @@ void launch_share(const void* xp, const void* W, const void* scales, float* part
 // 116 -> 95 us).
 template <bool W8, int MODE>
 void launch_wide(const void* xp, const void* W, const void* scales, float* part, int S, int M,
-                 int N, int K, const Epilogue& epi, hipStream_t s) {
+                 int N, int K, int G, const Epilogue& epi, hipStream_t s) {
   const int ntiles = N / 16, nks = K / 32;
-  int G = num_cus() / S;
-  if (G < 1) G = 1;
   const int tiles_per_wg = (ntiles + G - 1) / G;
   const int gx = (ntiles + tiles_per_wg - 1) / tiles_per_wg;
   int ks_per_split = (nks + S - 1) / S;
@@ -2233,7 +2211,7 @@ void launch_wide(const void* xp, const void* W, const void* scales, float* part,
 template <bool W8, int MODE, int S>
 bool launch_stream_ln(const LnTail& ln, const void* W, const void* scales, int M, int N, int K, const Epilogue& epi,
                       hipStream_t s) {
-  const int ntiles = N / 16, tpw = (ntiles + num_cus() - 1) / num_cus(), gx = (ntiles + tpw - 1) / tpw;
+  const int ntiles = N / 16, cus = num_cus(), tpw = (ntiles + cus - 1) / cus, gx = (ntiles + tpw - 1) / tpw;
   const int bytes = K * 32;
   static_assert(LN_MAX_K / 32 < 256 && LN_MAX_ROWS < 256, "packed below");
 #define LN_RUN(NT)                                                                                            \
@@ -2263,40 +2241,40 @@ bool launch_stream_ln(const LnTail& ln, int S, const void* W, const void* scales
 template <bool W8, int MODE, bool XR = false>
 void launch_stream(const void* xp, const void* W, const void* scales, float* part, int S, int M,
                    int N, int K, const Epilogue& epi, hipStream_t s, int64_t m_off = 0) {
+  // (the device is asked for once: 125m, one row, 278 us a step with three times as many questions, 270 with one more)
+  const int cus = num_cus(), G = cus / S < 1 ? 1 : cus / S, tpw = (N / 16 + G - 1) / G;
   if constexpr (!XR && MODE != MODE_SELECT) {
-    const int G = num_cus() / S < 1 ? 1 : num_cus() / S, tpw = (N / 16 + G - 1) / G;
     if (queue_takes(M, W8, tpw)) return launch_queue<W8, MODE>(xp, W, scales, part, S, M, N, K, tpw, epi, s);
-    if (M > 64) return launch_wide<W8, MODE>(xp, W, scales, part, S, M, N, K, epi, s);
+    if (M > 64) return launch_wide<W8, MODE>(xp, W, scales, part, S, M, N, K, G, epi, s);
   }
   if constexpr (!XR && !W8) {
-    const int G = num_cus() / S < 1 ? 1 : num_cus() / S;
-    if (M <= 64 && vocabulary_tiles((N / 16 + G - 1) / G)) {
-      if (M > 48) return launch_share<4, W8, MODE>(xp, W, scales, part, S, M, N, K, epi, s);
-      if (M > 32) return launch_share<3, W8, MODE>(xp, W, scales, part, S, M, N, K, epi, s);
-      if (M > 16) return launch_share<2, W8, MODE>(xp, W, scales, part, S, M, N, K, epi, s);
-      return launch_share<1, W8, MODE>(xp, W, scales, part, S, M, N, K, epi, s);
+    if (M <= 64 && vocabulary_tiles(tpw)) {
+      if (M > 48) return launch_share<4, W8, MODE>(xp, W, scales, part, S, M, N, K, G, epi, s);
+      if (M > 32) return launch_share<3, W8, MODE>(xp, W, scales, part, S, M, N, K, G, epi, s);
+      if (M > 16) return launch_share<2, W8, MODE>(xp, W, scales, part, S, M, N, K, G, epi, s);
+      return launch_share<1, W8, MODE>(xp, W, scales, part, S, M, N, K, G, epi, s);
     }
   }
-  if (!XR && MODE != MODE_SELECT && M > 32 && share_fits(N, S, W8)) {
+  if (!XR && MODE != MODE_SELECT && M > 32 && share_fits(tpw, W8)) {
     constexpr int PM = MODE == MODE_SELECT ? MODE_PLAIN : MODE;
     if (M > 48)
-      launch_share<4, W8, PM>(xp, W, scales, part, S, M, N, K, epi, s);
+      launch_share<4, W8, PM>(xp, W, scales, part, S, M, N, K, G, epi, s);
     else
-      launch_share<3, W8, PM>(xp, W, scales, part, S, M, N, K, epi, s);
+      launch_share<3, W8, PM>(xp, W, scales, part, S, M, N, K, G, epi, s);
     return;
   }
   switch ((M + 15) / 16) {
     case 1:
-      launch_stream_mb<1, W8, MODE, XR>(xp, W, scales, part, S, M, N, K, epi, s, m_off);
+      launch_stream_mb<1, W8, MODE, XR>(xp, W, scales, part, S, M, N, K, G, epi, s, m_off);
       break;
     case 2:
-      launch_stream_mb<2, W8, MODE, XR>(xp, W, scales, part, S, M, N, K, epi, s, m_off);
+      launch_stream_mb<2, W8, MODE, XR>(xp, W, scales, part, S, M, N, K, G, epi, s, m_off);
       break;
     case 3:
-      launch_stream_mb<3, W8, MODE, XR>(xp, W, scales, part, S, M, N, K, epi, s, m_off);
+      launch_stream_mb<3, W8, MODE, XR>(xp, W, scales, part, S, M, N, K, G, epi, s, m_off);
       break;
     default:
-      launch_stream_mb<4, W8, MODE, XR>(xp, W, scales, part, S, M, N, K, epi, s, m_off);
+      launch_stream_mb<4, W8, MODE, XR>(xp, W, scales, part, S, M, N, K, G, epi, s, m_off);
       break;
   }
 }
@@ -2681,13 +2659,13 @@ void launch_quad_partial(const void* x, const void* W, float* part, int64_t M, i
 int pick_row_splits(int64_t M, int N, int K) {
   if (M < 1 || N % 16 || K % 64) return 1;
   const int64_t tiles = ((M + TQ_BM - 1) / TQ_BM) * ((N + tq_bn(2) - 1) / tq_bn(2));
+  const int cus = num_cus();
   int best = 1;
   for (int S = 2; S <= 8; S *= 2)
-    if (tiles * S <= num_cus() && K % (64 * S) == 0 && K / S >= 512) best = S;
+    if (tiles * S <= cus && K % (64 * S) == 0 && K / S >= 512) best = S;
   // in queues, half as many are as fast from 2048 columns or 4096 of K on, and leave the tail half as much to add (us, 200 rows: 2048 x
   // 2048 in four 8.9, in two 8.4, 2560 x 2560 11.4 and 11.1, 1024 x 4096 in eight 9.4, in four 8.4)
-  if (best >= 4 && partial_form(M, N, K, best, num_cus()).queue > 3 && partial_form(M, N, K, best / 2, num_cus()).queue &&
-      K / best <= 1024)
+  if (best >= 4 && K / best <= 1024 && partial_form(M, N, K, best, cus).queue > 3 && partial_form(M, N, K, best / 2, cus).queue)
     return best / 2;
   if (best > 1 && best < 8 && M > 128 && K / best >= 4096 && K % (128 * best) == 0) best *= 2;
   return best;
@@ -2845,10 +2823,11 @@ int pick_splits(int64_t M, int N, int K, int wbytes, int most = 8) {
   // elsewhere: tiles that share one sweep over the activations (int8 has a 2 x 6 x 3 shape of the
   // shared-activation kernel for up to 18), and K steps per stage of the workgroup
   const int NT = MB > 2 ? (w8 && MB <= 4 ? SH_GROUP_W8 : SH_GROUP) : ST_NT;
+  const int cus = num_cus();
   int best = 1;
   double best_cost = 0;
   for (int S = 1; S <= most; S *= 2) {
-    const int G = num_cus() / S;
+    const int G = cus / S;
     if (G < 1) break;
     const int tpw = (ntiles + G - 1) / G;
     const bool queue = queue_takes((int)M, w8, tpw);

@@ -377,7 +377,9 @@ void launch_queue(const void* xp, const void* W, const void* scales, float* part
     Q_RUN(2);
     Q_RUN(3);
     Q_RUN(4);
+    Q_RUN(5);
     Q_RUN(6);
+    Q_RUN(7);
     Q_RUN(8);
   }
 #undef Q_RUN
