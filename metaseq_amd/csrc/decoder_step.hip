@@ -60,9 +60,10 @@ Splits pick_splits(const msa_decoder* d, int B) {
   return s;
 }
 
-StepBuffers carve(const msa_decoder* d, int B, const Splits& sp, char* base) {
+constexpr int MAX_SPLITS = 8;  // of pick_splits
+
+StepBuffers carve(const msa_decoder* d, int B, char* base) {
   const int64_t D = d->cfg.d_model, F = d->cfg.ffn, MP = packed_row_blocks(B) * 16;
-  const int64_t S = sp.out > sp.fc2 ? sp.out : sp.fc2;
   StepBuffers w{};
   int64_t off = 0;
   auto take = [&](int64_t n) {
@@ -76,7 +77,7 @@ StepBuffers carve(const msa_decoder* d, int B, const Splits& sp, char* base) {
   w.h = take(MP * D * 2);
   w.o = take(MP * D * 2);
   w.u = take(MP * F * 2);
-  w.part = take(S * B * D * 4);
+  w.part = take(MAX_SPLITS * B * D * 4);  // (more rows can take fewer slices: 32 of 2048 eight, 33 four)
   w.positions = take(B * 8);
   w.step_len = take(B * 4);
   // up to 64 rows the selection runs inside the vocabulary projection (partials per workgroup);
@@ -144,7 +145,7 @@ extern "C" void msa_decoder_destroy(msa_decoder* d) {
 
 extern "C" int64_t msa_decoder_step_workspace_bytes(msa_decoder* d, int B) {
   if (!d || B < 1 || B > MSA_PACKED_MAX_ROWS) return 0;
-  return carve(d, B, pick_splits(d, B), nullptr).bytes;
+  return carve(d, B, nullptr).bytes;
 }
 
 extern "C" int msa_decoder_step(msa_decoder* d, const msa_step_args* a, void* stream) {
@@ -161,7 +162,7 @@ extern "C" int msa_decoder_step(msa_decoder* d, const msa_step_args* a, void* st
   MSA_REQUIRE((a->flags & ~(MSA_EMBED_COL_FROM_LEN | MSA_STEP_NO_ADVANCE)) == 0,
               MSA_ERR_INVALID_ARG, "%s: unsupported flags 0x%x", name, a->flags);
   const Splits sp = pick_splits(d, B);
-  const StepBuffers w = carve(d, B, sp, (char*)a->workspace);
+  const StepBuffers w = carve(d, B, (char*)a->workspace);
   MSA_REQUIRE(a->workspace_bytes >= w.bytes, MSA_ERR_CAPACITY,
               "%s: workspace of %lld bytes, %lld needed", name, (long long)a->workspace_bytes,
               (long long)w.bytes);

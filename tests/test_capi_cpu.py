@@ -69,6 +69,21 @@ def test_argument_validation_needs_no_gpu():
     assert b"leaves a K range empty" in lib.msa_last_error()
 
 
+@pytest.mark.parametrize("int8", [0, 1])
+@pytest.mark.parametrize("width", [768, 1024, 2048, 4096, 5120, 9216])
+def test_a_workspace_for_more_rows_serves_fewer(width, int8):
+    """... also where more rows are summed in fewer slices."""
+    lib, h, one = _capi.load(), ctypes.c_void_p(), ctypes.c_void_p(4096)
+    conf = _capi.DecoderConfig(1, width, width // 128, 4 * width, 512, 40, 1, int8)
+    table = (_capi.LayerWeights * 1)()
+    for name, _ in _capi.LayerWeights._fields_:
+        setattr(table[0], name, 4096)
+    assert lib.msa_decoder_create(ctypes.byref(conf), one, one, one, one, one, table, ctypes.byref(h)) == 0
+    need = [lib.msa_decoder_step_workspace_bytes(h, b) for b in range(16, 65)]
+    lib.msa_decoder_destroy(h)
+    assert need == sorted(need) and need[0] > 0
+
+
 def test_decoder_handle_is_host_only_bookkeeping():
     """msa_decoder_create validates and copies a pointer table without touching a GPU; the
     workspace size grows with the row count; a bad configuration or a missing pointer is
