@@ -2241,7 +2241,7 @@ bool launch_stream_ln(const LnTail& ln, int S, const void* W, const void* scales
 template <bool W8, int MODE, bool XR = false>
 void launch_stream(const void* xp, const void* W, const void* scales, float* part, int S, int M,
                    int N, int K, const Epilogue& epi, hipStream_t s, int64_t m_off = 0) {
-  // (the device is asked for once: 125m, one row, 278 us a step with three times as many questions, 270 with one more)
+  // (the runtime is asked for the device once: 125m, one row, 268 us a step, with two more questions to a product 278)
   const int cus = num_cus(), G = cus / S < 1 ? 1 : cus / S, tpw = (N / 16 + G - 1) / G;
   if constexpr (!XR && MODE != MODE_SELECT) {
     if (queue_takes(M, W8, tpw)) return launch_queue<W8, MODE>(xp, W, scales, part, S, M, N, K, tpw, epi, s);

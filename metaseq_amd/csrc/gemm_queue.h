@@ -18,10 +18,11 @@ namespace {
 // waves' sums are added through LDS in fixed order, as many tiles at a time as fit, and all waves take part in the epilogue.
 //
 // us, shared-activation kernel and this: fp16 57 x 16384 x 4096 33.3 and 26.9, 57 x 12288 x 4096 23.7 and 21.5, 64 x 20480 x 5120
-// 47.9 and 38.0, 64 x 36864 x 9216 114 and 104, 64 x 3072 x 768 7.7 and 5.1, 128 x 16384 x 4096 38 and 35, 70 rows 39 and 28.7,
-// 128 x 3072 x 768 12.5 and 6.3, 128 x 8192 x 2048 22 and 14.5; int8 64 x 36864 x 9216 75 and 65.6, 64 x 27648 x 9216 65 and 53,
-// 128 x 27648 x 9216 102 and 76, 96 x 28672 x 7168 82 and 55.  Against the stream kernel: int8 32 x 9216 x 36864 in four slices 74.5
-// and 56, 8 x 36864 x 9216 60 and 54; fp16 32 x 5120 x 20480 in four slices 39.9 and 33.3.
+// 47.9 and 38.0, 64 x 36864 x 9216 114 and 104, 64 x 3072 x 768 7.7 and 5.1, 72 x 16384 x 4096 35 and 28.1, 104 rows 35.3 and
+// 33.0, 128 rows 38 and 35, 128 x 3072 x 768 12.5 and 6.3, 128 x 8192 x 2048 22 and 14.5; int8 64 x 36864 x 9216 75 and 65.6, 64 x
+// 27648 x 9216 65 and 53, 72 x 36864 x 9216 126 and 70, 104 rows 127 and 87, 128 x 27648 x 9216 102 and 76.  Against the
+// stream kernel: int8 32 x 9216 x 36864 in four slices 74.5 and 56, 8 x 36864 x 9216 60 and 54; fp16 32 x 5120 x 20480 in four
+// slices 39.9 and 33.3.
 // Other numbers of waves (57 x 16384 x 4096): 4 28.4, 6 27.1, 10 27.4, 12 28.7, 16 31.4.
 template <int MB, bool W8, int NT>
 struct QueueCfg {

@@ -904,8 +904,8 @@ class TransformerDecoder(IncrementalDecoder):
                           len_dev=None, prompts=None, after=None, last=False):
         """``_rows_layer`` for at most 128 rows (a short prompt): the layer's GEMM inputs are
         produced in the packed activation layout by the kernels in front of them, so that qkv,
-        out_proj, fc1 and fc2 run on the weight-streaming kernels of the decode step (56 rows, OPT-6.7B
-        shapes: 25 / 12.6 / 30 / 30 us against 32 / 15 / 45 / 52 on row-major rows)."""
+        out_proj, fc1 and fc2 run on the packed kernels of the decode step (57 rows, OPT-6.7B
+        shapes: 22 / 12 / 27 / 26 us against 32 / 15 / 45 / 52 on row-major rows)."""
         cfg = self.cfg
         D, H, hd, F = (cfg.decoder_embed_dim, cfg.decoder_attention_heads, cfg.head_dim,
                        cfg.decoder_ffn_embed_dim)
