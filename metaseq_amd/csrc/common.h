@@ -52,6 +52,8 @@ bool msa_launch_group_quad(const msa_group_linear_args& a, hipStream_t stream);
 // the delta rule sixteen tokens at a time, for calls with scratch (delta_chunks.hip)
 int msa_launch_delta_chunks(const msa_delta_args& a, const msa_batch* b, float* scratch, hipStream_t stream);
 int msa_launch_linear_post(const msa_linear_args& a, hipStream_t stream);
+// compute units of the current device; 256 where there is none (gemm_bf16.hip)
+int msa_compute_units();
 
 #define MSA_REQUIRE(cond, code, ...) \
   do {                               \

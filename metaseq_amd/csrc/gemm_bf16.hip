@@ -24,6 +24,8 @@ bool run_grouped(const msa_group_linear_args& a, const Epilogue& e, hipStream_t 
 
 }  // namespace
 
+int msa_compute_units() { return num_cus(); }
+
 // Routed products over 256-row tiles (msa_group_linear).  Returns false if the launch is refused.
 bool msa_launch_group_quad(const msa_group_linear_args& a, hipStream_t s) {
   Epilogue e{};

@@ -9,6 +9,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
 #include <new>
 
 #include "common.h"
@@ -78,6 +79,7 @@ struct Run {
   bool dry;  // only measure the workspace
   bool f32;
   int M, mb, es;  // rows, row blocks of packed activations (0: row-major), bytes per element
+  int cus;        // compute units
   char* base;
   int64_t off, peak;
 
@@ -104,6 +106,16 @@ struct Run {
     return msa_linear_bf16(x.p, W, y, y32, M, N, x.ld, n32, glu, limit,
                            in_flags() | (y_act && mb > 0 ? MSA_OUT_PACKED : 0u), stream);
   }
+  // Rows of fp32 sums that these rows, or any fewer, leave: a workspace for more rows serves fewer, though slices fall where rows
+  // rise (32 rows of 2048 x 8192 are summed in eight, 33 in four).  Eight slices of packed rows; beyond, what the rules of
+  // slices stop at: eight over two rounds of 256 x 64 tiles, two over one round of 256 x 256.
+  int64_t sums(int N, int least) const {
+    if (f32) return M;
+    const int64_t packed = 8 * std::min<int64_t>(M, MSA_PACKED_MAX_ROWS);
+    if (mb > 0) return packed;
+    const int64_t eight = 512ll * cus / ((N + 63) / 64), two = 256ll * cus / ((N + 255) / 256);
+    return std::max({packed, (int64_t)M * least, std::min<int64_t>(8ll * M, eight), std::min<int64_t>(2ll * M, two)});
+  }
   // fp32 sums of S slices
   float* partial(const Act& x, const void* W, int N, int& S, int& rc, int least = 1) {
     S = f32 ? 1 : msa_linear_bf16_splits(M, N, x.ld, mb > 0);
@@ -111,7 +123,7 @@ struct Run {
       S = S > least ? S : least;
       while (S > least && x.ld % (64 * S)) S /= 2;
     }
-    float* part = (float*)alloc((int64_t)S * M * N * 4);
+    float* part = (float*)alloc(std::max((int64_t)S * M, sums(N, least)) * N * 4);
     rc = MSA_OK;
     if (dry) return part;
     if (f32)
@@ -489,14 +501,15 @@ int Run::feed_forward(const msa_hybrid_layer& l, msa_tail_args& t) {
             l.limit_shared));
   const int tile_rows = f32 ? 64 : routed_rows(P, E, c.Dp, l.ff_expert, mb > 0);
   const int max_tiles = P / tile_rows + (E < P ? E : P);
+  const int64_t most_tiles = P / 16 + (E < P ? E : P);  // (of any tile: fewer rows can have lower ones, and more of them)
   int32_t* ids = (int32_t*)alloc((int64_t)P * 4);
   float* w = (float*)alloc((int64_t)P * 4);
   float* sg = shared ? (float*)alloc((int64_t)M * 4) : nullptr;
   int32_t* perm = (int32_t*)alloc((int64_t)P * 4);
   int32_t* inverse = (int32_t*)alloc((int64_t)P * 4);
   int32_t* group_end = (int32_t*)alloc((int64_t)E * 4);
-  int32_t* tile_group = (int32_t*)alloc((int64_t)max_tiles * 4);
-  int32_t* tile_row = (int32_t*)alloc((int64_t)max_tiles * 4);
+  int32_t* tile_group = (int32_t*)alloc(most_tiles * 4);
+  int32_t* tile_row = (int32_t*)alloc(most_tiles * 4);
   int32_t* n_tiles = (int32_t*)alloc(4);
   void* eh = alloc((int64_t)P * l.ff_expert * es);
   void* ey = alloc((int64_t)P * c.Dp * es);
@@ -668,6 +681,7 @@ int start(Run& r, const msa_hybrid* d, const msa_hybrid_step_args* a, void* stre
   r.M = b.M;
   r.mb = !r.f32 && b.M <= MSA_PACKED_MAX_ROWS ? packed_row_blocks(b.M) : 0;
   r.es = r.f32 ? 4 : 2;
+  r.cus = msa_compute_units();
   r.base = dry ? nullptr : (char*)a->workspace;
   r.off = r.peak = 0;
   return MSA_OK;

@@ -84,6 +84,41 @@ def test_a_workspace_for_more_rows_serves_fewer(width, int8):
     assert need == sorted(need) and need[0] > 0
 
 
+FEED_FORWARDS = {"dense": dict(ff_kind=_capi.MSA_FF_DENSE), "relu2": dict(ff_kind=_capi.MSA_FF_RELU2),
+                 # hardly a row, some rows and many to an expert; with few experts and with a shared one
+                 "routed": dict(ff_kind=_capi.MSA_FF_MOE, experts=64, top=8, ff_expert=1408),
+                 "few experts": dict(ff_kind=_capi.MSA_FF_MOE, experts=12, top=2, ff_expert=128),
+                 "shared": dict(ff_kind=_capi.MSA_FF_MOE, experts=64, top=4, ff_expert=704, ff_shared=704)}
+
+
+@pytest.mark.parametrize("dtype", [0, 1], ids=["bf16", "fp32"])
+@pytest.mark.parametrize("ff", FEED_FORWARDS)
+@pytest.mark.parametrize("width", [128, 512, 1024, 2048, 4096])
+def test_a_hybrid_workspace_for_more_rows_serves_fewer(width, ff, dtype):
+    """... where more rows are summed in fewer slices, or routed in fewer tiles."""
+    lib, h = _capi.load_hybrid(), ctypes.c_void_p()
+    t, cfg = _capi.HybridLayer(), _capi.HybridConfigC()
+    for s in (t, cfg):
+        for name, kind in s._fields_:
+            if kind is ctypes.c_void_p:
+                setattr(s, name, 4096)      # never followed
+    t.kind, t.channels, t.blocks, t.taps, t.ko, t.n_in = _capi.MSA_MIX_RGLRU, width, 1, 4, width, 2 * width
+    t.n_groups, t.keep, t.router_scale, t.ff = 1, 1, 1.0, 4 * width
+    for name, value in FEED_FORWARDS[ff].items():
+        setattr(t, name, value)
+    t.n_ff_in = {"dense": 8 * width, "relu2": 4 * width}.get(ff, (2 * t.ff_shared + t.experts + 16) // 16 * 16)
+    cfg.dtype, cfg.layers, cfg.D, cfg.Dp, cfg.vocab, cfg.Vp, cfg.eps, cfg.n_runs = dtype, 1, width, width, 16, 16, 1e-6, 0
+    assert lib.msa_hybrid_create(ctypes.byref(cfg), (_capi.HybridLayer * 1)(t), ctypes.byref(h)) == 0, lib.msa_last_error()
+    need = []
+    for rows in list(range(1, 300)) + [384, 511, 512, 513, 768, 769, 1024, 1025, 2048, 2049, 4096, 4097]:
+        a = _capi.HybridStepArgs()
+        a.batch.M = a.batch.nseg = rows
+        a.batch.max_count = a.batch.key_bound = a.capacity = 1
+        need.append(lib.msa_hybrid_workspace_bytes(h, ctypes.byref(a)))
+    lib.msa_hybrid_destroy(h)
+    assert need == sorted(need) and need[0] > 0
+
+
 def test_decoder_handle_is_host_only_bookkeeping():
     """msa_decoder_create validates and copies a pointer table without touching a GPU; the
     workspace size grows with the row count; a bad configuration or a missing pointer is
