@@ -32,16 +32,20 @@ bool folds(const msa_decoder* d, int B, int S) {
 // workspace layout for B rows
 struct StepBuffers {
   char *x, *x2, *q, *h, *o, *u, *part, *positions, *step_len, *select_ws, *attn_ws, *logits;
-  int64_t attn_keys;  // key positions per (b, h) that attn_ws holds scores for (0: none)
+  int64_t attn_keys;  // key positions per (b, h) that attn_ws holds scores for (0: none), of as many rows as can be split
   int64_t bytes;
 };
 
 // most keys the split attention's score buffer is sized for
-int64_t split_attention_keys(const msa_decoder* d, int B) {
-  const int hd = d->cfg.d_model / d->cfg.heads;
-  const int64_t keys = d->cfg.n_pos_rows < 8192 ? d->cfg.n_pos_rows : 8192;
-  // the form can only ever be chosen for few (b, h) pairs; ask with the longest history
-  return msa_attention_prefers_split(B, d->cfg.heads, hd, (int)keys) ? keys : 0;
+int64_t split_attention_keys(const msa_decoder* d) {
+  return d->cfg.n_pos_rows < 8192 ? d->cfg.n_pos_rows : 8192;
+}
+// and its rows: the form can only ever be chosen for few (b, h) pairs; ask with the longest history
+int split_attention_rows(const msa_decoder* d, int B) {
+  const int hd = d->cfg.d_model / d->cfg.heads, keys = (int)split_attention_keys(d);
+  if (!msa_attention_prefers_split(1, d->cfg.heads, hd, keys)) return 0;
+  while (!msa_attention_prefers_split(B, d->cfg.heads, hd, keys)) --B;
+  return B;
 }
 
 // split-K counts of out_proj and fc2 for B rows.  Computed per call (a few integer operations) and
@@ -62,6 +66,7 @@ Splits pick_splits(const msa_decoder* d, int B) {
 
 constexpr int MAX_SPLITS = 8;  // of pick_splits
 
+// A workspace for more rows serves fewer: every buffer is as large as any fewer rows need it.
 StepBuffers carve(const msa_decoder* d, int B, char* base) {
   const int64_t D = d->cfg.d_model, F = d->cfg.ffn, MP = packed_row_blocks(B) * 16;
   StepBuffers w{};
@@ -72,7 +77,7 @@ StepBuffers carve(const msa_decoder* d, int B, char* base) {
     return p;
   };
   w.x = take(B * D * 2);
-  w.x2 = take(B * D * 2);  // (at any B: a workspace for more rows serves fewer)
+  w.x2 = take(B * D * 2);
   w.q = take(B * D * 2);
   w.h = take(MP * D * 2);
   w.o = take(MP * D * 2);
@@ -82,10 +87,11 @@ StepBuffers carve(const msa_decoder* d, int B, char* base) {
   w.step_len = take(B * 4);
   // up to 64 rows the selection runs inside the vocabulary projection (partials per workgroup);
   // beyond, the projection stores its logits and a second kernel selects from them
-  w.select_ws = take(B <= 64 ? msa_lm_head_select_workspace_bytes(B) : 0);
-  w.logits = take(B <= 64 ? 0 : (int64_t)B * d->cfg.vocab * 2);
-  w.attn_keys = split_attention_keys(d, B);
-  w.attn_ws = take(msa_attention_split_workspace_bytes(B, d->cfg.heads, (int)w.attn_keys));
+  const int64_t select = msa_lm_head_select_workspace_bytes(B < 64 ? B : 64), logits = B <= 64 ? 0 : (int64_t)B * d->cfg.vocab * 2;
+  w.select_ws = w.logits = take(select > logits ? select : logits);
+  const int attn_rows = split_attention_rows(d, B);
+  w.attn_keys = attn_rows > 0 ? split_attention_keys(d) : 0;
+  w.attn_ws = take(msa_attention_split_workspace_bytes(attn_rows, d->cfg.heads, (int)w.attn_keys));
   w.bytes = off;
   return w;
 }

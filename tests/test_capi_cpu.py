@@ -70,16 +70,17 @@ def test_argument_validation_needs_no_gpu():
 
 
 @pytest.mark.parametrize("int8", [0, 1])
-@pytest.mark.parametrize("width", [768, 1024, 2048, 4096, 5120, 9216])
-def test_a_workspace_for_more_rows_serves_fewer(width, int8):
-    """... also where more rows are summed in fewer slices."""
+@pytest.mark.parametrize("vocab,positions", [(512, 40), (50272, 2050), (512, 8194)])
+@pytest.mark.parametrize("width", [128, 768, 1024, 2048, 4096, 5120, 9216])
+def test_a_workspace_for_more_rows_serves_fewer(width, vocab, positions, int8):
+    """... also where more rows are summed in fewer slices, where no two launches attend to them or no projection selects."""
     lib, h, one = _capi.load(), ctypes.c_void_p(), ctypes.c_void_p(4096)
-    conf = _capi.DecoderConfig(1, width, width // 128, 4 * width, 512, 40, 1, int8)
+    conf = _capi.DecoderConfig(1, width, width // 128, 4 * width, vocab, positions, 1, int8)
     table = (_capi.LayerWeights * 1)()
     for name, _ in _capi.LayerWeights._fields_:
         setattr(table[0], name, 4096)
     assert lib.msa_decoder_create(ctypes.byref(conf), one, one, one, one, one, table, ctypes.byref(h)) == 0
-    need = [lib.msa_decoder_step_workspace_bytes(h, b) for b in range(16, 65)]
+    need = [lib.msa_decoder_step_workspace_bytes(h, b) for b in range(1, 129)]
     lib.msa_decoder_destroy(h)
     assert need == sorted(need) and need[0] > 0
 
