@@ -61,15 +61,15 @@ struct Act {
 // tokens 121, 121; 260 tokens 150, 122.
 // Where there are fewer tiles than compute units (256 columns each from 64 rows on), low tiles have more workgroups to
 // spread the rows over: experts of 128, width 512, 140 tokens 11.2 in tiles of 16, 23 of 64 and 26 of 256.
-int routed_rows(int P, int E, int width, int ff, bool packed) {
+// The 256-row kernel reaches 4 GB of rows, the others any number.
+int routed_rows(int P, int E, int width, int ff, bool packed, int cus) {
   const int avg = P / E;
-  if ((int64_t)(E < P ? E : P) * ((2 * ff + 255) / 256) < 256)
-    return avg <= 16 ? 16 : avg <= 32 ? 32 : avg <= 64 || packed ? 64 : 256;
+  const int tall = packed || (int64_t)P * std::max(width, ff) * 2 >= (1ll << 32) ? 64 : 256;
+  if ((int64_t)std::min(E, P) * ((2 * ff + 255) / 256) < cus) return avg <= 16 ? 16 : avg <= 32 ? 32 : avg <= 64 ? 64 : tall;
   if (P <= 8 * (int64_t)E) return 16;
   if (packed) return 64;
   if (width <= 2048 && avg <= 24) return 32;
-  const int64_t K = width > ff ? width : ff;
-  return avg <= 16 || (avg <= 64 && P * K * 2 >= (1ll << 32)) ? 64 : 256;
+  return avg <= 16 ? 64 : tall;
 }
 
 struct Run {
@@ -499,7 +499,7 @@ int Run::feed_forward(const msa_hybrid_layer& l, msa_tail_args& t) {
   // the shared expert's hidden layer, the router logits and the shared gate's logit in one product
   HY(linear(h, l.w_ff_in, u.p, true, z, l.n_ff_in, n32, shared ? MSA_GLU_CLAMPED : MSA_GLU_NONE,
             l.limit_shared));
-  const int tile_rows = f32 ? 64 : routed_rows(P, E, c.Dp, l.ff_expert, mb > 0);
+  const int tile_rows = f32 ? 64 : routed_rows(P, E, c.Dp, l.ff_expert, mb > 0, cus);
   const int max_tiles = P / tile_rows + (E < P ? E : P);
   const int64_t most_tiles = P / 16 + (E < P ? E : P);  // (of any tile: fewer rows can have lower ones, and more of them)
   int32_t* ids = (int32_t*)alloc((int64_t)P * 4);

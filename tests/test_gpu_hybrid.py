@@ -2,13 +2,14 @@
 decoding, batches of unequal requests, re-used slots, single keys that must or must not be seen,
 long memories, and generation through the framework's own entry points."""
 import json
+from types import SimpleNamespace
 
 import numpy as np
 import pytest
 import torch
 
-from metaseq_amd import (Dictionary, GeneratorInterface, SequenceGenerator,
-                         TransformerLanguageModel)
+from metaseq_amd import (Dictionary, GeneratorInterface, HybridConfig, HybridDecoder, SequenceGenerator,
+                         TransformerLanguageModel, random_hybrid_state_dict)
 from metaseq_amd import generate, trace_run
 from metaseq_amd.service import ContinuousBatcher
 from oracle import hybrid_oracle as O
@@ -54,6 +55,19 @@ def test_mechanism_alone(name, dtype):
         case.check(case.run(t), want, "%s, %d tokens" % (name, n), close)
         case.check(case.run(t, [max(1, n - 6), 1]), want, "%s, %d tokens, decoded" % (name, n),
                    close)
+
+
+def test_more_routed_rows_than_a_tall_tile_reaches():
+    """4096 tokens of 64 experts each, 8192 wide: 4 GB of rows, which 256-row tiles do not reach, against two halves."""
+    cfg = HybridConfig.from_json(H.config([(H.rglru(width=64, blocks=2), H.moe(experts=64, top=64, groups=None, ff=128, shared=None))],
+                                          width=8192))
+    d = HybridDecoder(cfg, random_hybrid_state_dict(cfg, 41), device="cuda", dtype=BF16)
+    t = torch.randint(4, cfg.vocab_size, (4096,), generator=torch.Generator().manual_seed(3)).cuda()
+    got = []
+    for n in (4096, 2048):
+        cache = d.new_slot_cache(1, 4096)
+        got.append(torch.cat([d.extend(cache, [(0, piece)], want_all=True) for piece in t.split(n)]))
+    H.Case.check(SimpleNamespace(dtype=BF16), got[0], got[1], "4 GB of routed rows")
 
 
 @DTYPES
