@@ -2824,26 +2824,30 @@ int pick_splits(int64_t M, int N, int K, int wbytes, int most = 8) {
   // shared-activation kernel for up to 18), and K steps per stage of the workgroup
   const int NT = MB > 2 ? (w8 && MB <= 4 ? SH_GROUP_W8 : SH_GROUP) : ST_NT;
   const int cus = num_cus();
-  int best = 1;
+  auto tiles = [&](int S) { return (ntiles + cus / S - 1) / (cus / S); };
+  auto cost = [&](int S, bool queue) {
+    const int tpw = tiles(S), groups = (tpw + NT - 1) / NT, rows = queue_rows((int)M);
+    const double Ks = (double)K / S, w = tpw * 16.0 * Ks * wbytes;
+    double c = queue ? w + 0.45 * rows * 16.0 * Ks * 2 + 6500.0 * tpw * rows + 5.1 * S * N
+                     : w + groups * MB * 16.0 * Ks * 2 + 2.0 * tpw * 16 * M * 4;
+    if (!queue || MB <= 2) c *= 1.0 + 0.02 * S;  // ties go to fewer splits (fewer partial slices to sum)
+    if (!queue && MB > 2) c *= 2;                // the shared-activation kernel takes what is left
+    return c;
+  };
+  // Up to 32 rows fewer slices than the stream kernel would take only in queues: its waves' chains would be as much longer (fp16, 32
+  // rows of 5120 x 5120, fp32 sums off by 1.09e-7 in four slices, in two by 1.32e-7; and 15.9 us with the tail in queues, 16.3).
+  int best = 1, least = 1;
+  if (MB <= 2)
+    for (int S = 2; S <= most && S <= cus && nks / S >= ST_KG * 4; S *= 2)
+      if (cost(S, false) < cost(least, false)) least = S;
   double best_cost = 0;
-  for (int S = 1; S <= most; S *= 2) {
-    const int G = cus / S;
-    if (G < 1) break;
-    const int tpw = (ntiles + G - 1) / G;
-    const bool queue = queue_takes((int)M, w8, tpw);
+  for (int S = 1; S <= most && S <= cus; S *= 2) {
+    const bool queue = queue_takes((int)M, w8, tiles(S));
     const int stage = !queue ? (MB > 2 ? 16 : ST_KG * 4) : MB > 2 ? 8 * (w8 ? 2 : 1) : ST_KG * 4;
     if (nks / S < stage) break;  // every wave needs a full stage of K steps
-    const int groups = (tpw + NT - 1) / NT;
-    const double Ks = (double)K / S, w = tpw * 16.0 * Ks * wbytes;
-    const int rows = queue_rows((int)M);
-    double cost = queue ? w + 0.45 * rows * 16.0 * Ks * 2 + 6500.0 * tpw * rows + 5.1 * S * N
-                        : w + groups * MB * 16.0 * Ks * 2 + 2.0 * tpw * 16 * M * 4;
-    if (!queue || MB <= 2) cost *= 1.0 + 0.02 * S;  // ties go to fewer splits (fewer partial slices to sum)
-    if (!queue && MB > 2) cost *= 2;                // the shared-activation kernel takes what is left
-    if (S == 1 || cost < best_cost) {
-      best = S;
-      best_cost = cost;
-    }
+    if (!queue && S < least) continue;
+    const double c = cost(S, queue);
+    if (best_cost == 0 || c < best_cost) best = S, best_cost = c;
   }
   return best;
 }

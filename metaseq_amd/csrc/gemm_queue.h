@@ -16,6 +16,10 @@ namespace {
 // slot covers two steps).  A slot is read into registers, requested anew, and then multiplied.  Every activation
 // still comes to the CU once.  Two waves per SIMD where the sums and a slot fit 256 registers, one where they do not.  The
 // waves' sums are added through LDS in fixed order, as many tiles at a time as fit, and all waves take part in the epilogue.
+// Up to two row blocks take half or a quarter of the slices here that the stream kernel would take (pick_splits): a wave's sums
+// are set aside up to four times on its way, so that none is a longer chain than that kernel's.  fp32 sums, off by (stream kernel's
+// slices / fewer, one chain / set aside): int8 32 x 9216 x 36864 1.74e-7 / 2.28 / 1.39, fp16 24 x 5120 x 20480 1.42 / 1.76 / 1.27, 32 x
+// 12288 x 12288 1.45 / 1.89 / 1.27; 0.1 to 0.6 us (with its tail the first 62.0 and 62.5, the second 37.0 and 37.2).
 //
 // us, shared-activation kernel and this: fp16 57 x 16384 x 4096 33.3 and 26.9, 57 x 12288 x 4096 23.7 and 21.5, 64 x 20480 x 5120
 // 47.9 and 38.0, 64 x 36864 x 9216 114 and 104, 64 x 3072 x 768 7.7 and 5.1, 72 x 16384 x 4096 35 and 28.1, 104 rows 35.3 and
@@ -29,8 +33,9 @@ struct QueueCfg {
   static constexpr int STEPS = W8 ? 2 : 1;       // 32-wide steps of a slot
   static constexpr int LOADS = STEPS * MB + NT;  // of 1 KB each
   static constexpr int SLOT = LOADS * 1024;
+  static constexpr bool ASIDE = MB <= 2;  // sums are set aside after a quarter of the slots, of eight 32-wide steps at least
   // registers: sums, one slot's fragments, and some for addresses and the expansion of int8
-  static constexpr int REGS = 4 * (MB * NT + LOADS) + (W8 ? 20 : 8);
+  static constexpr int REGS = 4 * ((ASIDE ? 2 : 1) * MB * NT + LOADS) + (W8 ? 20 : 8);
   static constexpr int KL = REGS <= 256 && 8 * SLOT <= 160 * 1024 ? 8 : 4;
   static constexpr int FIT = 160 * 1024 / (KL * SLOT), R = FIT > 4 ? 4 : FIT;
   static constexpr int JFIT = 160 * 1024 / (KL * MB * 1024), J = JFIT > NT ? NT : JFIT;  // tiles summed at a time
@@ -97,11 +102,11 @@ __global__ __launch_bounds__((QueueCfg<MB, W8, NT>::KL * 64)) void linear_queue_
     });
   };
 
-  float4_t acc[NT][MB];
+  float4_t acc[NT][MB], aside[C::ASIDE ? NT : 1][MB];
 #pragma unroll
   for (int j = 0; j < NT; ++j)
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) acc[j][mb] = float4_t{0.f, 0.f, 0.f, 0.f};
+    for (int mb = 0; mb < MB; ++mb) acc[j][mb] = aside[C::ASIDE ? j : 0][mb] = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int r = 0; r < R; ++r)
     if (r < n) request(r, r);
@@ -109,7 +114,8 @@ __global__ __launch_bounds__((QueueCfg<MB, W8, NT>::KL * 64)) void linear_queue_
 #pragma unroll
   for (int j = 0; j < NT; ++j)
     if (W8) asm volatile("" : "+v"(sc[j]));
-  int slot = 0;
+  const int quarter = max((n + 3) / 4, 8 / STEPS);
+  int slot = 0, until = quarter;
   for (int i = 0; i < n; ++i) {
     // loads complete in order: slot i is there when no more than those of the R - 1 slots behind it are on their way
     if (i + R - 1 < n)
@@ -141,6 +147,20 @@ __global__ __launch_bounds__((QueueCfg<MB, W8, NT>::KL * 64)) void linear_queue_
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) acc[j][mb] = mfma_16x16x32<MODE>(a, x[u * MB + mb], acc[j][mb]);
       }
+    if constexpr (C::ASIDE)
+      if (--until == 0) {
+        until = quarter;
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+          for (int mb = 0; mb < MB; ++mb) aside[j][mb] += acc[j][mb], acc[j][mb] = float4_t{0.f, 0.f, 0.f, 0.f};
+      }
+  }
+  if constexpr (C::ASIDE) {
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) acc[j][mb] += aside[j][mb];
   }
 
   // the waves' sums in wave order, J tiles at a time: [wave][tile][row block][lane]

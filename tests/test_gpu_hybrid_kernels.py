@@ -124,6 +124,24 @@ def test_fp32_logits_of_a_vocabulary_are_no_single_chain_over_k(M, K, most):
     assert float((y.double() - want).norm() / want.norm()) <= most
 
 
+@pytest.mark.parametrize("M,N,K,most", [(24, 5120, 20480, 1.26e-7), (32, 9216, 9216, 1.16e-7), (32, 2560, 10240, 1.06e-7)])
+def test_fp32_sums_of_few_rows_are_no_longer_chains(M, N, K, most):
+    """In the number of slices that is suggested; `most`: what the stream kernel's sums have (in twice the slices, or as many)."""
+    lib = _capi.load_hybrid()
+    g = torch.Generator("cuda").manual_seed(M + N)
+    x = torch.randn(M, K, generator=g, device="cuda").to(BF16)
+    w = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).to(BF16)
+    S = lib.msa_linear_bf16_splits(M, N, K, 1)
+    part = torch.full((S, M, N), float("nan"), device="cuda")
+    check(lib.msa_linear_partial_bf16(ptr(pack_rows(x.cpu()).cuda()), ptr(pack_tiles(w)), ptr(part), M, N, K, S,
+                                      _capi.MSA_IN_PACKED, _capi.stream_ptr()), lib)
+    got = part[0].clone()
+    for s in range(1, S):
+        got += part[s]
+    want = x.double() @ w.double().t()
+    assert float((got.double() - want).norm() / want.norm()) <= most
+
+
 @pytest.mark.parametrize("M,N", [(4352, 16656), (600, 24576)])
 def test_linear_partial_bf16_wide_panels(M, N):
     """More than 64 columns of tiles, taken in panels of 16; sums of one and two slices."""

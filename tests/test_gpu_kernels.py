@@ -485,6 +485,37 @@ def test_linear_packed_rows_in_queues(lib, M, N, K, w8):
     assert_fp16_close(y, want, atol=float(want.abs().max()) * 2 ** -10, what="queue")
 
 
+# in the number of slices that is suggested; `most`: what the stream kernel's sums have (in twice the slices, or as many)
+@pytest.mark.parametrize("M,N,K,w8,most", [
+    (32, 9216, 36864, True, 1.76e-7), (16, 5120, 20480, True, 1.43e-7), (8, 12288, 12288, True, 1.47e-7), (24, 9216, 9216, True, 1.33e-7),
+    (24, 5120, 20480, False, 1.43e-7), (32, 5120, 5120, False, 1.11e-7), (17, 7168, 7168, False, 1.22e-7), (32, 2560, 10240, False, 1.19e-7)])
+def test_fp32_sums_of_few_rows_are_no_longer_chains(lib, M, N, K, w8, most):
+    """The error of fp32 sums grows with the root of the additions behind each."""
+    print("sums", M, N, K, w8, flush=True)
+    g = torch.Generator(DEV).manual_seed(M + N)
+    x = torch.randn(M, K, generator=g, device=DEV).half()
+    xp = G(pack_act(x.cpu()))
+    if w8:
+        q = torch.randint(-127, 128, (N, K), generator=g, device=DEV, dtype=torch.int8)
+        sc = (torch.rand(N, generator=g, device=DEV) * 0.01 + 0.01).half()
+        w, S = (q.float() * sc.float().unsqueeze(1)).half(), lib.msa_linear_default_splits_w8a16(M, N, K)
+    else:
+        w, S = (torch.randn(N, K, generator=g, device=DEV) * K ** -0.5).half(), lib.msa_linear_default_splits(M, N, K)
+    part = torch.full((S, M, N), float("nan"), device=DEV)
+    if w8:
+        ok(lib.msa_linear_partial_w8a16(P(xp), P(pack_w8(lib, q)), P(sc), P(part), M, N, K, S, IN_PACKED, None), lib)
+    else:
+        ok(lib.msa_linear_partial_f16(P(xp), P(pack_w(lib, w)), P(part), M, N, K, S, IN_PACKED, None), lib)
+    torch.cuda.synchronize()
+    got = part[0].clone()
+    for s in range(1, S):
+        got += part[s]
+    want = torch.cat([x.double() @ rows.double().t() for rows in w.split(2048)], 1)
+    err = float((got.double() - want).norm() / want.norm())
+    print(S, "slices", err, flush=True)
+    assert err <= most
+
+
 # 129 .. 256 row-major rows in queues: every number of row blocks and of tiles to a workgroup (256 compute units), the last
 # columns' workgroup with fewer, blocks whose rows run out, fewer 64-wide stages than waves and more than a queue holds
 QUEUE_ROWS = [(129, 16, 128), (160, 2064, 192), (161, 3072, 768), (192, 4112, 576), (193, 6160, 1088), (224, 8192, 320),
