@@ -113,6 +113,9 @@ int msa_moe_route(const float* z, int ldz, int M, int E, int n_groups, int keep,
 int msa_moe_plan(const int32_t* ids, int P, int E, int tile_rows, int32_t* perm, int32_t* inverse,
                  int32_t* group_end, int32_t* tile_group, int32_t* tile_row, int32_t* n_tiles,
                  int max_tiles, void* stream);
+/* The tile_rows that a step takes (bf16): P pairs over E experts of hidden size ff, `packed` activations of at most 128
+ * tokens or row-major ones; cus: compute units, 0: the device's. */
+int msa_moe_tile_rows(int P, int E, int width, int ff, int packed, int cus);
 
 /* e = table[token] * scale + sinusoid(pos), x = e + step, h = rmsnorm(x) * w (activation format).
  * table: bf16 [vocab, Dp]; inv_freq: double [(D + 1) / 2], the angle per position of column pair i (NULL:

@@ -201,6 +201,7 @@ HYBRID_SIGNATURES = {
     "msa_linear_bf16_splits": [c_int64, c_int, c_int, c_int],
     "msa_group_linear": [ctypes.POINTER(GroupLinearArgs), _P],
     "msa_moe_route": [_P, c_int, c_int, c_int, c_int, c_int, c_int, c_float, _P, _P, _P, _P],
+    "msa_moe_tile_rows": [c_int, c_int, c_int, c_int, c_int, c_int],
     "msa_moe_plan": [_P, c_int, c_int, c_int, _P, _P, _P, _P, _P, _P, c_int, _P],
     "msa_embed_rmsnorm": [c_int, _P, _P, c_int, _P, c_int, c_float, _P, c_int, c_int, c_float, _P,
                           _P, _P, _P, _P, c_int, _P],

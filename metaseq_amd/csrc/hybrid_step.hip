@@ -55,21 +55,30 @@ struct Act {
 // TB/s, of 64 at 5 to 6, the 256-row kernel, whose tiles are as high as an expert's rows need, at 5.5 to 5.8.  Both products of
 // 64 experts of 1408, width 4096, us, by tokens of which each has eight experts: 48 tokens in tiles of 16 rows 346, of 64 383; 64
 // tokens 374, 393; 96 tokens 459, 412; 128 tokens 543 (of 32 rows 537), 437; 160 tokens of 32 rows 445, 64 413, 256 389; 256
-// tokens of 32 rows 583, 64 462, 256 395; 320 tokens of 64 506, 256 404; 512 tokens 760, 427.  (Packed rows are no input of the
-// 256-row kernel, and 16 of them gathered into a fragment are four times the lines of row-major ones: tiles of 32 gain nothing.)
-// Up to 2048 wide an expert's product is short, and row-major tiles of 32 are ahead for longer: 150 tokens 109, of 256 120; 200
-// tokens 121, 121; 260 tokens 150, 122.
-// Where there are fewer tiles than compute units (256 columns each from 64 rows on), low tiles have more workgroups to
-// spread the rows over: experts of 128, width 512, 140 tokens 11.2 in tiles of 16, 23 of 64 and 26 of 256.
-// The 256-row kernel reaches 4 GB of rows, the others any number.
+// tokens of 32 rows 583, 64 462, 256 395; 320 tokens of 64 506, 256 404; 512 tokens 760, 427.
+// From 64 rows on a workgroup has 256 columns.  Where the narrower product has fewer of them than two to a compute unit, tiles
+// of 16 and 32 rows, whose workgroups have 32 columns, are ahead for longer, and of fewer than one for as long as there are few
+// rows at all (16 / 32 / 64 / 256 rows): 16 experts of 2816, width 512, 66 tokens 35 / 37 / 90, width 1024, 200 tokens 83 / 65 / 119 /
+// 93, width 3072, 260 tokens 255 / 220 / 226 / 166; 64 experts of 704, width 2048, 72 tokens 107 / 102 / 112, 96 tokens 120 / 116 / 118,
+// 200 tokens 157 / 122 / 124 / 122; 128 experts of 128 in 512, 140 tokens 11.2 in tiles of 16, 23 of 64 and 26 of 256.  A stage of 32 rows is half
+// of a sum of 512 (128 experts of 1408, 150 tokens 100 / 113).  Over 1092 pairs of tokens (33 to 1000) and layers (512 to 4096
+// wide, 16 to 128 experts of 256 to 2816) the tile chosen is 1.1 % slower than the best on average; heights by the rows alone, 16,
+// 32, 64, 256, were 11 %.
+// The 256-row kernel takes no packed rows and reaches 4 GB of them, the others any number.  The choice is one of speed: 64 and
+// 256 rows are one chain of sums over K, 16 and 32 four, and the results, bf16, are as far from 64 bits either way (K = 8192, 24
+// rows to an expert: 1.6605538e-3 from all four).
 int routed_rows(int P, int E, int width, int ff, bool packed, int cus) {
   const int avg = P / E;
   const int tall = packed || (int64_t)P * std::max(width, ff) * 2 >= (1ll << 32) ? 64 : 256;
-  if ((int64_t)std::min(E, P) * ((2 * ff + 255) / 256) < cus) return avg <= 16 ? 16 : avg <= 32 ? 32 : avg <= 64 ? 64 : tall;
+  const int64_t columns = (std::min(2 * ff, width) + 255) / 256, groups = std::min(E, P) * columns;
   if (P <= 8 * (int64_t)E) return 16;
-  if (packed) return 64;
-  if (width <= 2048 && avg <= 24) return 32;
-  return avg <= 16 ? 64 : tall;
+  if (groups >= 2 * cus) {
+    if (packed) return 64;
+    return avg <= 12 ? 32 : avg <= (width <= 3072 ? 24 : 16) ? 64 : tall;
+  }
+  if ((packed && avg < 10) || (width <= 512 && avg <= 16)) return 16;
+  if (groups < cus) return P * columns <= 14 * (int64_t)cus ? 32 : tall;
+  return avg <= (packed ? 11 : width <= 2048 ? 24 : 16) ? 32 : tall;
 }
 
 struct Run {
@@ -796,6 +805,11 @@ extern "C" int msa_hybrid_create(const msa_hybrid_config* cfg, const msa_hybrid_
   d->cfg.run_layer = d->cfg.run_pass = nullptr;
   *out = d;
   return MSA_OK;
+}
+
+extern "C" int msa_moe_tile_rows(int P, int E, int width, int ff, int packed, int cus) {
+  if (P < 1 || E < 1 || width < 1 || ff < 1) return 0;
+  return routed_rows(P, E, width, ff, packed != 0, cus > 0 ? cus : msa_compute_units());
 }
 
 extern "C" void msa_hybrid_destroy(msa_hybrid* d) {

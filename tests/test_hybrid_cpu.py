@@ -315,6 +315,19 @@ def test_a_step_reserves_what_the_delta_rule_takes(heads, vdim, short, long, per
     lib.msa_hybrid_destroy(h)
 
 
+@pytest.mark.parametrize("tokens,top,E,width,ff,rows", [
+    # low tiles where tall ones have too few workgroups, in either product
+    (66, 2, 16, 512, 2816, 16), (128, 2, 16, 1024, 2816, 32), (200, 2, 16, 1024, 2816, 32), (66, 8, 64, 2048, 704, 16),
+    (80, 4, 32, 1024, 1408, 32), (66, 8, 64, 512, 1408, 16), (260, 2, 16, 3072, 256, 32), (520, 2, 16, 2048, 1408, 256),
+    # and tall ones where they have enough
+    (32, 8, 64, 4096, 1408, 16), (80, 8, 64, 4096, 1408, 64), (96, 8, 64, 1024, 1408, 64), (150, 8, 64, 2048, 1408, 64),
+    (160, 8, 64, 4096, 1408, 256), (700, 8, 64, 2048, 704, 256),
+    # 4 GB of rows
+    (4095, 64, 64, 8192, 128, 256), (4096, 64, 64, 8192, 128, 64), (32768, 8, 64, 8192, 1408, 64)])
+def test_rows_to_a_tile_of_routed_products(tokens, top, E, width, ff, rows):
+    assert _capi.load_hybrid().msa_moe_tile_rows(tokens * top, E, width, ff, tokens <= 128, 256) == rows
+
+
 @pytest.mark.parametrize("vp", [16, 48, 64, 80, 96, 128, 256])
 @pytest.mark.parametrize("dp", [32, 64, 96, 128])
 def test_scratch_of_the_delta_rule_is_bounded(dp, vp):
