@@ -2815,7 +2815,10 @@ int check_linear_args(const char* name, const void* x, const void* W, const void
 // In the queue kernel activations, which come from L2, cost half of as many weights, and a tile's sums more than the bytes they
 // leave as: eight waves' go through LDS behind the loop.  Fitted to 130 products of 40 to 128 rows with their tails (us = 5 +
 // 0.0278 per KB of weights + 0.0126 per KB of activations + 0.18 per 16 x 16 sums + 0.14 per 1000 of slices x columns, to 4.5 %);
-// what it picks is 0.7 % slower than the best of 2, 4 and 8 slices on average.
+// The shared-activation kernel in one pass, of nine to twelve tiles, has its waves' sums added by two, not eight: fp16, 128 rows with
+// their tails, us, in two slices of queues and in four of it, 12288 x 12288 71 and 66, x 49152 233 and 211, 9216 x 36864 154 and 145,
+// 64 rows of 12288 x 49152 197 and 191, of 12288 x 12288 58 and 61; int8, 64 rows of 12288 x 49152 124 and 119, 128 rows 163 and 184.  What
+// is picked is 0.3 % slower than the best of 1, 2, 4 and 8 slices on average over 190 products of 40 to 128 rows.
 int pick_splits(int64_t M, int N, int K, int wbytes, int most = 8) {
   if (M < 1 || M > MSA_PACKED_MAX_ROWS || N % 16 || K % 64) return 1;
   const bool w8 = wbytes == 1;
@@ -2827,15 +2830,15 @@ int pick_splits(int64_t M, int N, int K, int wbytes, int most = 8) {
   auto tiles = [&](int S) { return (ntiles + cus / S - 1) / (cus / S); };
   auto cost = [&](int S, bool queue) {
     const int tpw = tiles(S), groups = (tpw + NT - 1) / NT, rows = queue_rows((int)M);
-    const double Ks = (double)K / S, w = tpw * 16.0 * Ks * wbytes;
-    double c = queue ? w + 0.45 * rows * 16.0 * Ks * 2 + 6500.0 * tpw * rows + 5.1 * S * N
-                     : w + groups * MB * 16.0 * Ks * 2 + 2.0 * tpw * 16 * M * 4;
-    if (!queue || MB <= 2) c *= 1.0 + 0.02 * S;  // ties go to fewer splits (fewer partial slices to sum)
-    if (!queue && MB > 2) c *= 2;                // the shared-activation kernel takes what is left
-    return c;
+    const double Ks = (double)K / S, w = tpw * 16.0 * Ks * wbytes, x = rows * 16.0 * Ks * 2, part = 5.1 * S * N;
+    if (MB > 2 && queue) return w + 0.45 * x + 6500.0 * tpw * rows + part;
+    if (MB > 2 && tpw <= SH_GROUP && (MB <= 4 || !w8)) return 1.05 * w + 0.45 * x + 3000.0 * tpw * rows + part + 80000.0;
+    const double c = queue ? w + 0.45 * x + 6500.0 * tpw * rows + part : w + groups * MB * 16.0 * Ks * 2 + 2.0 * tpw * 16 * M * 4;
+    return c * (MB > 2 ? 2 : 1) * (1.0 + 0.02 * S);  // ties go to fewer splits; of more rows, this is what is left
   };
   // Up to 32 rows fewer slices than the stream kernel would take only in queues: its waves' chains would be as much longer (fp16, 32
   // rows of 5120 x 5120, fp32 sums off by 1.09e-7 in four slices, in two by 1.32e-7; and 15.9 us with the tail in queues, 16.3).
+  // More than it would take only in queues, too: int8, 9 rows of 6640 x 8256, four 15.9 us, eight 19.7.
   int best = 1, least = 1;
   if (MB <= 2)
     for (int S = 2; S <= most && S <= cus && nks / S >= ST_KG * 4; S *= 2)
@@ -2845,7 +2848,7 @@ int pick_splits(int64_t M, int N, int K, int wbytes, int most = 8) {
     const bool queue = queue_takes((int)M, w8, tiles(S));
     const int stage = !queue ? (MB > 2 ? 16 : ST_KG * 4) : MB > 2 ? 8 * (w8 ? 2 : 1) : ST_KG * 4;
     if (nks / S < stage) break;  // every wave needs a full stage of K steps
-    if (!queue && S < least) continue;
+    if (!queue && MB <= 2 && S != least) continue;
     const double c = cost(S, queue);
     if (best_cost == 0 || c < best_cost) best = S, best_cost = c;
   }

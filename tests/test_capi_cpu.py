@@ -165,6 +165,18 @@ def test_only_products_that_fold_stop_at_four_slices(N, K, rows, fp16, bf16):
         assert hybrid.msa_linear_bf16_splits(M, N, K, 1) == bf16, M
 
 
+@pytest.mark.parametrize("M,N,K,fp16,int8", [
+    # queues of few tiles, or twice the slices in one pass of the shared-activation kernel
+    (128, 12288, 12288, 4, 2), (100, 12288, 49152, 4, 2), (128, 9216, 36864, 4, 2), (128, 5120, 20480, 8, 4),
+    (64, 12288, 12288, 2, 2), (64, 12288, 49152, 4, 4), (40, 12288, 49152, 4, 4), (57, 4096, 16384, 4, 4),
+    # up to 32 rows: as many as the stream kernel takes, unless queues take others
+    (9, 6640, 8256, 4, 4), (32, 5120, 5120, 4, 4), (32, 9216, 9216, 2, 2), (16, 9216, 9216, 4, 2), (32, 9216, 36864, 4, 4)])
+def test_slices_of_packed_rows(M, N, K, fp16, int8):
+    """(256 compute units)"""
+    core = _capi.load()
+    assert (core.msa_linear_default_splits(M, N, K), core.msa_linear_default_splits_w8a16(M, N, K)) == (fp16, int8)
+
+
 def tiles(M, N, K, S=0, cus=256):
     f = _capi.TileForm()
     assert _capi.load().msa_linear_tiles(M, N, K, S, cus, ctypes.byref(f)) == 0
