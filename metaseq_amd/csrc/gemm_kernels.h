@@ -1444,8 +1444,10 @@ struct GroupTiles {
 // ``part`` ([gridDim.z][M][N]); a later launch adds the slices in slice order.
 // m_own: the first row that the tile owns.
 // ONCE: one row of tiles (or experts of mostly one tile), so that a weight is read by one workgroup: its loads leave nothing in
-// the caches and are served faster (us: 200 x 50272 x 4096 101 -> 96, 100 x 50272 x 4096 84 -> 73, 70 x 16384 x 4096 43.9 -> 41.8,
-// eight slices of 200 x 4096 x 16384 41.5 -> 39.5; two rows of tiles would lose by it, 129 x 12288 x 4096 33.3 -> 39.3).
+// the caches and are served faster (us: 200 x 50272 x 4096 101 -> 96, 100 x 50272 x 4096 84 -> 73, 70 x 16384 x 4096 43.9 -> 41.8;
+// two rows of tiles would lose by it, 129 x 12288 x 4096 33.3 -> 39.3).  Sums in slices are not: by themselves they gain, 146 rows
+// of 8192 x 4608 27.4 -> 26.7, but not with the tail that reads them, 32.5 -> 34.4; bf16, 156 x 4096 x 3072 17.8 -> 19.9, 200 x
+// 4096 x 4096 22.0 -> 22.2; 4096 x 16384 of 130, 200 and 250 rows 44.1 -> 45.1, 46.3 -> 45.7, 49.3 -> 48.0.
 template <int MODE, int WF, bool PART, bool GROUPED, int RF, bool FEW, bool ONCE = false>
 __device__ __forceinline__ void quad_tile(const half_t* __restrict__ x, const void* __restrict__ Wp, int64_t M, int N,
                                           int K, int bx, int64_t m_own, int bz, const Epilogue& epi,
@@ -2141,7 +2143,7 @@ constexpr int QUEUE_TILES = 9;
 constexpr int queue_rows(int M) { return (M + 15) / 16; }  // row blocks that it multiplies, of eight from 65 rows on
 constexpr bool queue_takes(int M, bool w8, int tiles_per_wg) {
   const int mb = queue_rows(M);
-  if (tiles_per_wg > QUEUE_TILES || mb * tiles_per_wg > 64) return false;  // 64: QueueCfg::OK
+  if (tiles_per_wg > QUEUE_TILES || mb * tiles_per_wg > 64) return false;  // 64: QueueCfg::SUMS_FIT
   return mb > 2 || (tiles_per_wg >= 5 && (w8 || mb == 2));
 }
 
@@ -2487,11 +2489,11 @@ void launch_quad(const void* x, const void* W, const void* scales, int64_t M, in
 //   106 -> 86, 129 106 -> 89, 170 111 -> 95, 200 111 -> 101.
 template <int MODE, int WF, int RF>
 void launch_few_rows(const void* x, const void* W, int64_t M, int N, int K, const Epilogue& epi, hipStream_t s) {
-  static std::atomic<uint64_t> lds_allowed_s[2] = {};
+  static std::atomic<uint64_t> lds_allowed_s{0};
   const int ncol = (N + tq_bn(WF) - 1) / tq_bn(WF), nrow = (int)((M + tq_bm(RF) - 1) / tq_bm(RF));
-  auto kernel = nrow == 1 ? linear_quad_kernel<MODE, WF, false, false, RF, true, true>
-                          : linear_quad_kernel<MODE, WF, false, false, RF, true, false>;
-  if (!allow_lds((const void*)kernel, tq_lds_bytes(WF, RF), lds_allowed_s[nrow == 1])) return;
+  constexpr bool ONCE = WF == 8;  // tiles of 256 columns are one row, the others two
+  auto kernel = linear_quad_kernel<MODE, WF, false, false, RF, true, ONCE>;
+  if (!allow_lds((const void*)kernel, tq_lds_bytes(WF, RF), lds_allowed_s)) return;
   const TileOrder o{nrow == 1 ? 0 : -TQ_PANEL, 0};
   hipLaunchKernelGGL(kernel, quad_grid(ncol, nrow, o), dim3(TQ_THREADS), tq_lds_bytes(WF, RF), s, (const half_t*)x, W,
                      M, N, K, o.a, o.r, epi, (float*)nullptr, 0, GroupTiles{});
@@ -2503,12 +2505,11 @@ void launch_few_rows(const void* x, const void* W, int64_t M, int N, int K, cons
 template <int MODE, int WF>
 void launch_quad_partial_w(const void* x, const void* W, float* part, int64_t M, int N, int K,
                            int S, hipStream_t s) {
-  static std::atomic<uint64_t> lds_allowed_p[2] = {};
+  static std::atomic<uint64_t> lds_allowed_p{0};
+  auto kernel = linear_quad_kernel<MODE, WF, true>;
+  if (!allow_lds((const void*)kernel, tq_lds_bytes(WF), lds_allowed_p)) return;
   const int ncol = (N + tq_bn(WF) - 1) / tq_bn(WF);
   const int nrow = (int)((M + TQ_BM - 1) / TQ_BM);
-  auto kernel = nrow == 1 ? linear_quad_kernel<MODE, WF, true, false, 8, false, true>
-                          : linear_quad_kernel<MODE, WF, true, false, 8, false, false>;
-  if (!allow_lds((const void*)kernel, tq_lds_bytes(WF), lds_allowed_p[nrow == 1])) return;
   Epilogue e{};
   const TileOrder o = tile_order(ncol, nrow, WF);
   hipLaunchKernelGGL(kernel, quad_grid(ncol, nrow, o, S), dim3(TQ_THREADS), tq_lds_bytes(WF), s,

@@ -41,7 +41,7 @@ struct QueueCfg {
   static constexpr int JFIT = 160 * 1024 / (KL * MB * 1024), J = JFIT > NT ? NT : JFIT;  // tiles summed at a time
   static constexpr int RING = KL * R * SLOT, RED = KL * J * MB * 1024;
   static constexpr int LDS_BYTES = RING > RED ? RING : RED;
-  static constexpr bool OK = 4 * MB * NT <= 256;  // sums: one accumulator bank
+  static constexpr bool SUMS_FIT = 4 * MB * NT <= 256;  // one accumulator bank
   static_assert(R >= 1 && J >= 1, "a CU has 160 KB of LDS");
 };
 
@@ -350,6 +350,7 @@ template <int MB, bool W8, int MODE, int NT>
 void launch_queue_cfg(const void* xp, const void* W, const void* scales, float* part, int S, int M, int N, int K,
                       int tiles_per_wg, int gx, int ks_per_split, const Epilogue& epi, hipStream_t s) {
   using C = QueueCfg<MB, W8, NT>;
+  static_assert(C::SUMS_FIT, "queue_takes");
   static std::atomic<uint64_t> lds_allowed{0};  // one mask per instantiation
   auto kernel = linear_queue_kernel<MB, W8, MODE, NT>;
   if (!allow_lds((const void*)kernel, C::LDS_BYTES, lds_allowed)) return;  // the caller's launch check reports the error
