@@ -252,8 +252,11 @@ def test_sizes_of_the_kernel_tests_reach_the_kernels_that_they_name():
         assert tuple(tiles(M, N, 1408, S).pieces for S in (0, 1, 2)) == pieces, (M, N)
     for M, N, columns, rows in H.BF16_EVEN:
         assert of(M, N, 1408) == (_capi.MSA_TILES_EVEN, columns, rows), (M, N)
-    assert {tiles(M, N, K).columns for M, N, K in C.QUEUE_ROWS} == {16, 32, 48, 64, 80}
-    assert all(tiles(M, N, K).kind == _capi.MSA_TILES_QUEUE for M, N, K in C.QUEUE_ROWS)
+    assert {tiles(M, N, K).columns for M, N, K, _ in C.QUEUE_ROWS} == {16, 32, 48, 64, 80}
+    assert {tiles(*sizes).columns for sizes in C.QUEUE_ROWS if sizes[3] > 1} == {16, 32, 48, 64, 80}
+    assert all(tiles(M, N, K, s).kind == _capi.MSA_TILES_QUEUE for M, N, K, S in C.QUEUE_ROWS for s in (0, S))
+    for M, N, K in C.TILES_128:
+        assert of(M, N, K) == (_capi.MSA_TILES_FEW, 128, 128), (M, N, K)
     assert {r[2:4] for r in C.EVEN_DEEP} == {(128, 160), (128, 192), (128, 224), (256, 160), (256, 192), (256, 224), (256, 256)}
     assert {r[2:4] for r in C.PARTIALS_DEEP} == {r[2:4] for r in C.EVEN_DEEP}
 

@@ -280,8 +280,8 @@ def test_graph_replay_matches_eager_generation(min_len):
 
 @pytest.mark.parametrize("rows", [70, 128, 140])
 def test_batch_above_64_rows_generates_like_the_oracle(rows):
-    """65 .. 128 rows decode on packed activations with eight row blocks (the shared-activation
-    kernels, stored logits and the stand-alone selection kernel); more rows leave the packed path
+    """65 .. 128 rows decode on packed activations with eight row blocks (queues,
+    stored logits and the stand-alone selection kernel); more rows leave the packed path
     and run on row-major activations through the tiled kernels."""
     cfg = tiny_cfg(layers=2, dim=128, heads=2, vocab=96, max_pos=40)
     model, sd = build(cfg, seed=21)

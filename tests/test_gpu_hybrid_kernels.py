@@ -94,9 +94,9 @@ def test_linear_bf16(M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", [
-    # a wave per tile: vocabularies (13 and 14 tiles per workgroup) from one row on, one to three tiles of 33 to 64 rows,
-    # four of more; the last workgroup's tiles run out
+    # a wave per tile: vocabularies (13 and 14 tiles per workgroup) from one row on
     (1, 50272, 160), (17, 54000, 96), (33, 54000, 160), (64, 50272, 96), (65, 54000, 96), (128, 50272, 160),
+    # (queues: one to three tiles of 33 to 64 rows, four of more; the last workgroup's tiles run out)
     (40, 3088, 160), (50, 8176, 96), (64, 12272, 224), (33, 12288, 96), (100, 16368, 160)])
 def test_linear_bf16_of_a_wave_per_tile(M, N, K):
     test_linear_bf16(M, N, K)
@@ -106,6 +106,12 @@ def test_linear_bf16_of_a_wave_per_tile(M, N, K):
 @pytest.mark.parametrize("M,N,K", [(40, 16400, 320), (64, 28688, 192), (90, 24592, 576), (128, 20496, 320), (20, 32784, 192),
                                    (140, 6160, 576), (190, 10256, 320), (256, 8208, 1088)])
 def test_linear_bf16_in_queues(M, N, K):
+    test_linear_bf16(M, N, K)
+
+
+# more tiles to a workgroup than queues take: the shared-activation kernel in one pass, K that ends inside a stage
+@pytest.mark.parametrize("M,N,K", [(40, 49136, 192), (64, 40976, 320), (128, 36864, 320), (97, 40976, 192)])
+def test_linear_bf16_beyond_queues(M, N, K):
     test_linear_bf16(M, N, K)
 
 
@@ -241,7 +247,10 @@ def test_linear_f32(M, N, K):
 
 # one fp32 kernel serves every shape: the smaller ones do
 @pytest.mark.parametrize("M,N,K,dtype", [s + (BF16,) for s in SHAPES] + [
-    s + (F32,) for s in SHAPES if s[0] * s[1] <= 1 << 21])
+    s + (F32,) for s in SHAPES if s[0] * s[1] <= 1 << 21] + [
+    # in queues of two to nine tiles to a workgroup (256 compute units), packed and, from 129 rows on, row-major
+    s + (BF16,) for s in ((33, 4112, 128), (40, 8208, 192), (64, 20496, 192), (90, 32784, 128), (128, 24592, 192), (20, 20496, 320),
+                          (200, 2064, 576), (140, 4112, 192), (256, 8208, 320))])
 def test_linear_with_bias_activation_and_decays(M, N, K, dtype):
     """Every kernel behind msa_linear: a bias, relu^2, a second output, fp32 columns as they are and
     as decays (logits far out on both sides among them)."""

@@ -375,8 +375,8 @@ LINEAR_SHAPES = [
     (1, 96, 64), (8, 768, 768), (32, 3072, 768), (32, 768, 3072), (33, 2048, 2048),
     (64, 4096, 4096), (17, 50272, 768), (65, 768, 768), (200, 2304, 768), (513, 4096, 1024),
     (129, 1008, 96),
-    # 33 .. 64 rows: the shared-activation kernel with 1, 2 and 3 tiles per wave, a K range
-    # shorter than one stage, and two passes over the workgroup's tiles
+    # 33 .. 64 packed rows: queues of one and six tiles, a K range shorter than one round of the waves; two passes of
+    # the shared-activation kernel over the workgroup's tiles
     (64, 1008, 96), (50, 24576, 256), (40, 73728, 128),
     # enough 256 x 256 tiles to take the large tiled kernel, with ragged M and N edges; a bottom
     # block of at most 128 rows goes through the streaming kernel on row-major activations
@@ -387,8 +387,7 @@ LINEAR_SHAPES = [
     # few rows under a wide output: one row tile of the four-wave kernel plus a bottom block for
     # the streaming kernel; two row tiles, the second moved up over most of the first
     (300, 32768, 128), (420, 32768, 128),
-    # 65 .. 128 packed rows: the shared-activation kernel with eight row blocks and 1, 2 and 3
-    # tiles per wave, several passes over a workgroup's tiles, a K range of one stage
+    # 65 .. 128 packed rows: queues of five, six and eight row blocks, a vocabulary, a K range of few steps
     (128, 4096, 128), (70, 8192, 256), (96, 24576, 128), (128, 50272, 128), (127, 1008, 96),
     # 64 and 44 bottom rows with few tiles per workgroup: the streaming kernel's four-tile groups
     (4160, 4096, 256), (4140, 8192, 128),
@@ -516,35 +515,53 @@ def test_fp32_sums_of_few_rows_are_no_longer_chains(lib, M, N, K, w8, most):
     assert err <= most
 
 
+# more tiles to a workgroup than queues take: nine of eight row blocks, ten to twelve of fewer (the shared-activation kernel in one
+# pass) and one more, the last workgroup short of tiles, K that ends inside a stage and of less than one
+@pytest.mark.parametrize("M,N,K", [(113, 36848, 192), (128, 36864, 320), (65, 36880, 64), (97, 40976, 192), (128, 49136, 128), (70, 49152, 576),
+                                   (33, 36880, 320), (48, 40976, 576), (64, 45056, 320), (40, 49136, 192), (50, 45072, 64), (64, 49168, 128)])
+@pytest.mark.parametrize("w8", [False, True])
+def test_linear_packed_rows_beyond_queues(lib, M, N, K, w8):
+    test_linear_packed_rows_in_queues(lib, M, N, K, w8)
+
+
 # 129 .. 256 row-major rows in queues: every number of row blocks and of tiles to a workgroup (256 compute units), the last
-# columns' workgroup with fewer, blocks whose rows run out, fewer 64-wide stages than waves and more than a queue holds
-QUEUE_ROWS = [(129, 16, 128), (160, 2064, 192), (161, 3072, 768), (192, 4112, 576), (193, 6160, 1088), (224, 8192, 320),
-              (225, 8208, 576), (255, 10240, 192), (256, 6144, 1344), (256, 2048, 704), (130, 10224, 128), (200, 4000, 2048)]
+# columns' workgroup with fewer, blocks whose rows run out, fewer 64-wide stages than waves and more than a queue holds; whole
+# products and, in queues as well, slices of K
+QUEUE_ROWS = [(129, 16, 256, 2), (160, 2064, 768, 4), (161, 3072, 768, 2), (192, 4112, 640, 2), (193, 6160, 1088, 1), (224, 8192, 384, 1),
+              (225, 8208, 576, 1), (255, 10240, 192, 1), (256, 6144, 1344, 1), (256, 2048, 1024, 4), (130, 10224, 128, 1),
+              (200, 4000, 2048, 2), (224, 2560, 2048, 4), (190, 1024, 2048, 8), (140, 768, 1024, 8), (225, 1552, 512, 2)]
 
 
-@pytest.mark.parametrize("M,N,K", QUEUE_ROWS)
-def test_linear_f16_rows_in_queues(lib, M, N, K):
-    """A whole product with bias and, in place, a residual; two slices."""
-    print("queue rows", M, N, K, flush=True)
+@pytest.mark.parametrize("M,N,K,S", QUEUE_ROWS)
+def test_linear_f16_rows_in_queues(lib, M, N, K, S):
+    """A whole product with bias and, in place, a residual; slices, each the sums over its own part of K."""
+    print("queue rows", M, N, K, S, flush=True)
     x, W, b, res = rnd(M, K, seed=7), rnd(N, K, seed=8, std=0.05), rnd(N, seed=9, std=0.1), rnd(M, N, seed=10)
     want = _linear_want(x, W, b, res, False).half()
     Wp, y = pack_w(lib, G(W)), G(res).clone()
     ok(lib.msa_linear_f16(P(G(x)), P(Wp), P(G(b)), P(y), P(y), M, N, K, 0, None), lib)
     torch.cuda.synchronize()
     assert_fp16_close(y, want, atol=float(want.abs().max()) * 2 ** -10, what="queue rows")
-    S = 2 if K % 128 == 0 and K >= 256 else 1
-    part = torch.full((S, M, N), float("nan"), dtype=torch.float32, device=DEV)
+    part = torch.full((S + 1, M, N), float("nan"), dtype=torch.float32, device=DEV)
     ok(lib.msa_linear_partial_f16(P(G(x)), P(Wp), P(part), M, N, K, S, 0, None), lib)
     torch.cuda.synchronize()
-    assert (part.sum(0).cpu() - x.float() @ W.float().t()).abs().max() < 1e-3
+    assert bool(torch.isnan(part[S]).all()), "wrote past the last slice"
+    for xs, ws, got in zip(x.double().chunk(S, 1), W.double().chunk(S, 1), part):
+        want = xs @ ws.t()
+        # a sum of K / S fp32 terms
+        assert float((got.cpu().double() - want).abs().max()) <= 8 * 2.0 ** -24 * (K // S) ** 0.5 * float(want.abs().max())
 
 
-# 128 x 128 tiles (129 .. 256 rows; from a quarter of the chip to all of it, ragged edges, K of the ring's length
-# and more), shapes beside them whose K is too short for those, and 256 x 256 tiles of fewer rows under a wide output
-@pytest.mark.parametrize("M,N,K", [(129, 4096, 128), (160, 4112, 192), (255, 12304, 320), (256, 16384, 640),
-                                   (200, 12288, 4096), (129, 4096, 512), (160, 4112, 576), (255, 12288, 640),
-                                   (256, 16384, 4096), (65, 50272, 128), (130, 50000, 192), (255, 49168, 576),
-                                   (250, 65536, 128)])
+# 128 x 128 tiles: 129 .. 256 rows of more columns than queues take, up to 96 columns of tiles and, of long sums, 128; whole and
+# ragged ones
+TILES_128 = [(129, 10256, 512), (160, 11280, 576), (255, 12272, 640), (200, 12176, 704), (193, 14352, 4096), (200, 12288, 4096),
+             (255, 12288, 640), (256, 16384, 4096)]
+
+
+# those, sizes beside them (fewer columns, in queues; too short a K) and 256 x 256 tiles of fewer rows under a wide output
+@pytest.mark.parametrize("M,N,K", TILES_128 + [(129, 4096, 128), (160, 4112, 192), (255, 12304, 320), (256, 16384, 640),
+                                               (129, 4096, 512), (160, 4112, 576), (65, 50272, 128), (130, 50000, 192),
+                                               (255, 49168, 576), (250, 65536, 128)])
 @pytest.mark.parametrize("epi", ["plain", "bias_relu", "bias_res"])
 def test_linear_f16_few_rows(lib, M, N, K, epi):
     print("few rows", M, N, K, epi, flush=True)
@@ -760,8 +777,7 @@ def test_linear_rejects_bad_shapes(lib):
 @pytest.mark.parametrize("M,N,K", [(8, 768, 768), (64, 3072, 768), (32, 768, 3072),
                                    (200, 2304, 768), (48, 4096, 4096), (64, 24576, 256),
                                    (40, 73728, 128),
-                                   # 9 tiles per workgroup (12 waves as 4 x 3), the last
-                                   # workgroup short of tiles and a K range of 1.5 stages
+                                   # 9 tiles per workgroup: queues, the last workgroup short of tiles
                                    (64, 36864, 256), (50, 36784, 192), (40, 36864, 256),
                                    # 65 .. 128 packed rows
                                    (100, 3072, 768), (128, 36864, 256), (70, 1008, 192),
@@ -789,8 +805,8 @@ def test_linear_w8a16(lib, M, N, K):
 @pytest.mark.parametrize("M,N,K,S", [(32, 768, 768, 1), (32, 768, 3072, 4), (8, 4096, 4096, 4),
                                      (33, 2048, 8192, 8), (64, 768, 3072, 3),
                                      (48, 4608, 2048, 4),
-                                     # int8: 18 and 9 tiles per workgroup (12 waves as 2 x 6
-                                     # and 4 x 3), the second with a ragged last K slice
+                                     # 18 tiles per workgroup (int8: 12 waves as 2 x 6), and 9, in queues, with a
+                                     # ragged last K slice
                                      (64, 9216, 1024, 8), (64, 9216, 1152, 4),
                                      # 65 .. 128 rows
                                      (70, 4096, 4096, 4), (128, 768, 3072, 4), (100, 2048, 1024, 2)])
@@ -956,6 +972,48 @@ def test_qkv_proj_scatter(lib, B, T, H, hd, S0, w8):
         assert_fp16_close(Vc[:, :, S0:S0 + T], want_v.half(), atol=atol, what="V cache")
         # nothing outside the appended slice was touched
         assert float(Kc[:, :, :S0].abs().sum()) == 0 and float(Kc[:, :, S0 + T:].abs().sum()) == 0
+
+
+# two to nine tiles to a workgroup (256 compute units) and every number of row blocks, packed; row-major, 129 .. 256 rows, up to five
+QUEUE_QKV = [(40, 1, 11, 192), (4, 12, 22, 320), (64, 1, 43, 128), (33, 1, 54, 576), (60, 1, 75, 64), (5, 10, 96, 192),
+             (70, 1, 32, 320), (6, 16, 64, 128), (100, 1, 86, 192), (128, 1, 75, 576), (120, 1, 22, 64),
+             (24, 1, 43, 320), (32, 1, 96, 192), (9, 1, 64, 576), (180, 1, 5, 192), (3, 70, 16, 320), (256, 1, 26, 576)]
+
+
+@pytest.mark.parametrize("B,T,H,K,w8", [s + (w8,) for s in QUEUE_QKV for w8 in (False, True) if s[0] * s[1] <= 128 or not w8])
+def test_qkv_proj_in_queues(lib, B, T, H, K, w8):
+    """Keys and values at their places in the cache, queries scaled, each against the sums."""
+    print("qkv queues", B, T, H, K, w8, flush=True)
+    hd, S0, M = 128, 5, B * T
+    D, S_cap, flags = H * hd, S0 + T + 2, IN_PACKED if M <= 128 else 0
+    x, b = rnd(M, K, seed=M), G(rnd(3 * D, seed=3, std=0.1))
+    g = torch.Generator(DEV).manual_seed(H)
+    if w8:
+        q8 = torch.randint(-127, 128, (3 * D, K), generator=g, device=DEV, dtype=torch.int8)
+        sc = (torch.rand(3 * D, generator=g, device=DEV) * 5e-4 + 5e-4).half()
+        W, Wp = (q8.float() * sc.float().unsqueeze(1)).half(), pack_w8(lib, q8)
+    else:
+        W = (torch.randn(3 * D, K, generator=g, device=DEV) * 0.05).half()
+        Wp = pack_w(lib, W)
+    kc, vc = (torch.full((B, H, S_cap, hd), float("nan"), dtype=torch.float16, device=DEV) for _ in range(2))
+    qo = torch.full((M, D), float("nan"), dtype=torch.float16, device=DEV)
+    xin = G(pack_act(x) if flags else x)
+    if w8:
+        ok(lib.msa_qkv_proj_w8a16(P(xin), P(Wp), P(sc), P(b), P(qo), P(kc), P(vc), B, T, H, hd, S0, S_cap, K, flags, None, None), lib)
+    else:
+        ok(lib.msa_qkv_proj_f16(P(xin), P(Wp), P(b), P(qo), P(kc), P(vc), B, T, H, hd, S0, S_cap, K, flags, None, None), lib)
+    torch.cuda.synchronize()
+    for c in (kc, vc):
+        assert bool(torch.isnan(c[:, :, :S0]).all()) and bool(torch.isnan(c[:, :, S0 + T:]).all()), "wrote beside the new positions"
+    sums = G(x).float() @ W.float().t()
+    want = sums.half().float() + b.float()
+    # the bound of test_qkv_proj_rows_cut_evenly_over_more_stages
+    size = torch.maximum(sums.abs(), want.abs())
+    bound = 4 * size * 2.0 ** -11 + 8 * 2.0 ** -24 * K ** 0.5 * float(size.square().mean().sqrt()) + 2.0 ** -24
+    for got, i, scale in ((kc[:, :, S0:S0 + T].permute(0, 2, 1, 3).reshape(M, D), 0, 1.0),
+                          (vc[:, :, S0:S0 + T].permute(0, 2, 1, 3).reshape(M, D), 1, 1.0), (qo, 2, hd ** -0.5)):
+        of = slice(i * D, (i + 1) * D)
+        assert bool(((got.float() - want[:, of] * scale).abs() <= bound[:, of] * scale + (scale < 1) * 2.0 ** -11 * want[:, of].abs() * scale).all()), i
 
 
 @pytest.mark.parametrize("w8", [False, True])
@@ -1367,7 +1425,7 @@ def test_target_logprob(lib):
     # 13 and 14 tiles per workgroup: a wave per tile, every number of row blocks, K that ends inside a stage
     (1, 50272, 96), (16, 54000, 160), (17, 50272, 32), (33, 54000, 64), (48, 50272, 288), (64, 54000, 416),
     (65, 54000, 96), (128, 50272, 160),
-    # one, two and three tiles per workgroup of 33 to 64 rows, four of more; the last workgroup's tiles run out
+    # (queues: one, two and three tiles per workgroup of 33 to 64 rows, four of more; the last workgroup's tiles run out)
     (33, 4096, 1056), (64, 2304, 96), (48, 8176, 416), (64, 6160, 32), (33, 12272, 224), (64, 12288, 96),
     (65, 16368, 160), (128, 16384, 96)])
 def test_products_of_a_wave_per_tile(lib, M, N, K):
