@@ -2100,7 +2100,9 @@ void launch_stream_mb(const void* xp, const void* W, const void* scales, float* 
 }
 
 constexpr int SH_GROUP = 12;  // most tiles per pass of the shared-activation kernel (4 lanes x 3)
-constexpr int SH_GROUP_W8 = 18;  // int8 only: 6 lanes x 3
+// int8 only: 6 lanes x 3, from 14 tiles on (40 / 64 rows, us, against two passes of twelve or, of 14 tiles, the stream kernel: 57344 x 4096
+// 51 / 59 and 60 / 67, 65536 x 8192 100 / 117 and 123 / 136, 73728 x 12288 146 / 167 and 191 / 219)
+constexpr int SH_GROUP_W8 = 18;
 // A vocabulary of 16-bit weights (13 or 14 tiles per workgroup) is one pass of a wave per tile over all of K: no
 // sums between waves, the fewest registers and so the most loads in flight.  Measured, 50272 x 4096, us: 8 rows 69
 // -> 64, 32 rows 75 -> 65 (6.3 TB/s; both on the stream kernel before), 40 rows 75 -> 66, 64 rows 95 -> 66, 100 rows

@@ -33,7 +33,7 @@ struct QueueCfg {
   static constexpr int STEPS = W8 ? 2 : 1;       // 32-wide steps of a slot
   static constexpr int LOADS = STEPS * MB + NT;  // of 1 KB each
   static constexpr int SLOT = LOADS * 1024;
-  static constexpr bool ASIDE = MB <= 2;  // sums are set aside after a quarter of the slots, of eight 32-wide steps at least
+  static constexpr bool ASIDE = MB <= 2;  // slices' sums are set aside after a quarter of the slots, of eight 32-wide steps at least
   // registers: sums, one slot's fragments, and some for addresses and the expansion of int8
   static constexpr int REGS = 4 * ((ASIDE ? 2 : 1) * MB * NT + LOADS) + (W8 ? 20 : 8);
   static constexpr int KL = REGS <= 256 && 8 * SLOT <= 160 * 1024 ? 8 : 4;
@@ -114,7 +114,7 @@ __global__ __launch_bounds__((QueueCfg<MB, W8, NT>::KL * 64)) void linear_queue_
 #pragma unroll
   for (int j = 0; j < NT; ++j)
     if (W8) asm volatile("" : "+v"(sc[j]));
-  const int quarter = max((n + 3) / 4, 8 / STEPS);
+  const int quarter = part ? max((n + 3) / 4, 8 / STEPS) : n + 1;  // (whole products have the stream kernel's chains)
   int slot = 0, until = quarter;
   for (int i = 0; i < n; ++i) {
     // loads complete in order: slot i is there when no more than those of the R - 1 slots behind it are on their way
