@@ -70,18 +70,38 @@ def test_argument_validation_needs_no_gpu():
 
 
 @pytest.mark.parametrize("int8", [0, 1])
-@pytest.mark.parametrize("vocab,positions", [(512, 40), (50272, 2050), (512, 8194)])
-@pytest.mark.parametrize("width", [128, 768, 1024, 2048, 4096, 5120, 9216])
-def test_a_workspace_for_more_rows_serves_fewer(width, vocab, positions, int8):
-    """... also where more rows are summed in fewer slices, where no two launches attend to them or no projection selects."""
+@pytest.mark.parametrize("width", [768, 1024, 2048, 4096, 5120, 9216])
+def test_a_workspace_for_more_rows_serves_fewer(width, int8):
+    """... also where more rows are summed in fewer slices."""
+    lib, h, one = _capi.load(), ctypes.c_void_p(), ctypes.c_void_p(4096)
+    conf = _capi.DecoderConfig(1, width, width // 128, 4 * width, 512, 40, 1, int8)
+    table = (_capi.LayerWeights * 1)()
+    for name, _ in _capi.LayerWeights._fields_:
+        setattr(table[0], name, 4096)
+    assert lib.msa_decoder_create(ctypes.byref(conf), one, one, one, one, one, table, ctypes.byref(h)) == 0
+    need = [lib.msa_decoder_step_workspace_bytes(h, b) for b in range(16, 65)]
+    lib.msa_decoder_destroy(h)
+    assert need == sorted(need) and need[0] > 0
+
+
+def step_workspaces(width, int8, vocab, positions, rows):
     lib, h, one = _capi.load(), ctypes.c_void_p(), ctypes.c_void_p(4096)
     conf = _capi.DecoderConfig(1, width, width // 128, 4 * width, vocab, positions, 1, int8)
     table = (_capi.LayerWeights * 1)()
     for name, _ in _capi.LayerWeights._fields_:
         setattr(table[0], name, 4096)
     assert lib.msa_decoder_create(ctypes.byref(conf), one, one, one, one, one, table, ctypes.byref(h)) == 0
-    need = [lib.msa_decoder_step_workspace_bytes(h, b) for b in range(1, 129)]
+    need = [lib.msa_decoder_step_workspace_bytes(h, b) for b in rows]
     lib.msa_decoder_destroy(h)
+    return need
+
+
+@pytest.mark.parametrize("int8", [0, 1])
+@pytest.mark.parametrize("vocab,positions", [(512, 40), (50272, 2050), (512, 8194)])
+@pytest.mark.parametrize("width", [128, 768, 1024, 2048, 4096, 5120, 9216])
+def test_every_buffer_of_a_workspace_for_more_rows_serves_fewer(width, vocab, positions, int8):
+    """... also where no two launches attend to them, or no projection selects."""
+    need = step_workspaces(width, int8, vocab, positions, range(1, 129))
     assert need == sorted(need) and need[0] > 0
 
 
@@ -252,9 +272,10 @@ def test_sizes_of_the_kernel_tests_reach_the_kernels_that_they_name():
         assert tuple(tiles(M, N, 1408, S).pieces for S in (0, 1, 2)) == pieces, (M, N)
     for M, N, columns, rows in H.BF16_EVEN:
         assert of(M, N, 1408) == (_capi.MSA_TILES_EVEN, columns, rows), (M, N)
-    assert {tiles(M, N, K).columns for M, N, K, _ in C.QUEUE_ROWS} == {16, 32, 48, 64, 80}
-    assert {tiles(*sizes).columns for sizes in C.QUEUE_ROWS if sizes[3] > 1} == {16, 32, 48, 64, 80}
-    assert all(tiles(M, N, K, s).kind == _capi.MSA_TILES_QUEUE for M, N, K, S in C.QUEUE_ROWS for s in (0, S))
+    assert {tiles(M, N, K).columns for M, N, K in C.QUEUE_ROWS} == {16, 32, 48, 64, 80}
+    assert all(tiles(M, N, K).kind == _capi.MSA_TILES_QUEUE for M, N, K in C.QUEUE_ROWS)
+    assert {tiles(*sizes).columns for sizes in C.QUEUE_SLICES} == {16, 32, 48, 64, 80}
+    assert all(tiles(*sizes).kind == _capi.MSA_TILES_QUEUE for sizes in C.QUEUE_SLICES)
     for M, N, K in C.TILES_128:
         assert of(M, N, K) == (_capi.MSA_TILES_FEW, 128, 128), (M, N, K)
     assert {r[2:4] for r in C.EVEN_DEEP} == {(128, 160), (128, 192), (128, 224), (256, 160), (256, 192), (256, 224), (256, 256)}

@@ -525,25 +525,40 @@ def test_linear_packed_rows_beyond_queues(lib, M, N, K, w8):
 
 
 # 129 .. 256 row-major rows in queues: every number of row blocks and of tiles to a workgroup (256 compute units), the last
-# columns' workgroup with fewer, blocks whose rows run out, fewer 64-wide stages than waves and more than a queue holds; whole
-# products and, in queues as well, slices of K
-QUEUE_ROWS = [(129, 16, 256, 2), (160, 2064, 768, 4), (161, 3072, 768, 2), (192, 4112, 640, 2), (193, 6160, 1088, 1), (224, 8192, 384, 1),
-              (225, 8208, 576, 1), (255, 10240, 192, 1), (256, 6144, 1344, 1), (256, 2048, 1024, 4), (130, 10224, 128, 1),
-              (200, 4000, 2048, 2), (224, 2560, 2048, 4), (190, 1024, 2048, 8), (140, 768, 1024, 8), (225, 1552, 512, 2)]
+# columns' workgroup with fewer, blocks whose rows run out, fewer 64-wide stages than waves and more than a queue holds
+QUEUE_ROWS = [(129, 16, 128), (160, 2064, 192), (161, 3072, 768), (192, 4112, 576), (193, 6160, 1088), (224, 8192, 320),
+              (225, 8208, 576), (255, 10240, 192), (256, 6144, 1344), (256, 2048, 704), (130, 10224, 128), (200, 4000, 2048)]
 
 
-@pytest.mark.parametrize("M,N,K,S", QUEUE_ROWS)
-def test_linear_f16_rows_in_queues(lib, M, N, K, S):
-    """A whole product with bias and, in place, a residual; slices, each the sums over its own part of K."""
-    print("queue rows", M, N, K, S, flush=True)
+@pytest.mark.parametrize("M,N,K", QUEUE_ROWS)
+def test_linear_f16_rows_in_queues(lib, M, N, K):
+    """A whole product with bias and, in place, a residual; two slices where K is in whole ones of 128 or more."""
+    print("queue rows", M, N, K, flush=True)
     x, W, b, res = rnd(M, K, seed=7), rnd(N, K, seed=8, std=0.05), rnd(N, seed=9, std=0.1), rnd(M, N, seed=10)
     want = _linear_want(x, W, b, res, False).half()
     Wp, y = pack_w(lib, G(W)), G(res).clone()
     ok(lib.msa_linear_f16(P(G(x)), P(Wp), P(G(b)), P(y), P(y), M, N, K, 0, None), lib)
     torch.cuda.synchronize()
     assert_fp16_close(y, want, atol=float(want.abs().max()) * 2 ** -10, what="queue rows")
-    part = torch.full((S + 1, M, N), float("nan"), dtype=torch.float32, device=DEV)
+    S = 2 if K % 128 == 0 and K >= 256 else 1
+    part = torch.full((S, M, N), float("nan"), dtype=torch.float32, device=DEV)
     ok(lib.msa_linear_partial_f16(P(G(x)), P(Wp), P(part), M, N, K, S, 0, None), lib)
+    torch.cuda.synchronize()
+    assert (part.sum(0).cpu() - x.float() @ W.float().t()).abs().max() < 1e-3
+
+
+# slices of K in queues: every number of tiles to a workgroup, two to eight slices
+QUEUE_SLICES = [(129, 16, 256, 2), (160, 2064, 768, 4), (161, 3072, 768, 2), (192, 4112, 640, 2), (256, 2048, 1024, 4), (200, 4000, 2048, 2),
+                (224, 2560, 2048, 4), (190, 1024, 2048, 8), (140, 768, 1024, 8), (225, 1552, 512, 2)]
+
+
+@pytest.mark.parametrize("M,N,K,S", QUEUE_SLICES)
+def test_linear_partial_f16_rows_in_queues(lib, M, N, K, S):
+    """Each slice holds the sums over its own part of K."""
+    print("queue slices", M, N, K, S, flush=True)
+    x, W = rnd(M, K, seed=7), rnd(N, K, seed=8, std=0.05)
+    part = torch.full((S + 1, M, N), float("nan"), dtype=torch.float32, device=DEV)
+    ok(lib.msa_linear_partial_f16(P(G(x)), P(pack_w(lib, G(W))), P(part), M, N, K, S, 0, None), lib)
     torch.cuda.synchronize()
     assert bool(torch.isnan(part[S]).all()), "wrote past the last slice"
     for xs, ws, got in zip(x.double().chunk(S, 1), W.double().chunk(S, 1), part):
