@@ -494,7 +494,7 @@ class TransformerDecoder(IncrementalDecoder):
     @staticmethod
     def _packed_rows(B):
         """Rows the packed activation buffers of a B-row step hold: whole blocks of 16 up to 64
-        rows, 128 beyond (one kernel shape serves 65 .. 128 rows)."""
+        rows, 128 beyond (one layout of eight row blocks for 65 .. 128 rows)."""
         return ((B + 15) // 16) * 16 if B <= 64 else 128
 
     def _step_buffers(self, cache, B):
