@@ -20,6 +20,7 @@ namespace {
 struct Rows {  // the rows a workgroup works on
   int group;
   int64_t first, end;  // of y (and of x unless permuted)
+  bool alone;          // all of the group's: no other workgroup reads its weights
 };
 
 __device__ __forceinline__ bool find_rows(const msa_group_linear_args& a, int row_tile, int z,
@@ -28,12 +29,14 @@ __device__ __forceinline__ bool find_rows(const msa_group_linear_args& a, int ro
     if (row_tile >= *a.n_tiles) return false;
     r.group = a.tile_group[row_tile];
     r.first = a.tile_row[row_tile];
-    const int64_t ge = a.group_end[r.group];
+    const int64_t ge = a.group_end[r.group], before = a.group_end[r.group > 0 ? r.group - 1 : 0];
     r.end = r.first + a.tile_rows < ge ? r.first + a.tile_rows : ge;
+    r.alone = r.end == ge && r.first == (r.group > 0 ? before : 0);
   } else {
     r.group = z;
     r.first = (int64_t)row_tile * a.tile_rows;
     r.end = r.first + a.tile_rows < a.M ? r.first + a.tile_rows : a.M;
+    r.alone = gridDim.y == 1;
   }
   return r.first < r.end;
 }
@@ -68,16 +71,17 @@ __device__ __forceinline__ void store4(const msa_group_linear_args& a, int group
 
 // MT row blocks of 16 per workgroup, NT column tiles per wave, KW waves share a column range and
 // split K, U 32-wide steps per stage.
-// Bound: the weights' way from memory.  ONCE: hardly a weight is read by two workgroups, and loads that leave nothing in the
-// caches are served faster (64 experts of 1408, width 4096, 16 rows to an expert's tile, us: 1 token 33.4 -> 29.7 and 16.2 ->
-// 15.4, 16 tokens 198 -> 179 and 101 -> 90, which is 6.9 TB/s; 128 tokens, where every second expert has two such tiles, would
-// take 464 for 398).  Routed tiles are taken for that while the groups' mean is half a tile.
+// Bound: the weights' way from memory.  ONCE: no other workgroup reads the tile's weights, and loads that leave nothing in the
+// caches are served faster (64 experts of 1408, width 4096, tiles of 16 rows, us: 1 token of eight experts 33.9 -> 29.6, 16 tokens
+// 223 -> 197 and 113 -> 101, which is 6.9 TB/s).  Weights of a group of several tiles would come from memory for each (60 tokens
+// that all go to the same eight experts 82 -> 109 and 35 -> 53), so that every tile goes by its own group (84 and 35; half of the pairs
+// to eight experts 246 and 126 by the groups' mean, 233 and 114 by their own).
+// A stage's loads are pinned in front of the stage before's products: left to itself the compiler requests those of 64 rows behind
+// most of them (tiles of 64 rows, 96 tokens 249 -> 238 and 145 -> 125, 200 tokens 269 -> 260 and 165 -> 138).
 template <int MT, int NT, int KW, int U, bool GLU, bool ONCE>
-__global__ __launch_bounds__(256) void group_linear_bf16_kernel(msa_group_linear_args a) {
+__device__ __forceinline__ void group_tile(const msa_group_linear_args& a, const Rows& rw,
+                                           float4_t (&red)[KW > 1 ? KW : 1][KW > 1 ? 4 / KW * MT * NT : 1][64]) {
   constexpr int NW = 4 / KW;  // waves side by side over the columns
-  __shared__ float4_t red[KW > 1 ? KW : 1][KW > 1 ? NW * MT * NT : 1][64];
-  Rows rw;
-  if (!find_rows(a, blockIdx.y, blockIdx.z, rw)) return;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int kw = wave % KW, nw = wave / KW;
   const int nks = a.K >> 5, ntiles = a.N >> 4;
@@ -142,8 +146,11 @@ __global__ __launch_bounds__(256) void group_linear_bf16_kernel(msa_group_linear
   int idx = 0;
   for (; idx + 2 <= nst; idx += 2) {
     load(s[1], idx + 1);
+    __builtin_amdgcn_sched_barrier(0);
     mma(s[0], idx);
+    __builtin_amdgcn_sched_barrier(0);
     load(s[0], idx + 2);  // past the end: a clamped address, never multiplied
+    __builtin_amdgcn_sched_barrier(0);
     mma(s[1], idx + 1);
   }
   if (idx < nst) mma(s[0], idx);
@@ -178,15 +185,22 @@ __global__ __launch_bounds__(256) void group_linear_bf16_kernel(msa_group_linear
   }
 }
 
+template <int MT, int NT, int KW, int U, bool GLU>
+__global__ __launch_bounds__(256) void group_linear_bf16_kernel(msa_group_linear_args a) {
+  __shared__ float4_t red[KW > 1 ? KW : 1][KW > 1 ? 4 / KW * MT * NT : 1][64];
+  Rows rw;
+  if (!find_rows(a, blockIdx.y, blockIdx.z, rw)) return;
+  if (rw.alone)
+    group_tile<MT, NT, KW, U, GLU, true>(a, rw, red);
+  else
+    group_tile<MT, NT, KW, U, GLU, false>(a, rw, red);
+}
+
 template <int MT, int NT, int KW, int U>
 void launch_bf16(const msa_group_linear_args& a, int row_tiles, hipStream_t s) {
   constexpr int NB = 4 / KW * NT;
   const dim3 grid((a.N / 16 + NB - 1) / NB, row_tiles, a.tile_group ? 1 : a.groups);
-  const bool glu = a.glu != MSA_GLU_NONE, once = a.tile_group ? a.M * 2 <= (int64_t)a.groups * a.tile_rows : row_tiles == 1;
-  auto kernel = once ? (glu ? group_linear_bf16_kernel<MT, NT, KW, U, true, true>
-                            : group_linear_bf16_kernel<MT, NT, KW, U, false, true>)
-                     : (glu ? group_linear_bf16_kernel<MT, NT, KW, U, true, false>
-                            : group_linear_bf16_kernel<MT, NT, KW, U, false, false>);
+  auto kernel = a.glu != MSA_GLU_NONE ? group_linear_bf16_kernel<MT, NT, KW, U, true> : group_linear_bf16_kernel<MT, NT, KW, U, false>;
   hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, a);
 }
 

@@ -52,18 +52,18 @@ struct Act {
 
 // Rows to a tile of the routed products (bf16; P pairs over E experts, hidden size ff).  What counts is that hardly an
 // expert has two tiles, whose weights are then read twice, and how fast a tile's kernel reads them: tiles of 16 rows at 6.9
-// TB/s, of 64 at 5 to 6, the 256-row kernel, whose tiles are as high as an expert's rows need, at 5.5 to 5.8.  Both products of
-// 64 experts of 1408, width 4096, us, by tokens of which each has eight experts: 48 tokens in tiles of 16 rows 346, of 64 383; 64
-// tokens 374, 393; 96 tokens 459, 412; 128 tokens 543 (of 32 rows 537), 437; 160 tokens of 32 rows 445, 64 413, 256 389; 256
-// tokens of 32 rows 583, 64 462, 256 395; 320 tokens of 64 506, 256 404; 512 tokens 760, 427.
+// TB/s, of 64 at 5.5 to 6.5, the 256-row kernel, whose tiles are as high as an expert's rows need, at 5.5 to 5.8.  Both products of
+// 64 experts of 1408, width 4096, us, by tokens of which each has eight experts: 48 tokens in tiles of 16 rows 357, of 64 357; 64
+// tokens 384, 366; 96 tokens 444, 392; 128 tokens 549 (of 32 rows 536), 410; 160 tokens of 32 rows 444, 64 383, 256 385; 260
+// tokens of 32 rows 593, 64 418, 256 395; 320 tokens of 64 440, 256 404; 520 tokens 662, 444.
 // From 64 rows on a workgroup has 256 columns.  Where the narrower product has fewer of them than two to a compute unit, tiles
 // of 16 and 32 rows, whose workgroups have 32 columns, are ahead for longer, and of fewer than one for as long as there are few
-// rows at all (16 / 32 / 64 / 256 rows): 16 experts of 2816, width 512, 66 tokens 35 / 37 / 90, width 1024, 200 tokens 83 / 65 / 119 /
-// 93, width 3072, 260 tokens 255 / 220 / 226 / 166; 64 experts of 704, width 2048, 72 tokens 107 / 102 / 112, 96 tokens 120 / 116 / 118,
-// 200 tokens 157 / 122 / 124 / 122; 128 experts of 128 in 512, 140 tokens 11.2 in tiles of 16, 23 of 64 and 26 of 256.  A stage of 32 rows is half
-// of a sum of 512 (128 experts of 1408, 150 tokens 100 / 113).  Over 1092 pairs of tokens (33 to 1000) and layers (512 to 4096
-// wide, 16 to 128 experts of 256 to 2816) the tile chosen is 1.1 % slower than the best on average; heights by the rows alone, 16,
-// 32, 64, 256, were 11 %.
+// rows at all (16 / 32 / 64 / 256 rows): 16 experts of 2816, width 512, 64 tokens 32 / 36 / 63, width 1024, 200 tokens 89 / 73 / 91 /
+// 94, width 3072, 260 tokens 261 / 225 / 184 / 167; 64 experts of 704, width 2048, 72 tokens 104 / 104 / 108, 96 tokens 118 / 118 / 113,
+// 200 tokens 161 / 121 / 114 / 123; 128 experts of 128 in 512, 140 tokens 16 / 18 / 21 / 29.  A stage of 32 rows is half
+// of a sum of 512 (128 experts of 1408, 140 tokens 98 / 113).  Over 1953 pairs of tokens (34 to 1000) and layers (512 to 4096
+// wide, 16 to 128 experts of 128 to 2816) the tile chosen is 2.3 % slower than the best on average, with every line fitted
+// anew 2.1; heights by the rows alone, 16, 32, 64, 256, are 10 %.
 // The 256-row kernel takes no packed rows and reaches 4 GB of them, the others any number.  The choice is one of speed: 64 and
 // 256 rows are one chain of sums over K, 16 and 32 four, and the results, bf16, are as far from 64 bits either way (K = 8192, 24
 // rows to an expert: 1.6605538e-3 from all four).
