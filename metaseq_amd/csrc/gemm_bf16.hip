@@ -7,9 +7,11 @@ namespace {
 template <int MODE>
 bool run_grouped(const msa_group_linear_args& a, const Epilogue& e, hipStream_t s) {
   static std::atomic<uint64_t> lds_allowed[2] = {};
-  // up to 64 rows to an expert on average: nearly all have one tile (320 tokens of 8 in 64 experts of 1408, width 4096, 274 ->
-  // 261 and 149 -> 144 us; 512 tokens 275 -> 276 and 160 -> 151)
-  const bool once = a.M <= (int64_t)a.groups * 64;
+  // up to half a tile to an expert on average: many have one tile, whose weights pass by the caches (64 experts of 1408, width 4096,
+  // tokens of eight experts, us, none so / by the experts' mean of up to 64 / each by its own tile: 320 tokens 274 / 261 / 261 and 149 /
+  // 144 / 144; 512 tokens, half of the pairs to eight experts, 385 / 351 / 338 and 190 / 180 / 155; 400, all to eight, 97 / 101 / 97
+  // and 38 / 42 / 38; 900 tokens 320 / 320 / 319 and 177 / 177 / 165).  Beyond, no tile asks for its expert's (6038 tokens 541, 547 if it does).
+  const bool once = a.M <= (int64_t)a.groups * 128;
   auto kernel = once ? linear_quad_kernel<MODE, 8, false, true, 8, false, true>
                      : linear_quad_kernel<MODE, 8, false, true, 8, false, false>;
   if (!allow_lds((const void*)kernel, tq_lds_bytes(8), lds_allowed[once])) return false;

@@ -1443,7 +1443,7 @@ struct GroupTiles {
 // that starts at stage z * part_stages and stores its fp32 sums, with no epilogue, as slice z of
 // ``part`` ([gridDim.z][M][N]); a later launch adds the slices in slice order.
 // m_own: the first row that the tile owns.
-// ONCE: one row of tiles (or experts of mostly one tile), so that a weight is read by one workgroup: its loads leave nothing in
+// ONCE: one row of tiles (or an expert's only one), so that a weight is read by one workgroup: its loads leave nothing in
 // the caches and are served faster (us: 200 x 50272 x 4096 101 -> 96, 100 x 50272 x 4096 84 -> 73, 70 x 16384 x 4096 43.9 -> 41.8;
 // two rows of tiles would lose by it, 129 x 12288 x 4096 33.3 -> 39.3).  Sums in slices are not: by themselves they gain, 146 rows
 // of 8192 x 4608 27.4 -> 26.7, but not with the tail that reads them, 32.5 -> 34.4; bf16, 156 x 4096 x 3072 17.8 -> 19.9, 200 x
@@ -1938,13 +1938,25 @@ __device__ __forceinline__ void quad_place(int t, int ncol, int nrow, int rm_a, 
   }
 }
 
+// a group's last tile is as high as its rows need (48304 rows in 64 groups x 2816 x 4096 1154 -> 1125 us)
+template <int MODE, int WF, bool ONCE>
+__device__ __forceinline__ void quad_group_tile(const half_t* __restrict__ x, const void* __restrict__ Wp, int64_t M, int N, int K,
+                                                int bx, int64_t m_own, const Epilogue& epi, const GroupTiles& gt) {
+  if (M - m_own <= 128)
+    quad_tile<MODE, WF, false, true, 4, false, ONCE>(x, Wp, M, N, K, bx, m_own, 0, epi, nullptr, 0, gt);
+  else if (M - m_own <= 192)
+    quad_tile<MODE, WF, false, true, 6, false, ONCE>(x, Wp, M, N, K, bx, m_own, 0, epi, nullptr, 0, gt);
+  else
+    quad_tile<MODE, WF, false, true, 8, false, ONCE>(x, Wp, M, N, K, bx, m_own, 0, epi, nullptr, 0, gt);
+}
+
+// ONCE of a grouped product: where an expert has one tile
 template <int MODE, int WF, bool PART = false, bool GROUPED = false, int RF = 8, bool FEW = false, bool ONCE = false>
 __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
     const half_t* __restrict__ x, const void* __restrict__ Wp, int64_t M, int N, int K,
     int rm_a, int rm_r, Epilogue epi, float* __restrict__ part, int part_stages,
     GroupTiles gt = GroupTiles{}) {
   int bx = blockIdx.x, by = blockIdx.y;
-  int64_t g_first = 0;
   if constexpr (GROUPED) {
     const int ncol = gridDim.x, L = by * ncol + bx, total = *gt.n_tiles * ncol;
     const int per = (total + 7) / 8, t = (L & 7) * per + (L >> 3);
@@ -1952,21 +1964,20 @@ __global__ __launch_bounds__(TQ_THREADS) void linear_quad_kernel(
     by = t / ncol;
     bx = t - by * ncol;
     const int g = gt.tile_group[by];
-    g_first = gt.tile_row[by];
-    M = min((int64_t)gt.group_end[g], g_first + tq_bm(RF));
+    const int64_t first = gt.tile_row[by], end = gt.group_end[g], before = ONCE && g > 0 ? gt.group_end[g - 1] : 0;
+    M = min(end, first + tq_bm(RF));
     Wp = (const char*)Wp + (int64_t)g * N * K * 2;
+    if constexpr (ONCE)
+      if (first == before && M == end) return quad_group_tile<MODE, WF, true>(x, Wp, M, N, K, bx, first, epi, gt);
+    return quad_group_tile<MODE, WF, false>(x, Wp, M, N, K, bx, first, epi, gt);
   } else if (WF > 2 && rm_a < 0) {  // a row of the grid is a panel
     const int ncol = (N + tq_bn(WF) - 1) / tq_bn(WF), nrow = (int)((M + tq_bm(RF) - 1) / tq_bm(RF));
     if (!quad_panel(by, bx, ncol, nrow, bx, by)) return;
   } else if (rm_a > 0) {
     quad_regroup(by * gridDim.x + bx, gridDim.x, gridDim.y, rm_a, rm_r, bx, by);
   }
-  const int64_t m_own = GROUPED ? g_first : (int64_t)by * tq_bm(RF);
-  if constexpr (GROUPED) {  // a group's last tile is as high as its rows need (48304 rows in 64 groups x 2816 x 4096 1154 -> 1125 us)
-    if (M - m_own <= 128) return quad_tile<MODE, WF, PART, true, 4, FEW, ONCE>(x, Wp, M, N, K, bx, m_own, 0, epi, part, 0, gt);
-    if (M - m_own <= 192) return quad_tile<MODE, WF, PART, true, 6, FEW, ONCE>(x, Wp, M, N, K, bx, m_own, 0, epi, part, 0, gt);
-  }
-  quad_tile<MODE, WF, PART, GROUPED, RF, FEW, ONCE>(x, Wp, M, N, K, bx, m_own, blockIdx.z, epi, part, part_stages, gt);
+  if constexpr (!GROUPED)
+    quad_tile<MODE, WF, PART, false, RF, FEW, ONCE>(x, Wp, M, N, K, bx, (int64_t)by * tq_bm(RF), blockIdx.z, epi, part, part_stages, gt);
 }
 
 // Tiles that would begin a round without filling half of it, in pieces: the first n_full tiles (of all K slices, whole

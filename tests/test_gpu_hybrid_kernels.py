@@ -629,6 +629,48 @@ def test_group_linear_routed_tiles_read_once_or_often(rows, dense, N, K):
     close(y[:P], ref, 6e-3, "rows %d" % rows)
 
 
+# experts of one tile of every height and of several, the first and the last among them, where each asks for its own
+@pytest.mark.parametrize("rows,counts", [(16, [16, 0, 17, 1, 33, 15]), (32, [33, 32, 0, 64, 65, 1, 3, 31]), (64, [64, 65, 1, 128, 0, 129, 63]),
+                                         (256, [130, 192, 0, 257, 406, 449, 193, 1, 128, 256, 129, 0, 3, 0, 0, 385] + [1] * 8)])
+@pytest.mark.parametrize("kind", [-1, _capi.MSA_GLU_CLAMPED])
+def test_group_linear_tiles_of_experts_of_one_and_several(rows, counts, kind):
+    lib = _capi.load_hybrid()
+    print("experts", rows, kind, flush=True)
+    g, N, K = gen(rows + kind), 544, 576
+    E, P = len(counts), sum(counts)
+    assert rows < 256 or P <= E * 128
+    flat = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(P, generator=g)]
+    x = torch.randn(P, K, generator=g).to(BF16)
+    w = (torch.randn(E, N, K, generator=g) * K ** -0.5).to(BF16)
+    n_max = P // rows + E
+    ids = flat.int().cuda()
+    perm, inv = (torch.full((P,), -1, dtype=torch.int32, device="cuda") for _ in range(2))
+    end, n = torch.zeros(E, dtype=torch.int32, device="cuda"), torch.zeros(1, dtype=torch.int32, device="cuda")
+    tg, tr = (torch.full((n_max,), -1, dtype=torch.int32, device="cuda") for _ in range(2))
+    check(lib.msa_moe_plan(ptr(ids), P, E, rows, ptr(perm), ptr(inv), ptr(end), ptr(tg), ptr(tr), ptr(n), n_max,
+                           _capi.stream_ptr()), lib)
+    cols = N // 2 if kind >= 0 else N
+    xd, wd = x.cuda(), pack_tiles(w.view(E * N, K)).cuda()
+    y = torch.full((P + 1, cols), 7.0, dtype=BF16, device="cuda")
+    a = _capi.GroupLinearArgs()
+    a.dtype, a.glu, a.limit = 0, kind, 0.7
+    a.x, a.ldx, a.W, a.y, a.ldy = ptr(xd), K, ptr(wd), ptr(y), cols
+    a.N, a.K, a.groups, a.M = N, K, E, P
+    a.perm, a.tile_group, a.tile_row, a.n_tiles, a.group_end = ptr(perm), ptr(tg), ptr(tr), ptr(n), ptr(end)
+    a.rows_per_x, a.max_tiles, a.tile_rows = 1, n_max, rows
+    check(lib.msa_group_linear(ctypes.byref(a), _capi.stream_ptr()), lib)
+    torch.cuda.synchronize()
+    assert bool((y[P] == 7.0).all()), "wrote past the last row"
+    first, order = 0, torch.sort(flat, stable=True).indices
+    for e, count in enumerate(counts):
+        ref = x[order[first:first + count]].double() @ w[e].double().T
+        if kind >= 0:
+            ref = glu(kind, ref[:, 0::2], ref[:, 1::2], 0.7)
+        if count:
+            close(y[first:first + count], ref, 6e-3, "expert of %d" % count)
+        first += count
+
+
 @pytest.mark.parametrize("E,groups,keep,top", [(1, 1, 1, 1), (12, 1, 1, 5), (12, 4, 2, 3),
                                                (96, 8, 3, 10), (512, 16, 16, 8), (300, 100, 1, 3)])
 def test_route_and_plan(E, groups, keep, top):
