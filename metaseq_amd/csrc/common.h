@@ -49,6 +49,11 @@ int msa_launch_prefill_attention(const void* q, const void* Kc, const void* Vc,
 
 // routed products over 256-row tiles, bf16 (gemm_bf16.hip)
 bool msa_launch_group_quad(const msa_group_linear_args& a, hipStream_t stream);
+// whether the weights of all routed experts are more than the chip's 32 MB of L2 may hold until they are read again: then loads that pass by
+// the caches are the faster ones (both products of routed layers, us, through the caches / past them: 16 experts of 128, width 512,
+// 4 and 2 MB, 1 token 6.9 / 8.6; 64 experts of 128 in 512, 16 and 8 MB, 64 tokens 10.8 / 12.5; 16 experts of 256 in 2048, 32 and 16
+// MB, 64 tokens 16.1 / 15.7 and, the first so and the second not, 14.6; 64 experts of 256 in 1024, 64 and 32 MB, 26.2 / 24.5)
+inline bool group_weights_large(const msa_group_linear_args& a) { return (int64_t)a.groups * a.N * a.K * 2 >= 24 << 20; }
 // the delta rule sixteen tokens at a time, for calls with scratch (delta_chunks.hip)
 int msa_launch_delta_chunks(const msa_delta_args& a, const msa_batch* b, float* scratch, hipStream_t stream);
 int msa_launch_linear_post(const msa_linear_args& a, hipStream_t stream);

@@ -11,7 +11,7 @@ bool run_grouped(const msa_group_linear_args& a, const Epilogue& e, hipStream_t 
   // tokens of eight experts, us, none so / by the experts' mean of up to 64 / each by its own tile: 320 tokens 274 / 261 / 261 and 149 /
   // 144 / 144; 512 tokens, half of the pairs to eight experts, 385 / 351 / 338 and 190 / 180 / 155; 400, all to eight, 97 / 101 / 97
   // and 38 / 42 / 38; 900 tokens 320 / 320 / 319 and 177 / 177 / 165).  Beyond, no tile asks for its expert's (6038 tokens 541, 547 if it does).
-  const bool once = a.M <= (int64_t)a.groups * 128;
+  const bool once = a.M <= (int64_t)a.groups * 128 && group_weights_large(a);
   auto kernel = once ? linear_quad_kernel<MODE, 8, false, true, 8, false, true>
                      : linear_quad_kernel<MODE, 8, false, true, 8, false, false>;
   if (!allow_lds((const void*)kernel, tq_lds_bytes(8), lds_allowed[once])) return false;

@@ -26,12 +26,15 @@ struct Rows {  // the rows a workgroup works on
 __device__ __forceinline__ bool find_rows(const msa_group_linear_args& a, int row_tile, int z,
                                           Rows& r) {
   if (a.tile_group) {
-    if (row_tile >= *a.n_tiles) return false;
+    const int n = *a.n_tiles;
+    if (row_tile >= n) return false;
     r.group = a.tile_group[row_tile];
     r.first = a.tile_row[row_tile];
-    const int64_t ge = a.group_end[r.group], before = a.group_end[r.group > 0 ? r.group - 1 : 0];
+    // told by the tiles beside it, which are requested with its own (by the group's ends the weights wait for a round trip more)
+    const int before = a.tile_group[max(row_tile - 1, 0)], behind = a.tile_group[min(row_tile + 1, a.max_tiles - 1)];
+    r.alone = (int)(row_tile == 0 | before != r.group) & (int)(row_tile + 1 == n | behind != r.group);
+    const int64_t ge = a.group_end[r.group];
     r.end = r.first + a.tile_rows < ge ? r.first + a.tile_rows : ge;
-    r.alone = r.end == ge && r.first == (r.group > 0 ? before : 0);
   } else {
     r.group = z;
     r.first = (int64_t)row_tile * a.tile_rows;
@@ -186,11 +189,11 @@ __device__ __forceinline__ void group_tile(const msa_group_linear_args& a, const
 }
 
 template <int MT, int NT, int KW, int U, bool GLU>
-__global__ __launch_bounds__(256) void group_linear_bf16_kernel(msa_group_linear_args a) {
+__global__ __launch_bounds__(256) void group_linear_bf16_kernel(msa_group_linear_args a, bool large) {
   __shared__ float4_t red[KW > 1 ? KW : 1][KW > 1 ? 4 / KW * MT * NT : 1][64];
   Rows rw;
   if (!find_rows(a, blockIdx.y, blockIdx.z, rw)) return;
-  if (rw.alone)
+  if (rw.alone & large)
     group_tile<MT, NT, KW, U, GLU, true>(a, rw, red);
   else
     group_tile<MT, NT, KW, U, GLU, false>(a, rw, red);
@@ -201,7 +204,7 @@ void launch_bf16(const msa_group_linear_args& a, int row_tiles, hipStream_t s) {
   constexpr int NB = 4 / KW * NT;
   const dim3 grid((a.N / 16 + NB - 1) / NB, row_tiles, a.tile_group ? 1 : a.groups);
   auto kernel = a.glu != MSA_GLU_NONE ? group_linear_bf16_kernel<MT, NT, KW, U, true> : group_linear_bf16_kernel<MT, NT, KW, U, false>;
-  hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, a);
+  hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, a, !a.tile_group || group_weights_large(a));
 }
 
 // ---- fp32 -----------------------------------------------------------------------------------
