@@ -60,10 +60,10 @@ struct Act {
 // of 16 and 32 rows, whose workgroups have 32 columns, are ahead for longer, and of fewer than one for as long as there are few
 // rows at all (16 / 32 / 64 / 256 rows): 16 experts of 2816, width 512, 64 tokens 32 / 36 / 63, width 1024, 200 tokens 89 / 73 / 91 /
 // 94, width 3072, 260 tokens 261 / 225 / 184 / 167; 64 experts of 704, width 2048, 72 tokens 104 / 104 / 108, 96 tokens 118 / 118 / 113,
-// 200 tokens 161 / 121 / 114 / 123; 128 experts of 128 in 512, 140 tokens 16 / 18 / 21 / 29.  A stage of 32 rows is half
+// 200 tokens 161 / 121 / 114 / 123; 128 experts of 128 in 512, 140 tokens 16 / 18 / 21 / 29; 64 of 256 in 512, 230 tokens 21 / 21 / 26 / 29.  A stage of 32 rows is half
 // of a sum of 512 (128 experts of 1408, 140 tokens 98 / 113).  Over 1953 pairs of tokens (34 to 1000) and layers (512 to 4096
-// wide, 16 to 128 experts of 128 to 2816) the tile chosen is 2.3 % slower than the best on average, with every line fitted
-// anew 2.1; heights by the rows alone, 16, 32, 64, 256, are 10 %.
+// wide, 16 to 128 experts of 128 to 2816) the tile chosen is 2.2 % slower than the best on average, with every line fitted
+// anew 2.0; heights by the rows alone, 16, 32, 64, 256, are 10 %.
 // The 256-row kernel takes no packed rows and reaches 4 GB of them, the others any number.  The choice is one of speed: 64 and
 // 256 rows are one chain of sums over K, 16 and 32 four, and the results, bf16, are as far from 64 bits either way (K = 8192, 24
 // rows to an expert: 1.6605538e-3 from all four).
@@ -77,7 +77,7 @@ int routed_rows(int P, int E, int width, int ff, bool packed, int cus) {
     return avg <= 12 ? 32 : avg <= (width <= 3072 ? 24 : 16) ? 64 : tall;
   }
   if ((packed && avg < 10) || (width <= 512 && avg <= 16)) return 16;
-  if (groups < cus) return P * columns <= 14 * (int64_t)cus ? 32 : tall;
+  if (groups < cus) return P * columns <= 14 * (int64_t)cus || (width <= 512 && avg <= 40) ? 32 : tall;
   return avg <= (packed ? 11 : width <= 2048 ? 24 : 16) ? 32 : tall;
 }
 

@@ -316,6 +316,7 @@ def test_a_step_reserves_what_the_delta_rule_takes(heads, vdim, short, long, per
 
 
 @pytest.mark.parametrize("tokens,top,E,width,ff,rows", [
+    (230, 8, 64, 512, 256, 32), (320, 8, 64, 512, 256, 32), (340, 8, 64, 512, 256, 256),
     # low tiles where tall ones have too few workgroups, in either product
     (66, 2, 16, 512, 2816, 16), (128, 2, 16, 1024, 2816, 32), (200, 2, 16, 1024, 2816, 32), (66, 8, 64, 2048, 704, 16),
     (80, 4, 32, 1024, 1408, 32), (66, 8, 64, 512, 1408, 16), (260, 2, 16, 3072, 256, 32), (520, 2, 16, 2048, 1408, 256),
