@@ -7,7 +7,7 @@
 // barrier in the main loop.  Few rows (a decode step): the four waves split K and their sums meet
 // in LDS; many rows: every wave owns its own column tiles.  Loads run one stage ahead of the MFMAs.
 //
-// Routed products with more than 64 rows per expert run on the four-wave 256 x 256 kernel of the dense
+// Routed products of many rows per expert (tile_rows 256) run on the four-wave 256 x 256 kernel of the dense
 // products instead (gemm_kernels.h).
 //
 // fp32: 64 x 64 tiles through LDS on the vector ALU in full fp32; also the fp32 linear layers.
